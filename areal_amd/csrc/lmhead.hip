@@ -72,18 +72,50 @@ DEVI bool gemm_skipped(const GemmArgs& g) { return gate_closed(g.skip_if_set, g.
 // q. They are laid out as an RB x RS block of (B tiles) x (splits) so that they share operand
 // tiles through that XCD's L2. A launch with fewer workgroups than the chip has CUs can use
 // super-blocks of 8 instead, which spread over the XCDs more evenly (several share an XCD's round).
+//
+// The sweeps (a workgroup takes several A tiles against one B tile: the forward and the recompute
+// launch) and dHidden are laid out per XCD instead (xg > 0): the A tiles are cut into xg groups, the B
+// tiles into bg and the k range into kg, xg * bg * kg = 8, one combination per XCD, which cuts its A
+// group into S splits and its k range into zk copies. An XCD's workgroups follow each other copy by
+// copy, in a copy in blocks of RB B tiles, all splits of a block before the next block, so that 32
+// consecutive ones are RB B tiles x 32 / RB splits. Every XCD has the same number of tiles to
+// within one row or column of them, whatever the number of B tiles is.
 struct Sched {
   int bj0, nbj;  // B tiles [bj0, bj0 + nbj)
   int ai0, nai;  // A tiles [ai0, ai0 + nai)
-  int S;         // splits of the A-tile range
+  int S;         // splits of the A-tile range (xg > 0: of an XCD's A group)
   int RB, RS;    // RB * RS == 1 << sb_log2
   int sb_log2;   // log2 of the workgroups per super-block: 5 or 3
   int n_sb_j;    // super-blocks along j
   int n_sb;      // total super-blocks
+  int xg, bg;    // XCD layout (xg = 0: super-blocks); kg = 8 / (xg * bg)
+  int zk;        // copies per XCD
 };
 
-DEVI bool sched_decode(const Sched& sc, int id, int& bj, int& split, int& ai_begin, int& ai_end) {
-  const int xcd = id & 7, q = id >> 3;
+// z: the workgroup's copy of a split-K launch (XCD layout only; unchanged otherwise).
+DEVI bool sched_decode(const Sched& sc, int id, int& bj, int& split, int& ai_begin, int& ai_end, int& z) {
+  const int xcd = id & 7;
+  int q = id >> 3;
+  if (sc.xg > 0) {
+    const int ag = xcd % sc.xg, xb = xcd / sc.xg, bgi = xb % sc.bg, kgi = xb / sc.bg;
+    const int b0 = bgi * sc.nbj / sc.bg, nb = (bgi + 1) * sc.nbj / sc.bg - b0;
+    const int a0 = ag * sc.nai / sc.xg, na = (ag + 1) * sc.nai / sc.xg - a0;
+    // one tile per workgroup (S >= na): as many splits as the group has tiles
+    const int S = sc.S < na ? sc.S : na;
+    const int per_copy = nb * S;
+    if (q >= per_copy * sc.zk) return false;
+    const int copy = q / per_copy;
+    q -= copy * per_copy;
+    z = kgi * sc.zk + copy;
+    const int blk = q / (sc.RB * S), r = q - blk * sc.RB * S;
+    const int left = nb - blk * sc.RB, rb = left < sc.RB ? left : sc.RB;
+    const int sp = r / rb;
+    bj = sc.bj0 + b0 + blk * sc.RB + (r - sp * rb);
+    ai_begin = sc.ai0 + a0 + sp * na / S;
+    ai_end = sc.ai0 + a0 + (sp + 1) * na / S;
+    split = ag * sc.S + sp;
+    return ai_begin < ai_end;
+  }
   const int sb = (q >> sc.sb_log2) * 8 + xcd;
   const int r = q & ((1 << sc.sb_log2) - 1);
   if (sb >= sc.n_sb) return false;
@@ -99,6 +131,7 @@ DEVI bool sched_decode(const Sched& sc, int id, int& bj, int& split, int& ai_beg
 
 static Sched make_sched(int bj0, int nbj, int ai0, int nai, int S, int sb_wgs = 32) {
   Sched sc;
+  sc.xg = sc.bg = 0; sc.zk = 1;
   sc.bj0 = bj0; sc.nbj = nbj; sc.ai0 = ai0; sc.nai = nai; sc.S = S;
   sc.sb_log2 = sb_wgs == 8 ? 3 : 5;
   const int rs_max = sb_wgs == 8 ? 4 : 8;
@@ -110,7 +143,59 @@ static Sched make_sched(int bj0, int nbj, int ai0, int nai, int S, int sb_wgs = 
   sc.n_sb = sc.n_sb_j * n_sb_s;
   return sc;
 }
-static int sched_grid(const Sched& sc) { return ((sc.n_sb + 7) / 8) * 8 * (1 << sc.sb_log2); }
+static Sched make_xcd_sched(int nbj, int nai, int S, int xg, int bg, int zk, int RB) {
+  Sched sc = make_sched(0, nbj, 0, nai, S);
+  sc.xg = xg; sc.bg = bg; sc.zk = zk; sc.RB = RB;
+  return sc;
+}
+static int sched_grid(const Sched& sc) {
+  if (sc.xg > 0) {
+    const int na = (int)ceil_div_i64(sc.nai, sc.xg);
+    return 8 * (int)ceil_div_i64(sc.nbj, sc.bg) * (sc.S < na ? sc.S : na) * sc.zk;
+  }
+  return ((sc.n_sb + 7) / 8) * 8 * (1 << sc.sb_log2);
+}
+// Block width of an XCD's workgroups, and the distinct operand tiles that 32 neighbouring ones read
+// (nb B tiles, S splits): the fewer, the less traffic from outside the XCD's L2. 4 x 8 and 8 x 4 need
+// 12. A block whose workgroups are not a multiple of 32 leaves windows that straddle two blocks.
+static int xcd_block(int S) { return S >= 8 ? 4 : (S >= 4 ? 8 : (S >= 2 ? 16 : 32)); }
+static double xcd_distinct(int nb, int S) {
+  const int RB = xcd_block(S), rb = RB < nb ? RB : nb, rs = (int)ceil_div_i64(32, rb);
+  double d = rb + (rs < S ? rs : S);
+  if (nb > rb && rb * S % 32 != 0) d += rb * (rb * S > 32 ? 32.0 / (rb * S) : 1.0);
+  return d;
+}
+
+// The layout of a sweep of nai A tiles against each of nbj B tiles of nk k-tiles: the numbers of A
+// groups and of splits that the busiest XCD's 32 CUs finish first. A tile takes about 1.2 us per
+// k-tile (H = 896 to 5120) and 11 us for its softmax epilogue, a workgroup's start and end 5 us more
+// (nothing overlaps them); a CU that runs one workgroup waits for the longest of them, one that
+// runs several averages over their lengths to about a tile. Each distinct operand tile beyond
+// 12 costs about 0.5 % (2 x 16 and 32 x 1 measured 2 to 12 % slower at H = 4096), and XCDs that sweep
+// different parts of the vocabulary at a time 1 to 5 % more than ones that share them in the
+// memory-side cache (H = 896 to 4096).
+static Sched plan_sweep(int nbj, int nai, int nk) {
+  Sched best;
+  double best_cost = 0.0;
+  const double tile = 1.2 * nk + 11.0, start = 5.0;
+  for (int xg = 8; xg >= 1; xg >>= 1) {
+    if (xg > nai && xg > 1) continue;
+    const int nb = (int)ceil_div_i64(nbj, 8 / xg), na = (int)ceil_div_i64(nai, xg);
+    for (int S = 1; S <= nai / xg && S <= 64; ++S) {  // (no empty split: the merge reads every slot)
+      const int rounds = (int)ceil_div_i64((int64_t)nb * S, 32);
+      const double per = (double)na / S, distinct = xcd_distinct(nb, S);
+      const double tiles = rounds == 1 ? (double)ceil_div_i64(na, S) : rounds * per + 1.0;
+      const double apart = xg == 1 ? 0.0 : (xg == 2 ? 0.01 : (xg == 4 ? 0.02 : 0.05));
+      const double cost = (tiles * tile + rounds * start) *
+                          (1.0 + 0.005 * (distinct > 12 ? distinct - 12 : 0) + apart);
+      if (best_cost == 0.0 || cost < best_cost) {
+        best_cost = cost;
+        best = make_xcd_sched(nbj, nai, S, xg, 8 / xg, 1, xcd_block(S));
+      }
+    }
+  }
+  return best;
+}
 
 // ---------------------------------------------------------------------------------------
 // Main loop pieces
@@ -180,7 +265,8 @@ __global__ __launch_bounds__(NTHREADS) void gemm_nt_generic(GemmArgs g, Sched sc
   __shared__ __attribute__((aligned(16))) u16 lds[2 * 2 * OPER];
   int bj, split, ai_begin, ai_end;
   if (gemm_skipped(g)) return;
-  if (!sched_decode(sc, blockIdx.x, bj, split, ai_begin, ai_end)) return;
+  int z = 0;
+  if (!sched_decode(sc, blockIdx.x, bj, split, ai_begin, ai_end, z)) return;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wa = wave >> 1, wb = wave & 1;
@@ -1010,22 +1096,24 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
   static_assert(NA == 8 || (NA == 7 && A_KM), "narrow A tiles need a k-major A");
   constexpr int TM = NA * 32;  // A rows (output index i) per tile
   int bj, split, ai_begin, ai_end;
-  int wg = blockIdx.x, nk = g.K / BK;
-  if (g.ksplit > 1) {
+  int wg = blockIdx.x, nk = g.K / BK, z = 0;
+  if (gemm_skipped(g)) return;
+  if (g.ksplit > 1 && sc.xg == 0) {
     const int per_copy = gridDim.x / g.ksplit;  // a multiple of 8 super-blocks
-    const int z = wg / per_copy;
+    z = wg / per_copy;
     wg -= z * per_copy;
     wg = (wg & ~7) | ((wg - z * sc.n_sb) & 7);  // copies start on different XCDs
+  }
+  if (!sched_decode(sc, wg, bj, split, ai_begin, ai_end, z)) return;
+  if (g.ksplit > 1) {
     const int kt0 = z * g.kt_per_split;
     nk -= kt0;
     nk = nk < g.kt_per_split ? nk : g.kt_per_split;
+    if (nk <= 0) return;
     g.A += A_KM ? (int64_t)kt0 * BK * g.lda : (int64_t)kt0 * BK;
     g.B += B_KM ? (int64_t)kt0 * BK * g.ldb : (int64_t)kt0 * BK;
     Epi::split_output(ep, (int64_t)z * g.zstride);
-    if (nk <= 0) return;
   }
-  if (gemm_skipped(g)) return;
-  if (!sched_decode(sc, wg, bj, split, ai_begin, ai_end)) return;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1268,9 +1356,15 @@ DEVI float group_sum(float v) {
 // already covered): far below every real logit, finite so that 0 * it stays 0 in the entropy sum.
 constexpr float MASKED_LOGIT = -1e30f;
 
+// EDGE: the A tile may reach past the vocabulary. Either instance takes a ragged last B tile: a
+// wave whose 128 tokens all lie past the end leaves at once, and one that has any stores
+// all 128 rows, those past the end being rows [T, round_up(T, 128)) of the saved buffer (cleared
+// before anything reads them). Row predicates on the stores instead cost 4 to 7 % of the sweep, and
+// a launch of its own for the ragged tile kept 1 / S of the chip busy for the length of a sweep.
 template <bool EDGE, bool AFFINE, bool MOMENTS, bool SAVE>
 struct Fwd16 {
   static constexpr int NA = 8;
+  static constexpr bool RAGGED_B = true;
   typedef FwdParams Params;
   // SAVE: s and q are relative to the row reference of the saved exponentials (fixed for the whole
   // sweep: nothing is rescaled); otherwise relative to the running maximum m.
@@ -1293,6 +1387,7 @@ struct Fwd16 {
   // last tile of a ragged vocabulary overlaps its predecessor); entries below it take no part.
   static DEVI void tile(State& st, const Params& p, int v0, int t0, int lane, u16* stage, int v_new) {
     if (v_new >= v0 + 128) return;    // every row of this wave's sub-tile is a repeat
+    if (t0 >= p.T) return;            // no token
     const bool overlap = v_new > v0;  // wave-uniform
     const int vl = v0 + 4 * (lane >> 4);
     const int group = lane >> 4;
@@ -1302,11 +1397,12 @@ struct Fwd16 {
     float rr[SAVE ? 8 : 1];
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      const int t = t0 + b * 16 + (lane & 15);
-      const bool live = !EDGE || t < p.T;
-      const int64_t l = live ? p.labels[t] : -1;
+      // (a token past the end reads the last one's: a predicate per load would have each waited for in turn)
+      int t = t0 + b * 16 + (lane & 15);
+      t = t < p.T ? t : p.T - 1;
+      const int64_t l = p.labels[t];
       lab[b] = (l >= v_new && l < p.V) ? (int)l : -1;
-      if (SAVE) rr[b] = live ? p.probs_ref[t] : 0.f;
+      if (SAVE) rr[b] = p.probs_ref[t];
     }
     ML16_AGPR_FENCE();
     for_each_col([&](auto bc) {
@@ -1395,8 +1491,7 @@ struct Fwd16 {
         if (!EDGE && !overlap)
           flush_stage16<false, true>(stage, out, p.ldv, 16, 128, 0, lane);
         else
-          flush_stage16<true, true>(stage, out, p.ldv, EDGE ? p.T - (t0 + b * 16) : 16, (int)p.ldv - v0,
-                                    overlap ? v_new - v0 : 0, lane);
+          flush_stage16<true, true>(stage, out, p.ldv, 16, (int)p.ldv - v0, overlap ? v_new - v0 : 0, lane);
       }
       // the label's logit, if it is one of this lane's 32 entries
       float xl = 0.f;
@@ -1456,7 +1551,7 @@ struct Fwd16 {
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int t = t0 + ((lane >> 4) + 4 * k) * 16 + (lane & 15);
-      if (EDGE && t >= p.T) continue;
+      if (t >= p.T) continue;
       float* w = p.ws + (int64_t)slot * p.T + t;
       w[0 * PT] = st.m[k]; w[1 * PT] = st.s[k]; w[2 * PT] = st.q[k]; w[3 * PT] = st.xl[k];
       w[4 * PT] = st.mn[k];
@@ -1477,6 +1572,7 @@ template <bool E> using Fwd16AffineMomSave = Fwd16<E, true, true, true>;
 template <bool EDGE, bool AFFINE>
 struct Bwd16 {
   static constexpr int NA = 8;
+  static constexpr bool RAGGED_B = EDGE;
   typedef BwdParams Params;
   struct State {
     float nb[8], gs[8];
@@ -1560,12 +1656,7 @@ enum { KERNEL_GENERIC = 0, KERNEL16_NT = 4, KERNEL16_TN = 5, KERNEL16_MIX = 6 };
 bool k16_ok(int64_t K) { return K >= 2 * BK && K % BK == 0; }
 
 template <class Epi, int KERNEL>
-int launch_region(const GemmArgs& g, int bj0, int nbj, int ai0, int nai, int S,
-                  const typename Epi::Params& ep, hipStream_t stream) {
-  if (nbj <= 0 || nai <= 0) return AREAL_OK;
-  if (S > nai) S = nai;
-  if (S < 1) S = 1;
-  const Sched sc = make_sched(bj0, nbj, ai0, nai, S, g.sb_wgs == 8 ? 8 : 32);
+int launch_sched(const GemmArgs& g, const Sched& sc, const typename Epi::Params& ep, hipStream_t stream) {
   if constexpr (KERNEL >= KERNEL16_NT) {
     constexpr int VAR = KERNEL == KERNEL16_NT ? VAR_NT : KERNEL == KERNEL16_TN ? VAR_TN : VAR_MIX;
     // the loader addresses a tile as a 64-bit base plus 32-bit byte offsets per lane
@@ -1575,8 +1666,8 @@ int launch_region(const GemmArgs& g, int bj0, int nbj, int ai0, int nai, int S,
     if (!k16_ok(g.K) || (g.ksplit > 1 && (g.kt_per_split < 2 || g.K / BK - (g.ksplit - 1) * g.kt_per_split < 2)))
       return AREAL_ERR_UNSUPPORTED;
     // a k-major A operand carries its tile column in the lane offsets: one A tile per workgroup
-    if (VAR != VAR_NT && S != nai) return AREAL_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((gemm16_sweep<VAR, Epi>), dim3(sched_grid(sc) * (g.ksplit > 1 ? g.ksplit : 1)),
+    if (VAR != VAR_NT && sc.S < ceil_div_i64(sc.nai, sc.xg > 0 ? sc.xg : 1)) return AREAL_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL((gemm16_sweep<VAR, Epi>), dim3(sched_grid(sc) * (g.ksplit > 1 && sc.xg == 0 ? g.ksplit : 1)),
                        dim3(NTHREADS), 0, stream, g, sc, ep);
   } else {
     if (g.ksplit > 1) return AREAL_ERR_UNSUPPORTED;
@@ -1587,15 +1678,26 @@ int launch_region(const GemmArgs& g, int bj0, int nbj, int ai0, int nai, int S,
   return AREAL_OK;
 }
 
+template <class Epi, int KERNEL>
+int launch_region(const GemmArgs& g, int bj0, int nbj, int ai0, int nai, int S,
+                  const typename Epi::Params& ep, hipStream_t stream) {
+  if (nbj <= 0 || nai <= 0) return AREAL_OK;
+  if (S > nai) S = nai;
+  if (S < 1) S = 1;
+  return launch_sched<Epi, KERNEL>(g, make_sched(bj0, nbj, ai0, nai, S, g.sb_wgs == 8 ? 8 : 32), ep, stream);
+}
+
 // How a GEMM is cut into launches. The hand-scheduled kernel (k16: K a multiple of 64, at least
-// 128, and the caller's epilogue and operand layout allow it) runs the interior tiles with the
-// predicate-free epilogue, then the ragged last B tile and the ragged last A tile with the EDGE
-// epilogue. Everything else is one launch of the generic kernel over all tiles.
+// 128, and the caller's epilogue and operand layout allow it) sweeps the full A tiles in one launch
+// (a ragged last one folded into it, or behind it with the EDGE epilogue); stores run one launch.
+// Everything else is one launch of the generic kernel over all tiles.
 struct Regions {
   bool k16;
   int nai_full, nbj_full;  // tiles entirely inside M and N (k16), else all tiles
   bool ragged_a, ragged_b;
-  int S;                   // splits used for the interior and the ragged-B launch
+  int S;                   // splits of the A range (a k16 sweep: those of `sweep`, all XCDs)
+  const Sched* layout;     // k16 stores: layout of the launch if not the default super-blocks
+  Sched sweep;             // k16 sweeps: layout of the main launch, see plan_sweep_regions
   bool fold_a;             // the ragged last A tile runs as rows [M - 256, M) at the end of the last
                            // split's sweep (GemmArgs::overlap_last_a) instead of a launch of its own;
                            // set by fold_ragged_a() for the epilogues that support it
@@ -1610,6 +1712,7 @@ Regions plan_regions(int64_t M, int64_t N, int64_t K, int target_wgs, int S_fixe
   Regions r;
   r.k16 = allow16 && k16_ok(K);
   r.fold_a = false;
+  r.layout = nullptr;
   if (r.k16) {
     r.nai_full = (int)(M / TILE); r.nbj_full = (int)(N / TILE);
     r.ragged_a = (M % TILE) != 0; r.ragged_b = (N % TILE) != 0;
@@ -1623,40 +1726,50 @@ Regions plan_regions(int64_t M, int64_t N, int64_t K, int target_wgs, int S_fixe
   return r;
 }
 
+// The regions of a sweep (forward, recompute).
+Regions plan_sweep_regions(int64_t M, int64_t N, int64_t K, bool allow16 = true) {
+  Regions r = plan_regions(M, N, K, 512, 0, allow16);
+  fold_ragged_a(r, M);
+  if (r.k16 && r.nai_full > 0) {
+    r.sweep = plan_sweep(r.nbj_full + (r.ragged_b ? 1 : 0), r.nai_full + (r.fold_a ? 1 : 0), (int)(K / BK));
+    r.S = r.sweep.xg * r.sweep.S;
+  }
+  return r;
+}
+
 // Epi16<EDGE> is the epilogue written for the hand-scheduled kernel's accumulator layout, Epi32<EDGE>
 // the same arithmetic for the generic kernel's; ep_edge_a is the parameter block of the ragged-A
 // launch (it may differ from ep in where it writes its partial results).
-// MERGE_EDGES: epilogues whose bounds predicates are cheap (plain stores) run ONE launch of the
-// EDGE = true instance over all tiles when any tile is ragged: a separate launch for the last
-// row of tiles has too few workgroups to fill the chip and each walks the whole K range.
-template <template <bool> class Epi16, template <bool> class Epi32, class P, int KERNEL16, bool MERGE_EDGES = false>
+// SWEEP: r comes from plan_sweep_regions. Otherwise the epilogue is a plain store, whose bounds
+// predicates are cheap: ONE launch of the EDGE = true instance over all tiles when any tile is ragged
+// (a separate launch for the last row of tiles has too few workgroups to fill the chip and each
+// walks the whole K range).
+template <template <bool> class Epi16, template <bool> class Epi32, class P, int KERNEL16, bool SWEEP>
 int launch_gemm(const GemmArgs& g, const Regions& r, const P& ep, const P& ep_edge_a,
                 hipStream_t stream) {
-  int rc;
   if (!r.k16) {
     if constexpr (KERNEL16 != KERNEL16_NT) return AREAL_ERR_UNSUPPORTED;  // the generic kernel reads k-contiguous operands
     return launch_region<Epi32<true>, KERNEL_GENERIC>(g, 0, r.nbj_full, 0, r.nai_full, r.S, ep, stream);
   }
-  if (MERGE_EDGES && (r.ragged_a || r.ragged_b)) {
+  const int nbj = r.nbj_full + (r.ragged_b ? 1 : 0);
+  if constexpr (!SWEEP) {
     const int nai = r.nai_full + (r.ragged_a ? 1 : 0);
-    return launch_region<Epi16<true>, KERNEL16>(g, 0, r.nbj_full + (r.ragged_b ? 1 : 0), 0, nai,
-                                                r.S == r.nai_full ? nai : r.S, ep, stream);
+    const Sched sc = r.layout != nullptr ? *r.layout : make_sched(0, nbj, 0, nai, nai, g.sb_wgs == 8 ? 8 : 32);
+    return r.ragged_a || r.ragged_b ? launch_sched<Epi16<true>, KERNEL16>(g, sc, ep, stream)
+                                    : launch_sched<Epi16<false>, KERNEL16>(g, sc, ep, stream);
+  } else {
+    GemmArgs gm = g;
+    gm.overlap_last_a = r.fold_a ? 1 : 0;
+    int rc;
+    if (r.nai_full > 0) {
+      rc = r.ragged_b && !Epi16<false>::RAGGED_B ? launch_sched<Epi16<true>, KERNEL16>(gm, r.sweep, ep, stream)
+                                                 : launch_sched<Epi16<false>, KERNEL16>(gm, r.sweep, ep, stream);
+      if (rc != AREAL_OK) return rc;
+    }
+    if (r.ragged_a && !r.fold_a)
+      return launch_region<Epi16<true>, KERNEL16>(g, 0, nbj, r.nai_full, 1, 1, ep_edge_a, stream);
+    return AREAL_OK;
   }
-  GemmArgs gm = g;
-  int nai_main = r.nai_full;
-  if constexpr (KERNEL16 == KERNEL16_NT) {
-    if (r.fold_a) { gm.overlap_last_a = 1; ++nai_main; }
-  }
-  if ((rc = launch_region<Epi16<false>, KERNEL16>(gm, 0, r.nbj_full, 0, nai_main, r.S, ep, stream)) != AREAL_OK)
-    return rc;
-  if (r.ragged_b &&
-      (rc = launch_region<Epi16<true>, KERNEL16>(gm, r.nbj_full, 1, 0, nai_main, r.S, ep, stream)) != AREAL_OK)
-    return rc;
-  if (r.ragged_a && nai_main == r.nai_full &&
-      (rc = launch_region<Epi16<true>, KERNEL16>(g, 0, r.nbj_full + (r.ragged_b ? 1 : 0), r.nai_full, 1, 1,
-                                                 ep_edge_a, stream)) != AREAL_OK)
-    return rc;
-  return AREAL_OK;
 }
 
 int check_operand(const void* p, int64_t ld) {
@@ -1681,27 +1794,31 @@ bool narrow_a_tiles(int64_t M) {
   const int64_t n = ceil_div_i64(M, TILE);
   return M % TILE != 0 && M <= n * (TILE - 32);
 }
+// layout: of the hand-scheduled kernel's tiles (null: super-blocks).
 template <int KERNEL16>
-int launch_store(const GemmArgs& g, const StoreParams& ep, int mode, hipStream_t stream) {
+int launch_store(const GemmArgs& g, const StoreParams& ep, int mode, hipStream_t stream,
+                 const Sched* layout = nullptr) {
   bool allow16 = true;
   if (mode == 0 || mode == 3) allow16 = ep.ldo % 8 == 0 && aligned16(ep.out) && ep.M % 8 == 0;
-  const Regions r = plan_regions(ep.M, ep.N, g.K, 0, 1 << 20, allow16);
+  Regions r = plan_regions(ep.M, ep.N, g.K, 0, 1 << 20, allow16);
+  r.layout = layout;
   if constexpr (KERNEL16 != KERNEL16_NT) {
     // the modes the two backward contractions use: dWeight 0 - 2, dHidden 0, 1 and 3
     constexpr int UNUSED_MODE = KERNEL16 == KERNEL16_TN ? 3 : 2;
     if (r.k16 && mode != UNUSED_MODE && narrow_a_tiles(ep.M)) {
       const int nai = (int)ceil_div_i64(ep.M, TILE), nbj = (int)ceil_div_i64(ep.N, TILE);
-      if (mode == 0) return launch_region<Store16Narrow<0>, KERNEL16>(g, 0, nbj, 0, nai, nai, ep, stream);
-      if (mode == 1) return launch_region<Store16Narrow<1>, KERNEL16>(g, 0, nbj, 0, nai, nai, ep, stream);
+      const Sched sc = layout != nullptr ? *layout : make_sched(0, nbj, 0, nai, nai, g.sb_wgs == 8 ? 8 : 32);
+      if (mode == 0) return launch_sched<Store16Narrow<0>, KERNEL16>(g, sc, ep, stream);
+      if (mode == 1) return launch_sched<Store16Narrow<1>, KERNEL16>(g, sc, ep, stream);
       constexpr int LAST_MODE = KERNEL16 == KERNEL16_TN ? 2 : 3;
-      return launch_region<Store16Narrow<LAST_MODE>, KERNEL16>(g, 0, nbj, 0, nai, nai, ep, stream);
+      return launch_sched<Store16Narrow<LAST_MODE>, KERNEL16>(g, sc, ep, stream);
     }
   }
   switch (mode) {
-    case 0: return launch_gemm<Store16Bf16, StoreBf16, StoreParams, KERNEL16, true>(g, r, ep, ep, stream);
-    case 1: return launch_gemm<Store16F32, StoreF32, StoreParams, KERNEL16, true>(g, r, ep, ep, stream);
-    case 2: return launch_gemm<Accum16F32, AccumF32, StoreParams, KERNEL16, true>(g, r, ep, ep, stream);
-    default: return launch_gemm<Store16Bf16Scaled, StoreBf16Scaled, StoreParams, KERNEL16, true>(g, r, ep, ep, stream);
+    case 0: return launch_gemm<Store16Bf16, StoreBf16, StoreParams, KERNEL16, false>(g, r, ep, ep, stream);
+    case 1: return launch_gemm<Store16F32, StoreF32, StoreParams, KERNEL16, false>(g, r, ep, ep, stream);
+    case 2: return launch_gemm<Accum16F32, AccumF32, StoreParams, KERNEL16, false>(g, r, ep, ep, stream);
+    default: return launch_gemm<Store16Bf16Scaled, StoreBf16Scaled, StoreParams, KERNEL16, false>(g, r, ep, ep, stream);
   }
 }
 
@@ -1710,19 +1827,23 @@ int launch_store(const GemmArgs& g, const StoreParams& ep, int mode, hipStream_t
 // over copies of the schedule, each writing an fp32 partial result that
 // splitk_reduce_bf16_kernel sums.
 // The launch is a schedule of super-blocks of up to 32 workgroups; super-block sb of copy c
-// runs on XCD (sb + c * n_sb) % 8, whose 32 CUs take its workgroups as they free up. Cost of
-// z copies in units of one workgroup's full K range = the busiest XCD's rounds of 32
-// workgroups, each K / z long, plus a small charge per split for the reduction of the partial
-// results.
+// runs on XCD (sb + c * n_sb) % 8, whose 32 CUs take its workgroups as they free up.
+// sched_load: the workgroups of one copy per XCD.
+void sched_load(const Sched& sc, int64_t (&load)[8]) {
+  for (int sb = 0; sb < sc.n_sb; ++sb) {
+    const int sbj = sb % sc.n_sb_j, sbs = sb / sc.n_sb_j;
+    const int nb = sc.nbj - sbj * sc.RB < sc.RB ? sc.nbj - sbj * sc.RB : sc.RB;
+    const int ns = sc.S - sbs * sc.RS < sc.RS ? sc.S - sbs * sc.RS : sc.RS;
+    load[sb & 7] += (int64_t)(nb > 0 ? nb : 0) * (ns > 0 ? ns : 0);
+  }
+}
+// Cost of z copies in units of one workgroup's full K range = the busiest XCD's rounds of 32
+// workgroups, each K / z long, plus a small charge per split for the reduction of the partial results.
 double sched_cost(const Sched& sc, int z) {
-  int64_t load[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  int64_t one[8] = {0}, load[8] = {0};
+  sched_load(sc, one);
   for (int c = 0; c < z; ++c)
-    for (int sb = 0; sb < sc.n_sb; ++sb) {
-      const int sbj = sb % sc.n_sb_j, sbs = sb / sc.n_sb_j;
-      const int nb = sc.nbj - sbj * sc.RB < sc.RB ? sc.nbj - sbj * sc.RB : sc.RB;
-      const int ns = sc.S - sbs * sc.RS < sc.RS ? sc.S - sbs * sc.RS : sc.RS;
-      load[(sb + c * sc.n_sb) & 7] += (int64_t)(nb > 0 ? nb : 0) * (ns > 0 ? ns : 0);
-    }
+    for (int x = 0; x < 8; ++x) load[x] += one[(x - c * sc.n_sb) & 7];
   int64_t worst = 0;
   for (int x = 0; x < 8; ++x) worst = load[x] > worst ? load[x] : worst;
   return (double)ceil_div_i64(worst, 32) / z + 0.03 * (z - 1);
@@ -1740,22 +1861,45 @@ void split_ktiles(int nk, int& z, int& kps) {
   }
 }
 
-int dh_ksplit(int64_t H, int64_t T, int64_t K) {
-  const int64_t tiles = ceil_div_i64(H, TILE) * ceil_div_i64(T, TILE);
-  if (tiles >= 2048 || K % BK != 0) return 1;
-  const int64_t nk = K / BK;
+// Layout and copies of the dHidden launch by estimated microseconds of the busiest XCD: a k-tile takes
+// 1.15 us while 32 neighbouring workgroups read at most about 14 distinct tiles, and proportionally
+// longer beyond (the 128-byte row pieces of e come from outside L2 at about 3 TB/s), a workgroup's
+// start and its epilogue 8 us, the reduction of the partial results 5 us and their bytes (written
+// and read) at 4.5 TB/s. Few output tiles then go to all XCDs (kg > 1), each with its own k range.
+// z_fixed > 0: the number of copies is given (of a token chunk: that of the whole batch, so that
+// the chunking does not change the order of the sums).
+struct DhPlan { int z; Sched sc; };
+DhPlan plan_dh(int64_t H, int64_t T, int64_t K, int z_fixed = 0) {
   const int nai = (int)ceil_div_i64(H, TILE), nbj = (int)ceil_div_i64(T, TILE);
-  const Sched sc = make_sched(0, nbj, 0, nai, nai);
-  int best = 1;
-  double best_cost = sched_cost(sc, 1);
-  for (int z = 2; z <= 16 && z <= nk / 8; ++z) {
-    const double cost = sched_cost(sc, z);
-    if (cost < best_cost - 1e-9) { best_cost = cost; best = z; }
-  }
+  DhPlan best{z_fixed > 0 ? z_fixed : 1, make_sched(0, nbj, 0, nai, nai)};
+  if (K % BK != 0) return best;
+  const int64_t nk = K / BK;
+  double best_cost = 0.0;
+  for (int xg = 1; xg <= 8; xg <<= 1)
+    for (int bg = 8 / xg; bg >= 1; bg >>= 1) {
+      if (xg > nai || bg > nbj) continue;
+      const int kg = 8 / (xg * bg), na = (int)ceil_div_i64(nai, xg), nb = (int)ceil_div_i64(nbj, bg);
+      const int tiles = na * nb;
+      for (int zk = 1; zk <= 16 && (kg * zk == 1 || kg * zk <= nk / 8); ++zk) {
+        const int z = kg * zk;
+        if (z_fixed > 0 && z != z_fixed) continue;
+        const int copies = tiles >= 32 ? 1 : (int)ceil_div_i64(32, tiles);
+        double distinct = tiles >= 32 ? xcd_distinct(nb, na) : (double)(copies < zk ? copies : zk) * (na + nb);
+        const double slow = distinct > 14.0 ? distinct / 14.0 : 1.0;
+        const double rounds = (double)ceil_div_i64((int64_t)tiles * zk, 32);
+        double cost = rounds * (1.15 * slow * (double)nk / z + 8.0);
+        if (z > 1) cost += 5.0 + (double)z * (double)(T * H) * 8.0 / 4.5e6;
+        if (best_cost == 0.0 || cost < best_cost - 1e-9) {
+          best_cost = cost;
+          best = DhPlan{z, make_xcd_sched(nbj, nai, na, xg, bg, zk, xcd_block(na))};
+        }
+        if (tiles >= 1024 && z_fixed == 0) break;  // the chip is full without copies: not worth trying
+      }
+    }
   return best;
 }
-size_t dh_partial_bytes(int64_t H, int64_t T, int64_t K) {
-  const int z = dh_ksplit(H, T, K);
+size_t dh_partial_bytes(int64_t H, int64_t T, int64_t K, int z_fixed = 0) {
+  const int z = z_fixed > 0 ? z_fixed : plan_dh(H, T, K).z;
   return z > 1 ? (size_t)z * (size_t)(T * H) * sizeof(float) + 256 : 0;
 }
 
@@ -1769,20 +1913,21 @@ bool dh_weight_in_place(int64_t V) { return V % BK == 0 && V >= 2 * BK; }
 // dh_weight_in_place(V), else its transposed copy W^T [H, ldv].
 template <int KERNEL16>
 int launch_dhidden_k(const GemmArgs& g0, int64_t H, int64_t T, int64_t ldv, void* dhidden,
-                     float* partial, const float* tscale, hipStream_t stream) {
+                     float* partial, const float* tscale, int z_fixed, hipStream_t stream) {
   GemmArgs g = g0;
-  int z = dh_ksplit(H, T, ldv);
+  const DhPlan plan = plan_dh(H, T, ldv, z_fixed);
+  int z = plan.z;
   int kps = 0;
   if (z > 1) split_ktiles((int)(ldv / BK), z, kps);
   if (z <= 1 || partial == nullptr) {
     const StoreParams ep{dhidden, H, (int)H, (int)T, tscale};
-    return launch_store<KERNEL16>(g, ep, tscale != nullptr ? 3 : 0, stream);
+    return launch_store<KERNEL16>(g, ep, tscale != nullptr ? 3 : 0, stream, z <= 1 ? &plan.sc : nullptr);
   }
   g.ksplit = z;
   g.kt_per_split = kps;
   g.zstride = T * H * (int64_t)sizeof(float);
   const StoreParams ep{partial, H, (int)H, (int)T, nullptr};
-  int rc = launch_store<KERNEL16>(g, ep, 1, stream);
+  int rc = launch_store<KERNEL16>(g, ep, 1, stream, &plan.sc);
   if (rc != AREAL_OK) return rc;
   int64_t blocks = ceil_div_i64(T * H, 256 * 4);
   if (blocks > 65535) blocks = 65535;
@@ -1793,15 +1938,15 @@ int launch_dhidden_k(const GemmArgs& g0, int64_t H, int64_t T, int64_t ldv, void
 }
 int launch_dhidden(const u16* w, int64_t V, const u16* dl, int64_t ldv, int64_t H, int64_t T,
                    void* dhidden, float* partial, const float* tscale, const int* skip_if_set,
-                   hipStream_t stream) {
+                   int z_fixed, hipStream_t stream) {
   if (dh_weight_in_place(V)) {
     GemmArgs g{w, H, (int)H, dl, ldv, (int)T, (int)ldv, (int)H, 0};
     g.skip_if_set = skip_if_set;
-    return launch_dhidden_k<KERNEL16_MIX>(g, H, T, ldv, dhidden, partial, tscale, stream);
+    return launch_dhidden_k<KERNEL16_MIX>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream);
   }
   GemmArgs g{w, ldv, (int)H, dl, ldv, (int)T, (int)ldv, 0, 0};
   g.skip_if_set = skip_if_set;
-  return launch_dhidden_k<KERNEL16_NT>(g, H, T, ldv, dhidden, partial, tscale, stream);
+  return launch_dhidden_k<KERNEL16_NT>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream);
 }
 
 // dWeight [V, H] in bf16 has ceil(V / 256) x ceil(H / 256) output tiles, one per workgroup, in
@@ -1925,9 +2070,7 @@ size_t areal_lmhead_probs_bytes(int64_t T, int64_t V) {
 }
 
 static Regions fwd_regions(int64_t T, int64_t H, int64_t V) {
-  Regions r = plan_regions(V, T, H, 512, 0);
-  fold_ragged_a(r, V);
-  return r;
+  return plan_sweep_regions(V, T, H);
 }
 
 size_t areal_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V) {
@@ -1941,8 +2084,8 @@ size_t areal_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V) {
 // only when one of them is requested.
 //
 // probs / probs_ref / probs_status (all null or all set) keep the exponentials of the softmax
-// for areal_lmhead_bwd_saved: probs bf16 [round_up(T, 128)][round_up(V, 64)] (rows >= T are not
-// written) holds e = 2^(c2 x - probs_ref[t]); probs_ref fp32 [T] is a per-row reference taken
+// for areal_lmhead_bwd_saved: probs bf16 [round_up(T, 128)][round_up(V, 64)] (rows >= T are left
+// undefined) holds e = 2^(c2 x - probs_ref[t]); probs_ref fp32 [T] is a per-row reference taken
 // from a few logits of the row before the sweep; *probs_status (one int) is set to 0 when every
 // row's exponentials are in range and to 1 when some row's maximum lies more than REF_WINDOW
 // binades above its estimate: then probs must not be used and the backward has to recompute
@@ -1985,16 +2128,16 @@ int areal_lmhead_fwd(const void* hidden, const void* weight, const float* bias,
   }
   // (each launch_gemm names the epilogue for the hand-scheduled kernel and the one for the generic kernel)
   auto fwd_plain = [&](const GemmArgs& gg) {
-    if (!affine && !moments) return launch_gemm<Fwd16Plain, FwdPlain, FwdParams, KERNEL16_NT>(gg, r, ep, ep_a, stream);
-    if (!affine) return launch_gemm<Fwd16PlainMom, FwdPlainMom, FwdParams, KERNEL16_NT>(gg, r, ep, ep_a, stream);
-    if (!moments) return launch_gemm<Fwd16Affine, FwdAffine, FwdParams, KERNEL16_NT>(gg, r, ep, ep_a, stream);
-    return launch_gemm<Fwd16AffineMom, FwdAffineMom, FwdParams, KERNEL16_NT>(gg, r, ep, ep_a, stream);
+    if (!affine && !moments) return launch_gemm<Fwd16Plain, FwdPlain, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+    if (!affine) return launch_gemm<Fwd16PlainMom, FwdPlainMom, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+    if (!moments) return launch_gemm<Fwd16Affine, FwdAffine, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+    return launch_gemm<Fwd16AffineMom, FwdAffineMom, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
   };
   auto fwd_save = [&](const GemmArgs& gg) {
-    if (!affine && !moments) return launch_gemm<Fwd16PlainSave, FwdPlainSave, FwdParams, KERNEL16_NT>(gg, r, ep, ep_a, stream);
-    if (!affine) return launch_gemm<Fwd16PlainMomSave, FwdPlainMomSave, FwdParams, KERNEL16_NT>(gg, r, ep, ep_a, stream);
-    if (!moments) return launch_gemm<Fwd16AffineSave, FwdAffineSave, FwdParams, KERNEL16_NT>(gg, r, ep, ep_a, stream);
-    return launch_gemm<Fwd16AffineMomSave, FwdAffineMomSave, FwdParams, KERNEL16_NT>(gg, r, ep, ep_a, stream);
+    if (!affine && !moments) return launch_gemm<Fwd16PlainSave, FwdPlainSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+    if (!affine) return launch_gemm<Fwd16PlainMomSave, FwdPlainMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+    if (!moments) return launch_gemm<Fwd16AffineSave, FwdAffineSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+    return launch_gemm<Fwd16AffineMomSave, FwdAffineMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
   };
   auto merge = [&](int ref_sums, const float* ref, const int* gate, int gate_run_if_set) {
     hipLaunchKernelGGL(lmhead_merge_kernel, dim3((unsigned)ceil_div_i64(T, 64)), dim3(64 * MERGE_WAVES),
@@ -2041,7 +2184,7 @@ size_t areal_lmhead_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t
   if (ragged) elems += H * ldt + V * ldt;
   // slack for 256-byte sub-buffer alignment
   // (the last term: partial results of the bf16 dWeight store, one chunk covering the batch)
-  return (size_t)elems * 2 + dh_partial_bytes(H, Tc, ldv) + (Tc >= T ? dw_tail_bytes(H, V, Tc) : 0) + 6 * 256;
+  return (size_t)elems * 2 + dh_partial_bytes(H, Tc, ldv, plan_dh(H, T, ldv).z) + (Tc >= T ? dw_tail_bytes(H, V, Tc) : 0) + 6 * 256;
 }
 
 // Backward. grad_logprobs [T] fp32 = dLoss/dlogprobs. Writes dhidden [T,H] bf16 and the weight
@@ -2088,7 +2231,8 @@ int areal_lmhead_bwd(const void* hidden, const void* weight, const float* bias,
   u16* dl = carve(wp, Tc_max * ldv * 2);
   u16* hT = ragged ? carve(wp, H * ldt * 2) : nullptr;
   u16* dlT = ragged ? carve(wp, V * ldt * 2) : nullptr;
-  float* dh_part = dh_partial_bytes(H, Tc_max, ldv) ? (float*)carve(wp, dh_partial_bytes(H, Tc_max, ldv)) : nullptr;
+  const int dh_z = plan_dh(H, T, ldv).z;
+  float* dh_part = dh_z > 1 ? (float*)carve(wp, dh_partial_bytes(H, Tc_max, ldv, dh_z)) : nullptr;
   float* dw_part = (dw_bf16 && dw_tail_bytes(H, V, Tc_max)) ? (float*)carve(wp, dw_tail_bytes(H, V, Tc_max)) : nullptr;
 
   const float c2 = inv_temperature * LOG2E;
@@ -2114,20 +2258,19 @@ int areal_lmhead_bwd(const void* hidden, const void* weight, const float* bias,
       BwdParams ep{labels + t0, row_max + t0, sum_exp + t0, grad_logprobs + t0, (int)Tc,
                    (int)V, logit_scale, c2, inv_temperature, bias, dl, ldv, dlT, ldt_c};
       // the token-contiguous copy dlT is written by the generic kernel's epilogue only
-      Regions r = plan_regions(V, Tc, H, 512, 0, !need_dlT);
-      fold_ragged_a(r, V);
+      const Regions r = plan_sweep_regions(V, Tc, H, !need_dlT);
       if (need_dlT)
-        rc = affine ? launch_gemm<Bwd16Affine, BwdAffineT, BwdParams, KERNEL16_NT>(g, r, ep, ep, stream)
-                    : launch_gemm<Bwd16Plain, BwdPlainT, BwdParams, KERNEL16_NT>(g, r, ep, ep, stream);
+        rc = affine ? launch_gemm<Bwd16Affine, BwdAffineT, BwdParams, KERNEL16_NT, true>(g, r, ep, ep, stream)
+                    : launch_gemm<Bwd16Plain, BwdPlainT, BwdParams, KERNEL16_NT, true>(g, r, ep, ep, stream);
       else
-        rc = affine ? launch_gemm<Bwd16Affine, BwdAffine, BwdParams, KERNEL16_NT>(g, r, ep, ep, stream)
-                    : launch_gemm<Bwd16Plain, BwdPlain, BwdParams, KERNEL16_NT>(g, r, ep, ep, stream);
+        rc = affine ? launch_gemm<Bwd16Affine, BwdAffine, BwdParams, KERNEL16_NT, true>(g, r, ep, ep, stream)
+                    : launch_gemm<Bwd16Plain, BwdPlain, BwdParams, KERNEL16_NT, true>(g, r, ep, ep, stream);
       if (rc != AREAL_OK) return rc;
     }
     // 2. dHidden[t, h] = sum_v dl[t, v] * W^T[h, v]
     if (dhidden != nullptr) {
       if ((rc = launch_dhidden(w_in_place ? (const u16*)weight : wT, V, dl, ldv, H, Tc,
-                               (u16*)dhidden + t0 * H, dh_part, nullptr, nullptr, stream)) != AREAL_OK)
+                               (u16*)dhidden + t0 * H, dh_part, nullptr, nullptr, dh_z, stream)) != AREAL_OK)
         return rc;
     }
     // dBias[v] += sum_t dl[t, v]
@@ -2225,7 +2368,7 @@ int areal_lmhead_bwd_saved(const void* hidden, const void* weight, const int64_t
       AREAL_CHECK_LAUNCH();
     }
     if ((rc = launch_dhidden(w_in_place ? (const u16*)weight : wT, V, e, ldv, H, T, dhidden, dh_part,
-                             rowfac, probs_status, stream)) != AREAL_OK)
+                             rowfac, probs_status, 0, stream)) != AREAL_OK)
       return rc;
   }
   if (dbias != nullptr) {
