@@ -46,6 +46,10 @@ SIGNATURES: dict[str, tuple] = {
         I,
         [P, P, P, P, I64, I64, I64, F, F, P, P, P, P, P, P, P, P, P, SZ, P, P, P, SZ, P],
     ),
+    "areal_lmhead_fwd_ex": (
+        I,
+        [P, P, P, P, I64, I64, I64, F, F, P, P, P, P, P, P, P, P, P, SZ, P, P, P, P, P, SZ, P],
+    ),
     "areal_lmhead_bwd_workspace_bytes": (SZ, [I64, I64, I64, I64]),
     "areal_lmhead_bwd": (
         I,
@@ -72,6 +76,7 @@ SIGNATURES: dict[str, tuple] = {
         I,
         [P, P, P, P, P, P, I64, I64, I64, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, SZ, P],
     ),
+    "areal_actor_loss_call": (I, [P, P, P, SZ, P]),
     "areal_actor_loss_static": (
         I,
         [P, P, P, P, P, P, I64, I64, I64, P, P, P, P, P, P, P, P, P, P, P, P, P, P],
@@ -142,6 +147,7 @@ class LossConfig(ctypes.Structure):
     ]
 
 _lib = None
+_host = None
 
 
 ERR_UNSUPPORTED = -5  # AREAL_ERR_UNSUPPORTED
@@ -175,6 +181,22 @@ def load() -> ctypes.CDLL:
         )
     _lib = lib
     return lib
+
+
+def host():
+    """The native host path (``csrc/host.cpp``): allocation, launch and autograd node of a call."""
+    global _host
+    if _host is None:
+        load()  # checks the interface version of the library that _host.so links to
+        try:
+            from areal_amd import _host as module
+        except ImportError as e:
+            raise ArealHipError(
+                f"areal_amd/_host.so cannot be loaded ({e}): build it with `python -m areal_amd.build`"
+            ) from e
+        module.set_error_class(ArealHipError)
+        _host = module
+    return _host
 
 
 @functools.lru_cache(maxsize=1)

@@ -17,6 +17,7 @@ from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent / "csrc"
 LIB_PATH = Path(__file__).resolve().parent / "libareal_hip.so"
+HOST_PATH = Path(__file__).resolve().parent / "_host.so"  # csrc/host.cpp, imported as areal_amd._host
 
 # Packed fp32 VALU ops are switched off for every kernel: their results must not depend on
 # whether the compiler paired two scalar float operations.
@@ -42,6 +43,10 @@ def _hipcc() -> str:
     raise RuntimeError("hipcc not found; a ROCm toolchain is required to build areal_amd")
 
 
+def _rocm_home() -> str:
+    return str(Path(_hipcc()).resolve().parents[1]) if os.path.exists(_hipcc()) else "/opt/rocm"
+
+
 def sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
 
@@ -54,6 +59,39 @@ def _compile_one(src: Path, obj: Path) -> None:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{proc.stderr}")
+
+
+def _compile_host(obj: Path) -> None:
+    """``csrc/host.cpp`` against torch's headers (no device code in it)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    includes = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], _rocm_home() + "/include"]
+    cmd = [
+        shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        *[f"-I{p}" for p in includes], "-c", str(CSRC / "host.cpp"), "-o", str(obj),
+    ]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{proc.stderr}")
+
+
+def _link_host(obj: Path) -> None:
+    from torch.utils import cpp_extension
+
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    libs = [f"-l{n}" for n in ("c10", "torch_cpu", "torch", "torch_python", "c10_hip", "torch_hip")]
+    cmd = [
+        shutil.which("g++") or "g++", "-shared", str(obj), "-o", str(tmp), f"-L{LIB_PATH.parent}",
+        f"-l:{LIB_PATH.name}", *[f"-L{p}" for p in cpp_extension.library_paths()], *libs, "-Wl,-rpath,$ORIGIN",
+    ]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"link of _host.so failed:\n{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
 
 
 def generate_mainloop() -> Path:
@@ -109,6 +147,8 @@ def _up_to_date(src: Path, obj: Path) -> bool:
     if not obj.exists():
         return False
     deps = [src, CSRC / "common.hpp", Path(__file__)]
+    if src.name == "host.cpp":
+        deps = [src, CSRC.parents[1] / "include" / "areal_hip.h"]
     if src.name == "lmhead.hip":
         deps.append(CSRC / "mainloop16.inc")
     return all(obj.stat().st_mtime > d.stat().st_mtime for d in deps)
@@ -126,21 +166,26 @@ def build_all(verbose: bool = True, incremental: bool = False) -> Path:
         raise RuntimeError(f"no .hip sources under {CSRC}")
     objs = [build_dir / (s.stem + ".o") for s in srcs]
     todo = [(s, o) for s, o in zip(srcs, objs) if not (incremental and _up_to_date(s, o))]
+    host_obj = build_dir / "host.o"
+    todo_host = not (incremental and _up_to_date(CSRC / "host.cpp", host_obj))
     if verbose:
         print(f"[areal_amd.build] compiling {len(todo)} of {len(srcs)} HIP sources for gfx950", flush=True)
-    with ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as pool:
+    with ThreadPoolExecutor(max_workers=min(8, len(srcs) + 2)) as pool:
         check = None
+        host = pool.submit(_compile_host, host_obj) if todo_host else None
         if any(s.name == "lmhead.hip" for s, _ in todo):
             check = pool.submit(_check_lmhead, build_dir)
         list(pool.map(lambda so: _compile_one(*so), todo))
-        if check is not None:
-            check.result()
+        for extra in (check, host):
+            if extra is not None:
+                extra.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
     os.replace(tmp, LIB_PATH)
+    _link_host(host_obj)
     if verbose:
         print(f"[areal_amd.build] wrote {LIB_PATH}", flush=True)
     return LIB_PATH

@@ -1,0 +1,754 @@
+// Host path of the Python API: what a call does between its arguments and its kernel launches
+// (output and workspace allocation, the autograd node, the small results that travel back) in one
+// native call. A micro-batch's loss stage or a short lm_head step is bound by this work, not by its
+// kernels: the same sequence in Python (about twenty tensor calls, ctypes argument lists, a Python
+// autograd node) took 150 to 300 us of host time per call, this takes 10 to 30.
+//
+// Loaded as areal_amd._host; every kernel behind it is reached through the C ABI of
+// libareal_hip.so (include/areal_hip.h).
+#include <torch/extension.h>
+
+#include <torch/csrc/Exceptions.h>
+#include <ATen/core/CachingHostAllocator.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+
+#include <array>
+#include <atomic>
+#include <chrono>
+#include <cmath>
+#include <optional>
+#include <vector>
+
+#include "../../include/areal_hip.h"
+
+namespace {
+
+namespace py = pybind11;
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+PyObject* error_class = nullptr;  // areal_amd._lib.ArealHipError, set by the binding
+
+// Raises areal_amd._lib.ArealHipError, from any thread (the autograd engine's included).
+[[noreturn]] void fail(const std::string& message) {
+  py::gil_scoped_acquire gil;
+  PyErr_SetString(error_class != nullptr ? error_class : PyExc_RuntimeError, message.c_str());
+  python_error e;
+  e.persist();
+  throw e;
+}
+
+void check(int rc, const char* what) {
+  if (rc == AREAL_OK) return;
+  static const char* const names[] = {"ok", "bad argument", "pointer or leading dimension not suitably aligned",
+                                      "workspace too small", "kernel launch failed", "unsupported shape"};
+  const std::string name = rc <= 0 && rc >= -5 ? names[-rc] : std::to_string(rc);
+  fail(std::string(what) + " failed: " + name + " (code " + std::to_string(rc) + ")");
+}
+
+// All given tensors have to live on one HIP device.
+template <class... T>
+void require_gpu(const T&... ts) {
+  const Tensor* first = nullptr;
+  auto one = [&](const Tensor& t) {
+    if (!t.defined()) return;
+    if (!t.is_cuda())
+      fail("areal_amd kernels run on an MI355X only; got a tensor on " + t.device().str() +
+           " (there is no CPU fallback)");
+    if (first == nullptr) first = &t;
+    else if (t.device() != first->device())
+      fail("tensors on different devices: " + first->device().str() + " and " + t.device().str());
+  };
+  (one(ts), ...);
+  if (first == nullptr) fail("no tensor given");
+}
+
+Tensor or_undefined(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+
+areal_stream_t stream_of(const Tensor& t) {
+  return (areal_stream_t)c10::hip::getCurrentHIPStream(t.device().index()).stream();
+}
+
+Tensor empty(const Tensor& like, at::IntArrayRef shape, at::ScalarType type) {
+  return at::empty(shape, like.options().dtype(type).requires_grad(false));
+}
+Tensor empty_f32(const Tensor& like, int64_t n) { return empty(like, {n}, at::kFloat); }
+Tensor workspace(const Tensor& like, size_t bytes) {
+  return empty(like, {(int64_t)(bytes > 0 ? bytes : 1)}, at::kByte);
+}
+
+template <class T>
+T* ptr(const Tensor& t) { return t.defined() ? (T*)t.data_ptr() : nullptr; }
+
+// Flat fp32 / bool / int64 forms of an argument, as the kernels read it (no copy when it is already one).
+Tensor flat(const Tensor& t, at::ScalarType type) {
+  if (!t.defined()) return t;
+  Tensor d = t.requires_grad() ? t.detach() : t;
+  if (d.scalar_type() != type) d = type == at::kBool ? d.to(at::kBool) : d.to(type);
+  if (!d.is_contiguous()) d = d.contiguous();
+  return d.dim() == 1 ? d : d.view({-1});
+}
+
+// ---------------------------------------------------------------------------------------
+// Small results on their way to the host: the kernels write them into pinned host memory, which is
+// filled with a bit pattern no result has before they are launched. Waiting means looking at that
+// memory until the pattern is gone (about a microsecond after the kernel's store, where a copy
+// queued behind the kernel, its event and the synchronisation take about 15); after 200 us of that
+// the stream is synchronised instead. A result that nobody waits for keeps its memory out of the
+// pinned allocator's hands until the stream has passed the point of its destruction.
+// ---------------------------------------------------------------------------------------
+constexpr uint64_t PENDING = 0x7ff8a5c3d2e1f0b4ull;  // a NaN payload arithmetic does not make
+
+// Called from destructors: nothing may be thrown (a failure only means that the allocator is not told).
+void keep_until_passed(const Tensor& pinned, const c10::hip::HIPStream& stream) noexcept {
+  try {
+    at::getHostAllocator(at::kCUDA)->record_event(pinned.data_ptr(), pinned.storage().data_ptr().get_context(),
+                                                  c10::hip::HIPStreamMasqueradingAsCUDA(stream).unwrap());
+  } catch (...) {
+  }
+}
+
+struct HostResult {
+  Tensor host;  // fp64, pinned
+  c10::hip::HIPStream stream;
+  bool done = false;
+
+  HostResult(int64_t n, const Tensor& like)
+      : host(at::empty({n}, at::TensorOptions().dtype(at::kDouble).pinned_memory(true))),
+        stream(c10::hip::getCurrentHIPStream(like.device().index())) {
+    uint64_t* p = (uint64_t*)host.data_ptr();
+    for (int64_t i = 0; i < n; ++i) p[i] = PENDING;
+    std::atomic_thread_fence(std::memory_order_release);
+  }
+  ~HostResult() {
+    if (!done && !arrived()) keep_until_passed(host, stream);
+  }
+  double* data() { return (double*)host.data_ptr(); }
+  bool arrived() const {
+    const volatile uint64_t* p = (const volatile uint64_t*)host.data_ptr();
+    for (int64_t i = host.numel() - 1; i >= 0; --i)
+      if (p[i] == PENDING) return false;
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return true;
+  }
+  void wait() {
+    if (done) return;
+    py::gil_scoped_release no_gil;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    while (!arrived()) {
+      if (std::chrono::steady_clock::now() > until) {
+        stream.synchronize();
+        break;
+      }
+    }
+    done = true;
+  }
+  Tensor value() { wait(); return host; }
+  // {key: {sum, count, avg, min, max, denominator}} of rows `offset + 4 * row` of the result; avg, min and max
+  // are None under an empty denominator.
+  void fill(py::dict out, const std::vector<std::tuple<int, py::str, py::str>>& rows, int64_t offset) {
+    wait();
+    static PyObject *k_sum = PyUnicode_InternFromString("sum"), *k_count = PyUnicode_InternFromString("count"),
+                    *k_avg = PyUnicode_InternFromString("avg"), *k_min = PyUnicode_InternFromString("min"),
+                    *k_max = PyUnicode_InternFromString("max"),
+                    *k_den = PyUnicode_InternFromString("denominator");
+    const double* h = data() + offset;
+    auto set = [](py::dict& d, PyObject* k, const py::object& v) { PyDict_SetItem(d.ptr(), k, v.ptr()); };
+    for (const auto& [row, key, den] : rows) {
+      const double* r = h + 4 * row;
+      const bool empty = r[1] == 0.0;
+      py::dict d;
+      set(d, k_sum, py::float_(r[0]));
+      set(d, k_count, py::float_(r[1]));
+      set(d, k_avg, empty ? py::object(py::none()) : py::object(py::float_(r[0] / r[1])));
+      set(d, k_min, empty ? py::object(py::none()) : py::object(py::float_(r[2])));
+      set(d, k_max, empty ? py::object(py::none()) : py::object(py::float_(r[3])));
+      set(d, k_den, den);
+      PyDict_SetItem(out.ptr(), key.ptr(), d.ptr());
+    }
+  }
+};
+using HostResultPtr = std::shared_ptr<HostResult>;
+
+// ---------------------------------------------------------------------------------------
+// Scalar losses: a kernel has written the loss, d(loss sum)/dx per element and the token counts; the
+// node multiplies by upstream / count.
+// ---------------------------------------------------------------------------------------
+struct LossGraph {
+  Tensor loss, dsum, counters;
+};
+
+struct ScaledLoss : public torch::autograd::Function<ScaledLoss> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const LossGraph* g) {
+    ctx->save_for_backward({g->dsum, g->counters});
+    ctx->saved_data["shape"] = x.sizes().vec();
+    ctx->saved_data["type"] = (int64_t)x.scalar_type();
+    return g->loss;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &dsum = saved[0], &counters = saved[1];
+    const c10::hip::HIPGuard guard(dsum.device().index());
+    const Tensor up = flat(grads[0], at::kFloat);
+    Tensor out = at::empty_like(dsum);
+    check(areal_actor_loss_grad(ptr<float>(dsum), ptr<float>(up), ptr<double>(counters), ptr<float>(out),
+                                dsum.numel(), stream_of(dsum)),
+          "areal_actor_loss_grad");
+    out = out.view(ctx->saved_data["shape"].toIntVector());
+    const auto type = (at::ScalarType)ctx->saved_data["type"].toInt();
+    if (type != at::kFloat) out = out.to(type);
+    return {out, Tensor()};
+  }
+};
+
+Tensor attach(const Tensor& x, const Tensor& loss, const Tensor& dsum, const Tensor& counters) {
+  if (!dsum.defined()) return loss;
+  const LossGraph g{loss, dsum, counters};
+  return ScaledLoss::apply(x, &g);
+}
+bool wants_grad(const Tensor& x) { return x.requires_grad() && at::GradMode::is_enabled(); }
+
+// ---------------------------------------------------------------------------------------
+// PPO / CISPO actor loss (areal_actor_loss_call)
+// ---------------------------------------------------------------------------------------
+// What a call leaves behind besides the loss: nothing per token, the tensors of the reference's
+// `stat` dict, those and the further ones grpo_loss_fn logs, or reduced statistics.
+enum { OUT_NONE = 0, OUT_STAT = 1, OUT_LOGGED = 2, OUT_REDUCED = 3 };
+constexpr int N_STATS = 18;
+
+areal_loss_config loss_config(const std::array<double, 14>& v) {
+  areal_loss_config c;
+  c.loss_kind = (int)v[0]; c.clip_lo = (float)v[1]; c.clip_hi = (float)v[2]; c.has_c_clip = (int)v[3];
+  c.c_clip = (float)v[4]; c.seq_is = (int)v[5]; c.rs_enabled = (int)v[6]; c.rs_seq_level = (int)v[7];
+  c.rs_clamp = (int)v[8]; c.rs_metric = (int)v[9]; c.rs_agg = (int)v[10]; c.rs_upper = (float)v[11];
+  c.rs_has_lower = (int)v[12]; c.rs_lower = (float)v[13];
+  return c;
+}
+
+// (loss, {name: per-token tensor}, host result [9 (+ 18 * 4)]). keep_mask: also return the behave mask
+// in the modes that would not.
+py::tuple actor_loss(const Tensor& logprobs, const Tensor& proximal, const OptTensor& old_logprobs,
+                     const Tensor& advantages, const Tensor& loss_mask, const OptTensor& cu_seqlens,
+                     const std::array<double, 14>& config, int mode, bool keep_mask, bool nan_if_nonfinite,
+                     const OptTensor& entropy, const OptTensor& extra0, const OptTensor& extra1) {
+  const areal_loss_config cfg = loss_config(config);
+  const Tensor old_arg = or_undefined(old_logprobs);
+  require_gpu(proximal, loss_mask, logprobs, old_arg, advantages);
+  const c10::hip::HIPGuard guard(proximal.device().index());
+  const at::IntArrayRef shape = logprobs.sizes();
+  const Tensor lp = flat(logprobs, at::kFloat), prox = flat(proximal, at::kFloat),
+               old = flat(old_arg, at::kFloat), adv = flat(advantages, at::kFloat),
+               mask = flat(loss_mask, at::kBool);
+  const int64_t n = mask.numel();
+  const bool seq_is = cfg.loss_kind == 0 && cfg.seq_is, rs = cfg.rs_enabled != 0;
+  areal_actor_loss_io io{};
+  Tensor cu;
+  if ((rs && cfg.rs_seq_level) || seq_is) {
+    if (shape.size() == 2) {
+      io.n_seqs = shape[0];
+      io.uniform_len = shape[1];
+    } else {
+      cu = or_undefined(cu_seqlens).to(lp.device(), at::kInt).contiguous();
+      io.n_seqs = cu.numel() - 1;
+    }
+  }
+  const bool grad = wants_grad(logprobs), stats = mode == OUT_REDUCED;
+  const bool stat = mode == OUT_STAT || mode == OUT_LOGGED;
+  py::dict out;
+  auto f32 = [&](const char* name, bool want) {
+    if (!want) return (float*)nullptr;
+    const Tensor t = empty(lp, {n}, at::kFloat);
+    out[name] = shape.size() == 1 ? t : t.view(shape);
+    return ptr<float>(t);
+  };
+  auto u8 = [&](const char* name, bool want) {
+    if (!want) return (uint8_t*)nullptr;
+    const Tensor t = empty(lp, {n}, at::kBool);
+    out[name] = shape.size() == 1 ? t : t.view(shape);
+    return ptr<uint8_t>(t);
+  };
+  const Tensor ent = flat(or_undefined(entropy), at::kFloat), x0 = flat(or_undefined(extra0), at::kFloat),
+               x1 = flat(or_undefined(extra1), at::kFloat);
+  if (x0.defined() && x0.numel() != n)
+    throw py::value_error("extra statistic has " + std::to_string(x0.numel()) + " elements, expected " + std::to_string(n));
+  if (x1.defined() && x1.numel() != n)
+    throw py::value_error("extra statistic has " + std::to_string(x1.numel()) + " elements, expected " + std::to_string(n));
+  if (ent.defined() && ent.numel() != n)
+    throw py::value_error("entropy has " + std::to_string(ent.numel()) + " elements, expected " + std::to_string(n));
+  const Tensor loss = empty(lp, {}, at::kFloat);
+  const Tensor dlp = grad ? empty(lp, {n}, at::kFloat) : Tensor();
+  const int64_t n_results = 9 + (stats ? 4 * N_STATS : 0);
+  const Tensor results = empty(lp, {n_results}, at::kDouble);
+  auto host = std::make_shared<HostResult>(n_results, lp);
+  io.logprobs = ptr<float>(lp); io.proximal_logprobs = ptr<float>(prox); io.old_logprobs = ptr<float>(old);
+  io.advantages = ptr<float>(adv); io.loss_mask = ptr<uint8_t>(mask); io.cu_seqlens = ptr<int32_t>(cu);
+  io.entropy = ptr<float>(ent); io.extra0 = ptr<float>(x0); io.extra1 = ptr<float>(x1);
+  io.n_tokens = n;
+  io.loss = ptr<float>(loss); io.dlogprobs = ptr<float>(dlp);
+  io.stat_loss = f32("loss", stat);
+  io.stat_ratio = f32("importance_weight", stat);
+  io.stat_approx_kl = f32("approx_kl", stat);
+  io.clip_mask = u8("clip_mask", stat);
+  io.dual_clip_mask = u8("dual_clip_mask", stat);
+  // the per-sequence ratio aggregates over what rejection sampling left
+  io.new_mask = u8("new_mask", rs && seq_is);
+  io.behave_imp_weight = f32("behave_imp_weight", rs && (stat || seq_is));
+  io.behave_approx_kl = f32("behave_approx_kl", rs && stat);
+  io.behave_mask = u8("behave_mask", rs && (stat || keep_mask));
+  const bool logged = mode == OUT_LOGGED;
+  io.clip_ratio = f32("clip_ratio", logged);
+  io.dual_clip_ratio = f32("dual_clip_ratio", logged);
+  io.logp_diff = f32("logp_diff", logged);
+  io.logp_abs_diff = f32("logp_abs_diff", logged);
+  io.behave_filtered_ratio = f32("behave_filtered_ratio", logged && rs);
+  io.results = ptr<double>(results);
+  io.host_results = host->data();
+  io.with_stats = stats;
+  io.nan_if_nonfinite = nan_if_nonfinite;
+  const size_t bytes = stats ? areal_actor_loss_stats_workspace_bytes(n, io.n_seqs)
+                             : areal_actor_loss_workspace_bytes(n, io.n_seqs);
+  const Tensor ws = workspace(lp, bytes);
+  check(areal_actor_loss_call(&io, &cfg, ptr<void>(ws), bytes, stream_of(lp)), "areal_actor_loss_call");
+  return py::make_tuple(attach(logprobs, loss, dlp, results), out, host);
+}
+
+// Tokens whose proximal log-prob is not finite, and its statistics under the mask: a host result [9 + 18 * 4]
+// of which entry 8 and row 17 are set (for the losses whose own kernels do not read it).
+HostResultPtr proximal_stats(const Tensor& proximal, const Tensor& loss_mask) {
+  require_gpu(proximal, loss_mask);
+  const c10::hip::HIPGuard guard(proximal.device().index());
+  const Tensor prox = flat(proximal, at::kFloat), mask = flat(loss_mask, at::kBool);
+  areal_loss_config cfg{};
+  cfg.loss_kind = -1;
+  const Tensor results = empty(prox, {9 + 4 * N_STATS}, at::kDouble);
+  auto host = std::make_shared<HostResult>(9 + 4 * N_STATS, prox);
+  areal_actor_loss_io io{};
+  io.proximal_logprobs = ptr<float>(prox);
+  io.loss_mask = ptr<uint8_t>(mask);
+  io.n_tokens = mask.numel();
+  io.results = ptr<double>(results);
+  io.host_results = host->data();
+  io.with_stats = 1;
+  const size_t bytes = areal_actor_loss_stats_workspace_bytes(io.n_tokens, 0);
+  const Tensor ws = workspace(prox, bytes);
+  check(areal_actor_loss_call(&io, &cfg, ptr<void>(ws), bytes, stream_of(prox)), "areal_actor_loss_call");
+  return host;
+}
+
+// ---------------------------------------------------------------------------------------
+// SAPO and critic losses
+// ---------------------------------------------------------------------------------------
+constexpr int N_SAPO_STATS = 13;
+
+py::tuple sapo_loss(const Tensor& logprobs, const Tensor& old_logprobs, const Tensor& advantages,
+                    const Tensor& loss_mask, const OptTensor& cu_seqlens, double tau_pos, double tau_neg,
+                    bool seq_level, bool reduced, const OptTensor& entropy, const OptTensor& extra0,
+                    const OptTensor& extra1) {
+  require_gpu(logprobs, old_logprobs, advantages, loss_mask);
+  const c10::hip::HIPGuard guard(logprobs.device().index());
+  const at::IntArrayRef shape = logprobs.sizes();
+  const Tensor lp = flat(logprobs, at::kFloat), old = flat(old_logprobs, at::kFloat),
+               adv = flat(advantages, at::kFloat), mask = flat(loss_mask, at::kBool);
+  const int64_t n = mask.numel();
+  Tensor cu;
+  int64_t n_seqs = 0, uniform_len = 0;
+  if (seq_level) {
+    if (shape.size() == 2) {
+      n_seqs = shape[0];
+      uniform_len = shape[1];
+    } else {
+      cu = or_undefined(cu_seqlens).to(lp.device(), at::kInt).contiguous();
+      n_seqs = cu.numel() - 1;
+    }
+  }
+  const Tensor ent = flat(or_undefined(entropy), at::kFloat), x0 = flat(or_undefined(extra0), at::kFloat),
+               x1 = flat(or_undefined(extra1), at::kFloat);
+  for (const Tensor* t : {&x0, &x1, &ent})
+    if (t->defined() && t->numel() != n)
+      throw py::value_error("a statistic rides along with " + std::to_string(t->numel()) + " elements, expected " +
+                            std::to_string(n));
+  py::dict out;
+  auto f32 = [&](const char* name) {
+    if (reduced) return (float*)nullptr;
+    const Tensor t = empty(lp, {n}, at::kFloat);
+    out[name] = shape.size() == 1 ? t : t.view(shape);
+    return ptr<float>(t);
+  };
+  const Tensor loss = empty(lp, {}, at::kFloat);
+  const Tensor dsum = wants_grad(logprobs) ? empty(lp, {n}, at::kFloat) : Tensor();
+  const int64_t n_results = 8 + (reduced ? 4 * N_SAPO_STATS : 0);
+  const Tensor results = empty(lp, {n_results}, at::kDouble);
+  float *stat_loss = f32("loss"), *ratio = f32("importance_weight"), *kl = f32("approx_kl"),
+        *gate = f32("sapo_soft_gate"), *gp = f32("sapo_scaled_gate_pos"), *gn = f32("sapo_scaled_gate_neg");
+  const size_t bytes = areal_aux_loss_workspace_bytes(n, n_seqs);
+  const Tensor ws = workspace(lp, bytes);
+  check(areal_sapo_loss(ptr<float>(lp), ptr<float>(old), ptr<float>(adv), ptr<uint8_t>(mask), ptr<int32_t>(cu), n,
+                        n_seqs, uniform_len, (float)tau_pos, (float)tau_neg, seq_level, ptr<float>(loss),
+                        ptr<float>(dsum), stat_loss, ratio, kl, gate, gp, gn, ptr<double>(results), ptr<float>(ent),
+                        ptr<float>(x0), ptr<float>(x1), reduced ? ptr<double>(results) + 8 : nullptr, ptr<void>(ws),
+                        bytes, stream_of(lp)),
+        "areal_sapo_loss");
+  HostResultPtr host;
+  if (reduced) {
+    host = std::make_shared<HostResult>(n_results, lp);
+    if (hipMemcpyAsync(host->data(), results.data_ptr(), n_results * sizeof(double), hipMemcpyDeviceToHost,
+                       (hipStream_t)stream_of(lp)) != hipSuccess)
+      fail("copy of the statistics to the host failed");
+  }
+  return py::make_tuple(attach(logprobs, loss, dsum, results), out, host);
+}
+
+py::tuple critic_loss(const Tensor& value, const Tensor& old_value, const Tensor& target_value,
+                      const OptTensor& loss_mask, double eps_clip, bool huber) {
+  const Tensor mask_arg = or_undefined(loss_mask);
+  require_gpu(value, old_value, target_value, mask_arg);
+  const c10::hip::HIPGuard guard(value.device().index());
+  const Tensor v = flat(value, at::kFloat), old = flat(old_value, at::kFloat), target = flat(target_value, at::kFloat),
+               mask = flat(mask_arg, at::kBool);
+  const int64_t n = v.numel();
+  const Tensor loss = empty(v, {}, at::kFloat), stat_loss = empty(v, value.sizes(), at::kFloat),
+               clip = empty(v, value.sizes(), at::kBool), counters = empty(v, {8}, at::kDouble);
+  const Tensor dsum = wants_grad(value) ? empty(v, {n}, at::kFloat) : Tensor();
+  const size_t bytes = areal_aux_loss_workspace_bytes(n, 0);
+  const Tensor ws = workspace(v, bytes);
+  check(areal_critic_loss(ptr<float>(v), ptr<float>(old), ptr<float>(target), ptr<uint8_t>(mask), n, (float)eps_clip,
+                          huber, ptr<float>(loss), ptr<float>(dsum), ptr<float>(stat_loss), ptr<uint8_t>(clip),
+                          ptr<double>(counters), ptr<void>(ws), bytes, stream_of(v)),
+        "areal_critic_loss");
+  return py::make_tuple(attach(value, loss, dsum, counters), clip, stat_loss);
+}
+
+// ---------------------------------------------------------------------------------------
+// Fused lm_head (areal_amd/functional/lm_head.py says what the modes are)
+// ---------------------------------------------------------------------------------------
+int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
+
+// Largest token chunk (multiple of 256) whose backward workspace fits `budget`: bf16 dlogits of the chunk
+// plus the transposed weight (and, when T is not a multiple of 64, transposed copies of the last chunk's
+// hidden states and dlogits).
+int64_t default_token_chunk(int64_t T, int64_t H, int64_t V, int64_t budget) {
+  const bool ragged = T % 64 != 0;
+  const int64_t per_token = 2 * V + 64 + (ragged ? 2 * (V + H) : 0), fixed = 2 * H * (V + 64);
+  const int64_t room = budget - fixed;
+  int64_t chunk = room > 0 ? room / per_token : 0;
+  chunk = std::max<int64_t>(chunk, 256) / 256 * 256;
+  return std::min(std::max<int64_t>(chunk, 256), std::max<int64_t>(T, 1));
+}
+
+// Whether `bytes` fit 60 % of the device memory the allocator can still hand out: free on the device
+// plus what the caching allocator holds but has not given to a tensor. The device is only asked when
+// the latter alone does not settle it.
+bool fits_memory(int64_t bytes, int device) {
+  const auto stats = c10::hip::HIPCachingAllocator::getDeviceStats(device);
+  const size_t all = (size_t)c10::CachingAllocator::StatType::AGGREGATE;
+  const int64_t held = stats.reserved_bytes[all].current - stats.allocated_bytes[all].current;
+  if ((double)bytes <= 0.6 * (double)held) return true;
+  size_t free = 0, total = 0;
+  if (hipMemGetInfo(&free, &total) != hipSuccess) return false;
+  return (double)bytes <= 0.6 * (double)(held + (int64_t)free);
+}
+
+struct LMHeadArgs {
+  double temperature, logit_scale;
+  int64_t token_chunk;  // 0: the default
+  int save_probs;       // -1: decide by size
+  bool with_moments;
+  Tensor accum;         // fp32 accumulator of the weight gradient
+  Tensor owner;         // fp32 parameter whose .grad is that accumulator, see LMHeadState
+  int64_t save_limit, bwd_budget;
+};
+
+struct Status {  // an int in pinned host memory, -1 until the forward's last kernel has written it
+  Tensor host;
+  c10::hip::HIPStream stream;
+  explicit Status(const Tensor& like)
+      : host(at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true))),
+        stream(c10::hip::getCurrentHIPStream(like.device().index())) {
+    *(volatile int*)host.data_ptr() = -1;
+    std::atomic_thread_fence(std::memory_order_release);
+  }
+  ~Status() {
+    if (read() < 0) keep_until_passed(host, stream);
+  }
+  int read() const { return *(volatile int*)host.data_ptr(); }
+  int wait() {
+    if (read() >= 0) return read();
+    py::gil_scoped_release no_gil;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    while (read() < 0)
+      if (std::chrono::steady_clock::now() > until) {
+        stream.synchronize();
+        break;
+      }
+    return read();
+  }
+};
+
+// State of one forward for its backward. The exponentials are consumed by the first backward (it
+// rewrites entries of them in place); a second one recomputes.
+// owner: the fp32 master of `weight`. Its .grad is looked up when the backward runs: an existing one is
+// added to by the contraction, a missing one is allocated and stored to (not cleared first and then
+// read back: 3 x 4 bytes per weight less).
+struct LMHeadState {
+  Tensor probs, probs_ref, probs_status, label_logprobs, bias, accum, owner;
+  std::shared_ptr<Status> status;
+  double temperature = 1.0, logit_scale = 1.0;
+  int64_t token_chunk = 0, bwd_budget = 0;
+  std::vector<int64_t> hidden_shape;
+  at::ScalarType weight_type = at::kBFloat16, bias_type = at::kFloat;
+};
+
+variable_list lm_head_forward(const Tensor& hidden, const Tensor& weight, const Tensor& bias, const Tensor& labels,
+                              const LMHeadArgs& a, bool needs_grad, std::shared_ptr<LMHeadState>* state,
+                              variable_list* saved) {
+  const int64_t H = hidden.size(-1), V = weight.size(0);
+  const Tensor h2 = (hidden.dim() == 2 ? hidden : hidden.reshape({-1, H})).contiguous(), w = weight.contiguous();
+  const Tensor lab = flat(labels, at::kLong);
+  const Tensor bias_f = bias.defined() ? bias.detach().to(at::kFloat).contiguous() : Tensor();
+  const int64_t T = h2.size(0);
+  variable_list outs(6);
+  for (int i = 0; i < (a.with_moments ? 6 : 4); ++i) outs[i] = empty(h2, labels.sizes(), at::kFloat);
+  const int64_t need = 2 * round_up(T, 128) * round_up(V, 64);
+  const bool save = needs_grad && T > 0 &&
+                    (a.save_probs >= 0 ? a.save_probs != 0
+                                       : need <= a.save_limit && fits_memory(need, h2.device().index()));
+  // row_max, sum_exp [T] (and the copy of the log-probabilities and the row references) in one allocation
+  const int64_t Tp = round_up(T, 64);
+  const Tensor rows = empty_f32(h2, Tp * (save ? 4 : 2));
+  const Tensor row_max = rows.narrow(0, 0, T), sum_exp = rows.narrow(0, Tp, T);
+  Tensor probs, probs_ref, probs_status, lp_copy;
+  std::shared_ptr<Status> status;
+  if (save) {
+    probs = empty(h2, {round_up(T, 128), round_up(V, 64)}, at::kBFloat16);
+    lp_copy = rows.narrow(0, 2 * Tp, T);
+    probs_ref = rows.narrow(0, 3 * Tp, T);
+    probs_status = empty(h2, {1}, at::kInt);
+    status = std::make_shared<Status>(h2);
+  }
+  if (T > 0) {
+    const size_t bytes = areal_lmhead_fwd_workspace_bytes(T, H, V);
+    const Tensor ws = workspace(h2, bytes);
+    check(areal_lmhead_fwd_ex(ptr<void>(h2), ptr<void>(w), ptr<float>(bias_f), ptr<int64_t>(lab), T, H, V,
+                              (float)(1.0 / a.temperature), (float)a.logit_scale, ptr<float>(outs[0]),
+                              ptr<float>(outs[1]), ptr<float>(outs[2]), ptr<float>(outs[3]), ptr<float>(outs[4]),
+                              ptr<float>(outs[5]), ptr<float>(row_max), ptr<float>(sum_exp), ptr<void>(probs),
+                              save ? (size_t)need : 0, ptr<float>(probs_ref), ptr<int>(probs_status),
+                              ptr<float>(lp_copy), save ? ptr<int>(status->host) : nullptr, ptr<void>(ws), bytes,
+                              stream_of(h2)),
+          "areal_lmhead_fwd");
+  }
+  if (state != nullptr) {
+    auto st = std::make_shared<LMHeadState>();
+    st->probs = probs; st->probs_ref = probs_ref; st->probs_status = probs_status; st->label_logprobs = lp_copy;
+    st->bias = bias_f; st->accum = a.accum; st->owner = a.owner; st->status = status;
+    st->temperature = a.temperature; st->logit_scale = a.logit_scale; st->token_chunk = a.token_chunk;
+    st->bwd_budget = a.bwd_budget;
+    st->hidden_shape = hidden.sizes().vec();
+    st->weight_type = weight.scalar_type();
+    if (bias.defined()) st->bias_type = bias.scalar_type();
+    *state = st;
+    *saved = {h2, w, lab, row_max, sum_exp};
+  }
+  return outs;
+}
+
+// (dHidden, dWeight, dBias), each absent when it is not wanted. want_*: whose gradient autograd asks for.
+std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, const variable_list& saved,
+                                        const Tensor& grad, bool want_h, bool want_w, bool need_b) {
+  bool need_h = want_h, need_w = want_w;
+  // dWeight goes straight into the caller's fp32 accumulator when one was given: the contraction's
+  // epilogue adds to it and no gradient is returned for the weight
+  Tensor accum = st->accum;
+  bool add = accum.defined();
+  if (st->owner.defined()) {
+    accum = st->owner.grad();
+    add = accum.defined();
+  }
+  if (add || st->owner.defined()) need_w = true;
+  std::vector<OptTensor> none(3);
+  if (!(need_h || need_w || need_b)) return none;
+  const Tensor &h2 = saved[0], &w = saved[1], &lab = saved[2], &row_max = saved[3], &sum_exp = saved[4];
+  const c10::hip::HIPGuard guard(h2.device().index());
+  const int64_t T = h2.size(0), H = h2.size(1), V = w.size(0);
+  const Tensor g = flat(grad, at::kFloat);
+  // the kernels need one of dHidden / dWeight as an output; a bias-only request computes dHidden
+  need_h = need_h || (need_b && !need_w);
+  const Tensor dh = need_h ? at::empty_like(h2) : Tensor();
+  if (st->owner.defined() && !add) {
+    accum = empty(h2, {V, H}, at::kFloat);
+    st->owner.mutable_grad() = accum;
+  }
+  // (the kernels add to the bias gradient as well when they add to the weight's)
+  const Tensor db32 = need_b ? (add ? at::zeros({V}, h2.options().dtype(at::kFloat)) : empty_f32(h2, V)) : Tensor();
+  const Tensor probs = st->probs, probs_ref = st->probs_ref;
+  const float inv_t = (float)(1.0 / st->temperature), scale = (float)st->logit_scale;
+  // A contraction over the whole batch can store dWeight in bf16 itself: the saved mode always, the
+  // recompute mode when one token chunk covers the batch. Several chunks accumulate in fp32 and cast.
+  const int64_t chunk = T > 0 ? (st->token_chunk > 0 ? st->token_chunk
+                                                     : default_token_chunk(T, H, V, st->bwd_budget))
+                              : 1;
+  const bool bf16_out = !accum.defined() && T > 0 && st->weight_type == at::kBFloat16;
+  bool direct = bf16_out && (probs.defined() || chunk >= T);
+  Tensor dw_direct = need_w && direct ? empty(h2, {V, H}, at::kBFloat16) : Tensor();
+  Tensor dw32 = accum;
+  if (!accum.defined() && need_w && !direct) dw32 = empty(h2, {V, H}, at::kFloat);
+  const Tensor probs_status = st->probs_status, label_logprobs = st->label_logprobs;
+  st->probs = st->probs_ref = st->probs_status = Tensor();
+  bool recompute = !probs.defined();
+  const int mode = add ? 1 : 0;
+  if (T == 0) {
+    recompute = false;
+    if (dw32.defined() && !add) dw32.zero_();
+    if (db32.defined()) db32.zero_();
+  } else if (probs.defined()) {
+    // Queued before the host knows whether every row's saved exponentials were in range: the kernels
+    // read that status on the device and return at once if it is set.
+    const size_t bytes = areal_lmhead_bwd_saved_workspace_bytes(T, H, V);
+    const Tensor ws = workspace(h2, bytes);
+    check(areal_lmhead_bwd_saved(ptr<void>(h2), ptr<void>(w), ptr<int64_t>(lab), ptr<float>(row_max),
+                                 ptr<float>(sum_exp), ptr<float>(label_logprobs), ptr<float>(g), T, H, V, inv_t, scale,
+                                 ptr<void>(probs), (size_t)probs.numel() * 2, ptr<float>(probs_ref),
+                                 ptr<int>(probs_status), ptr<void>(dh),
+                                 need_w ? ptr<void>(direct ? dw_direct : dw32) : nullptr, direct ? 2 : mode,
+                                 ptr<float>(db32), ptr<void>(ws), bytes, stream_of(h2)),
+          "areal_lmhead_bwd_saved");
+    // The status travelled to pinned memory with the forward's last kernel. Looking at it now, with the
+    // launches above already queued, idles nothing; if it was set (a row's maximum far above its
+    // estimate) those launches did nothing and the recompute mode runs.
+    if (st->status->wait() != 0) {
+      recompute = true;
+      if (need_w && direct && chunk < T) {
+        direct = false;
+        dw_direct = Tensor();
+        dw32 = empty(h2, {V, H}, at::kFloat);
+      }
+    }
+  }
+  if (recompute) {
+    const size_t bytes = areal_lmhead_bwd_workspace_bytes(T, H, V, chunk);
+    const Tensor ws = workspace(h2, bytes);
+    check(areal_lmhead_bwd(ptr<void>(h2), ptr<void>(w), ptr<float>(st->bias), ptr<int64_t>(lab), ptr<float>(row_max),
+                           ptr<float>(sum_exp), ptr<float>(g), T, H, V, inv_t, scale, ptr<void>(dh),
+                           need_w ? ptr<void>(direct ? dw_direct : dw32) : nullptr, ptr<float>(db32),
+                           direct ? 2 : mode, chunk, ptr<void>(ws), bytes, stream_of(h2)),
+          "areal_lmhead_bwd");
+  }
+  Tensor dw = dw_direct;
+  if (dw32.defined() && !accum.defined()) {
+    if (st->weight_type == at::kFloat) {
+      dw = dw32;
+    } else {
+      dw = empty(h2, {V, H}, st->weight_type);
+      check(areal_cast_f32_to_bf16(ptr<float>(dw32), ptr<void>(dw), dw32.numel(), stream_of(h2)),
+            "areal_cast_f32_to_bf16");
+    }
+  }
+  if (want_h) none[0] = dh.view(st->hidden_shape);
+  if (dw.defined()) none[1] = dw;
+  if (db32.defined()) none[2] = db32.to(st->bias_type);
+  return none;
+}
+
+// (six per-token outputs, tensors to save, state); without needs_grad only the outputs.
+py::tuple lm_head(const Tensor& hidden, const Tensor& weight, const OptTensor& bias_arg, const Tensor& labels,
+                  double temperature, double logit_scale, int64_t token_chunk, int save_probs, bool with_moments,
+                  const OptTensor& accum, const OptTensor& owner, int64_t save_limit, int64_t bwd_budget,
+                  bool build_graph, bool needs_grad) {
+  const Tensor bias = or_undefined(bias_arg);
+  require_gpu(hidden, weight, labels, bias);
+  const c10::hip::HIPGuard guard(hidden.device().index());
+  const LMHeadArgs a{temperature, logit_scale, token_chunk, save_probs, with_moments, or_undefined(accum),
+                     or_undefined(owner), save_limit, bwd_budget};
+  std::shared_ptr<LMHeadState> state;
+  variable_list saved;
+  const variable_list outs = lm_head_forward(hidden, weight, bias, labels, a, needs_grad,
+                                             build_graph ? &state : nullptr, &saved);
+  py::tuple r(6);
+  for (int i = 0; i < 6; ++i) r[i] = outs[i].defined() ? py::cast(outs[i]) : py::none();
+  return build_graph ? py::make_tuple(r, saved, state) : r;
+}
+
+// ---------------------------------------------------------------------------------------
+// Logits-in path
+// ---------------------------------------------------------------------------------------
+struct Logits : public torch::autograd::Function<Logits> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& logits, const Tensor& labels, double temperature,
+                               bool with_entropy) {
+    const int64_t V = logits.size(-1);
+    Tensor rows = logits.scalar_type() == at::kFloat || logits.scalar_type() == at::kBFloat16 ? logits
+                                                                                            : logits.to(at::kFloat);
+    rows = rows.dim() == 2 ? rows : rows.reshape({-1, V});
+    if (rows.stride(-1) != 1 || (rows.size(0) > 1 && rows.stride(0) < V)) rows = rows.contiguous();
+    const int64_t T = rows.size(0);
+    const Tensor lab = flat(labels, at::kLong);
+    const Tensor lp = empty(rows, labels.sizes(), at::kFloat);
+    const Tensor ent = with_entropy ? empty(rows, labels.sizes(), at::kFloat) : Tensor();
+    const Tensor lse2 = empty_f32(rows, T);
+    check(areal_logits_logprobs_entropy_fwd(ptr<void>(rows), rows.scalar_type() == at::kBFloat16 ? 1 : 0,
+                                            T > 1 ? rows.stride(0) : V, ptr<int64_t>(lab), T, V,
+                                            (float)(1.0 / temperature), ptr<float>(lp), ptr<float>(ent),
+                                            ptr<float>(lse2), stream_of(rows)),
+          "areal_logits_logprobs_entropy_fwd");
+    ctx->save_for_backward({rows, lab, lse2, ent});
+    ctx->saved_data["temperature"] = temperature;
+    ctx->saved_data["shape"] = logits.sizes().vec();
+    ctx->saved_data["type"] = (int64_t)logits.scalar_type();
+    ctx->set_materialize_grads(false);
+    if (with_entropy) return {lp, ent};
+    return {lp};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    variable_list r(4);
+    const Tensor glp_arg = grads[0], gen_arg = grads.size() > 1 ? grads[1] : Tensor();
+    if (!glp_arg.defined() && !gen_arg.defined()) return r;
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &rows = saved[0], &lab = saved[1], &lse2 = saved[2], &ent = saved[3];
+    const c10::hip::HIPGuard guard(rows.device().index());
+    const int64_t T = rows.size(0), V = rows.size(1);
+    const Tensor glp = flat(glp_arg, at::kFloat), gen = flat(gen_arg, at::kFloat);
+    Tensor d = empty(rows, {T, V}, rows.scalar_type());
+    check(areal_logits_logprobs_entropy_bwd(ptr<void>(rows), rows.scalar_type() == at::kBFloat16 ? 1 : 0,
+                                            T > 1 ? rows.stride(0) : V, ptr<int64_t>(lab), T, V,
+                                            (float)(1.0 / ctx->saved_data["temperature"].toDouble()), ptr<float>(lse2),
+                                            ptr<float>(ent), ptr<float>(glp), ptr<float>(gen), ptr<void>(d), V,
+                                            stream_of(rows)),
+          "areal_logits_logprobs_entropy_bwd");
+    d = d.view(ctx->saved_data["shape"].toIntVector());
+    const auto type = (at::ScalarType)ctx->saved_data["type"].toInt();
+    r[0] = d.scalar_type() == type ? d : d.to(type);
+    return r;
+  }
+};
+
+variable_list logits_logprobs(const Tensor& logits, const Tensor& labels, double temperature, bool with_entropy) {
+  require_gpu(logits, labels);
+  const c10::hip::HIPGuard guard(logits.device().index());
+  return Logits::apply(logits, labels, temperature, with_entropy);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+  m.def("set_error_class", [](py::object cls) { error_class = cls.release().ptr(); });
+  py::class_<HostResult, HostResultPtr>(m, "HostResult")
+      .def("value", &HostResult::value)
+      .def("fill", &HostResult::fill);
+  m.def("actor_loss", &actor_loss);
+  m.def("proximal_stats", &proximal_stats);
+  m.def("sapo_loss", &sapo_loss);
+  m.def("critic_loss", &critic_loss);
+  py::class_<LMHeadState, std::shared_ptr<LMHeadState>>(m, "LMHeadState")
+      .def_property_readonly("probs", [](const LMHeadState& s) { return s.probs.defined() ? OptTensor(s.probs) : OptTensor(); })
+      .def_property_readonly("probs_ref", [](const LMHeadState& s) { return s.probs_ref.defined() ? OptTensor(s.probs_ref) : OptTensor(); })
+      .def_property_readonly("probs_status", [](const LMHeadState& s) { return s.probs_status.defined() ? OptTensor(s.probs_status) : OptTensor(); });
+  m.def("lm_head", &lm_head);
+  m.def("lm_head_backward", &lm_head_backward);
+  m.def("default_token_chunk", &default_token_chunk);
+  m.def("logits_logprobs", &logits_logprobs);
+}

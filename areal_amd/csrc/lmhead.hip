@@ -666,14 +666,18 @@ template <bool E> using FwdAffineMomSave = FwdEpi<E, true, true, true>;
 // ref_sums: the slots' sums S, Q are relative to row_ref[t] (the saving forward of the
 // hand-scheduled kernels) instead of to each slot's own maximum; the final expressions are then
 // evaluated in fp64, where c2 x - ref and log S (each up to REF_WINDOW binades) cancel.
-// gate / gate_run_if_set: as GemmArgs::skip_if_set / run_if_set.
+// gate / gate_run_if_set: as GemmArgs::skip_if_set / run_if_set. host_status (nullable, pinned host
+// memory; with a gate): receives the gate's value, whether or not the launch does anything.
 constexpr int MERGE_WAVES = 8;
 __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
     const float* __restrict__ ws, int P, int T, int V, int ref_sums, float c2,
     float* __restrict__ logprobs, float* __restrict__ entropy, float* __restrict__ vmin,
     float* __restrict__ vmax, float* __restrict__ vmean, float* __restrict__ vnorm,
     float* __restrict__ row_max, float* __restrict__ sum_exp, const float* __restrict__ row_ref,
-    int* __restrict__ status, const int* __restrict__ gate, int gate_run_if_set) {
+    int* __restrict__ status, const int* __restrict__ gate, int gate_run_if_set,
+    float* __restrict__ logprobs_copy, int* __restrict__ host_status) {
+  if (host_status != nullptr && blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(host_status, *gate, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   if (gate_closed(gate, gate_run_if_set)) return;
   __shared__ float sh_f[5][MERGE_WAVES][64];   // max, S, Q, label logit, min
   __shared__ double sh_d[2][MERGE_WAVES][64];  // sum x, sum x^2
@@ -724,6 +728,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
     if (logprobs) {
       const float lp = (float)(((double)xl * (double)c2 - rr) * ln2 - lnS);
       logprobs[t] = xl <= M ? fminf(lp, 0.f) : lp;
+      if (logprobs_copy) logprobs_copy[t] = logprobs[t];
     }
     if (entropy) entropy[t] = (float)(lnS - ln2 * (double)Q / (double)S);
     // what the backward kernels expect: the sum relative to the rounded product fl(c2 * max)
@@ -738,6 +743,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
     if (logprobs) {
       const float lp = fmaf(xl, c2, -ref_of(M, c2)) * LN2 - logS;
       logprobs[t] = xl <= M ? fminf(lp, 0.f) : lp;
+      if (logprobs_copy) logprobs_copy[t] = logprobs[t];
     }
     if (entropy) entropy[t] = logS - (Q * LN2) / S;
     if (sum_exp) sum_exp[t] = S;
@@ -2069,6 +2075,10 @@ size_t areal_lmhead_probs_bytes(int64_t T, int64_t V) {
   return (size_t)round_up_i64(T, 2 * BK) * (size_t)round_up_i64(V, BK) * 2;
 }
 
+int areal_lmhead_fwd_ex(const void*, const void*, const float*, const int64_t*, int64_t, int64_t, int64_t, float,
+                        float, float*, float*, float*, float*, float*, float*, float*, float*, void*, size_t,
+                        float*, int*, float*, int*, void*, size_t, hipStream_t);
+
 static Regions fwd_regions(int64_t T, int64_t H, int64_t V) {
   return plan_sweep_regions(V, T, H);
 }
@@ -2097,6 +2107,22 @@ int areal_lmhead_fwd(const void* hidden, const void* weight, const float* bias,
                      float* row_max, float* sum_exp, void* probs, size_t probs_bytes,
                      float* probs_ref, int* probs_status, void* workspace, size_t workspace_bytes,
                      hipStream_t stream) {
+  return areal_lmhead_fwd_ex(hidden, weight, bias, labels, T, H, V, inv_temperature, logit_scale, logprobs,
+                             entropy, vocab_min, vocab_max, vocab_mean, vocab_norm, row_max, sum_exp, probs,
+                             probs_bytes, probs_ref, probs_status, nullptr, nullptr, workspace,
+                             workspace_bytes, stream);
+}
+
+// ... with a second copy of the label log-probabilities (for a caller that keeps them for the
+// backward while its user may change the first) and *probs_status also in pinned host memory, written
+// by the last kernel (a copy queued behind it is a launch of its own); both nullable.
+int areal_lmhead_fwd_ex(const void* hidden, const void* weight, const float* bias,
+                        const int64_t* labels, int64_t T, int64_t H, int64_t V,
+                        float inv_temperature, float logit_scale, float* logprobs, float* entropy,
+                        float* vocab_min, float* vocab_max, float* vocab_mean, float* vocab_norm,
+                        float* row_max, float* sum_exp, void* probs, size_t probs_bytes,
+                        float* probs_ref, int* probs_status, float* logprobs_copy, int* host_status,
+                        void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (T < 0 || H <= 0 || V <= 0 || labels == nullptr) return AREAL_ERR_BAD_ARG;
   if ((probs == nullptr) != (probs_ref == nullptr) || (probs == nullptr) != (probs_status == nullptr))
     return AREAL_ERR_BAD_ARG;
@@ -2139,15 +2165,15 @@ int areal_lmhead_fwd(const void* hidden, const void* weight, const float* bias,
     if (!moments) return launch_gemm<Fwd16AffineSave, FwdAffineSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
     return launch_gemm<Fwd16AffineMomSave, FwdAffineMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
   };
-  auto merge = [&](int ref_sums, const float* ref, const int* gate, int gate_run_if_set) {
+  auto merge = [&](int ref_sums, const float* ref, const int* gate, int gate_run_if_set, int* host) {
     hipLaunchKernelGGL(lmhead_merge_kernel, dim3((unsigned)ceil_div_i64(T, 64)), dim3(64 * MERGE_WAVES),
                        0, stream, (const float*)workspace, P, (int)T, (int)V, ref_sums, c2, logprobs,
                        entropy, vocab_min, vocab_max, vocab_mean, vocab_norm, row_max, sum_exp, ref,
-                       probs_status, gate, gate_run_if_set);
+                       probs_status, gate, gate_run_if_set, logprobs_copy, host);
   };
   if (probs == nullptr) {
     if ((rc = fwd_plain(g)) != AREAL_OK) return rc;
-    merge(0, nullptr, nullptr, 0);
+    merge(0, nullptr, nullptr, 0, nullptr);
   } else if (r.k16) {
     // The saving sweep takes its sums relative to the row references, which is only right for rows
     // whose maximum is within the window above the estimate. The merge raises *probs_status if
@@ -2155,18 +2181,21 @@ int areal_lmhead_fwd(const void* hidden, const void* weight, const float* bias,
     // only in that case (otherwise every workgroup of them returns at once), so the outputs are
     // right either way without the host looking at the status in between.
     if ((rc = fwd_save(g)) != AREAL_OK) return rc;
-    merge(1, probs_ref, nullptr, 0);
+    merge(1, probs_ref, nullptr, 0, nullptr);
     AREAL_CHECK_LAUNCH();
     GemmArgs gf = g;
     gf.skip_if_set = probs_status;
     gf.run_if_set = 1;
     if ((rc = fwd_plain(gf)) != AREAL_OK) return rc;
-    merge(0, nullptr, probs_status, 1);
+    merge(0, nullptr, probs_status, 1, host_status);
   } else {
     // the generic kernel's saving epilogue keeps its sums relative to each tile's maximum: the
     // outputs do not depend on the row reference, only the saved buffer does
     if ((rc = fwd_save(g)) != AREAL_OK) return rc;
-    merge(0, probs_ref, nullptr, 0);
+    merge(0, probs_ref, nullptr, 0, nullptr);
+    if (host_status != nullptr &&
+        hipMemcpyAsync(host_status, probs_status, sizeof(int), hipMemcpyDeviceToHost, stream) != hipSuccess)
+      return AREAL_ERR_LAUNCH;
   }
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;

@@ -65,10 +65,16 @@ struct LossIO {
   float* behave_w;
   float* behave_kl;
   uint8_t* behave_mask;
+  float* clip_ratio;      // the masks and differences grpo_loss_fn logs, as fp32
+  float* dual_ratio;
+  float* logp_diff;
+  float* logp_abs_diff;
+  float* filtered_ratio;
   // fused logging statistics (loss_token_kernel<true> only)
   const float* entropy;   // optional per-token input
   const float* extra0;    // optional per-token inputs reduced over all tokens
   const float* extra1;
+  int stat_prox;          // also reduce prox (ST_PROX_LOGP)
 };
 
 // Logged statistics reduced inside the token pass (the tensors grpo_loss_fn hands to the stats
@@ -77,10 +83,12 @@ enum {
   ST_IMPORTANCE_WEIGHT = 0, ST_APPROX_KL, ST_NEW_LOGP, ST_OLD_LOGP, ST_ENTROPY, ST_ACTOR_LOSS,
   ST_CLIP_RATIO, ST_DUAL_CLIP_RATIO, ST_LOGP_DIFF, ST_LOGP_ABS_DIFF, ST_BEHAVE_FILTERED_RATIO,
   ST_BEHAVE_IMP_WEIGHT, ST_BEHAVE_APPROX_KL, ST_CLIPPED_NEW_LOGP, ST_CLIPPED_OLD_LOGP,
-  ST_EXTRA0, ST_EXTRA1, N_LOSS_STATS
+  ST_EXTRA0, ST_EXTRA1, ST_PROX_LOGP, N_LOSS_STATS
 };
-// denominators: 0 loss mask (before rejection), 1 clip mask, 2 behave mask, 3 every token
-__device__ const int STAT_DENOM[N_LOSS_STATS] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 2, 2, 1, 1, 3, 3};
+constexpr int N_LOSS_STATS_V1 = ST_PROX_LOGP;  // rows areal_actor_loss_stats returns
+// denominators: 0 loss mask (before rejection), 1 clip mask, 2 behave mask, 3 every token, 4 behave
+// mask under rejection sampling, else loss mask
+__device__ const int STAT_DENOM[N_LOSS_STATS] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 2, 2, 1, 1, 3, 3, 4};
 
 struct StatPartial {
   double sum;
@@ -89,17 +97,28 @@ struct StatPartial {
 
 struct Partial {
   double loss_sum;
-  long long n_valid, n_kept, n_filtered, n_clip, n_dual, n_behave;
+  long long n_valid, n_kept, n_filtered, n_clip, n_dual, n_behave, n_bad;
 };
+constexpr int N_COUNTS = 7;
 
-DEVI int seq_of(const LossIO& io, int64_t t) {
-  if (io.uniform_len > 0) return (int)(t / io.uniform_len);
-  int lo = 0, hi = io.n_seqs;  // find last s with cu[s] <= t
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if ((int64_t)io.cu[mid] <= t) lo = mid; else hi = mid;
-  }
-  return lo;
+DEVI int64_t seq_end(const LossIO& io, int s) {
+  return io.uniform_len > 0 ? (int64_t)(s + 1) * io.uniform_len : (int64_t)io.cu[s + 1];
+}
+// The sequence of token t (the last s that starts at or before t), by one wave; t is the same in all
+// lanes.
+DEVI int seq_search(const LossIO& io, int64_t t, int lane) {
+  int s;
+  if (io.uniform_len > 0) s = (int)(t / io.uniform_len);
+  else s = wave_count_le(io.cu + 1, io.n_seqs, t, lane);
+  return s < io.n_seqs ? s : io.n_seqs - 1;
+}
+// ... and from a sequence that starts at or before t.
+DEVI int seq_from(const LossIO& io, int s, int64_t t) {
+  while (s + 1 < io.n_seqs && seq_end(io, s) <= t) ++s;
+  return s;
+}
+DEVI bool needs_seq(const LossCfg& c) {
+  return (c.rs_enabled && c.rs_seq_level) || (c.loss_kind == LOSS_PPO && c.seq_is);
 }
 
 // torch.clamp keeps NaN (fminf/fmaxf would drop it).
@@ -157,54 +176,78 @@ DEVI T block_sum(T v, T* smem) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Segmented pass 1: per-sequence aggregate of the rejection metric (one block per sequence).
+// Segmented pass 1: per-sequence aggregate of the rejection metric.
 // Writes seq_rs[s] = {in_bounds, uniform weight exp(mean log ratio)}.
+// WPS waves per sequence: a block of 4 waves takes 4 / WPS sequences. Bound by HBM (9 bytes per
+// token): a lane takes four tokens with 16-byte loads, aligned whatever the sequence's start is
+// (VEC = 4), the loads of a group do not wait for its mask, and short sequences take a wave each so
+// that the lanes of a block are not idle. 4 Mi tokens in 2048 sequences: 38 us with one token per
+// lane and loads behind the mask.
 // ---------------------------------------------------------------------------------------
+template <int WPS, int VEC>
 __global__ __launch_bounds__(LOSS_THREADS) void seq_rs_kernel(LossIO io, LossCfg c, float* seq_rs) {
-  __shared__ double sm_d[8];
-  __shared__ float sm_f[8];
-  const int s = blockIdx.x;
-  int64_t t0, t1;
-  if (io.uniform_len > 0) { t0 = (int64_t)s * io.uniform_len; t1 = t0 + io.uniform_len; }
-  else { t0 = io.cu[s]; t1 = io.cu[s + 1]; }
+  constexpr int NW = LOSS_THREADS / 64, SPB = NW / WPS;
+  __shared__ double sm_d[2][NW];
+  __shared__ float sm_f[NW];
+  __shared__ int sm_i[2][NW];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int s = blockIdx.x * SPB + w / WPS;
+  const bool live = s < io.n_seqs;
+  int64_t t0 = 0, t1 = 0;
+  if (live) {
+    t0 = io.uniform_len > 0 ? (int64_t)s * io.uniform_len : (int64_t)io.cu[s];
+    t1 = seq_end(io, s);
+  }
   if (t1 > io.n) t1 = io.n;
   double sum_lr = 0.0, sum_m = 0.0;
   float mx = neg_inf();
-  long long cnt = 0;
+  int nan = 0, cnt = 0;
   const bool log_agg = (c.rs_metric == METRIC_RATIO);
-  for (int64_t t = t0 + threadIdx.x; t < t1; t += blockDim.x) {
-    if (!io.mask[t]) continue;
-    const float prox = io.prox[t], old = io.old[t];
+  auto token = [&](bool m, float prox, float old) {
+    if (!m) return;
     const float lr = sane_log_ratio(prox, old);
     const float v = log_agg ? lr : rs_metric(prox, old, 0.0f, c.rs_metric);  // (the ratio metric aggregates lr)
     cnt += 1;
     sum_lr += (double)lr;
     sum_m += (double)v;
-    mx = (v != v || mx != mx) ? __builtin_nanf("") : fmaxf(mx, v);
+    if (v != v) nan = 1;
+    else mx = fmaxf(mx, v);
+  };
+  const int64_t first = t0 & ~(int64_t)(VEC - 1);
+  for (int64_t t = first + (int64_t)((w % WPS) * 64 + lane) * VEC; t < t1; t += (int64_t)WPS * 64 * VEC) {
+    if (t + VEC <= io.n) {
+      bool m[VEC];
+      float prox[VEC], old[VEC];
+      load_mask<VEC>(io.mask, t, m);
+      load_f32<VEC>(io.prox, t, prox);
+      load_f32<VEC>(io.old, t, old);
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) token(m[i] && t + i >= t0 && t + i < t1, prox[i], old[i]);
+    } else {
+      for (int64_t u = t > t0 ? t : t0; u < t1; ++u) token(io.mask[u] != 0, io.prox[u], io.old[u]);
+    }
   }
-  sum_lr = block_sum(sum_lr, sm_d);
-  sum_m = block_sum(sum_m, sm_d);
-  // max with NaN propagation: reduce a NaN flag and the max separately
-  float nanflag = (mx != mx) ? 1.f : 0.f;
-  float mxc = (mx != mx) ? neg_inf() : mx;
-  mxc = wave_max(mxc);
-  nanflag = wave_max(nanflag);
-  {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  sum_lr = wave_sum(sum_lr);
+  sum_m = wave_sum(sum_m);
+  mx = wave_max(mx);
+  cnt = wave_sum(cnt);
+  nan = wave_sum(nan);
+  if (WPS > 1) {
+    if (lane == 0) { sm_d[0][w] = sum_lr; sm_d[1][w] = sum_m; sm_f[w] = mx; sm_i[0][w] = cnt; sm_i[1][w] = nan; }
     __syncthreads();
-    if (lane == 0) { sm_f[w] = mxc; sm_f[4 + w] = nanflag; }
-    __syncthreads();
-    mxc = fmaxf(fmaxf(sm_f[0], sm_f[1]), fmaxf(sm_f[2], sm_f[3]));
-    nanflag = fmaxf(fmaxf(sm_f[4], sm_f[5]), fmaxf(sm_f[6], sm_f[7]));
+    if (w % WPS != 0) return;
+    for (int k = 1; k < WPS; ++k) {
+      sum_lr += sm_d[0][w + k]; sum_m += sm_d[1][w + k];
+      mx = fmaxf(mx, sm_f[w + k]);
+      cnt += sm_i[0][w + k]; nan += sm_i[1][w + k];
+    }
   }
-  __shared__ long long sm_l[8];
-  const long long total = block_sum(cnt, sm_l);
-  if (threadIdx.x == 0) {
-    const float denom = (float)(total > 0 ? total : 1);
+  if (lane == 0 && live) {
+    const float denom = (float)(cnt > 0 ? cnt : 1);
     float agg;
     if (c.rs_agg == AGG_SUM) agg = (float)sum_m;
     else if (c.rs_agg == AGG_MEAN) agg = (float)sum_m / denom;
-    else agg = total == 0 ? 0.0f : (nanflag > 0.f ? __builtin_nanf("") : mxc);
+    else agg = cnt == 0 ? 0.0f : (nan > 0 ? __builtin_nanf("") : mx);
     const float seq_metric = log_agg ? expf(agg) : agg;
     seq_rs[2 * s + 0] = in_bounds(seq_metric, c) ? 1.0f : 0.0f;
     seq_rs[2 * s + 1] = log_agg ? expf((float)sum_lr / denom) : 0.0f;
@@ -213,14 +256,13 @@ __global__ __launch_bounds__(LOSS_THREADS) void seq_rs_kernel(LossIO io, LossCfg
 
 // Rejection sampling for one token. Returns the narrowed mask; sets w (not yet zeroed outside
 // the mask) and whether the token counts as filtered / clamped.
-DEVI bool rs_token(const LossIO& io, const LossCfg& c, int64_t t, bool m, float prox, float old, float& w,
+DEVI bool rs_token(const LossIO& io, const LossCfg& c, int s, bool m, float prox, float old, float& w,
                    bool& counted) {
   const float lr = sane_log_ratio(prox, old);
   w = expf(lr);
   bool keep = true;
   counted = false;
   if (c.rs_seq_level) {
-    const int s = seq_of(io, t);
     const bool seq_ok = io.seq_rs[2 * s] != 0.0f;
     if (c.rs_metric == METRIC_RATIO) w = io.seq_rs[2 * s + 1];
     if (c.rs_clamp) {
@@ -281,7 +323,7 @@ __global__ __launch_bounds__(LOSS_THREADS) void seq_is_kernel(LossIO io, LossCfg
 // Running sums of one thread. Counts fit 32 bits per thread (a thread sees n / gridsize tokens).
 struct TokenAcc {
   double loss_sum;
-  int n_valid, n_kept, n_filtered, n_clip, n_dual, n_behave;
+  int n_valid, n_kept, n_filtered, n_clip, n_dual, n_behave, n_bad;
 };
 
 // The logged statistics a thread reduces itself. The three 0/1-valued ones (clip_ratio,
@@ -319,24 +361,26 @@ struct TokenOut {
 };
 
 template <bool STATS>
-DEVI void token_body(const LossIO& io, const LossCfg& c, int64_t t, const TokenIn& in, TokenOut& out,
+DEVI void token_body(const LossIO& io, const LossCfg& c, int s, const TokenIn& in, TokenOut& out,
                      TokenAcc& acc, StatAcc<STATS>& st) {
   const bool m = in.m;
   bool m2 = m;
   float w = 1.0f;
   if (c.rs_enabled) {
     bool counted;
-    m2 = rs_token(io, c, t, m, in.prox, in.old, w, counted);
+    m2 = rs_token(io, c, s, m, in.prox, in.old, w, counted);
     w = m2 ? w : 0.0f;
     acc.n_filtered += counted;
   }
   out.m2 = m2;
   out.behave_w = w;
   acc.n_valid += m;
+  acc.n_bad += !__builtin_isfinite(in.prox);
   acc.n_kept += m2;
   if (STATS) {
     if (io.extra0) st.add(ST_EXTRA0, in.extra0);
     if (io.extra1) st.add(ST_EXTRA1, in.extra1);
+    if (io.stat_prox && !c.rs_enabled && m) st.add(ST_PROX_LOGP, in.prox);
   }
   out.dlp = 0.f; out.loss = 0.f; out.ratio = 0.f; out.kl = 0.f; out.behave_kl = 0.f;
   out.clip = false; out.dual = false; out.bm = false;
@@ -357,7 +401,6 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, int64_t t, const TokenI
   } else {
     float ratio, a = adv, dratio;  // dratio = d ratio / d lp[t] factor handled below
     if (c.seq_is) {
-      const int s = seq_of(io, t);
       ratio = m2 ? io.seq_is[4 * s + 0] : 0.0f;
       a = m2 ? io.seq_is[4 * s + 1] : 0.0f;
       dratio = 0.f;  // gradient assembled per sequence below
@@ -385,7 +428,6 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, int64_t t, const TokenI
     }
     if (c.seq_is) {
       // every kept token of the sequence receives ratio_s/count_s * sum_w_s * dpg_s
-      const int s = seq_of(io, t);
       dsel = m2 ? dpg * ratio * io.seq_is[4 * s + 2] * io.seq_is[4 * s + 3] : 0.0f;
     } else {
       dsel = dpg * dratio;
@@ -407,6 +449,7 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, int64_t t, const TokenI
     }
   }
   if (STATS) {
+    if (io.stat_prox && c.rs_enabled && out.bm) st.add(ST_PROX_LOGP, prox);
     if (m) {
       st.add(ST_IMPORTANCE_WEIGHT, ratio_out);
       st.add(ST_APPROX_KL, kl);
@@ -453,7 +496,7 @@ DEVI void token_group_load(const LossIO& io, const LossCfg& c, int64_t t, TokenL
   load_f32<VEC>(STATS ? io.extra1 : nullptr, t, in.x1);
 }
 template <bool STATS, int VEC>
-DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, const TokenLoad<VEC>& ld,
+DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, int s, const TokenLoad<VEC>& ld,
                               TokenAcc& acc, StatAcc<STATS>& st) {
   float dlp[VEC], loss[VEC], ratio[VEC], kl[VEC], bw[VEC], bkl[VEC];
   bool clip[VEC], dual[VEC], m2[VEC], bm[VEC];
@@ -461,7 +504,8 @@ DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, con
   for (int i = 0; i < VEC; ++i) {
     const TokenIn in{ld.lp[i], ld.prox[i], ld.old[i], ld.adv[i], ld.ent[i], ld.x0[i], ld.x1[i], ld.m[i]};
     TokenOut o;
-    token_body<STATS>(io, c, t + i, in, o, acc, st);
+    if (s >= 0) s = seq_from(io, s, t + i);
+    token_body<STATS>(io, c, s, in, o, acc, st);
     dlp[i] = o.dlp; loss[i] = o.loss; ratio[i] = o.ratio; kl[i] = o.kl; bw[i] = o.behave_w; bkl[i] = o.behave_kl;
     clip[i] = o.clip; dual[i] = o.dual; m2[i] = o.m2; bm[i] = o.bm;
   }
@@ -480,6 +524,22 @@ DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, con
   store_f32<VEC>(io.stat_kl, t, kl);
   store_mask<VEC>(io.clip_mask, t, clip);
   store_mask<VEC>(io.dual_mask, t, dual);
+  if (io.logp_diff != nullptr) {  // the five tensors that are logged besides: all of them or none
+    float cr[VEC], dr[VEC], df[VEC], ad[VEC], fr[VEC];
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+      cr[i] = clip[i] ? 1.f : 0.f;
+      dr[i] = dual[i] ? 1.f : 0.f;
+      df[i] = (ld.old[i] - ld.lp[i]) * (ld.m[i] ? 1.f : 0.f);
+      ad[i] = fabsf(df[i]);
+      fr[i] = ld.m[i] && !bm[i] ? 1.f : 0.f;
+    }
+    store_f32<VEC>(io.clip_ratio, t, cr);
+    store_f32<VEC>(io.dual_ratio, t, dr);
+    store_f32<VEC>(io.logp_diff, t, df);
+    store_f32<VEC>(io.logp_abs_diff, t, ad);
+    if (c.rs_enabled) store_f32<VEC>(io.filtered_ratio, t, fr);
+  }
 }
 
 // STATS: also reduce the logged statistics (sum, min, max per block) into stat_partials
@@ -488,21 +548,30 @@ template <bool STATS, int VEC>
 __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, LossCfg c,
                                                                    Partial* partials,
                                                                    StatPartial* stat_partials) {
-  TokenAcc acc{0.0, 0, 0, 0, 0, 0, 0};
+  TokenAcc acc{0.0, 0, 0, 0, 0, 0, 0, 0};
   StatAcc<STATS> st;
   st.init();
+  // Sequence-level options need each token's sequence: a wave searches the one of its first token
+  // (64 probes a round) and its lanes walk on from there, instead of a binary search per token.
+  const bool seq = needs_seq(c);
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
   const int64_t n_vec = io.n - io.n % VEC;
   TokenLoad<VEC> in;
-  for (int64_t t = gid * VEC; t < n_vec; t += nthreads * VEC) {
+  const int64_t wid = gid & ~(int64_t)63;
+  for (int64_t t = gid * VEC, tw = wid * VEC; tw < n_vec; t += nthreads * VEC, tw += nthreads * VEC) {
+    const int s = seq ? seq_search(io, tw, threadIdx.x & 63) : -1;
+    if (t >= n_vec) continue;
     token_group_load<STATS, VEC>(io, c, t, in);
-    token_group_compute<STATS, VEC>(io, c, t, in, acc, st);
+    token_group_compute<STATS, VEC>(io, c, t, s, in, acc, st);
   }
-  if (VEC > 1 && n_vec + gid < io.n) {
-    TokenLoad<1> tail;
-    token_group_load<STATS, 1>(io, c, n_vec + gid, tail);
-    token_group_compute<STATS, 1>(io, c, n_vec + gid, tail, acc, st);
+  if (VEC > 1 && n_vec + wid < io.n) {
+    const int s = seq ? seq_search(io, n_vec + wid, threadIdx.x & 63) : -1;
+    if (n_vec + gid < io.n) {
+      TokenLoad<1> tail;
+      token_group_load<STATS, 1>(io, c, n_vec + gid, tail);
+      token_group_compute<STATS, 1>(io, c, n_vec + gid, s, tail, acc, st);
+    }
   }
 
   // One barrier pair for everything the block hands on. A wave sums its counters as 32-bit integers
@@ -510,18 +579,19 @@ __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, Los
   // lanes only, and the 16 row results of the block are combined from LDS in a fixed order.
   constexpr int NW = LOSS_THREADS / 64, NROW = LOSS_THREADS / 16;
   __shared__ double sh_loss[NW];
-  __shared__ int sh_cnt[NW][6];
+  __shared__ int sh_cnt[NW][N_COUNTS];
   __shared__ double sh_sum[STATS ? NROW : 1][STATS ? N_LOSS_STATS : 1];
   __shared__ float sh_mn[STATS ? NROW : 1][STATS ? N_LOSS_STATS : 1], sh_mx[STATS ? NROW : 1][STATS ? N_LOSS_STATS : 1];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   {
     const double ls = wave_sum(acc.loss_sum);
-    const int cnt[6] = {wave_sum(acc.n_valid), wave_sum(acc.n_kept), wave_sum(acc.n_filtered),
-                        wave_sum(acc.n_clip), wave_sum(acc.n_dual), wave_sum(acc.n_behave)};
+    const int cnt[N_COUNTS] = {wave_sum(acc.n_valid), wave_sum(acc.n_kept), wave_sum(acc.n_filtered),
+                               wave_sum(acc.n_clip), wave_sum(acc.n_dual), wave_sum(acc.n_behave),
+                               wave_sum(acc.n_bad)};
     if (lane == 0) {
       sh_loss[w] = ls;
 #pragma unroll
-      for (int k = 0; k < 6; ++k) sh_cnt[w][k] = cnt[k];
+      for (int k = 0; k < N_COUNTS; ++k) sh_cnt[w][k] = cnt[k];
     }
   }
   if (STATS) {
@@ -537,11 +607,13 @@ __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, Los
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    Partial p{sh_loss[0], sh_cnt[0][0], sh_cnt[0][1], sh_cnt[0][2], sh_cnt[0][3], sh_cnt[0][4], sh_cnt[0][5]};
+    Partial p{sh_loss[0], sh_cnt[0][0], sh_cnt[0][1], sh_cnt[0][2], sh_cnt[0][3], sh_cnt[0][4], sh_cnt[0][5],
+              sh_cnt[0][6]};
     for (int i = 1; i < NW; ++i) {
       p.loss_sum += sh_loss[i];
       p.n_valid += sh_cnt[i][0]; p.n_kept += sh_cnt[i][1]; p.n_filtered += sh_cnt[i][2];
       p.n_clip += sh_cnt[i][3]; p.n_dual += sh_cnt[i][4]; p.n_behave += sh_cnt[i][5];
+      p.n_bad += sh_cnt[i][6];
     }
     partials[blockIdx.x] = p;
   }
@@ -561,19 +633,22 @@ __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, Los
 
 // counters: [0] loss_sum [1] n_valid [2] n_kept [3] n_filtered [4] n_clip [5] n_dual
 //           [6] n_behave [7] loss = loss_sum / max(n_valid, 1)
+//           [8] n_bad (tokens whose proximal log-prob is not finite; only with `extended`)
 // Block 0 folds the token kernel's block partials into the counters and the loss, in a fixed order
 // (thread partials -> wave shuffles -> 4 wave slots). With statistics, block 1 + k folds statistic
 // k into stats [N_LOSS_STATS][4] = {sum, count, min, max}; the count is the statistic's denominator.
 // The three 0/1-valued statistics are not reduced per token: their sums are token counts and
 // their extremes follow from whether every / any counted token has the value 1. Each block sums
-// the counts it needs itself, so one launch does everything.
+// the counts it needs itself, so one launch does everything. host (nullable): the same values into
+// pinned host memory, [9] counters and then the statistics, so that no copy has to be queued behind.
+// nan_if_bad: the loss is NaN when n_bad is not 0.
 __global__ __launch_bounds__(FINAL_THREADS) void loss_finalize_kernel(
     const Partial* __restrict__ partials, const StatPartial* __restrict__ stat_partials, int nparts,
     float* loss_out, double* __restrict__ counters, double n_tokens, double* __restrict__ stats,
-    int loss_active, int rs_enabled) {
+    int loss_active, int rs_enabled, int extended, int nan_if_bad, double* __restrict__ host) {
   constexpr int NW = FINAL_THREADS / 64;
   __shared__ double sh_d[NW][2];     // loss sum, statistic sum
-  __shared__ long long sh_l[NW][6];
+  __shared__ long long sh_l[NW][N_COUNTS];
   __shared__ float sh_f[NW][2];      // statistic minimum, maximum
   const int k = (int)blockIdx.x - 1;  // the block's statistic; block 0: the counters and the loss
   const bool reduced = k >= 0 && !(k == ST_CLIP_RATIO || k == ST_DUAL_CLIP_RATIO || k == ST_BEHAVE_FILTERED_RATIO);
@@ -585,18 +660,19 @@ __global__ __launch_bounds__(FINAL_THREADS) void loss_finalize_kernel(
 #pragma unroll
   for (int j = 0; j < PER_THREAD; ++j) {
     const int i = threadIdx.x + j * FINAL_THREADS;
-    pp[j] = i < nparts ? partials[i] : Partial{0.0, 0, 0, 0, 0, 0, 0};
+    pp[j] = i < nparts ? partials[i] : Partial{0.0, 0, 0, 0, 0, 0, 0, 0};
     sp[j] = StatPartial{0.0, pos_inf(), neg_inf()};
     if (reduced && i < nparts) sp[j] = stat_partials[(size_t)i * N_LOSS_STATS + k];
   }
   double ls = 0.0, sum = 0.0;
-  long long a[6] = {0, 0, 0, 0, 0, 0};
+  long long a[N_COUNTS] = {0, 0, 0, 0, 0, 0, 0};
   float mn = pos_inf(), mx = neg_inf();
 #pragma unroll
   for (int j = 0; j < PER_THREAD; ++j) {
     ls += pp[j].loss_sum;
     a[0] += pp[j].n_valid; a[1] += pp[j].n_kept; a[2] += pp[j].n_filtered;
     a[3] += pp[j].n_clip; a[4] += pp[j].n_dual; a[5] += pp[j].n_behave;
+    a[6] += pp[j].n_bad;
     sum += sp[j].sum;
     mn = stat_min(mn, sp[j].mn);
     mx = stat_max(mx, sp[j].mx);
@@ -604,7 +680,7 @@ __global__ __launch_bounds__(FINAL_THREADS) void loss_finalize_kernel(
   // wave results into LDS, one barrier, then thread 0 adds the waves in order
   ls = wave_sum(ls);
 #pragma unroll
-  for (int q = 0; q < 6; ++q) a[q] = wave_sum(a[q]);
+  for (int q = 0; q < N_COUNTS; ++q) a[q] = wave_sum(a[q]);
   if (reduced) {
     sum = wave_sum(sum);
     mn = wave_stat_min(mn);
@@ -614,31 +690,36 @@ __global__ __launch_bounds__(FINAL_THREADS) void loss_finalize_kernel(
   if (lane == 0) {
     sh_d[w][0] = ls; sh_d[w][1] = sum;
 #pragma unroll
-    for (int q = 0; q < 6; ++q) sh_l[w][q] = a[q];
+    for (int q = 0; q < N_COUNTS; ++q) sh_l[w][q] = a[q];
     sh_f[w][0] = mn; sh_f[w][1] = mx;
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
   ls = sh_d[0][0]; sum = sh_d[0][1]; mn = sh_f[0][0]; mx = sh_f[0][1];
 #pragma unroll
-  for (int q = 0; q < 6; ++q) a[q] = sh_l[0][q];
+  for (int q = 0; q < N_COUNTS; ++q) a[q] = sh_l[0][q];
   for (int i = 1; i < NW; ++i) {
     ls += sh_d[i][0]; sum += sh_d[i][1];
 #pragma unroll
-    for (int q = 0; q < 6; ++q) a[q] += sh_l[i][q];
+    for (int q = 0; q < N_COUNTS; ++q) a[q] += sh_l[i][q];
     mn = stat_min(mn, sh_f[i][0]); mx = stat_max(mx, sh_f[i][1]);
   }
   if (k < 0) {
-    counters[0] = ls;
-    for (int q = 0; q < 6; ++q) counters[1 + q] = (double)a[q];
     const double denom = a[0] > 0 ? (double)a[0] : 1.0;
     const float loss = (float)ls / (float)denom;
-    counters[7] = (double)loss;
-    if (loss_out) *loss_out = loss;
+    const double out[9] = {ls, (double)a[0], (double)a[1], (double)a[2], (double)a[3], (double)a[4],
+                           (double)a[5], (double)loss, (double)a[6]};
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+      if (q < 8 || extended) counters[q] = out[q];
+      if (host != nullptr) host[q] = out[q];
+    }
+    if (loss_out) *loss_out = nan_if_bad && a[6] > 0 ? __builtin_nanf("") : loss;
     return;
   }
   const long long n_valid = a[0], n_clip = a[3], n_dual = a[4], n_behave = a[5];
-  const int d = STAT_DENOM[k];
+  int d = STAT_DENOM[k];
+  if (d == 4) d = rs_enabled ? 2 : 0;
   const double count = d == 0 ? (double)n_valid : (d == 1 ? (double)n_clip : (d == 2 ? (double)n_behave : n_tokens));
   if (!reduced) {
     // ones among the n_valid tokens under the loss mask
@@ -655,6 +736,10 @@ __global__ __launch_bounds__(FINAL_THREADS) void loss_finalize_kernel(
   stats[4 * k + 1] = count;
   stats[4 * k + 2] = (double)mn;
   stats[4 * k + 3] = (double)mx;
+  if (host != nullptr) {
+    double* h = host + 9 + 4 * k;
+    h[0] = sum; h[1] = count; h[2] = (double)mn; h[3] = (double)mx;
+  }
 }
 
 // out[t] = dlp[t] * upstream[0] / max(n_valid, 1); VEC as in the token kernel
@@ -746,6 +831,13 @@ int scratch_for_current_device(void** out) {
   return AREAL_OK;
 }
 
+// What areal_actor_loss_call adds to the other entry points.
+struct LossMore {
+  float *clip_ratio, *dual_ratio, *logp_diff, *logp_abs_diff, *filtered_ratio;
+  int nan_if_bad;
+  double* host;
+};
+
 int actor_loss_impl(const float* logprobs, const float* proximal, const float* old_logprobs,
                     const float* advantages, const uint8_t* loss_mask, const int32_t* cu_seqlens,
                     int64_t n_tokens, int64_t n_seqs, int64_t uniform_len,
@@ -753,7 +845,7 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
                     float* stat_ratio, float* stat_approx_kl, uint8_t* clip_mask,
                     uint8_t* dual_clip_mask, uint8_t* new_mask, float* behave_imp_weight,
                     float* behave_approx_kl, uint8_t* behave_mask, double* counters,
-                    const LossStatsArgs* sa, void* workspace, size_t workspace_bytes,
+                    const LossStatsArgs* sa, const LossMore* more, void* workspace, size_t workspace_bytes,
                     hipStream_t stream);
 
 }  // namespace
@@ -789,7 +881,7 @@ int areal_actor_loss(const float* logprobs, const float* proximal, const float* 
   return actor_loss_impl(logprobs, proximal, old_logprobs, advantages, loss_mask, cu_seqlens, n_tokens,
                          n_seqs, uniform_len, cfg, loss, dlogprobs, stat_loss, stat_ratio,
                          stat_approx_kl, clip_mask, dual_clip_mask, new_mask, behave_imp_weight,
-                         behave_approx_kl, behave_mask, counters, nullptr, workspace, workspace_bytes,
+                         behave_approx_kl, behave_mask, counters, nullptr, nullptr, workspace, workspace_bytes,
                          stream);
 }
 
@@ -816,7 +908,7 @@ int areal_actor_loss_stats(const float* logprobs, const float* proximal, const f
   return actor_loss_impl(logprobs, proximal, old_logprobs, advantages, loss_mask, cu_seqlens, n_tokens,
                          n_seqs, uniform_len, cfg, loss, dlogprobs, stat_loss, stat_ratio,
                          stat_approx_kl, clip_mask, dual_clip_mask, new_mask, behave_imp_weight,
-                         behave_approx_kl, behave_mask, counters, &sa, workspace, workspace_bytes,
+                         behave_approx_kl, behave_mask, counters, &sa, nullptr, workspace, workspace_bytes,
                          stream);
 }
 
@@ -841,8 +933,41 @@ int areal_actor_loss_static(const float* logprobs, const float* proximal,
   return actor_loss_impl(logprobs, proximal, old_logprobs, advantages, loss_mask, cu_seqlens, n_tokens,
                          n_seqs, uniform_len, cfg, loss, dlogprobs, stat_loss, stat_ratio,
                          stat_approx_kl, clip_mask, dual_clip_mask, new_mask, behave_imp_weight,
-                         behave_approx_kl, behave_mask, counters, nullptr, ws, STATIC_SCRATCH_BYTES,
+                         behave_approx_kl, behave_mask, counters, nullptr, nullptr, ws, STATIC_SCRATCH_BYTES,
                          stream);
+}
+
+// areal_actor_loss with every optional input and output in one struct (include/areal_hip.h).
+struct areal_actor_loss_io {
+  const float *logprobs, *proximal, *old_logprobs, *advantages;
+  const uint8_t* loss_mask;
+  const int32_t* cu_seqlens;
+  const float *entropy, *extra0, *extra1;
+  int64_t n_tokens, n_seqs, uniform_len;
+  float *loss, *dlogprobs, *stat_loss, *stat_ratio, *stat_approx_kl;
+  uint8_t *clip_mask, *dual_clip_mask, *new_mask;
+  float *behave_imp_weight, *behave_approx_kl;
+  uint8_t* behave_mask;
+  float *clip_ratio, *dual_clip_ratio, *logp_diff, *logp_abs_diff, *behave_filtered_ratio;
+  double* results;
+  double* host_results;
+  int with_stats, nan_if_nonfinite;
+};
+int areal_actor_loss_call(const areal_actor_loss_io* a, const areal_loss_config* cfg, void* workspace,
+                          size_t workspace_bytes, hipStream_t stream) {
+  if (a == nullptr || a->results == nullptr) return AREAL_ERR_BAD_ARG;
+  if (a->logp_diff != nullptr && a->n_tokens > 0 &&
+      (a->old_logprobs == nullptr || a->clip_ratio == nullptr || a->dual_clip_ratio == nullptr ||
+       a->logp_abs_diff == nullptr))
+    return AREAL_ERR_BAD_ARG;
+  const LossStatsArgs sa{a->entropy, a->extra0, a->extra1, a->results + 9};
+  const LossMore more{a->clip_ratio, a->dual_clip_ratio, a->logp_diff, a->logp_abs_diff,
+                      a->behave_filtered_ratio, a->nan_if_nonfinite, a->host_results};
+  return actor_loss_impl(a->logprobs, a->proximal, a->old_logprobs, a->advantages, a->loss_mask, a->cu_seqlens,
+                         a->n_tokens, a->n_seqs, a->uniform_len, cfg, a->loss, a->dlogprobs, a->stat_loss,
+                         a->stat_ratio, a->stat_approx_kl, a->clip_mask, a->dual_clip_mask, a->new_mask,
+                         a->behave_imp_weight, a->behave_approx_kl, a->behave_mask, a->results,
+                         a->with_stats ? &sa : nullptr, &more, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"
@@ -856,7 +981,7 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
                     float* stat_ratio, float* stat_approx_kl, uint8_t* clip_mask,
                     uint8_t* dual_clip_mask, uint8_t* new_mask, float* behave_imp_weight,
                     float* behave_approx_kl, uint8_t* behave_mask, double* counters,
-                    const LossStatsArgs* sa, void* workspace, size_t workspace_bytes,
+                    const LossStatsArgs* sa, const LossMore* more, void* workspace, size_t workspace_bytes,
                     hipStream_t stream) {
   if (cfg == nullptr || n_tokens < 0 || counters == nullptr) return AREAL_ERR_BAD_ARG;
   const bool with_stats = sa != nullptr;
@@ -903,6 +1028,12 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
   io.entropy = with_stats ? sa->entropy : nullptr;
   io.extra0 = with_stats ? sa->extra0 : nullptr;
   io.extra1 = with_stats ? sa->extra1 : nullptr;
+  io.stat_prox = with_stats && more != nullptr ? 1 : 0;
+  io.clip_ratio = more != nullptr ? more->clip_ratio : nullptr;
+  io.dual_ratio = more != nullptr ? more->dual_ratio : nullptr;
+  io.logp_diff = more != nullptr ? more->logp_diff : nullptr;
+  io.logp_abs_diff = more != nullptr ? more->logp_abs_diff : nullptr;
+  io.filtered_ratio = more != nullptr ? more->filtered_ratio : nullptr;
 
   // four tokens per thread once that still gives every CU a block; a smaller batch is bound by
   // latency, not by bandwidth, and runs faster spread over four times as many threads
@@ -912,7 +1043,9 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
                     aligned_to(behave_imp_weight, 16) && aligned_to(behave_approx_kl, 16) &&
                     aligned_to(io.entropy, 16) && aligned_to(io.extra0, 16) && aligned_to(io.extra1, 16) &&
                     aligned_to(loss_mask, 4) && aligned_to(clip_mask, 4) && aligned_to(dual_clip_mask, 4) &&
-                    aligned_to(new_mask, 4) && aligned_to(behave_mask, 4);
+                    aligned_to(new_mask, 4) && aligned_to(behave_mask, 4) && aligned_to(io.clip_ratio, 16) &&
+                    aligned_to(io.dual_ratio, 16) && aligned_to(io.logp_diff, 16) &&
+                    aligned_to(io.logp_abs_diff, 16) && aligned_to(io.filtered_ratio, 16);
   // with statistics a block's end costs a third of eight tokens' work per thread: half the blocks
   int grid = loss_grid(n_tokens, vec4 ? 4 : 1);
   if (with_stats && grid > MAX_LOSS_BLOCKS / 2) grid = MAX_LOSS_BLOCKS / 2;
@@ -927,8 +1060,14 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
       hipLaunchKernelGGL((loss_token_kernel<false, 1>), dim3(grid), dim3(LOSS_THREADS), 0, stream, i, cc, partials, (StatPartial*)nullptr);
   };
   if (n_tokens > 0 && c.rs_enabled && c.rs_seq_level) {
-    hipLaunchKernelGGL(seq_rs_kernel, dim3((unsigned)n_seqs), dim3(LOSS_THREADS), 0, stream, io, c,
-                       seq_rs);
+    // below about 1024 tokens a sequence does not give four waves two groups of four per lane
+    const bool short_seqs = n_tokens < n_seqs * 1024;
+    const bool vec = aligned_to(proximal, 16) && aligned_to(old_logprobs, 16) && aligned_to(loss_mask, 4);
+    const dim3 grid_s((unsigned)(short_seqs ? ceil_div_i64(n_seqs, LOSS_THREADS / 64) : n_seqs)), block(LOSS_THREADS);
+    if (short_seqs && vec) hipLaunchKernelGGL((seq_rs_kernel<1, 4>), grid_s, block, 0, stream, io, c, seq_rs);
+    else if (short_seqs) hipLaunchKernelGGL((seq_rs_kernel<1, 1>), grid_s, block, 0, stream, io, c, seq_rs);
+    else if (vec) hipLaunchKernelGGL((seq_rs_kernel<4, 4>), grid_s, block, 0, stream, io, c, seq_rs);
+    else hipLaunchKernelGGL((seq_rs_kernel<4, 1>), grid_s, block, 0, stream, io, c, seq_rs);
     AREAL_CHECK_LAUNCH();
   }
   if (n_tokens > 0 && c.seq_is) {
@@ -945,9 +1084,12 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
   }
   token_pass(io, c, with_stats);
   AREAL_CHECK_LAUNCH();
-  hipLaunchKernelGGL(loss_finalize_kernel, dim3(with_stats ? 1 + N_LOSS_STATS : 1), dim3(FINAL_THREADS), 0, stream,
+  const int n_stats = with_stats ? (more != nullptr ? N_LOSS_STATS : N_LOSS_STATS_V1) : 0;
+  hipLaunchKernelGGL(loss_finalize_kernel, dim3(1 + n_stats), dim3(FINAL_THREADS), 0, stream,
                      partials, stat_partials, grid, loss, counters, (double)n_tokens,
-                     with_stats ? sa->stats : nullptr, c.loss_kind != LOSS_NONE ? 1 : 0, c.rs_enabled);
+                     with_stats ? sa->stats : nullptr, c.loss_kind != LOSS_NONE ? 1 : 0, c.rs_enabled,
+                     more != nullptr ? 1 : 0, more != nullptr ? more->nan_if_bad : 0,
+                     more != nullptr ? more->host : nullptr);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }

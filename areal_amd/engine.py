@@ -14,7 +14,7 @@ from typing import Any
 
 import torch
 
-from areal_amd.functional.lm_head import fused_lm_head_logprobs_entropy
+from areal_amd.functional.lm_head import _lm_head, fused_lm_head_logprobs_entropy
 
 
 def _labels(inputs: dict[str, Any]) -> torch.Tensor:
@@ -120,9 +120,9 @@ class FusedLMHeadAdapter:
     per micro-batch.  Its gradient reaches the fp32 parameter in one of two ways:
 
     * ``fuse_wgrad_accumulation=True`` (default): the dWeight contraction adds into the fp32
-      ``lm_head.weight.grad`` directly (created as zeros when missing), so gradients of several
-      micro-batches accumulate in fp32 without a bf16 ``[V, H]`` intermediate, the arrangement
-      of Megatron's fp32 ``main_grad`` (``vocab_parallel_head.py:873-879``);
+      ``lm_head.weight.grad`` directly (the first one after it was set to ``None`` stores it), so
+      gradients of several micro-batches accumulate in fp32 without a bf16 ``[V, H]`` intermediate,
+      the arrangement of Megatron's fp32 ``main_grad`` (``vocab_parallel_head.py:873-879``);
     * otherwise autograd routes a bf16 ``dWeight`` through the cast back to fp32 and its
       ``AccumulateGrad`` adds it to ``.grad``.
 
@@ -171,12 +171,12 @@ class FusedLMHeadAdapter:
         return self._compute_copy_value
 
     def _weight(self, hidden: torch.Tensor):
-        """(compute copy of lm_head.weight, fp32 accumulator or None)."""
+        """(compute copy of lm_head.weight, fp32 accumulator or None, its owner while it has none)."""
         param = self.module.lm_head.weight
         if param.dtype == self.compute_dtype:
-            return param, None
+            return param, None, None
         if not torch.is_grad_enabled():
-            return self._compute_copy(param), None
+            return self._compute_copy(param), None, None
         fused = (
             self.fuse_wgrad_accumulation
             and param.dtype == torch.float32
@@ -185,10 +185,10 @@ class FusedLMHeadAdapter:
             and hidden.requires_grad  # the backward is reached through the hidden states
         )
         if not fused:
-            return param.to(self.compute_dtype), None  # autograd casts the gradient back
+            return param.to(self.compute_dtype), None, None  # autograd casts the gradient back
         if param.grad is None:
-            param.grad = torch.zeros_like(param, memory_format=torch.contiguous_format)
-        return self._compute_copy(param), param.grad
+            return self._compute_copy(param), None, param
+        return self._compute_copy(param), param.grad, None
 
     def _bias(self):
         return getattr(self.module.lm_head, "bias", None)
@@ -198,7 +198,7 @@ class FusedLMHeadAdapter:
         """Forward-only label log-probabilities (``fsdp_engine.py:2107-2134, 2219-2249``)."""
         with torch.no_grad():
             hidden = self.hidden_states(model_inputs)
-            weight, _ = self._weight(hidden)
+            weight = self._weight(hidden)[0]
             out = fused_lm_head_logprobs_entropy(
                 hidden, weight, _labels(model_inputs), temperature=self.temperature, bias=self._bias()
             )
@@ -216,16 +216,23 @@ class FusedLMHeadAdapter:
         loss_multiplier: float = 1.0,
     ) -> torch.Tensor:
         """Scaled loss of one micro-batch (``fsdp_engine.py:2147-2217``)."""
-        hidden = self.hidden_states(model_inputs)
         local_weight = loss_weight_fn(mb_input)
+        return self._scaled_loss(
+            model_inputs, mb_input, loss_fn, local_weight, total_loss_weight, pad_length, loss_multiplier
+        )
+
+    def _scaled_loss(
+        self, model_inputs, mb_input, loss_fn, local_weight, total_loss_weight, pad_length, loss_multiplier
+    ) -> torch.Tensor:
+        hidden = self.hidden_states(model_inputs)
         if local_weight == 0:
             # zero with a graph edge to the base model and to lm_head.weight
             # (fsdp_engine.py:2158-2159)
             return (hidden.float().mean() + self.module.lm_head.weight[:1].float().mean()) * 0.0
-        weight, accum = self._weight(hidden)
-        out = fused_lm_head_logprobs_entropy(
-            hidden, weight, _labels(model_inputs), temperature=self.temperature, bias=self._bias(),
-            save_probs=self.save_probs, weight_grad_accum=accum,
+        weight, accum, owner = self._weight(hidden)
+        out = _lm_head(
+            hidden, weight, _labels(model_inputs), self.temperature, 1.0, self._bias(), None, self.save_probs,
+            False, accum, owner,
         )
         logprobs, entropy = out.logprobs, out.entropy
         vmin, vmax = out.vocab_min_logits, out.vocab_max_logits
@@ -248,16 +255,19 @@ class FusedLMHeadAdapter:
         pad_length=...)``.  Returns the detached scaled losses."""
         weights = [loss_weight_fn(mb["mb_input"]) for mb in micro_batches]
         dev = next((w.device for w in weights if torch.is_tensor(w)), None)
-        total = torch.stack(
-            [torch.as_tensor(w, device=dev).detach().to(torch.float32) for w in weights]
-        ).sum().clone()
+        stacked = torch.stack([torch.as_tensor(w, device=dev).detach().to(torch.float32) for w in weights])
+        # one read of all weights and their sum: a micro-batch that looked at its own weight would
+        # wait for the backward of the one before
+        *weights, total = torch.cat([stacked.reshape(-1), stacked.sum().reshape(1)]).tolist()
         assert total > 0, "Global total loss weight must be positive after all_reduce"
         losses = []
-        for mb in micro_batches:
-            loss = self.compute_logprobs_and_loss(
-                mb["model_inputs"], mb["mb_input"], loss_fn, loss_weight_fn, total,
-                pad_length=mb.get("pad_length", 0), loss_multiplier=loss_multiplier,
+        param = self.module.lm_head.weight
+        for mb, weight in zip(micro_batches, weights):
+            loss = self._scaled_loss(
+                mb["model_inputs"], mb["mb_input"], loss_fn, weight, total, mb.get("pad_length", 0), loss_multiplier,
             )
             loss.backward()
             losses.append(loss.detach())
+        if param.grad is None and param.requires_grad and self.fuse_wgrad_accumulation and param.dtype == torch.float32:
+            param.grad = torch.zeros_like(param, memory_format=torch.contiguous_format)  # no loss reached it
         return losses

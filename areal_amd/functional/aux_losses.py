@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 
 from areal_amd import _lib
-from areal_amd.functional.functional import _f32, _sequence_layout
+from areal_amd.functional.functional import _f32
 
 
 class _ScaledLoss(torch.autograd.Function):
@@ -87,72 +87,29 @@ def sapo_loss_fn(
             f"Invalid importance_sampling_level: {importance_sampling_level}. "
             "Must be 'token' or 'sequence'."
         )
-    lib = _lib.load()
-    shape = logprobs.shape
     seq_level = importance_sampling_level == "sequence"
-    old, adv = _f32(old_logprobs), _f32(advantages)
-    mask_bool = loss_mask.detach().bool().contiguous().view(-1)
-    dev = _lib.require_gpu(logprobs, old, adv, mask_bool)
-    n = int(mask_bool.numel())
-    cu, n_seqs, uniform_len = (None, 0, 0)
-    if seq_level:
-        cu, n_seqs, uniform_len = _sequence_layout(shape, cu_seqlens, dev)
-
-    names = ("stat_loss", "ratio", "approx_kl", "soft_gate", "gate_pos", "gate_neg")
     red = stat_reduction
-    ent = extras = None
+    extras = list(red.extras.values()) if red is not None else []
+    loss, out, host = _lib.host().sapo_loss(
+        logprobs, old_logprobs, advantages, loss_mask, cu_seqlens, tau_pos, tau_neg, seq_level, red is not None,
+        red.entropy if red is not None else None, extras[0] if extras else None,
+        extras[1] if len(extras) > 1 else None,
+    )
     if red is not None:
-        from areal_amd.functional.functional import SAPO_REDUCED_STAT_KEYS
-
-        extras = [_f32(t) for t in red.extras.values()]
-        ent = _f32(red.entropy) if red.entropy is not None else None
-        for t in extras + ([ent] if ent is not None else []):
-            if t.numel() != n:
-                raise ValueError(f"a statistic rides along with {t.numel()} elements, expected {n}")
-
-    def launch(want_grad: bool):
-        f32 = dict(dtype=torch.float32, device=dev)
-        out = {k: (torch.empty(n, **f32) if red is None else None) for k in names}
-        out["loss"] = torch.empty((), **f32)
-        out["dsum"] = torch.empty(n, **f32) if want_grad else None
-        # counters [8] and, with a reduction, stats [13][4] in one buffer: one copy to the host
-        n_stats = len(SAPO_REDUCED_STAT_KEYS) if red is not None else 0
-        both = torch.empty(8 + 4 * n_stats, dtype=torch.float64, device=dev)
-        out["counters"], out["both"] = both[:8], both
-        nbytes = lib.areal_aux_loss_workspace_bytes(n, n_seqs)
-        ws = _lib.workspace(nbytes, dev)
-        rc = lib.areal_sapo_loss(
-            _lib.ptr(_f32(logprobs)), _lib.ptr(old), _lib.ptr(adv), _lib.ptr(mask_bool),
-            _lib.ptr(cu), n, n_seqs, uniform_len, float(tau_pos), float(tau_neg), int(seq_level),
-            _lib.ptr(out["loss"]), _lib.ptr(out["dsum"]), _lib.ptr(out["stat_loss"]),
-            _lib.ptr(out["ratio"]), _lib.ptr(out["approx_kl"]), _lib.ptr(out["soft_gate"]),
-            _lib.ptr(out["gate_pos"]), _lib.ptr(out["gate_neg"]), _lib.ptr(out["counters"]),
-            _lib.ptr(ent), _lib.ptr(extras[0] if extras else None),
-            _lib.ptr(extras[1] if extras and len(extras) > 1 else None),
-            _lib.ptr(both[8:]) if red is not None else None,
-            _lib.ptr(ws), nbytes, _lib.stream_ptr(dev),
-        )
-        _lib.check(rc, "areal_sapo_loss")
-        return out
-
-    runner = _Launch(launch)
-    loss = _ScaledLoss.apply(logprobs, runner)
-    out = runner.out
-    if red is not None:
-        host = out["both"].cpu()  # the one host synchronisation of the call
-        red._fill_sapo(host[8:].view(-1, 4), host[:8], n)
-        return loss, dict(n_total_tokens=float(n), n_valid_tokens=float(host[1]),
-                          n_masked_tokens=float(n) - float(host[1]),
-                          masked_token_ratio=1.0 - float(host[1]) / max(float(n), 1.0))
+        n = loss_mask.numel()
+        red._fill_sapo(host, n)  # the one wait for the GPU of the call
+        n_valid = red.denominators["n_valid_tokens"]
+        return loss, dict(n_total_tokens=float(n), n_valid_tokens=n_valid, n_masked_tokens=float(n) - n_valid,
+                          masked_token_ratio=1.0 - n_valid / max(float(n), 1.0))
     stat = dict(
-        loss=out["stat_loss"].view(shape),
-        importance_weight=out["ratio"].view(shape),
-        approx_kl=out["approx_kl"].view(shape),
+        loss=out["loss"],
+        importance_weight=out["importance_weight"],
+        approx_kl=out["approx_kl"],
         clip_mask=torch.zeros_like(loss_mask, dtype=torch.bool),
         dual_clip_mask=torch.zeros_like(loss_mask, dtype=torch.bool),
-        sapo_soft_gate=out["soft_gate"].view(shape),
-        sapo_scaled_gate_pos=out["gate_pos"].view(shape),
-        sapo_scaled_gate_neg=out["gate_neg"].view(shape),
+        sapo_soft_gate=out["sapo_soft_gate"],
+        sapo_scaled_gate_pos=out["sapo_scaled_gate_pos"],
+        sapo_scaled_gate_neg=out["sapo_scaled_gate_neg"],
     )
     return loss, stat
 
@@ -171,37 +128,10 @@ def ppo_critic_loss_fn(
     assert target_value.dtype == torch.float32
     if loss_fn_type not in ("huber", "mse"):
         raise NotImplementedError(f"Unknown loss fn type: {loss_fn_type}")
-    lib = _lib.load()
-    shape = value.shape
-    old, target = _f32(old_value), _f32(target_value)
-    mask_bool = loss_mask.detach().bool().contiguous().view(-1) if loss_mask is not None else None
-    dev = _lib.require_gpu(value, old, target, mask_bool)
-    n = int(value.numel())
-
-    def launch(want_grad: bool):
-        out = {
-            "loss": torch.empty((), dtype=torch.float32, device=dev),
-            "dsum": torch.empty(n, dtype=torch.float32, device=dev) if want_grad else None,
-            "stat_loss": torch.empty(n, dtype=torch.float32, device=dev),
-            "clip_mask": torch.empty(n, dtype=torch.bool, device=dev),
-            "counters": torch.empty(8, dtype=torch.float64, device=dev),
-        }
-        nbytes = lib.areal_aux_loss_workspace_bytes(n, 0)
-        ws = _lib.workspace(nbytes, dev)
-        rc = lib.areal_critic_loss(
-            _lib.ptr(_f32(value)), _lib.ptr(old), _lib.ptr(target), _lib.ptr(mask_bool), n,
-            float(value_eps_clip), int(loss_fn_type == "huber"), _lib.ptr(out["loss"]),
-            _lib.ptr(out["dsum"]), _lib.ptr(out["stat_loss"]), _lib.ptr(out["clip_mask"]),
-            _lib.ptr(out["counters"]), _lib.ptr(ws), nbytes, _lib.stream_ptr(dev),
-        )
-        _lib.check(rc, "areal_critic_loss")
-        return out
-
-    runner = _Launch(launch)
-    loss = _ScaledLoss.apply(value, runner)
-    out = runner.out
-    stat = dict(clip_mask=out["clip_mask"].view(shape), loss=out["stat_loss"].view(shape))
-    return loss, stat
+    loss, clip_mask, stat_loss = _lib.host().critic_loss(
+        value, old_value, target_value, loss_mask, value_eps_clip, loss_fn_type == "huber"
+    )
+    return loss, dict(clip_mask=clip_mask, loss=stat_loss)
 
 
 class _SeqLogps(torch.autograd.Function):

@@ -12,6 +12,7 @@ synchronisations.
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import torch
@@ -60,21 +61,6 @@ SAPO_REDUCED_STAT_KEYS = (
 )
 
 
-class _HostCopy:
-    """A small device tensor on its way to pinned host memory: queued behind the kernels that
-    write it, waited for when the host first looks at it."""
-
-    def __init__(self, dev_tensor: torch.Tensor):
-        self._host = torch.empty(dev_tensor.shape, dtype=dev_tensor.dtype, pin_memory=True)
-        self._host.copy_(dev_tensor, non_blocking=True)
-        self._event = torch.cuda.Event()
-        self._event.record(torch.cuda.current_stream(dev_tensor.device))
-
-    def host(self) -> torch.Tensor:
-        self._event.synchronize()
-        return self._host
-
-
 class DeferredFloat:
     """A host scalar of a loss call made with ``defer_host_reads=True``: the device-to-host copy
     it comes from is waited for when the value is first used as a number (``float(x)``,
@@ -82,12 +68,12 @@ class DeferredFloat:
 
     __slots__ = ("_source", "_fn", "_value")
 
-    def __init__(self, source: _HostCopy, fn):
-        self._source, self._fn, self._value = source, fn, None
+    def __init__(self, source, fn):
+        self._source, self._fn, self._value = source, fn, None  # source: a HostResult of csrc/host.cpp
 
     def __float__(self) -> float:
         if self._value is None:
-            self._value = float(self._fn(self._source.host()))
+            self._value = float(self._fn(self._source.value()))
         return self._value
 
     def __repr__(self) -> str:
@@ -137,12 +123,6 @@ class DeferredFloat:
         return other / float(self)
 
 
-def _host_value(c, fn):
-    """``fn(counters)`` as a float now, or as a ``DeferredFloat`` when the counters are still on
-    their way to the host."""
-    return DeferredFloat(c, fn) if isinstance(c, _HostCopy) else float(fn(c))
-
-
 class StatReduction:
     """Ask a loss call to reduce its logged statistics inside the kernel's token pass.
 
@@ -173,20 +153,18 @@ class StatReduction:
         self.behave_mask: torch.Tensor | None = None
         self._results: dict[str, dict[str, float | None]] = {}
         self._denominators: dict[str, float] = {}
-        self._pending = None  # (host copy, arguments of _fill) of a call with deferred host reads
+        self._pending = None  # (host result, arguments of _fill) of a call with deferred host reads
 
     def _resolve(self) -> None:
         if self._pending is not None:
-            copy, n_tokens, has_rs, has_old = self._pending
-            self._pending = None
-            host = copy.host()
-            self._fill(host[8:].view(-1, 4), host[:8], n_tokens, has_rs, has_old)
+            args, self._pending = self._pending, None
+            self._fill(*args)
 
-    def _fill_sapo(self, host: torch.Tensor, counters, n_tokens: int) -> None:
+    def _fill_sapo(self, host, n_tokens: int) -> None:
         """Results of ``areal_sapo_loss``'s reduction. SAPO clips nothing: the clip ratios are
         zero on every token of the mask and the clipped-token statistics are empty."""
-        self._fill(host, counters, n_tokens, False, True, keys=SAPO_REDUCED_STAT_KEYS)
-        nv = float(counters[1])
+        self._fill(host, n_tokens, False, True, keys=SAPO_REDUCED_STAT_KEYS, offset=8)
+        nv = self._denominators["n_valid_tokens"]
         zero = dict(sum=0.0, count=nv, avg=None if nv == 0 else 0.0, min=None if nv == 0 else 0.0,
                     max=None if nv == 0 else 0.0, denominator="n_valid_tokens")
         self._results["clip_ratio"] = dict(zero)
@@ -202,30 +180,34 @@ class StatReduction:
         self._resolve()
         return self._denominators
 
-    def _fill(self, host: torch.Tensor, counters, n_tokens: int, has_rs: bool, has_old: bool,
-              keys=REDUCED_STAT_KEYS) -> None:
-        names = list(self.extras)
-        for i, (key, denom) in enumerate(keys):
-            if key == "entropy" and self.entropy is None:
-                continue
-            if key.startswith("behave_") and not has_rs:
-                continue
-            if key in ("old_logp", "logp_diff", "logp_abs_diff", "clipped_old_logp") and not has_old:
-                continue
-            if key.startswith("extra"):
-                j = int(key[-1])
-                if j >= len(names):
-                    continue
-                key = names[j]
-            s, c, mn, mx = host[i].tolist()
-            empty = c == 0
-            self._results[key] = dict(sum=s, count=c, avg=None if empty else s / c,
-                                     min=None if empty else mn, max=None if empty else mx,
-                                     denominator=denom)
-        self._denominators = dict(n_tokens=float(n_tokens), n_valid_tokens=float(counters[1]),
-                                  clipped_tokens=float(counters[4]), dual_clipped_tokens=float(counters[5]))
+    def _fill(self, host, n_tokens: int, has_rs: bool, has_old: bool, keys=REDUCED_STAT_KEYS, offset: int = 9) -> None:
+        rows = _stat_rows(keys, self.entropy is not None, has_rs, has_old, tuple(self.extras))
+        host.fill(self._results, rows, offset)
+        c = host.value()[:7].tolist()
+        self._denominators = dict(n_tokens=float(n_tokens), n_valid_tokens=c[1], clipped_tokens=c[4],
+                                  dual_clipped_tokens=c[5])
         if has_rs:
-            self._denominators["unclipped_behave_tokens"] = float(counters[6])
+            self._denominators["unclipped_behave_tokens"] = c[6]
+
+
+@functools.lru_cache(maxsize=64)
+def _stat_rows(keys, has_entropy: bool, has_rs: bool, has_old: bool, extras: tuple):
+    """``(row, key, denominator)`` of the statistics a call with these inputs reduces."""
+    rows = []
+    for i, (key, denom) in enumerate(keys):
+        if key == "entropy" and not has_entropy:
+            continue
+        if key.startswith("behave_") and not has_rs:
+            continue
+        if key in ("old_logp", "logp_diff", "logp_abs_diff", "clipped_old_logp") and not has_old:
+            continue
+        if key.startswith("extra"):
+            j = int(key[-1])
+            if j >= len(extras):
+                continue
+            key = extras[j]
+        rows.append((i, key, denom))
+    return rows
 
 
 def _fill_rs(cfg: _lib.LossConfig, rs: RejectionSamplingConfig | None) -> None:
@@ -246,6 +228,10 @@ def _fill_rs(cfg: _lib.LossConfig, rs: RejectionSamplingConfig | None) -> None:
     cfg.rs_lower = rs.lower if rs.lower is not None else 0.0
 
 
+def _native_config(cfg: _lib.LossConfig) -> list:
+    return [getattr(cfg, name) for name, _ in cfg._fields_]
+
+
 def _sequence_layout(shape, cu_seqlens, device):
     """(cu_seqlens int32 tensor or None, n_seqs, uniform_len) for a 1-D or 2-D batch."""
     if len(shape) == 2:
@@ -264,10 +250,8 @@ def _run_loss_kernel(
     mask_bool,
     cu_seqlens,
     want_grad: bool,
-    reduction: "StatReduction | None" = None,
 ):
-    """Launch ``areal_actor_loss`` (or, with a ``reduction``, ``areal_actor_loss_stats`` without
-    the per-token statistic tensors) and return its outputs and the device counters."""
+    """Launch ``areal_actor_loss`` and return its outputs and the device counters."""
     lib = _lib.load()
     dev = _lib.require_gpu(proximal, mask_bool, logprobs, old, advantages)
     n = int(mask_bool.numel())
@@ -278,9 +262,6 @@ def _run_loss_kernel(
     has_loss = cfg.loss_kind != LOSS_NONE
     f32 = dict(dtype=torch.float32, device=dev)
     u8 = dict(dtype=torch.bool, device=dev)
-    if reduction is not None:
-        return _run_loss_kernel_reduced(lib, dev, cfg, n, n_seqs, uniform_len, cu, logprobs, proximal, old,
-                                        advantages, mask_bool, want_grad, reduction)
     out = {
         "loss": torch.empty((), **f32) if has_loss else None,
         "dlp": torch.empty(n, **f32) if (has_loss and want_grad) else None,
@@ -310,85 +291,6 @@ def _run_loss_kernel(
     _lib.check(rc, "areal_actor_loss")
     out["counters_dev"] = counters
     return out
-
-
-def _run_loss_kernel_reduced(lib, dev, cfg, n, n_seqs, uniform_len, cu, logprobs, proximal, old,
-                             advantages, mask_bool, want_grad, reduction):
-    """The loss pass with the statistics reduced in the kernel: the only per-token outputs are
-    the gradient and, for the sequence-level importance ratio under rejection sampling, the
-    narrowed mask and behaviour weight that the per-sequence pass reads back."""
-    f32 = dict(dtype=torch.float32, device=dev)
-    need_seq_io = bool(cfg.rs_enabled and cfg.loss_kind == LOSS_PPO and cfg.seq_is)
-    out = {k: None for k in ("stat_loss", "ratio", "approx_kl", "clip_mask", "dual_clip_mask", "new_mask",
-                             "behave_imp_weight", "behave_approx_kl", "behave_mask")}
-    out["loss"] = torch.empty((), **f32)
-    out["dlp"] = torch.empty(n, **f32) if want_grad else None
-    if need_seq_io:
-        out["new_mask"] = torch.empty(n, dtype=torch.bool, device=dev)
-        out["behave_imp_weight"] = torch.empty(n, **f32)
-    if reduction.keep_behave_mask and cfg.rs_enabled:
-        out["behave_mask"] = reduction.behave_mask = torch.empty(n, dtype=torch.bool, device=dev)
-    # counters [8] and stats [17][4] share one buffer: one device-to-host copy serves both
-    n_stats = len(REDUCED_STAT_KEYS)
-    both = torch.empty(8 + 4 * n_stats, dtype=torch.float64, device=dev)
-    counters, stats = both[:8], both[8:]
-    extras = [_f32(t) for t in reduction.extras.values()]
-    for t in extras:
-        if t.numel() != n:
-            raise ValueError(f"extra statistic has {t.numel()} elements, expected {n}")
-    ent = _f32(reduction.entropy) if reduction.entropy is not None else None
-    if ent is not None and ent.numel() != n:
-        raise ValueError(f"entropy has {ent.numel()} elements, expected {n}")
-    nbytes = lib.areal_actor_loss_stats_workspace_bytes(n, n_seqs)
-    ws = _lib.workspace(nbytes, dev)
-    rc = lib.areal_actor_loss_stats(
-        _lib.ptr(logprobs), _lib.ptr(proximal), _lib.ptr(old), _lib.ptr(advantages),
-        _lib.ptr(mask_bool), _lib.ptr(cu), n, n_seqs, uniform_len, ctypes.byref(cfg),
-        _lib.ptr(ent), _lib.ptr(extras[0] if len(extras) > 0 else None),
-        _lib.ptr(extras[1] if len(extras) > 1 else None),
-        _lib.ptr(out["loss"]), _lib.ptr(out["dlp"]), None, None, None, None, None,
-        _lib.ptr(out["new_mask"]), _lib.ptr(out["behave_imp_weight"]), None, _lib.ptr(out["behave_mask"]),
-        _lib.ptr(counters), _lib.ptr(stats), _lib.ptr(ws), nbytes, _lib.stream_ptr(dev),
-    )
-    _lib.check(rc, "areal_actor_loss_stats")
-    out["counters_dev"] = counters
-    out["counters_and_stats_dev"] = both
-    return out
-
-
-class _ActorLoss(torch.autograd.Function):
-    """loss = sum(where(mask', pg, 0)) / N0 with the closed-form gradient w.r.t. logprobs."""
-
-    @staticmethod
-    def forward(ctx, logprobs, cfg, shape, proximal, old, advantages, mask_bool, cu_seqlens, sink,
-                reduction=None):
-        want_grad = logprobs.requires_grad
-        lp = _f32(logprobs)
-        out = _run_loss_kernel(cfg, shape, lp, proximal, old, advantages, mask_bool, cu_seqlens,
-                               want_grad, reduction)
-        sink.update(out)
-        if want_grad:
-            ctx.save_for_backward(out["dlp"], out["counters_dev"])
-        ctx.shape = logprobs.shape
-        ctx.in_dtype = logprobs.dtype
-        return out["loss"]
-
-    @staticmethod
-    def backward(ctx, grad_loss):
-        dlp, counters = ctx.saved_tensors
-        lib = _lib.load()
-        dev = dlp.device
-        g = grad_loss.detach().to(torch.float32).reshape(1).contiguous()
-        grad = torch.empty_like(dlp)
-        rc = lib.areal_actor_loss_grad(
-            _lib.ptr(dlp), _lib.ptr(g), _lib.ptr(counters), _lib.ptr(grad), dlp.numel(),
-            _lib.stream_ptr(dev),
-        )
-        _lib.check(rc, "areal_actor_loss_grad")
-        grad = grad.view(ctx.shape)
-        if ctx.in_dtype != torch.float32:
-            grad = grad.to(ctx.in_dtype)
-        return (grad,) + (None,) * 9
 
 
 def _check_rs_shapes(proximal_logprobs, old_logprobs, loss_mask):
@@ -452,64 +354,80 @@ def apply_rejection_sampling(
     )
 
 
+# What a loss call returns besides the loss (csrc/host.cpp): nothing, the reference's `stat` dict, that
+# and the further tensors grpo_loss_fn logs, reduced statistics.
+OUT_NONE, OUT_STAT, OUT_LOGGED, OUT_REDUCED = range(4)
+
+
 def _loss_common(cfg, logprobs, proximal_logprobs, old_logprobs, advantages, loss_mask,
-                 rejection_sampling, cu_seqlens, reduction=None, defer=False):
-    shape = logprobs.shape
+                 rejection_sampling, cu_seqlens, reduction, defer, out_mode, nan_if_nonfinite=False):
+    """``(loss, {name: per-token tensor}, host result)``; without ``defer`` the host result has
+    arrived when this returns (the call's one wait for the GPU)."""
     if rejection_sampling is not None:
         _check_rs_shapes(proximal_logprobs, old_logprobs, loss_mask)
         _check_rs_sequences(rejection_sampling, loss_mask, cu_seqlens)
     _fill_rs(cfg, rejection_sampling)
-    mask_bool = loss_mask.detach().bool().contiguous().view(-1)
-    sink: dict = {}
-    # the behaviour log-probs enter the kernel for rejection sampling and, with a reduction,
-    # for the old_logp / logp_diff statistics
-    want_old = rejection_sampling is not None or (reduction is not None and old_logprobs is not None)
-    loss = _ActorLoss.apply(
-        logprobs, cfg, shape, _f32(proximal_logprobs),
-        _f32(old_logprobs) if want_old else None,
-        _f32(advantages), mask_bool, cu_seqlens, sink, reduction,
+    if reduction is not None:
+        out_mode = OUT_REDUCED
+    # the behaviour log-probs enter the kernel for rejection sampling and for the old_logp / logp_diff
+    # statistics
+    want_old = old_logprobs is not None and (rejection_sampling is not None or out_mode >= OUT_LOGGED)
+    extras = list(reduction.extras.values()) if reduction is not None else []
+    loss, out, host = _lib.host().actor_loss(
+        logprobs, proximal_logprobs, old_logprobs if want_old else None, advantages, loss_mask, cu_seqlens,
+        _native_config(cfg), out_mode, reduction is not None and reduction.keep_behave_mask, nan_if_nonfinite,
+        reduction.entropy if reduction is not None else None,
+        extras[0] if len(extras) > 0 else None, extras[1] if len(extras) > 1 else None,
     )
-    if defer:
-        # no host synchronisation in this call: the copy is queued and whoever reads a host
-        # scalar (or the reduction's results) waits for it then
-        if reduction is None:
-            c = _HostCopy(sink["counters_dev"])
+    if reduction is not None:
+        if reduction.keep_behave_mask:
+            reduction.behave_mask = out.get("behave_mask")
+        args = (host, loss_mask.numel(), rejection_sampling is not None, want_old)
+        if defer:
+            reduction._pending = args
         else:
-            c = _HostCopy(sink["counters_and_stats_dev"])
-            reduction._pending = (c, int(mask_bool.numel()), rejection_sampling is not None, want_old)
-    elif reduction is None:
-        c = sink["counters_dev"].cpu()  # the one host synchronisation of the call
-    else:
-        host = sink["counters_and_stats_dev"].cpu()  # counters and reduced statistics, one copy
-        c = host[:8]
-        reduction._fill(host[8:].view(-1, 4), c, int(mask_bool.numel()), rejection_sampling is not None,
-                        want_old)
-    return loss, sink, c, shape
+            reduction._fill(*args)
+    elif not defer:
+        host.value()
+    return loss, out, host
 
 
-def _scalar_stats(loss_mask, c):
+def _scalar_stats(loss_mask, host, defer):
     n_total = float(loss_mask.numel())
+    if not defer:
+        n_valid = host.value()[1].item()
+        return dict(n_total_tokens=n_total, n_valid_tokens=n_valid, n_masked_tokens=n_total - n_valid,
+                    masked_token_ratio=1.0 - n_valid / max(n_total, 1.0))
     return dict(
         n_total_tokens=n_total,
-        n_valid_tokens=_host_value(c, lambda h: h[1]),
-        n_masked_tokens=_host_value(c, lambda h: n_total - float(h[1])),
-        masked_token_ratio=_host_value(c, lambda h: 1.0 - float(h[1]) / max(n_total, 1.0)),
+        n_valid_tokens=DeferredFloat(host, lambda h: h[1]),
+        n_masked_tokens=DeferredFloat(host, lambda h: n_total - float(h[1])),
+        masked_token_ratio=DeferredFloat(host, lambda h: 1.0 - float(h[1]) / max(n_total, 1.0)),
     )
 
 
-def _filtered_fraction(c):
-    return _host_value(c, lambda h: float(h[3]) / max(float(h[1]), 1.0))
+def _filtered_fraction(host, defer):
+    fn = lambda h: float(h[3]) / max(float(h[1]), 1.0)  # noqa: E731
+    return DeferredFloat(host, fn) if defer else fn(host.value())
 
 
-def _rs_stats(stat, sink, c, shape, rejection_sampling):
-    if rejection_sampling is None:
-        return
-    stat.update(
-        behave_approx_kl=sink["behave_approx_kl"].view(shape),
-        behave_imp_weight=sink["behave_imp_weight"].view(shape),
-        behave_mask=sink["behave_mask"].view(shape),
-        filtered_fraction=_filtered_fraction(c),
-    )
+_RS_STATS = ("behave_approx_kl", "behave_imp_weight", "behave_mask")
+
+
+def _check_level(logprobs, importance_sampling_level, cu_seqlens):
+    if importance_sampling_level == "sequence":
+        if logprobs.ndim == 1 and cu_seqlens is None:
+            raise ValueError(
+                "cu_seqlens is required for 1D tensors (packed format). "
+                "In AReaL, 1D tensors are produced by pack_tensor_dict() and always have "
+                "cu_seqlens. For a single sequence, use "
+                "cu_seqlens=torch.tensor([0, seq_len], dtype=torch.int32)."
+            )
+    elif importance_sampling_level != "token":
+        raise ValueError(
+            f"Invalid importance_sampling_level: {importance_sampling_level}. "
+            "Must be 'token' or 'sequence'."
+        )
 
 
 def ppo_actor_loss_fn(
@@ -533,19 +451,18 @@ def ppo_actor_loss_fn(
     statistics in the kernel instead of returning per-token tensors, see ``StatReduction``.
     ``defer_host_reads`` (not in the reference): the call does not wait for the GPU; the host
     scalars of ``stat`` are ``DeferredFloat`` objects that wait when they are first used."""
-    if importance_sampling_level == "sequence":
-        if logprobs.ndim == 1 and cu_seqlens is None:
-            raise ValueError(
-                "cu_seqlens is required for 1D tensors (packed format). "
-                "In AReaL, 1D tensors are produced by pack_tensor_dict() and always have "
-                "cu_seqlens. For a single sequence, use "
-                "cu_seqlens=torch.tensor([0, seq_len], dtype=torch.int32)."
-            )
-    elif importance_sampling_level != "token":
-        raise ValueError(
-            f"Invalid importance_sampling_level: {importance_sampling_level}. "
-            "Must be 'token' or 'sequence'."
-        )
+    loss, stat, _, _ = _ppo_loss(
+        logprobs, proximal_logprobs, old_logprobs, advantages, eps_clip, loss_mask, eps_clip_higher, c_clip,
+        rejection_sampling, importance_sampling_level, cu_seqlens, stat_reduction, defer_host_reads, OUT_STAT,
+    )
+    return loss, stat
+
+
+def _ppo_loss(logprobs, proximal_logprobs, old_logprobs, advantages, eps_clip, loss_mask, eps_clip_higher, c_clip,
+              rejection_sampling, importance_sampling_level, cu_seqlens, stat_reduction, defer, out_mode,
+              nan_if_nonfinite=False):
+    """``ppo_actor_loss_fn`` with the choice of outputs: ``(loss, stat, per-token outputs, host result)``."""
+    _check_level(logprobs, importance_sampling_level, cu_seqlens)
     if c_clip is not None:
         assert c_clip > 1.0, c_clip
     cfg = _lib.LossConfig()
@@ -555,25 +472,23 @@ def ppo_actor_loss_fn(
     cfg.has_c_clip = int(c_clip is not None)
     cfg.c_clip = c_clip if c_clip is not None else 0.0
     cfg.seq_is = int(importance_sampling_level == "sequence")
-    loss, sink, c, shape = _loss_common(
-        cfg, logprobs, proximal_logprobs, old_logprobs, advantages, loss_mask,
-        rejection_sampling, cu_seqlens, stat_reduction, defer_host_reads,
+    loss, out, host = _loss_common(
+        cfg, logprobs, proximal_logprobs, old_logprobs, advantages, loss_mask, rejection_sampling, cu_seqlens,
+        stat_reduction, defer, out_mode, nan_if_nonfinite,
     )
+    if out_mode == OUT_NONE:
+        return loss, None, out, host
     if stat_reduction is not None:
-        stat = _scalar_stats(loss_mask, c)
+        stat = _scalar_stats(loss_mask, host, defer)
+    else:
+        stat = dict(loss=out["loss"], importance_weight=out["importance_weight"], approx_kl=out["approx_kl"],
+                    clip_mask=out["clip_mask"], dual_clip_mask=out["dual_clip_mask"],
+                    **_scalar_stats(loss_mask, host, defer))
         if rejection_sampling is not None:
-            stat["filtered_fraction"] = _filtered_fraction(c)
-        return loss, stat
-    stat = dict(
-        loss=sink["stat_loss"].view(shape),
-        importance_weight=sink["ratio"].view(shape),
-        approx_kl=sink["approx_kl"].view(shape),
-        clip_mask=sink["clip_mask"].view(shape),
-        dual_clip_mask=sink["dual_clip_mask"].view(shape),
-        **_scalar_stats(loss_mask, c),
-    )
-    _rs_stats(stat, sink, c, shape, rejection_sampling)
-    return loss, stat
+            stat.update({k: out[k] for k in _RS_STATS})
+    if rejection_sampling is not None:
+        stat["filtered_fraction"] = _filtered_fraction(host, defer)
+    return loss, stat, out, host
 
 
 def cispo_loss_fn(
@@ -592,6 +507,16 @@ def cispo_loss_fn(
     """CISPO: clipped importance weight under stop-gradient times ``log pi`` (MiniMax-M1).
     Signature, errors and ``stat`` keys as in ``functional.py:678-793``; ``stat_reduction`` and
     ``defer_host_reads`` as in ``ppo_actor_loss_fn``."""
+    loss, stat, _, _ = _cispo_loss(
+        logprobs, proximal_logprobs, advantages, eps_clip, loss_mask, eps_clip_higher, old_logprobs,
+        rejection_sampling, cu_seqlens, stat_reduction, defer_host_reads, OUT_STAT,
+    )
+    return loss, stat
+
+
+def _cispo_loss(logprobs, proximal_logprobs, advantages, eps_clip, loss_mask, eps_clip_higher, old_logprobs,
+                rejection_sampling, cu_seqlens, stat_reduction, defer, out_mode, nan_if_nonfinite=False):
+    """``cispo_loss_fn`` with the choice of outputs, as ``_ppo_loss``."""
     if eps_clip_higher is None or eps_clip_higher <= 0:
         raise ValueError(
             "CISPO requires a positive eps_clip_higher; the asymmetric upper "
@@ -601,24 +526,21 @@ def cispo_loss_fn(
     cfg.loss_kind = LOSS_CISPO
     cfg.clip_lo = 1.0 - eps_clip
     cfg.clip_hi = 1.0 + eps_clip_higher
-    loss, sink, c, shape = _loss_common(
-        cfg, logprobs, proximal_logprobs, old_logprobs, advantages, loss_mask,
-        rejection_sampling, cu_seqlens, stat_reduction, defer_host_reads,
+    loss, out, host = _loss_common(
+        cfg, logprobs, proximal_logprobs, old_logprobs, advantages, loss_mask, rejection_sampling, cu_seqlens,
+        stat_reduction, defer, out_mode, nan_if_nonfinite,
     )
-    if stat_reduction is not None:
-        stat = {}
+    if out_mode == OUT_NONE:
+        return loss, None, out, host
+    stat = {}
+    if stat_reduction is None:
+        stat.update(loss=out["loss"], importance_weight=out["importance_weight"], approx_kl=out["approx_kl"],
+                    clip_mask=out["clip_mask"], dual_clip_mask=out["dual_clip_mask"])
         if rejection_sampling is not None:
-            stat["filtered_fraction"] = _filtered_fraction(c)
-        return loss, stat
-    stat = dict(
-        loss=sink["stat_loss"].view(shape),
-        importance_weight=sink["ratio"].view(shape),
-        approx_kl=sink["approx_kl"].view(shape),
-        clip_mask=sink["clip_mask"].view(shape),
-        dual_clip_mask=torch.zeros(shape, dtype=torch.bool, device=logprobs.device),
-    )
-    _rs_stats(stat, sink, c, shape, rejection_sampling)
-    return loss, stat
+            stat.update({k: out[k] for k in _RS_STATS})
+    if rejection_sampling is not None:
+        stat["filtered_fraction"] = _filtered_fraction(host, defer)
+    return loss, stat, out, host
 
 
 @torch.no_grad()

@@ -4,7 +4,7 @@ Host-side counterpart of the reference's chunked LM head
 (``areal/models/mcore/vocab_parallel_head.py:560-938`` and its wrapper
 ``chunked_lm_head_logprobs_entropy`` at ``:941-982``): same outputs
 (``ChunkedLMHeadOutput``), same error behaviour.  The arithmetic runs in the HIP kernels of
-``csrc/lmhead.hip`` through the C ABI.
+``csrc/lmhead.hip`` through the C ABI, allocation and the autograd node in ``csrc/host.cpp``.
 
 Two ways of carrying state to the backward:
 
@@ -41,17 +41,6 @@ DEFAULT_BWD_WORKSPACE_BYTES = 24 << 30
 SAVE_PROBS_BYTES_LIMIT = 40 << 30
 
 
-def _round_up(x: int, m: int) -> int:
-    return (x + m - 1) // m * m
-
-
-def _available_bytes(dev: torch.device) -> int:
-    """Device memory the allocator can still hand out: free on the device plus what the caching
-    allocator holds but has not given to a tensor."""
-    free, _ = torch.cuda.mem_get_info(dev)
-    return free + torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
-
-
 class ChunkedLMHeadOutput(NamedTuple):
     """Per-token outputs produced without materialising ``[T, V]`` logits.
 
@@ -67,189 +56,37 @@ class ChunkedLMHeadOutput(NamedTuple):
 
 
 def default_token_chunk(T: int, H: int, V: int, budget: int = DEFAULT_BWD_WORKSPACE_BYTES) -> int:
-    """Largest token chunk (multiple of 256) whose backward workspace fits ``budget``: bf16
-    dlogits of the chunk plus the transposed weight (and, when ``T`` is not a multiple of 64,
-    transposed copies of the last chunk's hidden states and dlogits)."""
-    ragged = T % 64 != 0
-    per_token = 2 * V + 64 + (2 * (V + H) if ragged else 0)
-    fixed = 2 * H * (V + 64)
-    chunk = max((budget - fixed) // per_token, 256)
-    chunk = (chunk // 256) * 256
-    return int(min(max(chunk, 256), max(T, 1)))
+    """Largest token chunk (multiple of 256) whose backward workspace fits ``budget``."""
+    return _lib.host().default_token_chunk(T, H, V, budget)
 
 
 class _FusedLMHead(torch.autograd.Function):
+    """The autograd node; its two directions are native (``lm_head`` and ``lm_head_backward`` of
+    ``csrc/host.cpp``).  ``probs``, ``probs_ref`` and ``probs_status`` are the saved exponentials,
+    their row references and whether they are usable, while the node holds them: plain
+    attributes, not saved tensors, because the backward rewrites entries of ``probs`` in place."""
+
     @staticmethod
-    def forward(
-        ctx, hidden, weight, bias, labels, temperature, logit_scale, token_chunk, save_probs,
-        with_moments, weight_grad_accum,
-    ):
-        lib = _lib.load()
-        dev = _lib.require_gpu(hidden, weight, labels, bias)
-        H = hidden.size(-1)
-        V = weight.size(0)
-        hidden_2d = hidden.reshape(-1, H).contiguous()
-        weight_c = weight.contiguous()
-        labels_1d = labels.reshape(-1).to(torch.int64).contiguous()
-        T = hidden_2d.size(0)
-        bias_f = bias.detach().float().contiguous() if bias is not None else None
-
-        # vocabulary mean / norm cost two more operations per logit in the sweep's epilogue: they
-        # are computed only on request
-        outs = [torch.empty(labels.shape, dtype=torch.float32, device=dev) for _ in range(4)]
-        outs += [
-            torch.empty(labels.shape, dtype=torch.float32, device=dev) if with_moments else None
-            for _ in range(2)
-        ]
-        outs += [torch.empty(T, dtype=torch.float32, device=dev) for _ in range(2)]
-        logprobs, entropy, vmin, vmax, vmean, vnorm, row_max, sum_exp = outs
-        # the caller has ruled out no_grad mode
-        needs_grad = any(ctx.needs_input_grad[:2]) or weight_grad_accum is not None
-        if save_probs is None:
-            need = 2 * _round_up(T, 128) * _round_up(V, 64)
-            save_probs = need <= SAVE_PROBS_BYTES_LIMIT and need <= 0.6 * _available_bytes(dev)
-        probs = probs_ref = probs_status = None
-        if save_probs and needs_grad and T > 0:
-            # rows padded to 128, columns to 64: areal_lmhead_probs_bytes(T, V)
-            probs = torch.empty(
-                (_round_up(T, 128), _round_up(V, 64)), dtype=torch.bfloat16, device=dev
-            )
-            probs_ref = torch.empty(T, dtype=torch.float32, device=dev)
-            probs_status = torch.empty(1, dtype=torch.int32, device=dev)
-        ctx.status_host = ctx.status_event = None
-        if T > 0:
-            nbytes = lib.areal_lmhead_fwd_workspace_bytes(T, H, V)
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            rc = lib.areal_lmhead_fwd(
-                _lib.ptr(hidden_2d), _lib.ptr(weight_c), _lib.ptr(bias_f), _lib.ptr(labels_1d),
-                T, H, V, 1.0 / temperature, logit_scale,
-                *[_lib.ptr(o) for o in outs],
-                _lib.ptr(probs), probs.numel() * 2 if probs is not None else 0,
-                _lib.ptr(probs_ref), _lib.ptr(probs_status),
-                _lib.ptr(ws), nbytes, _lib.stream_ptr(dev),
-            )
-            _lib.check(rc, "areal_lmhead_fwd")
-            if probs_status is not None:
-                # Whether every row's saved exponentials are in range travels to pinned host
-                # memory behind the forward, so the backward reads it without a device-to-host
-                # copy of its own between the loss and its first launch.
-                ctx.status_host = torch.empty(1, dtype=torch.int32, pin_memory=True)
-                ctx.status_host.copy_(probs_status, non_blocking=True)
-                ctx.status_event = torch.cuda.Event()
-                ctx.status_event.record(torch.cuda.current_stream(dev))
-
-        ctx.save_for_backward(hidden_2d, weight_c, labels_1d, row_max, sum_exp)
-        # Plain attributes, not saved tensors: the backward rewrites entries of probs in place.
-        ctx.probs = probs
-        ctx.probs_ref = probs_ref
-        ctx.probs_status = probs_status
-        ctx.label_logprobs = logprobs.detach().reshape(-1).clone() if probs is not None else None
-        ctx.bias_f = bias_f
-        ctx.temperature = temperature
-        ctx.logit_scale = logit_scale
-        ctx.token_chunk = token_chunk
-        ctx.hidden_shape = hidden.shape
-        ctx.weight_dtype = weight.dtype
-        ctx.bias_dtype = bias.dtype if bias is not None else None
-        ctx.weight_grad_accum = weight_grad_accum
+    def forward(ctx, hidden, weight, bias, labels, args):
+        # args: a tuple, so that the accumulator and its owner in it are no inputs of the node. The
+        # caller has ruled out no_grad mode.
+        accum, owner = args[5:7]
+        needs_grad = any(ctx.needs_input_grad[:2]) or accum is not None or owner is not None
+        outs, saved, state = _lib.host().lm_head(hidden, weight, bias, labels, *args, True, needs_grad)
+        ctx.save_for_backward(*saved)
+        ctx.state = state
+        ctx.probs, ctx.probs_ref, ctx.probs_status = state.probs, state.probs_ref, state.probs_status
         ctx.set_materialize_grads(False)
-        ctx.mark_non_differentiable(*[o for o in (entropy, vmin, vmax, vmean, vnorm) if o is not None])
-        return tuple(outs[:6])
+        ctx.mark_non_differentiable(*[o for o in outs[1:] if o is not None])
+        return outs
 
     @staticmethod
     def backward(ctx, grad_logprobs, *unused):
-        hidden_2d, weight_c, labels_1d, row_max, sum_exp = ctx.saved_tensors
-        need_h, need_w, need_b = ctx.needs_input_grad[:3]
-        want_h = need_h
-        # dWeight goes straight into the caller's fp32 accumulator when one was given (the master
-        # weight's .grad): the contraction's epilogue adds to it, nothing of size [V, H] is
-        # allocated and no gradient is returned for the weight
-        accum = ctx.weight_grad_accum
-        if accum is not None:
-            need_w = True
-        if grad_logprobs is None or not (need_h or need_w or need_b):
-            return (None,) * 10
-        lib = _lib.load()
-        dev = hidden_2d.device
-        T, H = hidden_2d.shape
-        V = weight_c.size(0)
-        g = grad_logprobs.reshape(-1).to(torch.float32).contiguous()
-        # the kernels need one of dHidden / dWeight as an output; a bias-only request computes dHidden
-        need_h = need_h or (need_b and not need_w)
-        dh = torch.empty_like(hidden_2d) if need_h else None
-        # (zeroed when the kernels add to it, which they do together with the weight accumulator)
-        db32 = None
-        if need_b:
-            db32 = (torch.zeros if accum is not None else torch.empty)(V, dtype=torch.float32, device=dev)
-        probs, probs_ref, probs_status = ctx.probs, ctx.probs_ref, ctx.probs_status
-        # A contraction over the whole batch can store dWeight in bf16 itself: the saved mode always,
-        # the recompute mode when one token chunk covers the batch. Several chunks accumulate in
-        # fp32 and cast at the end.
-        chunk = (ctx.token_chunk or default_token_chunk(T, H, V)) if T > 0 else 1
-        bf16_out = accum is None and T > 0 and ctx.weight_dtype == torch.bfloat16
-        direct = bf16_out and (probs is not None or chunk >= T)
-        dw_direct = torch.empty((V, H), dtype=torch.bfloat16, device=dev) if (need_w and direct) else None
-        dw32 = accum
-        if accum is None and need_w and not direct:
-            dw32 = torch.empty((V, H), dtype=torch.float32, device=dev)
+        if grad_logprobs is None:
+            return (None,) * 5
         ctx.probs = ctx.probs_ref = ctx.probs_status = None  # consumed; a second backward recomputes
-        recompute = probs is None
-        if T == 0:
-            recompute = False
-            if dw32 is not None and accum is None:
-                dw32.zero_()
-            if db32 is not None:
-                db32.zero_()
-        elif probs is not None:
-            # Queued before the host knows whether every row's saved exponentials were in range:
-            # the kernels read that status on the device and return at once if it is set.
-            nbytes = lib.areal_lmhead_bwd_saved_workspace_bytes(T, H, V)
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            rc = lib.areal_lmhead_bwd_saved(
-                _lib.ptr(hidden_2d), _lib.ptr(weight_c), _lib.ptr(labels_1d),
-                _lib.ptr(row_max), _lib.ptr(sum_exp), _lib.ptr(ctx.label_logprobs), _lib.ptr(g),
-                T, H, V, 1.0 / ctx.temperature, ctx.logit_scale,
-                _lib.ptr(probs), probs.numel() * 2, _lib.ptr(probs_ref), _lib.ptr(probs_status),
-                _lib.ptr(dh), _lib.ptr(dw_direct if direct else dw32),
-                2 if direct else (1 if accum is not None else 0),
-                _lib.ptr(db32), _lib.ptr(ws), nbytes, _lib.stream_ptr(dev),
-            )
-            _lib.check(rc, "areal_lmhead_bwd_saved")
-            # The status travelled to pinned memory behind the forward. Looking at it now, with
-            # the launches above already queued, idles nothing; if it was set (a row's maximum
-            # far above its estimate) those launches did nothing and the recompute mode runs.
-            ctx.status_event.synchronize()
-            if int(ctx.status_host[0]) != 0:
-                recompute = True
-                if need_w and direct and chunk < T:
-                    direct, dw_direct = False, None
-                    dw32 = torch.empty((V, H), dtype=torch.float32, device=dev)
-            del probs, probs_ref
-        if recompute:
-            nbytes = lib.areal_lmhead_bwd_workspace_bytes(T, H, V, chunk)
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            rc = lib.areal_lmhead_bwd(
-                _lib.ptr(hidden_2d), _lib.ptr(weight_c), _lib.ptr(ctx.bias_f),
-                _lib.ptr(labels_1d), _lib.ptr(row_max), _lib.ptr(sum_exp), _lib.ptr(g),
-                T, H, V, 1.0 / ctx.temperature, ctx.logit_scale,
-                _lib.ptr(dh), _lib.ptr(dw_direct if direct else dw32), _lib.ptr(db32),
-                2 if direct else (1 if accum is not None else 0), chunk,
-                _lib.ptr(ws), nbytes, _lib.stream_ptr(dev),
-            )
-            _lib.check(rc, "areal_lmhead_bwd")
-        dw = dw_direct
-        if dw32 is not None and accum is None:
-            if ctx.weight_dtype == torch.float32:
-                dw = dw32
-            else:
-                dw = torch.empty((V, H), dtype=ctx.weight_dtype, device=dev)
-                rc = lib.areal_cast_f32_to_bf16(
-                    _lib.ptr(dw32), _lib.ptr(dw), dw32.numel(), _lib.stream_ptr(dev)
-                )
-                _lib.check(rc, "areal_cast_f32_to_bf16")
-        dh = dh.view(ctx.hidden_shape) if (dh is not None and want_h) else None
-        db = db32.to(ctx.bias_dtype) if db32 is not None else None
-        return dh, dw, db, None, None, None, None, None, None, None
+        grads = _lib.host().lm_head_backward(ctx.state, ctx.saved_tensors, grad_logprobs, *ctx.needs_input_grad[:3])
+        return (*grads, None, None)
 
 
 def fused_lm_head_logprobs_entropy(
@@ -293,6 +130,18 @@ def fused_lm_head_logprobs_entropy(
     reference (``vocab_parallel_head.py:732-734``).
     """
     del vocab_chunk
+    return _lm_head(
+        hidden, weight, labels, temperature, logit_scale, bias, token_chunk, save_probs, with_moments,
+        weight_grad_accum, None,
+    )
+
+
+def _lm_head(
+    hidden, weight, labels, temperature, logit_scale, bias, token_chunk, save_probs, with_moments,
+    weight_grad_accum, weight_grad_owner,
+) -> ChunkedLMHeadOutput:
+    """``weight_grad_owner``: the fp32 parameter ``weight`` is a compute copy of; the weight gradient
+    is added to its ``.grad`` as it is when the backward runs, or becomes it."""
     if not math.isfinite(temperature) or temperature <= 0:
         raise ValueError(f"temperature must be positive, got {temperature}")
     if not math.isfinite(logit_scale) or logit_scale <= 0:
@@ -330,11 +179,15 @@ def fused_lm_head_logprobs_entropy(
             raise ValueError("weight_grad_accum must be contiguous")
     if not torch.is_grad_enabled():
         save_probs = False  # no backward will come: keep nothing
-        weight_grad_accum = None
-    values = _FusedLMHead.apply(
-        hidden, weight, bias, labels, float(temperature), float(logit_scale), token_chunk,
-        save_probs, bool(with_moments), weight_grad_accum,
+        weight_grad_accum = weight_grad_owner = None
+    args = (
+        temperature, logit_scale, token_chunk or 0, -1 if save_probs is None else int(save_probs), with_moments,
+        weight_grad_accum, weight_grad_owner, SAVE_PROBS_BYTES_LIMIT, DEFAULT_BWD_WORKSPACE_BYTES,
     )
+    if torch.is_grad_enabled():
+        values = _FusedLMHead.apply(hidden, weight, bias, labels, args)
+    else:
+        values = _lib.host().lm_head(hidden, weight, bias, labels, *args, False, False)
     return ChunkedLMHeadOutput(*values)
 
 

@@ -20,8 +20,12 @@ from areal_amd.data import KLEstimator, Normalization
 from areal_amd import _lib
 from areal_amd.functional.aux_losses import _Launch, _ScaledLoss, sapo_loss_fn
 from areal_amd.functional.functional import (
-    cispo_loss_fn,
-    ppo_actor_loss_fn,
+    OUT_LOGGED,
+    OUT_NONE,
+    OUT_REDUCED,
+    StatReduction,
+    _cispo_loss,
+    _ppo_loss,
     reward_overlong_penalty,
 )
 from areal_amd.ppo.gae import (
@@ -98,13 +102,15 @@ def grpo_loss_fn(
     if stats_mode not in ("tensors", "reduced"):
         raise ValueError(f"stats_mode must be 'tensors' or 'reduced', got {stats_mode!r}")
     reduction = None
+    versions = input_data.get("versions")
+    # with token versions the reduced mode evaluates further per-token tensors under the behave mask
+    versioned = versions is not None and current_version is not None
     if stats is not None and stats_mode == "reduced":
-        from areal_amd.functional.functional import StatReduction
-
         extras = {}
         if vocab_min_logits is not None and vocab_max_logits is not None:
             extras = dict(vocab_min_logits=vocab_min_logits, vocab_max_logits=vocab_max_logits)
-        reduction = StatReduction(entropy=entropy, extras=extras, keep_behave_mask=True)
+        reduction = StatReduction(entropy=entropy, extras=extras, keep_behave_mask=versioned)
+    out_mode = OUT_NONE if stats is None else (OUT_REDUCED if reduction is not None else OUT_LOGGED)
     if prox_logp_method not in PROX_LOGP_METHODS_ALL:
         raise ValueError(f"'{prox_logp_method}' is not a valid ProxLogpMethod")
     old_logp = input_data["logprobs"]
@@ -120,17 +126,17 @@ def grpo_loss_fn(
         prox_logp_method=prox_logp_method,
         old_logp=old_logp,
         logprobs=logprobs.detach(),
-        versions=input_data.get("versions"),
+        versions=versions,
         current_version=current_version,
     )
 
     # The reference stops here when the proximal log-probs hold a NaN or Inf (actor.py:924-928),
-    # which costs a host synchronisation before any loss kernel is queued. The same check runs
-    # on the device now and is read after the loss call's own synchronisation: same error, one
-    # idle gap of the GPU less per micro-batch.
-    prox_nonfinite = torch.isfinite(prox_logp).logical_not().any()
-    if not prox_logp.is_cuda:  # nothing to overlap with: report at once
-        _raise_if_nonfinite(prox_nonfinite, prox_logp_method)
+    # which costs a host synchronisation before any loss kernel is queued. The loss kernel counts
+    # such tokens in its own pass instead and the count comes back with its other counters: same
+    # error, no pass over the log-probs of its own. With deferred host reads it makes the loss NaN.
+    if not prox_logp.is_cuda:  # no kernel will look at it: report at once
+        _raise_if_nonfinite(torch.isfinite(prox_logp).logical_not().any(), prox_logp_method)
+    defer = defer_host_reads and not use_sapo_loss
 
     if m2_threshold is not None:
         loss_mask = _apply_m2po_masking(old_logp, prox_logp, loss_mask, m2_threshold)
@@ -146,18 +152,9 @@ def grpo_loss_fn(
                 "CISPO only supports importance_sampling_level='token'. "
                 "Sequence-level (GSPO-style) CISPO has no published surrogate."
             )
-        loss, stat = cispo_loss_fn(
-            logprobs=logprobs,
-            proximal_logprobs=prox_logp,
-            advantages=advantages,
-            eps_clip=eps_clip,
-            eps_clip_higher=eps_clip_higher,
-            loss_mask=loss_mask,
-            old_logprobs=old_logp,
-            rejection_sampling=rejection_sampling,
-            cu_seqlens=input_data.get("cu_seqlens"),
-            stat_reduction=reduction,
-            defer_host_reads=defer_host_reads,
+        loss, stat, out, host = _cispo_loss(
+            logprobs, prox_logp, advantages, eps_clip, loss_mask, eps_clip_higher, old_logp, rejection_sampling,
+            input_data.get("cu_seqlens"), reduction, defer, out_mode, nan_if_nonfinite=defer,
         )
     elif use_sapo_loss:
         if use_decoupled_loss:
@@ -165,6 +162,8 @@ def grpo_loss_fn(
                 "SAPO is not compatible with `use_decoupled_loss=True`. "
                 "Please set `actor.use_decoupled_loss=false` in your configuration."
             )
+        out = None
+        host = _lib.host().proximal_stats(prox_logp, loss_mask)
         loss, stat = sapo_loss_fn(
             logprobs=logprobs,
             old_logprobs=old_logp,
@@ -177,26 +176,14 @@ def grpo_loss_fn(
             stat_reduction=reduction,
         )
     else:
-        loss, stat = ppo_actor_loss_fn(
-            logprobs=logprobs,
-            old_logprobs=old_logp,
-            advantages=advantages,
-            eps_clip=eps_clip,
-            eps_clip_higher=eps_clip_higher,
-            loss_mask=loss_mask,
-            c_clip=c_clip,
-            proximal_logprobs=prox_logp,
-            rejection_sampling=rejection_sampling,
-            importance_sampling_level=importance_sampling_level,
-            cu_seqlens=input_data.get("cu_seqlens"),
-            stat_reduction=reduction,
-            defer_host_reads=defer_host_reads,
+        loss, stat, out, host = _ppo_loss(
+            logprobs, prox_logp, old_logp, advantages, eps_clip, loss_mask, eps_clip_higher, c_clip,
+            rejection_sampling, importance_sampling_level, input_data.get("cu_seqlens"), reduction, defer, out_mode,
+            nan_if_nonfinite=defer,
         )
 
-    if defer_host_reads and not use_sapo_loss:
-        loss = loss + torch.where(prox_nonfinite, float("nan"), 0.0).to(loss.dtype)
-    else:
-        _raise_if_nonfinite(prox_nonfinite, prox_logp_method)
+    if not defer:
+        _raise_if_nonfinite(host.value()[8] > 0, prox_logp_method)
 
     # joint distillation (actor.py:629-658)
     teacher_logp = input_data.get("teacher_logp")
@@ -214,37 +201,29 @@ def grpo_loss_fn(
             rkl_stat = term
 
     if reduction is not None:
-        defer = defer_host_reads and not use_sapo_loss
         if defer:
             stats["reduction"] = reduction
         else:
             stats.update(reduction.results)
             for name, count in reduction.denominators.items():
                 stats["denominator/" + name] = count
-        # the compute_logp diagnostics: per-token tensors as in the other mode, reduced right away
-        from areal_amd.stats import masked_stats
-
-        lp = logprobs.detach()
-        diag_mask = reduction.behave_mask if reduction.behave_mask is not None else loss_mask
-        diag: dict = {}
-        _collect_proximal_approximation_stats(
-            diag, prox_logp_method, prox_logp_gt, old_logp, lp, input_data.get("versions"),
-            current_version, diag_mask.view(loss_mask.shape),
-        )
-        den = diag.pop("compute_logp/n_valid_tokens")
-        if diag:
-            reduced = masked_stats(diag, {k: den for k in diag}, defer=defer)
+        if versioned:
+            _reduce_versioned_stats(
+                stats, prox_logp_method, prox_logp_gt, old_logp, logprobs.detach(), versions, current_version,
+                reduction, loss_mask, defer,
+            )
+        elif prox_logp_gt is not None:
+            # the one diagnostic that is left was reduced in the loss kernel's pass
             if defer:
-                stats["compute_logp_reduction"] = reduced
+                stats["compute_logp_reduction"] = _ProximalStats(host)
             else:
-                for k, v in reduced.items():
-                    stats[k] = dict(v, denominator="compute_logp/n_valid_tokens")
-                stats["denominator/compute_logp/n_valid_tokens"] = next(iter(reduced.values()))["count"]
-        if "versions" in input_data and current_version is not None and not defer:
-            _collect_version_staleness_stats(stats, input_data["versions"], current_version, diag_mask.view(loss_mask.shape))
+                host.fill(stats, _PROX_STAT_ROWS, 9)
+                stats["denominator/compute_logp/n_valid_tokens"] = stats["compute_logp/prox_logp_gt"]["count"]
         if vocab_mean_logits is not None or vocab_norm_logits is not None:
             more = {k: v for k, v in (("vocab_mean_logits", vocab_mean_logits), ("vocab_norm_logits", vocab_norm_logits))
                     if v is not None}
+            from areal_amd.stats import masked_stats
+
             extra = masked_stats(more, {k: None for k in more}, defer=defer)
             if defer:
                 stats["vocab_moments_reduction"] = extra
@@ -260,7 +239,10 @@ def grpo_loss_fn(
             stats["rkl_loss"] = rkl_stat
     elif stats is not None:
         lp = logprobs.detach()
-        logp_diff = (old_logp - lp) * loss_mask
+        if out is None:
+            logp_diff = (old_logp - lp) * loss_mask
+            out = dict(clip_ratio=stat["clip_mask"].float(), dual_clip_ratio=stat["dual_clip_mask"].float(),
+                       logp_diff=logp_diff, logp_abs_diff=logp_diff.abs())
         stats.update(
             n_valid_tokens=loss_mask,
             clipped_tokens=stat["clip_mask"],
@@ -271,17 +253,17 @@ def grpo_loss_fn(
             old_logp=old_logp,
             entropy=entropy.float(),
             actor_loss=stat["loss"],
-            clip_ratio=stat["clip_mask"].float(),
-            dual_clip_ratio=stat["dual_clip_mask"].float(),
-            logp_diff=logp_diff,
-            logp_abs_diff=logp_diff.abs(),
+            clip_ratio=out["clip_ratio"],
+            dual_clip_ratio=out["dual_clip_ratio"],
+            logp_diff=out["logp_diff"],
+            logp_abs_diff=out["logp_abs_diff"],
         )
         if "behave_imp_weight" in stat:
             stats.update(
                 unclipped_behave_tokens=stat["behave_mask"],
                 behave_imp_weight=stat["behave_imp_weight"],
                 behave_approx_kl=stat["behave_approx_kl"],
-                behave_filtered_ratio=(loss_mask & ~stat["behave_mask"]).float(),
+                behave_filtered_ratio=out["behave_filtered_ratio"],
             )
         for key in ("n_total_tokens", "n_valid_tokens", "n_masked_tokens", "masked_token_ratio"):
             if key in stat:
@@ -300,8 +282,7 @@ def grpo_loss_fn(
             )
         compute_logp_mask = stat.get("behave_mask", loss_mask)
         _collect_proximal_approximation_stats(
-            stats, prox_logp_method, prox_logp_gt, old_logp, lp, input_data.get("versions"),
-            current_version, compute_logp_mask,
+            stats, prox_logp_method, prox_logp_gt, old_logp, lp, versions, current_version, compute_logp_mask,
         )
         if "versions" in input_data and current_version is not None:
             _collect_version_staleness_stats(stats, input_data["versions"], current_version, compute_logp_mask)
@@ -310,6 +291,51 @@ def grpo_loss_fn(
         if vocab_norm_logits is not None:
             stats["vocab_norm_logits"] = vocab_norm_logits
     return loss
+
+
+# row of the proximal log-probs among the reduced statistics of areal_actor_loss_call
+_PROX_STAT_ROWS = [(17, "compute_logp/prox_logp_gt", "compute_logp/n_valid_tokens")]
+
+
+class _ProximalStats:
+    """``masked_stats({"compute_logp/prox_logp_gt": ...}, defer=True)`` from a loss call's own results."""
+
+    def __init__(self, host):
+        self._host = host
+        self._results = None
+
+    @property
+    def results(self) -> dict[str, dict[str, float | None]]:
+        if self._results is None:
+            out: dict = {}
+            self._host.fill(out, _PROX_STAT_ROWS, 9)
+            for v in out.values():
+                del v["denominator"]
+            self._results = out
+        return self._results
+
+
+def _reduce_versioned_stats(stats, prox_logp_method, prox_logp_gt, old_logp, lp, versions, current_version, reduction,
+                            loss_mask, defer) -> None:
+    """The ``compute_logp/...`` diagnostics and the staleness scalars of the reduced mode: per-token
+    tensors as in the other mode, reduced right away."""
+    from areal_amd.stats import masked_stats
+
+    mask = reduction.behave_mask if reduction.behave_mask is not None else loss_mask
+    mask = mask.view(loss_mask.shape)
+    diag: dict = {}
+    _collect_proximal_approximation_stats(
+        diag, prox_logp_method, prox_logp_gt, old_logp, lp, versions, current_version, mask
+    )
+    den = diag.pop("compute_logp/n_valid_tokens")
+    reduced = masked_stats(diag, {k: den for k in diag}, defer=defer)
+    if defer:
+        stats["compute_logp_reduction"] = reduced
+        return
+    for k, v in reduced.items():
+        stats[k] = dict(v, denominator="compute_logp/n_valid_tokens")
+    stats["denominator/compute_logp/n_valid_tokens"] = next(iter(reduced.values()))["count"]
+    _collect_version_staleness_stats(stats, versions, current_version, mask)
 
 
 def compute_prox_logp_approximations(

@@ -82,6 +82,18 @@ int areal_lmhead_fwd(const void* hidden, const void* weight, const float* bias,
                      float* probs_ref, int* probs_status, void* workspace, size_t workspace_bytes,
                      areal_stream_t stream);
 
+/* areal_lmhead_fwd with two more outputs (NULL allowed): logprobs_copy [T], the label
+ * log-probabilities once more, and host_status, an int in pinned host memory that receives
+ * *probs_status from the call's last kernel (its value before is for the caller to choose, so that
+ * the caller can see when it has arrived). */
+int areal_lmhead_fwd_ex(const void* hidden, const void* weight, const float* bias,
+                        const int64_t* labels, int64_t T, int64_t H, int64_t V,
+                        float inv_temperature, float logit_scale, float* logprobs, float* entropy,
+                        float* vocab_min, float* vocab_max, float* vocab_mean, float* vocab_norm,
+                        float* row_max, float* sum_exp, void* probs, size_t probs_bytes,
+                        float* probs_ref, int* probs_status, float* logprobs_copy, int* host_status,
+                        void* workspace, size_t workspace_bytes, areal_stream_t stream);
+
 size_t areal_lmhead_bwd_workspace_bytes(int64_t T, int64_t H, int64_t V, int64_t token_chunk);
 
 /* grad_logprobs [T] fp32. Writes dhidden [T,H] bf16 (NULL to skip) and dweight [V,H] (NULL to
@@ -220,6 +232,37 @@ int areal_actor_loss_stats(const float* logprobs, const float* proximal_logprobs
                            uint8_t* new_mask, float* behave_imp_weight, float* behave_approx_kl,
                            uint8_t* behave_mask, double* counters, double* stats, void* workspace,
                            size_t workspace_bytes, areal_stream_t stream);
+
+/* areal_actor_loss with every optional input and output in one struct (all fp32 / byte arrays of
+ * n_tokens; any output but `results` may be NULL; unused inputs NULL), and with what grpo_loss_fn
+ * (areal/trainer/ppo/actor.py:527-760) does around it folded in:
+ *   clip_ratio .. behave_filtered_ratio: the masks it logs as fp32 and the log-prob differences
+ *     under the loss mask (logp_diff set: clip_ratio, dual_clip_ratio, logp_abs_diff as well, and
+ *     old_logprobs; behave_filtered_ratio is written under rejection sampling only);
+ *   results [9 + 18 * 4] double: the 8 counters of areal_actor_loss, the number of tokens whose
+ *     proximal log-prob is not finite (actor.py:924-928), and with with_stats the statistics of
+ *     areal_actor_loss_stats followed by proximal_logprobs under the behave mask (without
+ *     rejection sampling: the loss mask);
+ *   host_results (NULL allowed): the same values in pinned host memory, written by the kernels;
+ *   nan_if_nonfinite: the loss is NaN when a proximal log-prob is not finite.
+ * Workspace as areal_actor_loss_workspace_bytes, with with_stats areal_actor_loss_stats_workspace_bytes. */
+typedef struct {
+  const float *logprobs, *proximal_logprobs, *old_logprobs, *advantages;
+  const uint8_t* loss_mask;
+  const int32_t* cu_seqlens;
+  const float *entropy, *extra0, *extra1;
+  int64_t n_tokens, n_seqs, uniform_len;
+  float *loss, *dlogprobs, *stat_loss, *stat_ratio, *stat_approx_kl;
+  uint8_t *clip_mask, *dual_clip_mask, *new_mask;
+  float *behave_imp_weight, *behave_approx_kl;
+  uint8_t* behave_mask;
+  float *clip_ratio, *dual_clip_ratio, *logp_diff, *logp_abs_diff, *behave_filtered_ratio;
+  double* results;
+  double* host_results;
+  int with_stats, nan_if_nonfinite;
+} areal_actor_loss_io;
+int areal_actor_loss_call(const areal_actor_loss_io* io, const areal_loss_config* cfg, void* workspace,
+                          size_t workspace_bytes, areal_stream_t stream);
 
 /* areal_actor_loss without the workspace argument: the block partials and per-sequence
  * aggregates live in a static device array inside the library (about 1.7 MB per GPU, held until
