@@ -168,8 +168,9 @@ DEVI float wave_min(float v) { return wave_reduce(v, [](float a, float b) { retu
 
 // #{i in [0, n) : ends[i] <= x} for a non-decreasing array, by one wave: every round probes 64
 // positions and keeps the gap after the last probe that is <= x.
+// (I: a pointer, or anything with operator[])
 template <class I>
-DEVI int wave_count_le(const I* ends, int n, int64_t x, int lane) {
+DEVI int wave_count_le(I ends, int n, int64_t x, int lane) {
   int base = 0, len = n;
   while (len > 0) {
     const int step = (len + 63) >> 6;

@@ -145,7 +145,17 @@ struct GaeArgs {
   int n_groups;
   double* seg_stats;
   int64_t seg_slots;
+  const int64_t* gseq;       // the groups' first sequences [G+1] instead of their token offsets (goff null)
 };
+// Token offset of the first token of a group; as an array of the groups' ends from index 1 on.
+struct GroupOffsets {
+  const int64_t* goff;
+  const int64_t* gseq;
+  const int32_t* cu;
+  int shift;
+  DEVI int64_t operator[](int j) const { return goff != nullptr ? goff[j + shift] : (int64_t)cu[gseq[j + shift]]; }
+};
+DEVI GroupOffsets group_offsets(const GaeArgs& g, int shift = 0) { return GroupOffsets{g.goff, g.gseq, g.cu, shift}; }
 
 DEVI int gae_seq_of(const GaeArgs& g, int64_t t) {
   if (g.uniform_len > 0) return (int)(t / g.uniform_len);
@@ -338,7 +348,7 @@ __global__ __launch_bounds__(GAE_THREADS) void gae_apply_kernel(GaeArgs g, const
 // by the state leaving it on the left. rs: the row sums of GaeArgs::row_stats (STATS only).
 // oa receives the advantages of the thread's owned tokens (zero elsewhere).
 // The thread's 8 consecutive tokens from t0 (a multiple of 8) as raw inputs; zeros where `want`
-// is false and beyond the array.
+// is false and beyond the array. Without values (no critic) they are zero too.
 DEVI void gae_load_items(const GaeArgs& g, int64_t t0, bool want, float (&rw)[GAE_ITEMS],
                          float (&v)[GAE_ITEMS], float (&ms)[GAE_ITEMS]) {
 #pragma unroll
@@ -348,7 +358,8 @@ DEVI void gae_load_items(const GaeArgs& g, int64_t t0, bool want, float (&rw)[GA
 #pragma unroll
     for (int q = 0; q < GAE_ITEMS / 4; ++q) {
       const f32x4 a = *(const f32x4*)(g.rewards + t0 + 4 * q);
-      const f32x4 b = *(const f32x4*)(g.values + t0 + 4 * q);
+      f32x4 b = {0.f, 0.f, 0.f, 0.f};
+      if (g.values != nullptr) b = *(const f32x4*)(g.values + t0 + 4 * q);
       const f32x4 c = *(const f32x4*)(g.mask + t0 + 4 * q);
 #pragma unroll
       for (int e = 0; e < 4; ++e) { rw[4 * q + e] = a[e]; v[4 * q + e] = b[e]; ms[4 * q + e] = c[e]; }
@@ -358,7 +369,7 @@ DEVI void gae_load_items(const GaeArgs& g, int64_t t0, bool want, float (&rw)[GA
     for (int i = 0; i < GAE_ITEMS; ++i) {
       const bool in = t0 + i < g.n;
       rw[i] = in ? g.rewards[t0 + i] : 0.f;
-      v[i] = in ? g.values[t0 + i] : 0.f;
+      v[i] = in && g.values != nullptr ? g.values[t0 + i] : 0.f;
       ms[i] = in ? g.mask[t0 + i] : 0.f;
     }
   }
@@ -595,7 +606,7 @@ DEVI void gae_tile_group_search(const GaeArgs& g, int64_t lo, int64_t hi, int* s
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (wave < 3) {
     const int64_t x = wave == 0 ? lo : (wave == 1 ? hi - 1 : hi);
-    const int r = wave_count_le(g.goff + 1, g.n_groups, x, lane);
+    const int r = wave_count_le(group_offsets(g, 1), g.n_groups, x, lane);
     if (lane == 0) s_grp[wave] = r;
   }
 }
@@ -614,7 +625,7 @@ DEVI GaeTileGroups gae_tile_groups(const GaeArgs& g, int64_t lo, const int* s_gr
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const int j = r.g_first + i <= g.n_groups ? r.g_first + i : g.n_groups;
-    r.b[i] = g.goff[j] - lo;
+    r.b[i] = group_offsets(g)[j] - lo;
   }
   return r;
 }
@@ -638,8 +649,8 @@ DEVI void gae_tile_group_stats(const GaeArgs& g, int64_t tile, int64_t lo, int64
     const int k = gi - tg.g_first;
     // the group's bounds relative to the thread's tokens, clamped to them
     // (selects, not an index: an indexed register array would live in scratch memory)
-    const int64_t d0 = (k == 0 ? tg.b[0] : k == 1 ? tg.b[1] : k == 2 ? tg.b[2] : g.goff[gi] - lo) - rel;
-    const int64_t d1 = (k == 0 ? tg.b[1] : k == 1 ? tg.b[2] : g.goff[gi + 1] - lo) - rel;
+    const int64_t d0 = (k == 0 ? tg.b[0] : k == 1 ? tg.b[1] : k == 2 ? tg.b[2] : group_offsets(g)[gi] - lo) - rel;
+    const int64_t d1 = (k == 0 ? tg.b[1] : k == 1 ? tg.b[2] : group_offsets(g)[gi + 1] - lo) - rel;
     const int i0 = d0 <= 0 ? 0 : (d0 >= GAE_ITEMS ? GAE_ITEMS : (int)d0);
     const int i1 = d1 <= 0 ? 0 : (d1 >= GAE_ITEMS ? GAE_ITEMS : (int)d1);
     double rs[5];
@@ -1061,6 +1072,63 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_stats5_kernel(NormArgs a) {
   }
 }
 
+// What the elements of group g are normalised with, from the five sums of the group (v[0..4]) and of the
+// batch (v[5..9]; only v[5] unless a level is "batch"); no leave-one-out here.
+struct NormParams {
+  double mean, std_d, eps;
+  bool mean64, std64;
+};
+DEVI NormParams norm_params(const NormArgs& a, int g, const double (&v)[10]) {
+  // mean context (see make_mean_ctx)
+  MeanCtx mc;
+  mc.level = a.mean_level; mc.identity = false; mc.zero = false; mc.loo = false; mc.cnt = 0.0; mc.sum = 0.0;
+  if (a.mean_level == LEVEL_BATCH) { mc.cnt = v[5]; mc.sum = v[6]; if (mc.cnt == 0.0) mc.zero = true; }
+  else if (a.mean_level == LEVEL_GROUP) {
+    if (g == a.tail_group) mc.zero = true;
+    else { mc.cnt = v[0]; mc.sum = v[1]; if (mc.cnt == 0.0) mc.zero = true; }
+  } else mc.zero = true;
+  NormParams np;
+  np.mean = elem_mean(mc, 0.f, 1.f, false);  // one value for the whole group
+  const double mean = np.mean;
+  auto ss_of = [&](double s2, double s3, double s4) {
+    const double ss = s4 - 2.0 * mean * s3 + mean * mean * s2;
+    return ss > 0.0 ? ss : 0.0;
+  };
+  double std_d = 1.0;
+  np.eps = a.eps;
+  if (a.std_level == LEVEL_BATCH) {
+    const double cnt = v[5], ss = ss_of(v[7], v[8], v[9]);
+    if (a.unbiased) std_d = cnt <= 1.0 ? 1.0 : sqrt(ss / (cnt - 1.0));
+    else std_d = cnt == 0.0 ? 1.0 : sqrt(ss / cnt);
+  } else if (a.std_level == LEVEL_GROUP) {
+    if (g == a.tail_group) std_d = 0.0;
+    else if (a.grows[g] == 1 && a.unbiased) std_d = 1.0;
+    else {
+      const double cnt = v[0], ss = ss_of(v[2], v[3], v[4]);
+      if (a.unbiased) std_d = cnt <= 1.0 ? 1.0 : sqrt(ss / (cnt - 1.0));
+      else std_d = cnt == 0.0 ? 1.0 : sqrt(ss / cnt);
+    }
+    std_d = (double)(float)std_d;
+  } else {
+    np.eps = 0.0;
+  }
+  np.std_d = std_d;
+  np.mean64 = a.mean_level == LEVEL_BATCH;
+  np.std64 = a.std_level == LEVEL_BATCH;
+  return np;
+}
+DEVI float norm_one(const NormParams& p, float x, float m, bool has_mask) {
+  if (p.mean64 || p.std64) {
+    double c = p.mean64 ? ((double)x - p.mean) : (double)(x - (float)p.mean);
+    if (has_mask) c = p.mean64 ? c * (double)m : (double)((float)c * m);
+    const double den = p.std64 ? (p.std_d + p.eps) : (double)((float)p.std_d + (float)p.eps);
+    return (float)(c / den);
+  }
+  float c = x - (float)p.mean;
+  if (has_mask) c = c * m;
+  return c / ((float)p.std_d + (float)p.eps);
+}
+
 // Apply pass of the two-launch form. Every block first sums what it needs of the five partial
 // arrays in one cooperative sweep (its group's five sums; the batch's count, or all five batch
 // sums when a level is "batch") and one fused block reduction, then derives the mean and the
@@ -1148,49 +1216,8 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_apply_cf_kernel(NormArgs a)
     for (int64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) a.out[i] = a.x[i];
     return;
   }
-  // mean context (see make_mean_ctx; no leave-one-out here)
-  MeanCtx mc;
-  mc.level = a.mean_level; mc.identity = false; mc.zero = false; mc.loo = false; mc.cnt = 0.0; mc.sum = 0.0;
-  if (a.mean_level == LEVEL_BATCH) { mc.cnt = v[5]; mc.sum = v[6]; if (mc.cnt == 0.0) mc.zero = true; }
-  else if (a.mean_level == LEVEL_GROUP) {
-    if (g == a.tail_group) mc.zero = true;
-    else { mc.cnt = v[0]; mc.sum = v[1]; if (mc.cnt == 0.0) mc.zero = true; }
-  } else mc.zero = true;
-  const double mean = elem_mean(mc, 0.f, 1.f, false);  // one value for the whole group
-  auto ss_of = [&](int base) {
-    const double ss = v[base + 4] - 2.0 * mean * v[base + 3] + mean * mean * v[base + 2];
-    return ss > 0.0 ? ss : 0.0;
-  };
-  double std_d = 1.0;
-  double eps = a.eps;
-  if (a.std_level == LEVEL_BATCH) {
-    const double cnt = v[5], ss = ss_of(5);
-    if (a.unbiased) std_d = cnt <= 1.0 ? 1.0 : sqrt(ss / (cnt - 1.0));
-    else std_d = cnt == 0.0 ? 1.0 : sqrt(ss / cnt);
-  } else if (a.std_level == LEVEL_GROUP) {
-    if (g == a.tail_group) std_d = 0.0;
-    else if (a.grows[g] == 1 && a.unbiased) std_d = 1.0;
-    else {
-      const double cnt = v[0], ss = ss_of(0);
-      if (a.unbiased) std_d = cnt <= 1.0 ? 1.0 : sqrt(ss / (cnt - 1.0));
-      else std_d = cnt == 0.0 ? 1.0 : sqrt(ss / cnt);
-    }
-    std_d = (double)(float)std_d;
-  } else {
-    eps = 0.0;
-  }
-  const bool mean64 = a.mean_level == LEVEL_BATCH, std64 = a.std_level == LEVEL_BATCH;
-  auto one = [&](float x, float m) -> float {
-    if (mean64 || std64) {
-      double c = mean64 ? ((double)x - mean) : (double)(x - (float)mean);
-      if (has_mask) c = mean64 ? c * (double)m : (double)((float)c * m);
-      const double den = std64 ? (std_d + eps) : (double)((float)std_d + (float)eps);
-      return (float)(c / den);
-    }
-    float c = x - (float)mean;
-    if (has_mask) c = c * m;
-    return c / ((float)std_d + (float)eps);
-  };
+  const NormParams np = norm_params(a, g, v);
+  auto one = [&](float x, float m) -> float { return norm_one(np, x, m, has_mask); };
   for (int64_t i = lo + threadIdx.x; i < mid_lo; i += blockDim.x) a.out[i] = one(a.x[i], has_mask ? a.mask[i] : 1.0f);
   for (int64_t i = i0; i < mid_hi; i += 4 * step) {
     if (i != i0) fetch(i);
@@ -1206,6 +1233,150 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_apply_cf_kernel(NormArgs a)
   }
   for (int64_t i = mid_hi + threadIdx.x; i < hi; i += blockDim.x)
     if (i >= mid_lo) a.out[i] = one(a.x[i], has_mask ? a.mask[i] : 1.0f);
+}
+
+// The apply pass after the packed GAE (GaeArgs::seg_stats) over blocks of SEG_APPLY_ELEMS consecutive
+// elements instead of (group, split): the grid depends on the number of elements alone, so nobody has
+// to know the longest group (which meant waiting for the GPU), and uneven groups leave no block idle. A
+// block finds the groups of its first and last element, requests its 16 elements per thread first, and
+// then takes its groups (one or two) in turn. Groups as GaeArgs: token offsets or first sequences.
+__global__ __launch_bounds__(NORM_THREADS) void norm_apply_seg_kernel(NormArgs a, GroupOffsets go) {
+  __shared__ double smem[4 * 10];
+  __shared__ int s_grp[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bool has_mask = a.mask != nullptr;
+  const int64_t lo = (int64_t)blockIdx.x * SEG_APPLY_ELEMS;
+  const int64_t hi = lo + SEG_APPLY_ELEMS < a.n ? lo + SEG_APPLY_ELEMS : a.n;
+  constexpr int U = SEG_APPLY_ELEMS / (4 * NORM_THREADS);
+  f32x4 xv[U], mv[U], r[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t j = lo + 4 * (tid + u * NORM_THREADS);
+    xv[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    mv[u] = f32x4{1.f, 1.f, 1.f, 1.f};
+    if (j + 4 <= a.n) {
+      xv[u] = *(const f32x4*)(a.x + j);
+      if (has_mask) mv[u] = *(const f32x4*)(a.mask + j);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (j + e < a.n) { xv[u][e] = a.x[j + e]; if (has_mask) mv[u][e] = a.mask[j + e]; }
+    }
+    r[u] = xv[u];
+  }
+  if (wave < 2) {
+    GroupOffsets ends = go;
+    ends.shift = 1;
+    const int k = wave_count_le(ends, a.G, wave == 0 ? lo : hi - 1, lane);
+    if (lane == 0) s_grp[wave] = k < a.G ? k : a.G - 1;
+  }
+  const bool any_batch = a.mean_level == LEVEL_BATCH || a.std_level == LEVEL_BATCH;
+  const int64_t st = GAE_SEG_WAVES * a.part_slots;
+  double v[10];
+#pragma unroll
+  for (int k = 0; k < 10; ++k) v[k] = 0.0;
+  if (any_batch) {
+    for (int64_t i = tid; i < st; i += NORM_THREADS) {
+#pragma unroll
+      for (int k = 0; k < 5; ++k) v[5 + k] += a.part[k * st + i];
+    }
+    block_sum_n<10>(v, smem);
+  }
+  __syncthreads();
+  const int g_first = s_grp[0], g_last = s_grp[1];
+  for (int g = g_first; g <= g_last; ++g) {
+    const int64_t g0 = go[g], g1 = go[g + 1];
+    __syncthreads();  // the previous group's readers are done
+    if (wave == 0) {
+      double w[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+      const int64_t p0 = GAE_SEG_WAVES * (g0 / a.part_tile + g);
+      const int64_t pn = g1 > g0 ? GAE_SEG_WAVES * ((g1 - 1) / a.part_tile - g0 / a.part_tile + 1) : 0;
+      for (int64_t i = lane; i < pn; i += 64) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) w[k] += a.part[k * st + p0 + i];
+      }
+#pragma unroll
+      for (int k = 0; k < 5; ++k) w[k] = wave_sum(w[k]);
+      if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) smem[k] = w[k];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 5; ++k) v[k] = smem[k];
+    double active = any_batch ? v[5] : v[0];
+    if (has_mask && !any_batch && active == 0.0) {  // nothing active in the group: is anything active at all?
+      double c = 0.0;
+      for (int64_t i = tid; i < st; i += NORM_THREADS) c += a.part[i];
+      active = block_sum_d(c, smem + 8);
+    }
+    if (!any_batch) v[5] = active;
+    if (has_mask && active == 0.0) continue;  // nothing active: the input is returned unchanged
+    const NormParams np = norm_params(a, g, v);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t j = lo + 4 * (tid + u * NORM_THREADS) + e;
+        if (j >= g0 && j < g1) r[u][e] = norm_one(np, xv[u][e], mv[u][e], has_mask);
+      }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t j = lo + 4 * (tid + u * NORM_THREADS);
+    if (j + 4 <= a.n) *(f32x4*)(a.out + j) = r[u];
+    else
+#pragma unroll
+      for (int e = 0; e < 4; ++e) if (j + e < a.n) a.out[j + e] = r[u][e];
+  }
+}
+
+// Reward scores of a batch (actor.py:197-206): clip((reward + bias) * scaling, -clip, clip) and, with
+// `normed`, their group or batch normalisation (no leave-one-out; groups of rows by a.goff), in one
+// launch of one block: a batch has at most a few thousand rows, and the chain of tensor operations and
+// the normalisation's two launches cost 5 us each. A wave takes whole groups.
+constexpr int SCORE_THREADS = 1024;
+__global__ __launch_bounds__(SCORE_THREADS) void reward_score_kernel(NormArgs a, float bias, float scaling, float clip,
+                                                                     int normed) {
+  constexpr int NW = SCORE_THREADS / 64;
+  __shared__ double sm[NW][2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  double b1 = 0.0, b4 = 0.0;
+  for (int64_t i = tid; i < a.n; i += SCORE_THREADS) {
+    float x = (a.x[i] + bias) * scaling;
+    if (!(x != x)) x = x < -clip ? -clip : (x > clip ? clip : x);
+    a.out[i] = x;
+    b1 += (double)x;
+    b4 += (double)x * (double)x;
+  }
+  if (!normed) return;
+  double v[10];
+#pragma unroll
+  for (int k = 0; k < 10; ++k) v[k] = 0.0;
+  b1 = wave_sum(b1);
+  b4 = wave_sum(b4);
+  if (lane == 0) { sm[wave][0] = b1; sm[wave][1] = b4; }
+  __syncthreads();  // (also makes the block's stores to out visible to the block)
+  for (int i = 0; i < NW; ++i) { v[6] += sm[i][0]; v[9] += sm[i][1]; }
+  v[5] = v[7] = (double)a.n;
+  v[8] = v[6];
+  for (int g = wave; g < a.G; g += NW) {
+    const int64_t g0 = a.goff[g], g1 = a.goff[g + 1];
+    double s1 = 0.0, s4 = 0.0;
+    for (int64_t i = g0 + lane; i < g1; i += 64) {
+      const double x = (double)a.out[i];
+      s1 += x;
+      s4 += x * x;
+    }
+    s1 = wave_sum(s1);
+    s4 = wave_sum(s4);
+    v[0] = v[2] = (double)(g1 - g0);
+    v[1] = v[3] = s1;
+    v[4] = s4;
+    const NormParams np = norm_params(a, g, v);
+    for (int64_t i = g0 + lane; i < g1; i += 64) a.out[i] = norm_one(np, a.out[i], 1.f, false);
+  }
 }
 
 // pass 2: sum of squared masked deviations per (group, split)
@@ -1510,6 +1681,8 @@ struct TurnArgs {
   float* ws_adv;           // [bs][L]
   float* ws_ret;           // [bs][L]
   int* status;             // bit 0: negative id, bit 1: id >= L, bit 2: ids go backwards
+  int roll;                // the ids are those of the token before (next-token convention): id[t + 1], -1 at the end
+  const float* addend;     // [bs][L] or null: added to the advantages
 };
 
 struct TurnCarry { int count; int maxid; double sum; };
@@ -1556,9 +1729,11 @@ __global__ __launch_bounds__(TURN_THREADS) void turn_gae_kernel(TurnArgs a) {
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x, L = a.L;
   const float* rw = a.rewards + row * L;
-  const float* vl = a.values + row * L;
+  const float* vl = a.values != nullptr ? a.values + row * L : nullptr;  // (no critic: zero)
+  auto value = [&](int64_t t) { return vl != nullptr ? vl[t] : 0.f; };
   const float* ms = a.mask + row * L;
-  const int32_t* id = a.turn_ids + row * L;
+  const int32_t* ids_row = a.turn_ids + row * L;
+  auto turn_id = [&](int64_t t) { return !a.roll ? ids_row[t] : (t + 1 < L ? ids_row[t + 1] : -1); };
   double* prefix = a.ws_prefix + row * (L + 1);
   float* tval = a.ws_val + row * L;
   float* tadv = a.ws_adv + row * L;
@@ -1576,7 +1751,7 @@ __global__ __launch_bounds__(TURN_THREADS) void turn_gae_kernel(TurnArgs a) {
     for (int i = 0; i < TURN_ITEMS; ++i) {
       const int64_t t = t0 + i;
       act[i] = t < L && ms[t] != 0.0f;
-      ids[i] = act[i] ? id[t] : -1;
+      ids[i] = act[i] ? turn_id(t) : -1;
       r[i] = act[i] ? rw[t] : 0.0f;
       if (act[i]) {
         if (ids[i] < 0) bad |= 1;
@@ -1608,7 +1783,7 @@ __global__ __launch_bounds__(TURN_THREADS) void turn_gae_kernel(TurnArgs a) {
     for (int i = 0; i < TURN_ITEMS; ++i) {
       if (start[i]) {
         prefix[k] = run_sum;            // active rewards strictly before this turn
-        tval[k] = vl[t0 + i];           // the turn's state value: value at its first token
+        tval[k] = value(t0 + i);           // the turn's state value: value at its first token
         ++k;
       }
       run_sum += (double)r[i];
@@ -1626,7 +1801,7 @@ __global__ __launch_bounds__(TURN_THREADS) void turn_gae_kernel(TurnArgs a) {
     const float gam = a.discount;
     const float lam = a.lam_seq ? a.lam_seq[row] : a.lam;
     const float c = gam * lam;
-    float nextv = (a.no_eos && a.no_eos[row]) ? vl[L - 1] : 0.0f;
+    float nextv = (a.no_eos && a.no_eos[row]) ? value(L - 1) : 0.0f;
     float last = 0.0f;
     for (int k = K - 1; k >= 0; --k) {
       const float R = (float)(prefix[k + 1] - prefix[k]);
@@ -1653,7 +1828,7 @@ __global__ __launch_bounds__(TURN_THREADS) void turn_gae_kernel(TurnArgs a) {
       const int64_t t = t0 + i;
       m[i] = t < L ? ms[t] : 0.0f;
       act[i] = m[i] != 0.0f;
-      ids[i] = act[i] ? id[t] : -1;
+      ids[i] = act[i] ? turn_id(t) : -1;
       if (act[i]) mx = mx > ids[i] ? mx : ids[i];
     }
     TurnCarry tot1;
@@ -1675,14 +1850,14 @@ __global__ __launch_bounds__(TURN_THREADS) void turn_gae_kernel(TurnArgs a) {
       const int64_t t = t0 + i;
       if (start[i]) ++k;
       if (t >= L) continue;
+      float adv = 0.0f, ret = value(t);
       if (act[i] && k > 0) {
         const float mm = m[i];
-        a.adv[row * L + t] = tadv[k - 1] * mm;
-        a.ret[row * L + t] = tret[k - 1] * mm + vl[t] * (1.0f - mm);
-      } else {
-        a.adv[row * L + t] = 0.0f;
-        a.ret[row * L + t] = vl[t];
+        adv = tadv[k - 1] * mm;
+        ret = tret[k - 1] * mm + ret * (1.0f - mm);
       }
+      a.adv[row * L + t] = a.addend != nullptr ? adv + a.addend[row * L + t] : adv;
+      a.ret[row * L + t] = ret;
     }
     carry2.count = tot2.count; carry2.maxid = tot1.maxid;
   }
@@ -1830,8 +2005,8 @@ int areal_gae_packed(const float* rewards, const float* values, const float* los
   return AREAL_OK;
 }
 
-// areal_gae_packed on a padded [n_seqs, uniform_len] batch whose rows are at least one tile (2048
-// tokens) long, which also leaves in row_stats [5][n_seqs] (fp64) the masked sums of each row's
+// areal_gae_packed on a padded [n_seqs, uniform_len] batch (values may be null: no critic, all zero), which
+// also leaves in row_stats [5][n_seqs] (fp64) the masked sums of each row's
 // advantages that areal_group_norm_from_row_stats turns into means and deviations: the
 // statistics pass of a normalisation of the advantages under the same mask, at no extra traffic.
 int areal_gae_padded_row_stats(const float* rewards, const float* values, const float* loss_mask,
@@ -1841,9 +2016,11 @@ int areal_gae_padded_row_stats(const float* rewards, const float* values, const 
                                hipStream_t stream) {
   if (n_seqs < 0 || uniform_len < 0) return AREAL_ERR_BAD_ARG;
   if (n_seqs == 0 || uniform_len == 0) return AREAL_OK;
-  if (!rewards || !values || !loss_mask || !advantages || !returns || !row_stats) return AREAL_ERR_BAD_ARG;
-  if (uniform_len < GAE_TILE || uniform_len > 64 * (int64_t)GAE_TILE || n_seqs > (1 << 30))
-    return AREAL_ERR_UNSUPPORTED;
+  if (!rewards || !loss_mask || !advantages || !returns || !row_stats) return AREAL_ERR_BAD_ARG;
+  if (uniform_len > 64 * (int64_t)GAE_TILE || n_seqs > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
+  // a block per row: rows of a fraction of a tile leave most of its lanes idle, which only shows once
+  // there are more rows than fit the chip at a time
+  if (uniform_len < GAE_TILE / 4 && n_seqs > 4096) return AREAL_ERR_UNSUPPORTED;
   GaeArgs g{rewards, values, loss_mask, nullptr, no_eos, lambda_seq, n_seqs * uniform_len, (int)n_seqs,
             uniform_len, discount, gae_lambda, advantages, returns, 1, row_stats};
   launch_gae_owned<true>(g, n_seqs, stream);
@@ -1893,6 +2070,73 @@ int areal_gae_packed_group_stats(const float* rewards, const float* values, cons
   return AREAL_OK;
 }
 
+// areal_gae_packed_group_stats followed by the group normalisation of its advantages, in two launches that
+// need nothing from the host: group j is the sequences [group_first[j], group_first[j + 1]) (int64,
+// device; group_first[n_groups] = n_seqs), group_rows their numbers. Levels and unsupported combinations
+// as areal_group_norm_from_segment_stats, unsupported batches as areal_gae_packed_group_stats; values may be null.
+int areal_gae_packed_normalized(const float* rewards, const float* values, const float* loss_mask,
+                                const int32_t* cu_seqlens, const uint8_t* no_eos, const float* lambda_seq,
+                                int64_t n_tokens, int64_t n_seqs, float discount, float gae_lambda,
+                                const int64_t* group_first, const int64_t* group_rows, int64_t n_groups,
+                                int tail_group, int mean_level, int std_level, int unbiased, double eps,
+                                float* advantages, float* returns, float* normalized, double* segment_stats,
+                                size_t segment_stats_bytes, hipStream_t stream) {
+  if (n_tokens < 0 || n_seqs < 0 || n_groups < 0) return AREAL_ERR_BAD_ARG;
+  if (n_tokens == 0) return AREAL_OK;
+  if (!rewards || !loss_mask || !advantages || !returns || !normalized || !cu_seqlens || !group_first ||
+      !group_rows || !segment_stats || n_seqs == 0 || n_groups == 0)
+    return AREAL_ERR_BAD_ARG;
+  if (mean_level < 0 || mean_level > 2 || std_level < 0 || std_level > 2) return AREAL_ERR_BAD_ARG;
+  if (mean_level == LEVEL_GROUP && std_level == LEVEL_BATCH) return AREAL_ERR_UNSUPPORTED;
+  if (n_seqs > (1 << 30) || n_groups > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
+  const int64_t nb = ceil_div_i64(n_tokens, GAE_TILE);
+  if (nb > (1 << 29)) return AREAL_ERR_UNSUPPORTED;
+  if (n_tokens / n_seqs > 8 * GAE_TILE || n_tokens / n_groups < 256) return AREAL_ERR_UNSUPPORTED;
+  if (segment_stats_bytes < areal_gae_segment_stats_bytes(n_tokens, n_groups)) return AREAL_ERR_WORKSPACE;
+  if (((uintptr_t)advantages | (uintptr_t)loss_mask | (uintptr_t)normalized) & 15) return AREAL_ERR_ALIGNMENT;
+  GaeArgs g{rewards, values, loss_mask, cu_seqlens, no_eos, lambda_seq, n_tokens, (int)n_seqs,
+            0, discount, gae_lambda, advantages, returns, 0, nullptr};
+  g.goff = nullptr; g.gseq = group_first; g.n_groups = (int)n_groups; g.seg_stats = segment_stats;
+  g.seg_slots = nb + n_groups;
+  const dim3 grid((unsigned)(ceil_div_i64(nb, 8) * 8));
+  if (lambda_seq != nullptr)
+    hipLaunchKernelGGL((gae_tile_kernel<true, true>), grid, dim3(GAE_THREADS), 0, stream, g);
+  else
+    hipLaunchKernelGGL((gae_tile_kernel<false, true>), grid, dim3(GAE_THREADS), 0, stream, g);
+  AREAL_CHECK_LAUNCH();
+  NormArgs a{};
+  a.x = advantages; a.mask = loss_mask; a.n = n_tokens; a.goff = nullptr; a.grows = group_rows;
+  a.G = (int)n_groups; a.tail_group = tail_group;
+  a.mean_level = mean_level; a.std_level = std_level; a.unbiased = unbiased; a.eps = eps;
+  a.part = segment_stats; a.out = normalized; a.closed_form = 1;
+  a.part_tile = GAE_TILE; a.part_slots = g.seg_slots;
+  const GroupOffsets go{nullptr, group_first, cu_seqlens, 0};
+  hipLaunchKernelGGL(norm_apply_seg_kernel, dim3((unsigned)ceil_div_i64(n_tokens, SEG_APPLY_ELEMS)), dim3(NORM_THREADS),
+                     0, stream, a, go);
+  AREAL_CHECK_LAUNCH();
+  return AREAL_OK;
+}
+
+// Reward scores of a batch: see reward_score_kernel. group_offsets (rows) / group_rows / n_groups as
+// areal_group_norm, n_groups 0: no normalisation.
+int areal_reward_scores(const float* rewards, int64_t n, float bias, float scaling, float clip,
+                        const int64_t* group_offsets, const int64_t* group_rows, int64_t n_groups, int tail_group,
+                        int mean_level, int std_level, int unbiased, double eps, float* out, hipStream_t stream) {
+  if (n < 0 || n_groups < 0) return AREAL_ERR_BAD_ARG;
+  if (n == 0) return AREAL_OK;
+  if (!rewards || !out || (n_groups > 0 && (!group_offsets || !group_rows))) return AREAL_ERR_BAD_ARG;
+  if (mean_level < 0 || mean_level > 2 || std_level < 0 || std_level > 2) return AREAL_ERR_BAD_ARG;
+  if (mean_level == LEVEL_GROUP && std_level == LEVEL_BATCH) return AREAL_ERR_UNSUPPORTED;
+  if (n > (1 << 24)) return AREAL_ERR_UNSUPPORTED;
+  NormArgs a{};
+  a.x = rewards; a.n = n; a.goff = group_offsets; a.grows = group_rows; a.G = (int)n_groups; a.tail_group = tail_group;
+  a.mean_level = mean_level; a.std_level = std_level; a.unbiased = unbiased; a.eps = eps; a.out = out;
+  hipLaunchKernelGGL(reward_score_kernel, dim3(1), dim3(SCORE_THREADS), 0, stream, a, bias, scaling, clip,
+                     n_groups > 0 ? 1 : 0);
+  AREAL_CHECK_LAUNCH();
+  return AREAL_OK;
+}
+
 size_t areal_turn_gae_workspace_bytes(int64_t bs, int64_t max_seqlen) {
   if (bs <= 0 || max_seqlen <= 0) return 0;
   return (size_t)bs * ((size_t)(max_seqlen + 1) * sizeof(double) + (size_t)max_seqlen * 3 * sizeof(float)) + 256;
@@ -1902,15 +2146,28 @@ size_t areal_turn_gae_workspace_bytes(int64_t bs, int64_t max_seqlen) {
 // int32 (-1 in prompt / tool gaps), no_eos [bs] (nullable), lambda_seq [bs] (nullable, else the
 // scalar). status (device int, zeroed by the caller) receives a bit mask of malformed turn ids
 // at active tokens: 1 negative, 2 not smaller than max_seqlen, 4 decreasing.
+int areal_turn_gae_ex(const float*, const float*, const float*, const int32_t*, int, const uint8_t*, const float*,
+                      const float*, int64_t, int64_t, float, float, float*, float*, int*, void*, size_t, hipStream_t);
+
 int areal_turn_gae(const float* rewards, const float* values, const float* loss_mask,
                    const int32_t* turn_ids, const uint8_t* no_eos, const float* lambda_seq,
                    int64_t bs, int64_t max_seqlen, float discount, float gae_lambda,
                    float* advantages, float* returns, int* status, void* workspace,
                    size_t workspace_bytes, hipStream_t stream) {
+  if (bs > 0 && max_seqlen > 0 && !values) return AREAL_ERR_BAD_ARG;
+  return areal_turn_gae_ex(rewards, values, loss_mask, turn_ids, 0, no_eos, lambda_seq, nullptr, bs, max_seqlen,
+                           discount, gae_lambda, advantages, returns, status, workspace, workspace_bytes, stream);
+}
+
+// ... with values nullable (all zero), roll_ids (the ids of the next-token convention are turn_ids[:, t + 1] and
+// -1 at the end) and addend [bs, max_seqlen] (nullable), which is added to the advantages.
+int areal_turn_gae_ex(const float* rewards, const float* values, const float* loss_mask, const int32_t* turn_ids,
+                      int roll_ids, const uint8_t* no_eos, const float* lambda_seq, const float* addend, int64_t bs,
+                      int64_t max_seqlen, float discount, float gae_lambda, float* advantages, float* returns,
+                      int* status, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (bs < 0 || max_seqlen < 0) return AREAL_ERR_BAD_ARG;
   if (bs == 0 || max_seqlen == 0) return AREAL_OK;
-  if (!rewards || !values || !loss_mask || !turn_ids || !advantages || !returns || !status)
-    return AREAL_ERR_BAD_ARG;
+  if (!rewards || !loss_mask || !turn_ids || !advantages || !returns || !status) return AREAL_ERR_BAD_ARG;
   if (bs > (1 << 30) || max_seqlen > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
   if (workspace == nullptr || workspace_bytes < areal_turn_gae_workspace_bytes(bs, max_seqlen))
     return AREAL_ERR_WORKSPACE;
@@ -1924,6 +2181,7 @@ int areal_turn_gae(const float* rewards, const float* values, const float* loss_
   a.ws_adv = a.ws_val + (size_t)bs * max_seqlen;
   a.ws_ret = a.ws_adv + (size_t)bs * max_seqlen;
   a.status = status;
+  a.roll = roll_ids; a.addend = addend;
   hipLaunchKernelGGL(turn_gae_kernel, dim3((unsigned)bs), dim3(TURN_THREADS), 0, stream, a);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;

@@ -732,6 +732,189 @@ variable_list logits_logprobs(const Tensor& logits, const Tensor& labels, double
   return Logits::apply(logits, labels, temperature, with_entropy);
 }
 
+// ---------------------------------------------------------------------------------------
+// Advantages
+// ---------------------------------------------------------------------------------------
+// What a group normalisation needs besides its data: (group offsets [G + 1], rows per group [G], longest
+// group, tail group, mean level, deviation level, leave one out, unbiased, eps).
+using NormTables = std::tuple<Tensor, Tensor, int64_t, int, int, int, int, int, double>;
+
+Tensor bytes_of(const Tensor& t, int64_t bs, int64_t L) {  // a mask as [bs, L] bytes
+  Tensor r = t.scalar_type() == at::kBool ? t : t.ne(0);
+  if (r.dim() != 2 || r.size(0) != bs || r.size(1) != L) r = r.reshape({bs, L});
+  return r.contiguous();
+}
+bool in_place_ok(const Tensor& t) { return t.scalar_type() == at::kFloat && t.is_contiguous() && !t.requires_grad(); }
+
+// Reward scores and their normalisation, then areal_advantage_prep. `score`: the scores themselves when
+// `scored`, else the raw rewards. Returns (loss mask, old log-probs, kl rewards, total rewards, kl rewards
+// for GAE, outcome rewards (both turn mode only), no-eos mask).
+py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double scaling, double clip,
+                         const std::optional<NormTables>& norm, const Tensor& loss_mask, const Tensor& attention_mask,
+                         const Tensor& logp_src, const OptTensor& ref_logp, bool recompute, int estimator, bool clamp,
+                         bool no_eos_zero, double kl_ctl, bool turn_mode) {
+  require_gpu(logp_src, loss_mask, attention_mask, score);
+  const c10::hip::HIPGuard guard(logp_src.device().index());
+  const int64_t bs = score.size(0), L = logp_src.size(-1);
+  const areal_stream_t stream = stream_of(logp_src);
+  Tensor sc = score.scalar_type() == at::kFloat ? score : score.to(at::kFloat);
+  sc = sc.contiguous();
+  if (!scored) {
+    const Tensor shaped = empty_f32(sc, bs);
+    if (norm.has_value()) {
+      const auto& [off, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = *norm;
+      check(areal_reward_scores(ptr<float>(sc), bs, (float)bias, (float)scaling, (float)clip, ptr<int64_t>(off),
+                                ptr<int64_t>(rows), rows.numel(), tail, mean_level, std_level, unbiased, eps,
+                                ptr<float>(shaped), stream),
+            "areal_reward_scores");
+    } else {
+      check(areal_reward_scores(ptr<float>(sc), bs, (float)bias, (float)scaling, (float)clip, nullptr, nullptr, 0, -1, 0,
+                                0, 0, 0.0, ptr<float>(shaped), stream),
+            "areal_reward_scores");
+    }
+    sc = shaped;
+  }
+  Tensor logp = logp_src.requires_grad() ? logp_src.detach() : logp_src;
+  const bool src_ok = in_place_ok(logp_src);
+  if (logp.dim() != 2) logp = logp.reshape({bs, L});
+  if (!in_place_ok(logp)) logp = logp.to(at::kFloat).contiguous();
+  const Tensor old = recompute && src_ok ? logp : empty(logp, {bs, L}, at::kFloat);
+  Tensor ref = or_undefined(ref_logp);
+  const bool ref_in_place = ref.defined() && in_place_ok(ref);
+  if (ref.defined()) ref = ref_in_place ? ref.reshape({bs, L}) : ref.detach().to(at::kFloat).contiguous().reshape({bs, L});
+  const Tensor lm = empty(logp, {bs, L}, at::kFloat), kl = empty(logp, {bs, L}, at::kFloat),
+               tot = empty(logp, {bs, L}, at::kFloat);
+  const Tensor gkl = turn_mode ? empty(logp, {bs, L}, at::kFloat) : Tensor(),
+               outcome = turn_mode ? empty(logp, {bs, L}, at::kFloat) : Tensor();
+  const Tensor seqlens = empty(logp, {bs}, at::kLong), no_eos = empty(logp, {bs}, at::kBool);
+  const Tensor lmb = bytes_of(loss_mask, bs, L), amb = bytes_of(attention_mask, bs, L);
+  check(areal_advantage_prep(ptr<uint8_t>(lmb), ptr<uint8_t>(amb), ptr<float>(logp), ptr<float>(ref), ptr<float>(sc), bs,
+                             L, recompute ? 0 : 1, estimator, clamp, no_eos_zero, ref_in_place, (float)kl_ctl,
+                             ptr<float>(lm), ptr<float>(old), ptr<float>(kl), ptr<float>(gkl), ptr<float>(outcome),
+                             ptr<float>(tot), ptr<int64_t>(seqlens), ptr<uint8_t>(no_eos), stream),
+        "areal_advantage_prep");
+  auto opt = [](const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); };
+  return py::make_tuple(lm, old.view(logp_src.sizes()), kl, tot, opt(gkl), opt(outcome), no_eos);
+}
+
+Tensor f32(const Tensor& t) {
+  if (!t.defined()) return t;
+  return (t.scalar_type() == at::kFloat ? t : t.to(at::kFloat)).contiguous();
+}
+
+// Token-level GAE of padded rows that leaves each row's masked sums: (advantages, returns, sums [5, bs]), or
+// nothing when the layout is not one for it.
+std::optional<std::tuple<Tensor, Tensor, Tensor>> gae_row_stats(const Tensor& rewards, const OptTensor& values,
+                                                                const Tensor& loss_mask, const Tensor& no_eos,
+                                                                double discount, double lambda,
+                                                                const OptTensor& lambda_seq) {
+  const Tensor v = f32(or_undefined(values)), lam = or_undefined(lambda_seq);
+  require_gpu(rewards, v, loss_mask, no_eos, lam);
+  const c10::hip::HIPGuard guard(rewards.device().index());
+  const int64_t bs = rewards.size(0), L = rewards.size(1);
+  const Tensor r = f32(rewards), m = f32(loss_mask), ne = no_eos.to(at::kBool).contiguous();
+  const Tensor adv = at::empty_like(r), ret = at::empty_like(r), sums = empty(r, {5, bs}, at::kDouble);
+  const int rc = areal_gae_padded_row_stats(ptr<float>(r), ptr<float>(v), ptr<float>(m), ptr<uint8_t>(ne), ptr<float>(lam),
+                                            bs, L, (float)discount, (float)lambda, ptr<float>(adv), ptr<float>(ret),
+                                            ptr<double>(sums), stream_of(r));
+  if (rc == AREAL_ERR_UNSUPPORTED) return std::nullopt;
+  check(rc, "areal_gae_padded_row_stats");
+  return std::make_tuple(adv, ret, sums);
+}
+
+// x (rows of one length) normalised with the sums gae_row_stats left.
+OptTensor norm_from_row_stats(const Tensor& x, const Tensor& mask, const Tensor& sums, const NormTables& norm) {
+  require_gpu(x, mask, sums);
+  const c10::hip::HIPGuard guard(x.device().index());
+  const auto& [off, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = norm;
+  const Tensor out = at::empty_like(x);
+  const int rc = areal_group_norm_from_row_stats(ptr<float>(x), ptr<float>(mask), x.size(0), x.size(1), ptr<int64_t>(off),
+                                                 ptr<int64_t>(rows), rows.numel(), longest, tail, mean_level, std_level,
+                                                 unbiased, eps, ptr<double>(sums), ptr<float>(out), stream_of(x));
+  if (rc == AREAL_ERR_UNSUPPORTED) return std::nullopt;
+  check(rc, "areal_group_norm_from_row_stats");
+  return out;
+}
+
+// Normalisation of x [rows, ...] under mask, with its own statistics passes.
+Tensor group_norm(const Tensor& x, const OptTensor& mask, const NormTables& norm) {
+  const Tensor m = f32(or_undefined(mask));
+  require_gpu(x, m);
+  const c10::hip::HIPGuard guard(x.device().index());
+  const auto& [off, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = norm;
+  const Tensor xf = f32(x), out = at::empty_like(xf);
+  const size_t bytes = areal_group_norm_workspace_bytes(rows.numel(), longest);
+  const Tensor ws = workspace(xf, bytes);
+  check(areal_group_norm(ptr<float>(xf), ptr<float>(m), xf.numel(), ptr<int64_t>(off), ptr<int64_t>(rows), rows.numel(),
+                         longest, tail, mean_level, std_level, loo, unbiased, eps, ptr<float>(out), ptr<void>(ws), bytes,
+                         stream_of(xf)),
+        "areal_group_norm");
+  return out;
+}
+
+// An int the device is writing, on its way to the host.
+struct HostInt {
+  std::shared_ptr<Status> status;
+  int wait() const { return status->wait(); }
+};
+
+// (advantages, returns, malformed-id flags)
+py::tuple turn_gae(const Tensor& rewards, const OptTensor& values, const Tensor& loss_mask, const Tensor& turn_ids,
+                   bool roll_ids, const Tensor& no_eos, double discount, double lambda, const OptTensor& lambda_seq,
+                   const OptTensor& addend) {
+  const Tensor v = f32(or_undefined(values)), lam = or_undefined(lambda_seq), add = f32(or_undefined(addend));
+  require_gpu(rewards, v, loss_mask, turn_ids, no_eos, lam, add);
+  const c10::hip::HIPGuard guard(rewards.device().index());
+  const int64_t bs = rewards.size(0), L = rewards.size(1);
+  const Tensor r = f32(rewards), m = f32(loss_mask), ne = no_eos.to(at::kBool).contiguous();
+  // ids beyond int32 cannot be valid (they must be smaller than the sequence length)
+  const Tensor ids = (turn_ids.scalar_type() == at::kInt ? turn_ids
+                      : turn_ids.scalar_type() == at::kLong ? turn_ids.clamp(-1, INT32_MAX).to(at::kInt)
+                                                            : turn_ids.to(at::kInt)).contiguous();
+  const Tensor adv = at::empty_like(r), ret = at::empty_like(r);
+  HostInt flags{std::make_shared<Status>(r)};
+  if (bs == 0 || L == 0) {
+    *(int*)flags.status->host.data_ptr() = 0;
+    return py::make_tuple(adv, ret, flags);
+  }
+  const Tensor status = at::zeros({1}, r.options().dtype(at::kInt));
+  const size_t bytes = areal_turn_gae_workspace_bytes(bs, L);
+  const Tensor ws = workspace(r, bytes);
+  const areal_stream_t stream = stream_of(r);
+  check(areal_turn_gae_ex(ptr<float>(r), ptr<float>(v), ptr<float>(m), ptr<int32_t>(ids), roll_ids, ptr<uint8_t>(ne),
+                          ptr<float>(lam), ptr<float>(add), bs, L, (float)discount, (float)lambda, ptr<float>(adv),
+                          ptr<float>(ret), ptr<int>(status), ptr<void>(ws), bytes, stream),
+        "areal_turn_gae");
+  if (hipMemcpyAsync(flags.status->host.data_ptr(), status.data_ptr(), sizeof(int), hipMemcpyDeviceToHost,
+                     (hipStream_t)stream) != hipSuccess)
+    fail("copy of the turn status to the host failed");
+  return py::make_tuple(adv, ret, flags);
+}
+
+// Packed GAE and the normalisation of its advantages: (normalised, returns, advantages), or nothing when
+// the batch is not one for the fused launches. norm: the groups' first sequences in place of offsets.
+std::optional<std::tuple<Tensor, Tensor, Tensor>> gae_packed_normalized(
+    const Tensor& rewards, const Tensor& values, const Tensor& loss_mask, const Tensor& cu_seqlens,
+    const OptTensor& no_eos_arg, double discount, double lambda, const OptTensor& lambda_seq, const NormTables& norm) {
+  const Tensor lam = or_undefined(lambda_seq);
+  require_gpu(rewards, values, loss_mask, cu_seqlens, lam);
+  const c10::hip::HIPGuard guard(rewards.device().index());
+  const Tensor r = f32(rewards), v = f32(values), m = f32(loss_mask), cu = cu_seqlens.to(at::kInt).contiguous();
+  const Tensor ne = no_eos_arg.has_value() ? no_eos_arg->to(r.device(), at::kBool).contiguous() : Tensor();
+  const auto& [first, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = norm;
+  const int64_t n = r.numel(), n_seqs = cu.numel() - 1;
+  const Tensor adv = at::empty_like(r), ret = at::empty_like(r), out = at::empty_like(r);
+  const size_t bytes = areal_gae_segment_stats_bytes(n, rows.numel());
+  const Tensor seg = workspace(r, bytes);
+  const int rc = areal_gae_packed_normalized(
+      ptr<float>(r), ptr<float>(v), ptr<float>(m), ptr<int32_t>(cu), ptr<uint8_t>(ne), ptr<float>(lam), n, n_seqs,
+      (float)discount, (float)lambda, ptr<int64_t>(first), ptr<int64_t>(rows), rows.numel(), tail, mean_level, std_level,
+      unbiased, eps, ptr<float>(adv), ptr<float>(ret), ptr<float>(out), ptr<double>(seg), bytes, stream_of(r));
+  if (rc == AREAL_ERR_UNSUPPORTED || rc == AREAL_ERR_ALIGNMENT) return std::nullopt;
+  check(rc, "areal_gae_packed_normalized");
+  return std::make_tuple(out, ret, adv);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -751,4 +934,11 @@ PYBIND11_MODULE(_host, m) {
   m.def("lm_head_backward", &lm_head_backward);
   m.def("default_token_chunk", &default_token_chunk);
   m.def("logits_logprobs", &logits_logprobs);
+  py::class_<HostInt>(m, "HostInt").def("wait", &HostInt::wait);
+  m.def("advantage_prep", &advantage_prep);
+  m.def("gae_row_stats", &gae_row_stats);
+  m.def("norm_from_row_stats", &norm_from_row_stats);
+  m.def("group_norm", &group_norm);
+  m.def("turn_gae", &turn_gae);
+  m.def("gae_packed_normalized", &gae_packed_normalized);
 }

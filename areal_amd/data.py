@@ -40,6 +40,11 @@ def _group_tables(groups: tuple, tail_rows: int, row_len: int, device_str: str):
     )
 
 
+@functools.lru_cache(maxsize=64)
+def _uniform_tables(group_size: int, n_groups: int, tail_rows: int, row_len: int, device_str: str):
+    return _group_tables((group_size,) * n_groups, tail_rows, row_len, device_str)
+
+
 class Normalization:
     """Adaptive normalisation with independent levels for mean and std:
     ``"batch"``, ``"group"`` (fixed ``group_size`` or explicit ``group_sizes``) or ``None``."""
@@ -80,36 +85,36 @@ class Normalization:
             self.mean_level, self.std_level,
         ):
             raise NotImplementedError("batch-level normalisation over several ranks is not built")
-        lib = _lib.load()
         dev = _lib.require_gpu(x, loss_mask)
-        bs = x.size(0)
-        xf = x.to(torch.float32).contiguous()
-        n = xf.numel()
-        out = torch.empty_like(xf)
+        n, bs = x.numel(), x.size(0)
         if n == 0:
-            return out
+            return torch.empty_like(x, dtype=torch.float32)
         if loss_mask is not None and loss_mask.shape != x.shape:
             loss_mask = loss_mask.expand_as(x)
-        mf = loss_mask.to(torch.float32).contiguous() if loss_mask is not None else None
-        row_len = n // bs
+        tables = self._tables(bs, n // bs, group_sizes, dev)
+        if tables is None:
+            return x.to(torch.float32).contiguous()
+        return _lib.host().group_norm(x, loss_mask, tables)
+
+    def _tables(self, bs: int, row_len: int, group_sizes, dev):
+        """The groups of ``bs`` rows of ``row_len`` elements and this configuration, as the native calls
+        take them (``NormTables`` of ``csrc/host.cpp``); ``None`` when there is nothing to normalise."""
         if self.mean_level == "group" or self.std_level == "group":
-            groups, tail = self._group_rows(bs, group_sizes)
+            if group_sizes is None:
+                groups, tail = (self.group_size, bs // self.group_size), bs % self.group_size
+                if groups[1] == 0 and tail == 0:
+                    return None
+                tables = _uniform_tables(*groups, tail, row_len, str(dev))
+            else:
+                groups, tail = self._group_rows(bs, group_sizes)
+                tables = _group_tables(groups, tail, row_len, str(dev))
         else:
-            groups, tail = (bs,), 0
-        if not groups and tail == 0:
-            return xf
-        offsets, rows, tail_group, max_len = _group_tables(groups, tail, row_len, str(dev))
-        n_groups = rows.numel()
-        nbytes = lib.areal_group_norm_workspace_bytes(n_groups, max_len)
-        ws = _lib.workspace(nbytes, dev)
-        rc = lib.areal_group_norm(
-            _lib.ptr(xf), _lib.ptr(mf), n, _lib.ptr(offsets), _lib.ptr(rows), n_groups, max_len,
-            tail_group, _LEVEL_ID[self.mean_level], _LEVEL_ID[self.std_level],
+            tables = _uniform_tables(bs, 1, 0, row_len, str(dev))
+        offsets, rows, tail_group, max_len = tables
+        return (
+            offsets, rows, max_len, tail_group, _LEVEL_ID[self.mean_level], _LEVEL_ID[self.std_level],
             int(bool(self.mean_leave1out)), int(bool(self.std_unbiased)), float(self.eps),
-            _lib.ptr(out), _lib.ptr(ws), nbytes, _lib.stream_ptr(dev),
         )
-        _lib.check(rc, "areal_group_norm")
-        return out
 
 
     def needs_one_statistics_pass(self) -> bool:
@@ -125,27 +130,11 @@ class Normalization:
         ``None`` when this configuration needs a second statistics pass."""
         if not self.needs_one_statistics_pass() or x.ndim != 2:
             return None
-        lib = _lib.load()
         dev = _lib.require_gpu(x, mask_f32, row_stats)
-        bs, row_len = x.shape
-        if self.mean_level == "group" or self.std_level == "group":
-            groups, tail = self._group_rows(bs, group_sizes)
-        else:
-            groups, tail = (bs,), 0
-        if not groups and tail == 0:
+        tables = self._tables(x.shape[0], x.shape[1], group_sizes, dev)
+        if tables is None:
             return x
-        offsets, rows, tail_group, max_len = _group_tables(groups, tail, row_len, str(dev))
-        out = torch.empty_like(x)
-        rc = lib.areal_group_norm_from_row_stats(
-            _lib.ptr(x), _lib.ptr(mask_f32), bs, row_len, _lib.ptr(offsets), _lib.ptr(rows), rows.numel(),
-            max_len, tail_group, _LEVEL_ID[self.mean_level], _LEVEL_ID[self.std_level],
-            int(bool(self.std_unbiased)), float(self.eps), _lib.ptr(row_stats), _lib.ptr(out),
-            _lib.stream_ptr(dev),
-        )
-        if rc == _lib.ERR_UNSUPPORTED:
-            return None
-        _lib.check(rc, "areal_group_norm_from_row_stats")
-        return out
+        return _lib.host().norm_from_row_stats(x, mask_f32, row_stats, tables)
 
 
     @torch.no_grad()

@@ -14,6 +14,7 @@ import math
 from typing import Any
 
 import torch
+import torch.distributed as dist
 
 from areal_amd.config import RejectionSamplingConfig
 from areal_amd.data import KLEstimator, Normalization
@@ -29,9 +30,11 @@ from areal_amd.functional.functional import (
     reward_overlong_penalty,
 )
 from areal_amd.ppo.gae import (
+    _check_turn_ids,
     _compute_token_level_gae,
-    _compute_turn_level_gae,
+    _raise_turn_id_errors,
     _token_level_gae_with_row_stats,
+    _turn_level_gae,
     compute_gae_lambda,
 )
 from areal_amd.ppo.lambda_fn import resolve_gae_lambda_fn
@@ -593,17 +596,27 @@ def compute_advantages(
             max_response_length=max_new_tokens,
         )
 
-    reward_score = (data["rewards"] + reward_bias) * reward_scaling
-    reward_score = torch.clip(reward_score, max=reward_clip, min=-reward_clip)
+    # One launch shapes the rewards and normalises them, if the normalisation needs one statistics pass;
+    # other normalisations are called on the shaped scores.
+    score, scored, score_tables = data["rewards"], False, None
     if reward_norm is not None:
-        reward_score = reward_norm(reward_score, group_sizes=group_sizes)
+        native = (
+            isinstance(reward_norm, Normalization) and reward_norm.needs_one_statistics_pass()
+            and score.ndim == 1 and score.is_cuda and score.dtype == torch.float32 and not dist.is_initialized()
+        )
+        if native:
+            score_tables = reward_norm._tables(bs, 1, group_sizes, dev)
+        if score_tables is None:
+            score = torch.clip((score + reward_bias) * reward_scaling, max=reward_clip, min=-reward_clip)
+            score, scored = reward_norm(score, group_sizes=group_sizes), True
+    elif score.ndim != 1 or score.dtype != torch.float32:
+        score = torch.clip((score + reward_bias) * reward_scaling, max=reward_clip, min=-reward_clip)
+        scored = True
 
-    # structural turn ids follow the same next-token convention as the mask and the log-probs
+    # structural turn ids follow the same next-token convention as the mask and the log-probs (the
+    # turn-level kernel reads them rolled; a lambda function gets a rolled copy)
     turn_ids = data.get("turn_ids")
-    if turn_ids is not None:
-        turn_ids = torch.roll(turn_ids, shifts=-1, dims=-1)
-        turn_ids[:, -1] = -1
-    elif gae_timestep_unit == "turn":
+    if turn_ids is None and gae_timestep_unit == "turn":
         raise ValueError(
             "actor.gae_timestep_unit='turn' requires rollout data to "
             "include 'turn_ids'."
@@ -625,54 +638,17 @@ def compute_advantages(
     # reference's in-place updates are kept: `old_logp *= loss_mask` also masks the tensor that
     # prox_logp names (and, in the recompute branch, the caller's prox_logp itself), and
     # `ref_logp *= loss_mask` masks the caller's ref_logp.
-    lib = _lib.load()
-    _lib.require_gpu(logp_src, data["loss_mask"], data["attention_mask"])
-    L = logp_src.shape[-1]
-
-    def as_bytes(t):
-        t = t.reshape(bs, L)
-        t = t if t.dtype == torch.bool else t != 0
-        return t.contiguous().view(torch.uint8)
-
-    def in_place_ok(t):
-        return t.dtype == torch.float32 and t.is_contiguous() and not t.requires_grad
-
-    f32 = dict(dtype=torch.float32, device=dev)
-    logp_in = logp_src.detach().reshape(bs, L)
-    if not in_place_ok(logp_in):
-        logp_in = logp_in.float().contiguous()
-    old_logp = logp_in if (recompute and in_place_ok(logp_src)) else torch.empty((bs, L), **f32)
-    ref_src = data.get("ref_logp")
-    ref_in = None
-    ref_in_place = False
-    if ref_src is not None:
-        ref_in_place = in_place_ok(ref_src)
-        ref_in = ref_src.reshape(bs, L) if ref_in_place else ref_src.detach().float().contiguous().reshape(bs, L)
     turn_mode = gae_timestep_unit == "turn"
-    loss_mask = torch.empty((bs, L), **f32)
-    kl_rewards = torch.empty((bs, L), **f32)
-    tot_rewards = torch.empty((bs, L), **f32)
-    gae_kl_rewards = torch.empty((bs, L), **f32) if turn_mode else None
-    gae_outcome_rewards = torch.empty((bs, L), **f32) if turn_mode else None
-    seqlens = torch.empty(bs, dtype=torch.int64, device=dev)
-    seq_no_eos_mask = torch.empty(bs, dtype=torch.bool, device=dev)
     if getattr(kl_estimator, "kl_estimator", None) not in ("k1", "k2", "k3"):
         raise TypeError("kl_estimator must be a KLEstimator (k1, k2 or k3)")
     est = {"k1": 1, "k2": 2, "k3": 3}[kl_estimator.kl_estimator]
-    # temporaries are named so that they outlive the launch (a freed block is handed to the next
-    # allocation at once)
-    lm_bytes, am_bytes = as_bytes(data["loss_mask"]), as_bytes(data["attention_mask"])
-    score_f = reward_score.float().contiguous()
-    rc = lib.areal_advantage_prep(
-        _lib.ptr(lm_bytes), _lib.ptr(am_bytes),
-        _lib.ptr(logp_in), _lib.ptr(ref_in), _lib.ptr(score_f), bs, L,
-        0 if recompute else 1, est, int(bool(kl_estimator.apply_clamp)), int(bool(mask_no_eos_with_zero)),
-        int(ref_in_place), float(kl_ctl), _lib.ptr(loss_mask), _lib.ptr(old_logp), _lib.ptr(kl_rewards),
-        _lib.ptr(gae_kl_rewards), _lib.ptr(gae_outcome_rewards), _lib.ptr(tot_rewards),
-        _lib.ptr(seqlens), _lib.ptr(seq_no_eos_mask), _lib.stream_ptr(dev),
+    loss_mask, old_logp, kl_rewards, tot_rewards, gae_kl_rewards, gae_outcome_rewards, seq_no_eos_mask = (
+        _lib.host().advantage_prep(
+            score, scored, reward_bias, reward_scaling, reward_clip, score_tables, data["loss_mask"],
+            data["attention_mask"], logp_src, data.get("ref_logp"), recompute, est, bool(kl_estimator.apply_clamp),
+            bool(mask_no_eos_with_zero), kl_ctl, turn_mode,
+        )
     )
-    _lib.check(rc, "areal_advantage_prep")
-    old_logp = old_logp.view(logp_src.shape)
     if recompute:
         data["logprobs"] = old_logp
         if old_logp.data_ptr() == logp_src.data_ptr():
@@ -682,28 +658,26 @@ def compute_advantages(
     # turn mode keeps the token KL as a local actor penalty instead of summing it into turns
     rewards = gae_outcome_rewards if turn_mode else tot_rewards
 
-    values = data["values"] if "values" in data else torch.zeros_like(rewards)
+    values = data.get("values")  # none: all zero
     if gae_lambda_fn is None and isinstance(gae_lambda, (str, bool)):
         gae_lambda_fn, _ = resolve_gae_lambda_fn(gae_lambda)
     if gae_lambda_fn is not None:
-        gae_lambda = compute_gae_lambda(gae_lambda_fn, gae_lambda_kwargs, loss_mask, turn_ids, gae_timestep_unit)
+        rolled = turn_ids
+        if turn_ids is not None:
+            rolled = torch.roll(turn_ids, shifts=-1, dims=-1)
+            rolled[:, -1] = -1
+        gae_lambda = compute_gae_lambda(gae_lambda_fn, gae_lambda_kwargs, loss_mask, rolled, gae_timestep_unit)
     elif not isinstance(gae_lambda, torch.Tensor):
         gae_lambda = float(gae_lambda)
         if not math.isfinite(gae_lambda):
             raise ValueError(f"Static gae_lambda must be finite, got {gae_lambda}")
     if gae_timestep_unit == "turn":
-        advantages, returns = _compute_turn_level_gae(
-            rewards=rewards,
-            values=values,
-            loss_mask=loss_mask,
-            turn_ids=turn_ids,
-            seq_no_eos_mask=seq_no_eos_mask,
-            discount=discount,
-            gae_lambda=gae_lambda,
+        _check_turn_ids(turn_ids, loss_mask)
+        advantages, returns, turn_flags = _turn_level_gae(
+            rewards, values, loss_mask, turn_ids, True, seq_no_eos_mask, discount, gae_lambda, gae_kl_rewards
         )
-        advantages = advantages + gae_kl_rewards
     else:
-        # With long padded rows and a normalisation that needs one statistics pass, the GAE kernel
+        # With padded rows and a normalisation that needs one statistics pass, the GAE kernel
         # sums each row's advantages under the mask while it writes them, and the normalisation
         # is its apply pass alone: two launches for the two stages (same results).
         fused = None
@@ -717,16 +691,18 @@ def compute_advantages(
         else:
             advantages, returns = _compute_token_level_gae(
                 rewards=rewards,
-                values=values,
+                values=values if values is not None else torch.zeros_like(rewards),
                 loss_mask=loss_mask,
                 seq_no_eos_mask=seq_no_eos_mask,
                 discount=discount,
                 gae_lambda=gae_lambda,
             )
-    data["returns"] = returns
     if adv_norm is not None:
         advantages = adv_norm(advantages, loss_mask, group_sizes=group_sizes)
+    if turn_mode:
+        _raise_turn_id_errors(turn_flags.wait())  # with everything queued: the GPU does not wait for the host
 
+    data["returns"] = returns
     data["advantages"] = advantages
     data["kl_rewards"] = kl_rewards
     data["tot_rewards"] = tot_rewards

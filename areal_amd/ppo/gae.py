@@ -72,27 +72,13 @@ def _compute_token_level_gae(
 def _token_level_gae_with_row_stats(rewards, values, loss_mask, seq_no_eos_mask, discount, gae_lambda):
     """``_compute_token_level_gae`` that also returns, per row, the masked sums of the advantages
     which ``Normalization.from_row_stats`` needs (``[5, bs]`` fp64), or ``None`` when the layout
-    does not allow it (rows shorter than one 2048-token tile)."""
+    does not allow it (very many rows of a fraction of a 2048-token tile). ``values=None``: all zero."""
     bs, max_seqlen = rewards.shape
-    if max_seqlen < 2048 or bs == 0:
+    if bs == 0 or max_seqlen == 0:
         return None
-    lib = _lib.load()
-    dev = _lib.require_gpu(rewards, values, loss_mask)
-    lam_seq, lam = _split_lambda(gae_lambda, bs, dev)
-    r = rewards.to(torch.float32).contiguous()
-    v = values.to(torch.float32).contiguous()
-    m = loss_mask.to(torch.float32).contiguous()
-    no_eos = seq_no_eos_mask.to(torch.bool).contiguous()
-    adv, ret = torch.empty_like(r), torch.empty_like(r)
-    row_stats = torch.empty((5, bs), dtype=torch.float64, device=dev)
-    rc = lib.areal_gae_padded_row_stats(
-        _lib.ptr(r), _lib.ptr(v), _lib.ptr(m), _lib.ptr(no_eos), _lib.ptr(lam_seq), bs, max_seqlen,
-        float(discount), float(lam), _lib.ptr(adv), _lib.ptr(ret), _lib.ptr(row_stats), _lib.stream_ptr(dev),
-    )
-    if rc == _lib.ERR_UNSUPPORTED:
-        return None
-    _lib.check(rc, "areal_gae_padded_row_stats")
-    return adv, ret, row_stats, m
+    lam_seq, lam = _split_lambda(gae_lambda, bs, rewards.device)
+    res = _lib.host().gae_row_stats(rewards, values, loss_mask, seq_no_eos_mask, discount, lam, lam_seq)
+    return (*res, loss_mask.to(torch.float32).contiguous()) if res is not None else None
 
 
 def compute_gae_packed(
@@ -141,31 +127,20 @@ def compute_gae_packed_normalized(
     statistics pass (the GAE kernel leaves the sums), else GAE and the three normalisation passes."""
     if rewards.ndim != 1:
         raise ValueError(f"packed GAE expects 1D tensors, got ndim={rewards.ndim}")
-    lib = _lib.load()
     dev = _lib.require_gpu(rewards, values, loss_mask, cu_seqlens)
-    cu = cu_seqlens.to(device=dev, dtype=torch.int32).contiguous()
-    n, n_seqs = rewards.numel(), cu.numel() - 1
-    r = rewards.to(torch.float32).contiguous()
-    v = values.to(torch.float32).contiguous()
-    m = loss_mask.to(torch.float32).contiguous()
+    n, n_seqs = rewards.numel(), cu_seqlens.numel() - 1
     if n > 0 and n_seqs > 0 and adv_norm.needs_one_statistics_pass():
         lam_seq, lam = _split_lambda(gae_lambda, n_seqs, dev)
-        no_eos = seq_no_eos_mask.to(device=dev, dtype=torch.bool).contiguous() if seq_no_eos_mask is not None else None
-        index, rows, _ = adv_norm._packed_groups(n_seqs, group_sizes, dev)
-        offsets = cu.to(torch.int64)[index]
-        nbytes = lib.areal_gae_segment_stats_bytes(n, rows.numel())
-        seg = torch.empty(nbytes // 8, dtype=torch.float64, device=dev)
-        adv, ret = torch.empty_like(r), torch.empty_like(r)
-        rc = lib.areal_gae_packed_group_stats(
-            _lib.ptr(r), _lib.ptr(v), _lib.ptr(m), _lib.ptr(cu), _lib.ptr(no_eos), _lib.ptr(lam_seq), n, n_seqs,
-            float(discount), float(lam), _lib.ptr(offsets), rows.numel(), _lib.ptr(adv), _lib.ptr(ret),
-            _lib.ptr(seg), nbytes, _lib.stream_ptr(dev),
-        )
-        if rc != _lib.ERR_UNSUPPORTED:
-            _lib.check(rc, "areal_gae_packed_group_stats")
-            normed = adv_norm.packed(adv, m, cu, group_sizes, max_group_tokens, segment_stats=seg)
-            return normed, ret, adv
-    adv, ret = compute_gae_packed(r, v, m, cu, seq_no_eos_mask, discount, gae_lambda)
+        tables = adv_norm._tables(n_seqs, 1, group_sizes, dev)
+        if tables is not None:
+            res = _lib.host().gae_packed_normalized(
+                rewards, values, loss_mask, cu_seqlens, seq_no_eos_mask, discount, lam, lam_seq, tables
+            )
+            if res is not None:
+                return res
+    m = loss_mask.to(torch.float32).contiguous()
+    adv, ret = compute_gae_packed(rewards, values, m, cu_seqlens, seq_no_eos_mask, discount, gae_lambda)
+    cu = cu_seqlens.to(device=dev, dtype=torch.int32).contiguous()
     return adv_norm.packed(adv, m, cu, group_sizes, max_group_tokens), ret, adv
 
 
@@ -174,6 +149,18 @@ _TURN_ID_ERRORS = (
     (2, "turn_ids at active loss tokens must be smaller than the sequence length"),
     (4, "turn_ids at active loss tokens must be temporally nondecreasing"),
 )
+
+
+def _check_turn_ids(turn_ids: torch.Tensor, loss_mask: torch.Tensor) -> None:
+    if turn_ids.shape != loss_mask.shape:
+        raise ValueError(f"turn_ids must have shape {loss_mask.shape}, got {turn_ids.shape}")
+    if turn_ids.device != loss_mask.device:
+        raise ValueError(
+            "turn_ids and loss_mask must be on the same device, got "
+            f"{turn_ids.device} and {loss_mask.device}"
+        )
+    if turn_ids.dtype not in (torch.uint8, torch.int8, torch.int16, torch.int32, torch.int64):
+        raise ValueError(f"turn_ids must use an integer dtype, got {turn_ids.dtype}")
 
 
 def _compute_turn_level_gae(
@@ -195,45 +182,26 @@ def _compute_turn_level_gae(
     reference's ``RuntimeError``; the reference uses device-side asserts there, which on a GPU
     would abort the process.  ``validate=False`` skips the read-back.
     """
-    if turn_ids.shape != loss_mask.shape:
-        raise ValueError(f"turn_ids must have shape {loss_mask.shape}, got {turn_ids.shape}")
-    if turn_ids.device != loss_mask.device:
-        raise ValueError(
-            "turn_ids and loss_mask must be on the same device, got "
-            f"{turn_ids.device} and {loss_mask.device}"
-        )
-    if turn_ids.dtype not in (torch.uint8, torch.int8, torch.int16, torch.int32, torch.int64):
-        raise ValueError(f"turn_ids must use an integer dtype, got {turn_ids.dtype}")
-    lib = _lib.load()
-    bs, max_seqlen = rewards.shape
-    r = rewards.to(torch.float32).contiguous()
-    v = values.to(torch.float32).contiguous()
-    m = loss_mask.to(torch.float32).contiguous()
-    # ids beyond int32 cannot be valid (they must be smaller than the sequence length)
-    ids = turn_ids.clamp(min=-1, max=2**31 - 1).to(torch.int32).contiguous()
-    dev = _lib.require_gpu(r, v, m, ids)
-    lam_seq, lam = _split_lambda(gae_lambda, bs, dev)
-    no_eos = seq_no_eos_mask.to(device=dev, dtype=torch.bool).contiguous()
-    adv = torch.empty((bs, max_seqlen), dtype=torch.float32, device=dev)
-    ret = torch.empty((bs, max_seqlen), dtype=torch.float32, device=dev)
-    if bs == 0 or max_seqlen == 0:
-        return adv, ret
-    status = torch.zeros(1, dtype=torch.int32, device=dev)
-    nbytes = lib.areal_turn_gae_workspace_bytes(bs, max_seqlen)
-    ws = _lib.workspace(nbytes, dev)
-    rc = lib.areal_turn_gae(
-        _lib.ptr(r), _lib.ptr(v), _lib.ptr(m), _lib.ptr(ids), _lib.ptr(no_eos), _lib.ptr(lam_seq),
-        bs, max_seqlen, float(discount), float(lam), _lib.ptr(adv), _lib.ptr(ret),
-        _lib.ptr(status), _lib.ptr(ws), nbytes, _lib.stream_ptr(dev),
+    _check_turn_ids(turn_ids, loss_mask)
+    adv, ret, flags = _turn_level_gae(
+        rewards, values, loss_mask, turn_ids, False, seq_no_eos_mask, discount, gae_lambda, None
     )
-    _lib.check(rc, "areal_turn_gae")
     if validate:
-        _raise_turn_id_errors(status)
+        _raise_turn_id_errors(flags.wait())
     return adv, ret
 
 
-def _raise_turn_id_errors(status: torch.Tensor) -> None:
-    flags = int(status.item())
+def _turn_level_gae(rewards, values, loss_mask, turn_ids, roll_ids, seq_no_eos_mask, discount, gae_lambda, addend):
+    """The launch of turn-level GAE: ``(advantages + addend, returns, flags of malformed ids)``, the
+    flags on their way to the host. ``values=None``: all zero; ``roll_ids``: ``turn_ids`` are not rolled
+    to the next-token convention yet."""
+    lam_seq, lam = _split_lambda(gae_lambda, rewards.shape[0], rewards.device)
+    return _lib.host().turn_gae(
+        rewards, values, loss_mask, turn_ids, roll_ids, seq_no_eos_mask, discount, lam, lam_seq, addend
+    )
+
+
+def _raise_turn_id_errors(flags: int) -> None:
     for bit, message in _TURN_ID_ERRORS:
         if flags & bit:
             raise RuntimeError(message)
@@ -252,15 +220,7 @@ def _build_gae_lambda_context(
     if turn_ids is None and gae_timestep_unit == "turn":
         raise ValueError("Turn-level GAE requires rollout data to include 'turn_ids'.")
     if turn_ids is not None:
-        if turn_ids.shape != loss_mask.shape:
-            raise ValueError(f"turn_ids must have shape {loss_mask.shape}, got {turn_ids.shape}")
-        if turn_ids.device != loss_mask.device:
-            raise ValueError(
-                "turn_ids and loss_mask must be on the same device, got "
-                f"{turn_ids.device} and {loss_mask.device}"
-            )
-        if turn_ids.dtype not in (torch.uint8, torch.int8, torch.int16, torch.int32, torch.int64):
-            raise ValueError(f"turn_ids must use an integer dtype, got {turn_ids.dtype}")
+        _check_turn_ids(turn_ids, loss_mask)
     lib = _lib.load()
     bs, max_seqlen = loss_mask.shape
     m = loss_mask.to(torch.float32).contiguous()
@@ -275,7 +235,7 @@ def _build_gae_lambda_context(
     )
     _lib.check(rc, "areal_gae_lambda_context")
     if validate and turn_ids is not None:
-        _raise_turn_id_errors(status)
+        _raise_turn_id_errors(int(status.item()))
     return {
         "effective_token_lengths": token_lengths,
         "turn_counts": turn_counts,

@@ -376,8 +376,9 @@ int areal_gae_packed(const float* rewards, const float* values, const float* los
                      float gae_lambda, float* advantages, float* returns, void* workspace,
                      size_t workspace_bytes, areal_stream_t stream);
 
-/* areal_gae_packed on a padded [n_seqs, uniform_len] batch with rows of at least 2048 tokens
- * (AREAL_ERR_UNSUPPORTED otherwise), which also leaves per row, in row_stats [5][n_seqs] fp64, the
+/* areal_gae_packed on a padded [n_seqs, uniform_len] batch (AREAL_ERR_UNSUPPORTED for rows over 131072
+ * tokens and for more than 4096 rows of fewer than 512; values may be NULL: all zero), which also
+ * leaves per row, in row_stats [5][n_seqs] fp64, the
  * sums of m, x m, m^2, m^2 x, m^2 x^2 (x = the advantage written, m = loss_mask): the statistics
  * pass of the advantage normalisation that follows in compute_advantages
  * (areal/trainer/ppo/actor.py:344-350: adv_norm(advantages, loss_mask)), at no extra traffic. */
@@ -404,6 +405,28 @@ int areal_gae_packed_group_stats(const float* rewards, const float* values, cons
                                  double* segment_stats, size_t segment_stats_bytes,
                                  areal_stream_t stream);
 
+/* areal_gae_packed_group_stats and the normalisation of its advantages over groups of whole sequences
+ * (what PPOActor.compute_advantages does after GAE, areal/trainer/ppo/actor.py:344-350) in two
+ * launches that take nothing from the host: group j is the sequences [group_first[j],
+ * group_first[j + 1]) (int64 [n_groups + 1], device), group_rows [n_groups] their numbers. values may
+ * be NULL (all zero). segment_stats is scratch of areal_gae_segment_stats_bytes(n_tokens, n_groups)
+ * bytes. Same restrictions as the two entry points it stands for. */
+int areal_gae_packed_normalized(const float* rewards, const float* values, const float* loss_mask,
+                                const int32_t* cu_seqlens, const uint8_t* no_eos, const float* lambda_seq,
+                                int64_t n_tokens, int64_t n_seqs, float discount, float gae_lambda,
+                                const int64_t* group_first, const int64_t* group_rows, int64_t n_groups,
+                                int tail_group, int mean_level, int std_level, int unbiased, double eps,
+                                float* advantages, float* returns, float* normalized, double* segment_stats,
+                                size_t segment_stats_bytes, areal_stream_t stream);
+
+/* Reward scores of a batch (areal/trainer/ppo/actor.py:197-206): clip((rewards + bias) * scaling, -clip,
+ * clip), then (n_groups > 0) their normalisation over groups of rows, one launch; group_offsets (row
+ * offsets), group_rows, tail_group, levels and eps as areal_group_norm without a mask or leave-one-out. */
+int areal_reward_scores(const float* rewards, int64_t n, float bias, float scaling, float clip,
+                        const int64_t* group_offsets, const int64_t* group_rows, int64_t n_groups,
+                        int tail_group, int mean_level, int std_level, int unbiased, double eps, float* out,
+                        areal_stream_t stream);
+
 /* Turn-level GAE (areal/trainer/ppo/gae.py:82-163) on padded [bs, max_seqlen] tensors: every
  * generated turn is one timestep. turn_ids int32 (-1 in prompt / tool gaps; non-decreasing over
  * the active tokens of a row), loss_mask fp32 (nonzero = active). *status (device int, zeroed
@@ -415,6 +438,15 @@ int areal_turn_gae(const float* rewards, const float* values, const float* loss_
                    int64_t bs, int64_t max_seqlen, float discount, float gae_lambda,
                    float* advantages, float* returns, int* status, void* workspace,
                    size_t workspace_bytes, areal_stream_t stream);
+
+/* areal_turn_gae with values nullable (all zero), roll_ids (the turn of token t is turn_ids[t + 1], and -1
+ * at a row's end: the next-token convention of actor.py:207-212) and addend (nullable, [bs, max_seqlen]),
+ * which is added to the advantages. */
+int areal_turn_gae_ex(const float* rewards, const float* values, const float* loss_mask,
+                      const int32_t* turn_ids, int roll_ids, const uint8_t* no_eos, const float* lambda_seq,
+                      const float* addend, int64_t bs, int64_t max_seqlen, float discount, float gae_lambda,
+                      float* advantages, float* returns, int* status, void* workspace,
+                      size_t workspace_bytes, areal_stream_t stream);
 
 /* Per-row lengths for per-sample lambda functions (_build_gae_lambda_context,
  * areal/trainer/ppo/gae.py:166-205): active tokens, and distinct turn ids among them (turn_ids
