@@ -499,7 +499,7 @@ DEVI float ref_plus(float m, float c2, float add) {  // fl(m c2) + add
   return x + add;
 }
 
-constexpr int NSTAT = 7;  // m, s, q, xlabel, min, sumx, sumx2
+constexpr int NSTAT = 7;  // m, s, q, xlabel (Fwd16: one value per token, no slots), min, sumx, sumx2
 
 struct FwdParams {
   const int64_t* labels; int T; int V;
@@ -659,18 +659,21 @@ template <bool E> using FwdPlainMomSave = FwdEpi<E, false, true, true>;
 template <bool E> using FwdAffineSave = FwdEpi<E, true, false, true>;
 template <bool E> using FwdAffineMomSave = FwdEpi<E, true, true, true>;
 
-// Merge the partial statistics of one token over all slots. A block is 64 tokens (lanes) x
-// MERGE_WAVES waves; wave w takes slots w, w + MERGE_WAVES, ... (loads stay coalesced along the
-// tokens, and a launch with few tokens and many slots still has enough threads in flight), the
-// partial results meet in LDS and wave 0 adds them in a fixed order.
+// Merge the partial statistics of one token over all slots. A block is TOK tokens x MERGE_WAVES waves,
+// a wave 64 / TOK slots at a time (loads stay coalesced along the tokens), the partial results meet in
+// LDS and wave 0 adds them in a fixed order. Latency-bound: with TOK = 64 the 509 tokens of a short batch
+// are 8 blocks whose waves walk 74 slots one after the other (33 us); TOK = 16 and one pass
+// for the saving sweep's sums take 9.8 (10007 tokens: 18.9 -> 9.9).
+// labels (nullable): the slots hold no label logits, a valid label's is entry t of that statistic's plane.
 // ref_sums: the slots' sums S, Q are relative to row_ref[t] (the saving forward of the
 // hand-scheduled kernels) instead of to each slot's own maximum; the final expressions are then
 // evaluated in fp64, where c2 x - ref and log S (each up to REF_WINDOW binades) cancel.
 // gate / gate_run_if_set: as GemmArgs::skip_if_set / run_if_set. host_status (nullable, pinned host
 // memory; with a gate): receives the gate's value, whether or not the launch does anything.
 constexpr int MERGE_WAVES = 8;
+template <int TOK>
 __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
-    const float* __restrict__ ws, int P, int T, int V, int ref_sums, float c2,
+    const float* __restrict__ ws, int P, int T, int V, const int64_t* __restrict__ labels, int ref_sums, float c2,
     float* __restrict__ logprobs, float* __restrict__ entropy, float* __restrict__ vmin,
     float* __restrict__ vmax, float* __restrict__ vmean, float* __restrict__ vnorm,
     float* __restrict__ row_max, float* __restrict__ sum_exp, const float* __restrict__ row_ref,
@@ -679,25 +682,34 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
   if (host_status != nullptr && blockIdx.x == 0 && threadIdx.x == 0)
     __hip_atomic_store(host_status, *gate, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   if (gate_closed(gate, gate_run_if_set)) return;
-  __shared__ float sh_f[5][MERGE_WAVES][64];   // max, S, Q, label logit, min
-  __shared__ double sh_d[2][MERGE_WAVES][64];  // sum x, sum x^2
+  constexpr int G = 64 / TOK, ROWS = MERGE_WAVES * G;
+  __shared__ float sh_f[5][ROWS][TOK];   // max, S, Q, label logit, min
+  __shared__ double sh_d[2][ROWS][TOK];  // sum x, sum x^2
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int t = blockIdx.x * 64 + lane;
+  const int tok = lane % TOK, grp = lane / TOK, row = wv * G + grp;
+  const int t = blockIdx.x * TOK + tok;
   const int tt = t < T ? t : T - 1;  // lanes past the end repeat the last token and write nothing
   const int64_t PT = (int64_t)P * T;
   const bool moments = vmean != nullptr || vnorm != nullptr;
   float M = neg_inf();
-  for (int p = wv; p < P; p += MERGE_WAVES) M = fmaxf(M, ws[(int64_t)p * T + tt]);
-  sh_f[0][wv][lane] = M;
-  __syncthreads();
+  if (!ref_sums) {  // the sums need the maximum first
+#pragma unroll 4
+    for (int p = row; p < P; p += ROWS) M = fmaxf(M, ws[(int64_t)p * T + tt]);
+    sh_f[0][row][tok] = M;
+    __syncthreads();
 #pragma unroll
-  for (int i = 0; i < MERGE_WAVES; ++i) M = fmaxf(M, sh_f[0][i][lane]);
+    for (int i = 0; i < MERGE_WAVES; ++i) M = fmaxf(M, sh_f[0][i * G + grp][tok]);
+#pragma unroll
+    for (int d = TOK; d < 64; d <<= 1) M = fmaxf(M, __shfl_xor(M, d));
+  }
   float S = 0.f, Q = 0.f, xl = 0.f, mn = pos_inf();
   double sx = 0.0, sx2 = 0.0;
-  for (int p = wv; p < P; p += MERGE_WAVES) {
+#pragma unroll 4
+  for (int p = row; p < P; p += ROWS) {
     const float* w = ws + (int64_t)p * T + tt;
     const float m = w[0];
     if (ref_sums) {
+      M = fmaxf(M, m);
       S += w[1 * PT];
       Q += w[2 * PT];
     } else if (m > neg_inf()) {
@@ -706,20 +718,35 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
       S += alpha * w[1 * PT];
       Q += alpha * fmaf(dl, w[1 * PT], w[2 * PT]);
     }
-    xl += w[3 * PT];
+    if (labels == nullptr) xl += w[3 * PT];
     mn = fminf(mn, w[4 * PT]);
     if (moments) { sx += (double)w[5 * PT]; sx2 += (double)w[6 * PT]; }
   }
-  sh_f[1][wv][lane] = S; sh_f[2][wv][lane] = Q; sh_f[3][wv][lane] = xl; sh_f[4][wv][lane] = mn;
-  sh_d[0][wv][lane] = sx; sh_d[1][wv][lane] = sx2;
+  if (ref_sums) sh_f[0][row][tok] = M;
+  sh_f[1][row][tok] = S; sh_f[2][row][tok] = Q; sh_f[3][row][tok] = xl; sh_f[4][row][tok] = mn;
+  sh_d[0][row][tok] = sx; sh_d[1][row][tok] = sx2;
   __syncthreads();
-  if (wv != 0 || t >= T) return;
+  if (wv != 0) return;
   S = 0.f; Q = 0.f; xl = 0.f; mn = pos_inf(); sx = 0.0; sx2 = 0.0;
 #pragma unroll
   for (int i = 0; i < MERGE_WAVES; ++i) {
-    S += sh_f[1][i][lane]; Q += sh_f[2][i][lane]; xl += sh_f[3][i][lane];
-    mn = fminf(mn, sh_f[4][i][lane]);
-    sx += sh_d[0][i][lane]; sx2 += sh_d[1][i][lane];
+    const int r = i * G + grp;
+    if (ref_sums) M = fmaxf(M, sh_f[0][r][tok]);
+    S += sh_f[1][r][tok]; Q += sh_f[2][r][tok]; xl += sh_f[3][r][tok];
+    mn = fminf(mn, sh_f[4][r][tok]);
+    sx += sh_d[0][r][tok]; sx2 += sh_d[1][r][tok];
+  }
+#pragma unroll
+  for (int d = TOK; d < 64; d <<= 1) {
+    M = fmaxf(M, __shfl_xor(M, d));
+    S += __shfl_xor(S, d); Q += __shfl_xor(Q, d); xl += __shfl_xor(xl, d);
+    mn = fminf(mn, __shfl_xor(mn, d));
+    sx += __shfl_xor(sx, d); sx2 += __shfl_xor(sx2, d);
+  }
+  if (grp != 0 || t >= T) return;
+  if (labels != nullptr) {
+    const int64_t l = labels[t];
+    xl = l >= 0 && l < V ? ws[3 * PT + t] : 0.f;
   }
   if (ref_sums) {
     const double ln2 = 0.6931471805599453094;
@@ -1236,18 +1263,28 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
 // stores carry the non-temporal hint so that they do not push the operand tiles the XCD's other
 // workgroups share out of L2.
 // EDGE: only rows < rows_valid and columns [cols_from, cols_valid) are written (both multiples of 8).
+// In two halves: the four LDS reads are issued together, and the caller puts work between them and
+// the stores (the wave is alone on its SIMD: a read that is waited for at once costs it about 130
+// cycles, and a predicate around each read and its store made that four times per column).
+DEVI void stage16_read(const u16* stage, int lane, u32x4 (&v)[4]) {
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+    v[p] = *(const u32x4*)((const char*)stage + (p * 4 + (lane >> 4)) * STAGE16_PITCH + (lane & 15) * 16);
+}
 template <bool EDGE, bool STREAM = false>
-DEVI void flush_stage16(const u16* stage, u16* out_row0, int64_t ld, int rows_valid, int cols_valid,
+DEVI void stage16_store(u32x4 (&v)[4], u16* out_row0, int64_t ld, int rows_valid, int cols_valid,
                         int cols_from, int lane) {
   const int piece = lane & 15;
+  u16* out = out_row0 + (int64_t)(lane >> 4) * ld + piece * 8;
+  // (used here, ahead of the predicates: the compiler would move the reads behind them)
+  asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+  const bool cols = !EDGE || (piece * 8 < cols_valid && piece * 8 >= cols_from);
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
-    const int row = p * 4 + (lane >> 4);
-    const u32x4 v = *(const u32x4*)((const char*)stage + row * STAGE16_PITCH + piece * 16);
-    if (!EDGE || (row < rows_valid && piece * 8 < cols_valid && piece * 8 >= cols_from)) {
-      u32x4* dst = (u32x4*)(out_row0 + (int64_t)row * ld + piece * 8);
-      if (STREAM) __builtin_nontemporal_store(v, dst);
-      else *dst = v;
+    if (!EDGE || (cols && p * 4 + (lane >> 4) < rows_valid)) {
+      u32x4* dst = (u32x4*)(out + (int64_t)(p * 4) * ld);
+      if (STREAM) __builtin_nontemporal_store(v[p], dst);
+      else *dst = v[p];
     }
   }
 }
@@ -1269,6 +1306,14 @@ struct Store16Impl {
   static DEVI void end(State&, const Params&, int, int, int, int) {}
   static DEVI void split_output(Params& p, int64_t bytes) { p.out = (char*)p.out + bytes; }
   static DEVI void tile(State&, const Params& p, int i0, int j0, int lane, u16* stage, int) {
+    // bf16: column b leaves the staging area while column b + 1 is fetched and converted
+    u32x4 left[4];
+    int cols_valid = p.M - i0;
+    if (NA < 8) cols_valid = cols_valid < NA * 16 ? cols_valid : NA * 16;
+    auto store_column = [&](int b) {
+      stage16_store<EDGE>(left, (u16*)p.out + (int64_t)(j0 + b * 16) * p.ldo + i0, p.ldo, p.N - (j0 + b * 16),
+                          cols_valid, 0, lane);
+    };
     for_each_col([&](auto bc) {
       constexpr int b = decltype(bc)::value;
       float x[32];
@@ -1279,19 +1324,21 @@ struct Store16Impl {
         // only takes this path when ldo % 8 == 0 and the output is 16-byte aligned)
         float js = 1.f;
         if (MODE == 3) js = (!EDGE || j < p.N) ? p.jscale[j] : 0.f;
+        u32x2 pk[NA];
 #pragma unroll
         for (int a = 0; a < NA; ++a) {
           float x0 = x[a * 4], x1 = x[a * 4 + 1], x2 = x[a * 4 + 2], x3 = x[a * 4 + 3];
           if (MODE == 3) { x0 *= js; x1 *= js; x2 *= js; x3 *= js; }
-          u32x2 v;
-          v[0] = pack_bf16x2(x0, x1);
-          v[1] = pack_bf16x2(x2, x3);
-          stage16_put(stage, lane, a, v);
+          pk[a][0] = pack_bf16x2(x0, x1);
+          pk[a][1] = pack_bf16x2(x2, x3);
         }
-        int cols_valid = p.M - i0;
-        if (NA < 8) cols_valid = cols_valid < NA * 16 ? cols_valid : NA * 16;
-        flush_stage16<EDGE>(stage, (u16*)p.out + (int64_t)(j0 + b * 16) * p.ldo + i0, p.ldo,
-                            p.N - (j0 + b * 16), cols_valid, 0, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b > 0) store_column(b - 1);
+#pragma unroll
+        for (int a = 0; a < NA; ++a) stage16_put(stage, lane, a, pk[a]);
+        stage16_read(stage, lane, left);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b == 7) store_column(b);
       } else {
 #pragma unroll
         for (int a = 0; a < NA; ++a) {
@@ -1318,10 +1365,15 @@ template <bool E> using Store16Bf16Scaled = Store16<E, 3>;
 // ---- forward: online softmax statistics (see FwdEpi). In a block column the 16 lanes l % 16 own
 // the 16 tokens and the four lane groups l / 16 own 4 of every 16 vocabulary entries, so a token's
 // 128 entries of the wave's sub-tile sit in four lanes. Per column those four lanes agree on the
-// column's maximum, sum their exponentials relative to it, and lane group jb % 4 folds the result
-// into the running statistics of token column jb, of which it keeps two (jb and jb + 4): ten to
-// fourteen registers per lane live across the main loop. Partial statistics go to slot
-// split * 2 + wa at the end of the sweep.
+// column's maximum (or use the row reference), sum their exponentials relative to it, and after every
+// fourth column lane group jb % 4 folds the result into the running statistics of token column jb, of
+// which it keeps two (jb and jb + 4): eight to twelve registers per lane live across the main loop.
+// Partial statistics go to slot split * 2 + wa at the end of the sweep; a label's logit, which one lane
+// of one tile of the launch holds, goes straight to the first T entries of that statistic's plane.
+// The epilogue is bound by its issue slots and exposed latencies (nothing else runs on its SIMD). Reducing
+// the columns four at a time, reading a staged column back while its sums run and keeping the label's
+// logit out of the reductions: 10007 x 1536 x 151936 without saving 3580 -> 3529 us, the saving sweep of
+// 8192 x 1536 2965 -> 2933 us, a step at 4096 x 896 2.8 % faster in all.
 // The four lanes that share a token are 16 and 32 lanes apart. v_permlane16_swap exchanges the
 // odd rows (of 16 lanes) of its first register with the even rows of its second, v_permlane32_swap
 // rows 2-3 of the first with rows 0-1 of the second: applied to two copies of a value they leave
@@ -1343,20 +1395,12 @@ DEVI float group_max(float v) {
   swap_rows32(a, b);
   return fmaxf(a, b);
 }
-DEVI float group_min(float v) {
-  float a = v, b = v;
-  swap_rows16(a, b);
-  a = b = fminf(a, b);
-  swap_rows32(a, b);
-  return fminf(a, b);
-}
-DEVI float group_sum(float v) {
-  float a = v, b = v;
-  swap_rows16(a, b);
-  a = b = a + b;
-  swap_rows32(a, b);
-  return a + b;
-}
+// Four token columns reduced at once: lane group g ends up with column g over the token's four lanes.
+// Columns c and c + 2 share a register after the first step (lanes 32 apart), all four after the
+// second (16 apart): 3 swaps and 3 operations for the four, where one column at a time takes 2
+// swaps, 2 operations and 2 copies each.
+template <class Op> DEVI float fold_cols32(float c, float c2, Op op) { swap_rows32(c, c2); return op(c, c2); }
+template <class Op> DEVI float fold_cols16(float c02, float c13, Op op) { swap_rows16(c02, c13); return op(c02, c13); }
 
 // A logit that takes no part (past the vocabulary, or a row that an earlier tile of the sweep
 // already covered): far below every real logit, finite so that 0 * it stays 0 in the entropy sum.
@@ -1375,14 +1419,14 @@ struct Fwd16 {
   // SAVE: s and q are relative to the row reference of the saved exponentials (fixed for the whole
   // sweep: nothing is rescaled); otherwise relative to the running maximum m.
   struct State {
-    float m[2], s[2], q[2], xl[2], mn[2], sx[MOMENTS ? 2 : 1], sx2[MOMENTS ? 2 : 1];
+    float m[2], s[2], q[2], mn[2], sx[MOMENTS ? 2 : 1], sx2[MOMENTS ? 2 : 1];
   };
   static DEVI void split_output(Params&, int64_t) {}
   static DEVI void open(State& st, const Params&, int, int, int, int, bool first) {
     if (first) {
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
-        st.m[k] = neg_inf(); st.s[k] = 0.f; st.q[k] = 0.f; st.xl[k] = 0.f; st.mn[k] = pos_inf();
+        st.m[k] = neg_inf(); st.s[k] = 0.f; st.q[k] = 0.f; st.mn[k] = pos_inf();
         if (MOMENTS) { st.sx[k] = 0.f; st.sx2[k] = 0.f; }
       }
     }
@@ -1410,10 +1454,15 @@ struct Fwd16 {
       lab[b] = (l >= v_new && l < p.V) ? (int)l : -1;
       if (SAVE) rr[b] = p.probs_ref[t];
     }
+    float* const label_logit = p.ws + 3 * (int64_t)p.P * p.T;
+    auto add = [](float a, float b) { return a + b; };
+    auto lower = [](float a, float b) { return fminf(a, b); };
+    auto upper = [](float a, float b) { return fmaxf(a, b); };
+    float cs[2], cq[2], cmn[2], cmx[2], csx[2], csx2[2];  // per-lane results of two columns, then of pairs
     ML16_AGPR_FENCE();
     for_each_col([&](auto bc) {
       constexpr int b = decltype(bc)::value;
-      constexpr int k = b >> 2;
+      constexpr int k = b >> 2, c = b & 3;
       float x[32];
       acc_col<b>(x);
       if (AFFINE) {
@@ -1472,81 +1521,98 @@ struct Fwd16 {
         // Exponentials relative to the row reference, summed and stored as they are: one fma, one
         // v_exp_f32, two sums and half a packed conversion per logit. The 16 tokens x 128 entries of
         // the column go through the staging area and leave as whole lines.
-        const float nr = -rr[b];
+        // (The sums run while the staged column comes back from LDS.)
+        const float nr = -rr[SAVE ? b : 0];
+        float t[32], e[32];
 #pragma unroll
         for (int a = 0; a < 8; ++a) {
-          float d[4];
 #pragma unroll
-          for (int e4 = 0; e4 < 4; ++e4) {
-            const float t = fmaf(x[a * 4 + e4], p.c2, nr);
-            const float e = fast_exp2(t);
-            s += e;
-            q = fmaf(t, e, q);
-            d[e4] = e;
+          for (int i = a * 4; i < a * 4 + 4; ++i) {
+            t[i] = fmaf(x[i], p.c2, nr);
+            e[i] = fast_exp2(t[i]);
           }
           u32x2 pk;
-          pk[0] = pack_bf16x2(d[0], d[1]);
-          pk[1] = pack_bf16x2(d[2], d[3]);
+          pk[0] = pack_bf16x2(e[a * 4], e[a * 4 + 1]);
+          pk[1] = pack_bf16x2(e[a * 4 + 2], e[a * 4 + 3]);
           stage16_put(stage, lane, a, pk);
-          // keeps the exponentials of one block next to the sums that consume them (left alone,
-          // the scheduler computes all 32 first and spills them)
+          // keeps the exponentials of one block together (left alone, the scheduler issues the 32 back to back)
           __builtin_amdgcn_sched_barrier(0);
           ML16_AGPR_FENCE();
         }
+        u32x4 left[4];
+        stage16_read(stage, lane, left);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+          s += e[i];
+          q = fmaf(t[i], e[i], q);
+        }
+        asm volatile("" : "+v"(s), "+v"(q) : : ML16_ACC_CLOBBERS);
+        __builtin_amdgcn_sched_barrier(0);
         u16* out = p.probs + (int64_t)(t0 + b * 16) * p.ldv + v0;
         if (!EDGE && !overlap)
-          flush_stage16<false, true>(stage, out, p.ldv, 16, 128, 0, lane);
+          stage16_store<false, true>(left, out, p.ldv, 16, 128, 0, lane);
         else
-          flush_stage16<true, true>(stage, out, p.ldv, 16, (int)p.ldv - v0, overlap ? v_new - v0 : 0, lane);
+          stage16_store<true, true>(left, out, p.ldv, 16, (int)p.ldv - v0, overlap ? v_new - v0 : 0, lane);
       }
-      // the label's logit, if it is one of this lane's 32 entries
-      float xl = 0.f;
+      // the label's logit, if it is one of this lane's 32 entries (about one wave in 70 has one)
       const bool hit = (lab[b] >= v0) && (lab[b] < v0 + 128);
       if (__builtin_amdgcn_ballot_w64(hit) != 0) {
+        float xl = 0.f;
 #pragma unroll
         for (int a = 0; a < 8; ++a)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             if (vidx(a, r) == lab[b]) xl = x[a * 4 + r];
+        const int t = t0 + b * 16 + (lane & 15);
+        if (hit && t < p.T && (((lab[b] - v0) >> 2) & 3) == group) label_logit[t] = xl;
       }
       // The partial results pass through an empty block here: their readers come later (the last
       // one after the last column), and the compiler otherwise moves the summation chains of
       // every column down there, keeping all the exponentials alive in scratch memory until then.
-      asm volatile("" : "+v"(s), "+v"(q), "+v"(tmin), "+v"(xl) : : ML16_ACC_CLOBBERS);
-      s = group_sum(s);
-      q = group_sum(q);
-      tmin = group_min(tmin);
-      xl = group_sum(xl);
-      if (SAVE) tmax = group_max(tmax);
-      if (MOMENTS) {
-        asm volatile("" : "+v"(sx), "+v"(sx2));
-        sx = group_sum(sx);
-        sx2 = group_sum(sx2);
+      asm volatile("" : "+v"(s), "+v"(q), "+v"(tmin), "+v"(tmax) : : ML16_ACC_CLOBBERS);
+      if (MOMENTS) asm volatile("" : "+v"(sx), "+v"(sx2));
+      if constexpr (c < 2) {
+        cs[c] = s; cq[c] = q; cmn[c] = tmin; cmx[c] = tmax;
+        if (MOMENTS) { csx[c] = sx; csx2[c] = sx2; }
+      } else {
+        cs[c - 2] = fold_cols32(cs[c - 2], s, add);
+        cq[c - 2] = fold_cols32(cq[c - 2], q, add);
+        cmn[c - 2] = fold_cols32(cmn[c - 2], tmin, lower);
+        cmx[c - 2] = fold_cols32(cmx[c - 2], tmax, upper);
+        if (MOMENTS) {
+          csx[c - 2] = fold_cols32(csx[c - 2], sx, add);
+          csx2[c - 2] = fold_cols32(csx2[c - 2], sx2, add);
+        }
       }
-      // lane group b % 4 folds the column into the running statistics of token column b
-      if (group == (b & 3)) {
+      if constexpr (c == 3) {  // lane group g takes token column 4 k + g
+        const float S = fold_cols16(cs[0], cs[1], add), Q = fold_cols16(cq[0], cq[1], add);
+        const float mx = fold_cols16(cmx[0], cmx[1], upper);
         if (SAVE) {
-          st.s[k] += s;
-          st.q[k] += q;
-          st.m[k] = fmaxf(st.m[k], tmax);
+          st.s[k] += S;
+          st.q[k] += Q;
+          st.m[k] = fmaxf(st.m[k], mx);
         } else {
           // both sets of sums move to the reference of the larger maximum
           const float m_old = st.m[k];
-          const float m_new = fmaxf(m_old, tmax);
+          const float m_new = fmaxf(m_old, mx);
           const float d_old = (m_old > neg_inf()) ? ref_diff(m_old, m_new, p.c2) : 0.f;
-          const float d_col = (!EDGE || tmax > neg_inf()) ? ref_diff(tmax, m_new, p.c2) : 0.f;
+          const float d_col = (!EDGE || mx > neg_inf()) ? ref_diff(mx, m_new, p.c2) : 0.f;
           const float a_old = fast_exp2(d_old), a_col = fast_exp2(d_col);
-          st.q[k] = a_old * fmaf(d_old, st.s[k], st.q[k]) + a_col * fmaf(d_col, s, q);
-          st.s[k] = a_old * st.s[k] + a_col * s;
+          st.q[k] = a_old * fmaf(d_old, st.s[k], st.q[k]) + a_col * fmaf(d_col, S, Q);
+          st.s[k] = a_old * st.s[k] + a_col * S;
           st.m[k] = m_new;
         }
-        st.mn[k] = fminf(st.mn[k], tmin);
-        st.xl[k] += xl;
-        if (MOMENTS) { st.sx[k] += sx; st.sx2[k] += sx2; }
+        st.mn[k] = fminf(st.mn[k], fold_cols16(cmn[0], cmn[1], lower));
+        if (MOMENTS) {
+          st.sx[k] += fold_cols16(csx[0], csx[1], add);
+          st.sx2[k] += fold_cols16(csx2[0], csx2[1], add);
+          asm volatile("" : "+v"(st.sx[k]), "+v"(st.sx2[k]));
+        }
+        asm volatile("" : "+v"(st.m[k]), "+v"(st.s[k]), "+v"(st.q[k]), "+v"(st.mn[k]) : : ML16_ACC_CLOBBERS);
+      } else if constexpr (c == 2) {
+        asm volatile("" : "+v"(cs[0]), "+v"(cq[0]), "+v"(cmn[0]), "+v"(cmx[0]) : : ML16_ACC_CLOBBERS);
       }
-      asm volatile("" : "+v"(st.m[k]), "+v"(st.s[k]), "+v"(st.q[k]), "+v"(st.xl[k]), "+v"(st.mn[k])
-                   : : ML16_ACC_CLOBBERS);
-      if (MOMENTS) asm volatile("" : "+v"(st.sx[k]), "+v"(st.sx2[k]));
       __builtin_amdgcn_sched_barrier(0);
     });
   }
@@ -1559,7 +1625,7 @@ struct Fwd16 {
       const int t = t0 + ((lane >> 4) + 4 * k) * 16 + (lane & 15);
       if (t >= p.T) continue;
       float* w = p.ws + (int64_t)slot * p.T + t;
-      w[0 * PT] = st.m[k]; w[1 * PT] = st.s[k]; w[2 * PT] = st.q[k]; w[3 * PT] = st.xl[k];
+      w[0 * PT] = st.m[k]; w[1 * PT] = st.s[k]; w[2 * PT] = st.q[k];
       w[4 * PT] = st.mn[k];
       if (MOMENTS) { w[5 * PT] = st.sx[k]; w[6 * PT] = st.sx2[k]; }
     }
@@ -1605,6 +1671,11 @@ struct Bwd16 {
   // (a tile that overlaps its predecessor rewrites the shared rows with the same values)
   static DEVI void tile(State& st, const Params& p, int v0, int t0, int lane, u16* stage, int) {
     const int vl = v0 + 4 * (lane >> 4);
+    u32x4 left[4];  // column b leaves the staging area while column b + 1 is computed
+    auto store_column = [&](int b) {
+      stage16_store<EDGE, true>(left, p.dl + (int64_t)(t0 + b * 16) * p.ldv + v0, p.ldv, p.T - (t0 + b * 16),
+                                (int)p.ldv - v0, 0, lane);
+    };
     for_each_col([&](auto bc) {
       constexpr int b = decltype(bc)::value;
       float x[32];
@@ -1612,6 +1683,7 @@ struct Bwd16 {
       const int t = t0 + b * 16 + (lane & 15);
       const float nb = st.nb[b], gs = st.gs[b];
       const int lab = st.lab[b];
+      u32x2 pk[8];
 #pragma unroll
       for (int a = 0; a < 8; ++a) {
         const int vq = vl + a * 16;
@@ -1631,13 +1703,16 @@ struct Bwd16 {
           if (EDGE && (v >= p.V || t >= p.T)) dv = 0.f;
           d[e] = dv;
         }
-        u32x2 pk;
-        pk[0] = pack_bf16x2(d[0], d[1]);
-        pk[1] = pack_bf16x2(d[2], d[3]);
-        stage16_put(stage, lane, a, pk);
+        pk[a][0] = pack_bf16x2(d[0], d[1]);
+        pk[a][1] = pack_bf16x2(d[2], d[3]);
       }
-      flush_stage16<EDGE, true>(stage, p.dl + (int64_t)(t0 + b * 16) * p.ldv + v0, p.ldv, p.T - (t0 + b * 16),
-                          (int)p.ldv - v0, 0, lane);
+      __builtin_amdgcn_sched_barrier(0);
+      if (b > 0) store_column(b - 1);
+#pragma unroll
+      for (int a = 0; a < 8; ++a) stage16_put(stage, lane, a, pk[a]);
+      stage16_read(stage, lane, left);
+      __builtin_amdgcn_sched_barrier(0);
+      if (b == 7) store_column(b);
     });
   }
 };
@@ -2166,8 +2241,11 @@ int areal_lmhead_fwd_ex(const void* hidden, const void* weight, const float* bia
     return launch_gemm<Fwd16AffineMomSave, FwdAffineMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
   };
   auto merge = [&](int ref_sums, const float* ref, const int* gate, int gate_run_if_set, int* host) {
-    hipLaunchKernelGGL(lmhead_merge_kernel, dim3((unsigned)ceil_div_i64(T, 64)), dim3(64 * MERGE_WAVES),
-                       0, stream, (const float*)workspace, P, (int)T, (int)V, ref_sums, c2, logprobs,
+    // blocks of 64 tokens only when they are at least one per CU
+    const int tok = T >= 64 * 256 ? 64 : 16;
+    hipLaunchKernelGGL((tok == 64 ? lmhead_merge_kernel<64> : lmhead_merge_kernel<16>),
+                       dim3((unsigned)ceil_div_i64(T, tok)), dim3(64 * MERGE_WAVES), 0, stream,
+                       (const float*)workspace, P, (int)T, (int)V, r.k16 ? labels : nullptr, ref_sums, c2, logprobs,
                        entropy, vocab_min, vocab_max, vocab_mean, vocab_norm, row_max, sum_exp, ref,
                        probs_status, gate, gate_run_if_set, logprobs_copy, host);
   };
