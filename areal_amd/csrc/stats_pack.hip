@@ -14,7 +14,8 @@ constexpr int PK_THREADS = 256;
 
 // 16 bytes at any address. The compiler picks the access the target allows for the alignment
 // (gfx950 runs with unaligned access enabled, where this is still one 16-byte instruction).
-struct __attribute__((packed, aligned(1))) Bytes16 { uint32_t w[4]; };
+// (A vector, not a struct: predicated copies of a struct went through LDS.)
+typedef uint32_t Bytes16 __attribute__((ext_vector_type(4), aligned(1)));
 
 // number of nonzero bytes among the four of x
 DEVI int nonzero_bytes(uint32_t x) {
@@ -34,7 +35,7 @@ __global__ __launch_bounds__(PK_THREADS) void rowlens_kernel(const uint8_t* mask
   for (int64_t i = threadIdx.x; i < n16; i += blockDim.x) {
     const Bytes16 v = *(const Bytes16*)(row + 16 * i);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) len += nonzero_bytes(v.w[k]);
+    for (int k = 0; k < 4; ++k) len += nonzero_bytes(v[k]);
   }
   for (int64_t s = 16 * n16 + threadIdx.x; s < S; s += blockDim.x) len += row[s] != 0;
   len = wave_sum(len);
@@ -96,24 +97,31 @@ __global__ __launch_bounds__(PK_THREADS) void cu_scan_kernel(const int32_t* lens
 }
 
 // Copy of n contiguous bytes by the whole block: 16 bytes per thread and access, whatever the
-// two addresses' alignment, four loads in flight per thread before the first store; then the
-// last n % 16 bytes one by one.
+// two addresses' alignment, four loads in flight per thread before the first store. A run whose
+// length is not a multiple of 16 ends with a piece that overlaps its predecessor (the same bytes twice).
+// Bound by the latency of its loads (a block moves 16 KiB at most): they are issued without a predicate,
+// at clamped indices. With a predicate each, every load was waited for before the next was issued:
+// unpacking 557 Ki tokens of 4 bytes into 256 rows took 18.0 us and takes 4.4, packing six tensors of them
+// 21.9 and 9.4.
 DEVI void block_copy_bytes(char* dst, const char* src, int64_t n) {
-  const int64_t n16 = n >> 4;
-  for (int64_t i0 = threadIdx.x; i0 < n16; i0 += 4 * (int64_t)blockDim.x) {
-    Bytes16 v[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t i = i0 + u * (int64_t)blockDim.x;
-      if (i < n16) v[u] = *(const Bytes16*)(src + 16 * i);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t i = i0 + u * (int64_t)blockDim.x;
-      if (i < n16) *(Bytes16*)(dst + 16 * i) = v[u];
-    }
+  if (n < 16) {
+    if ((int64_t)threadIdx.x < n) dst[threadIdx.x] = src[threadIdx.x];
+    return;
   }
-  for (int64_t i = 16 * n16 + threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+  const int64_t pieces = (n + 15) >> 4;
+  for (int64_t i0 = threadIdx.x; i0 < pieces; i0 += 4 * (int64_t)blockDim.x) {
+    Bytes16 v[4];
+    int64_t at[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t o = 16 * (i0 + u * (int64_t)blockDim.x);
+      at[u] = o < n - 16 ? o : n - 16;
+      v[u] = *(const Bytes16*)(src + at[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i0 + u * (int64_t)blockDim.x < pieces) *(Bytes16*)(dst + at[u]) = v[u];
+  }
 }
 
 // Several tensors packed in one launch. Block (c, k) writes packed tokens [c * chunk, (c + 1) *
@@ -153,7 +161,13 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
   }
 }
 
-struct Fill { char bytes[16]; int n; };
+// Fill pattern of n <= 16 bytes. When n divides 16 the words hold it repeated (16-byte stores).
+// (Words selected, not bytes indexed: an indexed argument would be copied to scratch memory.)
+struct Fill { uint32_t w[4]; int n; };
+DEVI char fill_byte(const Fill& f, int i) {
+  const uint32_t x = i < 8 ? (i < 4 ? f.w[0] : f.w[1]) : (i < 12 ? f.w[2] : f.w[3]);
+  return (char)(x >> (8 * (i & 3)));
+}
 
 // n bytes at dst (the start of an element) filled with the pattern by the whole block: 16-byte
 // stores of the repeated pattern when its length divides 16, byte by byte otherwise and at the end.
@@ -162,17 +176,12 @@ DEVI void block_fill_bytes(char* dst, int64_t n, const Fill& f) {
   if ((16 % f.n) == 0) {
     Bytes16 pat;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      uint32_t x = 0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) x |= (uint32_t)(uint8_t)f.bytes[(4 * w + k) % f.n] << (8 * k);
-      pat.w[w] = x;
-    }
+    for (int w = 0; w < 4; ++w) pat[w] = f.w[w];
     const int64_t n16 = n >> 4;
     for (int64_t i = threadIdx.x; i < n16; i += blockDim.x) *(Bytes16*)(dst + 16 * i) = pat;
     done = 16 * n16;
   }
-  for (int64_t i = done + threadIdx.x; i < n; i += blockDim.x) dst[i] = f.bytes[i % f.n];
+  for (int64_t i = done + threadIdx.x; i < n; i += blockDim.x) dst[i] = fill_byte(f, (int)(i % f.n));
 }
 
 // Tokens per block of the row-wise kernels below: 16 KiB of an element, at most 2048 tokens.
@@ -234,6 +243,59 @@ __global__ __launch_bounds__(PK_THREADS) void realign_kernel(const char* src, ch
       t = stop;
     }
     ++s;
+  }
+}
+
+// A packed batch with one more sequence behind it: block (c, k) writes tokens [c * chunk, (c + 1) * chunk)
+// of tensor k, those below `total` copied, the rest filled (arange: 0, 1, 2, ... in the int64 channels
+// of a token). No sequence moves, so nothing is searched; the first block also writes the two
+// cu_seqlens arrays. One launch: six tensors of 557 Ki tokens took six launches of 20 us, this 6.7 us.
+struct PadArgs {
+  const char* src[PK_MAX_TENSORS];
+  char* dst[PK_MAX_TENSORS];
+  int64_t eb[PK_MAX_TENSORS];
+  Fill fill[PK_MAX_TENSORS];
+  int arange;  // bit k: tensor k
+  const int32_t* cu;
+  int32_t* cu_copy;
+  int32_t* cu_new;
+  int n_seqs, n_tensors;
+  int64_t total, total_new;
+  int chunk;
+};
+__global__ __launch_bounds__(PK_THREADS) void pad_packed_kernel(PadArgs a) {
+  const int k = blockIdx.y;
+  if (k == 0 && blockIdx.x == 0) {
+    for (int i = threadIdx.x; i <= a.n_seqs; i += PK_THREADS) {
+      const int32_t c = a.cu[i];
+      a.cu_copy[i] = c;
+      a.cu_new[i] = c;
+    }
+    if (threadIdx.x == 0) a.cu_new[a.n_seqs + 1] = (int32_t)a.total_new;
+  }
+  if (k >= a.n_tensors) return;
+  const char* src = a.src[0]; char* dst = a.dst[0]; int64_t eb = a.eb[0];
+  uint32_t f0 = a.fill[0].w[0], f1 = a.fill[0].w[1], f2 = a.fill[0].w[2], f3 = a.fill[0].w[3];
+  int fn = a.fill[0].n;
+#pragma unroll
+  for (int i = 1; i < PK_MAX_TENSORS; ++i)
+    if (k == i) {
+      src = a.src[i]; dst = a.dst[i]; eb = a.eb[i];
+      f0 = a.fill[i].w[0]; f1 = a.fill[i].w[1]; f2 = a.fill[i].w[2]; f3 = a.fill[i].w[3];
+      fn = a.fill[i].n;
+    }
+  const int64_t t0 = (int64_t)blockIdx.x * a.chunk;
+  const int64_t t1 = t0 + a.chunk < a.total_new ? t0 + a.chunk : a.total_new;
+  const int64_t tc = t1 < a.total ? t1 : a.total, tf = t0 > a.total ? t0 : a.total;
+  if (t0 < tc) block_copy_bytes(dst + t0 * eb, src + t0 * eb, (tc - t0) * eb);
+  if (tf < t1) {
+    if ((a.arange >> k) & 1) {
+      const int64_t per = eb >> 3;  // int64 channels per token
+      for (int64_t i = threadIdx.x; i < (t1 - tf) * per; i += PK_THREADS)
+        ((int64_t*)(dst + tf * eb))[i] = tf - a.total + i / per;
+    } else {
+      block_fill_bytes(dst + tf * eb, (t1 - tf) * eb, Fill{{f0, f1, f2, f3}, fn});
+    }
   }
 }
 
@@ -317,9 +379,10 @@ __global__ __launch_bounds__(PK_THREADS) void stats_final_kernel(const StatPart*
 bool make_fill(const void* fill, int fill_bytes, Fill& f) {
   if (fill_bytes < 0 || fill_bytes > 16) return false;
   f.n = fill_bytes > 0 ? fill_bytes : 1;
-  for (int i = 0; i < 16; ++i) f.bytes[i] = 0;
+  for (int i = 0; i < 4; ++i) f.w[i] = 0;
   if (fill_bytes > 0 && fill != nullptr)
-    for (int i = 0; i < fill_bytes; ++i) f.bytes[i] = ((const char*)fill)[i];
+    for (int i = 0; i < 16; ++i)  // (a length that does not divide 16: the words past it are not read)
+      f.w[i >> 2] |= (uint32_t)((const uint8_t*)fill)[i % fill_bytes] << (8 * (i & 3));
   return true;
 }
 
@@ -420,6 +483,40 @@ int areal_realign_packed(const void* src, void* dst, const int32_t* cu_old, int6
   hipLaunchKernelGGL(realign_kernel, dim3((unsigned)chunks), dim3(PK_THREADS), 0, stream,
                      (const char*)src, (char*)dst, cu_old, (int)n_old, cu_new, (int)n_new,
                      elem_bytes, f, position_ids, total_new, (int)chunk);
+  AREAL_CHECK_LAUNCH();
+  return AREAL_OK;
+}
+
+// A packed batch padded to total_new > total tokens by one more sequence (data.py:927-969), up to 8
+// tensors (host arrays) in one launch: dst[k] [total_new] <- src[k] [total], the rest filled with
+// fills[16 k .. 16 k + fill_bytes[k]) repeated, or, where position_ids[k] != 0 (elem_bytes a multiple of
+// 8), with 0, 1, 2, ... cu_copy [n_seqs + 1] <- cu_seqlens, cu_new [n_seqs + 2] <- cu_seqlens, total_new.
+int areal_pad_packed_multi(const void* const* src, void* const* dst, const int64_t* elem_bytes, const void* fills,
+                           const int* fill_bytes, const int* position_ids, int n_tensors,
+                           const int32_t* cu_seqlens, int64_t n_seqs, int32_t* cu_copy, int32_t* cu_new,
+                           int64_t total, int64_t total_new, hipStream_t stream) {
+  if (n_tensors < 0 || n_tensors > PK_MAX_TENSORS || n_seqs < 0 || total < 0 || total_new <= total)
+    return AREAL_ERR_BAD_ARG;
+  if (!cu_seqlens || !cu_copy || !cu_new) return AREAL_ERR_BAD_ARG;
+  if (n_tensors > 0 && (!src || !dst || !elem_bytes || !fills || !fill_bytes || !position_ids)) return AREAL_ERR_BAD_ARG;
+  if (n_seqs > (1 << 30) || total_new >= ((int64_t)1 << 31)) return AREAL_ERR_UNSUPPORTED;
+  PadArgs a{};
+  int64_t max_eb = 1;
+  for (int k = 0; k < n_tensors; ++k) {
+    if (!dst[k] || elem_bytes[k] <= 0 || (total > 0 && !src[k])) return AREAL_ERR_BAD_ARG;
+    if (position_ids[k]) {
+      if (elem_bytes[k] % 8 != 0 || ((uintptr_t)dst[k] & 7)) return AREAL_ERR_ALIGNMENT;
+      a.arange |= 1 << k;
+    }
+    if (!make_fill((const char*)fills + 16 * k, fill_bytes[k], a.fill[k])) return AREAL_ERR_BAD_ARG;
+    a.src[k] = (const char*)src[k]; a.dst[k] = (char*)dst[k]; a.eb[k] = elem_bytes[k];
+    max_eb = elem_bytes[k] > max_eb ? elem_bytes[k] : max_eb;
+  }
+  a.cu = cu_seqlens; a.cu_copy = cu_copy; a.cu_new = cu_new; a.n_seqs = (int)n_seqs; a.n_tensors = n_tensors;
+  a.total = total; a.total_new = total_new; a.chunk = (int)pk_chunk_tokens(max_eb);
+  const int64_t chunks = ceil_div_i64(total_new, a.chunk);
+  hipLaunchKernelGGL(pad_packed_kernel, dim3((unsigned)chunks, (unsigned)(n_tensors > 0 ? n_tensors : 1)),
+                     dim3(PK_THREADS), 0, stream, a);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }

@@ -12,6 +12,7 @@ longest sequence, which the reference returns as Python ints as well).
 from __future__ import annotations
 
 import ctypes
+import itertools
 import math
 from typing import Any
 
@@ -29,8 +30,12 @@ def _elem_bytes(t: torch.Tensor, lead_dims: int) -> int:
 
 def _fill_bytes(dtype: torch.dtype, value: float):
     """Bit pattern of ``value`` in ``dtype`` as a ctypes buffer (<= 16 bytes)."""
-    raw = torch.tensor([value], dtype=dtype).view(torch.uint8).numpy().tobytes()
+    raw = _fill_pattern(dtype, value)
     return ctypes.create_string_buffer(raw, len(raw)), len(raw)
+
+
+def _fill_pattern(dtype: torch.dtype, value: float) -> bytes:
+    return torch.tensor([value], dtype=dtype).view(torch.uint8).numpy().tobytes()
 
 
 def pack_tensor_dict(data: dict[str, Any]) -> dict[str, Any]:
@@ -42,16 +47,17 @@ def pack_tensor_dict(data: dict[str, Any]) -> dict[str, Any]:
     lib = _lib.load()
     dev = _lib.require_gpu(attention_mask)
     bs, seq_len = attention_mask.shape
-    mask_u8 = (attention_mask != 0).contiguous().view(torch.uint8)
-    lens = torch.empty(bs, dtype=torch.int32, device=dev)
-    cu_seqlens = torch.empty(bs + 1, dtype=torch.int32, device=dev)
-    max_len = torch.empty(1, dtype=torch.int32, device=dev)
+    mask_u8 = attention_mask if attention_mask.dtype == torch.bool else attention_mask != 0
+    mask_u8 = mask_u8.contiguous().view(torch.uint8)
+    # one array, so that its last two entries (total and longest) travel to the host in one copy
+    lens = torch.empty(2 * bs + 2, dtype=torch.int32, device=dev)
+    cu_seqlens, max_len = lens[bs : 2 * bs + 1], lens[2 * bs + 1 :]
     rc = lib.areal_seqlens_from_mask(
         _lib.ptr(mask_u8), bs, seq_len, _lib.ptr(lens), _lib.ptr(cu_seqlens), _lib.ptr(max_len),
         _lib.stream_ptr(dev),
     )
     _lib.check(rc, "areal_seqlens_from_mask")
-    total_length, max_seqlen = torch.stack([cu_seqlens[-1], max_len[0]]).tolist()  # the one host copy
+    total_length, max_seqlen = lens[2 * bs :].tolist()  # the one host copy
     packed_data: dict[str, Any] = {}
     moved = []  # (contiguous source, packed destination) of the tensors that are packed
     for key, value in data.items():
@@ -117,10 +123,10 @@ def pad_packed_tensor_dict(
     dev = _lib.require_gpu(cu_seqlens)
     cu_seqlens = cu_seqlens.to(torch.int32).contiguous()
     max_seqlen = data["max_seqlen"]
-    old_cu_seqlens = cu_seqlens.clone()
     n_seqs = cu_seqlens.numel() - 1
     align_to_length = None
     if seq_align_to is not None:
+        old_cu_seqlens = cu_seqlens.clone()
         input_lens = cu_seqlens[1:] - cu_seqlens[:-1]
         lens_padded = input_lens + (-input_lens) % seq_align_to
         cu_padded = torch.zeros(n_seqs + 1, dtype=torch.int32, device=dev)
@@ -163,24 +169,58 @@ def pad_packed_tensor_dict(
     pad_length = pad_to_length - total_length
     if pad_length < 0:
         raise ValueError(f"pad_to_length {pad_to_length} is smaller than total length {total_length}.")
+    if seq_align_to is None:
+        old_cu_seqlens = torch.empty_like(cu_seqlens)
     if pad_length == 0:
+        if seq_align_to is None:
+            old_cu_seqlens.copy_(cu_seqlens)
         return data, pad_length, old_cu_seqlens, align_to_length
-    new_cu = torch.nn.functional.pad(cu_seqlens, (0, 1), value=pad_to_length)
+    # one more sequence behind the others: eight tensors per launch, the first of which also writes the
+    # two cu_seqlens arrays
+    new_cu = torch.empty(n_seqs + 2, dtype=torch.int32, device=dev)
+    cu_copy = old_cu_seqlens if seq_align_to is None else torch.empty_like(cu_seqlens)
     padded: dict[str, Any] = {}
+    moved = []  # (contiguous source, destination, is it the position ids)
     for key, value in data.items():
         if key == "cu_seqlens":
             padded[key] = new_cu
         elif key == "max_seqlen":
             padded[key] = max(max_seqlen, pad_length)
-        elif key == "position_ids":
-            padded[key] = _realign(lib, dev, value, cu_seqlens, n_seqs, new_cu, n_seqs + 1, pad_to_length,
-                                   0.0, True, False)
-        elif is_token_tensor(key, value, total_length):
-            padded[key] = _realign(lib, dev, value.reshape(total_length), cu_seqlens, n_seqs, new_cu,
-                                   n_seqs + 1, pad_to_length, pad_value, False, False)
-        else:
+        elif not is_token_tensor(key, value, total_length):
             padded[key] = value
+        elif key == "position_ids" and (value.dtype != torch.int64 or value.shape[:1] != (total_length,)):
+            padded[key] = _realign(lib, dev, value, cu_seqlens, n_seqs, _batch_pad(cu_seqlens, pad_to_length),
+                                   n_seqs + 1, pad_to_length, 0.0, True, False)
+        else:
+            _lib.require_gpu(value)
+            src = (value if key == "position_ids" else value.reshape(total_length)).contiguous()
+            padded[key] = torch.empty((pad_to_length, *src.shape[1:]), dtype=src.dtype, device=src.device)
+            moved.append((src, padded[key], key == "position_ids"))
+    _pad_tensors(lib, dev, moved, pad_value, cu_seqlens, n_seqs, cu_copy, new_cu, total_length, pad_to_length)
     return padded, pad_length, old_cu_seqlens, align_to_length
+
+
+def _batch_pad(cu_seqlens, pad_to_length):
+    return torch.nn.functional.pad(cu_seqlens, (0, 1), value=pad_to_length)
+
+
+def _pad_tensors(lib, dev, moved, pad_value, cu_seqlens, n_seqs, cu_copy, new_cu, total, total_new):
+    fills = {dtype: _fill_pattern(dtype, pad_value) for dtype in {s.dtype for s, _, ids in moved if not ids}}
+    for i in range(0, max(len(moved), 1), _PACK_MAX_TENSORS):
+        part = moved[i : i + _PACK_MAX_TENSORS]
+        n = len(part)
+        patterns = [b"\0" if ids else fills[s.dtype] for s, _, ids in part]
+        rc = lib.areal_pad_packed_multi(
+            (ctypes.c_void_p * n)(*[s.data_ptr() for s, _, _ in part]),
+            (ctypes.c_void_p * n)(*[d.data_ptr() for _, d, _ in part]),
+            (ctypes.c_int64 * n)(*[_elem_bytes(s, 1) for s, _, _ in part]),
+            b"".join(p.ljust(16, b"\0") for p in patterns),
+            (ctypes.c_int * n)(*[len(p) for p in patterns]),
+            (ctypes.c_int * n)(*[int(ids) for _, _, ids in part]),
+            n, _lib.ptr(cu_seqlens), n_seqs, _lib.ptr(cu_copy), _lib.ptr(new_cu), total, total_new,
+            _lib.stream_ptr(dev),
+        )
+        _lib.check(rc, "areal_pad_packed_multi")
 
 
 def unpack_reorder_pad(
@@ -198,8 +238,11 @@ def unpack_reorder_pad(
         assert len(set(backward_indices)) == n
     if sum(seqlens) != packed.shape[0]:
         raise ValueError(f"seqlens sum to {sum(seqlens)}, the packed tensor has {packed.shape[0]} rows")
-    cu = torch.tensor([0] + list(torch.tensor(seqlens, dtype=torch.int64).cumsum(0)), dtype=torch.int32).to(dev)
-    row_seq = torch.tensor(backward_indices, dtype=torch.int32).to(dev) if backward_indices is not None else None
+    # the offsets and the order travel in one copy
+    order = backward_indices if backward_indices is not None else ()
+    table = torch.tensor([0, *itertools.accumulate(seqlens), *order], dtype=torch.int32).to(dev)
+    cu = table[: n + 1]
+    row_seq = table[n + 1 :] if backward_indices is not None else None
     max_len = max(seqlens) if n > 0 else 0
     src = packed.contiguous()
     out = torch.empty((n, max_len, *packed.shape[1:]), dtype=packed.dtype, device=dev)

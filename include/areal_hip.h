@@ -548,6 +548,14 @@ int areal_realign_packed(const void* src, void* dst, const int32_t* cu_old, int6
                          const int32_t* cu_new, int64_t n_new, int64_t elem_bytes,
                          const void* fill, int fill_bytes, int position_ids, int64_t total_new,
                          areal_stream_t stream);
+/* One more sequence behind a packed batch (total -> total_new > total tokens), up to 8 tensors (HOST
+ * arrays) in one launch: dst[k] [total_new] = src[k] [total], then the first fill_bytes[k] of the 16 bytes
+ * at fills + 16 k repeated, or 0, 1, 2, ... (int64 elements) where position_ids[k] != 0. cu_copy [n_seqs + 1]
+ * and cu_new [n_seqs + 2] receive cu_seqlens, the latter with total_new behind it. */
+int areal_pad_packed_multi(const void* const* src, void* const* dst, const int64_t* elem_bytes,
+                           const void* fills, const int* fill_bytes, const int* position_ids,
+                           int n_tensors, const int32_t* cu_seqlens, int64_t n_seqs, int32_t* cu_copy,
+                           int32_t* cu_new, int64_t total, int64_t total_new, areal_stream_t stream);
 size_t areal_masked_stats_workspace_bytes(int K);
 /* out [K][4] double = {sum, count, min, max} of values[k] where masks[k] != 0 (NULL mask: all).
  * values / masks are HOST arrays of K <= 32 device pointers. */
