@@ -1335,7 +1335,8 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_apply_seg_kernel(NormArgs a
 // Reward scores of a batch (actor.py:197-206): clip((reward + bias) * scaling, -clip, clip) and, with
 // `normed`, their group or batch normalisation (no leave-one-out; groups of rows by a.goff), in one
 // launch of one block: a batch has at most a few thousand rows, and the chain of tensor operations and
-// the normalisation's two launches cost 5 us each. A wave takes whole groups.
+// the normalisation's two launches cost 5 us each. A wave takes whole groups. (Group levels alone:
+// reward_score_groups_kernel.)
 constexpr int SCORE_THREADS = 1024;
 __global__ __launch_bounds__(SCORE_THREADS) void reward_score_kernel(NormArgs a, float bias, float scaling, float clip,
                                                                      int normed) {
@@ -1377,6 +1378,39 @@ __global__ __launch_bounds__(SCORE_THREADS) void reward_score_kernel(NormArgs a,
     const NormParams np = norm_params(a, g, v);
     for (int64_t i = g0 + lane; i < g1; i += 64) a.out[i] = norm_one(np, a.out[i], 1.f, false);
   }
+}
+
+// The same where no level is the batch: a wave of any block takes a whole group and needs nothing
+// else, so the groups spread over the CUs (one block walks 64 groups of 16 rows in 10.2 us, latency of
+// one group after the other; this 4.7). Rows behind the last group are only shaped.
+__global__ __launch_bounds__(256) void reward_score_groups_kernel(NormArgs a, float bias, float scaling, float clip) {
+  const int lane = threadIdx.x & 63, g = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (g > a.G) return;
+  auto shaped = [&](int64_t i) {
+    const float x = (a.x[i] + bias) * scaling;
+    return x != x ? x : (x < -clip ? -clip : (x > clip ? clip : x));
+  };
+  const int64_t g0 = a.goff[g], g1 = g < a.G ? a.goff[g + 1] : a.n;
+  if (g == a.G) {
+    for (int64_t i = g0 + lane; i < g1; i += 64) a.out[i] = shaped(i);
+    return;
+  }
+  double v[10];
+#pragma unroll
+  for (int k = 0; k < 10; ++k) v[k] = 0.0;
+  double s1 = 0.0, s4 = 0.0;
+  for (int64_t i = g0 + lane; i < g1; i += 64) {
+    const double x = (double)shaped(i);
+    s1 += x;
+    s4 += x * x;
+  }
+  s1 = wave_sum(s1);
+  s4 = wave_sum(s4);
+  v[0] = v[2] = (double)(g1 - g0);
+  v[1] = v[3] = s1;
+  v[4] = s4;
+  const NormParams np = norm_params(a, g, v);
+  for (int64_t i = g0 + lane; i < g1; i += 64) a.out[i] = norm_one(np, shaped(i), 1.f, false);
 }
 
 // pass 2: sum of squared masked deviations per (group, split)
@@ -2131,8 +2165,12 @@ int areal_reward_scores(const float* rewards, int64_t n, float bias, float scali
   NormArgs a{};
   a.x = rewards; a.n = n; a.goff = group_offsets; a.grows = group_rows; a.G = (int)n_groups; a.tail_group = tail_group;
   a.mean_level = mean_level; a.std_level = std_level; a.unbiased = unbiased; a.eps = eps; a.out = out;
-  hipLaunchKernelGGL(reward_score_kernel, dim3(1), dim3(SCORE_THREADS), 0, stream, a, bias, scaling, clip,
-                     n_groups > 0 ? 1 : 0);
+  if (n_groups > 0 && mean_level != LEVEL_BATCH && std_level != LEVEL_BATCH)
+    hipLaunchKernelGGL(reward_score_groups_kernel, dim3((unsigned)ceil_div_i64(n_groups + 1, 4)), dim3(256), 0, stream,
+                       a, bias, scaling, clip);
+  else
+    hipLaunchKernelGGL(reward_score_kernel, dim3(1), dim3(SCORE_THREADS), 0, stream, a, bias, scaling, clip,
+                       n_groups > 0 ? 1 : 0);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }
