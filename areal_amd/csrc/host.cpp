@@ -12,6 +12,7 @@
 #include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -101,7 +102,9 @@ Tensor flat(const Tensor& t, at::ScalarType type) {
 // memory until the pattern is gone (about a microsecond after the kernel's store, where a copy
 // queued behind the kernel, its event and the synchronisation take about 15); after 200 us of that
 // the stream is synchronised instead. A result that nobody waits for keeps its memory out of the
-// pinned allocator's hands until the stream has passed the point of its destruction.
+// pinned allocator's hands until the stream has passed the point of its destruction. In a captured
+// graph, which may be replayed after that memory has gone to someone else, the results stay on the
+// device (`results`, the graph's own memory) and whoever asks for them copies them then.
 // ---------------------------------------------------------------------------------------
 constexpr uint64_t PENDING = 0x7ff8a5c3d2e1f0b4ull;  // a NaN payload arithmetic does not make
 
@@ -115,21 +118,27 @@ void keep_until_passed(const Tensor& pinned, const c10::hip::HIPStream& stream) 
 }
 
 struct HostResult {
-  Tensor host;  // fp64, pinned
+  Tensor host;    // fp64, pinned
+  Tensor device;  // the results of a captured call
   c10::hip::HIPStream stream;
   bool done = false;
 
-  HostResult(int64_t n, const Tensor& like)
-      : host(at::empty({n}, at::TensorOptions().dtype(at::kDouble).pinned_memory(true))),
-        stream(c10::hip::getCurrentHIPStream(like.device().index())) {
+  explicit HostResult(const Tensor& results) : stream(c10::hip::getCurrentHIPStream(results.device().index())) {
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) {
+      device = results;
+      return;
+    }
+    const int64_t n = results.numel();
+    host = at::empty({n}, at::TensorOptions().dtype(at::kDouble).pinned_memory(true));
     uint64_t* p = (uint64_t*)host.data_ptr();
     for (int64_t i = 0; i < n; ++i) p[i] = PENDING;
     std::atomic_thread_fence(std::memory_order_release);
   }
   ~HostResult() {
-    if (!done && !arrived()) keep_until_passed(host, stream);
+    if (!done && host.defined() && !arrived()) keep_until_passed(host, stream);
   }
   double* data() { return (double*)host.data_ptr(); }
+  double* target() { return host.defined() ? data() : nullptr; }  // where kernels write the results
   bool arrived() const {
     const volatile uint64_t* p = (const volatile uint64_t*)host.data_ptr();
     for (int64_t i = host.numel() - 1; i >= 0; --i)
@@ -140,6 +149,11 @@ struct HostResult {
   void wait() {
     if (done) return;
     py::gil_scoped_release no_gil;
+    if (device.defined()) {
+      host = device.cpu();
+      done = true;
+      return;
+    }
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
     while (!arrived()) {
       if (std::chrono::steady_clock::now() > until) {
@@ -285,7 +299,7 @@ py::tuple actor_loss(const Tensor& logprobs, const Tensor& proximal, const OptTe
   const Tensor dlp = grad ? empty(lp, {n}, at::kFloat) : Tensor();
   const int64_t n_results = 9 + (stats ? 4 * N_STATS : 0);
   const Tensor results = empty(lp, {n_results}, at::kDouble);
-  auto host = std::make_shared<HostResult>(n_results, lp);
+  auto host = std::make_shared<HostResult>(results);
   io.logprobs = ptr<float>(lp); io.proximal_logprobs = ptr<float>(prox); io.old_logprobs = ptr<float>(old);
   io.advantages = ptr<float>(adv); io.loss_mask = ptr<uint8_t>(mask); io.cu_seqlens = ptr<int32_t>(cu);
   io.entropy = ptr<float>(ent); io.extra0 = ptr<float>(x0); io.extra1 = ptr<float>(x1);
@@ -308,7 +322,7 @@ py::tuple actor_loss(const Tensor& logprobs, const Tensor& proximal, const OptTe
   io.logp_abs_diff = f32("logp_abs_diff", logged);
   io.behave_filtered_ratio = f32("behave_filtered_ratio", logged && rs);
   io.results = ptr<double>(results);
-  io.host_results = host->data();
+  io.host_results = host->target();
   io.with_stats = stats;
   io.nan_if_nonfinite = nan_if_nonfinite;
   const size_t bytes = stats ? areal_actor_loss_stats_workspace_bytes(n, io.n_seqs)
@@ -327,13 +341,13 @@ HostResultPtr proximal_stats(const Tensor& proximal, const Tensor& loss_mask) {
   areal_loss_config cfg{};
   cfg.loss_kind = -1;
   const Tensor results = empty(prox, {9 + 4 * N_STATS}, at::kDouble);
-  auto host = std::make_shared<HostResult>(9 + 4 * N_STATS, prox);
+  auto host = std::make_shared<HostResult>(results);
   areal_actor_loss_io io{};
   io.proximal_logprobs = ptr<float>(prox);
   io.loss_mask = ptr<uint8_t>(mask);
   io.n_tokens = mask.numel();
   io.results = ptr<double>(results);
-  io.host_results = host->data();
+  io.host_results = host->target();
   io.with_stats = 1;
   const size_t bytes = areal_actor_loss_stats_workspace_bytes(io.n_tokens, 0);
   const Tensor ws = workspace(prox, bytes);
@@ -396,8 +410,9 @@ py::tuple sapo_loss(const Tensor& logprobs, const Tensor& old_logprobs, const Te
         "areal_sapo_loss");
   HostResultPtr host;
   if (reduced) {
-    host = std::make_shared<HostResult>(n_results, lp);
-    if (hipMemcpyAsync(host->data(), results.data_ptr(), n_results * sizeof(double), hipMemcpyDeviceToHost,
+    host = std::make_shared<HostResult>(results);
+    if (host->target() != nullptr &&
+        hipMemcpyAsync(host->data(), results.data_ptr(), n_results * sizeof(double), hipMemcpyDeviceToHost,
                        (hipStream_t)stream_of(lp)) != hipSuccess)
       fail("copy of the statistics to the host failed");
   }
