@@ -162,7 +162,7 @@ class Variant:
         # the first k-tile of a pair (stage 0) advances by the selected amount
         post.setdefault(7 * step + 1, []).extend(self.advance(oper, eff=(stage == 0)))
 
-    def ktile(self, parity, init, dead=False, na=8):
+    def ktile(self, parity, init, dead=False, na=8, landed="8"):
         stage = parity
         barrier = ["s_barrier"]
         out = [f"; ---- k-tile on stage {stage}{' (dead: no MFMA)' if dead else ''}: k-step 0"]
@@ -173,7 +173,7 @@ class Variant:
         self.spread(self.a_reads(1, stage, 1, na), 9, 40, post)
         out += self.kstep(self.fa[0], self.fb[parity][0], init, pre, post, dead, na)
         # own A reads done and own loads of one k-tile ago landed (the 8 newest may be in flight)
-        out += ["s_waitcnt vmcnt(8) lgkmcnt(0)"] + barrier
+        out += [f"s_waitcnt vmcnt({landed}) lgkmcnt(0)"] + barrier
         out += [f"; ---- k-tile on stage {stage}: k-step 1"]
         # k-step 1: the A half of this stage is free: refill it; from the other stage (landed,
         # published by the barrier) A fragments of k-step 0 -> A buffer 0 and all B fragments
@@ -187,8 +187,9 @@ class Variant:
         out += ["s_waitcnt lgkmcnt(0)"] + barrier
         return out
 
-    def pair(self, init, dead_second=False, na=8):
-        return self.select_advance() + self.ktile(0, init, False, na) + self.ktile(1, False, dead_second, na)
+    def pair(self, init, dead_second=False, na=8, landed="8"):
+        return (self.select_advance() + self.ktile(0, init, False, na, landed)
+                + self.ktile(1, False, dead_second, na))
 
     def tile_loop(self, na=8):
         """One 256 x 256 tile: s48 pairs of k-tiles, the second k-tile of the last pair dead when
@@ -196,11 +197,15 @@ class Variant:
         are receiving) k-tiles 0 and 1 and the pointers are on the next k-tile to fetch.
         na < 8: a tile of 32 na x 256, each wave's sub-tile 16 na x 128: the loads, barriers and B
         fragment reads are those of the full tile; the fragment reads and MFMAs of the A blocks
-        ia >= na are left out."""
-        out = ["s_waitcnt vmcnt(0) lgkmcnt(0)", "s_barrier"]
+        ia >= na are left out.
+        %[pending] = vector memory operations (stores of the epilogue before) that every wave has issued
+        since its last operand load, or 0; %[landed] = 8 more. Such operations retire in order, so the
+        loads have landed when all but that many are done, and the first k-tile starts while the
+        stores are still on their way; the second one's loads are behind them."""
+        out = ["s_waitcnt vmcnt(%[pending]) lgkmcnt(0)", "s_barrier"]
         out += self.a_reads(0, 0, 0, na) + self.b_reads(0, 0)
         out += ["s_waitcnt lgkmcnt(0)", "s_barrier"]
-        out += self.pair(True, False, na)
+        out += self.pair(True, False, na, "%[landed]")
         out += [f"s_sub_u32 s{S_CNT}, s{S_CNT}, 1", f"s_cmp_eq_u32 s{S_CNT}, 0", "s_cbranch_scc1 2f", "1:",
                 # the last pair fetches the next tile's first k-tiles
                 f"s_cmp_eq_u32 s{S_CNT}, 1",

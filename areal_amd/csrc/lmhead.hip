@@ -1123,11 +1123,13 @@ DEVI void setup_operand16(int64_t ld, int first, int nvalid, int W, int oper, in
 // last 256-wide tile badly (896 = 3.5 x 256 = 4 x 224) wastes nothing. NA is the epilogue's (Epi::NA).
 template <int VAR, class Epi>
 __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, typename Epi::Params ep) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[RING16_BYTES + 4 * STAGE16_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[RING16_BYTES + 4 * (STAGE16_BYTES + Epi::TOKEN_BYTES)];
   constexpr bool A_KM = VAR != VAR_NT, B_KM = VAR == VAR_TN;
   constexpr int NA = Epi::NA;
   static_assert(NA == 8 || (NA == 7 && A_KM), "narrow A tiles need a k-major A");
   constexpr int TM = NA * 32;  // A rows (output index i) per tile
+  // Stores that every complete epilogue leaves in flight: the next tile starts without waiting for them.
+  constexpr int PENDING = Epi::PENDING_STORES;
   int bj, split, ai_begin, ai_end;
   int wg = blockIdx.x, nk = g.K / BK, z = 0;
   if (gemm_skipped(g)) return;
@@ -1199,6 +1201,11 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
                    ML16_MIX_VGPR_INPUTS(oa, ob, ra, rb)
                  : "memory", "scc");
 
+  // what the epilogue needs to know of the wave's 128 output rows j, from LDS at every tile of the sweep
+  unsigned char* const tokens = lds + RING16_BYTES + 4 * STAGE16_BYTES + wave * Epi::TOKEN_BYTES;
+  if constexpr (Epi::TOKEN_BYTES > 0) Epi::load_tokens(ep, bj * TILE + wb * 128, lane, tokens);
+  if (PENDING > 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the first tile follows no epilogue
+
   // What an epilogue carries from tile to tile of a sweep has to be small: over the main loop the
   // compiler only has v[0:ML16_*_FIRST_VGPR) for it.
   typename Epi::State st;
@@ -1213,35 +1220,40 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
                    : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
                    : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
                      ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_NT_VGPR_INPUTS(oa, ob, ra, rb)
+                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_NT_VGPR_INPUTS(oa, ob, ra, rb),
+                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
                    : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_NT_CLOBBERS, ML16_ACC_CLOBBERS);
     else if (VAR == VAR_TN && NA == 7)
       asm volatile(ML16_TN_TILE7
                    : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
                    : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
                      ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_TN_VGPR_INPUTS(oa, ob, ra, rb)
+                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_TN_VGPR_INPUTS(oa, ob, ra, rb),
+                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
                    : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_TN_CLOBBERS, ML16_ACC_CLOBBERS);
     else if (VAR == VAR_TN)
       asm volatile(ML16_TN_TILE
                    : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
                    : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
                      ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_TN_VGPR_INPUTS(oa, ob, ra, rb)
+                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_TN_VGPR_INPUTS(oa, ob, ra, rb),
+                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
                    : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_TN_CLOBBERS, ML16_ACC_CLOBBERS);
     else if (NA == 7)
       asm volatile(ML16_MIX_TILE7
                    : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
                    : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
                      ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_MIX_VGPR_INPUTS(oa, ob, ra, rb)
+                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_MIX_VGPR_INPUTS(oa, ob, ra, rb),
+                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
                    : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_MIX_CLOBBERS, ML16_ACC_CLOBBERS);
     else
       asm volatile(ML16_MIX_TILE
                    : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
                    : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
                      ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_MIX_VGPR_INPUTS(oa, ob, ra, rb)
+                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_MIX_VGPR_INPUTS(oa, ob, ra, rb),
+                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
                    : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_MIX_CLOBBERS, ML16_ACC_CLOBBERS);
     // The lane number goes through an empty block so that nothing of the epilogue's per-lane
     // address arithmetic is computed ahead of the main loop, which leaves the compiler only
@@ -1249,7 +1261,9 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
     Epi::open(st, ep, bj * TILE + wb * 128, split, wa, lane_e, ai == ai_begin);
-    Epi::tile(st, ep, a_row0(ai) + wa * (NA * 16), bj * TILE + wb * 128, lane_e, stage, ai * TM);
+    const bool complete = Epi::tile(st, ep, a_row0(ai) + wa * (NA * 16), bj * TILE + wb * 128, lane_e, stage, ai * TM,
+                                    tokens);
+    if (PENDING > 0 && !complete) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     Epi::close(st, ep, bj * TILE + wb * 128, split, wa, lane_e);
   }
   __builtin_amdgcn_s_waitcnt(0x0070);  // drain the trailing (unused) loads before LDS is released
@@ -1298,14 +1312,14 @@ DEVI void stage16_put(u16* stage, int lane, int ia, u32x2 v) {
 template <bool EDGE, int MODE, int NA_>
 struct Store16Impl {
   static_assert(NA_ == 8 || EDGE, "narrow tiles use the bounds-checked instance");
-  static constexpr int NA = NA_;
+  static constexpr int NA = NA_, TOKEN_BYTES = 0, PENDING_STORES = 0;
   typedef StoreParams Params;
   struct State {};
   static DEVI void open(State&, const Params&, int, int, int, int, bool) {}
   static DEVI void close(State&, const Params&, int, int, int, int) {}
   static DEVI void end(State&, const Params&, int, int, int, int) {}
   static DEVI void split_output(Params& p, int64_t bytes) { p.out = (char*)p.out + bytes; }
-  static DEVI void tile(State&, const Params& p, int i0, int j0, int lane, u16* stage, int) {
+  static DEVI bool tile(State&, const Params& p, int i0, int j0, int lane, u16* stage, int, const void*) {
     // bf16: column b leaves the staging area while column b + 1 is fetched and converted
     u32x4 left[4];
     int cols_valid = p.M - i0;
@@ -1352,6 +1366,7 @@ struct Store16Impl {
         }
       }
     });
+    return true;
   }
 };
 template <bool EDGE, int MODE> struct Store16 : Store16Impl<EDGE, MODE, 8> {};
@@ -1415,6 +1430,11 @@ template <bool EDGE, bool AFFINE, bool MOMENTS, bool SAVE>
 struct Fwd16 {
   static constexpr int NA = 8;
   static constexpr bool RAGGED_B = true;
+  static constexpr int TOKEN_BYTES = 1024;
+  // An interior tile's: 8 columns of 4. Waiting for them before the next tile starts cost 1.5 to 3 % of the
+  // sweep, together with the loads that load_tokens replaces (against dHidden's time in the same run: 4096 x 896
+  // 1.40 -> 1.36, 8192 x 1536 1.217 -> 1.201, 32768 x 4096 1.060 -> 1.042).
+  static constexpr int PENDING_STORES = SAVE && !EDGE ? 32 : 0;
   typedef FwdParams Params;
   // SAVE: s and q are relative to the row reference of the saved exponentials (fixed for the whole
   // sweep: nothing is rescaled); otherwise relative to the running maximum m.
@@ -1433,11 +1453,27 @@ struct Fwd16 {
   }
   static DEVI void close(State&, const Params&, int, int, int, int) {}
 
+  // Labels (-1: none in the vocabulary) and row references of the wave's 128 tokens, once per sweep. Fetched
+  // from memory at every tile they would be waited for behind the next tile's first operand loads.
+  static DEVI void load_tokens(const Params& p, int t0, int lane, void* tokens) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // (a token past the end reads the last one's)
+      int t = t0 + h * 64 + lane;
+      t = t < p.T ? t : p.T - 1;
+      const int64_t l = p.labels[t];
+      ((int*)tokens)[h * 64 + lane] = l >= 0 && l < p.V ? (int)l : -1;
+      if (SAVE) ((float*)tokens)[128 + h * 64 + lane] = p.probs_ref[t];
+    }
+  }
+
   // v_new: the first vocabulary entry of the tile that no earlier tile of the sweep covered (the
   // last tile of a ragged vocabulary overlaps its predecessor); entries below it take no part.
-  static DEVI void tile(State& st, const Params& p, int v0, int t0, int lane, u16* stage, int v_new) {
-    if (v_new >= v0 + 128) return;    // every row of this wave's sub-tile is a repeat
-    if (t0 >= p.T) return;            // no token
+  // Returns whether all PENDING_STORES stores were issued.
+  static DEVI bool tile(State& st, const Params& p, int v0, int t0, int lane, u16* stage, int v_new,
+                        const void* tokens) {
+    if (v_new >= v0 + 128) return false;  // every row of this wave's sub-tile is a repeat
+    if (t0 >= p.T) return false;          // no token
     const bool overlap = v_new > v0;  // wave-uniform
     const int vl = v0 + 4 * (lane >> 4);
     const int group = lane >> 4;
@@ -1447,13 +1483,10 @@ struct Fwd16 {
     float rr[SAVE ? 8 : 1];
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      // (a token past the end reads the last one's: a predicate per load would have each waited for in turn)
-      int t = t0 + b * 16 + (lane & 15);
-      t = t < p.T ? t : p.T - 1;
-      const int64_t l = p.labels[t];
-      lab[b] = (l >= v_new && l < p.V) ? (int)l : -1;
-      if (SAVE) rr[b] = p.probs_ref[t];
+      lab[b] = ((const int*)tokens)[b * 16 + (lane & 15)];
+      if (SAVE) rr[b] = ((const float*)tokens)[128 + b * 16 + (lane & 15)];
     }
+    const int v_from = overlap ? v_new : v0;
     float* const label_logit = p.ws + 3 * (int64_t)p.P * p.T;
     auto add = [](float a, float b) { return a + b; };
     auto lower = [](float a, float b) { return fminf(a, b); };
@@ -1556,7 +1589,7 @@ struct Fwd16 {
           stage16_store<true, true>(left, out, p.ldv, 16, (int)p.ldv - v0, overlap ? v_new - v0 : 0, lane);
       }
       // the label's logit, if it is one of this lane's 32 entries (about one wave in 70 has one)
-      const bool hit = (lab[b] >= v0) && (lab[b] < v0 + 128);
+      const bool hit = (lab[b] >= v_from) && (lab[b] < v0 + 128);
       if (__builtin_amdgcn_ballot_w64(hit) != 0) {
         float xl = 0.f;
 #pragma unroll
@@ -1615,6 +1648,7 @@ struct Fwd16 {
       }
       __builtin_amdgcn_sched_barrier(0);
     });
+    return !overlap;
   }
 
   static DEVI void end(State& st, const Params& p, int t0, int split, int wa, int lane) {
@@ -1645,6 +1679,7 @@ template <bool EDGE, bool AFFINE>
 struct Bwd16 {
   static constexpr int NA = 8;
   static constexpr bool RAGGED_B = EDGE;
+  static constexpr int TOKEN_BYTES = 0, PENDING_STORES = 0;
   typedef BwdParams Params;
   struct State {
     float nb[8], gs[8];
@@ -1669,7 +1704,7 @@ struct Bwd16 {
   static DEVI void split_output(Params&, int64_t) {}
 
   // (a tile that overlaps its predecessor rewrites the shared rows with the same values)
-  static DEVI void tile(State& st, const Params& p, int v0, int t0, int lane, u16* stage, int) {
+  static DEVI bool tile(State& st, const Params& p, int v0, int t0, int lane, u16* stage, int, const void*) {
     const int vl = v0 + 4 * (lane >> 4);
     u32x4 left[4];  // column b leaves the staging area while column b + 1 is computed
     auto store_column = [&](int b) {
@@ -1714,6 +1749,7 @@ struct Bwd16 {
       __builtin_amdgcn_sched_barrier(0);
       if (b == 7) store_column(b);
     });
+    return true;
   }
 };
 template <bool E> using Bwd16Plain = Bwd16<E, false>;
