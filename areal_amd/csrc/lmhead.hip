@@ -1980,7 +1980,10 @@ void split_ktiles(int nk, int& z, int& kps) {
 
 // Layout and copies of the dHidden launch by estimated microseconds of the busiest XCD: a k-tile takes
 // 1.15 us while 32 neighbouring workgroups read at most about 14 distinct tiles, and proportionally
-// longer beyond (the 128-byte row pieces of e come from outside L2 at about 3 TB/s), a workgroup's
+// longer beyond (the 128-byte row pieces of e come from outside L2 at about 3 TB/s; with fewer than 32
+// tiles per XCD, where more copies only mean more loads under way, 1 % a tile, and proportionally
+// beyond 26: dHidden of 509 x 896 138 -> 118 us with 32 copies for 24, whole steps of 256 x 896, 400 x 2560 and
+// 512 x 5120 6 to 10 % faster), a workgroup's
 // start and its epilogue 8 us, the reduction of the partial results 5 us and their bytes (written
 // and read) at 4.5 TB/s. Few output tiles then go to all XCDs (kg > 1), each with its own k range.
 // z_fixed > 0: the number of copies is given (of a token chunk: that of the whole batch, so that
@@ -2002,7 +2005,8 @@ DhPlan plan_dh(int64_t H, int64_t T, int64_t K, int z_fixed = 0) {
         if (z_fixed > 0 && z != z_fixed) continue;
         const int copies = tiles >= 32 ? 1 : (int)ceil_div_i64(32, tiles);
         double distinct = tiles >= 32 ? xcd_distinct(nb, na) : (double)(copies < zk ? copies : zk) * (na + nb);
-        const double slow = distinct > 14.0 ? distinct / 14.0 : 1.0;
+        double slow = distinct > 14.0 ? distinct / 14.0 : 1.0;
+        if (tiles < 32 && distinct > 14.0) slow = (1.0 + 0.01 * (distinct - 14.0)) * (distinct > 26.0 ? distinct / 26.0 : 1.0);
         const double rounds = (double)ceil_div_i64((int64_t)tiles * zk, 32);
         double cost = rounds * (1.15 * slow * (double)nk / z + 8.0);
         if (z > 1) cost += 5.0 + (double)z * (double)(T * H) * 8.0 / 4.5e6;
