@@ -1982,7 +1982,7 @@ void split_ktiles(int nk, int& z, int& kps) {
 // 1.15 us while 32 neighbouring workgroups read at most about 14 distinct tiles, and proportionally
 // longer beyond (the 128-byte row pieces of e come from outside L2 at about 3 TB/s; with fewer than 32
 // tiles per XCD, where more copies only mean more loads under way, 1 % a tile, and proportionally
-// beyond 26: dHidden of 509 x 896 138 -> 118 us with 32 copies for 24, whole steps of 256 x 896, 400 x 2560 and
+// beyond 26: dHidden of 509 x 896 138 -> 120 us with 32 copies for 24, whole steps of 256 x 896, 400 x 2560 and
 // 512 x 5120 6 to 10 % faster), a workgroup's
 // start and its epilogue 8 us, the reduction of the partial results 5 us and their bytes (written
 // and read) at 4.5 TB/s. Few output tiles then go to all XCDs (kg > 1), each with its own k range.

@@ -112,13 +112,30 @@ DEVI int seq_search(const LossIO& io, int64_t t, int lane) {
   else s = wave_count_le(io.cu + 1, io.n_seqs, t, lane);
   return s < io.n_seqs ? s : io.n_seqs - 1;
 }
-// ... and from a sequence that starts at or before t.
-DEVI int seq_from(const LossIO& io, int s, int64_t t) {
-  while (s + 1 < io.n_seqs && seq_end(io, s) <= t) ++s;
-  return s;
-}
 DEVI bool needs_seq(const LossCfg& c) {
   return (c.rs_enabled && c.rs_seq_level) || (c.loss_kind == LOSS_PPO && c.seq_is);
+}
+// A token's sequence and what the token kernel reads of it, in registers until the next one starts (a
+// thread's four tokens nearly always share it). s < 0: no sequences.
+struct SeqCtx {
+  int s;
+  int64_t end;        // its last token's successor (of the last sequence: none)
+  float rs_ok, rs_w;  // seq_rs
+  float ratio, adv, sum_w, inv_count;  // seq_is
+};
+// Moves on from a sequence that starts at or before t (first: loads it in any case).
+DEVI void seq_advance(const LossIO& io, const LossCfg& c, int64_t t, bool first, SeqCtx& q) {
+  if (!first && t < q.end) return;
+  for (;;) {
+    q.end = q.s + 1 < io.n_seqs ? seq_end(io, q.s) : INT64_MAX;
+    if (t < q.end) break;
+    ++q.s;
+  }
+  if (c.rs_enabled && c.rs_seq_level) { q.rs_ok = io.seq_rs[2 * q.s]; q.rs_w = io.seq_rs[2 * q.s + 1]; }
+  if (c.loss_kind == LOSS_PPO && c.seq_is) {
+    q.ratio = io.seq_is[4 * q.s]; q.adv = io.seq_is[4 * q.s + 1];
+    q.sum_w = io.seq_is[4 * q.s + 2]; q.inv_count = io.seq_is[4 * q.s + 3];
+  }
 }
 
 // torch.clamp keeps NaN (fminf/fmaxf would drop it).
@@ -256,15 +273,14 @@ __global__ __launch_bounds__(LOSS_THREADS) void seq_rs_kernel(LossIO io, LossCfg
 
 // Rejection sampling for one token. Returns the narrowed mask; sets w (not yet zeroed outside
 // the mask) and whether the token counts as filtered / clamped.
-DEVI bool rs_token(const LossIO& io, const LossCfg& c, int s, bool m, float prox, float old, float& w,
-                   bool& counted) {
+DEVI bool rs_token(const LossCfg& c, const SeqCtx& q, bool m, float prox, float old, float& w, bool& counted) {
   const float lr = sane_log_ratio(prox, old);
   w = expf(lr);
   bool keep = true;
   counted = false;
   if (c.rs_seq_level) {
-    const bool seq_ok = io.seq_rs[2 * s] != 0.0f;
-    if (c.rs_metric == METRIC_RATIO) w = io.seq_rs[2 * s + 1];
+    const bool seq_ok = q.rs_ok != 0.0f;
+    if (c.rs_metric == METRIC_RATIO) w = q.rs_w;
     if (c.rs_clamp) {
       const float orig = w;
       if (!seq_ok) w = torch_clamp(w, c.rs_has_lower ? c.rs_lower : 0.0f, c.rs_upper);
@@ -360,15 +376,15 @@ struct TokenOut {
   bool clip, dual, m2, bm;
 };
 
-template <bool STATS>
-DEVI void token_body(const LossIO& io, const LossCfg& c, int s, const TokenIn& in, TokenOut& out,
+template <bool STATS, bool LEAN>
+DEVI void token_body(const LossIO& io, const LossCfg& c, const SeqCtx& q, const TokenIn& in, TokenOut& out,
                      TokenAcc& acc, StatAcc<STATS>& st) {
   const bool m = in.m;
   bool m2 = m;
   float w = 1.0f;
   if (c.rs_enabled) {
     bool counted;
-    m2 = rs_token(io, c, s, m, in.prox, in.old, w, counted);
+    m2 = rs_token(c, q, m, in.prox, in.old, w, counted);
     w = m2 ? w : 0.0f;
     acc.n_filtered += counted;
   }
@@ -384,7 +400,7 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, int s, const TokenIn& i
   }
   out.dlp = 0.f; out.loss = 0.f; out.ratio = 0.f; out.kl = 0.f; out.behave_kl = 0.f;
   out.clip = false; out.dual = false; out.bm = false;
-  if (c.loss_kind == LOSS_NONE) return;
+  if (!LEAN && c.loss_kind == LOSS_NONE) return;
 
   const float lp = in.lp, prox = in.prox, adv = in.adv;
   const float kl = lp - prox;
@@ -401,8 +417,8 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, int s, const TokenIn& i
   } else {
     float ratio, a = adv, dratio;  // dratio = d ratio / d lp[t] factor handled below
     if (c.seq_is) {
-      ratio = m2 ? io.seq_is[4 * s + 0] : 0.0f;
-      a = m2 ? io.seq_is[4 * s + 1] : 0.0f;
+      ratio = m2 ? q.ratio : 0.0f;
+      a = m2 ? q.adv : 0.0f;
       dratio = 0.f;  // gradient assembled per sequence below
     } else {
       ratio = m ? expf(kl) : 0.0f;
@@ -428,7 +444,7 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, int s, const TokenIn& i
     }
     if (c.seq_is) {
       // every kept token of the sequence receives ratio_s/count_s * sum_w_s * dpg_s
-      dsel = m2 ? dpg * ratio * io.seq_is[4 * s + 2] * io.seq_is[4 * s + 3] : 0.0f;
+      dsel = m2 ? dpg * ratio * q.sum_w * q.inv_count : 0.0f;
     } else {
       dsel = dpg * dratio;
     }
@@ -495,8 +511,8 @@ DEVI void token_group_load(const LossIO& io, const LossCfg& c, int64_t t, TokenL
   load_f32<VEC>(STATS ? io.extra0 : nullptr, t, in.x0);
   load_f32<VEC>(STATS ? io.extra1 : nullptr, t, in.x1);
 }
-template <bool STATS, int VEC>
-DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, int s, const TokenLoad<VEC>& ld,
+template <bool STATS, int VEC, bool LEAN>
+DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, SeqCtx& q, const TokenLoad<VEC>& ld,
                               TokenAcc& acc, StatAcc<STATS>& st) {
   float dlp[VEC], loss[VEC], ratio[VEC], kl[VEC], bw[VEC], bkl[VEC];
   bool clip[VEC], dual[VEC], m2[VEC], bm[VEC];
@@ -504,10 +520,14 @@ DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, int
   for (int i = 0; i < VEC; ++i) {
     const TokenIn in{ld.lp[i], ld.prox[i], ld.old[i], ld.adv[i], ld.ent[i], ld.x0[i], ld.x1[i], ld.m[i]};
     TokenOut o;
-    if (s >= 0) s = seq_from(io, s, t + i);
-    token_body<STATS>(io, c, s, in, o, acc, st);
+    if (q.s >= 0) seq_advance(io, c, t + i, i == 0, q);
+    token_body<STATS, LEAN>(io, c, q, in, o, acc, st);
     dlp[i] = o.dlp; loss[i] = o.loss; ratio[i] = o.ratio; kl[i] = o.kl; bw[i] = o.behave_w; bkl[i] = o.behave_kl;
     clip[i] = o.clip; dual[i] = o.dual; m2[i] = o.m2; bm[i] = o.bm;
+  }
+  if (LEAN) {
+    store_f32<VEC>(io.dlp, t, dlp);
+    return;
   }
   if (c.rs_enabled) {
     store_mask<VEC>(io.new_mask, t, m2);
@@ -544,7 +564,11 @@ DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, int
 
 // STATS: also reduce the logged statistics (sum, min, max per block) into stat_partials
 // [gridDim.x][N_LOSS_STATS]; min / max propagate NaN as torch.min / torch.max do.
-template <bool STATS, int VEC>
+// LEAN: a loss, and no per-token output but its gradient. Bound by issue slots, not by the 21 bytes of a
+// token: the addresses of fifteen arrays that are not there do not fit the scalar registers, and their
+// tests and spills (300 reloads), with a sequence's end and aggregates fetched once and not per token, were
+// a sixth of it: 4 Mi tokens in 2048 sequences 32.2 -> 27.5 us.
+template <bool STATS, int VEC, bool LEAN>
 __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, LossCfg c,
                                                                    Partial* partials,
                                                                    StatPartial* stat_partials) {
@@ -560,17 +584,19 @@ __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, Los
   TokenLoad<VEC> in;
   const int64_t wid = gid & ~(int64_t)63;
   for (int64_t t = gid * VEC, tw = wid * VEC; tw < n_vec; t += nthreads * VEC, tw += nthreads * VEC) {
-    const int s = seq ? seq_search(io, tw, threadIdx.x & 63) : -1;
+    if (t < n_vec) token_group_load<STATS, VEC>(io, c, t, in);  // (in flight during the search)
+    SeqCtx q{};
+    q.s = seq ? seq_search(io, tw, threadIdx.x & 63) : -1;
     if (t >= n_vec) continue;
-    token_group_load<STATS, VEC>(io, c, t, in);
-    token_group_compute<STATS, VEC>(io, c, t, s, in, acc, st);
+    token_group_compute<STATS, VEC, LEAN>(io, c, t, q, in, acc, st);
   }
   if (VEC > 1 && n_vec + wid < io.n) {
-    const int s = seq ? seq_search(io, n_vec + wid, threadIdx.x & 63) : -1;
+    SeqCtx q{};
+    q.s = seq ? seq_search(io, n_vec + wid, threadIdx.x & 63) : -1;
     if (n_vec + gid < io.n) {
       TokenLoad<1> tail;
       token_group_load<STATS, 1>(io, c, n_vec + gid, tail);
-      token_group_compute<STATS, 1>(io, c, n_vec + gid, s, tail, acc, st);
+      token_group_compute<STATS, 1, LEAN>(io, c, n_vec + gid, q, tail, acc, st);
     }
   }
 
@@ -1050,14 +1076,23 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
   int grid = loss_grid(n_tokens, vec4 ? 4 : 1);
   if (with_stats && grid > MAX_LOSS_BLOCKS / 2) grid = MAX_LOSS_BLOCKS / 2;
   auto token_pass = [&](const LossIO& i, const LossCfg& cc, bool stats) {
-    if (stats && vec4)
-      hipLaunchKernelGGL((loss_token_kernel<true, 4>), dim3(grid), dim3(LOSS_THREADS), 0, stream, i, cc, partials, stat_partials);
-    else if (stats)
-      hipLaunchKernelGGL((loss_token_kernel<true, 1>), dim3(grid), dim3(LOSS_THREADS), 0, stream, i, cc, partials, stat_partials);
-    else if (vec4)
-      hipLaunchKernelGGL((loss_token_kernel<false, 4>), dim3(grid), dim3(LOSS_THREADS), 0, stream, i, cc, partials, (StatPartial*)nullptr);
-    else
-      hipLaunchKernelGGL((loss_token_kernel<false, 1>), dim3(grid), dim3(LOSS_THREADS), 0, stream, i, cc, partials, (StatPartial*)nullptr);
+    const bool lean = cc.loss_kind != LOSS_NONE && !i.stat_loss && !i.stat_ratio && !i.stat_kl && !i.clip_mask &&
+                      !i.dual_mask && !i.new_mask && !i.behave_w && !i.behave_kl && !i.behave_mask && !i.logp_diff;
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(LOSS_THREADS), 0, stream, i, cc, partials,
+                         stats ? stat_partials : (StatPartial*)nullptr);
+    };
+    if (lean) {
+      if (stats && vec4) launch(loss_token_kernel<true, 4, true>);
+      else if (stats) launch(loss_token_kernel<true, 1, true>);
+      else if (vec4) launch(loss_token_kernel<false, 4, true>);
+      else launch(loss_token_kernel<false, 1, true>);
+    } else {
+      if (stats && vec4) launch(loss_token_kernel<true, 4, false>);
+      else if (stats) launch(loss_token_kernel<true, 1, false>);
+      else if (vec4) launch(loss_token_kernel<false, 4, false>);
+      else launch(loss_token_kernel<false, 1, false>);
+    }
   };
   if (n_tokens > 0 && c.rs_enabled && c.rs_seq_level) {
     // below about 1024 tokens a sequence does not give four waves two groups of four per lane

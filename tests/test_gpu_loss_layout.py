@@ -98,3 +98,27 @@ def test_proximal_log_prob_that_is_not_finite(value, sapo):
         grpo_loss_fn(lp, torch.zeros_like(lp), data, **kw)
     if not sapo:
         assert torch.isnan(grpo_loss_fn(lp, torch.zeros_like(lp), data, defer_host_reads=True, **kw))
+
+
+@pytest.mark.parametrize("lens", [[1], [3, 0, 5], [1, 2, 3, 4, 5, 6, 7, 8, 9] * 30, [2, 0, 0, 1, 3] * 60000, [262144, 1, 5]])
+@pytest.mark.parametrize("level", ["token", "sequence"])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_gradient_does_not_depend_on_what_is_logged(lens, level, offset):
+    """Several sequences inside a thread's four tokens, empty ones among them; bit for bit."""
+    prox, old, mask, cu, g = _batch(lens, offset)
+    n, dev = prox.numel(), prox.device
+    lp = (prox + 0.1 * torch.randn(n, generator=g).to(dev)).requires_grad_(True)
+    data = dict(logprobs=old, prox_logp=prox, advantages=torch.randn(n, generator=g).to(dev), loss_mask=mask,
+                cu_seqlens=cu)
+    rs = (RejectionSamplingConfig(level="token", action="mask", metric="ratio", lower=0.9, upper=1.1) if level == "token"
+          else RejectionSamplingConfig(level="sequence", action="clamp", metric="ratio", agg="mean", upper=1.003))
+    results = []
+    for stats, mode in ((None, "tensors"), ({}, "tensors"), ({}, "reduced")):
+        lp.grad = None
+        loss = grpo_loss_fn(lp, torch.zeros(n, device=dev), data, eps_clip=0.2, eps_clip_higher=None, c_clip=None,
+                            rejection_sampling=rs, stats=stats, stats_mode=mode)
+        loss.backward()
+        results.append((loss.detach(), lp.grad))
+    for loss, grad in results[1:]:
+        assert torch.equal(grad, results[0][1])
+        torch.testing.assert_close(loss, results[0][0], rtol=1e-6, atol=1e-7)  # (other blocks: fp64 sums in another order)
