@@ -21,7 +21,9 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <initializer_list>
 #include <optional>
+#include <utility>
 #include <vector>
 
 #include "../../include/areal_hip.h"
@@ -68,6 +70,13 @@ void require_gpu(const T&... ts) {
   };
   (one(ts), ...);
   if (first == nullptr) fail("no tensor given");
+}
+
+// A kernel reads n elements of every array of a call, whatever an array's own size is.
+void require_numel(int64_t n, std::initializer_list<std::pair<const char*, const Tensor*>> arrays) {
+  for (const auto& [name, t] : arrays)
+    if (t->defined() && t->numel() != n)
+      fail(std::string(name) + " has " + std::to_string(t->numel()) + " elements, expected " + std::to_string(n));
 }
 
 Tensor or_undefined(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
@@ -253,6 +262,8 @@ py::tuple actor_loss(const Tensor& logprobs, const Tensor& proximal, const OptTe
                      const OptTensor& entropy, const OptTensor& extra0, const OptTensor& extra1) {
   const areal_loss_config cfg = loss_config(config);
   const Tensor old_arg = or_undefined(old_logprobs);
+  require_numel(loss_mask.numel(), {{"logprobs", &logprobs}, {"proximal_logprobs", &proximal},
+                                    {"old_logprobs", &old_arg}, {"advantages", &advantages}});
   require_gpu(proximal, loss_mask, logprobs, old_arg, advantages);
   const c10::hip::HIPGuard guard(proximal.device().index());
   const at::IntArrayRef shape = logprobs.sizes();
@@ -335,6 +346,7 @@ py::tuple actor_loss(const Tensor& logprobs, const Tensor& proximal, const OptTe
 // Tokens whose proximal log-prob is not finite, and its statistics under the mask: a host result [9 + 18 * 4]
 // of which entry 8 and row 17 are set (for the losses whose own kernels do not read it).
 HostResultPtr proximal_stats(const Tensor& proximal, const Tensor& loss_mask) {
+  require_numel(loss_mask.numel(), {{"proximal_logprobs", &proximal}});
   require_gpu(proximal, loss_mask);
   const c10::hip::HIPGuard guard(proximal.device().index());
   const Tensor prox = flat(proximal, at::kFloat), mask = flat(loss_mask, at::kBool);
@@ -364,6 +376,7 @@ py::tuple sapo_loss(const Tensor& logprobs, const Tensor& old_logprobs, const Te
                     const Tensor& loss_mask, const OptTensor& cu_seqlens, double tau_pos, double tau_neg,
                     bool seq_level, bool reduced, const OptTensor& entropy, const OptTensor& extra0,
                     const OptTensor& extra1) {
+  require_numel(loss_mask.numel(), {{"logprobs", &logprobs}, {"old_logprobs", &old_logprobs}, {"advantages", &advantages}});
   require_gpu(logprobs, old_logprobs, advantages, loss_mask);
   const c10::hip::HIPGuard guard(logprobs.device().index());
   const at::IntArrayRef shape = logprobs.sizes();
@@ -422,6 +435,7 @@ py::tuple sapo_loss(const Tensor& logprobs, const Tensor& old_logprobs, const Te
 py::tuple critic_loss(const Tensor& value, const Tensor& old_value, const Tensor& target_value,
                       const OptTensor& loss_mask, double eps_clip, bool huber) {
   const Tensor mask_arg = or_undefined(loss_mask);
+  require_numel(value.numel(), {{"old_value", &old_value}, {"target_value", &target_value}, {"loss_mask", &mask_arg}});
   require_gpu(value, old_value, target_value, mask_arg);
   const c10::hip::HIPGuard guard(value.device().index());
   const Tensor v = flat(value, at::kFloat), old = flat(old_value, at::kFloat), target = flat(target_value, at::kFloat),
