@@ -805,6 +805,8 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
     const float c = gam * (LAMBDAS ? g.lam_seq[s_last] : g.lam);
     const bool boot = g.no_eos != nullptr && g.no_eos[s_last] != 0;
     const int64_t n_right = (e - t_end + GAE_TILE - 1) / GAE_TILE;
+    // (without values the mask is read in their place and dropped: no branch between the loads)
+    const float* const values = g.values != nullptr ? g.values : g.mask;
     for (int64_t j = n_right; j > 0; j -= GAE_CARRY_BATCH) {
       const int64_t j0 = j > GAE_CARRY_BATCH ? j - GAE_CARRY_BATCH : 0;
       float rw[GAE_CARRY_BATCH][GAE_ITEMS], v[GAE_CARRY_BATCH][GAE_ITEMS], ms[GAE_CARRY_BATCH][GAE_ITEMS];
@@ -816,7 +818,7 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
 #pragma unroll
           for (int q = 0; q < GAE_ITEMS / 4; ++q) {
             const f32x4 a = *(const f32x4*)(g.rewards + t0 + 4 * q);
-            const f32x4 b = *(const f32x4*)(g.values + t0 + 4 * q);
+            const f32x4 b = *(const f32x4*)(values + t0 + 4 * q);
             const f32x4 m = *(const f32x4*)(g.mask + t0 + 4 * q);
 #pragma unroll
             for (int x = 0; x < 4; ++x) { rw[k][4 * q + x] = a[x]; v[k][4 * q + x] = b[x]; ms[k][4 * q + x] = m[x]; }
@@ -826,9 +828,13 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
           for (int i = 0; i < GAE_ITEMS; ++i) {
             const bool in = live && t0 + i < g.n;
             rw[k][i] = in ? g.rewards[t0 + i] : 0.f;
-            v[k][i] = in ? g.values[t0 + i] : 0.f;
+            v[k][i] = in ? values[t0 + i] : 0.f;
             ms[k][i] = in ? g.mask[t0 + i] : 0.f;
           }
+        }
+        if (g.values == nullptr) {
+#pragma unroll
+          for (int i = 0; i < GAE_ITEMS; ++i) v[k][i] = 0.f;
         }
       }
       MapF part[GAE_CARRY_BATCH];

@@ -5,6 +5,7 @@ one-launch reward scores; against the oracle (fp32 recurrences, fp64 sums: 1e-5 
 import pytest
 import torch
 
+from areal_amd import _lib
 from areal_amd.config import NormConfig
 from areal_amd.data import KLEstimator, Normalization
 from areal_amd.ppo.actor import compute_advantages
@@ -72,3 +73,34 @@ def test_packed_advantages(lens, group, levels):
         rows[i, : b - a], row_mask[i, : b - a] = want[a:b], mask[a:b]
     normed = N.normalization(rows, row_mask, mean_level=levels[0], std_level=levels[1], group_size=group)
     _close(got, torch.cat([normed[i, :k] for i, k in enumerate(lens)]))
+
+
+@pytest.mark.parametrize("lambdas", [False, True])
+@pytest.mark.parametrize("lens,group", [([2049], 1), ([7000, 3], 1), ([1500, 9000, 100, 2047], 2)])
+def test_packed_advantages_without_values(lens, group, lambdas):
+    """The C entry point with values = NULL: sequences that go on in the next tiles carry a state without them
+    (bitwise what explicit zeros give)."""
+    g = torch.Generator().manual_seed(sum(lens))
+    n, n_seqs = sum(lens), len(lens)
+    lib = _lib.load()
+    cu = torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32).to(DEV)
+    mask, rewards = (torch.rand(n, generator=g) > 0.2).float().to(DEV), torch.randn(n, generator=g).to(DEV)
+    lam = torch.rand(n_seqs, generator=g).to(DEV) if lambdas else None
+    no_eos = torch.arange(n_seqs, device=DEV) % 2 == 0
+    first = torch.arange(0, n_seqs + 1, group, device=DEV)
+    rows = torch.full((n_seqs // group,), group, device=DEV)
+    size = lib.areal_gae_segment_stats_bytes(n, rows.numel())
+
+    def call(values):
+        outs = [torch.empty(n, device=DEV) for _ in range(3)]
+        scratch = torch.empty(size, dtype=torch.uint8, device=DEV)
+        rc = lib.areal_gae_packed_normalized(
+            _lib.ptr(rewards), _lib.ptr(values), _lib.ptr(mask), _lib.ptr(cu), _lib.ptr(no_eos), _lib.ptr(lam), n, n_seqs,
+            1.0, 0.95, _lib.ptr(first), _lib.ptr(rows), rows.numel(), -1, 2, 2, 1, 1e-5, *[_lib.ptr(o) for o in outs],
+            _lib.ptr(scratch), size, _lib.stream_ptr(DEV),
+        )
+        _lib.check(rc, "areal_gae_packed_normalized")
+        return outs
+
+    for got, want in zip(call(None), call(torch.zeros(n, device=DEV))):
+        assert torch.equal(got, want)
