@@ -522,8 +522,8 @@ struct Status {  // an int in pinned host memory, -1 until the forward's last ke
 // State of one forward for its backward. The exponentials are consumed by the first backward (it
 // rewrites entries of them in place); a second one recomputes.
 // owner: the fp32 master of `weight`. Its .grad is looked up when the backward runs: an existing one is
-// added to by the contraction, a missing one is allocated and stored to (not cleared first and then
-// read back: 3 x 4 bytes per weight less).
+// added to by the contraction (behind it, if its strides are not the kernels'), a missing one is
+// allocated and stored to (not cleared first and then read back: 3 x 4 bytes per weight less).
 struct LMHeadState {
   Tensor probs, probs_ref, probs_status, label_logprobs, bias, accum, owner;
   std::shared_ptr<Status> status;
@@ -595,8 +595,13 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
   // epilogue adds to it and no gradient is returned for the weight
   Tensor accum = st->accum;
   bool add = accum.defined();
+  Tensor strided;  // a .grad of the owner that the kernels cannot write to: theirs is added to it at the end
   if (st->owner.defined()) {
     accum = st->owner.grad();
+    if (accum.defined() && !(accum.layout() == at::kStrided && accum.scalar_type() == at::kFloat &&
+                             accum.device() == saved[1].device() && accum.sizes() == saved[1].sizes() &&
+                             accum.is_contiguous()))
+      std::swap(strided, accum);
     add = accum.defined();
   }
   if (add || st->owner.defined()) need_w = true;
@@ -611,7 +616,7 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
   const Tensor dh = need_h ? at::empty_like(h2) : Tensor();
   if (st->owner.defined() && !add) {
     accum = empty(h2, {V, H}, at::kFloat);
-    st->owner.mutable_grad() = accum;
+    if (!strided.defined()) st->owner.mutable_grad() = accum;
   }
   // (the kernels add to the bias gradient as well when they add to the weight's)
   const Tensor db32 = need_b ? (add ? at::zeros({V}, h2.options().dtype(at::kFloat)) : empty_f32(h2, V)) : Tensor();
@@ -677,6 +682,10 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
       check(areal_cast_f32_to_bf16(ptr<float>(dw32), ptr<void>(dw), dw32.numel(), stream_of(h2)),
             "areal_cast_f32_to_bf16");
     }
+  }
+  if (strided.defined()) {
+    const at::NoGradGuard no_grad;
+    strided.add_(accum);
   }
   if (want_h) none[0] = dh.view(st->hidden_shape);
   if (dw.defined()) none[1] = dw;
