@@ -614,10 +614,7 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
   // the kernels need one of dHidden / dWeight as an output; a bias-only request computes dHidden
   need_h = need_h || (need_b && !need_w);
   const Tensor dh = need_h ? at::empty_like(h2) : Tensor();
-  if (st->owner.defined() && !add) {
-    accum = empty(h2, {V, H}, at::kFloat);
-    if (!strided.defined()) st->owner.mutable_grad() = accum;
-  }
+  if (st->owner.defined() && !add) accum = empty(h2, {V, H}, at::kFloat);
   // (the kernels add to the bias gradient as well when they add to the weight's)
   const Tensor db32 = need_b ? (add ? at::zeros({V}, h2.options().dtype(at::kFloat)) : empty_f32(h2, V)) : Tensor();
   const Tensor probs = st->probs, probs_ref = st->probs_ref;
@@ -683,9 +680,12 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
             "areal_cast_f32_to_bf16");
     }
   }
+  // with every launch queued: an error above leaves the owner's .grad as it was
   if (strided.defined()) {
     const at::NoGradGuard no_grad;
     strided.add_(accum);
+  } else if (st->owner.defined() && !add) {
+    st->owner.mutable_grad() = accum;
   }
   if (want_h) none[0] = dh.view(st->hidden_shape);
   if (dw.defined()) none[1] = dw;

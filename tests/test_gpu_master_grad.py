@@ -77,3 +77,26 @@ def test_batch_without_any_loss_leaves_a_gradient_of_zeros(dev, have_grad):
     adapter._scaled_loss = lambda inputs, *args: inputs["hidden"].float().sum()
     adapter.forward_backward_batch(micro, functools.partial(lambda: None), lambda mb: 1.0)
     assert torch.equal(param.grad, torch.ones_like(param) if have_grad else torch.zeros_like(param))
+
+
+def test_failing_backward_sets_no_gradient(dev):
+    """The backward's workspace does not fit: the error leaves no half-made gradient for a smaller batch to be
+    added to."""
+    param, weight, parts = _parts(dev, 1, t=4096, v=16384)
+    out = _forward(param, weight, parts[0], save_probs=False)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    # room for the gradient (8 MiB), not for the 128 MiB of dlogits
+    room = torch.cuda.memory_reserved(dev) + (64 << 20)
+    torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(dev).total_memory, dev)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            out.backward(parts[0][2], retain_graph=True)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert param.grad is None
+    out.backward(parts[0][2])
+    want = torch.zeros_like(param)
+    again = fused_lm_head_logprobs_entropy(parts[0][0], weight, parts[0][1], save_probs=False, weight_grad_accum=want)
+    again.logprobs.backward(parts[0][2])
+    assert torch.equal(param.grad, want)
