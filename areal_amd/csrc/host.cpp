@@ -617,7 +617,8 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
   if (st->owner.defined() && !add) accum = empty(h2, {V, H}, at::kFloat);
   // (the kernels add to the bias gradient as well when they add to the weight's)
   const Tensor db32 = need_b ? (add ? at::zeros({V}, h2.options().dtype(at::kFloat)) : empty_f32(h2, V)) : Tensor();
-  const Tensor probs = st->probs, probs_ref = st->probs_ref;
+  Tensor probs = st->probs;
+  const Tensor probs_ref = st->probs_ref;
   const float inv_t = (float)(1.0 / st->temperature), scale = (float)st->logit_scale;
   // A contraction over the whole batch can store dWeight in bf16 itself: the saved mode always, the
   // recompute mode when one token chunk covers the batch. Several chunks accumulate in fp32 and cast.
@@ -654,6 +655,7 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
     // estimate) those launches did nothing and the recompute mode runs.
     if (st->status->wait() != 0) {
       recompute = true;
+      probs = Tensor();  // (up to 40 GiB, the recompute's workspace up to 24: not both at a time)
       if (need_w && direct && chunk < T) {
         direct = false;
         dw_direct = Tensor();
