@@ -110,8 +110,10 @@ Tensor flat(const Tensor& t, at::ScalarType type) {
 // filled with a bit pattern no result has before they are launched. Waiting means looking at that
 // memory until the pattern is gone (about a microsecond after the kernel's store, where a copy
 // queued behind the kernel, its event and the synchronisation take about 15); after 200 us of that
-// the stream is synchronised instead. A result that nobody waits for keeps its memory out of the
-// pinned allocator's hands until the stream has passed the point of its destruction. In a captured
+// the host sleeps instead: until the stream is idle, or, where more may be queued before anyone waits,
+// until it has passed the point where mark() was called. A result that nobody waits for keeps its
+// memory out of the pinned allocator's hands until the stream has passed the point of its
+// destruction. In a captured
 // graph, which may be replayed after that memory has gone to someone else, the results stay on the
 // device (`results`, the graph's own memory) and whoever asks for them copies them then.
 // ---------------------------------------------------------------------------------------
@@ -126,10 +128,33 @@ void keep_until_passed(const Tensor& pinned, const c10::hip::HIPStream& stream) 
   }
 }
 
+// A point of a stream.
+struct Mark {
+  hipEvent_t event = nullptr;
+  Mark() = default;
+  Mark(const Mark&) = delete;
+  Mark& operator=(const Mark&) = delete;
+  ~Mark() {
+    if (event != nullptr) (void)hipEventDestroy(event);
+  }
+  void set(const c10::hip::HIPStream& stream) {
+    if (event == nullptr && hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess) {
+      event = nullptr;
+      fail("creation of an event failed");
+    }
+    if (hipEventRecord(event, stream.stream()) != hipSuccess) fail("recording an event failed");
+  }
+  void wait(const c10::hip::HIPStream& stream) const {  // without a mark: for all of the stream
+    if (event == nullptr) stream.synchronize();
+    else if (hipEventSynchronize(event) != hipSuccess) fail("waiting for an event failed");
+  }
+};
+
 struct HostResult {
   Tensor host;    // fp64, pinned
   Tensor device;  // the results of a captured call
   c10::hip::HIPStream stream;
+  Mark behind;
   bool done = false;
 
   explicit HostResult(const Tensor& results) : stream(c10::hip::getCurrentHIPStream(results.device().index())) {
@@ -166,11 +191,14 @@ struct HostResult {
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
     while (!arrived()) {
       if (std::chrono::steady_clock::now() > until) {
-        stream.synchronize();
+        behind.wait(stream);
         break;
       }
     }
     done = true;
+  }
+  void mark() {
+    if (!device.defined() && !arrived()) behind.set(stream);
   }
   Tensor value() { wait(); return host; }
   // {key: {sum, count, avg, min, max, denominator}} of rows `offset + 4 * row` of the result; avg, min and max
@@ -496,6 +524,7 @@ struct LMHeadArgs {
 struct Status {  // an int in pinned host memory, -1 until the forward's last kernel has written it
   Tensor host;
   c10::hip::HIPStream stream;
+  Mark behind;
   explicit Status(const Tensor& like)
       : host(at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true))),
         stream(c10::hip::getCurrentHIPStream(like.device().index())) {
@@ -512,10 +541,13 @@ struct Status {  // an int in pinned host memory, -1 until the forward's last ke
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
     while (read() < 0)
       if (std::chrono::steady_clock::now() > until) {
-        stream.synchronize();
+        behind.wait(stream);
         break;
       }
     return read();
+  }
+  void mark() {
+    if (read() < 0) behind.set(stream);
   }
 };
 
@@ -610,6 +642,7 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
   const Tensor &h2 = saved[0], &w = saved[1], &lab = saved[2], &row_max = saved[3], &sum_exp = saved[4];
   const c10::hip::HIPGuard guard(h2.device().index());
   const int64_t T = h2.size(0), H = h2.size(1), V = w.size(0);
+  if (st->probs.defined()) st->status->mark();  // what is queued below is not to be waited for
   const Tensor g = flat(grad, at::kFloat);
   // the kernels need one of dHidden / dWeight as an output; a bias-only request computes dHidden
   need_h = need_h || (need_b && !need_w);
@@ -651,8 +684,9 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
                                  ptr<float>(db32), ptr<void>(ws), bytes, stream_of(h2)),
           "areal_lmhead_bwd_saved");
     // The status travelled to pinned memory with the forward's last kernel. Looking at it now, with the
-    // launches above already queued, idles nothing; if it was set (a row's maximum far above its
-    // estimate) those launches did nothing and the recompute mode runs.
+    // launches above already queued, idles nothing, and waits for the forward (and what was queued up to
+    // this call) alone; if it was set (a row's maximum far above its estimate) those launches did nothing
+    // and the recompute mode runs.
     if (st->status->wait() != 0) {
       recompute = true;
       probs = Tensor();  // (up to 40 GiB, the recompute's workspace up to 24: not both at a time)
@@ -928,6 +962,7 @@ py::tuple turn_gae(const Tensor& rewards, const OptTensor& values, const Tensor&
   if (hipMemcpyAsync(flags.status->host.data_ptr(), status.data_ptr(), sizeof(int), hipMemcpyDeviceToHost,
                      (hipStream_t)stream) != hipSuccess)
     fail("copy of the turn status to the host failed");
+  flags.status->mark();  // the normalisation of the advantages is queued before anyone looks
   return py::make_tuple(adv, ret, flags);
 }
 
@@ -961,6 +996,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("set_error_class", [](py::object cls) { error_class = cls.release().ptr(); });
   py::class_<HostResult, HostResultPtr>(m, "HostResult")
       .def("value", &HostResult::value)
+      .def("mark", &HostResult::mark)
       .def("fill", &HostResult::fill);
   m.def("actor_loss", &actor_loss);
   m.def("proximal_stats", &proximal_stats);

@@ -379,6 +379,8 @@ def _loss_common(cfg, logprobs, proximal_logprobs, old_logprobs, advantages, los
         reduction.entropy if reduction is not None else None,
         extras[0] if len(extras) > 0 else None, extras[1] if len(extras) > 1 else None,
     )
+    if defer:
+        host.mark()  # whoever reads the results waits for this call, not for what is queued behind it
     if reduction is not None:
         if reduction.keep_behave_mask:
             reduction.behave_mask = out.get("behave_mask")
