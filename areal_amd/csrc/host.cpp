@@ -119,6 +119,10 @@ Tensor flat(const Tensor& t, at::ScalarType type) {
 // ---------------------------------------------------------------------------------------
 constexpr uint64_t PENDING = 0x7ff8a5c3d2e1f0b4ull;  // a NaN payload arithmetic does not make
 
+bool capturing() {
+  return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+}
+
 // Called from destructors: nothing may be thrown (a failure only means that the allocator is not told).
 void keep_until_passed(const Tensor& pinned, const c10::hip::HIPStream& stream) noexcept {
   try {
@@ -158,7 +162,7 @@ struct HostResult {
   bool done = false;
 
   explicit HostResult(const Tensor& results) : stream(c10::hip::getCurrentHIPStream(results.device().index())) {
-    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) {
+    if (capturing()) {
       device = results;
       return;
     }
@@ -521,23 +525,31 @@ struct LMHeadArgs {
   int64_t save_limit, bwd_budget;
 };
 
-struct Status {  // an int in pinned host memory, -1 until the forward's last kernel has written it
-  Tensor host;
+// An int that the device makes (`flag`), on its way to the host: in pinned memory, -1 until it has been
+// written there. Of a captured call it stays on the device, as HostResult's, and is read anew each time.
+struct Status {
+  Tensor host, device;
   c10::hip::HIPStream stream;
   Mark behind;
-  explicit Status(const Tensor& like)
-      : host(at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true))),
-        stream(c10::hip::getCurrentHIPStream(like.device().index())) {
+  explicit Status(const Tensor& flag) : stream(c10::hip::getCurrentHIPStream(flag.device().index())) {
+    if (capturing()) {
+      device = flag;
+      return;
+    }
+    host = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
     *(volatile int*)host.data_ptr() = -1;
     std::atomic_thread_fence(std::memory_order_release);
   }
   ~Status() {
-    if (read() < 0) keep_until_passed(host, stream);
+    if (host.defined() && !known()) keep_until_passed(host, stream);
   }
+  int* target() const { return host.defined() ? (int*)host.data_ptr() : nullptr; }  // where kernels write it
   int read() const { return *(volatile int*)host.data_ptr(); }
+  bool known() const { return host.defined() && read() >= 0; }
   int wait() {
-    if (read() >= 0) return read();
+    if (known()) return read();
     py::gil_scoped_release no_gil;
+    if (device.defined()) return device.cpu().item<int>();
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
     while (read() < 0)
       if (std::chrono::steady_clock::now() > until) {
@@ -547,7 +559,7 @@ struct Status {  // an int in pinned host memory, -1 until the forward's last ke
     return read();
   }
   void mark() {
-    if (read() < 0) behind.set(stream);
+    if (host.defined() && !known()) behind.set(stream);
   }
 };
 
@@ -590,7 +602,7 @@ variable_list lm_head_forward(const Tensor& hidden, const Tensor& weight, const 
     lp_copy = rows.narrow(0, 2 * Tp, T);
     probs_ref = rows.narrow(0, 3 * Tp, T);
     probs_status = empty(h2, {1}, at::kInt);
-    status = std::make_shared<Status>(h2);
+    status = std::make_shared<Status>(probs_status);
   }
   if (T > 0) {
     const size_t bytes = areal_lmhead_fwd_workspace_bytes(T, H, V);
@@ -600,7 +612,7 @@ variable_list lm_head_forward(const Tensor& hidden, const Tensor& weight, const 
                               ptr<float>(outs[1]), ptr<float>(outs[2]), ptr<float>(outs[3]), ptr<float>(outs[4]),
                               ptr<float>(outs[5]), ptr<float>(row_max), ptr<float>(sum_exp), ptr<void>(probs),
                               save ? (size_t)need : 0, ptr<float>(probs_ref), ptr<int>(probs_status),
-                              ptr<float>(lp_copy), save ? ptr<int>(status->host) : nullptr, ptr<void>(ws), bytes,
+                              ptr<float>(lp_copy), save ? status->target() : nullptr, ptr<void>(ws), bytes,
                               stream_of(h2)),
           "areal_lmhead_fwd");
   }
@@ -642,7 +654,11 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
   const Tensor &h2 = saved[0], &w = saved[1], &lab = saved[2], &row_max = saved[3], &sum_exp = saved[4];
   const c10::hip::HIPGuard guard(h2.device().index());
   const int64_t T = h2.size(0), H = h2.size(1), V = w.size(0);
-  if (st->probs.defined()) st->status->mark();  // what is queued below is not to be waited for
+  if (st->probs.defined()) {
+    if (!st->status->known() && capturing())
+      fail("this lm_head backward reads a result of its forward on the host and cannot be captured: use save_probs=False");
+    st->status->mark();  // what is queued below is not to be waited for
+  }
   const Tensor g = flat(grad, at::kFloat);
   // the kernels need one of dHidden / dWeight as an output; a bias-only request computes dHidden
   need_h = need_h || (need_b && !need_w);
@@ -926,10 +942,9 @@ Tensor group_norm(const Tensor& x, const OptTensor& mask, const NormTables& norm
   return out;
 }
 
-// An int the device is writing, on its way to the host.
 struct HostInt {
-  std::shared_ptr<Status> status;
-  int wait() const { return status->wait(); }
+  std::shared_ptr<Status> status;  // null: 0
+  int wait() const { return status != nullptr ? status->wait() : 0; }
 };
 
 // (advantages, returns, malformed-id flags)
@@ -946,12 +961,9 @@ py::tuple turn_gae(const Tensor& rewards, const OptTensor& values, const Tensor&
                       : turn_ids.scalar_type() == at::kLong ? turn_ids.clamp(-1, INT32_MAX).to(at::kInt)
                                                             : turn_ids.to(at::kInt)).contiguous();
   const Tensor adv = at::empty_like(r), ret = at::empty_like(r);
-  HostInt flags{std::make_shared<Status>(r)};
-  if (bs == 0 || L == 0) {
-    *(int*)flags.status->host.data_ptr() = 0;
-    return py::make_tuple(adv, ret, flags);
-  }
+  if (bs == 0 || L == 0) return py::make_tuple(adv, ret, HostInt{});
   const Tensor status = at::zeros({1}, r.options().dtype(at::kInt));
+  const HostInt flags{std::make_shared<Status>(status)};
   const size_t bytes = areal_turn_gae_workspace_bytes(bs, L);
   const Tensor ws = workspace(r, bytes);
   const areal_stream_t stream = stream_of(r);
@@ -959,7 +971,8 @@ py::tuple turn_gae(const Tensor& rewards, const OptTensor& values, const Tensor&
                           ptr<float>(lam), ptr<float>(add), bs, L, (float)discount, (float)lambda, ptr<float>(adv),
                           ptr<float>(ret), ptr<int>(status), ptr<void>(ws), bytes, stream),
         "areal_turn_gae");
-  if (hipMemcpyAsync(flags.status->host.data_ptr(), status.data_ptr(), sizeof(int), hipMemcpyDeviceToHost,
+  if (flags.status->target() != nullptr &&
+      hipMemcpyAsync(flags.status->target(), status.data_ptr(), sizeof(int), hipMemcpyDeviceToHost,
                      (hipStream_t)stream) != hipSuccess)
     fail("copy of the turn status to the host failed");
   flags.status->mark();  // the normalisation of the advantages is queued before anyone looks
