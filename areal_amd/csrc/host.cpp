@@ -947,10 +947,10 @@ struct HostInt {
   int wait() const { return status != nullptr ? status->wait() : 0; }
 };
 
-// (advantages, returns, malformed-id flags)
+// (advantages, returns, malformed-id flags: absent unless they are wanted)
 py::tuple turn_gae(const Tensor& rewards, const OptTensor& values, const Tensor& loss_mask, const Tensor& turn_ids,
                    bool roll_ids, const Tensor& no_eos, double discount, double lambda, const OptTensor& lambda_seq,
-                   const OptTensor& addend) {
+                   const OptTensor& addend, bool want_flags) {
   const Tensor v = f32(or_undefined(values)), lam = or_undefined(lambda_seq), add = f32(or_undefined(addend));
   require_gpu(rewards, v, loss_mask, turn_ids, no_eos, lam, add);
   const c10::hip::HIPGuard guard(rewards.device().index());
@@ -961,9 +961,11 @@ py::tuple turn_gae(const Tensor& rewards, const OptTensor& values, const Tensor&
                       : turn_ids.scalar_type() == at::kLong ? turn_ids.clamp(-1, INT32_MAX).to(at::kInt)
                                                             : turn_ids.to(at::kInt)).contiguous();
   const Tensor adv = at::empty_like(r), ret = at::empty_like(r);
-  if (bs == 0 || L == 0) return py::make_tuple(adv, ret, HostInt{});
+  std::optional<HostInt> flags;
+  if (want_flags) flags.emplace();
+  if (bs == 0 || L == 0) return py::make_tuple(adv, ret, flags);
   const Tensor status = at::zeros({1}, r.options().dtype(at::kInt));
-  const HostInt flags{std::make_shared<Status>(status)};
+  if (want_flags) flags->status = std::make_shared<Status>(status);
   const size_t bytes = areal_turn_gae_workspace_bytes(bs, L);
   const Tensor ws = workspace(r, bytes);
   const areal_stream_t stream = stream_of(r);
@@ -971,11 +973,12 @@ py::tuple turn_gae(const Tensor& rewards, const OptTensor& values, const Tensor&
                           ptr<float>(lam), ptr<float>(add), bs, L, (float)discount, (float)lambda, ptr<float>(adv),
                           ptr<float>(ret), ptr<int>(status), ptr<void>(ws), bytes, stream),
         "areal_turn_gae");
-  if (flags.status->target() != nullptr &&
-      hipMemcpyAsync(flags.status->target(), status.data_ptr(), sizeof(int), hipMemcpyDeviceToHost,
+  if (!want_flags) return py::make_tuple(adv, ret, flags);
+  if (flags->status->target() != nullptr &&
+      hipMemcpyAsync(flags->status->target(), status.data_ptr(), sizeof(int), hipMemcpyDeviceToHost,
                      (hipStream_t)stream) != hipSuccess)
     fail("copy of the turn status to the host failed");
-  flags.status->mark();  // the normalisation of the advantages is queued before anyone looks
+  flags->status->mark();  // the normalisation of the advantages is queued before anyone looks
   return py::make_tuple(adv, ret, flags);
 }
 

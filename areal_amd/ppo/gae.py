@@ -184,20 +184,22 @@ def _compute_turn_level_gae(
     """
     _check_turn_ids(turn_ids, loss_mask)
     adv, ret, flags = _turn_level_gae(
-        rewards, values, loss_mask, turn_ids, False, seq_no_eos_mask, discount, gae_lambda, None
+        rewards, values, loss_mask, turn_ids, False, seq_no_eos_mask, discount, gae_lambda, None, validate
     )
     if validate:
         _raise_turn_id_errors(flags.wait())
     return adv, ret
 
 
-def _turn_level_gae(rewards, values, loss_mask, turn_ids, roll_ids, seq_no_eos_mask, discount, gae_lambda, addend):
+def _turn_level_gae(
+    rewards, values, loss_mask, turn_ids, roll_ids, seq_no_eos_mask, discount, gae_lambda, addend, want_flags=True
+):
     """The launch of turn-level GAE: ``(advantages + addend, returns, flags of malformed ids)``, the
-    flags on their way to the host. ``values=None``: all zero; ``roll_ids``: ``turn_ids`` are not rolled
-    to the next-token convention yet."""
+    flags on their way to the host (``want_flags=False``: none, and nothing is queued for them).
+    ``values=None``: all zero; ``roll_ids``: ``turn_ids`` are not rolled to the next-token convention yet."""
     lam_seq, lam = _split_lambda(gae_lambda, rewards.shape[0], rewards.device)
     return _lib.host().turn_gae(
-        rewards, values, loss_mask, turn_ids, roll_ids, seq_no_eos_mask, discount, lam, lam_seq, addend
+        rewards, values, loss_mask, turn_ids, roll_ids, seq_no_eos_mask, discount, lam, lam_seq, addend, want_flags
     )
 
 

@@ -123,3 +123,15 @@ def test_captured_backward_from_saved_exponentials_is_refused(dev):
     got = got.clone()
     torch.cuda.synchronize()
     assert torch.equal(got, step(False))
+
+
+def test_turn_gae_without_validation_takes_no_host_memory(dev):
+    """``validate=False``: nobody reads the flags, so no pinned memory is taken and no copy queued for them."""
+    inputs = _turn_inputs(dev)
+    requests = lambda: torch.cuda.host_memory_stats()["active_requests.allocated"]  # noqa: E731
+    want = _compute_turn_level_gae(**inputs)
+    torch.cuda.synchronize()
+    before = requests()
+    got = _compute_turn_level_gae(**inputs, validate=False)
+    assert requests() == before
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
