@@ -836,16 +836,20 @@ Tensor bytes_of(const Tensor& t, int64_t bs, int64_t L) {  // a mask as [bs, L] 
 }
 bool in_place_ok(const Tensor& t) { return t.scalar_type() == at::kFloat && t.is_contiguous() && !t.requires_grad(); }
 
-// Reward scores and their normalisation, then areal_advantage_prep. `score`: the scores themselves when
+// Reward scores and their normalisation, then areal_advantage_prep, over bs rows. `score`: the scores themselves when
 // `scored`, else the raw rewards. Returns (loss mask, old log-probs, kl rewards, total rewards, kl rewards
 // for GAE, outcome rewards (both turn mode only), no-eos mask).
 py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double scaling, double clip,
                          const std::optional<NormTables>& norm, const Tensor& loss_mask, const Tensor& attention_mask,
                          const Tensor& logp_src, const OptTensor& ref_logp, bool recompute, int estimator, bool clamp,
-                         bool no_eos_zero, double kl_ctl, bool turn_mode) {
+                         bool no_eos_zero, double kl_ctl, bool turn_mode, int64_t bs) {
+  const int64_t L = logp_src.size(-1);
+  const Tensor ref_arg = or_undefined(ref_logp);
+  require_numel(bs, {{"rewards", &score}});
+  require_numel(bs * L, {{"logprobs", &logp_src}, {"loss_mask", &loss_mask}, {"attention_mask", &attention_mask},
+                         {"ref_logp", &ref_arg}});
   require_gpu(logp_src, loss_mask, attention_mask, score);
   const c10::hip::HIPGuard guard(logp_src.device().index());
-  const int64_t bs = score.size(0), L = logp_src.size(-1);
   const areal_stream_t stream = stream_of(logp_src);
   Tensor sc = score.scalar_type() == at::kFloat ? score : score.to(at::kFloat);
   sc = sc.contiguous();
@@ -869,7 +873,7 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
   if (logp.dim() != 2) logp = logp.reshape({bs, L});
   if (!in_place_ok(logp)) logp = logp.to(at::kFloat).contiguous();
   const Tensor old = recompute && src_ok ? logp : empty(logp, {bs, L}, at::kFloat);
-  Tensor ref = or_undefined(ref_logp);
+  Tensor ref = ref_arg;
   const bool ref_in_place = ref.defined() && in_place_ok(ref);
   if (ref.defined()) ref = ref_in_place ? ref.reshape({bs, L}) : ref.detach().to(at::kFloat).contiguous().reshape({bs, L});
   const Tensor lm = empty(logp, {bs, L}, at::kFloat), kl = empty(logp, {bs, L}, at::kFloat),

@@ -646,7 +646,7 @@ def compute_advantages(
         _lib.host().advantage_prep(
             score, scored, reward_bias, reward_scaling, reward_clip, score_tables, data["loss_mask"],
             data["attention_mask"], logp_src, data.get("ref_logp"), recompute, est, bool(kl_estimator.apply_clamp),
-            bool(mask_no_eos_with_zero), kl_ctl, turn_mode,
+            bool(mask_no_eos_with_zero), kl_ctl, turn_mode, bs,
         )
     )
     if recompute:

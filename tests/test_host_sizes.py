@@ -1,5 +1,6 @@
-"""A loss kernel reads as many elements of each array as the loss mask (the critic's value) has: an array of
-another size is refused before any kernel could read past its end. Needs no GPU: sizes are compared first."""
+"""A loss kernel reads as many elements of each array as the loss mask (the critic's value) has, reward shaping as
+many as the batch has rows and slots: an array of another size is refused before any kernel could read past its end.
+Needs no GPU: sizes are compared first."""
 
 import pytest
 import torch
@@ -7,7 +8,7 @@ import torch
 from areal_amd import _lib
 from areal_amd.functional import cispo_loss_fn, ppo_actor_loss_fn, ppo_critic_loss_fn
 from areal_amd.functional.aux_losses import sapo_loss_fn
-from areal_amd.ppo.actor import grpo_loss_fn
+from areal_amd.ppo.actor import compute_advantages, grpo_loss_fn
 
 N = 6
 MASK = torch.ones(N, dtype=torch.bool)
@@ -52,3 +53,15 @@ def test_critic_loss(name, size):
     value, old, target, mask = _arrays(name, size, "value", "old_value", "target_value", "loss_mask")
     with pytest.raises(_lib.ArealHipError, match=f"{name} has {size} elements, expected {N}"):
         ppo_critic_loss_fn(value, old, target, 0.2, mask)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 4])
+@pytest.mark.parametrize("name", ["rewards", "logprobs", "loss_mask", "attention_mask", "ref_logp"])
+def test_advantages(name, rows):
+    bs, length = 3, 5
+    z = torch.zeros(bs, length)
+    data = dict(input_ids=z.long(), rewards=torch.zeros(bs), logprobs=z, loss_mask=z > 0, attention_mask=z > 0, ref_logp=z)
+    data[name] = data[name][:1].expand(rows, *data[name].shape[1:]).contiguous()
+    n = data[name].numel()
+    with pytest.raises(_lib.ArealHipError, match=f"{name} has {n} elements, expected {bs if name == 'rewards' else bs * length}"):
+        compute_advantages(data)
