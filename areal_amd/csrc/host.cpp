@@ -79,6 +79,13 @@ void require_numel(int64_t n, std::initializer_list<std::pair<const char*, const
       fail(std::string(name) + " has " + std::to_string(t->numel()) + " elements, expected " + std::to_string(n));
 }
 
+// Autograd nodes have no forward-mode formula and say so; where a call makes no node (nothing asks for a
+// gradient), a tangent would be dropped without a word.
+void refuse_tangent(const Tensor& t) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(/*level=*/0).defined(),
+                              "areal_amd: forward-mode AD is not implemented");
+}
+
 Tensor or_undefined(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 
 areal_stream_t stream_of(const Tensor& t) {
@@ -292,6 +299,7 @@ py::tuple actor_loss(const Tensor& logprobs, const Tensor& proximal, const OptTe
                      const Tensor& advantages, const Tensor& loss_mask, const OptTensor& cu_seqlens,
                      const std::array<double, 14>& config, int mode, bool keep_mask, bool nan_if_nonfinite,
                      const OptTensor& entropy, const OptTensor& extra0, const OptTensor& extra1) {
+  refuse_tangent(logprobs);
   const areal_loss_config cfg = loss_config(config);
   const Tensor old_arg = or_undefined(old_logprobs);
   require_numel(loss_mask.numel(), {{"logprobs", &logprobs}, {"proximal_logprobs", &proximal},
@@ -408,6 +416,7 @@ py::tuple sapo_loss(const Tensor& logprobs, const Tensor& old_logprobs, const Te
                     const Tensor& loss_mask, const OptTensor& cu_seqlens, double tau_pos, double tau_neg,
                     bool seq_level, bool reduced, const OptTensor& entropy, const OptTensor& extra0,
                     const OptTensor& extra1) {
+  refuse_tangent(logprobs);
   require_numel(loss_mask.numel(), {{"logprobs", &logprobs}, {"old_logprobs", &old_logprobs}, {"advantages", &advantages}});
   require_gpu(logprobs, old_logprobs, advantages, loss_mask);
   const c10::hip::HIPGuard guard(logprobs.device().index());
@@ -466,6 +475,7 @@ py::tuple sapo_loss(const Tensor& logprobs, const Tensor& old_logprobs, const Te
 
 py::tuple critic_loss(const Tensor& value, const Tensor& old_value, const Tensor& target_value,
                       const OptTensor& loss_mask, double eps_clip, bool huber) {
+  refuse_tangent(value);
   const Tensor mask_arg = or_undefined(loss_mask);
   require_numel(value.numel(), {{"old_value", &old_value}, {"target_value", &target_value}, {"loss_mask", &mask_arg}});
   require_gpu(value, old_value, target_value, mask_arg);
@@ -751,6 +761,7 @@ py::tuple lm_head(const Tensor& hidden, const Tensor& weight, const OptTensor& b
                   const OptTensor& accum, const OptTensor& owner, int64_t save_limit, int64_t bwd_budget,
                   bool build_graph, bool needs_grad) {
   const Tensor bias = or_undefined(bias_arg);
+  for (const Tensor* t : {&hidden, &weight, &bias}) refuse_tangent(*t);
   require_gpu(hidden, weight, labels, bias);
   const c10::hip::HIPGuard guard(hidden.device().index());
   const LMHeadArgs a{temperature, logit_scale, token_chunk, save_probs, with_moments, or_undefined(accum),
