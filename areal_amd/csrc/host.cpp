@@ -967,10 +967,10 @@ py::tuple turn_gae(const Tensor& rewards, const OptTensor& values, const Tensor&
                    bool roll_ids, const Tensor& no_eos, double discount, double lambda, const OptTensor& lambda_seq,
                    const OptTensor& addend, bool want_flags) {
   const Tensor v = f32(or_undefined(values)), lam = or_undefined(lambda_seq), add = f32(or_undefined(addend));
-  require_gpu(rewards, v, loss_mask, turn_ids, no_eos, lam, add);
+  require_gpu(rewards, v, loss_mask, turn_ids, lam, add);
   const c10::hip::HIPGuard guard(rewards.device().index());
   const int64_t bs = rewards.size(0), L = rewards.size(1);
-  const Tensor r = f32(rewards), m = f32(loss_mask), ne = no_eos.to(at::kBool).contiguous();
+  const Tensor r = f32(rewards), m = f32(loss_mask), ne = no_eos.to(r.device(), at::kBool).contiguous();
   // ids beyond int32 cannot be valid (they must be smaller than the sequence length)
   const Tensor ids = (turn_ids.scalar_type() == at::kInt ? turn_ids
                       : turn_ids.scalar_type() == at::kLong ? turn_ids.clamp(-1, INT32_MAX).to(at::kInt)
