@@ -1344,6 +1344,12 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_apply_seg_kernel(NormArgs a
 // the normalisation's two launches cost 5 us each. A wave takes whole groups. (Group levels alone:
 // reward_score_groups_kernel.)
 constexpr int SCORE_THREADS = 1024;
+// As torch.clip: NaN stays, and the upper bound is the last word (a negative clip).
+DEVI float shaped_reward(float reward, float bias, float scaling, float clip) {
+  float x = (reward + bias) * scaling;
+  x = x < -clip ? -clip : x;
+  return x > clip ? clip : x;
+}
 __global__ __launch_bounds__(SCORE_THREADS) void reward_score_kernel(NormArgs a, float bias, float scaling, float clip,
                                                                      int normed) {
   constexpr int NW = SCORE_THREADS / 64;
@@ -1351,8 +1357,7 @@ __global__ __launch_bounds__(SCORE_THREADS) void reward_score_kernel(NormArgs a,
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   double b1 = 0.0, b4 = 0.0;
   for (int64_t i = tid; i < a.n; i += SCORE_THREADS) {
-    float x = (a.x[i] + bias) * scaling;
-    if (!(x != x)) x = x < -clip ? -clip : (x > clip ? clip : x);
+    const float x = shaped_reward(a.x[i], bias, scaling, clip);
     a.out[i] = x;
     b1 += (double)x;
     b4 += (double)x * (double)x;
@@ -1392,10 +1397,7 @@ __global__ __launch_bounds__(SCORE_THREADS) void reward_score_kernel(NormArgs a,
 __global__ __launch_bounds__(256) void reward_score_groups_kernel(NormArgs a, float bias, float scaling, float clip) {
   const int lane = threadIdx.x & 63, g = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (g > a.G) return;
-  auto shaped = [&](int64_t i) {
-    const float x = (a.x[i] + bias) * scaling;
-    return x != x ? x : (x < -clip ? -clip : (x > clip ? clip : x));
-  };
+  auto shaped = [&](int64_t i) { return shaped_reward(a.x[i], bias, scaling, clip); };
   const int64_t g0 = a.goff[g], g1 = g < a.G ? a.goff[g + 1] : a.n;
   if (g == a.G) {
     for (int64_t i = g0 + lane; i < g1; i += 64) a.out[i] = shaped(i);
@@ -2167,7 +2169,6 @@ int areal_reward_scores(const float* rewards, int64_t n, float bias, float scali
   if (!rewards || !out || (n_groups > 0 && (!group_offsets || !group_rows))) return AREAL_ERR_BAD_ARG;
   if (mean_level < 0 || mean_level > 2 || std_level < 0 || std_level > 2) return AREAL_ERR_BAD_ARG;
   if (mean_level == LEVEL_GROUP && std_level == LEVEL_BATCH) return AREAL_ERR_UNSUPPORTED;
-  if (n > (1 << 24)) return AREAL_ERR_UNSUPPORTED;
   NormArgs a{};
   a.x = rewards; a.n = n; a.goff = group_offsets; a.grows = group_rows; a.G = (int)n_groups; a.tail_group = tail_group;
   a.mean_level = mean_level; a.std_level = std_level; a.unbiased = unbiased; a.eps = eps; a.out = out;

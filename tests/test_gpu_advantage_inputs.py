@@ -1,8 +1,10 @@
-"""Inputs of the advantage calls off the common path: the no-EOS mask of turn-level GAE in host memory."""
+"""Inputs of the advantage calls off the common path: the no-EOS mask of turn-level GAE in host memory, a
+negative reward clip, more reward scores than 2^24."""
 
 import pytest
 import torch
 
+from areal_amd import _lib
 from areal_amd.ppo.gae import _compute_turn_level_gae
 
 pytestmark = pytest.mark.gpu
@@ -18,3 +20,25 @@ def test_turn_gae_moves_its_no_eos_mask(dev):
     want = _compute_turn_level_gae(*x, no_eos.to(dev), 0.99, 0.9)
     got = _compute_turn_level_gae(*x, no_eos, 0.99, 0.9)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("n,clip,group", [(37, -0.5, 0), (37, -0.5, 4), (2**24 + 3, 1.5, 0), (2**24 + 3, 1.5, 16)])
+def test_reward_scores(dev, n, clip, group):
+    """Bitwise the tensor operations when nothing is normalised; a group's scores against fp64."""
+    x = torch.randn(n, device=dev, generator=torch.Generator(dev).manual_seed(n))
+    x[5] = float("nan")
+    groups = n // group if group else 0
+    offsets = torch.arange(groups + 1, device=dev, dtype=torch.int64) * group
+    rows = torch.full((groups,), group, device=dev, dtype=torch.int64)
+    out = torch.empty_like(x)
+    rc = _lib.load().areal_reward_scores(
+        _lib.ptr(x), n, 0.25, 2.0, clip, _lib.ptr(offsets) if groups else None, _lib.ptr(rows) if groups else None,
+        groups, -1, 2, 2, 1, 1e-5, _lib.ptr(out), _lib.stream_ptr(x.device))
+    _lib.check(rc, "areal_reward_scores")
+    want = torch.clip((x + 0.25) * 2.0, min=-clip, max=clip)
+    if groups:
+        w = want[: groups * group].double().view(groups, group)
+        want[: groups * group] = ((w - w.mean(1, keepdim=True)) / (w.std(1, keepdim=True) + 1e-5)).float().view(-1)
+        torch.testing.assert_close(out, want, rtol=1e-5, atol=1e-5, equal_nan=True)
+    else:
+        assert torch.equal(out.nan_to_num(7.0), want.nan_to_num(7.0))
