@@ -149,6 +149,7 @@ struct Mark {
     if (event != nullptr) (void)hipEventDestroy(event);
   }
   void set(const c10::hip::HIPStream& stream) {
+    const c10::hip::HIPGuard guard(stream.device_index());  // an event belongs to the device it is made on
     if (event == nullptr && hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess) {
       event = nullptr;
       fail("creation of an event failed");
