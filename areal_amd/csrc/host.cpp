@@ -122,7 +122,8 @@ Tensor flat(const Tensor& t, at::ScalarType type) {
 // memory out of the pinned allocator's hands until the stream has passed the point of its
 // destruction. In a captured
 // graph, which may be replayed after that memory has gone to someone else, the results stay on the
-// device (`results`, the graph's own memory) and whoever asks for them copies them then.
+// device (`results`, the graph's own memory) and whoever asks for them first copies them then; that copy
+// is what every later reader gets, whatever has been replayed in between.
 // ---------------------------------------------------------------------------------------
 constexpr uint64_t PENDING = 0x7ff8a5c3d2e1f0b4ull;  // a NaN payload arithmetic does not make
 

@@ -1,5 +1,6 @@
 """A loss call in a captured graph: its results are the graph's own memory and not host memory that
-someone else has by the time of a replay, so every replay's statistics can be read behind it."""
+someone else has by the time of a replay, so the statistics read behind a replay are that replay's (one read: the
+first is kept)."""
 
 import pytest
 import torch
