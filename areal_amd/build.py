@@ -146,9 +146,13 @@ def _check_lmhead(build_dir: Path) -> None:
 def _up_to_date(src: Path, obj: Path) -> bool:
     if not obj.exists():
         return False
-    deps = [src, CSRC / "common.hpp", Path(__file__)]
+    deps = [src, CSRC.parents[1] / "include" / "areal_hip.h", Path(__file__)]
     if src.name == "host.cpp":
-        deps = [src, CSRC.parents[1] / "include" / "areal_hip.h"]
+        import torch
+
+        deps.append(Path(torch.__file__).with_name("version.py"))  # compiled against the installed torch's headers
+    else:
+        deps.append(CSRC / "common.hpp")
     if src.name == "lmhead.hip":
         deps.append(CSRC / "mainloop16.inc")
     return all(obj.stat().st_mtime > d.stat().st_mtime for d in deps)

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "../../include/areal_hip.h"  // status codes, structs, and a check of every entry point's definition
+
 #define DEVI __device__ __forceinline__
 
 typedef unsigned short u16;
@@ -14,16 +16,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-// Error codes returned by every extern "C" entry point (0 = success).
-enum ArealStatus : int {
-  AREAL_OK = 0,
-  AREAL_ERR_BAD_ARG = -1,        // null pointer, negative size, unsupported flag
-  AREAL_ERR_ALIGNMENT = -2,      // pointer or leading dimension not 16-byte aligned
-  AREAL_ERR_WORKSPACE = -3,      // workspace smaller than *_workspace_bytes()
-  AREAL_ERR_LAUNCH = -4,         // hipGetLastError() != hipSuccess after a launch
-  AREAL_ERR_UNSUPPORTED = -5,    // shape outside what the kernels implement
-};
 
 #define AREAL_CHECK_LAUNCH()                                   \
   do {                                                         \

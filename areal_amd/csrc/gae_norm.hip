@@ -2191,9 +2191,6 @@ size_t areal_turn_gae_workspace_bytes(int64_t bs, int64_t max_seqlen) {
 // int32 (-1 in prompt / tool gaps), no_eos [bs] (nullable), lambda_seq [bs] (nullable, else the
 // scalar). status (device int, zeroed by the caller) receives a bit mask of malformed turn ids
 // at active tokens: 1 negative, 2 not smaller than max_seqlen, 4 decreasing.
-int areal_turn_gae_ex(const float*, const float*, const float*, const int32_t*, int, const uint8_t*, const float*,
-                      const float*, int64_t, int64_t, float, float, float*, float*, int*, void*, size_t, hipStream_t);
-
 int areal_turn_gae(const float* rewards, const float* values, const float* loss_mask,
                    const int32_t* turn_ids, const uint8_t* no_eos, const float* lambda_seq,
                    int64_t bs, int64_t max_seqlen, float discount, float gae_lambda,

@@ -2190,10 +2190,6 @@ size_t areal_lmhead_probs_bytes(int64_t T, int64_t V) {
   return (size_t)round_up_i64(T, 2 * BK) * (size_t)round_up_i64(V, BK) * 2;
 }
 
-int areal_lmhead_fwd_ex(const void*, const void*, const float*, const int64_t*, int64_t, int64_t, int64_t, float,
-                        float, float*, float*, float*, float*, float*, float*, float*, float*, void*, size_t,
-                        float*, int*, float*, int*, void*, size_t, hipStream_t);
-
 static Regions fwd_regions(int64_t T, int64_t H, int64_t V) {
   return plan_sweep_regions(V, T, H);
 }

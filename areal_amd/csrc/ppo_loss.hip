@@ -796,23 +796,6 @@ int loss_grid(int64_t n, int vec = 1) {
   return (int)b;
 }
 
-}  // namespace
-
-// Plain-C mirror of LossCfg (see include/areal_hip.h).
-struct areal_loss_config {
-  int loss_kind;
-  float clip_lo, clip_hi;
-  int has_c_clip;
-  float c_clip;
-  int seq_is;
-  int rs_enabled, rs_seq_level, rs_clamp, rs_metric, rs_agg;
-  float rs_upper;
-  int rs_has_lower;
-  float rs_lower;
-};
-
-namespace {
-
 constexpr size_t STAT_PARTIAL_BYTES = (size_t)MAX_LOSS_BLOCKS * N_LOSS_STATS * sizeof(StatPartial);
 
 size_t loss_workspace_bytes(int64_t n_seqs, bool with_stats) {
@@ -963,22 +946,7 @@ int areal_actor_loss_static(const float* logprobs, const float* proximal,
                          stream);
 }
 
-// areal_actor_loss with every optional input and output in one struct (include/areal_hip.h).
-struct areal_actor_loss_io {
-  const float *logprobs, *proximal, *old_logprobs, *advantages;
-  const uint8_t* loss_mask;
-  const int32_t* cu_seqlens;
-  const float *entropy, *extra0, *extra1;
-  int64_t n_tokens, n_seqs, uniform_len;
-  float *loss, *dlogprobs, *stat_loss, *stat_ratio, *stat_approx_kl;
-  uint8_t *clip_mask, *dual_clip_mask, *new_mask;
-  float *behave_imp_weight, *behave_approx_kl;
-  uint8_t* behave_mask;
-  float *clip_ratio, *dual_clip_ratio, *logp_diff, *logp_abs_diff, *behave_filtered_ratio;
-  double* results;
-  double* host_results;
-  int with_stats, nan_if_nonfinite;
-};
+// areal_actor_loss with every optional input and output in one struct.
 int areal_actor_loss_call(const areal_actor_loss_io* a, const areal_loss_config* cfg, void* workspace,
                           size_t workspace_bytes, hipStream_t stream) {
   if (a == nullptr || a->results == nullptr) return AREAL_ERR_BAD_ARG;
@@ -989,7 +957,7 @@ int areal_actor_loss_call(const areal_actor_loss_io* a, const areal_loss_config*
   const LossStatsArgs sa{a->entropy, a->extra0, a->extra1, a->results + 9};
   const LossMore more{a->clip_ratio, a->dual_clip_ratio, a->logp_diff, a->logp_abs_diff,
                       a->behave_filtered_ratio, a->nan_if_nonfinite, a->host_results};
-  return actor_loss_impl(a->logprobs, a->proximal, a->old_logprobs, a->advantages, a->loss_mask, a->cu_seqlens,
+  return actor_loss_impl(a->logprobs, a->proximal_logprobs, a->old_logprobs, a->advantages, a->loss_mask, a->cu_seqlens,
                          a->n_tokens, a->n_seqs, a->uniform_len, cfg, a->loss, a->dlogprobs, a->stat_loss,
                          a->stat_ratio, a->stat_approx_kl, a->clip_mask, a->dual_clip_mask, a->new_mask,
                          a->behave_imp_weight, a->behave_approx_kl, a->behave_mask, a->results,
