@@ -395,7 +395,9 @@ int areal_gae_padded_row_stats(const float* rewards, const float* values, const 
  * areal_gae_segment_stats_bytes(n_tokens, n_groups) bytes) receives the five sums of
  * areal_gae_padded_row_stats per (2048-token tile, group) segment, for
  * areal_group_norm_from_segment_stats. One launch. AREAL_ERR_UNSUPPORTED when sequences average
- * more than 16384 tokens or groups fewer than 256: run areal_gae_packed and areal_group_norm. */
+ * more than 16384 tokens or groups fewer than 256: run areal_gae_packed and areal_group_norm.
+ * (For callers that want the sums, or normalise something else with them; the Python package
+ * calls areal_gae_packed_normalized.) */
 size_t areal_gae_segment_stats_bytes(int64_t n_tokens, int64_t n_groups);
 int areal_gae_packed_group_stats(const float* rewards, const float* values, const float* loss_mask,
                                  const int32_t* cu_seqlens, const uint8_t* no_eos,
