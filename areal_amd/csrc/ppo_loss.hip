@@ -13,6 +13,7 @@
 #include "common.hpp"
 
 #include <mutex>
+#include <type_traits>
 
 namespace {
 
@@ -112,7 +113,7 @@ DEVI int seq_search(const LossIO& io, int64_t t, int lane) {
   else s = wave_count_le(io.cu + 1, io.n_seqs, t, lane);
   return s < io.n_seqs ? s : io.n_seqs - 1;
 }
-DEVI bool needs_seq(const LossCfg& c) {
+__host__ DEVI bool needs_seq(const LossCfg& c) {
   return (c.rs_enabled && c.rs_seq_level) || (c.loss_kind == LOSS_PPO && c.seq_is);
 }
 // A token's sequence and what the token kernel reads of it, in registers until the next one starts (a
@@ -273,12 +274,13 @@ __global__ __launch_bounds__(LOSS_THREADS) void seq_rs_kernel(LossIO io, LossCfg
 
 // Rejection sampling for one token. Returns the narrowed mask; sets w (not yet zeroed outside
 // the mask) and whether the token counts as filtered / clamped.
+template <bool SEQ>
 DEVI bool rs_token(const LossCfg& c, const SeqCtx& q, bool m, float prox, float old, float& w, bool& counted) {
   const float lr = sane_log_ratio(prox, old);
   w = expf(lr);
   bool keep = true;
   counted = false;
-  if (c.rs_seq_level) {
+  if (SEQ && c.rs_seq_level) {
     const bool seq_ok = q.rs_ok != 0.0f;
     if (c.rs_metric == METRIC_RATIO) w = q.rs_w;
     if (c.rs_clamp) {
@@ -376,7 +378,7 @@ struct TokenOut {
   bool clip, dual, m2, bm;
 };
 
-template <bool STATS, bool LEAN>
+template <bool STATS, bool LEAN, bool SEQ>
 DEVI void token_body(const LossIO& io, const LossCfg& c, const SeqCtx& q, const TokenIn& in, TokenOut& out,
                      TokenAcc& acc, StatAcc<STATS>& st) {
   const bool m = in.m;
@@ -384,7 +386,7 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, const SeqCtx& q, const 
   float w = 1.0f;
   if (c.rs_enabled) {
     bool counted;
-    m2 = rs_token(c, q, m, in.prox, in.old, w, counted);
+    m2 = rs_token<SEQ>(c, q, m, in.prox, in.old, w, counted);
     w = m2 ? w : 0.0f;
     acc.n_filtered += counted;
   }
@@ -416,7 +418,7 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, const SeqCtx& q, const 
     ratio_out = ratio;
   } else {
     float ratio, a = adv, dratio;  // dratio = d ratio / d lp[t] factor handled below
-    if (c.seq_is) {
+    if (SEQ && c.seq_is) {
       ratio = m2 ? q.ratio : 0.0f;
       a = m2 ? q.adv : 0.0f;
       dratio = 0.f;  // gradient assembled per sequence below
@@ -442,7 +444,7 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, const SeqCtx& q, const 
       pg = torch_min(pg, pg3);
       dpg *= keep;
     }
-    if (c.seq_is) {
+    if (SEQ && c.seq_is) {
       // every kept token of the sequence receives ratio_s/count_s * sum_w_s * dpg_s
       dsel = m2 ? dpg * ratio * q.sum_w * q.inv_count : 0.0f;
     } else {
@@ -454,7 +456,7 @@ DEVI void token_body(const LossIO& io, const LossCfg& c, const SeqCtx& q, const 
   }
   if (c.rs_enabled) {
     pg = pg * w;
-    if (!(c.loss_kind == LOSS_PPO && c.seq_is)) dsel = dsel * w;
+    if (!(SEQ && c.loss_kind == LOSS_PPO && c.seq_is)) dsel = dsel * w;
     const bool bm = (w > 0.0f) && m2;
     acc.n_behave += bm;
     out.bm = bm;
@@ -511,7 +513,7 @@ DEVI void token_group_load(const LossIO& io, const LossCfg& c, int64_t t, TokenL
   load_f32<VEC>(STATS ? io.extra0 : nullptr, t, in.x0);
   load_f32<VEC>(STATS ? io.extra1 : nullptr, t, in.x1);
 }
-template <bool STATS, int VEC, bool LEAN>
+template <bool STATS, int VEC, bool LEAN, bool SEQ>
 DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, SeqCtx& q, const TokenLoad<VEC>& ld,
                               TokenAcc& acc, StatAcc<STATS>& st) {
   float dlp[VEC], loss[VEC], ratio[VEC], kl[VEC], bw[VEC], bkl[VEC];
@@ -520,8 +522,8 @@ DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, Seq
   for (int i = 0; i < VEC; ++i) {
     const TokenIn in{ld.lp[i], ld.prox[i], ld.old[i], ld.adv[i], ld.ent[i], ld.x0[i], ld.x1[i], ld.m[i]};
     TokenOut o;
-    if (q.s >= 0) seq_advance(io, c, t + i, i == 0, q);
-    token_body<STATS, LEAN>(io, c, q, in, o, acc, st);
+    if (SEQ && q.s >= 0) seq_advance(io, c, t + i, i == 0, q);
+    token_body<STATS, LEAN, SEQ>(io, c, q, in, o, acc, st);
     dlp[i] = o.dlp; loss[i] = o.loss; ratio[i] = o.ratio; kl[i] = o.kl; bw[i] = o.behave_w; bkl[i] = o.behave_kl;
     clip[i] = o.clip; dual[i] = o.dual; m2[i] = o.m2; bm[i] = o.bm;
   }
@@ -568,7 +570,10 @@ DEVI void token_group_compute(const LossIO& io, const LossCfg& c, int64_t t, Seq
 // token: the addresses of fifteen arrays that are not there do not fit the scalar registers, and their
 // tests and spills (300 reloads), with a sequence's end and aggregates fetched once and not per token, were
 // a sixth of it: 4 Mi tokens in 2048 sequences 32.2 -> 27.5 us.
-template <bool STATS, int VEC, bool LEAN>
+// SEQ: a sequence-level option is on (needs_seq). Without one the search, the walk and the sequence's
+// values cost the same issue slots for nothing: 4 Mi tokens with token-level bounds, this kernel, the
+// finalize and the gradient's scaling 47.4 -> 44.2 us, with statistics 53.2 -> 40.1.
+template <bool STATS, int VEC, bool LEAN, bool SEQ>
 __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, LossCfg c,
                                                                    Partial* partials,
                                                                    StatPartial* stat_partials) {
@@ -577,7 +582,6 @@ __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, Los
   st.init();
   // Sequence-level options need each token's sequence: a wave searches the one of its first token
   // (64 probes a round) and its lanes walk on from there, instead of a binary search per token.
-  const bool seq = needs_seq(c);
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t nthreads = (int64_t)gridDim.x * blockDim.x;
   const int64_t n_vec = io.n - io.n % VEC;
@@ -586,17 +590,17 @@ __global__ __launch_bounds__(LOSS_THREADS) void loss_token_kernel(LossIO io, Los
   for (int64_t t = gid * VEC, tw = wid * VEC; tw < n_vec; t += nthreads * VEC, tw += nthreads * VEC) {
     if (t < n_vec) token_group_load<STATS, VEC>(io, c, t, in);  // (in flight during the search)
     SeqCtx q{};
-    q.s = seq ? seq_search(io, tw, threadIdx.x & 63) : -1;
+    q.s = SEQ ? seq_search(io, tw, threadIdx.x & 63) : -1;
     if (t >= n_vec) continue;
-    token_group_compute<STATS, VEC, LEAN>(io, c, t, q, in, acc, st);
+    token_group_compute<STATS, VEC, LEAN, SEQ>(io, c, t, q, in, acc, st);
   }
   if (VEC > 1 && n_vec + wid < io.n) {
     SeqCtx q{};
-    q.s = seq ? seq_search(io, n_vec + wid, threadIdx.x & 63) : -1;
+    q.s = SEQ ? seq_search(io, n_vec + wid, threadIdx.x & 63) : -1;
     if (n_vec + gid < io.n) {
       TokenLoad<1> tail;
       token_group_load<STATS, 1>(io, c, n_vec + gid, tail);
-      token_group_compute<STATS, 1, LEAN>(io, c, n_vec + gid, q, tail, acc, st);
+      token_group_compute<STATS, 1, LEAN, SEQ>(io, c, n_vec + gid, q, tail, acc, st);
     }
   }
 
@@ -1050,17 +1054,19 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
       hipLaunchKernelGGL(kernel, dim3(grid), dim3(LOSS_THREADS), 0, stream, i, cc, partials,
                          stats ? stat_partials : (StatPartial*)nullptr);
     };
-    if (lean) {
-      if (stats && vec4) launch(loss_token_kernel<true, 4, true>);
-      else if (stats) launch(loss_token_kernel<true, 1, true>);
-      else if (vec4) launch(loss_token_kernel<false, 4, true>);
-      else launch(loss_token_kernel<false, 1, true>);
-    } else {
-      if (stats && vec4) launch(loss_token_kernel<true, 4, false>);
-      else if (stats) launch(loss_token_kernel<true, 1, false>);
-      else if (vec4) launch(loss_token_kernel<false, 4, false>);
-      else launch(loss_token_kernel<false, 1, false>);
-    }
+    auto pick = [&](auto st, auto le, auto se) {
+      constexpr bool S = decltype(st)::value, L = decltype(le)::value, Q = decltype(se)::value;
+      if (vec4) launch(loss_token_kernel<S, 4, L, Q>);
+      else launch(loss_token_kernel<S, 1, L, Q>);
+    };
+    auto pick_seq = [&](auto st, auto le) {
+      if (needs_seq(cc)) pick(st, le, std::true_type{});
+      else pick(st, le, std::false_type{});
+    };
+    if (stats && lean) pick_seq(std::true_type{}, std::true_type{});
+    else if (stats) pick_seq(std::true_type{}, std::false_type{});
+    else if (lean) pick_seq(std::false_type{}, std::true_type{});
+    else pick_seq(std::false_type{}, std::false_type{});
   };
   if (n_tokens > 0 && c.rs_enabled && c.rs_seq_level) {
     // below about 1024 tokens a sequence does not give four waves two groups of four per lane
