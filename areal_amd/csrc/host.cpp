@@ -1,8 +1,9 @@
 // Host path of the Python API: what a call does between its arguments and its kernel launches
 // (output and workspace allocation, the autograd node, the small results that travel back) in one
 // native call. A micro-batch's loss stage or a short lm_head step is bound by this work, not by its
-// kernels: the same sequence in Python (about twenty tensor calls, ctypes argument lists, a Python
-// autograd node) took 150 to 300 us of host time per call, this takes 10 to 30.
+// kernels: the loss stage of 32 Ki tokens with its statistics, forward and backward (16 us of kernels),
+// takes 94 us where the same sequence in Python (about twenty tensor calls, ctypes argument lists, a
+// Python autograd node) and its kernels took 335.
 //
 // Loaded as areal_amd._host; every kernel behind it is reached through the C ABI of
 // libareal_hip.so (include/areal_hip.h).

@@ -97,10 +97,12 @@ def grpo_loss_fn(
     ``{"sum", "count", "avg", "min", "max", "denominator"}``, ``stats["denominator/<name>"]``
     the token counts (what the tracker's export computes from the clones, ``actor.py:662-733``,
     ``stats_tracker.py:455-560``).  The ``compute_logp/...`` diagnostics of the proximal
-    approximations (``actor.py:1138-1226``) are functions of tensors the loss kernel does not
-    see; they are evaluated as in the other mode and reduced at once by one launch of the masked
-    statistics kernel, under the same denominator (``stats["denominator/compute_logp/
-    n_valid_tokens"]``); the staleness statistics are host scalars in both modes.
+    approximations (``actor.py:1138-1226``) have their own denominator
+    (``stats["denominator/compute_logp/n_valid_tokens"]``). Without token versions the proximal
+    log-probs are the only one, reduced in the loss kernel's pass as well. With ``versions`` and
+    ``current_version`` the others are functions of tensors the loss kernel does not see: they are
+    evaluated as in the other mode and reduced at once by one launch of the masked statistics
+    kernel. The staleness statistics are host scalars in both modes.
     """
     if stats_mode not in ("tensors", "reduced"):
         raise ValueError(f"stats_mode must be 'tensors' or 'reduced', got {stats_mode!r}")
