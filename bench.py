@@ -767,9 +767,9 @@ def main() -> None:
     if args.workload == "qwen3-8b" and saved:
         kib = 1024.0
         traffic_detail = {
-            KERNEL_FWD_SAVE + " forward": 3.1562e7 * kib * 2.0 + 9.729e6 * kib,  # fetch: mean of 7 launches
-            KERNEL_DHIDDEN + " dHidden": 2.9199e7 * kib * 2.0 + 2.6419e5 * kib,
-            KERNEL_DWEIGHT + " dWeight": (2.9205e7 + 1.5956e5) * kib * 2.0 + 1.2219e6 * kib,  # with its 384-row tail
+            KERNEL_FWD_SAVE + " forward": 3.1644e7 * kib * 2.0 + 9.7305e6 * kib,  # fetch: median of 7 launches
+            KERNEL_DHIDDEN + " dHidden": 2.9203e7 * kib * 2.0 + 2.6214e5 * kib,
+            KERNEL_DWEIGHT + " dWeight": (2.9191e7 + 1.5973e5) * kib * 2.0 + 1.2124e6 * kib,  # with its 384-row tail
         }
         traffic = sum(traffic_detail.values()) / 3.0
         traffic_source = ("offline rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this command "
