@@ -72,7 +72,7 @@ def _compute_token_level_gae(
 def _token_level_gae_with_row_stats(rewards, values, loss_mask, seq_no_eos_mask, discount, gae_lambda):
     """``_compute_token_level_gae`` that also returns, per row, the masked sums of the advantages
     which ``Normalization.from_row_stats`` needs (``[5, bs]`` fp64), or ``None`` when the layout
-    does not allow it (very many rows of a fraction of a 2048-token tile). ``values=None``: all zero."""
+    does not allow it (more than 1024 rows of fewer than 1792 slots). ``values=None``: all zero."""
     bs, max_seqlen = rewards.shape
     if bs == 0 or max_seqlen == 0:
         return None

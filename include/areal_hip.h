@@ -377,7 +377,7 @@ int areal_gae_packed(const float* rewards, const float* values, const float* los
                      size_t workspace_bytes, areal_stream_t stream);
 
 /* areal_gae_packed on a padded [n_seqs, uniform_len] batch (AREAL_ERR_UNSUPPORTED for rows over 131072
- * tokens and for more than 4096 rows of fewer than 512; values may be NULL: all zero), which also
+ * tokens and for more than 1024 rows of fewer than 1792; values may be NULL: all zero), which also
  * leaves per row, in row_stats [5][n_seqs] fp64, the
  * sums of m, x m, m^2, m^2 x, m^2 x^2 (x = the advantage written, m = loss_mask): the statistics
  * pass of the advantage normalisation that follows in compute_advantages
