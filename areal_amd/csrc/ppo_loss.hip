@@ -198,8 +198,8 @@ DEVI T block_sum(T v, T* smem) {
 // Writes seq_rs[s] = {in_bounds, uniform weight exp(mean log ratio)}.
 // WPS waves per sequence: a block of 4 waves takes 4 / WPS sequences. Bound by HBM (9 bytes per
 // token): a lane takes four tokens with 16-byte loads, aligned whatever the sequence's start is
-// (VEC = 4), the loads of a group do not wait for its mask, and short sequences take a wave each so
-// that the lanes of a block are not idle. 4 Mi tokens in 2048 sequences: 38 us with one token per
+// (VEC = 4), the loads of a group do not wait for its mask, and many short sequences take a wave each
+// so that the lanes of a block are not idle. 4 Mi tokens in 2048 sequences: 38 us with one token per
 // lane and loads behind the mask.
 // ---------------------------------------------------------------------------------------
 template <int WPS, int VEC>
@@ -1069,8 +1069,13 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
     else pick_seq(std::false_type{}, std::false_type{});
   };
   if (n_tokens > 0 && c.rs_enabled && c.rs_seq_level) {
-    // below about 1024 tokens a sequence does not give four waves two groups of four per lane
-    const bool short_seqs = n_tokens < n_seqs * 1024;
+    // A wave per sequence where there are many short ones. Its block waits for the longest of its four, so
+    // that lengths that differ set the line (this kernel, us, a wave against a block per sequence, 4 Mi tokens
+    // of lognormal / equal lengths: mean 128 61.3 / 16.8 against 53.6 / 38.5, 384 25.8 / 11.7 against 21.5 /
+    // 17.1, 512 31.8 / 10.7 against 18.4 / 14.0, 1024 55.5 / 9.4 against 19.8 / 11.3), and a block each is no
+    // dearer while few enough for the chip (256 Ki tokens: 2048 of 128 8.2 / 4.8 against 6.4 / 5.6, 1024 of 256
+    // 11.9 / 4.6 against 5.6 / 4.6).
+    const bool short_seqs = n_seqs > 4096 && n_tokens <= n_seqs * 384;
     const bool vec = aligned_to(proximal, 16) && aligned_to(old_logprobs, 16) && aligned_to(loss_mask, 4);
     const dim3 grid_s((unsigned)(short_seqs ? ceil_div_i64(n_seqs, LOSS_THREADS / 64) : n_seqs)), block(LOSS_THREADS);
     if (short_seqs && vec) hipLaunchKernelGGL((seq_rs_kernel<1, 4>), grid_s, block, 0, stream, io, c, seq_rs);

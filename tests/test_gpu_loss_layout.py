@@ -1,5 +1,5 @@
-"""The loss stage where its layout changes: sequences around the length from which four waves share
-one, alignments that rule out 16-byte loads, batches around one wave and around the four-token form,
+"""The loss stage where its layout changes: sequences around the number and length from which a wave
+takes one, alignments that rule out 16-byte loads, batches around one wave and around the four-token form,
 and what the loss kernel does besides the loss (fp32 copies of the masks, statistics of the proximal
 log-probs, tokens that are not finite)."""
 
@@ -48,6 +48,14 @@ def test_sequence_rejection(lens, offset, metric, agg):
                               upper=upper)
     assert torch.equal(got.loss_mask.cpu(), want.loss_mask)
     torch.testing.assert_close(got.behave_imp_weight.cpu(), want.behave_imp_weight, rtol=1e-5, atol=1e-6)
+
+
+# more than 4096 sequences take a wave each up to a mean of 384 tokens
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("lens", [[7] * 4096, [7, 1, 0, 300] * 1025, [2, 5000] + [65] * 4095, [384] * 4097, [385] * 4097])
+@pytest.mark.parametrize("metric,agg", [("kl_k2", "mean"), ("ratio", "mean")])
+def test_sequence_rejection_of_many_sequences(lens, offset, metric, agg):
+    test_sequence_rejection(lens, offset, metric, agg)
 
 
 @pytest.mark.parametrize("offset", [0, 1])
