@@ -80,6 +80,10 @@ DEVI bool gemm_skipped(const GemmArgs& g) { return gate_closed(g.skip_if_set, g.
 // copy, in a copy in blocks of RB B tiles, all splits of a block before the next block, so that 32
 // consecutive ones are RB B tiles x 32 / RB splits. Every XCD has the same number of tiles to
 // within one row or column of them, whatever the number of B tiles is.
+//
+// dWeight is laid out as a flat list (xg < 0): the tiles in blocks of RB B tiles x all A tiles, an
+// eighth of the list per XCD, and the XCD's part dealt to its 32 CUs tile by tile. A workgroup takes
+// `chain` of them, 32 apart, so that the next tile's first k-tiles arrive while this one is stored.
 struct Sched {
   int bj0, nbj;  // B tiles [bj0, bj0 + nbj)
   int ai0, nai;  // A tiles [ai0, ai0 + nai)
@@ -88,14 +92,35 @@ struct Sched {
   int sb_log2;   // log2 of the workgroups per super-block: 5 or 3
   int n_sb_j;    // super-blocks along j
   int n_sb;      // total super-blocks
-  int xg, bg;    // XCD layout (xg = 0: super-blocks); kg = 8 / (xg * bg)
+  int xg, bg;    // XCD layout (xg = 0: super-blocks, xg < 0: flat list); kg = 8 / (xg * bg)
   int zk;        // copies per XCD
+  int chain;     // flat list: tiles per workgroup
 };
+
+// Tile `step` of workgroup `id` in the flat list.
+DEVI bool flat_decode(const Sched& sc, int id, int step, int& bj, int& ai) {
+  const int xcd = id & 7, n = sc.nbj * sc.nai;
+  const int t0 = (int)((int64_t)xcd * n / 8), t1 = (int)((int64_t)(xcd + 1) * n / 8);
+  const int t = t0 + ((id >> 8) * sc.chain + step) * 32 + ((id >> 3) & 31);
+  if (step >= sc.chain || t >= t1) return false;
+  const int blk = t / (sc.RB * sc.nai), r = t - blk * sc.RB * sc.nai;
+  const int left = sc.nbj - blk * sc.RB, rb = left < sc.RB ? left : sc.RB;
+  ai = r / rb;
+  bj = sc.bj0 + blk * sc.RB + (r - ai * rb);
+  ai += sc.ai0;
+  return true;
+}
 
 // z: the workgroup's copy of a split-K launch (XCD layout only; unchanged otherwise).
 DEVI bool sched_decode(const Sched& sc, int id, int& bj, int& split, int& ai_begin, int& ai_end, int& z) {
   const int xcd = id & 7;
   int q = id >> 3;
+  if (sc.xg < 0) {
+    split = 0;
+    if (!flat_decode(sc, id, 0, bj, ai_begin)) return false;
+    ai_end = ai_begin + 1;
+    return true;
+  }
   if (sc.xg > 0) {
     const int ag = xcd % sc.xg, xb = xcd / sc.xg, bgi = xb % sc.bg, kgi = xb / sc.bg;
     const int b0 = bgi * sc.nbj / sc.bg, nb = (bgi + 1) * sc.nbj / sc.bg - b0;
@@ -131,7 +156,7 @@ DEVI bool sched_decode(const Sched& sc, int id, int& bj, int& split, int& ai_beg
 
 static Sched make_sched(int bj0, int nbj, int ai0, int nai, int S, int sb_wgs = 32) {
   Sched sc;
-  sc.xg = sc.bg = 0; sc.zk = 1;
+  sc.xg = sc.bg = 0; sc.zk = sc.chain = 1;
   sc.bj0 = bj0; sc.nbj = nbj; sc.ai0 = ai0; sc.nai = nai; sc.S = S;
   sc.sb_log2 = sb_wgs == 8 ? 3 : 5;
   const int rs_max = sb_wgs == 8 ? 4 : 8;
@@ -148,17 +173,33 @@ static Sched make_xcd_sched(int nbj, int nai, int S, int xg, int bg, int zk, int
   sc.xg = xg; sc.bg = bg; sc.zk = zk; sc.RB = RB;
   return sc;
 }
+// Block width of an XCD's workgroups: the fewer distinct operand tiles 32 neighbouring ones read
+// (nb B tiles, S splits), the less traffic from outside the XCD's L2. 4 x 8 and 8 x 4 need
+// 12. A block whose workgroups are not a multiple of 32 leaves windows that straddle two blocks.
+static int xcd_block(int S) { return S >= 8 ? 4 : (S >= 4 ? 8 : (S >= 2 ? 16 : 32)); }
+// chain: the workgroups may take several tiles. They then take up to 16 each, the same number of rounds
+// of 256 to all. A workgroup per tile starts each one cold (scheduling, kernel arguments, 128 KB of
+// operands before the first MFMA) and ends it waiting for nothing: dWeight of 509 x 896 (8 k-tiles per tile)
+// 183 us in 10 rounds, 160 in one chain; 8192 x 1536 into fp32 3084 -> 2982 adding, 2803 -> 2771 storing; with
+// 64 k-tiles per tile (4096 x 896) 737 -> 734. More than 16 would leave a CU that another stream holds up
+// with a long queue of its own, for less than half a per cent.
+static Sched make_flat_sched(int nbj, int nai, bool chain) {
+  Sched sc = make_sched(0, nbj, 0, nai, nai);
+  sc.xg = -1;
+  sc.RB = xcd_block(nai);
+  const int64_t rounds = ceil_div_i64((int64_t)nbj * nai, 256);
+  if (chain) sc.chain = (int)ceil_div_i64(rounds, ceil_div_i64(rounds, 16));
+  return sc;
+}
 static int sched_grid(const Sched& sc) {
+  if (sc.xg < 0) return 256 * (int)ceil_div_i64((int64_t)sc.nbj * sc.nai, (int64_t)256 * sc.chain);
   if (sc.xg > 0) {
     const int na = (int)ceil_div_i64(sc.nai, sc.xg);
     return 8 * (int)ceil_div_i64(sc.nbj, sc.bg) * (sc.S < na ? sc.S : na) * sc.zk;
   }
   return ((sc.n_sb + 7) / 8) * 8 * (1 << sc.sb_log2);
 }
-// Block width of an XCD's workgroups, and the distinct operand tiles that 32 neighbouring ones read
-// (nb B tiles, S splits): the fewer, the less traffic from outside the XCD's L2. 4 x 8 and 8 x 4 need
-// 12. A block whose workgroups are not a multiple of 32 leaves windows that straddle two blocks.
-static int xcd_block(int S) { return S >= 8 ? 4 : (S >= 4 ? 8 : (S >= 2 ? 16 : 32)); }
+// The distinct operand tiles of 32 neighbouring workgroups in such blocks.
 static double xcd_distinct(int nb, int S) {
   const int RB = xcd_block(S), rb = RB < nb ? RB : nb, rs = (int)ceil_div_i64(32, rb);
   double d = rb + (rs < S ? rs : S);
@@ -1069,10 +1110,31 @@ enum { VAR_NT = 0, VAR_TN = 1, VAR_MIX = 2 };
 // fragment reads, lane l on row l % 16 at chunk ks * 4 + l / 16)
 DEVI int swz16(int r) { return r & 7; }
 
+// The 256 columns that the loads of a k-major operand fetch for a tile that starts at column `first`
+// (a multiple of 32) of nvalid: those from `first` on, or the last 256 of the operand when fewer are
+// left. Returns the window's first column; the tile starts (first - window) / 16 blocks into it.
+DEVI int km_window(int first, int nvalid) {
+  if (first + TILE <= nvalid) return first;
+  const int w = (nvalid - TILE + 15) & ~15;
+  return w > 0 ? w : 0;
+}
+// LDS read addresses (stage 0) of a k-major operand's fragments: wave row / column W reads the nblk
+// blocks of 16 columns from block W * nblk + shift of the window on (blocks behind the window hold
+// columns past the end, whose results are discarded: they wrap to any block).
+DEVI void km_fragments(int W, int nblk, int shift, int oper, int lane, uint32_t lds_base, uint32_t (&rd)[8]) {
+  const int G = lane >> 4, q = lane & 15, r4 = q >> 2;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    const int y = W * nblk + shift + x;
+    rd[x] = lds_base + oper * ML16_OPER_BYTES + (G * 8 + r4) * 512 + ((((y >> 1) & 7) ^ r4) << 6) +
+            ((((y & 1) ^ G) & 1) << 5) + (q & 3) * 8;
+  }
+}
+
 // Per-lane byte offsets of the 8 direct loads of one operand half, and the LDS read addresses
-// (stage 0) of its fragments. KM: k-major operand (`first` = its tile of 32 nblk columns, nvalid =
-// readable columns; the loads fetch 256 columns from the tile's first one whatever nblk is, and
-// wave row / column W reads the nblk blocks of 16 columns from block W * nblk on); otherwise
+// (stage 0) of its fragments. KM: k-major operand (`first` = the tile's first column, nvalid =
+// readable columns; offsets from the window's first column, the same for every tile of an operand
+// whose columns are a multiple of 16 and at least 256, or that has one tile); otherwise
 // k-contiguous (`first` = the tile's first row, nvalid = rows; nblk = 8).
 template <bool KM>
 DEVI void setup_operand16(int64_t ld, int first, int nvalid, int W, int oper, int wave, int lane,
@@ -1092,27 +1154,22 @@ DEVI void setup_operand16(int64_t ld, int first, int nvalid, int W, int oper, in
     // instruction i of a wave fills k-rows wave*16 + 2*i + (lane >> 5); the 64-byte chunks of a
     // row are swizzled with k & 3 and the halves of a chunk swapped in rows with k & 8
     const int hl = lane >> 5, piece = lane & 31;
+    const int window = km_window(first, nvalid);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int kr = wave * 16 + 2 * i + hl;
       const int k3 = kr & 3, cf = ((kr >> 3) & 1) * 2;
-      int gp = first * (nblk * 4) + (((piece >> 2) ^ k3) << 2) + ((piece & 3) ^ cf);
-      const int last = nvalid / 8 - 1;
+      int gp = (((piece >> 2) ^ k3) << 2) + ((piece & 3) ^ cf);
+      const int last = (nvalid - window) / 8 - 1;
       gp = gp < last ? gp : last;  // columns past the end are discarded later
       off[i] = 2u * ((uint32_t)kr * (uint32_t)ld + (uint32_t)(gp * 8));
     }
-    const int G = lane >> 4, q = lane & 15, r4 = q >> 2;
-#pragma unroll
-    for (int x = 0; x < 8; ++x) {
-      const int y = W * nblk + x;  // block of 16 columns inside the 256 loaded ones
-      rd[x] = lds_base + oper * ML16_OPER_BYTES + (G * 8 + r4) * 512 + ((((y >> 1) & 7) ^ r4) << 6) +
-              ((((y & 1) ^ G) & 1) << 5) + (q & 3) * 8;
-    }
+    km_fragments(W, nblk, (first - window) >> 4, oper, lane, lds_base, rd);
   }
 }
 
-// A workgroup sweeps the A tiles [ai_begin, ai_end) against one B tile. Requirements checked by
-// the host: K % 64 == 0 and K >= 128; a sweep of more than one A tile has only full A tiles (a
+// A workgroup sweeps the A tiles [ai_begin, ai_end) against one B tile, or (VAR_TN on a flat list) takes
+// a chain of tiles of either operand. Requirements checked by the host: K % 64 == 0 and K >= 128; a sweep of more than one A tile has only full A tiles (a
 // ragged last one as rows [M - 256, M), see GemmArgs::overlap_last_a) and a k-contiguous A (the
 // loader's lane offsets are those of the first tile); every copy of a split-K launch has at least
 // two k-tiles (an even number in all but the last, see split_ktiles).
@@ -1161,20 +1218,20 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
     return (VAR == VAR_NT && g.overlap_last_a != 0 && r + TILE > g.M) ? g.M - TILE : r;
   };
   uint32_t oa[8], ob[8], ra[8], rb[8];
-  setup_operand16<A_KM>(g.lda, A_KM ? ai_begin : a_row0(ai_begin), A_KM ? g.acols : g.M, wa, 0, wave, lane,
-                        lds_base, oa, ra, NA);
-  setup_operand16<B_KM>(g.ldb, B_KM ? bj : bj * TILE, B_KM ? g.bcols : g.N, wb, 1, wave, lane, lds_base, ob, rb);
+  setup_operand16<A_KM>(g.lda, a_row0(ai_begin), A_KM ? g.acols : g.M, wa, 0, wave, lane, lds_base, oa, ra, NA);
+  setup_operand16<B_KM>(g.ldb, bj * TILE, B_KM ? g.bcols : g.N, wb, 1, wave, lane, lds_base, ob, rb);
 
-  // pointers to the next k-tile to fetch and their advance per k-tile in bytes. A k-major
-  // operand's tile column is part of the lane offsets, so its pointer only carries the k offset.
+  // pointers to the next k-tile to fetch and their advance per k-tile in bytes
   const uint32_t stride_a = A_KM ? (uint32_t)(BK * g.lda * 2) : 128u;
   const uint32_t stride_b = B_KM ? (uint32_t)(BK * g.ldb * 2) : 128u;
   auto a_tile_ptr = [&](int ai) -> const char* {
-    return (const char*)(A_KM ? g.A : g.A + (int64_t)a_row0(ai) * g.lda);
+    return (const char*)(A_KM ? g.A + km_window(ai * TM, g.acols) : g.A + (int64_t)a_row0(ai) * g.lda);
+  };
+  auto b_tile_ptr = [&](int b) -> const char* {
+    return (const char*)(B_KM ? g.B + km_window(b * TILE, g.bcols) : g.B + (int64_t)b * TILE * g.ldb);
   };
   const char* pa = a_tile_ptr(ai_begin);
-  const char* pb = (const char*)(B_KM ? g.B : g.B + (int64_t)bj * TILE * g.ldb);
-  const char* pb_next = pb;
+  const char* pb = b_tile_ptr(bj);
   const uint32_t ldsw = lds_base + (uint32_t)wave * 8192u;
   // an odd number of k-tiles: one more pair whose second k-tile is dead (see gen_mainloop16.py)
   const int npairs = (nk + 1) >> 1;
@@ -1209,10 +1266,16 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
   // What an epilogue carries from tile to tile of a sweep has to be small: over the main loop the
   // compiler only has v[0:ML16_*_FIRST_VGPR) for it.
   typename Epi::State st;
-  for (int ai = ai_begin; ai < ai_end; ++ai) {
-    // where the loader goes when this tile's k range is exhausted: the next A tile of the
-    // sweep, or (after the last tile) this tile again, whose first k-tiles are loaded and never used
-    const char* pa_next = a_tile_ptr(ai + 1 < ai_end ? ai + 1 : ai);
+  int ai = ai_begin;
+  for (int step = 1;; ++step) {
+    // where the loader goes when this tile's k range is exhausted: the next A tile of the sweep or tile of
+    // the chain, or (after the last one) this tile again, whose first k-tiles are loaded and never used
+    int ai_next = ai + 1, bj_next = bj;
+    bool more = ai_next < ai_end;
+    if (VAR == VAR_TN) more = sc.xg < 0 && flat_decode(sc, wg, step, bj_next, ai_next);
+    if (!more) { ai_next = ai; bj_next = bj; }
+    const char* pa_next = a_tile_ptr(ai_next);
+    const char* pb_next = b_tile_ptr(bj_next);
     int cnt = npairs;
     if (npairs == 1) { pa = pa_next; pb = pb_next; }
     if (VAR == VAR_NT)
@@ -1260,11 +1323,18 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
     // v[0:ML16_*_FIRST_VGPR) for values that live across it.
     int lane_e = lane;
     asm volatile("" : "+v"(lane_e));
-    Epi::open(st, ep, bj * TILE + wb * 128, split, wa, lane_e, ai == ai_begin);
+    Epi::open(st, ep, bj * TILE + wb * 128, split, wa, lane_e, step == 1);
     const bool complete = Epi::tile(st, ep, a_row0(ai) + wa * (NA * 16), bj * TILE + wb * 128, lane_e, stage, ai * TM,
                                     tokens);
     if (PENDING > 0 && !complete) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     Epi::close(st, ep, bj * TILE + wb * 128, split, wa, lane_e);
+    if (!more) break;
+    if (VAR == VAR_TN) {
+      if (ai_next != ai) km_fragments(wa, NA, (ai_next * TM - km_window(ai_next * TM, g.acols)) >> 4, 0, lane_e, lds_base, ra);
+      if (bj_next != bj) km_fragments(wb, 8, (bj_next * TILE - km_window(bj_next * TILE, g.bcols)) >> 4, 1, lane_e, lds_base, rb);
+    }
+    ai = ai_next;
+    bj = bj_next;
   }
   __builtin_amdgcn_s_waitcnt(0x0070);  // drain the trailing (unused) loads before LDS is released
   Epi::end(st, ep, bj * TILE + wb * 128, split, wa, lane);
@@ -1312,7 +1382,9 @@ DEVI void stage16_put(u16* stage, int lane, int ia, u32x2 v) {
 template <bool EDGE, int MODE, int NA_>
 struct Store16Impl {
   static_assert(NA_ == 8 || EDGE, "narrow tiles use the bounds-checked instance");
-  static constexpr int NA = NA_, TOKEN_BYTES = 0, PENDING_STORES = 0;
+  static constexpr int NA = NA_, TOKEN_BYTES = 0;
+  // A whole sub-tile's stores: 8 columns of 4 (bf16) or of NA (fp32, of which the last 48 may be in flight).
+  static constexpr int PENDING_STORES = MODE == 0 || MODE == 3 ? 32 : 48;
   typedef StoreParams Params;
   struct State {};
   static DEVI void open(State&, const Params&, int, int, int, int, bool) {}
@@ -1366,7 +1438,7 @@ struct Store16Impl {
         }
       }
     });
-    return true;
+    return !EDGE || (p.N - j0 >= 128 && p.M - i0 >= NA * 16);
   }
 };
 template <bool EDGE, int MODE> struct Store16 : Store16Impl<EDGE, MODE, 8> {};
@@ -1772,6 +1844,9 @@ enum { KERNEL_GENERIC = 0, KERNEL16_NT = 4, KERNEL16_TN = 5, KERNEL16_MIX = 6 };
 // K ranges the hand-scheduled main loop takes: at least two whole k-tiles.
 bool k16_ok(int64_t K) { return K >= 2 * BK && K % BK == 0; }
 
+// Whether all n tiles of a k-major operand have the same lane offsets (setup_operand16).
+bool km_chainable(int cols, int n) { return n == 1 || (cols >= TILE && cols % 16 == 0); }
+
 template <class Epi, int KERNEL>
 int launch_sched(const GemmArgs& g, const Sched& sc, const typename Epi::Params& ep, hipStream_t stream) {
   if constexpr (KERNEL >= KERNEL16_NT) {
@@ -1782,8 +1857,11 @@ int launch_sched(const GemmArgs& g, const Sched& sc, const typename Epi::Params&
     // every copy of a split-K launch needs two k-tiles too (split_ktiles() sees to the last one)
     if (!k16_ok(g.K) || (g.ksplit > 1 && (g.kt_per_split < 2 || g.K / BK - (g.ksplit - 1) * g.kt_per_split < 2)))
       return AREAL_ERR_UNSUPPORTED;
-    // a k-major A operand carries its tile column in the lane offsets: one A tile per workgroup
-    if (VAR != VAR_NT && sc.S < ceil_div_i64(sc.nai, sc.xg > 0 ? sc.xg : 1)) return AREAL_ERR_UNSUPPORTED;
+    // a k-major A operand: one A tile per workgroup, or a chain of tiles with the same lane offsets
+    if (sc.xg < 0 && (VAR != VAR_TN || g.ksplit > 1)) return AREAL_ERR_UNSUPPORTED;
+    if (sc.chain > 1 && !(km_chainable(g.acols, sc.ai0 + sc.nai) && km_chainable(g.bcols, sc.bj0 + sc.nbj)))
+      return AREAL_ERR_UNSUPPORTED;
+    if (VAR != VAR_NT && sc.xg >= 0 && sc.S < ceil_div_i64(sc.nai, sc.xg > 0 ? sc.xg : 1)) return AREAL_ERR_UNSUPPORTED;
     hipLaunchKernelGGL((gemm16_sweep<VAR, Epi>), dim3(sched_grid(sc) * (g.ksplit > 1 && sc.xg == 0 ? g.ksplit : 1)),
                        dim3(NTHREADS), 0, stream, g, sc, ep);
   } else {
@@ -1918,6 +1996,12 @@ int launch_store(const GemmArgs& g, const StoreParams& ep, int mode, hipStream_t
   bool allow16 = true;
   if (mode == 0 || mode == 3) allow16 = ep.ldo % 8 == 0 && aligned16(ep.out) && ep.M % 8 == 0;
   Regions r = plan_regions(ep.M, ep.N, g.K, 0, 1 << 20, allow16);
+  Sched flat;
+  if (KERNEL16 == KERNEL16_TN && layout == nullptr && g.ksplit <= 1) {
+    const int nai = (int)ceil_div_i64(ep.M, TILE), nbj = (int)ceil_div_i64(ep.N, TILE);
+    flat = make_flat_sched(nbj, nai, km_chainable(g.acols, nai) && km_chainable(g.bcols, nbj));
+    layout = &flat;
+  }
   r.layout = layout;
   if constexpr (KERNEL16 != KERNEL16_NT) {
     // the modes the two backward contractions use: dWeight 0 - 2, dHidden 0, 1 and 3
@@ -2070,12 +2154,11 @@ int launch_dhidden(const u16* w, int64_t V, const u16* dl, int64_t ldv, int64_t 
   return launch_dhidden_k<KERNEL16_NT>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream);
 }
 
-// dWeight [V, H] in bf16 has ceil(V / 256) x ceil(H / 256) output tiles, one per workgroup, in
-// super-blocks of 32 that go round-robin to the XCDs. When their number is not a multiple of 8 the
-// last round occupies a few XCDs for a whole K range while the others idle (594 x 16 tiles: 298
-// super-blocks, 38 rounds on two XCDs against 37 on six). The B tiles of that last partial round
-// are then contracted by a second launch that splits the token (K) range over z copies of its
-// schedule, fp32 partial results summed by splitk_reduce_bf16_kernel.
+// dWeight [V, H] in bf16 has ceil(V / 256) x ceil(H / 256) output tiles. When their number is not a
+// multiple of the chip's 256 CUs the last round occupies a few of them for a whole K range while the
+// others idle (594 x 16 tiles: 37.1 rounds). The B tiles of that last partial round are then contracted
+// by a second launch that splits the token (K) range over z copies of its schedule, fp32 partial results
+// summed by splitk_reduce_bf16_kernel.
 struct DwTail {
   int nbj_main;  // B tiles of the first launch
   int z, kps;    // copies and k-tiles per copy of the second (z <= 1: there is none)
@@ -2086,27 +2169,23 @@ DwTail plan_dw_tail(int64_t H, int64_t V, int64_t Tpad) {
   const int nai = (int)ceil_div_i64(H, TILE), nbj = (int)ceil_div_i64(V, TILE);
   DwTail t{nbj, 1, 0, 0, 32};
   if (!k16_ok(Tpad) || H % 8 != 0) return t;
-  const Sched sc = make_sched(0, nbj, 0, nai, nai);
-  if (sc.n_sb % 8 == 0) return t;
-  const int n_sb_s = sc.n_sb / sc.n_sb_j;
-  int nj = sc.n_sb_j;
-  while (nj > 0 && (nj * n_sb_s) % 8 != 0) --nj;
-  if (nj == 0) return t;
+  const int64_t tiles = (int64_t)nbj * nai, rounds = tiles / 256;
+  if (rounds == 0 || tiles % 256 == 0) return t;
+  const int nbj_main = (int)(rounds * 256 / nai);
   const int64_t nk = Tpad / BK;
   int best = 1, best_sb = 32;
-  double best_cost = sched_cost(make_sched(nj * sc.RB, nbj - nj * sc.RB, 0, nai, nai), 1);
+  double best_cost = sched_cost(make_sched(nbj_main, nbj - nbj_main, 0, nai, nai), 1);
   for (int sb_wgs = 32; sb_wgs >= 8; sb_wgs -= 24) {
-    const Sched st = make_sched(nj * sc.RB, nbj - nj * sc.RB, 0, nai, nai, sb_wgs);
+    const Sched st = make_sched(nbj_main, nbj - nbj_main, 0, nai, nai, sb_wgs);
     for (int z = 2; z <= 8 && z <= nk / 8; ++z) {
       const double cost = sched_cost(st, z);
       if (cost < best_cost - 1e-9) { best_cost = cost; best = z; best_sb = sb_wgs; }
     }
   }
-  // rounds of a whole K range: before, and after with the first launch's even rounds. A k-tile
-  // takes about a microsecond; the two extra launches have to be paid for.
-  const double before = (double)ceil_div_i64(sc.n_sb, 8), after = (double)(nj * n_sb_s / 8) + best_cost;
-  if (best <= 1 || (before - after) * (double)nk < 16.0) return t;
-  t.nbj_main = nj * sc.RB;
+  // rounds of a whole K range: one more, or the second launch's. A k-tile takes about a microsecond;
+  // the two extra launches have to be paid for.
+  if (best <= 1 || (1.0 - best_cost) * (double)nk < 16.0) return t;
+  t.nbj_main = nbj_main;
   t.z = best;
   t.sb_wgs = best_sb;
   split_ktiles((int)nk, t.z, t.kps);
