@@ -536,6 +536,7 @@ struct LMHeadArgs {
   Tensor accum;         // fp32 accumulator of the weight gradient
   Tensor owner;         // fp32 parameter whose .grad is that accumulator, see LMHeadState
   int64_t save_limit, bwd_budget;
+  bool logprobs_only = false;  // no other output (and no backward)
 };
 
 // An int that the device makes (`flag`), on its way to the host: in pinned memory, -1 until it has been
@@ -599,15 +600,19 @@ variable_list lm_head_forward(const Tensor& hidden, const Tensor& weight, const 
   const Tensor bias_f = bias.defined() ? bias.detach().to(at::kFloat).contiguous() : Tensor();
   const int64_t T = h2.size(0);
   variable_list outs(6);
-  for (int i = 0; i < (a.with_moments ? 6 : 4); ++i) outs[i] = empty(h2, labels.sizes(), at::kFloat);
+  for (int i = 0; i < (a.logprobs_only ? 1 : a.with_moments ? 6 : 4); ++i) outs[i] = empty(h2, labels.sizes(), at::kFloat);
   const int64_t need = 2 * round_up(T, 128) * round_up(V, 64);
   const bool save = needs_grad && T > 0 &&
                     (a.save_probs >= 0 ? a.save_probs != 0
                                        : need <= a.save_limit && fits_memory(need, h2.device().index()));
   // row_max, sum_exp [T] (and the copy of the log-probabilities and the row references) in one allocation
   const int64_t Tp = round_up(T, 64);
-  const Tensor rows = empty_f32(h2, Tp * (save ? 4 : 2));
-  const Tensor row_max = rows.narrow(0, 0, T), sum_exp = rows.narrow(0, Tp, T);
+  Tensor rows, row_max, sum_exp;
+  if (!a.logprobs_only) {
+    rows = empty_f32(h2, Tp * (save ? 4 : 2));
+    row_max = rows.narrow(0, 0, T);
+    sum_exp = rows.narrow(0, Tp, T);
+  }
   Tensor probs, probs_ref, probs_status, lp_copy;
   std::shared_ptr<Status> status;
   if (save) {
@@ -762,13 +767,13 @@ std::vector<OptTensor> lm_head_backward(const std::shared_ptr<LMHeadState>& st, 
 py::tuple lm_head(const Tensor& hidden, const Tensor& weight, const OptTensor& bias_arg, const Tensor& labels,
                   double temperature, double logit_scale, int64_t token_chunk, int save_probs, bool with_moments,
                   const OptTensor& accum, const OptTensor& owner, int64_t save_limit, int64_t bwd_budget,
-                  bool build_graph, bool needs_grad) {
+                  bool build_graph, bool needs_grad, bool logprobs_only) {
   const Tensor bias = or_undefined(bias_arg);
   for (const Tensor* t : {&hidden, &weight, &bias}) refuse_tangent(*t);
   require_gpu(hidden, weight, labels, bias);
   const c10::hip::HIPGuard guard(hidden.device().index());
   const LMHeadArgs a{temperature, logit_scale, token_chunk, save_probs, with_moments, or_undefined(accum),
-                     or_undefined(owner), save_limit, bwd_budget};
+                     or_undefined(owner), save_limit, bwd_budget, logprobs_only && !needs_grad && !build_graph};
   std::shared_ptr<LMHeadState> state;
   variable_list saved;
   const variable_list outs = lm_head_forward(hidden, weight, bias, labels, a, needs_grad,

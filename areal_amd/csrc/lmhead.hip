@@ -706,7 +706,9 @@ template <bool E> using FwdAffineMomSave = FwdEpi<E, true, true, true>;
 // are 8 blocks whose waves walk 74 slots one after the other (33 us); TOK = 16 and one pass
 // for the saving sweep's sums take 9.8 (10007 tokens: 18.9 -> 9.9).
 // labels (nullable): the slots hold no label logits, a valid label's is entry t of that statistic's plane.
-// ref_sums: the slots' sums S, Q are relative to row_ref[t] (the saving forward of the
+// ref_sums = 2: the slots hold a reference of their own (in binades) and the sum relative to it, nothing
+// else (Logp16); the final expression is evaluated in fp64 as for 1.
+// ref_sums = 1: the slots' sums S, Q are relative to row_ref[t] (the saving forward of the
 // hand-scheduled kernels) instead of to each slot's own maximum; the final expressions are then
 // evaluated in fp64, where c2 x - ref and log S (each up to REF_WINDOW binades) cancel.
 // gate / gate_run_if_set: as GemmArgs::skip_if_set / run_if_set. host_status (nullable, pinned host
@@ -733,7 +735,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
   const int64_t PT = (int64_t)P * T;
   const bool moments = vmean != nullptr || vnorm != nullptr;
   float M = neg_inf();
-  if (!ref_sums) {  // the sums need the maximum first
+  if (ref_sums != 1) {  // the sums need the maximum first
 #pragma unroll 4
     for (int p = row; p < P; p += ROWS) M = fmaxf(M, ws[(int64_t)p * T + tt]);
     sh_f[0][row][tok] = M;
@@ -749,6 +751,10 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
   for (int p = row; p < P; p += ROWS) {
     const float* w = ws + (int64_t)p * T + tt;
     const float m = w[0];
+    if (ref_sums == 2) {
+      S += exp2f(m - M) * w[1 * PT];
+      continue;
+    }
     if (ref_sums) {
       M = fmaxf(M, m);
       S += w[1 * PT];
@@ -763,7 +769,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
     mn = fminf(mn, w[4 * PT]);
     if (moments) { sx += (double)w[5 * PT]; sx2 += (double)w[6 * PT]; }
   }
-  if (ref_sums) sh_f[0][row][tok] = M;
+  if (ref_sums == 1) sh_f[0][row][tok] = M;
   sh_f[1][row][tok] = S; sh_f[2][row][tok] = Q; sh_f[3][row][tok] = xl; sh_f[4][row][tok] = mn;
   sh_d[0][row][tok] = sx; sh_d[1][row][tok] = sx2;
   __syncthreads();
@@ -772,7 +778,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
 #pragma unroll
   for (int i = 0; i < MERGE_WAVES; ++i) {
     const int r = i * G + grp;
-    if (ref_sums) M = fmaxf(M, sh_f[0][r][tok]);
+    if (ref_sums == 1) M = fmaxf(M, sh_f[0][r][tok]);
     S += sh_f[1][r][tok]; Q += sh_f[2][r][tok]; xl += sh_f[3][r][tok];
     mn = fminf(mn, sh_f[4][r][tok]);
     sx += sh_d[0][r][tok]; sx2 += sh_d[1][r][tok];
@@ -787,7 +793,14 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
   if (grp != 0 || t >= T) return;
   if (labels != nullptr) {
     const int64_t l = labels[t];
-    xl = l >= 0 && l < V ? ws[3 * PT + t] : 0.f;
+    const bool valid = l >= 0 && l < V;
+    xl = valid ? ws[3 * PT + t] : 0.f;
+    if (ref_sums == 2) {
+      const float lp = (float)(((double)xl * (double)c2 - (double)M) * 0.6931471805599453094 - log((double)S));
+      logprobs[t] = valid && xl == xl ? fminf(lp, 0.f) : lp;  // (as below: a label's logit is at most the maximum)
+      if (logprobs_copy) logprobs_copy[t] = logprobs[t];
+      return;
+    }
   }
   if (ref_sums) {
     const double ln2 = 0.6931471805599453094;
@@ -1543,7 +1556,7 @@ struct Fwd16 {
   // last tile of a ragged vocabulary overlaps its predecessor); entries below it take no part.
   // Returns whether all PENDING_STORES stores were issued.
   static DEVI bool tile(State& st, const Params& p, int v0, int t0, int lane, u16* stage, int v_new,
-                        const void* tokens) {
+                        void* tokens) {
     if (v_new >= v0 + 128) return false;  // every row of this wave's sub-tile is a repeat
     if (t0 >= p.T) return false;          // no token
     // (Wave-uniform. Two bodies: one for both held the 32 logits of a column in other registers than the
@@ -1759,6 +1772,141 @@ template <bool E> using Fwd16PlainSave = Fwd16<E, false, false, true>;
 template <bool E> using Fwd16PlainMomSave = Fwd16<E, false, true, true>;
 template <bool E> using Fwd16AffineSave = Fwd16<E, true, false, true>;
 template <bool E> using Fwd16AffineMomSave = Fwd16<E, true, true, true>;
+
+// ---- forward for the label log-probabilities alone (see Fwd16): the sum of a token's exponentials relative to
+// a reference of its own, the largest logit of the first column. Per logit one accumulator read, one fma, one v_exp_f32 and one addition; no maximum is taken (nor minimum, nor
+// the entropy's sum) unless a column's sum shows that the reference is too low by LOGP_WINDOW binades,
+// which the first column's always does. The column is then summed again relative to a new reference while
+// its logits are still in registers, and the sums so far move to it: right for any logits, without a launch
+// that estimates references and a repeat behind it. The references lie in LDS between the tiles.
+// 10007 x 1536 x 151936: 3384 -> 3297 us against the sweep with all outputs, with the merge and host side the whole call
+// 3361 -> 3244.
+constexpr float LOGP_WINDOW = 84.f;
+constexpr float LOGP_NO_REF = -3e38f;  // so far below every logit that the first column's sum overflows
+template <bool EDGE, bool AFFINE>
+struct Logp16 {
+  static constexpr int NA = 8;
+  static constexpr bool RAGGED_B = true;
+  static constexpr int TOKEN_BYTES = 1024, PENDING_STORES = 0;
+  typedef FwdParams Params;
+  // lane group g: token columns g and g + 4, their sums and the references these are relative to
+  struct State { float s[2], ref[2]; };
+  static DEVI void split_output(Params&, int64_t) {}
+  static DEVI void open(State& st, const Params&, int, int, int, int, bool first) {
+    if (first) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) { st.s[k] = 0.f; st.ref[k] = LOGP_NO_REF; }
+    }
+  }
+  static DEVI void close(State&, const Params&, int, int, int, int) {}
+  static DEVI void load_tokens(const Params& p, int t0, int lane, void* tokens) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int t = t0 + h * 64 + lane;
+      t = t < p.T ? t : p.T - 1;
+      const int64_t l = p.labels[t];
+      ((int*)tokens)[h * 64 + lane] = l >= 0 && l < p.V ? (int)l : -1;
+      ((float*)tokens)[128 + h * 64 + lane] = LOGP_NO_REF;
+    }
+  }
+  static DEVI bool tile(State& st, const Params& p, int v0, int t0, int lane, u16*, int v_new, void* tokens) {
+    if (v_new >= v0 + 128 || t0 >= p.T) return true;
+    if (EDGE || v_new > v0) columns<true>(st, p, v0, t0, lane, v_new, tokens);
+    else columns<false>(st, p, v0, t0, lane, v_new, tokens);
+    return true;
+  }
+  template <bool MASKED>
+  static DEVI void columns(State& st, const Params& p, int v0, int t0, int lane, int v_new, void* tokens) {
+    const int vl = v0 + 4 * (lane >> 4), group = lane >> 4;
+    auto vidx = [&](int a, int r) { return vl + a * 16 + r; };
+    auto out = [&](int i) { return MASKED && (vidx(i >> 2, i & 3) >= p.V || vidx(i >> 2, i & 3) < v_new); };
+    int lab[8];
+    float ref[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      lab[b] = ((const int*)tokens)[b * 16 + (lane & 15)];
+      ref[b] = ((const float*)tokens)[128 + b * 16 + (lane & 15)];
+    }
+    const int v_from = v_new > v0 ? v_new : v0;
+    float* const label_logit = p.ws + 3 * (int64_t)p.P * p.T;
+    auto add = [](float a, float b) { return a + b; };
+    float cs[2];
+    ML16_AGPR_FENCE();
+    for_each_col([&](auto bc) {
+      constexpr int b = decltype(bc)::value;
+      constexpr int k = b >> 2, c = b & 3;
+      float x[32];
+      acc_col<b>(x);
+      if (AFFINE) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+          float bv = 0.f;
+          if (p.bias != nullptr && (!MASKED || vidx(i >> 2, i & 3) < p.V)) bv = p.bias[vidx(i >> 2, i & 3)];
+          x[i] = (x[i] + bv) * p.scale;
+        }
+      }
+      auto sum = [&](float r) {
+        float s = 0.f;
+#pragma unroll
+        for (int a = 0; a < 8; ++a) {
+#pragma unroll
+          for (int i = a * 4; i < a * 4 + 4; ++i) {
+            const float e = fast_exp2(fmaf(x[i], p.c2, -r));
+            s += out(i) ? 0.f : e;
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          ML16_AGPR_FENCE();
+        }
+        return s;
+      };
+      float s = sum(ref[b]);
+      asm volatile("" : "+v"(s) : : ML16_ACC_CLOBBERS);
+      // a column's 32 exponentials within the window add up to 2^89 at most (NaN takes this way too)
+      if (__builtin_amdgcn_ballot_w64(!(s <= 0x1p90f)) != 0) {
+        float m = neg_inf();
+#pragma unroll
+        for (int i = 0; i < 32; ++i) m = fmaxf(m, out(i) ? neg_inf() : x[i]);
+        m = group_max(m) * p.c2;
+        const float r = m - ref[b] > LOGP_WINDOW ? m : ref[b];
+        if (group == c) {
+          st.s[k] *= fast_exp2(ref[b] - r);
+          st.ref[k] = r;
+        }
+        ((float*)tokens)[128 + b * 16 + (lane & 15)] = r;  // (the same from all four lanes of a token)
+        s = sum(r);
+        asm volatile("" : "+v"(s) : : ML16_ACC_CLOBBERS);
+      }
+      const bool hit = (lab[b] >= v_from) && (lab[b] < v0 + 128);
+      if (__builtin_amdgcn_ballot_w64(hit) != 0) {
+        float xl = 0.f;
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+          if (vidx(i >> 2, i & 3) == lab[b]) xl = x[i];
+        const int t = t0 + b * 16 + (lane & 15);
+        if (hit && t < p.T && (((lab[b] - v0) >> 2) & 3) == group) label_logit[t] = xl;
+      }
+      if constexpr (c < 2) cs[c] = s;
+      else cs[c - 2] = fold_cols32(cs[c - 2], s, add);
+      if constexpr (c == 3) {
+        st.s[k] += fold_cols16(cs[0], cs[1], add);
+        asm volatile("" : "+v"(st.s[k]), "+v"(st.ref[k]) : : ML16_ACC_CLOBBERS);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+  static DEVI void end(State& st, const Params& p, int t0, int split, int wa, int lane) {
+    const int64_t PT = (int64_t)p.P * p.T;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int t = t0 + ((lane >> 4) + 4 * k) * 16 + (lane & 15);
+      if (t >= p.T) continue;
+      float* w = p.ws + (int64_t)(p.slot_base + split * 2 + wa) * p.T + t;
+      w[0 * PT] = st.ref[k]; w[1 * PT] = st.s[k];
+    }
+  }
+};
+template <bool E> using Logp16Plain = Logp16<E, false>;
+template <bool E> using Logp16Affine = Logp16<E, true>;
 
 // ---- recompute: dlogits = (onehot - p) * g * invT * scale in bf16, [Tc, ldv] (see BwdEpi)
 template <bool EDGE, bool AFFINE>
@@ -2293,9 +2441,9 @@ size_t areal_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V) {
 }
 
 // Forward. hidden [T,H] bf16, weight [V,H] bf16, labels [T] int64 (labels outside [0, V) give
-// a label logit of 0). Outputs are fp32 [T]; any output pointer other than row_max / sum_exp
-// may be null; vocab_mean and vocab_norm cost two extra operations per logit and are computed
-// only when one of them is requested.
+// a label logit of 0). Outputs are fp32 [T]; any output pointer may be null; vocab_mean and
+// vocab_norm cost two extra operations per logit and are computed only when one of them is requested,
+// and logprobs without any other output takes a sweep of its own (Logp16).
 //
 // probs / probs_ref / probs_status (all null or all set) keep the exponentials of the softmax
 // for areal_lmhead_bwd_saved: probs bf16 [round_up(T, 128)][round_up(V, 64)] (rows >= T are left
@@ -2378,7 +2526,15 @@ int areal_lmhead_fwd_ex(const void* hidden, const void* weight, const float* bia
                        entropy, vocab_min, vocab_max, vocab_mean, vocab_norm, row_max, sum_exp, ref,
                        probs_status, gate, gate_run_if_set, logprobs_copy, host);
   };
-  if (probs == nullptr) {
+  // The sweep for log-probabilities alone is never the slower one: an epilogue of less work and no other launches.
+  const bool logp_only = entropy == nullptr && vocab_min == nullptr && vocab_max == nullptr && !moments &&
+                         row_max == nullptr && sum_exp == nullptr && logprobs != nullptr;
+  if (probs == nullptr && logp_only && r.k16) {
+    rc = affine ? launch_gemm<Logp16Affine, FwdAffine, FwdParams, KERNEL16_NT, true>(g, r, ep, ep_a, stream)
+                : launch_gemm<Logp16Plain, FwdPlain, FwdParams, KERNEL16_NT, true>(g, r, ep, ep_a, stream);
+    if (rc != AREAL_OK) return rc;
+    merge(2, nullptr, nullptr, 0, nullptr);
+  } else if (probs == nullptr) {
     if ((rc = fwd_plain(g)) != AREAL_OK) return rc;
     merge(0, nullptr, nullptr, 0, nullptr);
   } else if (r.k16) {

@@ -38,8 +38,9 @@ def compute_logprobs(
     if hidden.ndim == 3 and hidden.shape[0] == 1:
         hidden = hidden.squeeze(0)
     with torch.no_grad():
-        out = fused_lm_head_logprobs_entropy(
-            hidden, lm_head_weight, _labels(inputs), temperature=temperature
+        out = _lm_head(
+            hidden, lm_head_weight, _labels(inputs), temperature, 1.0, None, None, None, False, None, None,
+            logprobs_only=True,
         )
     logprobs = out.logprobs
     return logprobs[:-pad_length] if pad_length > 0 else logprobs
@@ -199,8 +200,9 @@ class FusedLMHeadAdapter:
         with torch.no_grad():
             hidden = self.hidden_states(model_inputs)
             weight = self._weight(hidden)[0]
-            out = fused_lm_head_logprobs_entropy(
-                hidden, weight, _labels(model_inputs), temperature=self.temperature, bias=self._bias()
+            out = _lm_head(
+                hidden, weight, _labels(model_inputs), self.temperature, 1.0, self._bias(), None, None, False, None,
+                None, logprobs_only=True,
             )
         logprobs = out.logprobs
         return logprobs[:-pad_length] if pad_length > 0 else logprobs

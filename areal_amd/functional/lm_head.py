@@ -72,7 +72,7 @@ class _FusedLMHead(torch.autograd.Function):
         # caller has ruled out no_grad mode.
         accum, owner = args[5:7]
         needs_grad = any(ctx.needs_input_grad[:2]) or accum is not None or owner is not None
-        outs, saved, state = _lib.host().lm_head(hidden, weight, bias, labels, *args, True, needs_grad)
+        outs, saved, state = _lib.host().lm_head(hidden, weight, bias, labels, *args, True, needs_grad, False)
         ctx.save_for_backward(*saved)
         ctx.state = state
         ctx.probs, ctx.probs_ref, ctx.probs_status = state.probs, state.probs_ref, state.probs_status
@@ -138,10 +138,11 @@ def fused_lm_head_logprobs_entropy(
 
 def _lm_head(
     hidden, weight, labels, temperature, logit_scale, bias, token_chunk, save_probs, with_moments,
-    weight_grad_accum, weight_grad_owner,
+    weight_grad_accum, weight_grad_owner, logprobs_only=False,
 ) -> ChunkedLMHeadOutput:
     """``weight_grad_owner``: the fp32 parameter ``weight`` is a compute copy of; the weight gradient
-    is added to its ``.grad`` as it is when the backward runs, or becomes it."""
+    is added to its ``.grad`` as it is when the backward runs, or becomes it.
+    ``logprobs_only`` (in no_grad mode): the other outputs are ``None`` and the sweep does not compute them."""
     if not math.isfinite(temperature) or temperature <= 0:
         raise ValueError(f"temperature must be positive, got {temperature}")
     if not math.isfinite(logit_scale) or logit_scale <= 0:
@@ -187,7 +188,7 @@ def _lm_head(
     if torch.is_grad_enabled():
         values = _FusedLMHead.apply(hidden, weight, bias, labels, args)
     else:
-        values = _lib.host().lm_head(hidden, weight, bias, labels, *args, False, False)
+        values = _lib.host().lm_head(hidden, weight, bias, labels, *args, False, False, logprobs_only)
     return ChunkedLMHeadOutput(*values)
 
 

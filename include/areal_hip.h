@@ -57,8 +57,8 @@ size_t areal_lmhead_fwd_workspace_bytes(int64_t T, int64_t H, int64_t V);
 size_t areal_lmhead_probs_bytes(int64_t T, int64_t V);
 
 /* hidden [T,H] bf16, weight [V,H] bf16 (H % 8 == 0, 16-byte aligned), bias [V] fp32 or NULL,
- * labels [T] int64. Outputs fp32 [T]; row_max and sum_exp are the state saved for backward
- * (vocab_parallel_head.py:704-713). logits = (hidden . weight^T + bias) * logit_scale.
+ * labels [T] int64. Outputs fp32 [T], each may be NULL; row_max and sum_exp are the state saved
+ * for backward (vocab_parallel_head.py:704-713). logits = (hidden . weight^T + bias) * logit_scale.
  *
  * probs / probs_ref / probs_status (all NULL, or all set) additionally keep the softmax
  * exponentials for areal_lmhead_bwd_saved, the counterpart of autograd saving the logits in the
