@@ -17,6 +17,10 @@
 
 namespace {
 
+// 16- and 8-byte accesses at any address of the element type
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef u32x2 u32x2_any __attribute__((aligned(1)));
+
 constexpr int GAE_THREADS = 256;
 constexpr int GAE_ITEMS = 8;
 constexpr int GAE_TILE = GAE_THREADS * GAE_ITEMS;
@@ -387,13 +391,14 @@ DEVI void gae_owned_items(int64_t t0, int64_t t_begin, int64_t t_end, int& i_lo,
 enum { GAE_LAYOUT_CU = 0, GAE_LAYOUT_ROWS = 1, GAE_LAYOUT_ONE_ROW = 2 };
 
 // (rw, v, ms): the tile's inputs as gae_load_items leaves them (at least the owned tokens).
-// LAMBDAS: a lambda per sequence (GaeArgs::lam_seq).
+// LAMBDAS: a lambda per sequence (GaeArgs::lam_seq). row_boot (one row): GaeArgs::no_eos of the row, if the caller
+// has it at hand (0 / 1).
 template <bool STATS, int LAYOUT, bool LAMBDAS>
 DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t t_end, int s_first,
                        int n_own, const int32_t* cu_own, double& A0, double& nv0,
                        double (&rs)[STATS ? 5 : 1], MapF* smem, MapF* all,
                        const float (&rw)[GAE_ITEMS], const float (&v)[GAE_ITEMS],
-                       const float (&ms)[GAE_ITEMS], float (&oa)[GAE_ITEMS]) {
+                       const float (&ms)[GAE_ITEMS], float (&oa)[GAE_ITEMS], int row_boot = -1) {
   constexpr bool uniform = LAYOUT != GAE_LAYOUT_CU;
   const int tid = threadIdx.x;
   const int64_t t0 = tile * GAE_TILE + (int64_t)tid * GAE_ITEMS;
@@ -450,7 +455,8 @@ DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t 
         }
         if (i == e_loc - 1) {
           ends |= 1u << i;
-          if (g.no_eos != nullptr && g.no_eos[s_first + sq] != 0) boot |= 1u << i;
+          if (LAYOUT == GAE_LAYOUT_ONE_ROW && row_boot >= 0) boot |= (unsigned)row_boot << i;
+          else if (g.no_eos != nullptr && g.no_eos[s_first + sq] != 0) boot |= 1u << i;
         }
       }
     }
@@ -519,8 +525,8 @@ DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t 
     if (valid == (1u << GAE_ITEMS) - 1u) {
 #pragma unroll
       for (int q = 0; q < GAE_ITEMS / 4; ++q) {
-        *(f32x4*)(g.adv + t0 + 4 * q) = f32x4{oa[4 * q], oa[4 * q + 1], oa[4 * q + 2], oa[4 * q + 3]};
-        *(f32x4*)(g.ret + t0 + 4 * q) = f32x4{orr[4 * q], orr[4 * q + 1], orr[4 * q + 2], orr[4 * q + 3]};
+        *(f32x4_any*)(g.adv + t0 + 4 * q) = f32x4{oa[4 * q], oa[4 * q + 1], oa[4 * q + 2], oa[4 * q + 3]};
+        *(f32x4_any*)(g.ret + t0 + 4 * q) = f32x4{orr[4 * q], orr[4 * q + 1], orr[4 * q + 2], orr[4 * q + 3]};
       }
     } else {
 #pragma unroll
@@ -1599,15 +1605,15 @@ struct PrepArgs {
   uint8_t* no_eos_out;       // [bs]
 };
 
-DEVI void adv_prep_token(const PrepArgs& a, float lm, float lp, float rf_in, bool has_ref, bool at_end,
+DEVI void adv_prep_token(const PrepArgs& a, int estimator, float lm, float lp, float rf_in, bool has_ref, bool at_end,
                          bool at_out, float score, float neg_ctl, float& old, float& ref, float& kl,
                          float& gkl, float& oc) {
   old = lp * lm;
   ref = has_ref ? rf_in * lm : 0.f * lm;
   const float diff = old - ref;
   float est;
-  if (a.estimator == 1) est = diff;
-  else if (a.estimator == 2) est = diff * diff / 2.0f;
+  if (estimator == 1) est = diff;
+  else if (estimator == 2) est = diff * diff / 2.0f;
   else { const float neg = -diff; est = expf(neg) - 1.f - neg; }
   if (a.apply_clamp) est = fminf(fmaxf(est, -10.f), 10.f);
   kl = neg_ctl * est;
@@ -1615,9 +1621,12 @@ DEVI void adv_prep_token(const PrepArgs& a, float lm, float lp, float rf_in, boo
   oc = at_out ? score : 0.f;
 }
 
-// VEC: L % 16 == 0 and every array 16-byte aligned: four tokens per thread and step, 16-byte
-// loads and stores (the rolled neighbour of a group's last token is one extra scalar load).
-template <bool VEC>
+// Four tokens per thread and step, 16-byte loads and stores at whatever alignment the row has (the rolled
+// neighbour of a group's last token is one extra scalar load), the row's last L % 4 tokens one by one. One token
+// per thread and step, which rows of another length than a multiple of 16 used to take: a batch of
+// 1000 x 8191 131 -> 111 us in all.
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
 __global__ __launch_bounds__(NORM_THREADS) void adv_prep_kernel(PrepArgs a) {
   __shared__ double smem[4];
   const int64_t b = blockIdx.x, L = a.L;
@@ -1625,21 +1634,16 @@ __global__ __launch_bounds__(NORM_THREADS) void adv_prep_kernel(PrepArgs a) {
   const uint8_t* lmk = a.loss_mask + b * L;
   const float* lp = a.logp + b * L;
   float* rf = a.ref_logp ? a.ref_logp + b * L : nullptr;
-  double cnt = 0.0;
-  if (VEC) {
-    for (int64_t t = (int64_t)threadIdx.x * 16; t < L; t += (int64_t)blockDim.x * 16) {
-      const u32x4 w = *(const u32x4*)(am + t);
-      int c = 0;
+  int cnt = 0;
+  for (int64_t t = (int64_t)threadIdx.x * 16; t + 16 <= L; t += (int64_t)blockDim.x * 16) {
+    const u32x4 w = *(const u32x4_any*)(am + t);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) c += ((w[i] >> (8 * k)) & 0xffu) ? 1 : 0;
-      cnt += (double)c;
-    }
-  } else {
-    for (int64_t t = threadIdx.x; t < L; t += blockDim.x) cnt += am[t] ? 1.0 : 0.0;
+      for (int k = 0; k < 4; ++k) cnt += ((w[i] >> (8 * k)) & 0xffu) ? 1 : 0;
   }
-  const int64_t seqlen = (int64_t)block_sum_d(cnt, smem);
+  if (threadIdx.x < (L & 15)) cnt += am[(L & ~(int64_t)15) + threadIdx.x] ? 1 : 0;
+  const int64_t seqlen = (int64_t)block_sum_d((double)cnt, smem);
   const bool no_eos = seqlen == L;
   if (threadIdx.x == 0) { a.seqlens_out[b] = seqlen; a.no_eos_out[b] = no_eos ? 1 : 0; }
   const int64_t t_end = seqlen - 1 >= 0 ? seqlen - 1 : seqlen - 1 + L;  // rewards[b, seqlen - 1] = 0
@@ -1648,41 +1652,40 @@ __global__ __launch_bounds__(NORM_THREADS) void adv_prep_kernel(PrepArgs a) {
   if (a.mask_no_eos_with_zero && no_eos) score = 0.f;
   const float neg_ctl = -a.kl_ctl;
   const bool has_ref = rf != nullptr;
-  if (VEC) {
-    for (int64_t t = (int64_t)threadIdx.x * 4; t < L; t += (int64_t)blockDim.x * 4) {
-      const int64_t tn = t + 4 < L ? t + 4 : 0;  // the roll's neighbour of the group's last token
-      const uint32_t mw = *(const uint32_t*)(lmk + t);
-      const float lmv[4] = {((mw >> 8) & 0xffu) ? 1.f : 0.f, ((mw >> 16) & 0xffu) ? 1.f : 0.f,
-                            (mw >> 24) ? 1.f : 0.f, lmk[tn] ? 1.f : 0.f};
-      const f32x4 lv = *(const f32x4*)(lp + t);
-      const float lpv[4] = {a.roll_logp ? lv[1] : lv[0], a.roll_logp ? lv[2] : lv[1],
-                            a.roll_logp ? lv[3] : lv[2], a.roll_logp ? lp[tn] : lv[3]};
-      f32x4 rv = {0.f, 0.f, 0.f, 0.f};
-      if (has_ref) rv = *(const f32x4*)(rf + t);
-      f32x4 o_lm, o_old, o_ref, o_kl, o_gkl, o_oc, o_tot;
+  const int64_t L4 = L & ~(int64_t)3;
+  for (int64_t t = (int64_t)threadIdx.x * 4; t < L4; t += (int64_t)blockDim.x * 4) {
+    const int64_t tn = t + 4 < L ? t + 4 : 0;  // the roll's neighbour of the group's last token
+    const uint32_t mw = *(const u32_any*)(lmk + t);
+    const float lmv[4] = {((mw >> 8) & 0xffu) ? 1.f : 0.f, ((mw >> 16) & 0xffu) ? 1.f : 0.f,
+                          (mw >> 24) ? 1.f : 0.f, lmk[tn] ? 1.f : 0.f};
+    const f32x4 lv = *(const f32x4_any*)(lp + t);
+    const float lpv[4] = {a.roll_logp ? lv[1] : lv[0], a.roll_logp ? lv[2] : lv[1],
+                          a.roll_logp ? lv[3] : lv[2], a.roll_logp ? lp[tn] : lv[3]};
+    f32x4 rv = {0.f, 0.f, 0.f, 0.f};
+    if (has_ref) rv = *(const f32x4_any*)(rf + t);
+    f32x4 o_lm, o_old, o_ref, o_kl, o_gkl, o_oc, o_tot;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float old, ref, kl, gkl, oc;
-        adv_prep_token(a, lmv[i], lpv[i], rv[i], has_ref, t + i == t_end, t + i == t_out, score, neg_ctl,
-                       old, ref, kl, gkl, oc);
-        o_lm[i] = lmv[i]; o_old[i] = old; o_ref[i] = ref; o_kl[i] = kl; o_gkl[i] = gkl; o_oc[i] = oc;
-        o_tot[i] = gkl + oc;
-      }
-      if (has_ref && a.ref_in_place) *(f32x4*)(rf + t) = o_ref;
-      *(f32x4*)(a.lm_out + b * L + t) = o_lm;
-      *(f32x4*)(a.old_out + b * L + t) = o_old;
-      *(f32x4*)(a.kl_out + b * L + t) = o_kl;
-      if (a.gkl_out) *(f32x4*)(a.gkl_out + b * L + t) = o_gkl;
-      if (a.outcome_out) *(f32x4*)(a.outcome_out + b * L + t) = o_oc;
-      *(f32x4*)(a.tot_out + b * L + t) = o_tot;
+    for (int i = 0; i < 4; ++i) {
+      float old, ref, kl, gkl, oc;
+      adv_prep_token(a, a.estimator, lmv[i], lpv[i], rv[i], has_ref, t + i == t_end, t + i == t_out, score, neg_ctl,
+                     old, ref, kl, gkl, oc);
+      o_lm[i] = lmv[i]; o_old[i] = old; o_ref[i] = ref; o_kl[i] = kl; o_gkl[i] = gkl; o_oc[i] = oc;
+      o_tot[i] = gkl + oc;
     }
-    return;
+    if (has_ref && a.ref_in_place) *(f32x4_any*)(rf + t) = o_ref;
+    *(f32x4_any*)(a.lm_out + b * L + t) = o_lm;
+    *(f32x4_any*)(a.old_out + b * L + t) = o_old;
+    *(f32x4_any*)(a.kl_out + b * L + t) = o_kl;
+    if (a.gkl_out) *(f32x4_any*)(a.gkl_out + b * L + t) = o_gkl;
+    if (a.outcome_out) *(f32x4_any*)(a.outcome_out + b * L + t) = o_oc;
+    *(f32x4_any*)(a.tot_out + b * L + t) = o_tot;
   }
-  for (int64_t t = threadIdx.x; t < L; t += blockDim.x) {
+  const int64_t t = L4 + threadIdx.x;
+  if (t < L) {
     const int64_t tn = t + 1 < L ? t + 1 : 0;
     const float lm = lmk[tn] ? 1.f : 0.f;
     float old, ref, kl, gkl, oc;
-    adv_prep_token(a, lm, a.roll_logp ? lp[tn] : lp[t], has_ref ? rf[t] : 0.f, has_ref, t == t_end,
+    adv_prep_token(a, a.estimator, lm, a.roll_logp ? lp[tn] : lp[t], has_ref ? rf[t] : 0.f, has_ref, t == t_end,
                    t == t_out, score, neg_ctl, old, ref, kl, gkl, oc);
     if (has_ref && a.ref_in_place) rf[t] = ref;
     a.lm_out[b * L + t] = lm;
@@ -1691,6 +1694,214 @@ __global__ __launch_bounds__(NORM_THREADS) void adv_prep_kernel(PrepArgs a) {
     if (a.gkl_out) a.gkl_out[b * L + t] = gkl;
     if (a.outcome_out) a.outcome_out[b * L + t] = oc;
     a.tot_out[b * L + t] = gkl + oc;
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// The whole of token-level advantages in front of their normalisation in one launch: a row's reward score
+// (reward_score_groups_kernel's), adv_prep_kernel and gae_owned_kernel with the row sums, a block per row walking its
+// tiles from the right, with the results of the three. Short batches are bound by latency (loads, sums, scan,
+// each behind a barrier): the arrays that need neither the row's length nor its score are written while the
+// last wave works the score out. Large ones are bound by HBM: the shaped rewards and the mask go from the shaping to
+// the scan in registers instead of through memory.
+// Kernels of the three calls and of this one: 64 x 1000 without a critic 17.5 -> 9.4 us; 1024 x 8192 with critic
+// and reference 87 -> 78 us (46 B a slot in place of 54, 4.9 TB/s). Whole calls, without a critic: 64 x 1000 33.1
+// -> 24.9, 1024 x 2048 35.8 -> 28.5, 256 x 8192 42.9 -> 35.5, 328 x 5555 41.8 -> 31.8, 1024 x 8192 100.4 -> 90.4; the rule
+// for the rows' number and length is areal_gae_padded_row_stats'.
+// A thread loads the mask and the log-probs of its 8 tokens from the tokens behind them (the roll), at
+// whatever alignment that is; the one thread of a row whose tokens reach its end picks them one by one. Four
+// tokens are stored before the next four are worked out, and what the block shares is in scalar registers: with
+// all 8 at a time the loop over tiles does not fit the 128 registers of four blocks a CU (58 spilled,
+// 1024 x 8192 105 us).
+// ---------------------------------------------------------------------------------------
+struct AdvGaeArgs {
+  PrepArgs p;                 // reward_score: the scores, with score_mode 0
+  GaeArgs g;                  // rewards and mask unused
+  int score_mode;             // 1: scores are shaped here, 2: and normalised within groups
+  NormArgs score;             // x = raw rewards [bs], groups of rows
+  float bias, scaling, clip;
+};
+
+// Score of row b, by a whole wave. The sums run in reward_score_groups_kernel's order.
+DEVI float row_score(const AdvGaeArgs& a, int64_t b) {
+  if (a.score_mode == 0) return a.p.reward_score[b];
+  const NormArgs& n = a.score;
+  auto shaped = [&](int64_t i) { return shaped_reward(n.x[i], a.bias, a.scaling, a.clip); };
+  const int lane = threadIdx.x & 63;
+  if (a.score_mode == 1 || b >= n.goff[n.G]) return shaped(b);
+  int lo = 0, hi = n.G;  // goff[lo] <= b < goff[hi]
+  while (hi - lo > 1) {
+    const int step = (hi - lo + 63) >> 6, i = lo + lane * step;
+    const uint64_t le = __builtin_amdgcn_ballot_w64(i < hi && n.goff[i] <= b);
+    lo += (__builtin_popcountll(le) - 1) * step;
+    hi = lo + step < hi ? lo + step : hi;
+  }
+  const int64_t g0 = n.goff[lo], g1 = n.goff[lo + 1];
+  double v[10], s1 = 0.0, s4 = 0.0;
+#pragma unroll
+  for (int k = 0; k < 10; ++k) v[k] = 0.0;
+  for (int64_t i = g0 + lane; i < g1; i += 64) {
+    const double x = (double)shaped(i);
+    s1 += x;
+    s4 += x * x;
+  }
+  s1 = wave_sum(s1);
+  s4 = wave_sum(s4);
+  v[0] = v[2] = (double)(g1 - g0);
+  v[1] = v[3] = s1;
+  v[4] = s4;
+  return norm_one(norm_params(n, lo, v), shaped(b), 1.f, false);
+}
+
+
+// Inputs of a thread's 8 tokens from t0 of a row on: rolled mask bytes and log-probs, reference, values. END: they
+// may reach the end of the row.
+struct PrepItems {
+  u32x2 m;
+  float lp[GAE_ITEMS], rf[GAE_ITEMS], v[GAE_ITEMS];
+};
+template <bool END>
+DEVI void prep_load(const AdvGaeArgs& a, int64_t row, int t0, PrepItems& x) {
+  const int L = (int)a.p.L, roll = a.p.roll_logp ? 1 : 0;
+  const uint8_t* const lm = a.p.loss_mask + row;
+  const float *const lp = a.p.logp + row, *const rf = a.p.ref_logp != nullptr ? a.p.ref_logp + row : nullptr,
+              *const v = a.g.values != nullptr ? a.g.values + row : nullptr;
+#pragma unroll
+  for (int i = 0; i < GAE_ITEMS; ++i) x.lp[i] = x.rf[i] = x.v[i] = 0.f;
+  x.m = u32x2{0u, 0u};
+  if (END && t0 >= L) return;
+  if (!END || t0 + GAE_ITEMS < L) {
+    x.m = *(const u32x2_any*)(lm + t0 + 1);
+#pragma unroll
+    for (int q = 0; q < GAE_ITEMS; q += 4) {
+      const f32x4 w = *(const f32x4_any*)(lp + t0 + q + roll);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x.lp[q + e] = w[e];
+    }
+    if (rf != nullptr) {
+#pragma unroll
+      for (int q = 0; q < GAE_ITEMS; q += 4) {
+        const f32x4 w = *(const f32x4_any*)(rf + t0 + q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.rf[q + e] = w[e];
+      }
+    }
+    if (v != nullptr) {
+#pragma unroll
+      for (int q = 0; q < GAE_ITEMS; q += 4) {
+        const f32x4 w = *(const f32x4_any*)(v + t0 + q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.v[q + e] = w[e];
+      }
+    }
+    return;
+  }
+  // the end of the row: its last token's neighbour is its first
+#pragma unroll
+  for (int i = 0; i < GAE_ITEMS; ++i) {
+    const int t = t0 + i, tn = t + 1 < L ? t + 1 : 0;
+    if (t >= L) break;
+    x.m[i >> 2] |= (uint32_t)lm[tn] << (8 * (i & 3));
+    x.lp[i] = lp[roll ? tn : t];
+    if (rf != nullptr) x.rf[i] = rf[t];
+    if (v != nullptr) x.v[i] = v[t];
+  }
+}
+
+template <int EST, bool ONE_TILE>
+__global__ __launch_bounds__(GAE_THREADS, 4) void adv_gae_kernel(AdvGaeArgs a) {
+  __shared__ MapF smem[GAE_THREADS / 64];
+  __shared__ MapF all[GAE_THREADS];
+  __shared__ double s_rs[4 * 5];
+  __shared__ float s_score;
+  const PrepArgs& p = a.p;
+  const int tid = threadIdx.x, L = (int)p.L;
+  const int64_t b = blockIdx.x, row = b * L;
+  int tile = ONE_TILE ? 0 : (L - 1) / GAE_TILE;
+  int t0 = tile * GAE_TILE + tid * GAE_ITEMS;
+  PrepItems x;
+  prep_load<true>(a, row, t0, x);
+  int cnt = 0;
+  const uint8_t* am = p.attn_mask + row;
+  for (int t = tid * 8; t + 8 <= L; t += GAE_TILE) {
+    const u32x2 w = *(const u32x2_any*)(am + t);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) cnt += ((w[k >> 2] >> (8 * (k & 3))) & 0xffu) ? 1 : 0;
+  }
+  if (tid < (L & 7)) cnt += am[(L & ~7) + tid] ? 1 : 0;
+  if (tid >= GAE_THREADS - 64) {
+    const float sc = row_score(a, b);
+    if (tid == GAE_THREADS - 1) s_score = sc;
+  }
+  const float neg_ctl = -p.kl_ctl;
+  const bool has_ref = p.ref_logp != nullptr;
+  GaeArgs g = a.g;  // the row alone
+  g.adv += row;
+  g.ret += row;
+  double A0 = 0.0, nv0 = 0.0, rs[5] = {0.0};
+  int t_zero = 0, t_out = 0, no_eos = 0;
+  float score = 0.f;
+  for (bool first = true;; first = false) {
+    float rw[GAE_ITEMS], ms[GAE_ITEMS], oa[GAE_ITEMS];  // rw: first the KL rewards
+    auto store4 = [&](float* to, int q, const f32x4& w) {
+      if (t0 + q + 4 <= L) {
+        *(f32x4_any*)(to + row + t0 + q) = w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+          if (t0 + q + e < L) to[row + t0 + q + e] = w[e];
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < GAE_ITEMS; q += 4) {
+      f32x4 o_lm, o_old, o_ref, o_kl;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = q + e;
+        const float lm = (x.m[i >> 2] >> (8 * (i & 3))) & 0xffu ? 1.f : 0.f;
+        float old, ref, kl, gkl, oc;
+        adv_prep_token(p, EST, lm, x.lp[i], x.rf[i], has_ref, false, false, 0.f, neg_ctl, old, ref, kl, gkl, oc);
+        o_lm[e] = lm; o_old[e] = old; o_ref[e] = ref; o_kl[e] = kl;
+        ms[i] = lm;
+        rw[i] = kl;
+      }
+      if (has_ref && p.ref_in_place) store4(p.ref_logp, q, o_ref);
+      store4(p.lm_out, q, o_lm);
+      store4(p.old_out, q, o_old);
+      store4(p.kl_out, q, o_kl);
+    }
+    if (first) {  // (in scalar registers from here on)
+      const int seqlen = __builtin_amdgcn_readfirstlane((int)block_sum_d((double)cnt, s_rs));
+      no_eos = seqlen == L ? 1 : 0;
+      if (tid == 0) { p.seqlens_out[b] = seqlen; p.no_eos_out[b] = (uint8_t)no_eos; }
+      t_zero = seqlen > 0 ? seqlen - 1 : L - 1;
+      t_out = seqlen > 2 ? seqlen - 2 : 0;
+      const float sc = s_score;
+      score = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, sc)));
+      if (p.mask_no_eos_with_zero && no_eos) score = 0.f;
+    }
+#pragma unroll
+    for (int q = 0; q < GAE_ITEMS; q += 4) {
+      f32x4 o_tot;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = t0 + q + e;
+        const float gkl = t == t_zero ? 0.f : rw[q + e], oc = t == t_out ? score : 0.f;
+        o_tot[e] = gkl + oc;
+        rw[q + e] = o_tot[e];
+      }
+      store4(p.tot_out, q, o_tot);
+    }
+    gae_one_tile<true, GAE_LAYOUT_ONE_ROW, false>(g, tile, 0, L, 0, 1, nullptr, A0, nv0, rs, smem, all, rw, x.v, ms, oa,
+                                                  no_eos);
+    if (ONE_TILE || --tile < 0) break;
+    t0 -= GAE_TILE;
+    prep_load<false>(a, row, t0, x);
+  }
+  block_sum_n<5>(rs, s_rs);
+  if (tid == 0) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) a.g.row_stats[(int64_t)k * a.g.n_seqs + b] = rs[k];
   }
 }
 
@@ -1978,6 +2189,17 @@ void launch_gae_owned(const GaeArgs& g, int64_t grid, hipStream_t stream) {
   }
 }
 
+// Whether the row sums ride in the scan of padded rows.
+bool row_sums_fit(int64_t n_seqs, int64_t uniform_len) {
+  if (uniform_len > 64 * (int64_t)GAE_TILE || n_seqs > (1 << 30)) return false;
+  // A block per row: rows shorter than a tile leave lanes idle. While all blocks are resident (4 a CU) that
+  // is cheaper than a launch of its own for the sums (all kernels of an advantage computation, rows x
+  // slots: 64 x 1000 21.4 against 24.4 us, 1024 x 1000 33.4 against 35.4, 1024 x 64 20.8 against 21.3), with
+  // more rows it is not (2048 x 1536 54.9 against 52.7, 4096 x 64 44.9 against 25.0, 16384 x 256 142 against
+  // 63). Rows of nearly a tile fill their block whatever their number (2048 x 2047 66.0 against 69.6).
+  return uniform_len >= GAE_TILE - GAE_TILE / 8 || n_seqs <= 1024;
+}
+
 }  // namespace
 
 extern "C" {
@@ -2059,13 +2281,7 @@ int areal_gae_padded_row_stats(const float* rewards, const float* values, const 
   if (n_seqs < 0 || uniform_len < 0) return AREAL_ERR_BAD_ARG;
   if (n_seqs == 0 || uniform_len == 0) return AREAL_OK;
   if (!rewards || !loss_mask || !advantages || !returns || !row_stats) return AREAL_ERR_BAD_ARG;
-  if (uniform_len > 64 * (int64_t)GAE_TILE || n_seqs > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
-  // A block per row: rows shorter than a tile leave lanes idle. While all blocks are resident (4 a CU) that
-  // is cheaper than a launch of its own for the sums (all kernels of an advantage computation, rows x
-  // slots: 64 x 1000 21.4 against 24.4 us, 1024 x 1000 33.4 against 35.4, 1024 x 64 20.8 against 21.3), with
-  // more rows it is not (2048 x 1536 54.9 against 52.7, 4096 x 64 44.9 against 25.0, 16384 x 256 142 against
-  // 63). Rows of nearly a tile fill their block whatever their number (2048 x 2047 66.0 against 69.6).
-  if (uniform_len < GAE_TILE - GAE_TILE / 8 && n_seqs > 1024) return AREAL_ERR_UNSUPPORTED;
+  if (!row_sums_fit(n_seqs, uniform_len)) return AREAL_ERR_UNSUPPORTED;
   GaeArgs g{rewards, values, loss_mask, nullptr, no_eos, lambda_seq, n_seqs * uniform_len, (int)n_seqs,
             uniform_len, discount, gae_lambda, advantages, returns, 1, row_stats};
   launch_gae_owned<true>(g, n_seqs, stream);
@@ -2434,12 +2650,57 @@ int areal_advantage_prep(const uint8_t* loss_mask, const uint8_t* attn_mask, con
   PrepArgs a{loss_mask, attn_mask, logp, ref_logp, reward_score, L, roll_logp, estimator,
              apply_clamp, mask_no_eos_with_zero, ref_in_place, kl_ctl, lm_out, old_out, kl_out,
              gkl_out, outcome_out, tot_out, seqlens_out, no_eos_out};
-  auto al16 = [](const void* q) { return q == nullptr || ((uintptr_t)q & 15) == 0; };
-  const bool vec = L % 16 == 0 && al16(loss_mask) && al16(attn_mask) && al16(logp) && al16(ref_logp) &&
-                   al16(lm_out) && al16(old_out) && al16(kl_out) && al16(gkl_out) && al16(outcome_out) &&
-                   al16(tot_out);
-  if (vec) hipLaunchKernelGGL(adv_prep_kernel<true>, dim3((unsigned)bs), dim3(NORM_THREADS), 0, stream, a);
-  else hipLaunchKernelGGL(adv_prep_kernel<false>, dim3((unsigned)bs), dim3(NORM_THREADS), 0, stream, a);
+  hipLaunchKernelGGL(adv_prep_kernel, dim3((unsigned)bs), dim3(NORM_THREADS), 0, stream, a);
+  AREAL_CHECK_LAUNCH();
+  return AREAL_OK;
+}
+
+// Reward scores, areal_advantage_prep and areal_gae_padded_row_stats of a padded [bs, L] batch in one launch
+// (adv_gae_kernel), with their results. score_mode 0: rewards are the scores; 1: they are shaped first;
+// 2: and normalised within groups of rows (group_offsets / group_rows / n_groups / tail_group / levels as
+// areal_reward_scores, no level the batch). AREAL_ERR_UNSUPPORTED for the layouts that
+// areal_gae_padded_row_stats does not take either: make the three calls.
+int areal_advantages_row_stats(const float* rewards, int score_mode, float bias, float scaling, float clip,
+                               const int64_t* group_offsets, const int64_t* group_rows, int64_t n_groups, int tail_group,
+                               int mean_level, int std_level, int unbiased, double eps, const uint8_t* loss_mask,
+                               const uint8_t* attn_mask, const float* logp, float* ref_logp, const float* values,
+                               int64_t bs, int64_t L, int roll_logp, int estimator, int apply_clamp,
+                               int mask_no_eos_with_zero, int ref_in_place, float kl_ctl, float discount,
+                               float gae_lambda, float* lm_out, float* old_out, float* kl_out, float* tot_out,
+                               int64_t* seqlens_out, uint8_t* no_eos_out, float* advantages, float* returns,
+                               double* row_stats, hipStream_t stream) {
+  if (bs < 0 || L < 0 || estimator < 1 || estimator > 3 || score_mode < 0 || score_mode > 2) return AREAL_ERR_BAD_ARG;
+  if (bs == 0) return AREAL_OK;
+  if (L == 0) return AREAL_ERR_BAD_ARG;
+  if (!rewards || !loss_mask || !attn_mask || !logp || !lm_out || !old_out || !kl_out || !tot_out || !seqlens_out ||
+      !no_eos_out || !advantages || !returns || !row_stats)
+    return AREAL_ERR_BAD_ARG;
+  if (score_mode == 2 && (!group_offsets || !group_rows || n_groups <= 0)) return AREAL_ERR_BAD_ARG;
+  if (score_mode == 2 && (mean_level < 0 || mean_level > 2 || std_level < 0 || std_level > 2)) return AREAL_ERR_BAD_ARG;
+  if (score_mode == 2 && (mean_level == LEVEL_BATCH || std_level == LEVEL_BATCH)) return AREAL_ERR_UNSUPPORTED;
+  if (!row_sums_fit(bs, L)) return AREAL_ERR_UNSUPPORTED;
+  // with the log-probs rolled a thread reads its neighbour's token: not in place
+  if (roll_logp && logp == old_out) return AREAL_ERR_BAD_ARG;
+  AdvGaeArgs a{};
+  a.p = PrepArgs{loss_mask, attn_mask, logp, ref_logp, rewards, L, roll_logp, estimator, apply_clamp,
+                 mask_no_eos_with_zero, ref_in_place, kl_ctl, lm_out, old_out, kl_out, nullptr, nullptr, tot_out,
+                 seqlens_out, no_eos_out};
+  a.g = GaeArgs{nullptr, values, nullptr, nullptr, nullptr, nullptr, bs * L, (int)bs, L, discount, gae_lambda, advantages,
+                returns, 1, row_stats};
+  a.score_mode = score_mode;
+  a.bias = bias; a.scaling = scaling; a.clip = clip;
+  a.score.x = rewards; a.score.n = bs; a.score.goff = group_offsets; a.score.grows = group_rows;
+  a.score.G = (int)n_groups; a.score.tail_group = tail_group; a.score.mean_level = mean_level;
+  a.score.std_level = std_level; a.score.unbiased = unbiased; a.score.eps = eps;
+  const dim3 gr((unsigned)bs), bl(GAE_THREADS);
+  auto launch = [&](auto one_tile) {
+    constexpr bool ONE = decltype(one_tile)::value;
+    if (estimator == 1) hipLaunchKernelGGL((adv_gae_kernel<1, ONE>), gr, bl, 0, stream, a);
+    else if (estimator == 2) hipLaunchKernelGGL((adv_gae_kernel<2, ONE>), gr, bl, 0, stream, a);
+    else hipLaunchKernelGGL((adv_gae_kernel<3, ONE>), gr, bl, 0, stream, a);
+  };
+  if (L <= GAE_TILE) launch(std::true_type{});
+  else launch(std::false_type{});
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }

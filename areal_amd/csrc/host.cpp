@@ -855,13 +855,21 @@ Tensor bytes_of(const Tensor& t, int64_t bs, int64_t L) {  // a mask as [bs, L] 
 }
 bool in_place_ok(const Tensor& t) { return t.scalar_type() == at::kFloat && t.is_contiguous() && !t.requires_grad(); }
 
+Tensor f32(const Tensor& t) {
+  if (!t.defined()) return t;
+  return (t.scalar_type() == at::kFloat ? t : t.to(at::kFloat)).contiguous();
+}
+
 // Reward scores and their normalisation, then areal_advantage_prep, over bs rows. `score`: the scores themselves when
 // `scored`, else the raw rewards. Returns (loss mask, old log-probs, kl rewards, total rewards, kl rewards
-// for GAE, outcome rewards (both turn mode only), no-eos mask).
+// for GAE, outcome rewards (both turn mode only), no-eos mask, and with `gae` = (values, discount, lambda) where one
+// launch does it all: advantages, returns and their row sums).
+using GaeOptions = std::tuple<OptTensor, double, double>;
 py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double scaling, double clip,
                          const std::optional<NormTables>& norm, const Tensor& loss_mask, const Tensor& attention_mask,
                          const Tensor& logp_src, const OptTensor& ref_logp, bool recompute, int estimator, bool clamp,
-                         bool no_eos_zero, double kl_ctl, bool turn_mode, int64_t bs) {
+                         bool no_eos_zero, double kl_ctl, bool turn_mode, int64_t bs,
+                         const std::optional<GaeOptions>& gae) {
   const int64_t L = logp_src.size(-1);
   const Tensor ref_arg = or_undefined(ref_logp);
   require_numel(bs, {{"rewards", &score}});
@@ -872,21 +880,6 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
   const areal_stream_t stream = stream_of(logp_src);
   Tensor sc = score.scalar_type() == at::kFloat ? score : score.to(at::kFloat);
   sc = sc.contiguous();
-  if (!scored) {
-    const Tensor shaped = empty_f32(sc, bs);
-    if (norm.has_value()) {
-      const auto& [off, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = *norm;
-      check(areal_reward_scores(ptr<float>(sc), bs, (float)bias, (float)scaling, (float)clip, ptr<int64_t>(off),
-                                ptr<int64_t>(rows), rows.numel(), tail, mean_level, std_level, unbiased, eps,
-                                ptr<float>(shaped), stream),
-            "areal_reward_scores");
-    } else {
-      check(areal_reward_scores(ptr<float>(sc), bs, (float)bias, (float)scaling, (float)clip, nullptr, nullptr, 0, -1, 0,
-                                0, 0, 0.0, ptr<float>(shaped), stream),
-            "areal_reward_scores");
-    }
-    sc = shaped;
-  }
   Tensor logp = logp_src.requires_grad() ? logp_src.detach() : logp_src;
   const bool src_ok = in_place_ok(logp_src);
   if (logp.dim() != 2) logp = logp.reshape({bs, L});
@@ -897,22 +890,54 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
   if (ref.defined()) ref = ref_in_place ? ref.reshape({bs, L}) : ref.detach().to(at::kFloat).contiguous().reshape({bs, L});
   const Tensor lm = empty(logp, {bs, L}, at::kFloat), kl = empty(logp, {bs, L}, at::kFloat),
                tot = empty(logp, {bs, L}, at::kFloat);
-  const Tensor gkl = turn_mode ? empty(logp, {bs, L}, at::kFloat) : Tensor(),
-               outcome = turn_mode ? empty(logp, {bs, L}, at::kFloat) : Tensor();
   const Tensor seqlens = empty(logp, {bs}, at::kLong), no_eos = empty(logp, {bs}, at::kBool);
   const Tensor lmb = bytes_of(loss_mask, bs, L), amb = bytes_of(attention_mask, bs, L);
+  auto opt = [](const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); };
+  auto norm_args = [&](auto&& call) {
+    if (!norm.has_value()) return call(nullptr, nullptr, 0, -1, 0, 0, 0, 0.0);
+    const auto& [off, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = *norm;
+    return call(ptr<int64_t>(off), ptr<int64_t>(rows), rows.numel(), tail, mean_level, std_level, unbiased, eps);
+  };
+  // (a score that is not one per row, or values of another size, are for the calls that look at them)
+  if (gae.has_value() && !turn_mode && bs > 0 && L > 0) {
+    const Tensor v = f32(or_undefined(std::get<0>(*gae)));
+    if (!v.defined() || (v.is_cuda() && v.sizes() == lm.sizes())) {
+      const Tensor adv = at::empty_like(lm), ret = at::empty_like(lm), sums = empty(lm, {5, bs}, at::kDouble);
+      const int rc = norm_args([&](const int64_t* off, const int64_t* rows, int64_t n, int tail, int mean_level,
+                                   int std_level, int unbiased, double eps) {
+        return areal_advantages_row_stats(
+            ptr<float>(sc), scored ? 0 : norm.has_value() ? 2 : 1, (float)bias, (float)scaling, (float)clip, off, rows, n,
+            tail, mean_level, std_level, unbiased, eps, ptr<uint8_t>(lmb), ptr<uint8_t>(amb), ptr<float>(logp),
+            ptr<float>(ref), ptr<float>(v), bs, L, recompute ? 0 : 1, estimator, clamp, no_eos_zero, ref_in_place,
+            (float)kl_ctl, (float)std::get<1>(*gae), (float)std::get<2>(*gae), ptr<float>(lm), ptr<float>(old),
+            ptr<float>(kl), ptr<float>(tot), ptr<int64_t>(seqlens), ptr<uint8_t>(no_eos), ptr<float>(adv),
+            ptr<float>(ret), ptr<double>(sums), stream);
+      });
+      if (rc != AREAL_ERR_UNSUPPORTED) {
+        check(rc, "areal_advantages_row_stats");
+        return py::make_tuple(lm, old.view(logp_src.sizes()), kl, tot, OptTensor(), OptTensor(), no_eos,
+                              py::make_tuple(adv, ret, sums));
+      }
+    }
+  }
+  if (!scored) {
+    const Tensor shaped = empty_f32(sc, bs);
+    check(norm_args([&](const int64_t* off, const int64_t* rows, int64_t n, int tail, int mean_level, int std_level,
+                        int unbiased, double eps) {
+            return areal_reward_scores(ptr<float>(sc), bs, (float)bias, (float)scaling, (float)clip, off, rows, n, tail,
+                                       mean_level, std_level, unbiased, eps, ptr<float>(shaped), stream);
+          }),
+          "areal_reward_scores");
+    sc = shaped;
+  }
+  const Tensor gkl = turn_mode ? empty(logp, {bs, L}, at::kFloat) : Tensor(),
+               outcome = turn_mode ? empty(logp, {bs, L}, at::kFloat) : Tensor();
   check(areal_advantage_prep(ptr<uint8_t>(lmb), ptr<uint8_t>(amb), ptr<float>(logp), ptr<float>(ref), ptr<float>(sc), bs,
                              L, recompute ? 0 : 1, estimator, clamp, no_eos_zero, ref_in_place, (float)kl_ctl,
                              ptr<float>(lm), ptr<float>(old), ptr<float>(kl), ptr<float>(gkl), ptr<float>(outcome),
                              ptr<float>(tot), ptr<int64_t>(seqlens), ptr<uint8_t>(no_eos), stream),
         "areal_advantage_prep");
-  auto opt = [](const Tensor& t) { return t.defined() ? OptTensor(t) : OptTensor(); };
-  return py::make_tuple(lm, old.view(logp_src.sizes()), kl, tot, opt(gkl), opt(outcome), no_eos);
-}
-
-Tensor f32(const Tensor& t) {
-  if (!t.defined()) return t;
-  return (t.scalar_type() == at::kFloat ? t : t.to(at::kFloat)).contiguous();
+  return py::make_tuple(lm, old.view(logp_src.sizes()), kl, tot, opt(gkl), opt(outcome), no_eos, py::none());
 }
 
 // Token-level GAE of padded rows that leaves each row's masked sums: (advantages, returns, sums [5, bs]), or

@@ -644,11 +644,23 @@ def compute_advantages(
     if getattr(kl_estimator, "kl_estimator", None) not in ("k1", "k2", "k3"):
         raise TypeError("kl_estimator must be a KLEstimator (k1, k2 or k3)")
     est = {"k1": 1, "k2": 2, "k3": 3}[kl_estimator.kl_estimator]
-    loss_mask, old_logp, kl_rewards, tot_rewards, gae_kl_rewards, gae_outcome_rewards, seq_no_eos_mask = (
+    values = data.get("values")  # none: all zero
+    # With a fixed lambda and a normalisation that needs one statistics pass, token-level GAE and each row's
+    # masked sums ride in the same launch, and so does the scores' part of it.
+    one_pass = isinstance(adv_norm, Normalization) and adv_norm.needs_one_statistics_pass()
+    gae_options = None
+    if (
+        one_pass and not turn_mode and gae_lambda_fn is None and logp_src.ndim == 2
+        and isinstance(gae_lambda, (int, float)) and not isinstance(gae_lambda, bool) and math.isfinite(gae_lambda)
+    ):
+        gae_options = (values, discount, float(gae_lambda))
+    (
+        loss_mask, old_logp, kl_rewards, tot_rewards, gae_kl_rewards, gae_outcome_rewards, seq_no_eos_mask, scanned,
+    ) = (
         _lib.host().advantage_prep(
             score, scored, reward_bias, reward_scaling, reward_clip, score_tables, data["loss_mask"],
             data["attention_mask"], logp_src, data.get("ref_logp"), recompute, est, bool(kl_estimator.apply_clamp),
-            bool(mask_no_eos_with_zero), kl_ctl, turn_mode, bs,
+            bool(mask_no_eos_with_zero), kl_ctl, turn_mode, bs, gae_options,
         )
     )
     if recompute:
@@ -660,7 +672,6 @@ def compute_advantages(
     # turn mode keeps the token KL as a local actor penalty instead of summing it into turns
     rewards = gae_outcome_rewards if turn_mode else tot_rewards
 
-    values = data.get("values")  # none: all zero
     if gae_lambda_fn is None and isinstance(gae_lambda, (str, bool)):
         gae_lambda_fn, _ = resolve_gae_lambda_fn(gae_lambda)
     if gae_lambda_fn is not None:
@@ -683,8 +694,10 @@ def compute_advantages(
         # sums each row's advantages under the mask while it writes them, and the normalisation
         # is its apply pass alone: two launches for the two stages (same results).
         fused = None
-        if isinstance(adv_norm, Normalization) and adv_norm.needs_one_statistics_pass() and rewards.ndim == 2:
-            fused = _token_level_gae_with_row_stats(rewards, values, loss_mask, seq_no_eos_mask, discount, gae_lambda)
+        if one_pass and rewards.ndim == 2:
+            fused = _token_level_gae_with_row_stats(
+                rewards, values, loss_mask, seq_no_eos_mask, discount, gae_lambda, scanned
+            )
         if fused is not None:
             advantages, returns, row_stats, mask_f32 = fused
             normed = adv_norm.from_row_stats(advantages, mask_f32, row_stats, group_sizes=group_sizes)

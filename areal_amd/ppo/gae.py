@@ -69,10 +69,15 @@ def _compute_token_level_gae(
     )
 
 
-def _token_level_gae_with_row_stats(rewards, values, loss_mask, seq_no_eos_mask, discount, gae_lambda):
+def _token_level_gae_with_row_stats(
+    rewards, values, loss_mask, seq_no_eos_mask, discount, gae_lambda, scanned=None
+):
     """``_compute_token_level_gae`` that also returns, per row, the masked sums of the advantages
     which ``Normalization.from_row_stats`` needs (``[5, bs]`` fp64), or ``None`` when the layout
-    does not allow it (more than 1024 rows of fewer than 1792 slots). ``values=None``: all zero."""
+    does not allow it (more than 1024 rows of fewer than 1792 slots). ``values=None``: all zero.
+    ``scanned``: advantages, returns and sums, if the launch that shaped the rewards left them."""
+    if scanned is not None:
+        return (*scanned, loss_mask)
     bs, max_seqlen = rewards.shape
     if bs == 0 or max_seqlen == 0:
         return None

@@ -514,6 +514,22 @@ int areal_advantage_prep(const uint8_t* loss_mask, const uint8_t* attn_mask, con
                          float* kl_out, float* gkl_out, float* outcome_out, float* tot_out,
                          int64_t* seqlens_out, uint8_t* no_eos_out, areal_stream_t stream);
 
+/* Reward scores (areal_reward_scores), areal_advantage_prep and areal_gae_padded_row_stats of a padded
+ * [bs, L] batch in one launch, with their results. score_mode 0: rewards are the scores; 1: they are
+ * shaped first; 2: shaped and normalised within groups of rows (no level may be the batch).
+ * AREAL_ERR_UNSUPPORTED for row counts and lengths that areal_gae_padded_row_stats does not take. */
+int areal_advantages_row_stats(const float* rewards, int score_mode, float bias, float scaling, float clip,
+                               const int64_t* group_offsets, const int64_t* group_rows,
+                               int64_t n_groups, int tail_group, int mean_level, int std_level,
+                               int unbiased, double eps, const uint8_t* loss_mask,
+                               const uint8_t* attn_mask, const float* logp, float* ref_logp,
+                               const float* values, int64_t bs, int64_t L, int roll_logp, int estimator,
+                               int apply_clamp, int mask_no_eos_with_zero, int ref_in_place, float kl_ctl,
+                               float discount, float gae_lambda, float* lm_out, float* old_out,
+                               float* kl_out, float* tot_out, int64_t* seqlens_out, uint8_t* no_eos_out,
+                               float* advantages, float* returns, double* row_stats,
+                               areal_stream_t stream);
+
 /* masked_normalization with dim = the trailing dimensions (areal/utils/functional/functional.py:16-53,
  * the `dim` argument): x, mask (NULL allowed) and out are [rows, cols]; every row is whitened with
  * its own masked mean and variance. */
