@@ -119,6 +119,11 @@ SIGNATURES: dict[str, tuple] = {
         [P, P, P, P, P, P, I64, I64, F, F, P, P, I64, I, I, I, I, D, P, P, P, P, SZ, P],
     ),
     "areal_reward_scores": (I, [P, I64, F, F, F, P, P, I64, I, I, I, I, D, P, P]),
+    "areal_advantages_row_stats": (
+        I,
+        [P, I, F, F, F, P, P, I64, I, I, I, I, D, P, P, P, P, P, I64, I64, I, I, I, I, I, F, F, F, P, P, P, P, P, P, P, P,
+         P, P],
+    ),
     "areal_turn_gae_ex": (I, [P, P, P, P, I, P, P, P, I64, I64, F, F, P, P, P, P, SZ, P]),
     "areal_gae_lambda_context": (I, [P, P, I64, I64, P, P, P, P]),
     "areal_group_norm_workspace_bytes": (SZ, [I64, I64]),
