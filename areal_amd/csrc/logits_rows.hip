@@ -1,4 +1,6 @@
-// Logits-in label log-probabilities and entropy (forward and backward), one workgroup per row.
+// Logits-in label log-probabilities and entropy: the forward one workgroup per row, the backward one per 8 KiB of a
+// row. Bound by HBM. Rows of any start and length are read in 16-byte steps: with 2-byte accesses for vocabularies
+// that are no multiple of 8, 4000 x 50257 bf16 took 232 us forward and 302 backward, now 71 and 132.
 //
 // Follows areal/utils/functional/vocab_parallel.py:16-30: log_softmax(logits.float() / T),
 // gather at the label, entropy = -sum p log p; row chunking (:42-82) does not change values.
@@ -6,36 +8,37 @@
 // and writes d loss / d logits in the dtype of the logits:
 //     d lp_label / d x_j = (1[j == label] - p_j) / T
 //     d entropy  / d x_j = -p_j (log p_j + entropy) / T
+#include <algorithm>
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace {
 
-constexpr int ROW_THREADS = 256;
 constexpr float LOG2E_F = 1.4426950408889634f;
 constexpr float LN2_F = 0.6931471805599453f;
 
-// Vector loads and stores carry the non-temporal hint: every logit is read once per kernel (and every
+// Vector accesses carry the non-temporal hint: every logit is read once per kernel (and every
 // dlogit written once), and a plain read of a [4096, 151936] bf16 array in this access pattern
-// measures 6.15 TB/s without the hint, 7.04 TB/s with it.
+// measures 6.15 TB/s without the hint, 7.04 TB/s with it. `Vec` loads from any element (gfx950 runs
+// with unaligned access enabled: still one 16-byte instruction); stores are aligned by their caller.
 template <typename T> struct Elem;
 template <> struct Elem<float> {
+  typedef f32x4 Vec __attribute__((aligned(4)));
   static constexpr int VEC = 4;
   static DEVI float load(const float* p) { return *p; }
-  static DEVI void loadv(const float* p, float (&o)[4]) {
-    const f32x4 v = __builtin_nontemporal_load((const f32x4*)p);
-    o[0] = v[0]; o[1] = v[1]; o[2] = v[2]; o[3] = v[3];
-  }
+  static DEVI void widen(const f32x4& v, float* o) { o[0] = v[0]; o[1] = v[1]; o[2] = v[2]; o[3] = v[3]; }
   static DEVI void store(float* p, float v) { *p = v; }
-  static DEVI void storev(float* p, const float (&o)[4]) {
+  static DEVI void storev(float* p, const float* o) {
     f32x4 v = {o[0], o[1], o[2], o[3]};
     __builtin_nontemporal_store(v, (f32x4*)p);
   }
 };
 template <> struct Elem<u16> {  // bf16 bit patterns
+  typedef u32x4 Vec __attribute__((aligned(2)));
   static constexpr int VEC = 8;
   static DEVI float load(const u16* p) { return bf16_bits_to_f32(*p); }
-  static DEVI void loadv(const u16* p, float (&o)[8]) {
-    const u32x4 v = __builtin_nontemporal_load((const u32x4*)p);
+  static DEVI void widen(const u32x4& v, float* o) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       o[2 * i] = __builtin_bit_cast(float, v[i] << 16);
@@ -43,7 +46,7 @@ template <> struct Elem<u16> {  // bf16 bit patterns
     }
   }
   static DEVI void store(u16* p, float v) { *p = f32_to_bf16_bits(v); }
-  static DEVI void storev(u16* p, const float (&o)[8]) {
+  static DEVI void storev(u16* p, const float* o) {
     u32x4 v;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -51,6 +54,44 @@ template <> struct Elem<u16> {  // bf16 bit patterns
     __builtin_nontemporal_store(v, (u32x4*)p);
   }
 };
+
+// U vectors, `step` vectors apart: all loads before the first use.
+template <typename T, int U>
+DEVI void load_group(const T* p, int64_t step, float (&z)[U * Elem<T>::VEC]) {
+  typename Elem<T>::Vec v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    v[u] = __builtin_nontemporal_load((const typename Elem<T>::Vec*)(p + u * step * Elem<T>::VEC));
+#pragma unroll
+  for (int u = 0; u < U; ++u) Elem<T>::widen(v[u], z + u * Elem<T>::VEC);
+}
+
+// A row of V elements at p: `head` elements up to the first 16-byte boundary, `vecs` whole vectors, the rest.
+template <typename T> struct RowSplit {
+  int head, vecs, edge;  // edge: elements in front of and behind the vectors (fewer than two vectors)
+  DEVI RowSplit(const T* p, int V) {
+    const int h = (int)((16 - ((uintptr_t)p & 15)) & 15) / (int)sizeof(T);
+    head = h < V ? h : V;
+    vecs = (V - head) / Elem<T>::VEC;
+    edge = V - vecs * Elem<T>::VEC;
+  }
+  DEVI int edge_index(int e) const { return e < head ? e : vecs * Elem<T>::VEC + e; }
+};
+
+// Vectors a thread loads before it uses the first. Forward, 4096 x 151936 bf16: 1, 2, 4 and 8 are alike (189 to
+// 191 us: eight blocks of 256 threads a CU keep enough in flight); one block of 1024 per row at 300 rows 31.7 us with
+// one, 28.2 with two or four, 32.3 with eight.
+constexpr int FWD_GROUP = 2;
+// Below this many rows a row gets 1024 threads instead of 256: at 1024 x 151936 bf16 four blocks of 256 a CU
+// take 52.2 us and blocks of 1024 62.1; at 300 rows blocks of 256 took 53.3 us, of 1024 28.2; at 16 28.1 and 16.6.
+constexpr int64_t FWD_FEW_ROWS = 1024;
+// A block of the backward takes one run of BWD_GROUP * BWD_THREADS vectors of a row (8 KiB), so that the blocks in
+// flight read and write one stretch of memory in order: a block per row, 2048 places at once, took 485 us at
+// 4096 x 151936 bf16 (5.1 TB/s), this 401 (6.2 TB/s); one vector per thread 417, three 405, four 399 (and 140.9 us
+// against 131.9 at 4000 x 50257). At 16 rows a block per row left the chip idle: 31.9 us, this 6.9.
+constexpr int BWD_GROUP = 2;
+constexpr int BWD_THREADS = 256;
+constexpr int64_t BWD_MAX_BLOCKS = 1 << 23;  // a launch is limited to 2^32 threads
 
 struct Online {
   float m, s, q;  // max of z2 = x*c2, sum 2^(z2-m), sum (z2-m) 2^(z2-m)
@@ -80,9 +121,10 @@ DEVI void online_add(Online& st, const float (&x)[N], float c2) {
     }
     st.m = vm;
   }
+  const float m = st.m > neg_inf() ? st.m : 0.f;  // nothing but -inf so far: sums of nothing, not of inf - inf
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    const float t = fmaf(x[i], c2, -st.m);
+    const float t = fmaf(x[i], c2, -m);
     const float e = fast_exp2(t);
     st.s += e;
     st.q = fmaf(t, e, st.q);
@@ -106,31 +148,34 @@ DEVI Online block_merge(Online st, Online* smem) {
 }
 
 // lse2[t] = max + log2(sum) in base-2 units of z2 = x * inv_temp * log2(e).
-template <typename T, bool VECTOR>
-__global__ __launch_bounds__(ROW_THREADS) void rows_fwd_kernel(const T* __restrict__ logits,
-                                                               int64_t ld,
-                                                               const int64_t* __restrict__ labels,
-                                                               int V, float inv_temp,
-                                                               float* __restrict__ logprobs,
-                                                               float* __restrict__ entropy,
-                                                               float* __restrict__ lse2_out) {
-  __shared__ Online smem[ROW_THREADS / 64];
+template <typename T, int THREADS>
+__global__ __launch_bounds__(THREADS) void rows_fwd_kernel(const T* __restrict__ logits, int64_t ld,
+                                                           const int64_t* __restrict__ labels, int V,
+                                                           float inv_temp, float* __restrict__ logprobs,
+                                                           float* __restrict__ entropy,
+                                                           float* __restrict__ lse2_out) {
+  __shared__ Online smem[THREADS / 64];
   const int64_t row = blockIdx.x;
   const T* x = logits + row * ld;
   const float c2 = inv_temp * LOG2E_F;
   Online st{neg_inf(), 0.f, 0.f};
-  constexpr int VEC = Elem<T>::VEC;
-  if (VECTOR) {
-    for (int v0 = threadIdx.x * VEC; v0 < V; v0 += ROW_THREADS * VEC) {
-      float z[VEC];
-      Elem<T>::loadv(x + v0, z);
-      online_add(st, z, c2);
-    }
-  } else {
-    for (int v = threadIdx.x; v < V; v += ROW_THREADS) {
-      float z[1] = {Elem<T>::load(x + v)};
-      online_add(st, z, c2);
-    }
+  constexpr int VEC = Elem<T>::VEC, U = FWD_GROUP;
+  const RowSplit<T> rs(x, V);
+  const T* body = x + rs.head;
+  int v = threadIdx.x;
+  for (; v + (U - 1) * THREADS < rs.vecs; v += U * THREADS) {
+    float z[U * VEC];
+    load_group<T, U>(body + (int64_t)v * VEC, THREADS, z);
+    online_add(st, z, c2);
+  }
+  for (; v < rs.vecs; v += THREADS) {
+    float z[VEC];
+    load_group<T, 1>(body + (int64_t)v * VEC, 0, z);
+    online_add(st, z, c2);
+  }
+  if ((int)threadIdx.x < rs.edge) {
+    float z[1] = {Elem<T>::load(x + rs.edge_index(threadIdx.x))};
+    online_add(st, z, c2);
   }
   const Online r = block_merge(st, smem);
   if (threadIdx.x == 0) {
@@ -150,61 +195,71 @@ __global__ __launch_bounds__(ROW_THREADS) void rows_fwd_kernel(const T* __restri
   }
 }
 
-template <typename T, bool VECTOR>
-__global__ __launch_bounds__(ROW_THREADS) void rows_bwd_kernel(
+// Block (row, part) writes part `part` of `parts` equal runs of vectors of the row.
+template <typename T, bool ENT>
+__global__ __launch_bounds__(BWD_THREADS) void rows_bwd_kernel(
     const T* __restrict__ logits, int64_t ld, const int64_t* __restrict__ labels, int V,
     float inv_temp, const float* __restrict__ lse2, const float* __restrict__ entropy,
     const float* __restrict__ grad_lp, const float* __restrict__ grad_ent, T* __restrict__ dlogits,
-    int64_t ldd) {
-  const int64_t row = blockIdx.x;
+    int64_t ldd, unsigned parts, unsigned part_vecs) {
+  const int64_t row = blockIdx.x / parts;
+  const unsigned part = blockIdx.x % parts;
   const T* x = logits + row * ld;
   T* d = dlogits + row * ldd;
   const float c2 = inv_temp * LOG2E_F;
   const float l2 = lse2[row];
   const float glp = (grad_lp ? grad_lp[row] : 0.f) * inv_temp;
-  const float gen = (grad_ent ? grad_ent[row] : 0.f) * inv_temp;
-  const float ent = (grad_ent ? entropy[row] : 0.f);
+  const float gen = ENT ? grad_ent[row] * inv_temp : 0.f;
+  const float ent = ENT ? entropy[row] : 0.f;
   const int64_t lab64 = labels[row];
   const int lab = (lab64 >= 0 && lab64 < V) ? (int)lab64 : -1;
-  constexpr int VEC = Elem<T>::VEC;
-  if (VECTOR) {
-    for (int v0 = threadIdx.x * VEC; v0 < V; v0 += ROW_THREADS * VEC) {
-      float z[VEC];
-      Elem<T>::loadv(x + v0, z);
+  auto gradient = [&](float z, bool label) {
+    const float t = fmaf(z, c2, -l2);
+    const float p = fast_exp2(t);
+    float g = -p * glp;
+    if (label) g += glp;
+    if (ENT) g -= gen * p * (t * LN2_F + ent);
+    return g;
+  };
+  constexpr int VEC = Elem<T>::VEC, U = BWD_GROUP;
+  const RowSplit<T> rs(d, V);
+  // vectors of this part: [v, end)
+  const int begin = (int)(part * part_vecs);
+  const int end = rs.vecs - begin < (int)part_vecs ? rs.vecs : begin + (int)part_vecs;
+  auto group = [&](auto n, int v) {
+    constexpr int N = decltype(n)::value;
+    float z[N * VEC];
+    const int at = rs.head + v * VEC;
+    load_group<T, N>(x + at, BWD_THREADS, z);
 #pragma unroll
-      for (int i = 0; i < VEC; ++i) {
-        const float t = fmaf(z[i], c2, -l2);
-        const float p = fast_exp2(t);
-        float g = -p * glp;
-        if (v0 + i == lab) g += glp;
-        if (grad_ent) g -= gen * p * (t * LN2_F + ent);
-        z[i] = g;
-      }
-      Elem<T>::storev(d + v0, z);
+    for (int u = 0; u < N; ++u) {
+      const int to_label = lab - (at + u * BWD_THREADS * VEC);
+#pragma unroll
+      for (int i = 0; i < VEC; ++i) z[u * VEC + i] = gradient(z[u * VEC + i], to_label == i);
+      Elem<T>::storev(d + at + u * BWD_THREADS * VEC, z + u * VEC);
     }
-  } else {
-    for (int v = threadIdx.x; v < V; v += ROW_THREADS) {
-      const float t = fmaf(Elem<T>::load(x + v), c2, -l2);
-      const float p = fast_exp2(t);
-      float g = -p * glp;
-      if (v == lab) g += glp;
-      if (grad_ent) g -= gen * p * (t * LN2_F + ent);
-      Elem<T>::store(d + v, g);
-    }
+  };
+  int v = begin + threadIdx.x;
+  for (; v + (U - 1) * BWD_THREADS < end; v += U * BWD_THREADS) group(std::integral_constant<int, U>{}, v);
+  for (; v < end; v += BWD_THREADS) group(std::integral_constant<int, 1>{}, v);
+  if (part == 0 && (int)threadIdx.x < rs.edge) {
+    const int at = rs.edge_index(threadIdx.x);
+    Elem<T>::store(d + at, gradient(Elem<T>::load(x + at), at == lab));
   }
 }
 
 template <typename T>
 int launch_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int64_t T_, int64_t V,
                     float inv_temp, float* lp, float* ent, float* lse2, hipStream_t stream) {
-  constexpr int VEC = Elem<T>::VEC;
-  const bool vec = (V % VEC == 0) && (ld % VEC == 0) && (((uintptr_t)logits & 15) == 0);
-  if (vec)
-    hipLaunchKernelGGL((rows_fwd_kernel<T, true>), dim3((unsigned)T_), dim3(ROW_THREADS), 0, stream,
+  auto launch = [&](auto threads) {
+    constexpr int THREADS = decltype(threads)::value;
+    hipLaunchKernelGGL((rows_fwd_kernel<T, THREADS>), dim3((unsigned)T_), dim3(THREADS), 0, stream,
                        (const T*)logits, ld, labels, (int)V, inv_temp, lp, ent, lse2);
+  };
+  if (T_ < FWD_FEW_ROWS)
+    launch(std::integral_constant<int, 1024>{});
   else
-    hipLaunchKernelGGL((rows_fwd_kernel<T, false>), dim3((unsigned)T_), dim3(ROW_THREADS), 0,
-                       stream, (const T*)logits, ld, labels, (int)V, inv_temp, lp, ent, lse2);
+    launch(std::integral_constant<int, 256>{});
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }
@@ -213,17 +268,19 @@ template <typename T>
 int launch_rows_bwd(const void* logits, int64_t ld, const int64_t* labels, int64_t T_, int64_t V,
                     float inv_temp, const float* lse2, const float* ent, const float* glp,
                     const float* gent, void* dlogits, int64_t ldd, hipStream_t stream) {
-  constexpr int VEC = Elem<T>::VEC;
-  const bool vec = (V % VEC == 0) && (ld % VEC == 0) && (ldd % VEC == 0) &&
-                   (((uintptr_t)logits & 15) == 0) && (((uintptr_t)dlogits & 15) == 0);
-  if (vec)
-    hipLaunchKernelGGL((rows_bwd_kernel<T, true>), dim3((unsigned)T_), dim3(ROW_THREADS), 0, stream,
-                       (const T*)logits, ld, labels, (int)V, inv_temp, lse2, ent, glp, gent,
-                       (T*)dlogits, ldd);
+  const int64_t vecs = V / Elem<T>::VEC, per = BWD_GROUP * BWD_THREADS;
+  int64_t parts = std::max<int64_t>(ceil_div_i64(vecs, per), 1);
+  parts = std::min(parts, std::max<int64_t>(BWD_MAX_BLOCKS / T_, 1));
+  const int64_t part_vecs = round_up_i64(ceil_div_i64(vecs, parts), per);
+  auto launch = [&](auto with_entropy) {
+    hipLaunchKernelGGL((rows_bwd_kernel<T, decltype(with_entropy)::value>), dim3((unsigned)(T_ * parts)),
+                       dim3(BWD_THREADS), 0, stream, (const T*)logits, ld, labels, (int)V, inv_temp, lse2, ent, glp,
+                       gent, (T*)dlogits, ldd, (unsigned)parts, (unsigned)part_vecs);
+  };
+  if (gent)
+    launch(std::true_type{});
   else
-    hipLaunchKernelGGL((rows_bwd_kernel<T, false>), dim3((unsigned)T_), dim3(ROW_THREADS), 0,
-                       stream, (const T*)logits, ld, labels, (int)V, inv_temp, lse2, ent, glp, gent,
-                       (T*)dlogits, ldd);
+    launch(std::false_type{});
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }

@@ -1,0 +1,48 @@
+"""Logits-in kernels at rows of any start and length, either side of the rules on row and block counts."""
+
+import pytest
+import torch
+
+from areal_amd.functional import gather_logprobs_entropy
+from oracle import logprob as L
+
+pytestmark = pytest.mark.gpu
+
+
+# 8 elements are a vector of bf16, 4 of fp32; a block of the backward takes 512 vectors; 1024 rows are the
+# forward's line between blocks of 1024 and of 256 threads
+@pytest.mark.parametrize("rows, vocab, pitch", [
+    (3, 1, 1), (5, 7, 7), (5, 8, 11), (4, 15, 15), (3, 2047, 2049), (3, 2049, 2056), (2, 4095, 4097), (2, 4103, 4103),
+    (3, 16391, 16396), (1023, 333, 333), (1024, 333, 333), (1025, 37, 41),
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_ragged_rows(dev, rows, vocab, pitch, dtype):
+    g = torch.Generator().manual_seed(rows * pitch)
+    base = (torch.randn(rows * pitch + 3, generator=g) * 2).to(dtype)
+    y = torch.randint(0, vocab, (rows,), generator=g)
+    y[0], y[-1] = 0, vocab - 1
+    w_lp, w_ent = torch.randn(rows, generator=g), torch.randn(rows, generator=g)
+    for start in (0, 1, 3):  # rows of any start, a pitch wider than the row
+        x = base[start:start + rows * pitch].view(rows, pitch)[:, :vocab]
+        xg = base.to(dev)[start:start + rows * pitch].view(rows, pitch)[:, :vocab].detach().requires_grad_(True)
+        lp, ent = gather_logprobs_entropy(xg, y.to(dev), 0.9)
+        want_lp, want_ent = L.gather_logprobs_entropy(x, y, 0.9)
+        torch.testing.assert_close(lp.cpu(), want_lp, rtol=1e-5, atol=2e-5)
+        torch.testing.assert_close(ent.cpu(), want_ent, rtol=1e-5, atol=2e-5)
+        ((lp * w_lp.to(dev)).sum() + (ent * w_ent.to(dev)).sum()).backward()
+        want = L.logits_backward(x, y, w_lp, w_ent, 0.9)
+        tol = dict(rtol=1e-5, atol=2e-5) if dtype == torch.float32 else dict(rtol=1e-2, atol=1e-4)
+        torch.testing.assert_close(xg.grad.cpu().float(), want, **tol)
+        xg.grad = None
+        (gather_logprobs_entropy(xg, y.to(dev), 0.9)[0] * w_lp.to(dev)).sum().backward()
+        torch.testing.assert_close(xg.grad.cpu().float(), L.logits_backward(x, y, w_lp, None, 0.9), **tol)
+
+
+def test_excluded_vocabulary_keeps_its_logprob(dev):
+    """Logits of -inf (a masked vocabulary) count nothing, also where a thread meets nothing else."""
+    g = torch.Generator().manual_seed(2)
+    x = torch.randn(6, 5003, generator=g)
+    x[:, 100:4000] = float("-inf")
+    y = torch.randint(0, 100, (6,), generator=g)
+    lp, _ = gather_logprobs_entropy(x.to(dev), y.to(dev))
+    torch.testing.assert_close(lp.cpu(), torch.log_softmax(x, -1)[torch.arange(6), y], rtol=1e-5, atol=2e-5)
