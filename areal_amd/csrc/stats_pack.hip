@@ -57,10 +57,10 @@ DEVI int wave_inclusive_sum(int v) {
 }
 
 // cu = exclusive prefix sums of lens, *max_len = max(lens) (one block; 4 entries per thread and
-// round, two barriers per round).
+// round, two barriers per round). host (nullable, host memory): the total and the longest.
 constexpr int SCAN_ITEMS = 4;
 __global__ __launch_bounds__(PK_THREADS) void cu_scan_kernel(const int32_t* lens, int64_t B,
-                                                             int32_t* cu, int32_t* max_len) {
+                                                             int32_t* cu, int32_t* max_len, double* host) {
   __shared__ int sm_sum[PK_THREADS / 64], sm_max[PK_THREADS / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   int carry = 0, mx = 0;
@@ -93,8 +93,15 @@ __global__ __launch_bounds__(PK_THREADS) void cu_scan_kernel(const int32_t* lens
   if (threadIdx.x == 0) {
     for (int i = 1; i < PK_THREADS / 64; ++i) mx = sm_max[i] > mx ? sm_max[i] : mx;
     *max_len = mx;
+    if (host != nullptr) {
+      host[0] = (double)carry;
+      host[1] = (double)mx;
+    }
   }
 }
+
+// One integer of a queued call's results to host memory, for a caller that looks there until it has arrived.
+__global__ void int_to_host_kernel(const int32_t* x, double* host) { host[0] = (double)*x; }
 
 // Copy of n contiguous bytes by the whole block: 16 bytes per thread and access, whatever the
 // two addresses' alignment, four loads in flight per thread before the first store. A run whose
@@ -392,8 +399,8 @@ extern "C" {
 
 // attention_mask [B, S] bytes (nonzero = token) -> lens [B], cu_seqlens [B+1], *max_len, all
 // int32 on the device (data.py:513-517).
-int areal_seqlens_from_mask(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
-                            int32_t* cu_seqlens, int32_t* max_len, hipStream_t stream) {
+int areal_seqlens_from_mask_ex(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
+                               int32_t* cu_seqlens, int32_t* max_len, double* host, hipStream_t stream) {
   if (B < 0 || S < 0) return AREAL_ERR_BAD_ARG;
   if (!cu_seqlens || !max_len || (B > 0 && (!attention_mask || !lens))) return AREAL_ERR_BAD_ARG;
   if (B > (1 << 30) || B * S >= ((int64_t)1 << 31)) return AREAL_ERR_UNSUPPORTED;
@@ -403,7 +410,19 @@ int areal_seqlens_from_mask(const uint8_t* attention_mask, int64_t B, int64_t S,
     AREAL_CHECK_LAUNCH();
   }
   hipLaunchKernelGGL(cu_scan_kernel, dim3(1), dim3(PK_THREADS), 0, stream, lens, B, cu_seqlens,
-                     max_len);
+                     max_len, host);
+  AREAL_CHECK_LAUNCH();
+  return AREAL_OK;
+}
+
+int areal_seqlens_from_mask(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
+                            int32_t* cu_seqlens, int32_t* max_len, hipStream_t stream) {
+  return areal_seqlens_from_mask_ex(attention_mask, B, S, lens, cu_seqlens, max_len, nullptr, stream);
+}
+
+int areal_int_to_host(const int32_t* value, double* host, hipStream_t stream) {
+  if (!value || !host) return AREAL_ERR_BAD_ARG;
+  hipLaunchKernelGGL(int_to_host_kernel, dim3(1), dim3(1), 0, stream, value, host);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }

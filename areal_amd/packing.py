@@ -5,8 +5,9 @@ Same signatures and return structures as the reference's ``areal/utils/data.py``
 reorder -> pad-and-stack composition of ``reorder_and_pad_outputs``
 (``areal/engine/core/train_engine.py:110-144``).  Every per-sequence Python loop of the
 reference (one ``.item()`` or slice assignment per sequence and tensor) is one gather kernel by
-``cu_seqlens`` here; a call performs one device-to-host copy (the total length and the
-longest sequence, which the reference returns as Python ints as well).
+``cu_seqlens`` here; a call waits for the GPU once (for the total length and the
+longest sequence, which the reference returns as Python ints as well). What a call does around its
+kernels is native (``csrc/host.cpp``).
 """
 
 from __future__ import annotations
@@ -21,7 +22,6 @@ import torch
 from areal_amd import _lib
 
 N_TOKENS_PER_PAGE = 256  # data.py:819
-_PACK_MAX_TENSORS = 8  # tensors per areal_pack_padded_multi launch
 
 
 def _elem_bytes(t: torch.Tensor, lead_dims: int) -> int:
@@ -35,6 +35,8 @@ def _fill_bytes(dtype: torch.dtype, value: float):
 
 
 def _fill_pattern(dtype: torch.dtype, value: float) -> bytes:
+    if type(value) in (int, float) and value == 0 and math.copysign(1.0, value) > 0:
+        return bytes(dtype.itemsize)  # zero is all zero bits in every type
     return torch.tensor([value], dtype=dtype).view(torch.uint8).numpy().tobytes()
 
 
@@ -44,46 +46,21 @@ def pack_tensor_dict(data: dict[str, Any]) -> dict[str, Any]:
     assert "attention_mask" in data, "Input data must contain 'attention_mask' key."
     attention_mask = data["attention_mask"]
     assert attention_mask.ndim == 2, "Attention mask must be a 2D tensor."
-    lib = _lib.load()
-    dev = _lib.require_gpu(attention_mask)
+    host = _lib.host()
     bs, seq_len = attention_mask.shape
-    mask_u8 = attention_mask if attention_mask.dtype == torch.bool else attention_mask != 0
-    mask_u8 = mask_u8.contiguous().view(torch.uint8)
-    # one array, so that its last two entries (total and longest) travel to the host in one copy
-    lens = torch.empty(2 * bs + 2, dtype=torch.int32, device=dev)
-    cu_seqlens, max_len = lens[bs : 2 * bs + 1], lens[2 * bs + 1 :]
-    rc = lib.areal_seqlens_from_mask(
-        _lib.ptr(mask_u8), bs, seq_len, _lib.ptr(lens), _lib.ptr(cu_seqlens), _lib.ptr(max_len),
-        _lib.stream_ptr(dev),
-    )
-    _lib.check(rc, "areal_seqlens_from_mask")
-    total_length, max_seqlen = lens[2 * bs :].tolist()  # the one host copy
+    cu_seqlens, total_length, max_seqlen = host.seqlens_of_mask(attention_mask)
     packed_data: dict[str, Any] = {}
-    moved = []  # (contiguous source, packed destination) of the tensors that are packed
+    moved = []  # keys of the tensors that are packed
     for key, value in data.items():
         if key == "attention_mask":
             packed_data["cu_seqlens"] = cu_seqlens
             packed_data["max_seqlen"] = max_seqlen
             continue
+        packed_data[key] = value
         if torch.is_tensor(value) and value.ndim >= 2 and value.shape[0] == bs and value.shape[1] == seq_len:
-            _lib.require_gpu(value)
-            src = value.contiguous()
-            packed = torch.empty((total_length, *value.shape[2:]), dtype=value.dtype, device=value.device)
-            moved.append((src, packed))
-            packed_data[key] = packed
-        else:
-            packed_data[key] = value
-    # eight tensors per launch
-    for i in range(0, len(moved), _PACK_MAX_TENSORS):
-        part = moved[i : i + _PACK_MAX_TENSORS]
-        n = len(part)
-        srcs = (ctypes.c_void_p * n)(*[s.data_ptr() for s, _ in part])
-        dsts = (ctypes.c_void_p * n)(*[d.data_ptr() for _, d in part])
-        sizes = (ctypes.c_int64 * n)(*[_elem_bytes(s, 2) for s, _ in part])
-        rc = lib.areal_pack_padded_multi(
-            srcs, dsts, sizes, n, _lib.ptr(cu_seqlens), bs, seq_len, total_length, _lib.stream_ptr(dev),
-        )
-        _lib.check(rc, "areal_pack_padded_multi")
+            moved.append(key)
+    packed = host.pack_rows([data[key] for key in moved], cu_seqlens, bs, seq_len, total_length)
+    packed_data.update(zip(moved, packed))
     return packed_data
 
 
@@ -135,7 +112,7 @@ def pad_packed_tensor_dict(
             [cu_seqlens[-1], cu_padded[-1], lens_padded.max()]
         ).tolist()
     else:
-        total_length = int(cu_seqlens[-1].item())
+        total_length = _lib.host().last_value(cu_seqlens)
 
     def is_token_tensor(key, value, total):
         if key == "position_ids":
@@ -180,7 +157,8 @@ def pad_packed_tensor_dict(
     new_cu = torch.empty(n_seqs + 2, dtype=torch.int32, device=dev)
     cu_copy = old_cu_seqlens if seq_align_to is None else torch.empty_like(cu_seqlens)
     padded: dict[str, Any] = {}
-    moved = []  # (contiguous source, destination, is it the position ids)
+    moved, sources, patterns = [], [], []  # keys of the tensors that are copied, what is copied, its fill
+    fills: dict[torch.dtype, bytes] = {}
     for key, value in data.items():
         if key == "cu_seqlens":
             padded[key] = new_cu
@@ -192,35 +170,23 @@ def pad_packed_tensor_dict(
             padded[key] = _realign(lib, dev, value, cu_seqlens, n_seqs, _batch_pad(cu_seqlens, pad_to_length),
                                    n_seqs + 1, pad_to_length, 0.0, True, False)
         else:
-            _lib.require_gpu(value)
-            src = (value if key == "position_ids" else value.reshape(total_length)).contiguous()
-            padded[key] = torch.empty((pad_to_length, *src.shape[1:]), dtype=src.dtype, device=src.device)
-            moved.append((src, padded[key], key == "position_ids"))
-    _pad_tensors(lib, dev, moved, pad_value, cu_seqlens, n_seqs, cu_copy, new_cu, total_length, pad_to_length)
+            padded[key] = value
+            moved.append(key)
+            if key == "position_ids":  # they go on from 0
+                sources.append(value)
+                patterns.append(b"")
+                continue
+            sources.append(value.reshape(total_length))
+            if value.dtype not in fills:
+                fills[value.dtype] = _fill_pattern(value.dtype, pad_value)
+            patterns.append(fills[value.dtype])
+    outs = _lib.host().pad_rows(sources, patterns, cu_seqlens, cu_copy, new_cu, total_length, pad_to_length)
+    padded.update(zip(moved, outs))
     return padded, pad_length, old_cu_seqlens, align_to_length
 
 
 def _batch_pad(cu_seqlens, pad_to_length):
     return torch.nn.functional.pad(cu_seqlens, (0, 1), value=pad_to_length)
-
-
-def _pad_tensors(lib, dev, moved, pad_value, cu_seqlens, n_seqs, cu_copy, new_cu, total, total_new):
-    fills = {dtype: _fill_pattern(dtype, pad_value) for dtype in {s.dtype for s, _, ids in moved if not ids}}
-    for i in range(0, max(len(moved), 1), _PACK_MAX_TENSORS):
-        part = moved[i : i + _PACK_MAX_TENSORS]
-        n = len(part)
-        patterns = [b"\0" if ids else fills[s.dtype] for s, _, ids in part]
-        rc = lib.areal_pad_packed_multi(
-            (ctypes.c_void_p * n)(*[s.data_ptr() for s, _, _ in part]),
-            (ctypes.c_void_p * n)(*[d.data_ptr() for _, d, _ in part]),
-            (ctypes.c_int64 * n)(*[_elem_bytes(s, 1) for s, _, _ in part]),
-            b"".join(p.ljust(16, b"\0") for p in patterns),
-            (ctypes.c_int * n)(*[len(p) for p in patterns]),
-            (ctypes.c_int * n)(*[int(ids) for _, _, ids in part]),
-            n, _lib.ptr(cu_seqlens), n_seqs, _lib.ptr(cu_copy), _lib.ptr(new_cu), total, total_new,
-            _lib.stream_ptr(dev),
-        )
-        _lib.check(rc, "areal_pad_packed_multi")
 
 
 def unpack_reorder_pad(
@@ -233,6 +199,10 @@ def unpack_reorder_pad(
     packed sequence ``backward_indices[r]``, zero padded."""
     lib = _lib.load()
     dev = _lib.require_gpu(packed)
+    if type(seqlens) is list and (backward_indices is None or type(backward_indices) is list):
+        out = _lib.host().unpack_rows(packed, seqlens, backward_indices)
+        if out is not None:
+            return out
     n = len(seqlens)
     if backward_indices is not None:
         assert len(set(backward_indices)) == n

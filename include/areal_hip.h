@@ -548,6 +548,11 @@ int areal_masked_norm_rows(const float* x, const float* mask, int64_t rows, int6
  * ------------------------------------------------------------------------------------- */
 int areal_seqlens_from_mask(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
                             int32_t* cu_seqlens, int32_t* max_len, areal_stream_t stream);
+/* The same; host (nullable) is memory of the host that the device can write: {total, longest}. */
+int areal_seqlens_from_mask_ex(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
+                               int32_t* cu_seqlens, int32_t* max_len, double* host, areal_stream_t stream);
+/* *host (memory of the host that the device can write) = *value, in stream order. */
+int areal_int_to_host(const int32_t* value, double* host, areal_stream_t stream);
 int areal_pack_padded(const void* padded, void* packed, const int32_t* cu_seqlens, int64_t B,
                       int64_t S, int64_t elem_bytes, int64_t total, areal_stream_t stream);
 /* The tensors of one batch (pack_tensor_dict's loop over the dict, data.py:519-543) in one launch:

@@ -1,0 +1,73 @@
+"""Native host path of packing: the argument forms either side of its line to the general path."""
+
+import pytest
+import torch
+
+from areal_amd.packing import pack_tensor_dict, pad_packed_tensor_dict, unpack_reorder_pad
+from oracle import packing as P
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("order", [None, [2, 0, 3, 1]])
+@pytest.mark.parametrize("trailing", [(), (3,)])
+def test_unpack_takes_the_same_forms_by_either_path(dev, order, trailing):
+    lens = [3, 0, 300, 17]
+    x = torch.arange(320 * (3 if trailing else 1), device=dev).reshape(320, *trailing)
+    want = torch.zeros(4, 300, *trailing, dtype=x.dtype)
+    starts = [0, 3, 3, 303]
+    for r, s in enumerate(order or range(4)):
+        want[r, : lens[s]] = x[starts[s] : starts[s] + lens[s]].cpu()
+    as_tensors = [torch.tensor(n) for n in lens]
+    for form in (lens, tuple(lens), as_tensors):
+        for o in (order, None if order is None else tuple(order)):
+            assert torch.equal(unpack_reorder_pad(x, form, o).cpu(), want)
+    with pytest.raises(ValueError):
+        unpack_reorder_pad(x, [3, 0, 300, 16], order)
+    with pytest.raises(AssertionError):
+        unpack_reorder_pad(x, lens, [0, 1, 1, 2])
+
+
+def test_unpack_tables_of_several_calls_in_flight(dev):
+    """Each call's offsets are its own, whatever is still queued."""
+    g = torch.Generator().manual_seed(0)
+    calls = []
+    for _ in range(50):
+        lens = torch.randint(0, 40, (33,), generator=g).tolist()
+        calls.append((torch.randn(sum(lens), generator=g), lens, torch.randperm(33, generator=g).tolist()))
+    outs = [unpack_reorder_pad(x.to(dev, non_blocking=True), lens, order) for x, lens, order in calls]
+    for out, (x, lens, order) in zip(outs, calls):
+        rows = x.split(lens)
+        for r, s in enumerate(order):
+            assert torch.equal(out[r, : lens[s]].cpu(), rows[s]) and not out[r, lens[s] :].any()
+
+
+@pytest.mark.parametrize("pad_value", [0.0, -0.0, 0, 1.0, True])
+def test_pad_fills_every_type(dev, pad_value):
+    total, to = 100, 356
+    data = dict(
+        cu_seqlens=torch.tensor([0, 40, total], dtype=torch.int32), max_seqlen=60,
+        f=torch.randn(total), h=torch.randn(total).bfloat16(), d=torch.randn(total).double(),
+        i=torch.arange(total), b=torch.rand(total) > 0.5, u=torch.arange(total).to(torch.uint8),
+        c=torch.randn(total, dtype=torch.complex64), e=torch.randn(total).half(), j=torch.arange(total).int(),
+        position_ids=torch.cat([torch.arange(40), torch.arange(60)]),
+    )
+    got = pad_packed_tensor_dict({k: v.to(dev) if torch.is_tensor(v) else v for k, v in data.items()}, to, pad_value)
+    want = P.pad_packed_tensor_dict(data, to, pad_value)
+    assert got[1] == want[1] and torch.equal(got[2].cpu(), want[2])
+    for k, w in want[0].items():
+        if torch.is_tensor(w):
+            assert got[0][k].dtype == w.dtype and torch.equal(got[0][k].cpu(), w), k
+            if w.is_floating_point():
+                assert torch.equal(got[0][k].cpu().signbit(), w.signbit()), k
+        else:
+            assert got[0][k] == w
+
+
+def test_nothing_to_move(dev):
+    mask = torch.tensor([[1, 1, 0], [1, 0, 0]], device=dev)
+    packed = pack_tensor_dict(dict(attention_mask=mask, name="x"))
+    assert packed["cu_seqlens"].tolist() == [0, 2, 3] and packed["max_seqlen"] == 2 and packed["name"] == "x"
+    padded, pad, old, _ = pad_packed_tensor_dict(packed, 8)
+    assert pad == 5 and old.tolist() == [0, 2, 3] and padded["cu_seqlens"].tolist() == [0, 2, 3, 8]
+    assert padded["max_seqlen"] == 5
