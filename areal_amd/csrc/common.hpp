@@ -59,6 +59,7 @@ DEVI float bf16_bits_to_f32(u16 b) {
 constexpr int DPP_ROW_SHL = 0x100;  // + n (1..15): lane i reads lane i + n of its row
 constexpr int DPP_ROW_SHR = 0x110;  // + n: lane i reads lane i - n of its row
 constexpr int DPP_ROW_ROR = 0x120;  // + n: lane i reads lane (i - n) mod 16 of its row
+constexpr int DPP_WAVE_SHL1 = 0x130;  // lane i reads lane i + 1 of the wave (lane 63 has no source)
 constexpr int DPP_WAVE_SHR1 = 0x138;  // lane i reads lane i - 1 of the wave (lane 0 has no source)
 
 // x of the lane CTRL names; a lane whose source falls outside its row keeps `old`.
@@ -152,6 +153,9 @@ DEVI T wave_inclusive_scan(T v, T identity, Op op) {
 // The value of the lane before (lane 0: the identity).
 template <typename T>
 DEVI T wave_shift_up(T v, T identity) { return dpp_move<DPP_WAVE_SHR1>(identity, v); }
+// v of the next lane, `identity` in lane 63.
+template <typename T>
+DEVI T wave_shift_down(T v, T identity) { return dpp_move<DPP_WAVE_SHL1>(identity, v); }
 
 template <typename T>
 DEVI T wave_sum(T v) { return wave_reduce(v, [](T a, T b) { return a + b; }); }

@@ -349,7 +349,7 @@ __global__ __launch_bounds__(GAE_THREADS) void gae_apply_kernel(GaeArgs g, const
 // block's to write. cu_own[i] = cu[s_first + i] for i in [0, n_own] covers every sequence that
 // holds one of those tokens (cu_own[0] <= t_begin, cu_own[n_own] >= t_end); with uniform rows
 // cu_own is unused. (A0, nv0) is the fp64 state entering the tile from its right and is replaced
-// by the state leaving it on the left. rs: the row sums of GaeArgs::row_stats (STATS only).
+// by the state leaving it on the left.
 // oa receives the advantages of the thread's owned tokens (zero elsewhere).
 // The thread's 8 consecutive tokens from t0 (a multiple of 8) as raw inputs; zeros where `want`
 // is false and beyond the array. Without values (no critic) they are zero too.
@@ -386,19 +386,17 @@ DEVI void gae_owned_items(int64_t t0, int64_t t_begin, int64_t t_end, int& i_lo,
   i_hi = d_hi < GAE_ITEMS ? (d_hi > 0 ? (int)d_hi : 0) : GAE_ITEMS;
 }
 
-// How a tile finds its sequences: in cu_seqlens, as rows of uniform length, or as part of the one
-// row the block walks.
-enum { GAE_LAYOUT_CU = 0, GAE_LAYOUT_ROWS = 1, GAE_LAYOUT_ONE_ROW = 2 };
+// How a tile finds its sequences: in cu_seqlens, or as rows of uniform length.
+enum { GAE_LAYOUT_CU = 0, GAE_LAYOUT_ROWS = 1 };
 
 // (rw, v, ms): the tile's inputs as gae_load_items leaves them (at least the owned tokens).
-// LAMBDAS: a lambda per sequence (GaeArgs::lam_seq). row_boot (one row): GaeArgs::no_eos of the row, if the caller
-// has it at hand (0 / 1).
-template <bool STATS, int LAYOUT, bool LAMBDAS>
+// LAMBDAS: a lambda per sequence (GaeArgs::lam_seq).
+template <int LAYOUT, bool LAMBDAS>
 DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t t_end, int s_first,
                        int n_own, const int32_t* cu_own, double& A0, double& nv0,
-                       double (&rs)[STATS ? 5 : 1], MapF* smem, MapF* all,
+                       MapF* smem, MapF* all,
                        const float (&rw)[GAE_ITEMS], const float (&v)[GAE_ITEMS],
-                       const float (&ms)[GAE_ITEMS], float (&oa)[GAE_ITEMS], int row_boot = -1) {
+                       const float (&ms)[GAE_ITEMS], float (&oa)[GAE_ITEMS]) {
   constexpr bool uniform = LAYOUT != GAE_LAYOUT_CU;
   const int tid = threadIdx.x;
   const int64_t t0 = tile * GAE_TILE + (int64_t)tid * GAE_ITEMS;
@@ -418,11 +416,7 @@ DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t 
     const int64_t tf = t0 + i_lo;
     int sq;
     int e_loc;  // local index one past the last token of sequence sq (clamped)
-    if (LAYOUT == GAE_LAYOUT_ONE_ROW) {
-      sq = 0;
-      const int64_t e = t_end - t0;
-      e_loc = e < 2 * GAE_ITEMS ? (int)e : 2 * GAE_ITEMS;
-    } else if (LAYOUT == GAE_LAYOUT_ROWS) {
+    if (LAYOUT == GAE_LAYOUT_ROWS) {
       sq = (int)(tf / g.uniform_len) - s_first;
       const int64_t e = (int64_t)(sq + s_first + 1) * g.uniform_len - t0;
       e_loc = e < 2 * GAE_ITEMS ? (int)e : 2 * GAE_ITEMS;
@@ -455,8 +449,7 @@ DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t 
         }
         if (i == e_loc - 1) {
           ends |= 1u << i;
-          if (LAYOUT == GAE_LAYOUT_ONE_ROW && row_boot >= 0) boot |= (unsigned)row_boot << i;
-          else if (g.no_eos != nullptr && g.no_eos[s_first + sq] != 0) boot |= 1u << i;
+          if (g.no_eos != nullptr && g.no_eos[s_first + sq] != 0) boot |= 1u << i;
         }
       }
     }
@@ -508,20 +501,6 @@ DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t 
       oa[i] = A;
       orr[i] = oa[i] + v[i];
     }
-    if constexpr (STATS) {
-#pragma unroll
-      for (int i = 0; i < GAE_ITEMS; ++i) {
-        if (!((valid >> i) & 1u) || ms[i] == 0.f) continue;
-        const double x = (double)oa[i];
-        if (ms[i] == 1.f) {  // the usual 0/1 mask: one fp64 multiplication per token
-          rs[0] += 1.0; rs[1] += x; rs[2] += 1.0; rs[3] += x; rs[4] += x * x;
-        } else {
-          const double m = (double)ms[i];
-          const double xm = x * m, mm = m * m;
-          rs[0] += m; rs[1] += xm; rs[2] += mm; rs[3] += xm * m; rs[4] += xm * xm;
-        }
-      }
-    }
     if (valid == (1u << GAE_ITEMS) - 1u) {
 #pragma unroll
       for (int q = 0; q < GAE_ITEMS / 4; ++q) {
@@ -540,6 +519,145 @@ DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t 
   A0 = A1; nv0 = nv1;
 }
 
+// ---------------------------------------------------------------------------------------
+// One row walked by one block (gae_owned_kernel<ONE_ROW>, adv_gae_kernel), tile by tile of the row from the right. A
+// thread has two quads of 4 tokens a tile, WAVE_QUADS tokens apart, so that every access of a wave is 1 KiB in one
+// piece; the maps of the two quads are scanned side by side. With 8 tokens in a row to a thread, each of its 16-byte
+// stores left every other 16 bytes of a line to the next instruction: adv_gae_kernel with inputs new to the caches, at
+// 1024 x 8192 with critic and reference, 81 us, in quads 70; at 1000 x 8191 without a critic 78 and 67.
+// ---------------------------------------------------------------------------------------
+constexpr int QUAD = 4, WAVE_QUADS = 64 * QUAD;  // tokens of one 16-byte access of a thread / of a wave
+constexpr int ROW_QUADS = GAE_ITEMS / QUAD;
+typedef MapF RowMaps[2][GAE_THREADS / 64];  // of the waves, in LDS, alternating from tile to tile
+
+// Row token of the calling thread's first quad.
+DEVI int row_tile_token(int tile) {
+  const int tid = threadIdx.x;
+  return tile * GAE_TILE + (tid >> 6) * ROW_QUADS * WAVE_QUADS + (tid & 63) * QUAD;
+}
+
+// Quad q of the thread's tokens from t0 on of a row of L tokens. STREAM: non-temporal, which pays for some of
+// adv_gae_kernel's arrays (log-probs and KL rewards: 70 -> 66 and 67 -> 60 us in the cases above) and for all of
+// them does not (73 and 75).
+template <bool STREAM>
+DEVI void row_store(float* to, int t0, int L, int q, const f32x4& w) {
+  const int tq = t0 + q * WAVE_QUADS;
+  if (tq + QUAD <= L) {
+    if constexpr (STREAM) __builtin_nontemporal_store(w, (f32x4_any*)(to + tq));
+    else *(f32x4_any*)(to + tq) = w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < QUAD - 1; ++e)
+      if (tq + e < L) to[tq + e] = w[e];
+  }
+}
+
+// The mask of a thread's tokens as bytes (nonzero = 1) or floats. again(): what was worked out from it before is not
+// held in registers beyond this point.
+struct ByteMask {
+  uint32_t (&m)[ROW_QUADS];
+  DEVI float operator()(int i) const { return (m[i / QUAD] >> (8 * (i % QUAD))) & 0xffu ? 1.f : 0.f; }
+  DEVI void again() const {
+#pragma unroll
+    for (int q = 0; q < ROW_QUADS; ++q) asm volatile("" : "+v"(m[q]));
+  }
+};
+struct FloatMask {
+  const float (&m)[GAE_ITEMS];
+  DEVI float operator()(int i) const { return m[i]; }
+  DEVI void again() const {}
+};
+
+// rw, v: rewards and values of the thread's tokens (zero beyond the row). mask_of(i): their mask, zero beyond the row
+// (which makes such a token the identity). boot: whether the row's last value is bootstrapped. (A0, nv0): the fp64 state entering the tile from its
+// right, replaced by the one leaving it on the left. rs: the row's sums of GaeArgs::row_stats (STATS). adv, ret: the row.
+template <bool STATS, bool BINARY, class Mask>
+DEVI void gae_row_tile(float gam, float lam, int tile, int t0, int L, bool boot, float (&rw)[GAE_ITEMS],
+                       float (&v)[GAE_ITEMS], const Mask& mask_of, RowMaps& maps, double& A0, double& nv0,
+                       double (&rs)[STATS ? 5 : 1], float* adv, float* ret) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const float c0 = gam * lam;
+  const int last = L - 1 - t0;
+  const bool wave_has_end = __builtin_amdgcn_ballot_w64(last >= 0 && last < WAVE_QUADS + QUAD) != 0;
+  auto token_map = [&](int i) -> MapF {
+    const float m = mask_of(i);
+    MapF f;
+    f.a11 = fmaf(c0, m, 1.f - m);
+    f.a12 = gam * m;
+    f.a22 = 1.f - m;
+    f.b1 = (rw[i] - v[i]) * m;
+    f.b2 = v[i] * m;
+    if (wave_has_end) {
+      if (last == (i / QUAD) * WAVE_QUADS + i % QUAD) f = MapF{0.f, 0.f, 0.f, 0.f, boot ? v[i] : 0.f};
+    }
+    return f;
+  };
+  MapF incl[ROW_QUADS], total[ROW_QUADS];
+#pragma unroll
+  for (int q = 0; q < ROW_QUADS; ++q) {
+    MapF mine = token_map(QUAD * q + QUAD - 1);
+#pragma unroll
+    for (int e = QUAD - 2; e >= 0; --e) mine = compose(token_map(QUAD * q + e), mine);
+    incl[q] = wave_suffix_scan(mine, total[q]);
+  }
+  MapF* const waves = maps[tile & 1];  // (the other half's readers are past the barrier behind it)
+  if (lane == 0) waves[wave] = compose(total[0], total[1]);
+  __syncthreads();
+  auto advance = [](const MapF& f, double& A, double& nv) {
+    const double A1 = fma((double)f.a11, A, fma((double)f.a12, nv, (double)f.b1));
+    nv = fma((double)f.a22, nv, (double)f.b2);
+    A = A1;
+  };
+  double Aw = A0, nw = nv0;  // the state entering the wave's tokens
+#pragma unroll
+  for (int w = GAE_THREADS / 64 - 1; w >= 0; --w) {
+    if (w == wave) { Aw = A0; nw = nv0; }
+    advance(waves[w], A0, nv0);
+  }
+  // (the token maps are worked out again rather than held: 40 registers)
+#pragma unroll
+  for (int i = 0; i < GAE_ITEMS; ++i) asm volatile("" : "+v"(rw[i]), "+v"(v[i]));
+  mask_of.again();
+#pragma unroll
+  for (int q = ROW_QUADS - 1; q >= 0; --q) {
+    const MapF id = map_identity_t<float>();
+    const MapF excl = {wave_shift_down(incl[q].a11, id.a11), wave_shift_down(incl[q].a12, id.a12),
+                       wave_shift_down(incl[q].a22, id.a22), wave_shift_down(incl[q].b1, id.b1),
+                       wave_shift_down(incl[q].b2, id.b2)};
+    double At = Aw, nt = nw;
+    advance(excl, At, nt);
+    float A = (float)At, nv = (float)nt;
+    f32x4 o_adv, o_ret;
+#pragma unroll
+    for (int e = QUAD - 1; e >= 0; --e) {
+      const int i = QUAD * q + e;
+      const MapF f = token_map(i);
+      const float A2 = fmaf(f.a11, A, fmaf(f.a12, nv, f.b1));
+      nv = fmaf(f.a22, nv, f.b2);
+      A = A2;
+      o_adv[e] = A;
+      o_ret[e] = A + v[i];
+      if constexpr (STATS) {
+        const float m = mask_of(i);
+        if (m != 0.f) {
+          const double x = (double)A;
+          if (BINARY || m == 1.f) {  // the usual 0/1 mask: one fp64 multiplication per token
+            rs[0] += 1.0; rs[1] += x; rs[4] += x * x;
+            if (!BINARY) { rs[2] += 1.0; rs[3] += x; }
+          } else {
+            const double md = (double)m;
+            const double xm = x * md, mm = md * md;
+            rs[0] += md; rs[1] += xm; rs[2] += mm; rs[3] += xm * md; rs[4] += xm * xm;
+          }
+        }
+      }
+    }
+    row_store<false>(adv, t0, L, q, o_adv);
+    row_store<false>(ret, t0, L, q, o_ret);
+    advance(total[q], Aw, nw);
+  }
+}
+
 // (Blocks of 1024 threads, one 8192-token tile per padded row instead of four serial tiles of
 // 2048, measured slower: 46.7 against 30.8 us on [1024, 8192]; one such block fills a CU's
 // registers and the latency of its single pass is not covered by anything.)
@@ -547,6 +665,51 @@ DEVI void gae_one_tile(const GaeArgs& g, int64_t tile, int64_t t_begin, int64_t 
 // ONE_ROW: block = row (GaeArgs::block_per_seq); LAMBDAS: a lambda per row.
 template <bool STATS, bool ONE_ROW, bool LAMBDAS>
 __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
+  if constexpr (ONE_ROW) {
+    __shared__ RowMaps maps;
+    const int b = blockIdx.x, L = (int)g.uniform_len;
+    const int64_t row = (int64_t)b * L;
+    const float lam = LAMBDAS ? g.lam_seq[b] : g.lam;
+    const bool boot = g.no_eos != nullptr && g.no_eos[b] != 0;
+    double A0 = 0.0, nv0 = 0.0;  // state entering the current tile from its right
+    double rs[STATS ? 5 : 1] = {0.0};
+    for (int tile = (L - 1) / GAE_TILE; tile >= 0; --tile) {
+      const int t0 = row_tile_token(tile);
+      float rw[GAE_ITEMS], v[GAE_ITEMS], ms[GAE_ITEMS];
+      auto load = [&](const float* from, float (&x)[GAE_ITEMS]) {
+#pragma unroll
+        for (int i = 0; i < GAE_ITEMS; ++i) x[i] = 0.f;
+        if (from == nullptr) return;
+#pragma unroll
+        for (int q = 0; q < ROW_QUADS; ++q) {
+          const int tq = t0 + q * WAVE_QUADS;
+          if (tq + QUAD <= L) {
+            const f32x4 w = *(const f32x4_any*)(from + row + tq);
+#pragma unroll
+            for (int e = 0; e < QUAD; ++e) x[QUAD * q + e] = w[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < QUAD; ++e)
+              if (tq + e < L) x[QUAD * q + e] = from[row + tq + e];
+          }
+        }
+      };
+      load(g.rewards, rw);
+      load(g.values, v);
+      load(g.mask, ms);
+      gae_row_tile<STATS, false>(g.discount, lam, tile, t0, L, boot, rw, v, FloatMask{ms}, maps, A0, nv0, rs,
+                                 g.adv + row, g.ret + row);
+    }
+    if constexpr (STATS) {
+      __shared__ double s_rs[4 * 5];
+      block_sum_n<5>(rs, s_rs);
+      if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) g.row_stats[(int64_t)k * g.n_seqs + b] = rs[k];
+      }
+    }
+    return;
+  }
   __shared__ MapF smem[GAE_THREADS / 64];
   __shared__ MapF all[GAE_THREADS];
   const int tid = threadIdx.x;
@@ -554,12 +717,9 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
   // ranges keeps neighbouring ranges on one XCD.
   const int64_t per_xcd = (gridDim.x + 7) >> 3;
   const int64_t range = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  // rows of at least a tile: only every (L / TILE)-th range would own a row, so the grid is one
-  // block per row instead, (lo, hi] = the range holding the row's end
-  const int64_t lo = ONE_ROW ? ((int64_t)(blockIdx.x + 1) * g.uniform_len - 1)
-                                     : range * GAE_TILE;
-  if (!ONE_ROW && (range >= per_xcd * 8 || lo >= g.n)) return;
-  const int64_t hi = ONE_ROW ? lo + 1 : (lo + GAE_TILE < g.n ? lo + GAE_TILE : g.n);
+  const int64_t lo = range * GAE_TILE;
+  if (range >= per_xcd * 8 || lo >= g.n) return;
+  const int64_t hi = lo + GAE_TILE < g.n ? lo + GAE_TILE : g.n;
   // owned rows [s_first, s_last]: lo < end(s) <= hi
   const int s_first = (int)(lo / g.uniform_len);
   const int s_last = (int)(hi / g.uniform_len) - 1;
@@ -569,23 +729,14 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
   const int64_t t_end = (int64_t)(s_last + 1) * g.uniform_len;
 
   double A0 = 0.0, nv0 = 0.0;  // state entering the current tile from its right
-  double rs[STATS ? 5 : 1] = {0.0};
   for (int64_t tile = (t_end - 1) / GAE_TILE; tile >= t_begin / GAE_TILE; --tile) {
     const int64_t t0 = tile * GAE_TILE + (int64_t)tid * GAE_ITEMS;
     int i_lo, i_hi;
     gae_owned_items(t0, t_begin, t_end, i_lo, i_hi);
     float rw[GAE_ITEMS], v[GAE_ITEMS], ms[GAE_ITEMS], oa[GAE_ITEMS];
     gae_load_items(g, t0, i_lo < i_hi, rw, v, ms);
-    gae_one_tile<STATS, ONE_ROW ? GAE_LAYOUT_ONE_ROW : GAE_LAYOUT_ROWS, LAMBDAS>(
-        g, tile, t_begin, t_end, s_first, n_own, nullptr, A0, nv0, rs, smem, all, rw, v, ms, oa);
-  }
-  if constexpr (STATS) {  // block = row: uniform for the block
-    __shared__ double s_rs[4 * 5];
-    block_sum_n<5>(rs, s_rs);
-    if (tid == 0) {
-#pragma unroll
-      for (int k = 0; k < 5; ++k) g.row_stats[(int64_t)k * g.n_seqs + blockIdx.x] = rs[k];
-    }
+    gae_one_tile<GAE_LAYOUT_ROWS, LAMBDAS>(g, tile, t_begin, t_end, s_first, n_own, nullptr, A0, nv0, smem, all, rw, v,
+                                           ms, oa);
   }
 }
 
@@ -885,10 +1036,8 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
       }
     }
   }
-  double rs[1];
   float oa[GAE_ITEMS];
-  gae_one_tile<false, GAE_LAYOUT_CU, LAMBDAS>(g, tile, t_begin, t_end, s_first, n_own, cu_own, A0, nv0, rs, smem,
-                                              all, rw, v, ms, oa);
+  gae_one_tile<GAE_LAYOUT_CU, LAMBDAS>(g, tile, t_begin, t_end, s_first, n_own, cu_own, A0, nv0, smem, all, rw, v, ms, oa);
   if constexpr (STATS) gae_tile_group_stats(g, tile, lo, hi, tg, oa, ms);
 }
 
@@ -1705,14 +1854,12 @@ __global__ __launch_bounds__(NORM_THREADS) void adv_prep_kernel(PrepArgs a) {
 // last wave works the score out. Large ones are bound by HBM: the shaped rewards and the mask go from the shaping to
 // the scan in registers instead of through memory.
 // Kernels of the three calls and of this one: 64 x 1000 without a critic 17.5 -> 9.4 us; 1024 x 8192 with critic
-// and reference 87 -> 78 us (46 B a slot in place of 54, 4.9 TB/s). Whole calls, without a critic: 64 x 1000 33.1
-// -> 24.9, 1024 x 2048 35.8 -> 28.5, 256 x 8192 42.9 -> 35.5, 328 x 5555 41.8 -> 31.8, 1024 x 8192 100.4 -> 90.4; the rule
-// for the rows' number and length is areal_gae_padded_row_stats'.
-// A thread loads the mask and the log-probs of its 8 tokens from the tokens behind them (the roll), at
-// whatever alignment that is; the one thread of a row whose tokens reach its end picks them one by one. Four
-// tokens are stored before the next four are worked out, and what the block shares is in scalar registers: with
-// all 8 at a time the loop over tiles does not fit the 128 registers of four blocks a CU (58 spilled,
-// 1024 x 8192 105 us).
+// and reference 90 -> 66 us (46 B a slot in place of 54, 5.8 TB/s with inputs new to the caches). The rule for the
+// rows' number and length is row_sums_fit. Reference and values with the non-temporal hint: 65 us there, but
+// 20.2 against 18.0 at 400 x 3001, whose inputs are still in the last-level cache.
+// A thread has the tokens of gae_row_tile.
+// It loads the mask and the log-probs of its tokens from the tokens behind them (the roll), at whatever alignment
+// that is; the one thread of a row whose tokens reach its end picks them one by one.
 // ---------------------------------------------------------------------------------------
 struct AdvGaeArgs {
   PrepArgs p;                 // reward_score: the scores, with score_mode 0
@@ -1754,10 +1901,10 @@ DEVI float row_score(const AdvGaeArgs& a, int64_t b) {
 }
 
 
-// Inputs of a thread's 8 tokens from t0 of a row on: rolled mask bytes and log-probs, reference, values. END: they
-// may reach the end of the row.
+// Inputs of a thread's two quads from t0 and t0 + WAVE_QUADS of a row on: rolled mask bytes and log-probs, reference,
+// values. END: they may reach the end of the row.
 struct PrepItems {
-  u32x2 m;
+  uint32_t m[ROW_QUADS];
   float lp[GAE_ITEMS], rf[GAE_ITEMS], v[GAE_ITEMS];
 };
 template <bool END>
@@ -1768,57 +1915,50 @@ DEVI void prep_load(const AdvGaeArgs& a, int64_t row, int t0, PrepItems& x) {
               *const v = a.g.values != nullptr ? a.g.values + row : nullptr;
 #pragma unroll
   for (int i = 0; i < GAE_ITEMS; ++i) x.lp[i] = x.rf[i] = x.v[i] = 0.f;
-  x.m = u32x2{0u, 0u};
-  if (END && t0 >= L) return;
-  if (!END || t0 + GAE_ITEMS < L) {
-    x.m = *(const u32x2_any*)(lm + t0 + 1);
 #pragma unroll
-    for (int q = 0; q < GAE_ITEMS; q += 4) {
-      const f32x4 w = *(const f32x4_any*)(lp + t0 + q + roll);
+  for (int q = 0; q < ROW_QUADS; ++q) {
+    const int tq = t0 + q * WAVE_QUADS;
+    x.m[q] = 0u;
+    if (!END || tq + QUAD < L) {
+      x.m[q] = *(const u32_any*)(lm + tq + 1);
+      const f32x4 w = *(const f32x4_any*)(lp + tq + roll);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x.lp[q + e] = w[e];
-    }
-    if (rf != nullptr) {
+      for (int e = 0; e < QUAD; ++e) x.lp[QUAD * q + e] = w[e];
+      if (rf != nullptr) {
+        const f32x4 u = *(const f32x4_any*)(rf + tq);
 #pragma unroll
-      for (int q = 0; q < GAE_ITEMS; q += 4) {
-        const f32x4 w = *(const f32x4_any*)(rf + t0 + q);
+        for (int e = 0; e < QUAD; ++e) x.rf[QUAD * q + e] = u[e];
+      }
+      if (v != nullptr) {
+        const f32x4 u = *(const f32x4_any*)(v + tq);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x.rf[q + e] = w[e];
+        for (int e = 0; e < QUAD; ++e) x.v[QUAD * q + e] = u[e];
+      }
+    } else {
+      // the end of the row: its last token's neighbour is its first
+#pragma unroll
+      for (int e = 0; e < QUAD; ++e) {
+        const int t = tq + e, tn = t + 1 < L ? t + 1 : 0;
+        if (t >= L) break;
+        x.m[q] |= (uint32_t)lm[tn] << (8 * e);
+        x.lp[QUAD * q + e] = lp[roll ? tn : t];
+        if (rf != nullptr) x.rf[QUAD * q + e] = rf[t];
+        if (v != nullptr) x.v[QUAD * q + e] = v[t];
       }
     }
-    if (v != nullptr) {
-#pragma unroll
-      for (int q = 0; q < GAE_ITEMS; q += 4) {
-        const f32x4 w = *(const f32x4_any*)(v + t0 + q);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x.v[q + e] = w[e];
-      }
-    }
-    return;
-  }
-  // the end of the row: its last token's neighbour is its first
-#pragma unroll
-  for (int i = 0; i < GAE_ITEMS; ++i) {
-    const int t = t0 + i, tn = t + 1 < L ? t + 1 : 0;
-    if (t >= L) break;
-    x.m[i >> 2] |= (uint32_t)lm[tn] << (8 * (i & 3));
-    x.lp[i] = lp[roll ? tn : t];
-    if (rf != nullptr) x.rf[i] = rf[t];
-    if (v != nullptr) x.v[i] = v[t];
   }
 }
 
 template <int EST, bool ONE_TILE>
 __global__ __launch_bounds__(GAE_THREADS, 4) void adv_gae_kernel(AdvGaeArgs a) {
-  __shared__ MapF smem[GAE_THREADS / 64];
-  __shared__ MapF all[GAE_THREADS];
+  __shared__ RowMaps maps;
   __shared__ double s_rs[4 * 5];
   __shared__ float s_score;
   const PrepArgs& p = a.p;
   const int tid = threadIdx.x, L = (int)p.L;
   const int64_t b = blockIdx.x, row = b * L;
   int tile = ONE_TILE ? 0 : (L - 1) / GAE_TILE;
-  int t0 = tile * GAE_TILE + tid * GAE_ITEMS;
+  int t0 = row_tile_token(tile);
   PrepItems x;
   prep_load<true>(a, row, t0, x);
   int cnt = 0;
@@ -1835,40 +1975,28 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void adv_gae_kernel(AdvGaeArgs a) {
   }
   const float neg_ctl = -p.kl_ctl;
   const bool has_ref = p.ref_logp != nullptr;
-  GaeArgs g = a.g;  // the row alone
-  g.adv += row;
-  g.ret += row;
-  double A0 = 0.0, nv0 = 0.0, rs[5] = {0.0};
+  double A0 = 0.0, nv0 = 0.0, rs[5] = {0.0};  // state entering the tile from its right; sums of the row
   int t_zero = 0, t_out = 0, no_eos = 0;
   float score = 0.f;
   for (bool first = true;; first = false) {
-    float rw[GAE_ITEMS], ms[GAE_ITEMS], oa[GAE_ITEMS];  // rw: first the KL rewards
-    auto store4 = [&](float* to, int q, const f32x4& w) {
-      if (t0 + q + 4 <= L) {
-        *(f32x4_any*)(to + row + t0 + q) = w;
-      } else {
+    float rw[GAE_ITEMS];  // first the KL rewards
+    const ByteMask mask_of{x.m};
 #pragma unroll
-        for (int e = 0; e < 3; ++e)
-          if (t0 + q + e < L) to[row + t0 + q + e] = w[e];
-      }
-    };
-#pragma unroll
-    for (int q = 0; q < GAE_ITEMS; q += 4) {
+    for (int q = 0; q < ROW_QUADS; ++q) {
       f32x4 o_lm, o_old, o_ref, o_kl;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = q + e;
-        const float lm = (x.m[i >> 2] >> (8 * (i & 3))) & 0xffu ? 1.f : 0.f;
+      for (int e = 0; e < QUAD; ++e) {
+        const int i = QUAD * q + e;
+        const float lm = mask_of(i);
         float old, ref, kl, gkl, oc;
         adv_prep_token(p, EST, lm, x.lp[i], x.rf[i], has_ref, false, false, 0.f, neg_ctl, old, ref, kl, gkl, oc);
         o_lm[e] = lm; o_old[e] = old; o_ref[e] = ref; o_kl[e] = kl;
-        ms[i] = lm;
         rw[i] = kl;
       }
-      if (has_ref && p.ref_in_place) store4(p.ref_logp, q, o_ref);
-      store4(p.lm_out, q, o_lm);
-      store4(p.old_out, q, o_old);
-      store4(p.kl_out, q, o_kl);
+      if (has_ref && p.ref_in_place) row_store<false>(p.ref_logp + row, t0, L, q, o_ref);
+      row_store<false>(p.lm_out + row, t0, L, q, o_lm);
+      row_store<true>(p.old_out + row, t0, L, q, o_old);
+      row_store<true>(p.kl_out + row, t0, L, q, o_kl);
     }
     if (first) {  // (in scalar registers from here on)
       const int seqlen = __builtin_amdgcn_readfirstlane((int)block_sum_d((double)cnt, s_rs));
@@ -1881,23 +2009,25 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void adv_gae_kernel(AdvGaeArgs a) {
       if (p.mask_no_eos_with_zero && no_eos) score = 0.f;
     }
 #pragma unroll
-    for (int q = 0; q < GAE_ITEMS; q += 4) {
+    for (int q = 0; q < ROW_QUADS; ++q) {
       f32x4 o_tot;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = t0 + q + e;
-        const float gkl = t == t_zero ? 0.f : rw[q + e], oc = t == t_out ? score : 0.f;
+      for (int e = 0; e < QUAD; ++e) {
+        const int t = t0 + q * WAVE_QUADS + e;
+        const float gkl = t == t_zero ? 0.f : rw[QUAD * q + e], oc = t == t_out ? score : 0.f;
         o_tot[e] = gkl + oc;
-        rw[q + e] = o_tot[e];
+        rw[QUAD * q + e] = o_tot[e];
       }
-      store4(p.tot_out, q, o_tot);
+      row_store<false>(p.tot_out + row, t0, L, q, o_tot);
     }
-    gae_one_tile<true, GAE_LAYOUT_ONE_ROW, false>(g, tile, 0, L, 0, 1, nullptr, A0, nv0, rs, smem, all, rw, x.v, ms, oa,
-                                                  no_eos);
+    gae_row_tile<true, true>(a.g.discount, a.g.lam, tile, t0, L, no_eos != 0, rw, x.v, mask_of, maps, A0, nv0, rs,
+                             a.g.adv + row, a.g.ret + row);
     if (ONE_TILE || --tile < 0) break;
     t0 -= GAE_TILE;
     prep_load<false>(a, row, t0, x);
   }
+  rs[2] = rs[0];  // the mask is 0 or 1
+  rs[3] = rs[1];
   block_sum_n<5>(rs, s_rs);
   if (tid == 0) {
 #pragma unroll
@@ -2195,8 +2325,8 @@ bool row_sums_fit(int64_t n_seqs, int64_t uniform_len) {
   // A block per row: rows shorter than a tile leave lanes idle. While all blocks are resident (4 a CU) that
   // is cheaper than a launch of its own for the sums (all kernels of an advantage computation, rows x
   // slots: 64 x 1000 21.4 against 24.4 us, 1024 x 1000 33.4 against 35.4, 1024 x 64 20.8 against 21.3), with
-  // more rows it is not (2048 x 1536 54.9 against 52.7, 4096 x 64 44.9 against 25.0, 16384 x 256 142 against
-  // 63). Rows of nearly a tile fill their block whatever their number (2048 x 2047 66.0 against 69.6).
+  // many more short rows it is not, one launch for everything included (4096 x 256 43.6 against 35.9, 4096 x 512
+  // 47.6 against 42.5, 8192 x 512 83.0 against 61.3). Rows of nearly a tile fill their block whatever their number.
   return uniform_len >= GAE_TILE - GAE_TILE / 8 || n_seqs <= 1024;
 }
 
