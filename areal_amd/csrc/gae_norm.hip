@@ -2043,10 +2043,17 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void adv_gae_kernel(AdvGaeArgs a) {
 // active rewards taken just before the start (turn reward = difference of consecutive
 // prefixes). Thread 0 then runs the recurrence over the compact turns right to left, and pass
 // 2 hands every token its turn's advantage and return.
-// Per row workspace: prefix [L+1] double, value/adv/ret [L] float each.
+// Per row workspace: prefix [L+1] double, value/adv/ret [L] float each; a row of at most TURN_LDS turns (a
+// conversation has tens) keeps them in LDS.
+// A row is bound by latency: loads, two scans behind barriers per tile of the row, the recurrence. Blocks of up to
+// 1024 threads therefore, so that a row is one or two tiles, 16-byte accesses, and the recurrence from LDS (from global
+// memory it waited for a load per turn): 128 x 8192 53 -> 21 us, 512 x 4096 36 -> 19,
+// 1024 x 8192 88 -> 58, 64 x 1000 9.0 -> 6.2.
 // ---------------------------------------------------------------------------------------
 constexpr int TURN_THREADS = 256;
 constexpr int TURN_ITEMS = 4;
+constexpr int TURN_LDS = 512;
+typedef int i32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 struct TurnArgs {
   const float* rewards;
@@ -2071,7 +2078,8 @@ struct TurnArgs {
 struct TurnCarry { int count; int maxid; double sum; };
 
 // Exclusive scan over the block of (start count, running max id, reward sum), chunk carry
-// included. smem: [TURN_THREADS] of each.
+// included. smem: an entry per wave of each.
+template <int THREADS>
 DEVI TurnCarry turn_block_exclusive(int cnt, int mx, double sm, const TurnCarry& carry, int* s_cnt,
                                     int* s_max, double* s_sum, TurnCarry& chunk_total) {
   // s_cnt / s_max / s_sum: one entry per wave. Scans inside a wave through DPP, the waves' totals
@@ -2090,7 +2098,8 @@ DEVI TurnCarry turn_block_exclusive(int cnt, int mx, double sm, const TurnCarry&
     ex.sum += s_sum[i];
   }
   chunk_total = carry;
-  for (int i = 0; i < TURN_THREADS / 64; ++i) {
+#pragma unroll
+  for (int i = 0; i < THREADS / 64; ++i) {
     chunk_total.count += s_cnt[i];
     chunk_total.maxid = chunk_total.maxid > s_max[i] ? chunk_total.maxid : s_max[i];
     chunk_total.sum += s_sum[i];
@@ -2104,145 +2113,177 @@ DEVI TurnCarry turn_block_exclusive(int cnt, int mx, double sm, const TurnCarry&
   return ex;
 }
 
-__global__ __launch_bounds__(TURN_THREADS) void turn_gae_kernel(TurnArgs a) {
-  __shared__ int s_cnt[TURN_THREADS];
-  __shared__ int s_max[TURN_THREADS];
-  __shared__ double s_sum[TURN_THREADS];
-  __shared__ int s_k;
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void turn_gae_kernel(TurnArgs a) {
+  __shared__ int s_cnt[THREADS / 64], s_max[THREADS / 64];
+  __shared__ double s_sum[THREADS / 64];
+  __shared__ double s_prefix[TURN_LDS + 1];
+  __shared__ float s_val[TURN_LDS], s_adv[TURN_LDS], s_ret[TURN_LDS];
+  constexpr int TILE = THREADS * TURN_ITEMS;
   const int tid = threadIdx.x;
   const int64_t row = blockIdx.x, L = a.L;
   const float* rw = a.rewards + row * L;
   const float* vl = a.values != nullptr ? a.values + row * L : nullptr;  // (no critic: zero)
-  auto value = [&](int64_t t) { return vl != nullptr ? vl[t] : 0.f; };
   const float* ms = a.mask + row * L;
+  const float* add = a.addend != nullptr ? a.addend + row * L : nullptr;
   const int32_t* ids_row = a.turn_ids + row * L;
-  auto turn_id = [&](int64_t t) { return !a.roll ? ids_row[t] : (t + 1 < L ? ids_row[t + 1] : -1); };
   double* prefix = a.ws_prefix + row * (L + 1);
   float* tval = a.ws_val + row * L;
   float* tadv = a.ws_adv + row * L;
   float* tret = a.ws_ret + row * L;
+  auto load4 = [&](const float* from, int64_t t0, float (&x)[TURN_ITEMS]) {
+    if (from != nullptr && t0 + TURN_ITEMS <= L) {
+      const f32x4 w = *(const f32x4_any*)(from + t0);
+#pragma unroll
+      for (int i = 0; i < TURN_ITEMS; ++i) x[i] = w[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < TURN_ITEMS; ++i) x[i] = from != nullptr && t0 + i < L ? from[t0 + i] : 0.f;
+    }
+  };
   int bad = 0;
+
+  // A tile's tokens of this thread: mask, active ones and turn starts among them (bits), turns that started
+  // before the first of them; with SUMS also their active rewards and the sum of those before them.
+  float m[TURN_ITEMS], r[TURN_ITEMS];
+  unsigned act, start;
+  int k0;
+  double sum0;
+  auto scan_tile = [&](auto sums, int64_t t0, TurnCarry& carry) {
+    constexpr bool SUMS = decltype(sums)::value;
+    int ids[TURN_ITEMS];
+    load4(ms, t0, m);
+    if (t0 + TURN_ITEMS < L) {
+      const i32x4_any w = *(const i32x4_any*)(ids_row + t0 + (a.roll ? 1 : 0));
+#pragma unroll
+      for (int i = 0; i < TURN_ITEMS; ++i) ids[i] = w[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < TURN_ITEMS; ++i) {
+        const int64_t t = t0 + i + (a.roll ? 1 : 0);
+        ids[i] = t < L ? ids_row[t] : -1;
+      }
+    }
+    if (SUMS) load4(rw, t0, r);
+    int mx = -1;
+    double sm = 0.0;
+    act = start = 0;
+#pragma unroll
+    for (int i = 0; i < TURN_ITEMS; ++i) {
+      const bool on = m[i] != 0.0f;
+      if (SUMS) r[i] = on ? r[i] : 0.0f;
+      if (!on) continue;
+      act |= 1u << i;
+      if (ids[i] < 0) bad |= 1;
+      if ((int64_t)ids[i] >= L) bad |= 2;
+      mx = mx > ids[i] ? mx : ids[i];
+      if (SUMS) sm += (double)r[i];
+    }
+    // the number of starts in a thread depends on the maximum to its left, so scan the maximum
+    // and the reward sums first, then count starts, then scan the counts
+    TurnCarry tot1, tot2;
+    const TurnCarry ex1 = turn_block_exclusive<THREADS>(0, mx, sm, carry, s_cnt, s_max, s_sum, tot1);
+    int run_max = ex1.maxid;
+#pragma unroll
+    for (int i = 0; i < TURN_ITEMS; ++i) {
+      if (!((act >> i) & 1u)) continue;
+      if (ids[i] > run_max) start |= 1u << i;
+      if (ids[i] < run_max) bad |= 4;
+      run_max = run_max > ids[i] ? run_max : ids[i];
+    }
+    const TurnCarry ex2 = turn_block_exclusive<THREADS>(__popc(start), -1, 0.0, TurnCarry{carry.count, -1, 0.0}, s_cnt,
+                                                        s_max, s_sum, tot2);
+    k0 = ex2.count;
+    sum0 = ex1.sum;
+    carry = TurnCarry{tot2.count, tot1.maxid, tot1.sum};
+  };
 
   // ---- pass 1: compact the turns
   TurnCarry carry{0, -1, 0.0};
-  for (int64_t base = 0; base < L; base += TURN_THREADS * TURN_ITEMS) {
+  for (int64_t base = 0; base < L; base += TILE) {
     const int64_t t0 = base + (int64_t)tid * TURN_ITEMS;
-    int ids[TURN_ITEMS]; bool act[TURN_ITEMS]; float r[TURN_ITEMS];
-    int cnt = 0, mx = -1; double sm = 0.0;
-    // thread-local: starts relative to the maximum seen inside the thread's own items
+    scan_tile(std::true_type{}, t0, carry);
+    int k = k0;
+    double run_sum = sum0;
 #pragma unroll
     for (int i = 0; i < TURN_ITEMS; ++i) {
-      const int64_t t = t0 + i;
-      act[i] = t < L && ms[t] != 0.0f;
-      ids[i] = act[i] ? turn_id(t) : -1;
-      r[i] = act[i] ? rw[t] : 0.0f;
-      if (act[i]) {
-        if (ids[i] < 0) bad |= 1;
-        if ((int64_t)ids[i] >= L) bad |= 2;
-        mx = mx > ids[i] ? mx : ids[i];
-        sm += (double)r[i];
-      }
-    }
-    (void)cnt;
-    // the number of starts in a thread depends on the maximum to its left, so scan the maximum
-    // and the reward sums first, then count starts, then scan the counts
-    TurnCarry tot1;
-    const TurnCarry ex1 = turn_block_exclusive(0, mx, sm, carry, s_cnt, s_max, s_sum, tot1);
-    int run_max = ex1.maxid;
-    bool start[TURN_ITEMS];
-#pragma unroll
-    for (int i = 0; i < TURN_ITEMS; ++i) {
-      start[i] = act[i] && ids[i] > run_max;
-      if (act[i] && ids[i] < run_max) bad |= 4;
-      if (act[i]) run_max = run_max > ids[i] ? run_max : ids[i];
-      cnt += start[i];
-    }
-    TurnCarry tot2;
-    const TurnCarry ex2 = turn_block_exclusive(cnt, -1, 0.0, TurnCarry{carry.count, -1, 0.0}, s_cnt,
-                                               s_max, s_sum, tot2);
-    int k = ex2.count;
-    double run_sum = ex1.sum;
-#pragma unroll
-    for (int i = 0; i < TURN_ITEMS; ++i) {
-      if (start[i]) {
-        prefix[k] = run_sum;            // active rewards strictly before this turn
-        tval[k] = value(t0 + i);           // the turn's state value: value at its first token
+      if ((start >> i) & 1u) {
+        const float v = vl != nullptr ? vl[t0 + i] : 0.f;  // the turn's state value: value at its first token
+        if (k < TURN_LDS) { s_prefix[k] = run_sum; s_val[k] = v; }
+        prefix[k] = run_sum;  // active rewards strictly before this turn
+        tval[k] = v;
         ++k;
       }
       run_sum += (double)r[i];
     }
-    carry.count = tot2.count; carry.maxid = tot1.maxid; carry.sum = tot1.sum;
   }
-  if (tid == 0) { prefix[carry.count] = carry.sum; s_k = carry.count; }
+  const int K = carry.count;  // (the same in every thread)
+  if (tid == 0) {
+    prefix[K] = carry.sum;
+    if (K <= TURN_LDS) s_prefix[K] = carry.sum;
+  }
   if (bad) atomicOr(a.status, bad);
+  bad = 0;
   __syncthreads();
   __threadfence_block();
-  const int K = s_k;
 
   // ---- recurrence over the turns, right to left (gae.py:139-150)
+  const bool in_lds = K <= TURN_LDS;
   if (tid == 0) {
     const float gam = a.discount;
     const float lam = a.lam_seq ? a.lam_seq[row] : a.lam;
     const float c = gam * lam;
-    float nextv = (a.no_eos && a.no_eos[row]) ? value(L - 1) : 0.0f;
-    float last = 0.0f;
-    for (int k = K - 1; k >= 0; --k) {
-      const float R = (float)(prefix[k + 1] - prefix[k]);
-      const float V = tval[k];
-      const float delta = (R + gam * nextv) - V;
-      const float g = delta + c * last;
-      tadv[k] = g;
-      tret[k] = g + V;
-      nextv = V;
-      last = g;
-    }
+    auto recur = [&](const double* prefix, const float* tval, float* tadv, float* tret) {
+      float nextv = (a.no_eos && a.no_eos[row]) ? (vl != nullptr ? vl[L - 1] : 0.f) : 0.0f;
+      float last = 0.0f;
+      for (int k = K - 1; k >= 0; --k) {
+        const float R = (float)(prefix[k + 1] - prefix[k]);
+        const float V = tval[k];
+        const float delta = (R + gam * nextv) - V;
+        const float g = delta + c * last;
+        tadv[k] = g;
+        tret[k] = g + V;
+        nextv = V;
+        last = g;
+      }
+    };
+    if (in_lds) recur(s_prefix, s_val, s_adv, s_ret);
+    else recur(prefix, tval, tadv, tret);
   }
   __syncthreads();
   __threadfence_block();
 
-  // ---- pass 2: every token takes the result of its turn (gae.py:152-157)
+  // ---- pass 2: every token takes the result of its turn (gae.py:152-157); a row of one tile still has what
+  // pass 1 found
   TurnCarry carry2{0, -1, 0.0};
-  for (int64_t base = 0; base < L; base += TURN_THREADS * TURN_ITEMS) {
+  for (int64_t base = 0; base < L; base += TILE) {
     const int64_t t0 = base + (int64_t)tid * TURN_ITEMS;
-    int ids[TURN_ITEMS]; bool act[TURN_ITEMS]; float m[TURN_ITEMS];
-    int mx = -1;
+    float v[TURN_ITEMS], ad[TURN_ITEMS];
+    load4(vl, t0, v);
+    load4(add, t0, ad);
+    if (L > TILE) scan_tile(std::false_type{}, t0, carry2);
+    int k = k0;  // turns started strictly before this thread's first token
+    f32x4 o_adv, o_ret;
 #pragma unroll
     for (int i = 0; i < TURN_ITEMS; ++i) {
-      const int64_t t = t0 + i;
-      m[i] = t < L ? ms[t] : 0.0f;
-      act[i] = m[i] != 0.0f;
-      ids[i] = act[i] ? turn_id(t) : -1;
-      if (act[i]) mx = mx > ids[i] ? mx : ids[i];
-    }
-    TurnCarry tot1;
-    const TurnCarry ex1 = turn_block_exclusive(0, mx, 0.0, carry2, s_cnt, s_max, s_sum, tot1);
-    int run_max = ex1.maxid, cnt = 0;
-    bool start[TURN_ITEMS];
-#pragma unroll
-    for (int i = 0; i < TURN_ITEMS; ++i) {
-      start[i] = act[i] && ids[i] > run_max;
-      if (act[i]) run_max = run_max > ids[i] ? run_max : ids[i];
-      cnt += start[i];
-    }
-    TurnCarry tot2;
-    const TurnCarry ex2 = turn_block_exclusive(cnt, -1, 0.0, TurnCarry{carry2.count, -1, 0.0}, s_cnt,
-                                               s_max, s_sum, tot2);
-    int k = ex2.count;  // turns started strictly before this thread's first token
-#pragma unroll
-    for (int i = 0; i < TURN_ITEMS; ++i) {
-      const int64_t t = t0 + i;
-      if (start[i]) ++k;
-      if (t >= L) continue;
-      float adv = 0.0f, ret = value(t);
-      if (act[i] && k > 0) {
+      if ((start >> i) & 1u) ++k;
+      float adv = 0.0f, ret = v[i];
+      if (((act >> i) & 1u) && k > 0) {
         const float mm = m[i];
-        adv = tadv[k - 1] * mm;
-        ret = tret[k - 1] * mm + ret * (1.0f - mm);
+        adv = (in_lds ? s_adv[k - 1] : tadv[k - 1]) * mm;
+        ret = (in_lds ? s_ret[k - 1] : tret[k - 1]) * mm + ret * (1.0f - mm);
       }
-      a.adv[row * L + t] = a.addend != nullptr ? adv + a.addend[row * L + t] : adv;
-      a.ret[row * L + t] = ret;
+      o_adv[i] = add != nullptr ? adv + ad[i] : adv;
+      o_ret[i] = ret;
     }
-    carry2.count = tot2.count; carry2.maxid = tot1.maxid;
+    if (t0 + TURN_ITEMS <= L) {
+      *(f32x4_any*)(a.adv + row * L + t0) = o_adv;
+      *(f32x4_any*)(a.ret + row * L + t0) = o_ret;
+    } else {
+#pragma unroll
+      for (int i = 0; i < TURN_ITEMS - 1; ++i)
+        if (t0 + i < L) { a.adv[row * L + t0 + i] = o_adv[i]; a.ret[row * L + t0 + i] = o_ret[i]; }
+    }
   }
 }
 
@@ -2282,7 +2323,7 @@ __global__ __launch_bounds__(TURN_THREADS) void gae_context_kernel(const float* 
     }
     TurnCarry tot;
     // count: active tokens; max: running turn id; sum unused
-    const TurnCarry ex = turn_block_exclusive(nact, mx, 0.0, carry, s_cnt, s_max, s_sum, tot);
+    const TurnCarry ex = turn_block_exclusive<TURN_THREADS>(nact, mx, 0.0, carry, s_cnt, s_max, s_sum, tot);
     int run_max = ex.maxid;
 #pragma unroll
     for (int i = 0; i < TURN_ITEMS; ++i) {
@@ -2573,7 +2614,17 @@ int areal_turn_gae_ex(const float* rewards, const float* values, const float* lo
   a.ws_ret = a.ws_adv + (size_t)bs * max_seqlen;
   a.status = status;
   a.roll = roll_ids; a.addend = addend;
-  hipLaunchKernelGGL(turn_gae_kernel, dim3((unsigned)bs), dim3(TURN_THREADS), 0, stream, a);
+  auto launch = [&](auto threads) {
+    hipLaunchKernelGGL((turn_gae_kernel<decltype(threads)::value>), dim3((unsigned)bs), dim3(decltype(threads)::value), 0,
+                       stream, a);
+  };
+  // A row in as few tiles as can be while all rows' blocks are resident (rows x slots, us with blocks of 256 / 512 /
+  // 1024 threads: 128 x 8192 37.5 / 26.9 / 20.8, 512 x 4096 24.6 / 19.9 / 19.1, 1024 x 2001 18.3 / 16.7 / -; but
+  // 1024 x 8192 58.4 / 67.1 / 80.9).
+  if (max_seqlen > 512 * TURN_ITEMS && bs <= 512) launch(std::integral_constant<int, 1024>{});
+  else if (max_seqlen > 256 * TURN_ITEMS && max_seqlen <= 512 * TURN_ITEMS && bs <= 1024)
+    launch(std::integral_constant<int, 512>{});
+  else launch(std::integral_constant<int, 256>{});
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }
