@@ -797,7 +797,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
     xl = valid ? ws[3 * PT + t] : 0.f;
     if (ref_sums == 2) {
       const float lp = (float)(((double)xl * (double)c2 - (double)M) * 0.6931471805599453094 - log((double)S));
-      logprobs[t] = valid && xl == xl ? fminf(lp, 0.f) : lp;  // (as below: a label's logit is at most the maximum)
+      logprobs[t] = valid && lp > 0.f ? 0.f : lp;  // (as below: a label's logit is at most the maximum)
       if (logprobs_copy) logprobs_copy[t] = logprobs[t];
       return;
     }
@@ -808,7 +808,7 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
     const double lnS = log((double)S);
     if (logprobs) {
       const float lp = (float)(((double)xl * (double)c2 - rr) * ln2 - lnS);
-      logprobs[t] = xl <= M ? fminf(lp, 0.f) : lp;
+      logprobs[t] = xl <= M && lp > 0.f ? 0.f : lp;
       if (logprobs_copy) logprobs_copy[t] = logprobs[t];
     }
     if (entropy) entropy[t] = (float)(lnS - ln2 * (double)Q / (double)S);
@@ -820,10 +820,11 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
     const float logS = logf(S);
     // label exponent against the same rounded reference the sums use. For a label inside the
     // vocabulary (xl <= M) the result is <= 0 in exact arithmetic; the last rounding may leave
-    // +1e-8 when p = 1 to fp32 precision.
+    // +1e-8 when p = 1 to fp32 precision. (Compared, not fminf, which would make 0 of the NaN of a row with a
+    // NaN or infinite logit that is not the label's.)
     if (logprobs) {
       const float lp = fmaf(xl, c2, -ref_of(M, c2)) * LN2 - logS;
-      logprobs[t] = xl <= M ? fminf(lp, 0.f) : lp;
+      logprobs[t] = xl <= M && lp > 0.f ? 0.f : lp;
       if (logprobs_copy) logprobs_copy[t] = logprobs[t];
     }
     if (entropy) entropy[t] = logS - (Q * LN2) / S;
