@@ -96,12 +96,17 @@ constexpr int64_t BWD_MAX_BLOCKS = 1 << 23;  // a launch is limited to 2^32 thre
 struct Online {
   float m, s, q;  // max of z2 = x*c2, sum 2^(z2-m), sum (z2-m) 2^(z2-m)
 };
+// Sums of a part without a finite logit are 0, or NaN where it met a NaN or (the entropy's) a -inf, and stay so.
 DEVI void online_merge(Online& a, const Online& b) {
   const float m = fmaxf(a.m, b.m);
-  if (!(m > neg_inf())) return;
   float s = 0.f, q = 0.f;
-  if (a.m > neg_inf()) { const float d = a.m - m, al = fast_exp2(d); s += al * a.s; q += al * fmaf(d, a.s, a.q); }
-  if (b.m > neg_inf()) { const float d = b.m - m, al = fast_exp2(d); s += al * b.s; q += al * fmaf(d, b.s, b.q); }
+  auto part = [&](const Online& o) {
+    const float d = o.m > neg_inf() ? o.m - m : 0.f, al = fast_exp2(d);
+    s += al * o.s;
+    q += al * fmaf(d, o.s, o.q);
+  };
+  part(a);
+  part(b);
   a.m = m; a.s = s; a.q = q;
 }
 // x: raw logits; the exponents are z2 = x * c2 (c2 > 0). The running maximum is kept as the
@@ -121,7 +126,9 @@ DEVI void online_add(Online& st, const float (&x)[N], float c2) {
     }
     st.m = vm;
   }
-  const float m = st.m > neg_inf() ? st.m : 0.f;  // nothing but -inf so far: sums of nothing, not of inf - inf
+  // Nothing but -inf so far: exponentials of 0, not of inf - inf. A logit of -inf leaves the log-probabilities
+  // alone and makes the entropy NaN, as p log p = 0 x -inf does.
+  const float m = st.m > neg_inf() ? st.m : 0.f;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     const float t = fmaf(x[i], c2, -m);
@@ -187,7 +194,8 @@ __global__ __launch_bounds__(THREADS) void rows_fwd_kernel(const T* __restrict__
       // the label's exponent as the sums saw it: relative to the running maximum, by one fused
       // multiply-subtract
       const float tl = fmaf(Elem<T>::load(x + lab), c2, -r.m);
-      lp = fminf((tl - log2s) * LN2_F, 0.f);
+      lp = (tl - log2s) * LN2_F;
+      lp = lp > 0.f ? 0.f : lp;  // (NaN stays)
     }
     if (logprobs) logprobs[row] = lp;
     if (entropy) entropy[row] = (log2s - r.q / r.s) * LN2_F;

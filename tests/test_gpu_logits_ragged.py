@@ -46,3 +46,27 @@ def test_excluded_vocabulary_keeps_its_logprob(dev):
     y = torch.randint(0, 100, (6,), generator=g)
     lp, _ = gather_logprobs_entropy(x.to(dev), y.to(dev))
     torch.testing.assert_close(lp.cpu(), torch.log_softmax(x, -1)[torch.arange(6), y], rtol=1e-5, atol=2e-5)
+
+
+# a thread's first elements, its last, the row's edges; one NaN that a thread of its own meets (rows of 5 and 9)
+@pytest.mark.parametrize("rows", [3, 1023, 1024])
+@pytest.mark.parametrize("vocab", [5, 9, 333, 2051])
+@pytest.mark.parametrize("value", [float("-inf"), float("nan"), float("inf")])
+def test_logits_that_are_not_finite(dev, value, vocab, rows):
+    """As ``torch.log_softmax`` has them, on either side of the forward's line on rows: a NaN or +inf makes the row
+    NaN, -inf leaves the log-probabilities of the others alone and the entropy (0 x -inf) NaN."""
+    g = torch.Generator().manual_seed(rows + vocab)
+    base = torch.randn(rows * vocab + 3, generator=g)
+    y = torch.randint(0, vocab, (rows,), generator=g)
+    for start in (0, 1, 3):
+        x = base[start:start + rows * vocab].view(rows, vocab).clone()
+        for i in range(0, rows, 2):
+            x[i, (7 * i) % vocab] = value
+            if value == float("-inf") and i % 4 == 0:  # whole threads of nothing else
+                x[i, : vocab - 2] = value
+        xg = base.to(dev)[start:start + rows * vocab].view(rows, vocab)
+        xg.copy_(x.to(dev))
+        lp, ent = gather_logprobs_entropy(xg, y.to(dev))
+        want_lp, want_ent = L.gather_logprobs_entropy(x, y)
+        torch.testing.assert_close(lp.cpu(), want_lp, rtol=1e-5, atol=2e-5, equal_nan=True)
+        torch.testing.assert_close(ent.cpu(), want_ent, rtol=1e-5, atol=2e-5, equal_nan=True)
