@@ -1775,15 +1775,22 @@ template <bool E> using Fwd16AffineSave = Fwd16<E, true, false, true>;
 template <bool E> using Fwd16AffineMomSave = Fwd16<E, true, true, true>;
 
 // ---- forward for the label log-probabilities alone (see Fwd16): the sum of a token's exponentials relative to
-// a reference of its own, the largest logit of the first column. Per logit one accumulator read, one fma, one v_exp_f32 and one addition; no maximum is taken (nor minimum, nor
-// the entropy's sum) unless a column's sum shows that the reference is too low by LOGP_WINDOW binades,
-// which the first column's always does. The column is then summed again relative to a new reference while
-// its logits are still in registers, and the sums so far move to it: right for any logits, without a launch
-// that estimates references and a repeat behind it. The references lie in LDS between the tiles.
+// a reference of its own, at first the largest logit of the first column. Per logit one accumulator read, one
+// fma, one v_exp_f32 and one addition; no maximum is taken (nor minimum, nor the entropy's sum) unless a
+// column's sum shows that the reference is too low by LOGP_WINDOW binades, which the first column's always
+// does. The column is then summed again relative to a new reference while its logits are still in
+// registers, and the sums so far move to it: right for any logits, without a launch that estimates
+// references and a repeat behind it. The references lie in LDS between the tiles.
+// The window is narrow for the sake of the largest exponents, which are rounded at their own size: beside the
+// sweep with all outputs (sums relative to the running maximum) the error of a label 30 to 55 nats above the
+// others was 5.8e-8 against up to 2.5e-6 with 84 binades and is 5.8e-8 with 7 (60 rows of each; from
+// 16 to 25 nats the largest errors are the same, with 15 binades they are 1.4 times as large). A row then moves its reference once or
+// twice per range of the vocabulary.
 // 10007 x 1536 x 151936: 3384 -> 3297 us against the sweep with all outputs, with the merge and host side the whole call
 // 3361 -> 3244.
-constexpr float LOGP_WINDOW = 84.f;
-constexpr float LOGP_NO_REF = -3e38f;  // so far below every logit that the first column's sum overflows
+constexpr float LOGP_WINDOW = 7.f;
+constexpr float LOGP_COLUMN = 0x1p12f;  // a lane's 32 exponentials within the window add up to this at most
+constexpr float LOGP_NO_REF = -3e38f;   // so far below every logit that the first column's sum overflows
 template <bool EDGE, bool AFFINE>
 struct Logp16 {
   static constexpr int NA = 8;
@@ -1862,8 +1869,7 @@ struct Logp16 {
       };
       float s = sum(ref[b]);
       asm volatile("" : "+v"(s) : : ML16_ACC_CLOBBERS);
-      // a column's 32 exponentials within the window add up to 2^89 at most (NaN takes this way too)
-      if (__builtin_amdgcn_ballot_w64(!(s <= 0x1p90f)) != 0) {
+      if (__builtin_amdgcn_ballot_w64(!(s <= LOGP_COLUMN)) != 0) {  // (NaN takes this way too)
         float m = neg_inf();
 #pragma unroll
         for (int i = 0; i < 32; ++i) m = fmaxf(m, out(i) ? neg_inf() : x[i]);

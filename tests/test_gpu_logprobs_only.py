@@ -86,3 +86,23 @@ def test_rows_that_are_not_finite_are_those_of_the_full_sweep(dev):
     assert torch.equal(got.isnan(), full.isnan())
     ok = ~full.isnan()
     torch.testing.assert_close(got[ok], full[ok], rtol=1e-6, atol=1e-5)
+
+
+@pytest.mark.parametrize("V", [40000, 151936])  # (several tiles of the vocabulary to a workgroup)
+@pytest.mark.parametrize("lead", [12, 30, 40, 55])
+def test_confident_tokens(dev, lead, V):
+    """A label that stands alone, ``lead`` nats above normal logits. The logits are exact (one product each, of
+    bf16 values), so the error is that of the sums: as near as the sweep with all outputs, and where nothing but the label
+    counts (30 nats on) an ulp of its exponential and one of the sum, 2^-22."""
+    T, H = 128, 128
+    g = torch.Generator().manual_seed(lead + V)
+    hidden, weight = torch.eye(T, H), torch.randn(V, H, generator=g)
+    labels = torch.randint(0, V, (T,), generator=g)
+    weight[labels, torch.arange(T)] = lead + torch.randn(T, generator=g)
+    hidden, weight, labels = hidden.bfloat16().to(dev), weight.bfloat16().to(dev), labels.to(dev)
+    want, _ = _want(hidden, weight, labels)
+    got = compute_logprobs(hidden, weight, dict(rolled_input_ids=labels))
+    with torch.no_grad():
+        full = fused_lm_head_logprobs_entropy(hidden, weight, labels).logprobs
+    error, of_full = ((x.double() - want).abs().max().item() for x in (got, full))
+    assert error <= (2.0 ** -22 if lead >= 30 else 2.0 ** -22 + 1.5 * of_full), (error, of_full)
