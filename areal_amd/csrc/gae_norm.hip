@@ -2371,6 +2371,14 @@ bool row_sums_fit(int64_t n_seqs, int64_t uniform_len) {
   return uniform_len >= GAE_TILE - GAE_TILE / 8 || n_seqs <= 1024;
 }
 
+// Whether the normalisation of the scores rides in front of it (score_mode 2 of adv_gae_kernel): every row's last
+// wave sums its whole group, which costs nothing while the other waves of all resident blocks (4 a CU) wait for memory,
+// but adds up over rows x group. One launch against a launch for the scores in front, us: kernels of 1536 x 1800 in
+// groups of 16 / 1024 rows 23.0 / 24.0 against 23.9 / 28.8; whole advantage computations of 2048 x 2048 in groups of 16 /
+// 2048 rows 38.9 / 64.2 against 39.5 / 61.9, of 4096 x 2048 in groups of 16 / 4096 rows 66.0 / 142.8 against
+// 63.7 / 110.6, of one group of 8192 x 1800 430 against 274.
+bool scores_fit(int64_t n_seqs) { return n_seqs <= 2048; }
+
 }  // namespace
 
 extern "C" {
@@ -2840,7 +2848,8 @@ int areal_advantage_prep(const uint8_t* loss_mask, const uint8_t* attn_mask, con
 // (adv_gae_kernel), with their results. score_mode 0: rewards are the scores; 1: they are shaped first;
 // 2: and normalised within groups of rows (group_offsets / group_rows / n_groups / tail_group / levels as
 // areal_reward_scores, no level the batch). AREAL_ERR_UNSUPPORTED for the layouts that
-// areal_gae_padded_row_stats does not take either: make the three calls.
+// areal_gae_padded_row_stats does not take either (make the three calls) and, in mode 2, for more rows than
+// scores_fit (areal_reward_scores first, then mode 0).
 int areal_advantages_row_stats(const float* rewards, int score_mode, float bias, float scaling, float clip,
                                const int64_t* group_offsets, const int64_t* group_rows, int64_t n_groups, int tail_group,
                                int mean_level, int std_level, int unbiased, double eps, const uint8_t* loss_mask,
@@ -2859,7 +2868,7 @@ int areal_advantages_row_stats(const float* rewards, int score_mode, float bias,
   if (score_mode == 2 && (!group_offsets || !group_rows || n_groups <= 0)) return AREAL_ERR_BAD_ARG;
   if (score_mode == 2 && (mean_level < 0 || mean_level > 2 || std_level < 0 || std_level > 2)) return AREAL_ERR_BAD_ARG;
   if (score_mode == 2 && (mean_level == LEVEL_BATCH || std_level == LEVEL_BATCH)) return AREAL_ERR_UNSUPPORTED;
-  if (!row_sums_fit(bs, L)) return AREAL_ERR_UNSUPPORTED;
+  if (!row_sums_fit(bs, L) || (score_mode == 2 && !scores_fit(bs))) return AREAL_ERR_UNSUPPORTED;
   // with the log-probs rolled a thread reads its neighbour's token: not in place
   if (roll_logp && logp == old_out) return AREAL_ERR_BAD_ARG;
   AdvGaeArgs a{};

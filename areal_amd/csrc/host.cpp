@@ -899,29 +899,7 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
     const auto& [off, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = *norm;
     return call(ptr<int64_t>(off), ptr<int64_t>(rows), rows.numel(), tail, mean_level, std_level, unbiased, eps);
   };
-  // (a score that is not one per row, or values of another size, are for the calls that look at them)
-  if (gae.has_value() && !turn_mode && bs > 0 && L > 0) {
-    const Tensor v = f32(or_undefined(std::get<0>(*gae)));
-    if (!v.defined() || (v.is_cuda() && v.sizes() == lm.sizes())) {
-      const Tensor adv = at::empty_like(lm), ret = at::empty_like(lm), sums = empty(lm, {5, bs}, at::kDouble);
-      const int rc = norm_args([&](const int64_t* off, const int64_t* rows, int64_t n, int tail, int mean_level,
-                                   int std_level, int unbiased, double eps) {
-        return areal_advantages_row_stats(
-            ptr<float>(sc), scored ? 0 : norm.has_value() ? 2 : 1, (float)bias, (float)scaling, (float)clip, off, rows, n,
-            tail, mean_level, std_level, unbiased, eps, ptr<uint8_t>(lmb), ptr<uint8_t>(amb), ptr<float>(logp),
-            ptr<float>(ref), ptr<float>(v), bs, L, recompute ? 0 : 1, estimator, clamp, no_eos_zero, ref_in_place,
-            (float)kl_ctl, (float)std::get<1>(*gae), (float)std::get<2>(*gae), ptr<float>(lm), ptr<float>(old),
-            ptr<float>(kl), ptr<float>(tot), ptr<int64_t>(seqlens), ptr<uint8_t>(no_eos), ptr<float>(adv),
-            ptr<float>(ret), ptr<double>(sums), stream);
-      });
-      if (rc != AREAL_ERR_UNSUPPORTED) {
-        check(rc, "areal_advantages_row_stats");
-        return py::make_tuple(lm, old.view(logp_src.sizes()), kl, tot, OptTensor(), OptTensor(), no_eos,
-                              py::make_tuple(adv, ret, sums));
-      }
-    }
-  }
-  if (!scored) {
+  auto shape_scores = [&] {
     const Tensor shaped = empty_f32(sc, bs);
     check(norm_args([&](const int64_t* off, const int64_t* rows, int64_t n, int tail, int mean_level, int std_level,
                         int unbiased, double eps) {
@@ -930,7 +908,38 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
           }),
           "areal_reward_scores");
     sc = shaped;
+    scored = true;
+  };
+  // (a score that is not one per row, or values of another size, are for the calls that look at them)
+  if (gae.has_value() && !turn_mode && bs > 0 && L > 0) {
+    const Tensor v = f32(or_undefined(std::get<0>(*gae)));
+    if (!v.defined() || (v.is_cuda() && v.sizes() == lm.sizes())) {
+      const Tensor adv = at::empty_like(lm), ret = at::empty_like(lm), sums = empty(lm, {5, bs}, at::kDouble);
+      auto one_launch = [&] {
+        return norm_args([&](const int64_t* off, const int64_t* rows, int64_t n, int tail, int mean_level,
+                             int std_level, int unbiased, double eps) {
+          return areal_advantages_row_stats(
+              ptr<float>(sc), scored ? 0 : norm.has_value() ? 2 : 1, (float)bias, (float)scaling, (float)clip, off, rows,
+              n, tail, mean_level, std_level, unbiased, eps, ptr<uint8_t>(lmb), ptr<uint8_t>(amb), ptr<float>(logp),
+              ptr<float>(ref), ptr<float>(v), bs, L, recompute ? 0 : 1, estimator, clamp, no_eos_zero, ref_in_place,
+              (float)kl_ctl, (float)std::get<1>(*gae), (float)std::get<2>(*gae), ptr<float>(lm), ptr<float>(old),
+              ptr<float>(kl), ptr<float>(tot), ptr<int64_t>(seqlens), ptr<uint8_t>(no_eos), ptr<float>(adv),
+              ptr<float>(ret), ptr<double>(sums), stream);
+        });
+      };
+      int rc = one_launch();
+      if (rc == AREAL_ERR_UNSUPPORTED && !scored) {  // it may take the scores ready-made
+        shape_scores();
+        rc = one_launch();
+      }
+      if (rc != AREAL_ERR_UNSUPPORTED) {
+        check(rc, "areal_advantages_row_stats");
+        return py::make_tuple(lm, old.view(logp_src.sizes()), kl, tot, OptTensor(), OptTensor(), no_eos,
+                              py::make_tuple(adv, ret, sums));
+      }
+    }
   }
+  if (!scored) shape_scores();
   const Tensor gkl = turn_mode ? empty(logp, {bs, L}, at::kFloat) : Tensor(),
                outcome = turn_mode ? empty(logp, {bs, L}, at::kFloat) : Tensor();
   check(areal_advantage_prep(ptr<uint8_t>(lmb), ptr<uint8_t>(amb), ptr<float>(logp), ptr<float>(ref), ptr<float>(sc), bs,

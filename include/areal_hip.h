@@ -517,7 +517,8 @@ int areal_advantage_prep(const uint8_t* loss_mask, const uint8_t* attn_mask, con
 /* Reward scores (areal_reward_scores), areal_advantage_prep and areal_gae_padded_row_stats of a padded
  * [bs, L] batch in one launch, with their results. score_mode 0: rewards are the scores; 1: they are
  * shaped first; 2: shaped and normalised within groups of rows (no level may be the batch).
- * AREAL_ERR_UNSUPPORTED for row counts and lengths that areal_gae_padded_row_stats does not take. */
+ * AREAL_ERR_UNSUPPORTED for row counts and lengths that areal_gae_padded_row_stats does not take, and in
+ * mode 2 for more than 2048 rows. */
 int areal_advantages_row_stats(const float* rewards, int score_mode, float bias, float scaling, float clip,
                                const int64_t* group_offsets, const int64_t* group_rows,
                                int64_t n_groups, int tail_group, int mean_level, int std_level,

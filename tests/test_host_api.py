@@ -75,6 +75,17 @@ def test_bf16_weight_gradient_needs_a_single_token_chunk():
     assert lib.areal_lmhead_bwd(*args, 3, 512, fake, 1 << 30, None) == -1  # bad argument
 
 
+def test_one_launch_advantages_take_the_scores_of_few_rows_only():
+    """areal_advantages_row_stats normalises the scores in front of the scan, where each row sums its whole
+    group, for up to 2048 rows; for more it says so before anything is launched or read."""
+    lib = _lib.load()
+    fake = 0x10000  # never dereferenced: the rule comes first
+    rc = lib.areal_advantages_row_stats(
+        fake, 2, 0.0, 1.0, 20.0, fake, fake, 1, -1, 2, 2, 1, 1e-5, fake, fake, fake, None, None, 2049, 2048, 1, 1, 0, 0, 0,
+        0.1, 0.99, 0.95, fake, fake, fake, fake, fake, fake, fake, fake, fake, None)
+    assert rc == _lib.ERR_UNSUPPORTED
+
+
 def test_no_cpu_fallback():
     h = torch.randn(4, 8).bfloat16()
     w = torch.randn(16, 8).bfloat16()
