@@ -876,7 +876,7 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
   require_numel(bs, {{"rewards", &score}});
   require_numel(bs * L, {{"logprobs", &logp_src}, {"loss_mask", &loss_mask}, {"attention_mask", &attention_mask},
                          {"ref_logp", &ref_arg}});
-  require_gpu(logp_src, loss_mask, attention_mask, score);
+  require_gpu(logp_src, loss_mask, attention_mask, score, ref_arg);
   const c10::hip::HIPGuard guard(logp_src.device().index());
   const areal_stream_t stream = stream_of(logp_src);
   Tensor sc = score.scalar_type() == at::kFloat ? score : score.to(at::kFloat);
@@ -913,7 +913,7 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
   // (a score that is not one per row, or values of another size, are for the calls that look at them)
   if (gae.has_value() && !turn_mode && bs > 0 && L > 0) {
     const Tensor v = f32(or_undefined(std::get<0>(*gae)));
-    if (!v.defined() || (v.is_cuda() && v.sizes() == lm.sizes())) {
+    if (!v.defined() || (v.device() == lm.device() && v.sizes() == lm.sizes())) {
       const Tensor adv = at::empty_like(lm), ret = at::empty_like(lm), sums = empty(lm, {5, bs}, at::kDouble);
       auto one_launch = [&] {
         return norm_args([&](const int64_t* off, const int64_t* rows, int64_t n, int tail, int mean_level,

@@ -1,10 +1,13 @@
-"""Inputs of the advantage calls off the common path: the no-EOS mask of turn-level GAE in host memory, a
-negative reward clip, more reward scores than 2^24."""
+"""Inputs of the advantage calls off the common path: the no-EOS mask of turn-level GAE in host memory, arrays
+that are refused there, a negative reward clip, more reward scores than 2^24."""
 
 import pytest
 import torch
 
 from areal_amd import _lib
+from areal_amd.config import NormConfig
+from areal_amd.data import KLEstimator, Normalization
+from areal_amd.ppo.actor import compute_advantages
 from areal_amd.ppo.gae import _compute_turn_level_gae
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +45,23 @@ def test_reward_scores(dev, n, clip, group):
         torch.testing.assert_close(out, want, rtol=1e-5, atol=1e-5, equal_nan=True)
     else:
         assert torch.equal(out.nan_to_num(7.0), want.nan_to_num(7.0))
+
+
+def _batch(dev, bs, length):
+    g = torch.Generator().manual_seed(bs)
+    attn = torch.ones(bs, length, dtype=torch.bool)
+    data = dict(input_ids=torch.zeros(bs, length, dtype=torch.long), attention_mask=attn, loss_mask=attn,
+                logprobs=torch.randn(bs, length, generator=g), ref_logp=torch.randn(bs, length, generator=g),
+                values=torch.randn(bs, length, generator=g), rewards=torch.randn(bs, generator=g),
+                turn_ids=(torch.arange(length) // 10).to(torch.int32).expand(bs, length).contiguous())
+    return {k: v.to(dev) for k, v in data.items()}
+
+
+@pytest.mark.parametrize("unit", ["token", "turn"])
+@pytest.mark.parametrize("name", ["ref_logp", "values", "logprobs", "loss_mask", "attention_mask", "rewards"])
+def test_arrays_in_host_memory_are_refused(dev, name, unit):
+    data = _batch(dev, 6, 100)
+    data[name] = data[name].cpu()
+    with pytest.raises(_lib.ArealHipError, match="MI355X only"):
+        compute_advantages(data, kl_ctl=0.1, kl_estimator=KLEstimator("k1"), gae_timestep_unit=unit,
+                           adv_norm=Normalization(NormConfig(mean_level="group", std_level="group", group_size=2)))
