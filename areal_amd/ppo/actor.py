@@ -586,7 +586,6 @@ def compute_advantages(
     if kl_estimator is None:
         kl_estimator = KLEstimator("k1")
     bs = data["input_ids"].shape[0]
-    dev = data["input_ids"].device
 
     if overlong_reward_penalty:
         assert overlong_tokens is not None
@@ -607,7 +606,7 @@ def compute_advantages(
             and score.ndim == 1 and score.is_cuda and score.dtype == torch.float32 and not dist.is_initialized()
         )
         if native:
-            score_tables = reward_norm._tables(bs, 1, group_sizes, dev)
+            score_tables = reward_norm._tables(bs, 1, group_sizes, score.device)
         if score_tables is None:
             score = torch.clip((score + reward_bias) * reward_scaling, max=reward_clip, min=-reward_clip)
             score, scored = reward_norm(score, group_sizes=group_sizes), True

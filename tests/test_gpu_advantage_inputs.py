@@ -65,3 +65,14 @@ def test_arrays_in_host_memory_are_refused(dev, name, unit):
     with pytest.raises(_lib.ArealHipError, match="MI355X only"):
         compute_advantages(data, kl_ctl=0.1, kl_estimator=KLEstimator("k1"), gae_timestep_unit=unit,
                            adv_norm=Normalization(NormConfig(mean_level="group", std_level="group", group_size=2)))
+
+
+def test_token_ids_in_host_memory(dev):
+    """Nothing reads them: the groups' tables go where the rewards are."""
+    options = dict(kl_ctl=0.1, kl_estimator=KLEstimator("k1"))
+    here, there = _batch(dev, 6, 100), _batch(dev, 6, 100)
+    there["input_ids"] = there["input_ids"].cpu()
+    for data in (here, there):
+        norm = Normalization(NormConfig(mean_level="group", std_level="group", group_size=3))
+        compute_advantages(data, reward_norm=norm, adv_norm=norm, **options)
+    assert torch.equal(here["advantages"], there["advantages"])
