@@ -81,7 +81,7 @@ DEVI bool gemm_skipped(const GemmArgs& g) { return gate_closed(g.skip_if_set, g.
 // consecutive ones are RB B tiles x 32 / RB splits. Every XCD has the same number of tiles to
 // within one row or column of them, whatever the number of B tiles is.
 //
-// dWeight is laid out as a flat list (xg < 0): the tiles in blocks of RB B tiles x all A tiles, an
+// dWeight may be laid out as a flat list (xg < 0, see dw_flat): the tiles in blocks of RB B tiles x all A tiles, an
 // eighth of the list per XCD, and the XCD's part dealt to its 32 CUs tile by tile. A workgroup takes
 // `chain` of them, 32 apart, so that the next tile's first k-tiles arrive while this one is stored.
 struct Sched {
@@ -183,6 +183,16 @@ static int xcd_block(int S) { return S >= 8 ? 4 : (S >= 4 ? 8 : (S >= 2 ? 16 : 3
 // 183 us in 10 rounds, 160 in one chain; 8192 x 1536 into fp32 3084 -> 2982 adding, 2803 -> 2771 storing; with
 // 64 k-tiles per tile (4096 x 896) 737 -> 734. More than 16 would leave a CU that another stream holds up
 // with a long queue of its own, for less than half a per cent.
+// dWeight as a flat list or in super-blocks. In super-blocks the XCDs take neighbouring blocks in turn and read the same
+// A tiles (of the hidden states) at about the same time; in their eighths of a flat list they are at any place, and
+// with more than the 8 A tiles that a window of 32 workgroups covers they read different ones, which do not all
+// stay in the last-level cache over a long K range. A short one gains more from the chain. Backward of the weight alone,
+// super-blocks / flat list, us, up to 8 A tiles: 4096 x 896 826 / 816, 4096 x 1536 1367 / 1280, 32768 x 1536 10201 / 10091, 32768 x
+// 2048 13137 / 13105; more, at most 128 k-tiles: 4096 x 4096 3499 / 3386, 8192 x 4096 6728 / 6592, 8192 x 5120 8416 / 8299,
+// 8192 x 8192 11060 / 10965; longer: 12288 x 4096 9702 / 9665, 16384 x 2560 8588 / 8491, 16384 x 3584 11916 / 12184, 16384 x 8192
+// 22518 / 23143, 32768 x 3584 24000 / 25051, 32768 x 4096 26358 / 26617, 32768 x 5120 32369 / 34350. Added into fp32, with
+// dHidden: 16384 x 1536 10488 / 10273, 8192 x 4096 13800 / 13957, 16384 x 4096 26848 / 27388, 32768 x 4096 51782 / 53065.
+static bool dw_flat(int64_t H, int64_t K) { return H <= 8 * TILE || K <= 128 * BK; }
 static Sched make_flat_sched(int nbj, int nai, bool chain) {
   Sched sc = make_sched(0, nbj, 0, nai, nai);
   sc.xg = -1;
@@ -2175,7 +2185,7 @@ int launch_store(const GemmArgs& g, const StoreParams& ep, int mode, hipStream_t
   if (mode == 0 || mode == 3) allow16 = ep.ldo % 8 == 0 && aligned16(ep.out) && ep.M % 8 == 0;
   Regions r = plan_regions(ep.M, ep.N, g.K, 0, 1 << 20, allow16);
   Sched flat;
-  if (KERNEL16 == KERNEL16_TN && layout == nullptr && g.ksplit <= 1) {
+  if (KERNEL16 == KERNEL16_TN && layout == nullptr && g.ksplit <= 1 && dw_flat(g.acols, g.K)) {
     const int nai = (int)ceil_div_i64(ep.M, TILE), nbj = (int)ceil_div_i64(ep.N, TILE);
     flat = make_flat_sched(nbj, nai, km_chainable(g.acols, nai) && km_chainable(g.bcols, nbj));
     layout = &flat;
@@ -2334,7 +2344,8 @@ int launch_dhidden(const u16* w, int64_t V, const u16* dl, int64_t ldv, int64_t 
 
 // dWeight [V, H] in bf16 has ceil(V / 256) x ceil(H / 256) output tiles. When their number is not a
 // multiple of the chip's 256 CUs the last round occupies a few of them for a whole K range while the
-// others idle (594 x 16 tiles: 37.1 rounds). The B tiles of that last partial round are then contracted
+// others idle (594 x 16 tiles: 37.1 rounds); in super-blocks, which go round-robin to the XCDs, when their
+// number is not a multiple of 8. The B tiles of that last partial round are then contracted
 // by a second launch that splits the token (K) range over z copies of its schedule, fp32 partial results
 // summed by splitk_reduce_bf16_kernel.
 struct DwTail {
@@ -2347,9 +2358,22 @@ DwTail plan_dw_tail(int64_t H, int64_t V, int64_t Tpad) {
   const int nai = (int)ceil_div_i64(H, TILE), nbj = (int)ceil_div_i64(V, TILE);
   DwTail t{nbj, 1, 0, 0, 32};
   if (!k16_ok(Tpad) || H % 8 != 0) return t;
-  const int64_t tiles = (int64_t)nbj * nai, rounds = tiles / 256;
-  if (rounds == 0 || tiles % 256 == 0) return t;
-  const int nbj_main = (int)(rounds * 256 / nai);
+  int nbj_main;
+  double rest = 1.0;  // rounds of a whole K range that the main launch is without
+  if (dw_flat(H, Tpad)) {
+    const int64_t tiles = (int64_t)nbj * nai, rounds = tiles / 256;
+    if (rounds == 0 || tiles % 256 == 0) return t;
+    nbj_main = (int)(rounds * 256 / nai);
+  } else {
+    const Sched sc = make_sched(0, nbj, 0, nai, nai);
+    if (sc.n_sb % 8 == 0) return t;
+    const int n_sb_s = sc.n_sb / sc.n_sb_j;
+    int nj = sc.n_sb_j;
+    while (nj > 0 && (nj * n_sb_s) % 8 != 0) --nj;
+    nbj_main = nj * sc.RB;
+    rest = (double)(ceil_div_i64(sc.n_sb, 8) - nj * n_sb_s / 8);
+  }
+  if (nbj_main == 0) return t;
   const int64_t nk = Tpad / BK;
   int best = 1, best_sb = 32;
   double best_cost = sched_cost(make_sched(nbj_main, nbj - nbj_main, 0, nai, nai), 1);
@@ -2360,9 +2384,9 @@ DwTail plan_dw_tail(int64_t H, int64_t V, int64_t Tpad) {
       if (cost < best_cost - 1e-9) { best_cost = cost; best = z; best_sb = sb_wgs; }
     }
   }
-  // rounds of a whole K range: one more, or the second launch's. A k-tile takes about a microsecond;
+  // rounds of a whole K range: the rest's, or the second launch's. A k-tile takes about a microsecond;
   // the two extra launches have to be paid for.
-  if (best <= 1 || (1.0 - best_cost) * (double)nk < 16.0) return t;
+  if (best <= 1 || (rest - best_cost) * (double)nk < 16.0) return t;
   t.nbj_main = nbj_main;
   t.z = best;
   t.sb_wgs = best_sb;
@@ -2377,7 +2401,7 @@ size_t dw_tail_bytes(int64_t H, int64_t V, int64_t Tpad) {
 }
 
 // dWeight [V, H] in bf16 = B^T A over the K token rows of the k-major operands g.A [K, H] and
-// g.B [K, ldv]: whole rounds of super-blocks in one launch, then (plan_dw_tail) the remaining
+// g.B [K, ldv]: whole rounds in one launch, then (plan_dw_tail) the remaining
 // vocabulary rows with the token range split, through dw_part (dw_tail_bytes(H, V, K) bytes).
 int launch_dweight_bf16(GemmArgs g, int64_t H, int64_t V, int64_t ldv, void* dweight, float* dw_part,
                         hipStream_t stream) {

@@ -61,6 +61,11 @@ def test_workspace_size_queries_run_without_gpu():
     assert saved(32768, 4096, 151936) - saved(32768, 4096, 151552) == 6 * 384 * 4096 * 4 + 256
     # 144 x 2 tiles = 9 super-blocks: the last 16 tile columns (the test shape of tests/test_gpu_lmhead.py)
     assert saved(2048, 512, 36764) > 2 * (36764 - 128 * 256) * 512 * 4
+    # a hidden size of more than 8 tiles and a token range of more than 8192: super-blocks. 501 x 32 tiles are 126 x 4 of them, whole
+    # rounds of 8; of 594 x 20 tiles 144 x 3 super-blocks are whole rounds, the other 4480 rows get 2 copies
+    parts = lambda T, H, V: saved(T, H, V) - (4 * T + 2 * T * H + 5 * 256)  # noqa: E731
+    assert parts(16384, 8192, 128256) == 0
+    assert parts(32768, 5120, 151936) == 2 * 4480 * 5120 * 4 + 256
     assert lib.areal_gae_workspace_bytes(0) == 0
     assert lib.areal_actor_loss_workspace_bytes(10, 3) > 0
 
