@@ -1,7 +1,8 @@
 """Advantages with a fixed lambda run as one launch in front of their normalisation; a lambda per row takes the
 calls it was made of (reward scores, shaping, scan of padded rows). With the same lambda in both forms, the shaped
-arrays are the same bits and the scan, whose tiles start elsewhere, differs by fp32 rounding: 20 compositions
-of maps, |difference| <= 64 * 2^-24 of the largest magnitude.
+arrays are the same bits and what comes of the scan, whose row sums differ by the order in which the compiler adds
+them, agrees to |difference| <= 64 * 2^-24 of the largest magnitude. (Both walk a row by the same code:
+test_gpu_advantage_rows.py has the scan against the oracle.)
 
 Row lengths around a thread's 8 tokens and the tile, none a multiple of anything; rows without tokens, with one,
 with two, full ones; arrays at any address; every estimator; scores shaped, normalised in groups (whole, ragged, one

@@ -10,6 +10,7 @@ Tolerances as in test_gpu_lmhead.py: logprobs / entropy 2e-3 absolute, gradients
 import pytest
 import torch
 
+from areal_amd import _lib
 from areal_amd.functional import fused_lm_head_logprobs_entropy
 
 pytestmark = pytest.mark.gpu
@@ -41,8 +42,7 @@ def _case_list():
         h = hiddens[int(torch.randint(len(hiddens), (1,), generator=g))]
         v = vocabs[int(torch.randint(len(vocabs), (1,), generator=g))]
         cases.append((t, h, v))
-    # dWeight's last partial round of super-blocks with a ragged hidden size (2.5 tiles) and a
-    # ragged vocabulary: 80 x 3 tiles
+    # a ragged hidden size (2.5 tiles) and a ragged vocabulary: 80 x 3 dWeight tiles, not a round of 256 workgroups
     cases.append((2048, 640, 20403))
     # token count 64 short of a multiple of 128 with a contraction long enough to split
     cases.append((1984, 256, 9000))
@@ -144,3 +144,36 @@ def test_model_family_shapes(dev, H, V, save_probs):
     assert (out.entropy - ent).abs().max().item() < 2e-3
     assert _rel(h.grad.float(), dh) < 1e-2
     assert _rel(w.grad.float(), dw) < 1e-2
+
+
+def _tail_copies(T, H, V):
+    """fp32 copies of the rows behind dWeight's last whole round in the workspace of the saved backward, which holds beside
+    them row factors, scaled hidden states, a transposed weight where V is ragged, and dHidden's copies."""
+    up = lambda n, k: -(-n // k) * k  # noqa: E731
+    nai = up(H, 256) // 256
+    rows = V - up(V, 256) // 256 * nai // 256 * 256 // nai * 256
+    rest = _lib.load().areal_lmhead_bwd_saved_workspace_bytes(T, H, V)
+    rest -= 4 * T + 2 * up(T, 128) * H + (2 * H * up(V, 64) if V % 64 else 0) + 5 * 256
+    copies = lambda n, size: 4 * n * size * H + 256 if n > 1 else 0  # noqa: E731
+    found = {n for n in range(9) for dh in range(129) if rest == copies(dh, T) + copies(n, rows)}
+    assert len(found - {1}) == 1, found
+    return max(found - {1})
+
+
+@pytest.mark.parametrize("T,H,V", [(2048, 640, 25003), (2000, 896, 17480), (4096, 1608, 12000)])
+def test_split_tail_of_dweight(dev, T, H, V):
+    """More dWeight tiles than whole rounds of 256 workgroups, the rest contracted by a second launch that splits the
+    token range: narrow tiles (640 = 3 x 224 - 32, 896 = 4 x 224), a hidden size that no chain takes (1608 is no multiple of
+    16), ragged vocabularies. Every element against fp32 torch: 2 % of the gradient's largest magnitude, the bound of bf16 operands and
+    outputs."""
+    assert _tail_copies(T, H, V) >= 2
+    g = torch.Generator(device=dev).manual_seed(T + H + V)
+    hidden = torch.randn(T, H, generator=g, device=dev).bfloat16()
+    weight = (torch.randn(V, H, generator=g, device=dev) * (2.0 / H ** 0.5)).bfloat16().requires_grad_(True)
+    labels = torch.randint(0, V, (T,), generator=g, device=dev)
+    grad = torch.randn(T, generator=g, device=dev)
+    fused_lm_head_logprobs_entropy(hidden, weight, labels, save_probs=True).logprobs.backward(grad)
+    d = -torch.softmax(hidden.float() @ weight.detach().float().t(), -1)
+    d[torch.arange(T, device=dev), labels] += 1
+    want = (d * grad[:, None]).t() @ hidden.float()
+    assert (weight.grad.float() - want).abs().max().item() <= 2e-2 * want.abs().max().item()

@@ -59,7 +59,7 @@ def test_workspace_size_queries_run_without_gpu():
     # whole rounds and need none.
     saved = lib.areal_lmhead_bwd_saved_workspace_bytes
     assert saved(32768, 4096, 151936) - saved(32768, 4096, 151552) == 6 * 384 * 4096 * 4 + 256
-    # 144 x 2 tiles = 9 super-blocks: the last 16 tile columns (the test shape of tests/test_gpu_lmhead.py)
+    # 144 x 2 tiles are 32 more than a round of 256: the last 16 tile columns (the test shape of tests/test_gpu_lmhead.py)
     assert saved(2048, 512, 36764) > 2 * (36764 - 128 * 256) * 512 * 4
     # a hidden size of more than 8 tiles and a token range of more than 8192: super-blocks. 501 x 32 tiles are 126 x 4 of them, whole
     # rounds of 8; of 594 x 20 tiles 144 x 3 super-blocks are whole rounds, the other 4480 rows get 2 copies
