@@ -1764,7 +1764,7 @@ DEVI void adv_prep_token(const PrepArgs& a, int estimator, float lm, float lp, f
   if (estimator == 1) est = diff;
   else if (estimator == 2) est = diff * diff / 2.0f;
   else { const float neg = -diff; est = expf(neg) - 1.f - neg; }
-  if (a.apply_clamp) est = fminf(fmaxf(est, -10.f), 10.f);
+  if (a.apply_clamp) est = est < -10.f ? -10.f : est > 10.f ? 10.f : est;  // (torch.clamp keeps NaN)
   kl = neg_ctl * est;
   gkl = at_end ? 0.f : kl;
   oc = at_out ? score : 0.f;

@@ -1,5 +1,5 @@
 """Inputs of the advantage calls off the common path: the no-EOS mask of turn-level GAE in host memory, arrays
-that are refused there, a negative reward clip, more reward scores than 2^24."""
+that are refused there, log-probabilities that are not finite, a negative reward clip, more reward scores than 2^24."""
 
 import pytest
 import torch
@@ -76,3 +76,20 @@ def test_token_ids_in_host_memory(dev):
         norm = Normalization(NormConfig(mean_level="group", std_level="group", group_size=3))
         compute_advantages(data, reward_norm=norm, adv_norm=norm, **options)
     assert torch.equal(here["advantages"], there["advantages"])
+
+
+@pytest.mark.parametrize("unit", ["token", "turn"])
+@pytest.mark.parametrize("estimator", ["k1", "k2", "k3"])
+@pytest.mark.parametrize("length", [100, 2051])
+def test_logprobs_that_are_not_finite(dev, length, estimator, unit):
+    """The clamped estimate keeps NaN, as ``torch.clamp`` does, and bounds the infinities."""
+    data = _batch(dev, 6, length)
+    data["loss_mask"][:, 0] = False  # (a prompt: no turn)
+    data["logprobs"][0, 7], data["logprobs"][1, 50], data["ref_logp"][2, length - 3] = float("nan"), float("-inf"), float("nan")
+    data["logprobs"][3, 20], data["ref_logp"][4, 30] = 30.0, float("-inf")
+    estimate = KLEstimator(estimator)
+    out = compute_advantages(data, kl_ctl=0.1, kl_estimator=estimate, gae_timestep_unit=unit,
+                             adv_norm=Normalization(NormConfig(mean_level="group", std_level="group", group_size=2)))
+    want = -0.1 * estimate(out["logprobs"], out["ref_logp"])
+    assert want.isnan().any() and want.abs().eq(1.0).any()
+    torch.testing.assert_close(out["kl_rewards"], want, rtol=1e-6, atol=1e-7, equal_nan=True)
