@@ -2,7 +2,7 @@
 (NaN for the whole row), from every sweep that makes one, and never the 0 of a certain token.
 
 A weight row of NaN makes one logit of every token NaN; one with an infinite entry makes it +inf or -inf by the sign of the
-hidden value (-inf counts nothing). Finite results: |error| <= 2^-20 of the largest |logit| + 2^-18, as for fp32 sums."""
+hidden value (-inf counts nothing). One such row, and 500 in a row: whole tiles without another logit. Finite results: |error| <= 2^-20 of the largest |logit| + 2^-18, as for fp32 sums."""
 
 import pytest
 import torch
@@ -16,13 +16,14 @@ pytestmark = pytest.mark.gpu
 # 128: the hand-scheduled sweeps, 72: the generic one; 1600 ends in a last tile that overlaps its predecessor
 @pytest.mark.parametrize("T,H,V", [(140, 128, 1536), (140, 128, 1600), (70, 72, 600)])
 @pytest.mark.parametrize("entry", [float("nan"), float("inf")])
+@pytest.mark.parametrize("rows", [1, 500])
 @pytest.mark.parametrize("sweep", ["logprobs_only", "no_grad", "saved", "recompute"])
-def test_one_bad_weight_row(dev, sweep, entry, T, H, V):
+def test_bad_weight_rows(dev, sweep, rows, entry, T, H, V):
     g = torch.Generator().manual_seed(V)
     hidden = torch.randn(T, H, generator=g).bfloat16()
     weight = (torch.randn(V, H, generator=g) * 0.1).bfloat16()
     bad = V - 7
-    weight[bad, 0] = entry
+    weight[bad + 1 - rows:bad + 1, 0] = entry
     labels = torch.randint(0, V, (T,), generator=g)
     labels[5], labels[6] = bad, bad
     x = hidden.float() @ weight.float().t()
