@@ -1,7 +1,8 @@
 """dWeight launches of more tiles than the chip has CUs: a workgroup then takes several of them, the next
 one's operands arriving while this one is stored. Ragged last tiles of either operand (fetched through a
 window that ends with the operand), 256- and 224-wide tiles, an operand of one tile, an odd number of
-k-tiles, and a hidden size that the chain does not take (not a multiple of 16).
+k-tiles, and a hidden size that the chain does not take (not a multiple of 16). The last four lie either side of the
+rule on 8 tiles of hidden size and 8192 tokens, beyond which the tiles are laid out in super-blocks instead.
 
 Every element is compared with fp32 torch: |error| <= 2 % of the gradient's largest magnitude, the bound of
 bf16 operands and outputs that the elementwise test of the tile widths uses."""
@@ -17,6 +18,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("mode", ["saved", "recompute", "fp32", "fp32_accumulate"])
 @pytest.mark.parametrize("T,H,V", [
     (130, 1056, 16448), (256, 1792, 12992), (192, 2496, 16384), (128, 520, 32768), (200, 128, 70000), (320, 256, 140032),
+    (8192, 2056, 9000), (8320, 2048, 9000), (8320, 2056, 9000), (8320, 2304, 8192),
 ])
 def test_every_element_of_a_chain(dev, T, H, V, mode):
     g = torch.Generator(device=dev).manual_seed(T + H + V)
