@@ -1854,7 +1854,7 @@ __global__ __launch_bounds__(NORM_THREADS) void adv_prep_kernel(PrepArgs a) {
 // last wave works the score out. Large ones are bound by HBM: the shaped rewards and the mask go from the shaping to
 // the scan in registers instead of through memory.
 // Kernels of the three calls and of this one: 64 x 1000 without a critic 17.5 -> 9.4 us; 1024 x 8192 with critic
-// and reference 90 -> 66 us (46 B a slot in place of 54, 5.8 TB/s with inputs new to the caches). The rule for the
+// and reference 90 -> 66 us (42 B a slot in place of 50, 5.3 TB/s with inputs new to the caches). The rule for the
 // rows' number and length is row_sums_fit. Reference and values with the non-temporal hint: 65 us there, but
 // 20.2 against 18.0 at 400 x 3001, whose inputs are still in the last-level cache.
 // A thread has the tokens of gae_row_tile.
