@@ -1800,11 +1800,11 @@ template <bool E> using Fwd16AffineMomSave = Fwd16<E, true, true, true>;
 // does. The column is then summed again relative to a new reference while its logits are still in
 // registers, and the sums so far move to it: right for any logits, without a launch that estimates
 // references and a repeat behind it. The references lie in LDS between the tiles.
-// The window is narrow for the sake of the largest exponents, which are rounded at their own size: beside the
-// sweep with all outputs (sums relative to the running maximum) the error of a label 30 to 55 nats above the
-// others was 5.8e-8 against up to 2.5e-6 with 84 binades and is 5.8e-8 with 7 (60 rows of each; from
-// 16 to 25 nats the largest errors are the same, with 15 binades they are 1.4 times as large). A row then moves its reference once or
-// twice per range of the vocabulary.
+// The window is narrow for the sake of the largest exponents, which are rounded at their own size. Largest error of
+// 128 tokens with exact logits against 64 bits, window of 84 binades / of 7 / sweep with all outputs: normal
+// logits 5.1e-7 / 5.1e-7 / 1.1e-6; a label 16 nats above them 8.6e-7 / 5.9e-7 / 5.9e-7, 25 nats 1.3e-6 / 6.6e-7 / 6.6e-7,
+// 30 nats 1.4e-6 / 1.4e-7 / 1.4e-7, 55 nats 2.6e-6 / 5.9e-8 / 5.9e-8, at the same speed. (15 binades: 1.4
+// times the sweep's at 16 nats.) A row moves its reference once or twice per range of the vocabulary.
 // 10007 x 1536 x 151936: 3384 -> 3297 us against the sweep with all outputs, with the merge and host side the whole call
 // 3361 -> 3244.
 constexpr float LOGP_WINDOW = 7.f;
