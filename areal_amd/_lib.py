@@ -126,6 +126,12 @@ SIGNATURES: dict[str, tuple] = {
         [P, I, F, F, F, P, P, I64, I, I, I, I, D, P, P, P, P, P, I64, I64, I, I, I, I, I, F, F, F, P, P, P, P, P, P, P, P,
          P, P],
     ),
+    "areal_advantages_normalized_workspace_bytes": (SZ, [I64]),
+    "areal_advantages_normalized": (
+        I,
+        [P, I, F, F, F, P, P, I64, I, I, I, I, D, P, P, P, P, P, I64, I64, I, I, I, I, I, F, F, F, P, P, P, P, P, P, P, P,
+         P, P, SZ, P],
+    ),
     "areal_turn_gae_ex": (I, [P, P, P, P, I, P, P, P, I64, I64, F, F, P, P, P, P, SZ, P]),
     "areal_gae_lambda_context": (I, [P, P, I64, I64, P, P, P, P]),
     "areal_group_norm_workspace_bytes": (SZ, [I64, I64]),
@@ -159,6 +165,17 @@ class LossConfig(ctypes.Structure):
         ("rs_has_lower", c_int),
         ("rs_lower", c_float),
     ]
+
+
+
+class GroupNormSpec(ctypes.Structure):
+    """``areal_group_norm_spec``: normalisation within groups of rows."""
+
+    _fields_ = [
+        ("group_offsets", P), ("n_groups", I64), ("max_group_rows", I64), ("tail_group", I), ("mean_level", I),
+        ("std_level", I), ("leave_one_out", I), ("unbiased", I), ("wait_us", I), ("eps", D),
+    ]
+
 
 _lib = None
 _host = None

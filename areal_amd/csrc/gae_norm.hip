@@ -13,6 +13,10 @@
 // Affine maps compose associatively and constant maps absorb whatever lies to their right, so
 // one unsegmented suffix scan over the whole packed array gives every sequence its own
 // recurrence. Maps are held in fp64 (five coefficients); outputs are rounded to fp32.
+#include <algorithm>
+#include <atomic>
+#include <random>
+
 #include "common.hpp"
 
 namespace {
@@ -570,11 +574,12 @@ struct FloatMask {
 
 // rw, v: rewards and values of the thread's tokens (zero beyond the row). mask_of(i): their mask, zero beyond the row
 // (which makes such a token the identity). boot: whether the row's last value is bootstrapped. (A0, nv0): the fp64 state entering the tile from its
-// right, replaced by the one leaving it on the left. rs: the row's sums of GaeArgs::row_stats (STATS). adv, ret: the row.
-template <bool STATS, bool BINARY, class Mask>
+// right, replaced by the one leaving it on the left. rs: the row's sums of GaeArgs::row_stats (STATS). put_adv(q, x): takes
+// the advantages of quad q. ret: the row.
+template <bool STATS, bool BINARY, class Mask, class PutAdv>
 DEVI void gae_row_tile(float gam, float lam, int tile, int t0, int L, bool boot, float (&rw)[GAE_ITEMS],
                        float (&v)[GAE_ITEMS], const Mask& mask_of, RowMaps& maps, double& A0, double& nv0,
-                       double (&rs)[STATS ? 5 : 1], float* adv, float* ret) {
+                       double (&rs)[STATS ? 5 : 1], const PutAdv& put_adv, float* ret) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const float c0 = gam * lam;
   const int last = L - 1 - t0;
@@ -652,7 +657,7 @@ DEVI void gae_row_tile(float gam, float lam, int tile, int t0, int L, bool boot,
         }
       }
     }
-    row_store<false>(adv, t0, L, q, o_adv);
+    put_adv(q, o_adv);
     row_store<false>(ret, t0, L, q, o_ret);
     advance(total[q], Aw, nw);
   }
@@ -697,8 +702,9 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
       load(g.rewards, rw);
       load(g.values, v);
       load(g.mask, ms);
-      gae_row_tile<STATS, false>(g.discount, lam, tile, t0, L, boot, rw, v, FloatMask{ms}, maps, A0, nv0, rs,
-                                 g.adv + row, g.ret + row);
+      gae_row_tile<STATS, false>(
+          g.discount, lam, tile, t0, L, boot, rw, v, FloatMask{ms}, maps, A0, nv0, rs,
+          [&](int q, const f32x4& w) { row_store<false>(g.adv + row, t0, L, q, w); }, g.ret + row);
     }
     if constexpr (STATS) {
       __shared__ double s_rs[4 * 5];
@@ -1239,7 +1245,9 @@ struct NormParams {
   double mean, std_d, eps;
   bool mean64, std64;
 };
-DEVI NormParams norm_params(const NormArgs& a, int g, const double (&v)[10]) {
+// rows(): the number of rows of the group (asked for only where it counts).
+template <class Rows>
+DEVI NormParams norm_params(const NormArgs& a, int g, const double (&v)[10], const Rows& rows) {
   // mean context (see make_mean_ctx)
   MeanCtx mc;
   mc.level = a.mean_level; mc.identity = false; mc.zero = false; mc.loo = false; mc.cnt = 0.0; mc.sum = 0.0;
@@ -1263,7 +1271,7 @@ DEVI NormParams norm_params(const NormArgs& a, int g, const double (&v)[10]) {
     else std_d = cnt == 0.0 ? 1.0 : sqrt(ss / cnt);
   } else if (a.std_level == LEVEL_GROUP) {
     if (g == a.tail_group) std_d = 0.0;
-    else if (a.grows[g] == 1 && a.unbiased) std_d = 1.0;
+    else if (a.unbiased && rows() == 1) std_d = 1.0;
     else {
       const double cnt = v[0], ss = ss_of(v[2], v[3], v[4]);
       if (a.unbiased) std_d = cnt <= 1.0 ? 1.0 : sqrt(ss / (cnt - 1.0));
@@ -1277,6 +1285,9 @@ DEVI NormParams norm_params(const NormArgs& a, int g, const double (&v)[10]) {
   np.mean64 = a.mean_level == LEVEL_BATCH;
   np.std64 = a.std_level == LEVEL_BATCH;
   return np;
+}
+DEVI NormParams norm_params(const NormArgs& a, int g, const double (&v)[10]) {
+  return norm_params(a, g, v, [&] { return a.grows[g]; });
 }
 DEVI float norm_one(const NormParams& p, float x, float m, bool has_mask) {
   if (p.mean64 || p.std64) {
@@ -1867,7 +1878,152 @@ struct AdvGaeArgs {
   int score_mode;             // 1: scores are shaped here, 2: and normalised within groups
   NormArgs score;             // x = raw rewards [bs], groups of rows
   float bias, scaling, clip;
+  // NORM: normalisation of the advantages within groups of rows (goff in elements), see adv_normalise_row
+  NormArgs norm;
+  uint64_t *sums, *left;      // [bs][4] and [bs] in the workspace
+  uint64_t call;              // a number no other call has
+  unsigned wait_ticks;        // of the 100 MHz clock
 };
+
+// ---- Normalisation in the launch that made the advantages: a row's block keeps them in LDS, hands the row's sums to
+// the blocks of its group and waits for theirs, up to ADV_GROUP_ROWS rows. The batch's advantages then go to memory once
+// instead of being written, read back with the mask and written again by a launch of its own (46 against 54 B a
+// slot, and 5 us less for a small batch).
+// The sums of a row are sealed words: three numbers and a check word made of them and the call's number. They go
+// out and come in as agent-scope atomics (past the XCD's own L2), in any order: whoever reads four words that fit has all of
+// them, whatever the workspace held before (a chance of 2^-64 a row otherwise), and nothing has to be cleared.
+// No wait is unbounded: the blocks of a group lie next to each other in the grid, but nobody promises that they
+// are on the chip together. A block whose time is up stores its row as it is and leaves a note (`left`); it, or any
+// block of the group that finds all sums, then takes the note (one of them, by compare and swap) and normalises that row
+// from memory. Leaving a note is followed by another look at the sums, publishing one's sums precedes the look for notes:
+// of the block that leaves one and the last of the group to publish, one sees the other.
+constexpr int ADV_GROUP_ROWS = 64;                   // one lane per row
+constexpr int ADV_NORM_TILES = 4;                    // of a row, 8 mask bits each
+constexpr unsigned ADV_WAIT_TICKS = 20000;           // 200 us
+DEVI uint64_t sums_seal(uint64_t call, const uint64_t (&w)[3]) {
+  return call + w[0] * 0x9e3779b97f4a7c15ull + w[1] * 0xbf58476d1ce4e5b9ull + w[2] * 0x94d049bb133111ebull;
+}
+DEVI void publish_sums(const AdvGaeArgs& a, int64_t b, const double (&s)[3]) {  // by one thread
+  uint64_t w[3];
+  uint64_t* const to = a.sums + 4 * b;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    w[k] = __builtin_bit_cast(uint64_t, s[k]);
+    __hip_atomic_store(to + k, w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __hip_atomic_store(to + 3, sums_seal(a.call, w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The sums of rows [r0, r0 + n), added up by a whole wave (lane i: row r0 + i) in the order of the apply kernel's;
+// false when they were not all there within `ticks`.
+DEVI bool gather_sums(const AdvGaeArgs& a, int64_t r0, int n, unsigned ticks, double (&s)[3]) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t* const from = a.sums + 4 * (r0 + lane);
+  const uint64_t start = wall_clock64();
+  bool have = lane >= n;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) s[k] = 0.0;
+  for (;;) {
+    if (!have) {
+      uint64_t w[3];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) w[k] = __hip_atomic_load(from + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const uint64_t seal = __hip_atomic_load(from + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      have = seal == sums_seal(a.call, w);
+      if (have) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s[k] = __builtin_bit_cast(double, w[k]);
+      }
+    }
+    if (__builtin_amdgcn_ballot_w64(!have) == 0) break;
+    if (wall_clock64() - start >= ticks) return false;
+    __builtin_amdgcn_s_sleep(1);
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) s[k] = wave_sum(s[k]);
+  return true;
+}
+struct RowGroup { int g, first, rows; };  // group of a row: its first row and their number
+DEVI RowGroup row_group(const NormArgs& n, int64_t row, int64_t L) {  // by a whole wave; row: the row's first element
+  const int g = wave_count_le(n.goff + 1, n.G, row, threadIdx.x & 63);
+  const int64_t e0 = n.goff[g], e1 = n.goff[g + 1];
+  return RowGroup{g, (int)(e0 / L), (int)((e1 - e0) / L)};
+}
+// Row b from LDS (x, `bits`: the mask of the thread's tokens, 8 a tile), after its scan; s: its sums.
+DEVI void adv_normalise_row(const AdvGaeArgs& a, int64_t b, const RowGroup& rg, const float* x, uint32_t bits,
+                            const double (&s)[3]) {
+  __shared__ double s_sum[3];
+  __shared__ int s_flag;
+  __shared__ uint64_t s_todo;
+  const int tid = threadIdx.x, L = (int)a.p.L;
+  float* const adv = a.g.adv + b * L;
+  auto of_tiles = [&](auto&& f) {
+    for (int tile = (L - 1) / GAE_TILE; tile >= 0; --tile) {
+      const int t0 = row_tile_token(tile);
+#pragma unroll
+      for (int q = 0; q < ROW_QUADS; ++q)
+        row_store<false>(adv, t0, L, q, f(*(const f32x4*)(x + t0 + q * WAVE_QUADS), bits >> (8 * tile + QUAD * q)));
+    }
+  };
+  if (tid == 0) publish_sums(a, b, s);
+  uint64_t todo = 0;  // (first wave) rows of the group whose blocks have left
+  auto gather = [&](unsigned ticks) {
+    if (tid < 64) {
+      double v[3];
+      const bool all = gather_sums(a, rg.first, rg.rows, ticks, v);
+      if (tid == 0) {
+        s_flag = all ? 1 : 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s_sum[k] = v[k];
+      }
+      if (all) {
+        const bool note = tid < rg.rows && __hip_atomic_load(a.left + rg.first + tid, __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT) == a.call;
+        todo = __builtin_amdgcn_ballot_w64(note);
+      }
+    }
+    __syncthreads();
+    return s_flag != 0;
+  };
+  if (!gather(a.wait_ticks)) {
+    of_tiles([&](const f32x4& w, uint32_t) { return w; });
+    __threadfence();
+    __syncthreads();
+    if (tid == 0) atomicExch((unsigned long long*)a.left + b, (unsigned long long)a.call);
+    if (!gather(0)) return;
+    // (its own note among the others' now)
+  } else {
+    double v[10];
+    v[0] = v[2] = s_sum[0]; v[1] = v[3] = s_sum[1]; v[4] = s_sum[2];
+#pragma unroll
+    for (int k = 5; k < 10; ++k) v[k] = 0.0;
+    const NormParams np = norm_params(a.norm, rg.g, v, [&] { return rg.rows; });
+    of_tiles([&](const f32x4& w, uint32_t m) {
+      f32x4 r;
+#pragma unroll
+      for (int e = 0; e < QUAD; ++e) r[e] = norm_one(np, w[e], (m >> e) & 1u ? 1.f : 0.f, true);
+      return r;
+    });
+  }
+  if (tid == 0) s_todo = todo;
+  __syncthreads();
+  for (uint64_t rest = s_todo; rest != 0; rest &= rest - 1) {
+    const int64_t r = rg.first + __builtin_ctzll(rest);
+    __syncthreads();
+    if (tid == 0)
+      s_flag = atomicCAS((unsigned long long*)a.left + r, (unsigned long long)a.call, (unsigned long long)~a.call) == a.call;
+    __syncthreads();
+    if (s_flag == 0) continue;  // somebody else's
+    __threadfence();
+    double v[10];
+    v[0] = v[2] = s_sum[0]; v[1] = v[3] = s_sum[1]; v[4] = s_sum[2];
+#pragma unroll
+    for (int k = 5; k < 10; ++k) v[k] = 0.0;
+    const NormParams np = norm_params(a.norm, rg.g, v, [&] { return rg.rows; });
+    float* const to = a.g.adv + r * L;
+    const float* const m = a.p.lm_out + r * L;
+    for (int t = tid; t < L; t += GAE_THREADS) to[t] = norm_one(np, to[t], m[t], true);
+  }
+}
 
 // Score of row b, by a whole wave. The sums run in reward_score_groups_kernel's order.
 DEVI float row_score(const AdvGaeArgs& a, int64_t b) {
@@ -1949,8 +2105,10 @@ DEVI void prep_load(const AdvGaeArgs& a, int64_t row, int t0, PrepItems& x) {
   }
 }
 
-template <int EST, bool ONE_TILE>
+template <int EST, bool ONE_TILE, bool NORM>
 __global__ __launch_bounds__(GAE_THREADS, 4) void adv_gae_kernel(AdvGaeArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float row_adv[];  // NORM: whole tiles
+  __shared__ RowGroup s_group;
   __shared__ RowMaps maps;
   __shared__ double s_rs[4 * 5];
   __shared__ float s_score;
@@ -1973,9 +2131,14 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void adv_gae_kernel(AdvGaeArgs a) {
     const float sc = row_score(a, b);
     if (tid == GAE_THREADS - 1) s_score = sc;
   }
+  if (NORM && tid < 64) {
+    const RowGroup rg = row_group(a.norm, row, L);
+    if (tid == 0) s_group = rg;
+  }
   const float neg_ctl = -p.kl_ctl;
   const bool has_ref = p.ref_logp != nullptr;
   double A0 = 0.0, nv0 = 0.0, rs[5] = {0.0};  // state entering the tile from its right; sums of the row
+  uint32_t bits = 0;
   int t_zero = 0, t_out = 0, no_eos = 0;
   float score = 0.f;
   for (bool first = true;; first = false) {
@@ -2020,18 +2183,32 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void adv_gae_kernel(AdvGaeArgs a) {
       }
       row_store<false>(p.tot_out + row, t0, L, q, o_tot);
     }
-    gae_row_tile<true, true>(a.g.discount, a.g.lam, tile, t0, L, no_eos != 0, rw, x.v, mask_of, maps, A0, nv0, rs,
-                             a.g.adv + row, a.g.ret + row);
+    if constexpr (NORM) {
+#pragma unroll
+      for (int i = 0; i < GAE_ITEMS; ++i) bits |= (mask_of(i) != 0.f ? 1u : 0u) << (8 * tile + i);
+    }
+    gae_row_tile<true, true>(
+        a.g.discount, a.g.lam, tile, t0, L, no_eos != 0, rw, x.v, mask_of, maps, A0, nv0, rs,
+        [&](int q, const f32x4& w) {
+          if constexpr (NORM) *(f32x4*)(row_adv + t0 + q * WAVE_QUADS) = w;
+          else row_store<false>(a.g.adv + row, t0, L, q, w);
+        },
+        a.g.ret + row);
     if (ONE_TILE || --tile < 0) break;
     t0 -= GAE_TILE;
     prep_load<false>(a, row, t0, x);
   }
-  rs[2] = rs[0];  // the mask is 0 or 1
-  rs[3] = rs[1];
-  block_sum_n<5>(rs, s_rs);
-  if (tid == 0) {
-#pragma unroll
-    for (int k = 0; k < 5; ++k) a.g.row_stats[(int64_t)k * a.g.n_seqs + b] = rs[k];
+  // (the mask is 0 or 1)
+  double s[3] = {rs[0], rs[1], rs[4]};
+  block_sum_n<3>(s, s_rs);
+  if constexpr (NORM) {
+    adv_normalise_row(a, b, s_group, row_adv, bits, s);
+  } else if (tid == 0) {
+    double* const to = a.g.row_stats + b;
+    const int64_t st = a.g.n_seqs;
+    to[0] = to[2 * st] = s[0];
+    to[st] = to[3 * st] = s[1];
+    to[4 * st] = s[2];
   }
 }
 
@@ -2360,6 +2537,16 @@ void launch_gae_owned(const GaeArgs& g, int64_t grid, hipStream_t stream) {
   }
 }
 
+// A number no other call has, and no memory by chance.
+uint64_t next_call_number() {
+  static const uint64_t seed = ((uint64_t)std::random_device{}() << 32) ^ std::random_device{}();
+  static std::atomic<uint64_t> calls{0};
+  uint64_t z = seed + (calls.fetch_add(1, std::memory_order_relaxed) + 1) * 0x9e3779b97f4a7c15ull;  // splitmix64
+  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
+  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
+  return z ^ (z >> 31);
+}
+
 // Whether the row sums ride in the scan of padded rows.
 bool row_sums_fit(int64_t n_seqs, int64_t uniform_len) {
   if (uniform_len > 64 * (int64_t)GAE_TILE || n_seqs > (1 << 30)) return false;
@@ -2378,6 +2565,65 @@ bool row_sums_fit(int64_t n_seqs, int64_t uniform_len) {
 // 2048 rows 38.9 / 64.2 against 39.5 / 61.9, of 4096 x 2048 in groups of 16 / 4096 rows 66.0 / 142.8 against
 // 63.7 / 110.6, of one group of 8192 x 1800 430 against 274.
 bool scores_fit(int64_t n_seqs) { return n_seqs <= 2048; }
+
+// Arguments of adv_gae_kernel from those of areal_advantages_row_stats (with norm: advantages normalised, no row sums).
+int adv_gae_args(AdvGaeArgs& a, const float* rewards, int score_mode, float bias, float scaling, float clip,
+                        const int64_t* group_offsets, const int64_t* group_rows, int64_t n_groups, int tail_group,
+                        int mean_level, int std_level, int unbiased, double eps, const uint8_t* loss_mask,
+                        const uint8_t* attn_mask, const float* logp, float* ref_logp, const float* values, int64_t bs,
+                        int64_t L, int roll_logp, int estimator, int apply_clamp, int mask_no_eos_with_zero,
+                        int ref_in_place, float kl_ctl, float discount, float gae_lambda, float* lm_out, float* old_out,
+                        float* kl_out, float* tot_out, int64_t* seqlens_out, uint8_t* no_eos_out, float* advantages,
+                        float* returns, double* row_stats, const areal_group_norm_spec* norm) {
+  if (bs < 0 || L < 0 || estimator < 1 || estimator > 3 || score_mode < 0 || score_mode > 2) return AREAL_ERR_BAD_ARG;
+  if (bs == 0) return AREAL_OK;
+  if (L == 0) return AREAL_ERR_BAD_ARG;
+  if (!rewards || !loss_mask || !attn_mask || !logp || !lm_out || !old_out || !kl_out || !tot_out || !seqlens_out ||
+      !no_eos_out || !advantages || !returns || (!row_stats && norm == nullptr))
+    return AREAL_ERR_BAD_ARG;
+  if (score_mode == 2 && (!group_offsets || !group_rows || n_groups <= 0)) return AREAL_ERR_BAD_ARG;
+  if (score_mode == 2 && (mean_level < 0 || mean_level > 2 || std_level < 0 || std_level > 2)) return AREAL_ERR_BAD_ARG;
+  if (score_mode == 2 && (mean_level == LEVEL_BATCH || std_level == LEVEL_BATCH)) return AREAL_ERR_UNSUPPORTED;
+  if (!row_sums_fit(bs, L) || (score_mode == 2 && !scores_fit(bs))) return AREAL_ERR_UNSUPPORTED;
+  // with the log-probs rolled a thread reads its neighbour's token: not in place
+  if (roll_logp && logp == old_out) return AREAL_ERR_BAD_ARG;
+  a.p = PrepArgs{loss_mask, attn_mask, logp, ref_logp, rewards, L, roll_logp, estimator, apply_clamp,
+                 mask_no_eos_with_zero, ref_in_place, kl_ctl, lm_out, old_out, kl_out, nullptr, nullptr, tot_out,
+                 seqlens_out, no_eos_out};
+  a.g = GaeArgs{nullptr, values, nullptr, nullptr, nullptr, nullptr, bs * L, (int)bs, L, discount, gae_lambda, advantages,
+                returns, 1, row_stats};
+  a.score_mode = score_mode;
+  a.bias = bias; a.scaling = scaling; a.clip = clip;
+  a.score.x = rewards; a.score.n = bs; a.score.goff = group_offsets; a.score.grows = group_rows;
+  a.score.G = (int)n_groups; a.score.tail_group = tail_group; a.score.mean_level = mean_level;
+  a.score.std_level = std_level; a.score.unbiased = unbiased; a.score.eps = eps;
+  if (norm == nullptr) return AREAL_OK;
+  if (!norm->group_offsets || norm->n_groups <= 0 || norm->max_group_rows <= 0) return AREAL_ERR_BAD_ARG;
+  if (norm->mean_level < 0 || norm->mean_level > 2 || norm->std_level < 0 || norm->std_level > 2) return AREAL_ERR_BAD_ARG;
+  if (norm->mean_level == LEVEL_BATCH || norm->std_level == LEVEL_BATCH || norm->leave_one_out || norm->tail_group >= 0 ||
+      norm->n_groups > (1 << 30) || norm->max_group_rows > ADV_GROUP_ROWS || L > ADV_NORM_TILES * (int64_t)GAE_TILE)
+    return AREAL_ERR_UNSUPPORTED;
+  a.norm.goff = norm->group_offsets; a.norm.G = (int)norm->n_groups; a.norm.tail_group = -1;
+  a.norm.mean_level = norm->mean_level; a.norm.std_level = norm->std_level; a.norm.unbiased = norm->unbiased;
+  a.norm.eps = norm->eps;
+  return AREAL_OK;
+}
+template <bool NORM>
+int launch_adv_gae(const AdvGaeArgs& a, hipStream_t stream) {
+  const int64_t L = a.p.L;
+  const dim3 gr((unsigned)a.g.n_seqs), bl(GAE_THREADS);
+  const size_t lds = NORM ? (size_t)ceil_div_i64(L, GAE_TILE) * GAE_TILE * sizeof(float) : 0;
+  auto launch = [&](auto one_tile) {
+    constexpr bool ONE = decltype(one_tile)::value;
+    if (a.p.estimator == 1) hipLaunchKernelGGL((adv_gae_kernel<1, ONE, NORM>), gr, bl, lds, stream, a);
+    else if (a.p.estimator == 2) hipLaunchKernelGGL((adv_gae_kernel<2, ONE, NORM>), gr, bl, lds, stream, a);
+    else hipLaunchKernelGGL((adv_gae_kernel<3, ONE, NORM>), gr, bl, lds, stream, a);
+  };
+  if (L <= GAE_TILE) launch(std::true_type{});
+  else launch(std::false_type{});
+  AREAL_CHECK_LAUNCH();
+  return AREAL_OK;
+}
 
 }  // namespace
 
@@ -2859,40 +3105,52 @@ int areal_advantages_row_stats(const float* rewards, int score_mode, float bias,
                                float gae_lambda, float* lm_out, float* old_out, float* kl_out, float* tot_out,
                                int64_t* seqlens_out, uint8_t* no_eos_out, float* advantages, float* returns,
                                double* row_stats, hipStream_t stream) {
-  if (bs < 0 || L < 0 || estimator < 1 || estimator > 3 || score_mode < 0 || score_mode > 2) return AREAL_ERR_BAD_ARG;
-  if (bs == 0) return AREAL_OK;
-  if (L == 0) return AREAL_ERR_BAD_ARG;
-  if (!rewards || !loss_mask || !attn_mask || !logp || !lm_out || !old_out || !kl_out || !tot_out || !seqlens_out ||
-      !no_eos_out || !advantages || !returns || !row_stats)
-    return AREAL_ERR_BAD_ARG;
-  if (score_mode == 2 && (!group_offsets || !group_rows || n_groups <= 0)) return AREAL_ERR_BAD_ARG;
-  if (score_mode == 2 && (mean_level < 0 || mean_level > 2 || std_level < 0 || std_level > 2)) return AREAL_ERR_BAD_ARG;
-  if (score_mode == 2 && (mean_level == LEVEL_BATCH || std_level == LEVEL_BATCH)) return AREAL_ERR_UNSUPPORTED;
-  if (!row_sums_fit(bs, L) || (score_mode == 2 && !scores_fit(bs))) return AREAL_ERR_UNSUPPORTED;
-  // with the log-probs rolled a thread reads its neighbour's token: not in place
-  if (roll_logp && logp == old_out) return AREAL_ERR_BAD_ARG;
   AdvGaeArgs a{};
-  a.p = PrepArgs{loss_mask, attn_mask, logp, ref_logp, rewards, L, roll_logp, estimator, apply_clamp,
-                 mask_no_eos_with_zero, ref_in_place, kl_ctl, lm_out, old_out, kl_out, nullptr, nullptr, tot_out,
-                 seqlens_out, no_eos_out};
-  a.g = GaeArgs{nullptr, values, nullptr, nullptr, nullptr, nullptr, bs * L, (int)bs, L, discount, gae_lambda, advantages,
-                returns, 1, row_stats};
-  a.score_mode = score_mode;
-  a.bias = bias; a.scaling = scaling; a.clip = clip;
-  a.score.x = rewards; a.score.n = bs; a.score.goff = group_offsets; a.score.grows = group_rows;
-  a.score.G = (int)n_groups; a.score.tail_group = tail_group; a.score.mean_level = mean_level;
-  a.score.std_level = std_level; a.score.unbiased = unbiased; a.score.eps = eps;
-  const dim3 gr((unsigned)bs), bl(GAE_THREADS);
-  auto launch = [&](auto one_tile) {
-    constexpr bool ONE = decltype(one_tile)::value;
-    if (estimator == 1) hipLaunchKernelGGL((adv_gae_kernel<1, ONE>), gr, bl, 0, stream, a);
-    else if (estimator == 2) hipLaunchKernelGGL((adv_gae_kernel<2, ONE>), gr, bl, 0, stream, a);
-    else hipLaunchKernelGGL((adv_gae_kernel<3, ONE>), gr, bl, 0, stream, a);
-  };
-  if (L <= GAE_TILE) launch(std::true_type{});
-  else launch(std::false_type{});
-  AREAL_CHECK_LAUNCH();
-  return AREAL_OK;
+  const int rc = adv_gae_args(a, rewards, score_mode, bias, scaling, clip, group_offsets, group_rows, n_groups, tail_group,
+                              mean_level, std_level, unbiased, eps, loss_mask, attn_mask, logp, ref_logp, values, bs, L,
+                              roll_logp, estimator, apply_clamp, mask_no_eos_with_zero, ref_in_place, kl_ctl, discount,
+                              gae_lambda, lm_out, old_out, kl_out, tot_out, seqlens_out, no_eos_out, advantages, returns,
+                              row_stats, nullptr);
+  return rc != AREAL_OK || bs == 0 ? rc : launch_adv_gae<false>(a, stream);
+}
+
+// areal_advantages_row_stats with the advantages normalised within groups of rows in the same launch (see
+// adv_normalise_row; the same bits as areal_group_norm_from_row_stats on its sums). AREAL_ERR_UNSUPPORTED, besides
+// what areal_advantages_row_stats does not take: a level of the batch, leave one out, ungrouped rows, groups of more than
+// 64 rows, rows of more than 8192 slots, and a stream that is being captured (a graph's replays would all carry one
+// call's number, and find the sums of the replay before them).
+size_t areal_advantages_normalized_workspace_bytes(int64_t bs) { return bs > 0 ? (size_t)bs * 5 * sizeof(uint64_t) + 256 : 0; }
+
+int areal_advantages_normalized(const float* rewards, int score_mode, float bias, float scaling, float clip,
+                                const int64_t* group_offsets, const int64_t* group_rows, int64_t n_groups, int tail_group,
+                                int mean_level, int std_level, int unbiased, double eps, const uint8_t* loss_mask,
+                                const uint8_t* attn_mask, const float* logp, float* ref_logp, const float* values,
+                                int64_t bs, int64_t L, int roll_logp, int estimator, int apply_clamp,
+                                int mask_no_eos_with_zero, int ref_in_place, float kl_ctl, float discount,
+                                float gae_lambda, float* lm_out, float* old_out, float* kl_out, float* tot_out,
+                                int64_t* seqlens_out, uint8_t* no_eos_out, float* advantages, float* returns,
+                                const areal_group_norm_spec* norm, void* workspace, size_t workspace_bytes,
+                                hipStream_t stream) {
+  if (norm == nullptr) return AREAL_ERR_BAD_ARG;
+  AdvGaeArgs a{};
+  const int rc = adv_gae_args(a, rewards, score_mode, bias, scaling, clip, group_offsets, group_rows, n_groups, tail_group,
+                              mean_level, std_level, unbiased, eps, loss_mask, attn_mask, logp, ref_logp, values, bs, L,
+                              roll_logp, estimator, apply_clamp, mask_no_eos_with_zero, ref_in_place, kl_ctl, discount,
+                              gae_lambda, lm_out, old_out, kl_out, tot_out, seqlens_out, no_eos_out, advantages, returns,
+                              nullptr, norm);
+  if (rc != AREAL_OK || bs == 0) return rc;
+  if (workspace == nullptr || workspace_bytes < areal_advantages_normalized_workspace_bytes(bs)) return AREAL_ERR_WORKSPACE;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+    (void)hipGetLastError();
+    return AREAL_ERR_UNSUPPORTED;
+  }
+  if (capture != hipStreamCaptureStatusNone) return AREAL_ERR_UNSUPPORTED;
+  a.sums = (uint64_t*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
+  a.left = a.sums + 4 * bs;
+  a.call = next_call_number();
+  a.wait_ticks = norm->wait_us < 0 ? ADV_WAIT_TICKS : 100u * (unsigned)std::min(norm->wait_us, 1000);
+  return launch_adv_gae<true>(a, stream);
 }
 
 }  // extern "C"

@@ -863,9 +863,10 @@ Tensor f32(const Tensor& t) {
 
 // Reward scores and their normalisation, then areal_advantage_prep, over bs rows. `score`: the scores themselves when
 // `scored`, else the raw rewards. Returns (loss mask, old log-probs, kl rewards, total rewards, kl rewards
-// for GAE, outcome rewards (both turn mode only), no-eos mask, and with `gae` = (values, discount, lambda) where one
-// launch does it all: advantages, returns and their row sums).
-using GaeOptions = std::tuple<OptTensor, double, double>;
+// for GAE, outcome rewards (both turn mode only), no-eos mask, and with `gae` = (values, discount, lambda, normalisation
+// of the advantages) where one launch does it all: advantages, returns and their row sums, or no sums where
+// the advantages came out normalised).
+using GaeOptions = std::tuple<OptTensor, double, double, std::optional<NormTables>>;
 py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double scaling, double clip,
                          const std::optional<NormTables>& norm, const Tensor& loss_mask, const Tensor& attention_mask,
                          const Tensor& logp_src, const OptTensor& ref_logp, bool recompute, int estimator, bool clamp,
@@ -914,18 +915,34 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
   if (gae.has_value() && !turn_mode && bs > 0 && L > 0) {
     const Tensor v = f32(or_undefined(std::get<0>(*gae)));
     if (!v.defined() || (v.device() == lm.device() && v.sizes() == lm.sizes())) {
-      const Tensor adv = at::empty_like(lm), ret = at::empty_like(lm), sums = empty(lm, {5, bs}, at::kDouble);
-      auto one_launch = [&] {
+      const Tensor adv = at::empty_like(lm), ret = at::empty_like(lm);
+      Tensor sums;
+      auto launch = [&](auto entry, auto... behind) {
         return norm_args([&](const int64_t* off, const int64_t* rows, int64_t n, int tail, int mean_level,
                              int std_level, int unbiased, double eps) {
-          return areal_advantages_row_stats(
-              ptr<float>(sc), scored ? 0 : norm.has_value() ? 2 : 1, (float)bias, (float)scaling, (float)clip, off, rows,
-              n, tail, mean_level, std_level, unbiased, eps, ptr<uint8_t>(lmb), ptr<uint8_t>(amb), ptr<float>(logp),
-              ptr<float>(ref), ptr<float>(v), bs, L, recompute ? 0 : 1, estimator, clamp, no_eos_zero, ref_in_place,
-              (float)kl_ctl, (float)std::get<1>(*gae), (float)std::get<2>(*gae), ptr<float>(lm), ptr<float>(old),
-              ptr<float>(kl), ptr<float>(tot), ptr<int64_t>(seqlens), ptr<uint8_t>(no_eos), ptr<float>(adv),
-              ptr<float>(ret), ptr<double>(sums), stream);
+          return entry(ptr<float>(sc), scored ? 0 : norm.has_value() ? 2 : 1, (float)bias, (float)scaling, (float)clip,
+                       off, rows, n, tail, mean_level, std_level, unbiased, eps, ptr<uint8_t>(lmb), ptr<uint8_t>(amb),
+                       ptr<float>(logp), ptr<float>(ref), ptr<float>(v), bs, L, recompute ? 0 : 1, estimator, clamp,
+                       no_eos_zero, ref_in_place, (float)kl_ctl, (float)std::get<1>(*gae), (float)std::get<2>(*gae),
+                       ptr<float>(lm), ptr<float>(old), ptr<float>(kl), ptr<float>(tot), ptr<int64_t>(seqlens),
+                       ptr<uint8_t>(no_eos), ptr<float>(adv), ptr<float>(ret), behind..., stream);
         });
+      };
+      auto one_launch = [&] {
+        const auto& adv_norm = std::get<3>(*gae);
+        if (adv_norm.has_value()) {
+          const auto& [off, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = *adv_norm;
+          const areal_group_norm_spec spec{ptr<int64_t>(off), rows.numel(), longest / L, tail, mean_level, std_level,
+                                           loo, unbiased, -1, eps};
+          const size_t bytes = areal_advantages_normalized_workspace_bytes(bs);
+          const Tensor ws = workspace(lm, bytes);
+          const int rc = launch(areal_advantages_normalized, &spec, ptr<void>(ws), bytes);
+          if (rc != AREAL_ERR_UNSUPPORTED) return rc;
+        }
+        sums = empty(lm, {5, bs}, at::kDouble);
+        const int rc = launch(areal_advantages_row_stats, ptr<double>(sums));
+        if (rc != AREAL_OK) sums = Tensor();
+        return rc;
       };
       int rc = one_launch();
       if (rc == AREAL_ERR_UNSUPPORTED && !scored) {  // it may take the scores ready-made
@@ -935,7 +952,7 @@ py::tuple advantage_prep(const Tensor& score, bool scored, double bias, double s
       if (rc != AREAL_ERR_UNSUPPORTED) {
         check(rc, "areal_advantages_row_stats");
         return py::make_tuple(lm, old.view(logp_src.sizes()), kl, tot, OptTensor(), OptTensor(), no_eos,
-                              py::make_tuple(adv, ret, sums));
+                              py::make_tuple(adv, ret, opt(sums)));
       }
     }
   }

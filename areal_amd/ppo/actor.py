@@ -652,7 +652,8 @@ def compute_advantages(
         one_pass and not turn_mode and gae_lambda_fn is None and logp_src.ndim == 2
         and isinstance(gae_lambda, (int, float)) and not isinstance(gae_lambda, bool) and math.isfinite(gae_lambda)
     ):
-        gae_options = (values, discount, float(gae_lambda))
+        gae_options = (values, discount, float(gae_lambda),
+                       adv_norm._tables(*logp_src.shape, group_sizes, logp_src.device) if logp_src.numel() > 0 else None)
     (
         loss_mask, old_logp, kl_rewards, tot_rewards, gae_kl_rewards, gae_outcome_rewards, seq_no_eos_mask, scanned,
     ) = (
@@ -699,9 +700,12 @@ def compute_advantages(
             )
         if fused is not None:
             advantages, returns, row_stats, mask_f32 = fused
-            normed = adv_norm.from_row_stats(advantages, mask_f32, row_stats, group_sizes=group_sizes)
-            if normed is not None:
-                advantages, adv_norm = normed, None
+            if row_stats is None:  # normalised in that launch
+                adv_norm = None
+            else:
+                normed = adv_norm.from_row_stats(advantages, mask_f32, row_stats, group_sizes=group_sizes)
+                if normed is not None:
+                    advantages, adv_norm = normed, None
         else:
             advantages, returns = _compute_token_level_gae(
                 rewards=rewards,

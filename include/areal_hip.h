@@ -531,6 +531,33 @@ int areal_advantages_row_stats(const float* rewards, int score_mode, float bias,
                                float* advantages, float* returns, double* row_stats,
                                areal_stream_t stream);
 
+/* Normalisation of the advantages within groups of whole rows: group_offsets [n_groups + 1] element offsets
+ * (multiples of the row length, a partition of the batch), the rows of the longest group, levels 0 (none) or 2
+ * (group). wait_us: how long a row waits for its group before it leaves its normalisation to another (at most 1000,
+ * negative: 200). */
+typedef struct {
+  const int64_t* group_offsets;
+  int64_t n_groups, max_group_rows;
+  int tail_group, mean_level, std_level, leave_one_out, unbiased, wait_us;
+  double eps;
+} areal_group_norm_spec;
+
+/* areal_advantages_row_stats whose advantages come out normalised, in one launch. AREAL_ERR_UNSUPPORTED also for
+ * a level of the batch, leave one out, ungrouped rows (tail_group >= 0), groups of more than 64 rows, rows of
+ * more than 8192 slots and a stream that is being captured. */
+size_t areal_advantages_normalized_workspace_bytes(int64_t bs);
+int areal_advantages_normalized(const float* rewards, int score_mode, float bias, float scaling, float clip,
+                                const int64_t* group_offsets, const int64_t* group_rows,
+                                int64_t n_groups, int tail_group, int mean_level, int std_level,
+                                int unbiased, double eps, const uint8_t* loss_mask,
+                                const uint8_t* attn_mask, const float* logp, float* ref_logp,
+                                const float* values, int64_t bs, int64_t L, int roll_logp, int estimator,
+                                int apply_clamp, int mask_no_eos_with_zero, int ref_in_place, float kl_ctl,
+                                float discount, float gae_lambda, float* lm_out, float* old_out,
+                                float* kl_out, float* tot_out, int64_t* seqlens_out, uint8_t* no_eos_out,
+                                float* advantages, float* returns, const areal_group_norm_spec* norm,
+                                void* workspace, size_t workspace_bytes, areal_stream_t stream);
+
 /* masked_normalization with dim = the trailing dimensions (areal/utils/functional/functional.py:16-53,
  * the `dim` argument): x, mask (NULL allowed) and out are [rows, cols]; every row is whitened with
  * its own masked mean and variance. */
