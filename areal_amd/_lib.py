@@ -126,6 +126,11 @@ SIGNATURES: dict[str, tuple] = {
         [P, I, F, F, F, P, P, I64, I, I, I, I, D, P, P, P, P, P, I64, I64, I, I, I, I, I, F, F, F, P, P, P, P, P, P, P, P,
          P, P],
     ),
+    "areal_gae_packed_normalized_workspace_bytes": (SZ, [I64, I64]),
+    "areal_gae_packed_normalized_ex": (
+        I,
+        [P, P, P, P, P, P, I64, I64, F, F, P, P, I64, I64, I, I, I, I, D, I, P, P, P, P, SZ, P],
+    ),
     "areal_advantages_normalized_workspace_bytes": (SZ, [I64]),
     "areal_advantages_normalized": (
         I,

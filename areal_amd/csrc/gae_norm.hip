@@ -127,6 +127,77 @@ DEVI void block_sum_n(double (&v)[N], double* smem /* [4][N] */) {
   }
 }
 
+// ---- Sums handed from block to block inside a launch (adv_normalise_row, gae_tile_normalise): sealed words, N numbers
+// and a check word made of them and the call's number, and a flag per entry, the call's number again, stored when they have
+// left. All go out and come in as agent-scope atomics (past the XCD's own L2); flags lie next to each other, so that
+// looking again costs a line or two (with the words themselves looked at, 900 waiting blocks of 14 entries each slowed
+// down the ones they waited for: packed GAE
+// of 1.79 Mi tokens 31.4 -> 29.0 us). Whoever reads words that fit has
+// all of them, whatever the memory held before (a chance of 2^-64 an entry otherwise), and nothing has to be cleared.
+// Every word goes through a mix of its own: sums are doubles with few bits set (a count of 512 has one above its
+// exponent's), and a sum of their products with odd numbers took entries for whole of which two counts were missing.
+template <int N>
+DEVI uint64_t sums_seal(uint64_t call, const uint64_t (&w)[N]) {
+  uint64_t h = call;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    h ^= w[k];
+    h = (h ^ (h >> 32)) * 0xbf58476d1ce4e5b9ull;
+    h = (h ^ (h >> 29)) * 0x94d049bb133111ebull;
+  }
+  return h ^ (h >> 32);
+}
+template <int N>
+DEVI void publish_sums(uint64_t* to, uint64_t* flag, uint64_t call, const double (&s)[N]) {  // by one thread
+  uint64_t w[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    w[k] = __builtin_bit_cast(uint64_t, s[k]);
+    __hip_atomic_store(to + k, w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __hip_atomic_store(to + N, sums_seal(call, w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the seal is what the reader relies on)
+  __hip_atomic_store(flag, call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The sums of n entries PITCH words apart, added up by a whole wave: lane i takes every 64th from the i-th on, then the
+// wave's sum. False when they were not all there at `deadline`.
+template <int PITCH, int N>
+DEVI bool gather_sums(const uint64_t* from, const uint64_t* flags, int n, uint64_t call, uint64_t deadline, double (&s)[N]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < N; ++k) s[k] = 0.0;
+  for (int i = lane; i - lane < n; i += 64) {
+    bool have = i >= n;
+    for (;;) {
+      if (!have && __hip_atomic_load(flags + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == call) {
+        const uint64_t* const entry = from + (int64_t)PITCH * i;
+        uint64_t w[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) w[k] = __hip_atomic_load(entry + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t seal = __hip_atomic_load(entry + N, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        have = seal == sums_seal(call, w);
+        if (have) {
+#pragma unroll
+          for (int k = 0; k < N; ++k) s[k] += __builtin_bit_cast(double, w[k]);
+        }
+      }
+      if (__builtin_amdgcn_ballot_w64(!have) == 0) break;
+      if (wall_clock64() >= deadline) return false;
+      __builtin_amdgcn_s_sleep(4);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) s[k] = wave_sum(s[k]);
+  return true;
+}
+DEVI bool note_left(const uint64_t* left, uint64_t call) {
+  return __hip_atomic_load(left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == call;
+}
+DEVI void leave_note(uint64_t* left, uint64_t call) { atomicExch((unsigned long long*)left, (unsigned long long)call); }
+DEVI bool take_note(uint64_t* left, uint64_t call) {
+  return atomicCAS((unsigned long long*)left, (unsigned long long)call, (unsigned long long)~call) == call;
+}
+
 struct GaeArgs {
   const float* rewards;
   const float* values;
@@ -749,17 +820,16 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
 // Single-pass GAE for packed sequences of ordinary length, one block per tile. What enters the
 // tile from its right is the state of the sequence that crosses the tile's right edge, and it
 // depends only on that sequence's tokens beyond the edge: the block reads them too (rewards,
-// values, mask; nothing written), one tile's worth at a time, and composes their maps onto the
-// zero state; a wave whose 512 tokens lie beyond the sequence's end skips its share. No block
-// waits for another, and the remainder is read once per tile of the sequence, from L2 mostly:
+// values, mask; nothing written), a run of chunks of 512 per wave, the next chunk on its way while one is
+// composed, and applies the waves' maps to the zero state (512 x 8192 tokens 59.9 -> 54.3 us, 64 x 8192 30.7 -> 25.8
+// against steps of a whole tile with two barriers each). No block waits for another, and the remainder is read once per tile of the sequence, from L2 mostly:
 // the blocks of an XCD are neighbours in the array. Against blocks that walk the sequences they
 // own tile by tile, carrying the state (the padded-row kernel above, which also took cu_seqlens
 // once): faster on 64 x 16384 tokens and on 4 x 32768, where a walking block has 16 tiles in a row.
 // The kernel is bound by vector instruction issue (about 1150 vector and 250 scalar instructions
 // per wave and tile on 1024 sequences of mean length 1760) with four blocks resident per CU, so
-// that all blocks of a 1.8 M-token batch run at once; that leaves 128 registers. Two remainder
-// tiles per round need 148 and spill 20 of them into scratch memory: 19.9 against 15.4 us.
-constexpr int GAE_CARRY_BATCH = 1;
+// that all blocks of a 1.8 M-token batch run at once; that leaves 128 registers.
+constexpr int GAE_CHUNK = 64 * GAE_ITEMS;  // tokens of a wave's step through the crossing sequence
 constexpr int GAE_CU_LDS = 16 * GAE_THREADS;  // entries of cu_seqlens the block can hold (>= TILE + 2)
 
 // Groups of a tile for GaeArgs::seg_stats: those of the tile's first and last token and of the next
@@ -793,27 +863,30 @@ DEVI GaeTileGroups gae_tile_groups(const GaeArgs& g, int64_t lo, const int* s_gr
   return r;
 }
 
+// Where the k-th group of the tile lies, relative to the tile's first token.
+// (selects, not an index: an indexed register array would live in scratch memory)
+DEVI void tile_group_bounds(const GaeArgs& g, const GaeTileGroups& tg, int64_t lo, int k, int64_t& b0, int64_t& b1) {
+  b0 = k == 0 ? tg.b[0] : k == 1 ? tg.b[1] : k == 2 ? tg.b[2] : group_offsets(g)[tg.g_first + k] - lo;
+  b1 = k == 0 ? tg.b[1] : k == 1 ? tg.b[2] : group_offsets(g)[tg.g_first + k + 1] - lo;
+}
 // The five masked sums of the tile's advantages per group and wave (GaeArgs::seg_stats): x = oa
 // (zero for tokens outside every sequence), m = the thread's 8 mask values (zero beyond the
-// array). Every wave writes its own entry, so no wave waits for another. Every thread of the
-// block calls it.
-DEVI void gae_tile_group_stats(const GaeArgs& g, int64_t tile, int64_t lo, int64_t hi,
-                               const GaeTileGroups& tg, const float (&oa)[GAE_ITEMS],
-                               const float (&ms)[GAE_ITEMS]) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t rel = (int64_t)tid * GAE_ITEMS;  // the thread's first token relative to lo
-  const int64_t st = GAE_SEG_WAVES * g.seg_slots;
+// array). put(group, sums) gets each wave's own, in every lane: no wave waits for another. Groups [g_begin, g_end) of
+// the tile; every thread of the block calls it.
+template <class Put>
+DEVI void gae_tile_group_sums(const GaeArgs& g, int64_t lo, const GaeTileGroups& tg, int g_begin, int g_end,
+                              const float (&oa)[GAE_ITEMS], const float (&ms)[GAE_ITEMS], const Put& put) {
+  const int64_t rel = (int64_t)threadIdx.x * GAE_ITEMS;  // the thread's first token relative to lo
   // the usual 0/1 mask (decided per wave): sum m^2 = sum m, sum m^2 x = sum m x, and sum m is a count
   bool other = false;
 #pragma unroll
   for (int i = 0; i < GAE_ITEMS; ++i) other |= ms[i] != 0.f && ms[i] != 1.f;
   const bool binary = __builtin_amdgcn_ballot_w64(other) == 0;
-  for (int gi = tg.g_first; gi <= tg.g_last; ++gi) {
-    const int k = gi - tg.g_first;
+  for (int gi = g_begin; gi < g_end; ++gi) {
     // the group's bounds relative to the thread's tokens, clamped to them
-    // (selects, not an index: an indexed register array would live in scratch memory)
-    const int64_t d0 = (k == 0 ? tg.b[0] : k == 1 ? tg.b[1] : k == 2 ? tg.b[2] : group_offsets(g)[gi] - lo) - rel;
-    const int64_t d1 = (k == 0 ? tg.b[1] : k == 1 ? tg.b[2] : group_offsets(g)[gi + 1] - lo) - rel;
+    int64_t d0, d1;
+    tile_group_bounds(g, tg, lo, gi - tg.g_first, d0, d1);
+    d0 -= rel; d1 -= rel;
     const int i0 = d0 <= 0 ? 0 : (d0 >= GAE_ITEMS ? GAE_ITEMS : (int)d0);
     const int i1 = d1 <= 0 ? 0 : (d1 >= GAE_ITEMS ? GAE_ITEMS : (int)d1);
     double rs[5];
@@ -845,11 +918,20 @@ DEVI void gae_tile_group_stats(const GaeArgs& g, int64_t tile, int64_t lo, int64
 #pragma unroll
       for (int q = 0; q < 5; ++q) rs[q] = wave_sum(rs[q]);
     }
+    put(gi, rs);
+  }
+}
+DEVI void gae_tile_group_stats(const GaeArgs& g, int64_t tile, int64_t lo, int64_t hi,
+                               const GaeTileGroups& tg, const float (&oa)[GAE_ITEMS],
+                               const float (&ms)[GAE_ITEMS]) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t st = GAE_SEG_WAVES * g.seg_slots;
+  gae_tile_group_sums(g, lo, tg, tg.g_first, tg.g_last + 1, oa, ms, [&](int gi, const double (&rs)[5]) {
     if (lane == 0) {
 #pragma unroll
       for (int q = 0; q < 5; ++q) g.seg_stats[(int64_t)q * st + GAE_SEG_WAVES * (tile + gi) + wave] = rs[q];
     }
-  }
+  });
   // slots that no segment maps to: before the first tile's first group, between this tile's last
   // group and the next tile's first, and after the last tile's last group
   const int64_t z_lo = tile == 0 ? 0 : tile + tg.g_first;
@@ -862,13 +944,13 @@ DEVI void gae_tile_group_stats(const GaeArgs& g, int64_t tile, int64_t lo, int64
   }
 }
 
-// STATS: also leaves the per-(tile, group) sums of GaeArgs::seg_stats.
-template <bool LAMBDAS, bool STATS>
-__global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
+// STATS: tail(tile, lo, hi, groups of the tile, advantages, masks) gets what the group sums are made of.
+template <bool LAMBDAS, bool STATS, class Tail>
+DEVI void gae_tile(const GaeArgs& g, const Tail& tail) {
   __shared__ MapF smem[GAE_THREADS / 64];
   __shared__ int s_grp[3];
   __shared__ MapF all[GAE_THREADS];
-  __shared__ MapF s_part[GAE_THREADS / 64][GAE_CARRY_BATCH];
+  __shared__ Map s_part[GAE_SEG_WAVES];
   __shared__ int32_t s_cu[GAE_CU_LDS];
   __shared__ int s_own[2];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -916,7 +998,7 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
     if constexpr (STATS) {
       const float zero[GAE_ITEMS] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       __syncthreads();
-      gae_tile_group_stats(g, tile, lo, hi, gae_tile_groups(g, lo, s_grp), zero, ms);
+      tail(tile, lo, hi, gae_tile_groups(g, lo, s_grp), zero, ms);
     }
     return;
   }
@@ -959,92 +1041,90 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
   GaeTileGroups tg;
   if constexpr (STATS) tg = gae_tile_groups(g, lo, s_grp);  // a barrier has passed since the search
 
-  // the crossing sequence's tokens [t_end, e): in whole tiles from t_end (a multiple of the tile
-  // when e > t_end), the rightmost batch first
+  // the crossing sequence's tokens [t_end, e), from t_end (a multiple of the tile when e > t_end)
   double A0 = 0.0, nv0 = 0.0;
   const int64_t e = (int64_t)cu_own[n_own];
   if (e > t_end) {
     const float gam = g.discount;
     const float c = gam * (LAMBDAS ? g.lam_seq[s_last] : g.lam);
     const bool boot = g.no_eos != nullptr && g.no_eos[s_last] != 0;
-    const int64_t n_right = (e - t_end + GAE_TILE - 1) / GAE_TILE;
     // (without values the mask is read in their place and dropped: no branch between the loads)
     const float* const values = g.values != nullptr ? g.values : g.mask;
-    for (int64_t j = n_right; j > 0; j -= GAE_CARRY_BATCH) {
-      const int64_t j0 = j > GAE_CARRY_BATCH ? j - GAE_CARRY_BATCH : 0;
-      float rw[GAE_CARRY_BATCH][GAE_ITEMS], v[GAE_CARRY_BATCH][GAE_ITEMS], ms[GAE_CARRY_BATCH][GAE_ITEMS];
+    // Runs of whole chunks of 512 tokens, one run per wave: each wave composes its own from the right, the next chunk
+    // on its way, and the block meets once at the end.
+    const int64_t chunks = (e - t_end + GAE_CHUNK - 1) / GAE_CHUNK, per_wave = (chunks + GAE_SEG_WAVES - 1) / GAE_SEG_WAVES;
+    const int64_t c_lo = wave * per_wave, c_hi = c_lo + per_wave < chunks ? c_lo + per_wave : chunks;
+    float crw[GAE_ITEMS], cv[GAE_ITEMS], cms[GAE_ITEMS];
+    auto fetch = [&](int64_t chunk) {
+      const int64_t t0 = t_end + chunk * GAE_CHUNK + (int64_t)lane * GAE_ITEMS;
+      if (t0 + GAE_ITEMS <= g.n) {
 #pragma unroll
-      for (int k = 0; k < GAE_CARRY_BATCH; ++k) {
-        const int64_t t0 = t_end + (j0 + k) * GAE_TILE + (int64_t)tid * GAE_ITEMS;
-        const bool live = j0 + k < j && t0 < e;
-        if (live && t0 + GAE_ITEMS <= g.n) {
+        for (int q = 0; q < GAE_ITEMS / 4; ++q) {
+          const f32x4 a = *(const f32x4*)(g.rewards + t0 + 4 * q);
+          const f32x4 b = *(const f32x4*)(values + t0 + 4 * q);
+          const f32x4 m = *(const f32x4*)(g.mask + t0 + 4 * q);
 #pragma unroll
-          for (int q = 0; q < GAE_ITEMS / 4; ++q) {
-            const f32x4 a = *(const f32x4*)(g.rewards + t0 + 4 * q);
-            const f32x4 b = *(const f32x4*)(values + t0 + 4 * q);
-            const f32x4 m = *(const f32x4*)(g.mask + t0 + 4 * q);
-#pragma unroll
-            for (int x = 0; x < 4; ++x) { rw[k][4 * q + x] = a[x]; v[k][4 * q + x] = b[x]; ms[k][4 * q + x] = m[x]; }
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < GAE_ITEMS; ++i) {
-            const bool in = live && t0 + i < g.n;
-            rw[k][i] = in ? g.rewards[t0 + i] : 0.f;
-            v[k][i] = in ? values[t0 + i] : 0.f;
-            ms[k][i] = in ? g.mask[t0 + i] : 0.f;
-          }
+          for (int x = 0; x < 4; ++x) { crw[4 * q + x] = a[x]; cv[4 * q + x] = b[x]; cms[4 * q + x] = m[x]; }
         }
-        if (g.values == nullptr) {
+      } else {
 #pragma unroll
-          for (int i = 0; i < GAE_ITEMS; ++i) v[k][i] = 0.f;
+        for (int i = 0; i < GAE_ITEMS; ++i) {
+          const bool in = t0 + i < g.n;
+          crw[i] = in ? g.rewards[t0 + i] : 0.f;
+          cv[i] = in ? values[t0 + i] : 0.f;
+          cms[i] = in ? g.mask[t0 + i] : 0.f;
         }
       }
-      MapF part[GAE_CARRY_BATCH];
+      if (g.values == nullptr) {
 #pragma unroll
-      for (int k = 0; k < GAE_CARRY_BATCH; ++k) {
-        const int64_t t0 = t_end + (j0 + k) * GAE_TILE + (int64_t)tid * GAE_ITEMS;
-        MapF acc = map_identity_t<float>();
-        part[k] = acc;
-        // a wave whose 512 tokens all lie beyond the sequence contributes the identity
-        if (!(j0 + k < j && t0 - (int64_t)lane * GAE_ITEMS < e)) continue;
-#pragma unroll
-        for (int i = GAE_ITEMS - 1; i >= 0; --i) {
-          const int64_t t = t0 + i;
-          // beyond the sequence (or the batch): identity; its last token: the constant map
-          const float m = (j0 + k < j && t < e) ? ms[k][i] : 0.f;
-          MapF f;
-          f.a11 = fmaf(c, m, 1.f - m);
-          f.a12 = gam * m;
-          f.a22 = 1.f - m;
-          f.b1 = (rw[k][i] - v[k][i]) * m;
-          f.b2 = v[k][i] * m;
-          if (j0 + k < j && t == e - 1) f = MapF{0.f, 0.f, 0.f, 0.f, boot ? v[k][i] : 0.f};
-          acc = compose(f, acc);
-        }
-        part[k] = wave_total_map(acc);
+        for (int i = 0; i < GAE_ITEMS; ++i) cv[i] = 0.f;
       }
-      __syncthreads();  // the previous batch's readers are done
-      if (lane == 0) {
+    };
+    Map run = map_identity();
+    if (c_lo < c_hi) fetch(c_hi - 1);
+    for (int64_t chunk = c_hi - 1; chunk >= c_lo; --chunk) {
+      const int64_t t0 = t_end + chunk * GAE_CHUNK + (int64_t)lane * GAE_ITEMS;
+      const int64_t left = e - t0;  // the thread's tokens of the sequence
+      float xr[GAE_ITEMS], xv[GAE_ITEMS], xm[GAE_ITEMS];
 #pragma unroll
-        for (int k = 0; k < GAE_CARRY_BATCH; ++k) s_part[wave][k] = part[k];
+      for (int i = 0; i < GAE_ITEMS; ++i) { xr[i] = crw[i]; xv[i] = cv[i]; xm[i] = cms[i]; }
+      if (chunk > c_lo) fetch(chunk - 1);
+      MapF acc = map_identity_t<float>();
+#pragma unroll
+      for (int i = GAE_ITEMS - 1; i >= 0; --i) {
+        // beyond the sequence (or the batch): identity; its last token: the constant map
+        const float m = i < left ? xm[i] : 0.f;
+        MapF f;
+        f.a11 = fmaf(c, m, 1.f - m);
+        f.a12 = gam * m;
+        f.a22 = 1.f - m;
+        f.b1 = (xr[i] - xv[i]) * m;
+        f.b2 = xv[i] * m;
+        if (i == left - 1) f = MapF{0.f, 0.f, 0.f, 0.f, boot ? xv[i] : 0.f};
+        acc = compose(f, acc);
       }
-      __syncthreads();
+      const MapF part = wave_total_map(acc);
+      run = compose(Map{(double)part.a11, (double)part.a12, (double)part.a22, (double)part.b1, (double)part.b2}, run);
+    }
+    if (lane == 0) s_part[wave] = run;
+    __syncthreads();
 #pragma unroll
-      for (int k = GAE_CARRY_BATCH - 1; k >= 0; --k) {
-        if (j0 + k >= j) continue;
-        MapF tot = s_part[GAE_THREADS / 64 - 1][k];
-#pragma unroll
-        for (int w = GAE_THREADS / 64 - 2; w >= 0; --w) tot = compose(s_part[w][k], tot);
-        const double A1 = fma((double)tot.a11, A0, fma((double)tot.a12, nv0, (double)tot.b1));
-        const double nv1 = fma((double)tot.a22, nv0, (double)tot.b2);
-        A0 = A1; nv0 = nv1;
-      }
+    for (int w = GAE_SEG_WAVES - 1; w >= 0; --w) {
+      const Map m = s_part[w];
+      const double A1 = fma(m.a11, A0, fma(m.a12, nv0, m.b1));
+      nv0 = fma(m.a22, nv0, m.b2);
+      A0 = A1;
     }
   }
   float oa[GAE_ITEMS];
   gae_one_tile<GAE_LAYOUT_CU, LAMBDAS>(g, tile, t_begin, t_end, s_first, n_own, cu_own, A0, nv0, smem, all, rw, v, ms, oa);
-  if constexpr (STATS) gae_tile_group_stats(g, tile, lo, hi, tg, oa, ms);
+  if constexpr (STATS) tail(tile, lo, hi, tg, oa, ms);
+}
+// STATS: also leaves the per-(tile, group) sums of GaeArgs::seg_stats.
+template <bool LAMBDAS, bool STATS>
+__global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
+  gae_tile<LAMBDAS, STATS>(g, [&](int64_t tile, int64_t lo, int64_t hi, const GaeTileGroups& tg, const float (&oa)[GAE_ITEMS],
+                                  const float (&ms)[GAE_ITEMS]) { gae_tile_group_stats(g, tile, lo, hi, tg, oa, ms); });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1299,6 +1379,141 @@ DEVI float norm_one(const NormParams& p, float x, float m, bool has_mask) {
   float c = x - (float)p.mean;
   if (has_mask) c = c * m;
   return c / ((float)p.std_d + (float)p.eps);
+}
+
+// ---- Packed GAE and the normalisation of its advantages within groups of sequences in one launch: a tile's block keeps its
+// advantages in registers, publishes its sums per group and waits for those of the other tiles of its groups, each
+// wave for another group. A launch of its own read advantages and masks back and searched the groups again, several loads
+// that wait for each other. Both forms, GAE included, us: 1024 sequences of 1750 tokens in groups of 16 32.0 -> 27.8, 4096 of
+// 100 in fours (five groups to a tile) 55.9 -> 34.2, 64 of 300 22.2 -> 16.1, 64 of 8192 in eights 35.5 -> 32.2. The rule for
+// the sizes of groups stands at areal_gae_packed_normalized_ex.
+// No wait is unbounded, as with adv_normalise_row: when the time is up, the block leaves a note for the (tile, group)
+// segment, whose advantages are in memory anyway, and a wave that finds all sums of a group looks for notes of its tiles and
+// takes them. Leaving a note is followed by another look at the sums, publishing comes before the look for notes.
+constexpr int SUMS_PITCH = 8;  // words an entry: five sums, their seal, a line of 64 bytes to itself
+struct GaeNormArgs {
+  GaeArgs g;
+  NormArgs norm;              // levels; out: the normalised advantages
+  uint64_t *sums, *flags, *left;  // [seg_slots][SUMS_PITCH] and twice [seg_slots] in the workspace
+  uint64_t call;
+  unsigned wait_ticks;
+};
+DEVI void gae_tile_normalise(const GaeNormArgs& a, int64_t tile, int64_t lo, int64_t hi, const GaeTileGroups& tg,
+                             const float (&oa)[GAE_ITEMS], const float (&ms)[GAE_ITEMS]) {
+  __shared__ double s_sum[GAE_SEG_WAVES][GAE_SEG_WAVES][5];  // [group][wave]
+  __shared__ float s_mean[GAE_SEG_WAVES], s_den[GAE_SEG_WAVES];
+  __shared__ int s_lo[GAE_SEG_WAVES], s_hi[GAE_SEG_WAVES], s_state[GAE_SEG_WAVES];
+  constexpr int NONE = 0, READY = 1, LEFT = 2;
+  const GaeArgs& g = a.g;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, rel = tid * GAE_ITEMS;
+  auto entry = [&](int64_t k, int gi) { return a.sums + SUMS_PITCH * (k + gi); };
+  for (int gb = tg.g_first; gb <= tg.g_last; gb += GAE_SEG_WAVES) {
+    const int g_end = gb + GAE_SEG_WAVES <= tg.g_last + 1 ? gb + GAE_SEG_WAVES : tg.g_last + 1;
+    gae_tile_group_sums(g, lo, tg, gb, g_end, oa, ms, [&](int gi, const double (&rs)[5]) {
+      if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) s_sum[gi - gb][wave][k] = rs[k];
+      }
+    });
+    __syncthreads();
+    if (lane == 0 && gb + wave < g_end) {
+      double rs[5];
+#pragma unroll
+      for (int k = 0; k < 5; ++k)
+        rs[k] = (s_sum[wave][0][k] + s_sum[wave][1][k]) + (s_sum[wave][2][k] + s_sum[wave][3][k]);
+      publish_sums(entry(tile, gb + wave), a.flags + tile + gb + wave, a.call, rs);
+    }
+    if (gb + GAE_SEG_WAVES <= tg.g_last) __syncthreads();
+  }
+  const uint64_t deadline = wall_clock64() + a.wait_ticks;
+  float r[GAE_ITEMS];
+  unsigned keep = 0;  // tokens of groups that were left
+#pragma unroll
+  for (int i = 0; i < GAE_ITEMS; ++i) r[i] = 0.f;  // (a token of no group is one of no sequence)
+  for (int gb = tg.g_first; gb <= tg.g_last; gb += GAE_SEG_WAVES) {
+    const int gi = gb + wave;
+    int64_t b0 = 0, b1 = 0;  // the wave's group, relative to the tile
+    if (gi <= tg.g_last) tile_group_bounds(g, tg, lo, gi - tg.g_first, b0, b1);
+    const bool mine = b0 < b1;
+    const int64_t rows = mine ? a.norm.grows[gi] : 0;
+    const int64_t k0 = (lo + b0) / GAE_TILE, k1 = (lo + b1 - 1) / GAE_TILE;
+    float mean = 0.f, den = 1.f;
+    auto gather = [&](uint64_t until) {
+      double s[5], v[10];
+      if (!gather_sums<SUMS_PITCH>(entry(k0, gi), a.flags + k0 + gi, (int)(k1 - k0 + 1), a.call, until, s)) return false;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) { v[k] = s[k]; v[5 + k] = 0.0; }
+      const NormParams np = norm_params(a.norm, gi, v, [&] { return rows; });
+      mean = (float)np.mean;
+      den = (float)np.std_d + (float)np.eps;
+      return true;
+    };
+    auto take_notes = [&] {  // of the wave's group
+      for (int64_t kb = k0; kb <= k1; kb += 64) {
+        uint64_t notes = __builtin_amdgcn_ballot_w64(kb + lane <= k1 && note_left(a.left + kb + lane + gi, a.call));
+        for (; notes != 0; notes &= notes - 1) {
+          const int64_t k = kb + __builtin_ctzll(notes);
+          int got = 0;
+          if (lane == 0) got = take_note(a.left + k + gi, a.call) ? 1 : 0;
+          if (__builtin_amdgcn_readfirstlane(got) == 0) continue;  // somebody else's
+          __threadfence();
+          const int64_t s0 = k * GAE_TILE > lo + b0 ? k * GAE_TILE : lo + b0;
+          const int64_t s1 = (k + 1) * GAE_TILE < lo + b1 ? (k + 1) * GAE_TILE : lo + b1;
+          for (int64_t t = s0 + lane; t < s1; t += 64) {
+            const float c = (g.adv[t] - mean) * g.mask[t];
+            a.norm.out[t] = c / den;
+          }
+        }
+      }
+    };
+    const bool ready = mine && gather(deadline);
+    if (lane == 0) {
+      s_mean[wave] = mean;
+      s_den[wave] = den;
+      s_lo[wave] = (int)(b0 > 0 ? b0 : 0);
+      s_hi[wave] = (int)(b1 < GAE_TILE ? b1 : GAE_TILE);
+      s_state[wave] = !mine ? NONE : ready ? READY : LEFT;
+    }
+    __syncthreads();
+    bool left = false;
+    for (int w = 0; w < GAE_SEG_WAVES; ++w) {
+      if (s_state[w] == NONE) continue;
+      const float wm = s_mean[w], wd = s_den[w];
+      const int i0 = s_lo[w] - rel, i1 = s_hi[w] - rel;
+      left |= s_state[w] == LEFT;
+#pragma unroll
+      for (int i = 0; i < GAE_ITEMS; ++i) {
+        if (i < i0 || i >= i1) continue;
+        if (s_state[w] == LEFT) keep |= 1u << i;
+        else r[i] = (oa[i] - wm) * ms[i] / wd;
+      }
+    }
+    __syncthreads();
+    if (ready) take_notes();
+    if (left) {
+      __threadfence();  // the block's advantages are in memory
+      __syncthreads();
+      if (mine && !ready) {
+        if (lane == 0) leave_note(a.left + tile + gi, a.call);
+        if (gather(0)) take_notes();
+      }
+    }
+  }
+  const int64_t t0 = lo + rel;
+  if (keep == 0 && t0 + GAE_ITEMS <= hi) {
+#pragma unroll
+    for (int q = 0; q < GAE_ITEMS / 4; ++q)
+      *(f32x4_any*)(a.norm.out + t0 + 4 * q) = f32x4{r[4 * q], r[4 * q + 1], r[4 * q + 2], r[4 * q + 3]};
+  } else {
+#pragma unroll
+    for (int i = 0; i < GAE_ITEMS; ++i)
+      if (t0 + i < hi && ((keep >> i) & 1u) == 0) a.norm.out[t0 + i] = r[i];
+  }
+}
+template <bool LAMBDAS>
+__global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_norm_kernel(GaeNormArgs a) {
+  gae_tile<LAMBDAS, true>(a.g, [&](int64_t tile, int64_t lo, int64_t hi, const GaeTileGroups& tg, const float (&oa)[GAE_ITEMS],
+                                   const float (&ms)[GAE_ITEMS]) { gae_tile_normalise(a, tile, lo, hi, tg, oa, ms); });
 }
 
 // Apply pass of the two-launch form. Every block first sums what it needs of the five partial
@@ -1880,7 +2095,7 @@ struct AdvGaeArgs {
   float bias, scaling, clip;
   // NORM: normalisation of the advantages within groups of rows (goff in elements), see adv_normalise_row
   NormArgs norm;
-  uint64_t *sums, *left;      // [bs][4] and [bs] in the workspace
+  uint64_t *sums, *flags, *left;  // [bs][4] and twice [bs] in the workspace
   uint64_t call;              // a number no other call has
   unsigned wait_ticks;        // of the 100 MHz clock
 };
@@ -1889,9 +2104,6 @@ struct AdvGaeArgs {
 // the blocks of its group and waits for theirs, up to ADV_GROUP_ROWS rows. The batch's advantages then go to memory once
 // instead of being written, read back with the mask and written again by a launch of its own (46 against 54 B a
 // slot, and 5 us less for a small batch).
-// The sums of a row are sealed words: three numbers and a check word made of them and the call's number. They go
-// out and come in as agent-scope atomics (past the XCD's own L2), in any order: whoever reads four words that fit has all of
-// them, whatever the workspace held before (a chance of 2^-64 a row otherwise), and nothing has to be cleared.
 // No wait is unbounded: the blocks of a group lie next to each other in the grid, but nobody promises that they
 // are on the chip together. A block whose time is up stores its row as it is and leaves a note (`left`); it, or any
 // block of the group that finds all sums, then takes the note (one of them, by compare and swap) and normalises that row
@@ -1899,49 +2111,6 @@ struct AdvGaeArgs {
 // of the block that leaves one and the last of the group to publish, one sees the other.
 constexpr int ADV_GROUP_ROWS = 64;                   // one lane per row
 constexpr int ADV_NORM_TILES = 4;                    // of a row, 8 mask bits each
-constexpr unsigned ADV_WAIT_TICKS = 20000;           // 200 us
-DEVI uint64_t sums_seal(uint64_t call, const uint64_t (&w)[3]) {
-  return call + w[0] * 0x9e3779b97f4a7c15ull + w[1] * 0xbf58476d1ce4e5b9ull + w[2] * 0x94d049bb133111ebull;
-}
-DEVI void publish_sums(const AdvGaeArgs& a, int64_t b, const double (&s)[3]) {  // by one thread
-  uint64_t w[3];
-  uint64_t* const to = a.sums + 4 * b;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    w[k] = __builtin_bit_cast(uint64_t, s[k]);
-    __hip_atomic_store(to + k, w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __hip_atomic_store(to + 3, sums_seal(a.call, w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// The sums of rows [r0, r0 + n), added up by a whole wave (lane i: row r0 + i) in the order of the apply kernel's;
-// false when they were not all there within `ticks`.
-DEVI bool gather_sums(const AdvGaeArgs& a, int64_t r0, int n, unsigned ticks, double (&s)[3]) {
-  const int lane = threadIdx.x & 63;
-  const uint64_t* const from = a.sums + 4 * (r0 + lane);
-  const uint64_t start = wall_clock64();
-  bool have = lane >= n;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) s[k] = 0.0;
-  for (;;) {
-    if (!have) {
-      uint64_t w[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) w[k] = __hip_atomic_load(from + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const uint64_t seal = __hip_atomic_load(from + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      have = seal == sums_seal(a.call, w);
-      if (have) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) s[k] = __builtin_bit_cast(double, w[k]);
-      }
-    }
-    if (__builtin_amdgcn_ballot_w64(!have) == 0) break;
-    if (wall_clock64() - start >= ticks) return false;
-    __builtin_amdgcn_s_sleep(1);
-  }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) s[k] = wave_sum(s[k]);
-  return true;
-}
 struct RowGroup { int g, first, rows; };  // group of a row: its first row and their number
 DEVI RowGroup row_group(const NormArgs& n, int64_t row, int64_t L) {  // by a whole wave; row: the row's first element
   const int g = wave_count_le(n.goff + 1, n.G, row, threadIdx.x & 63);
@@ -1964,21 +2133,19 @@ DEVI void adv_normalise_row(const AdvGaeArgs& a, int64_t b, const RowGroup& rg, 
         row_store<false>(adv, t0, L, q, f(*(const f32x4*)(x + t0 + q * WAVE_QUADS), bits >> (8 * tile + QUAD * q)));
     }
   };
-  if (tid == 0) publish_sums(a, b, s);
+  if (tid == 0) publish_sums(a.sums + 4 * b, a.flags + b, a.call, s);
   uint64_t todo = 0;  // (first wave) rows of the group whose blocks have left
   auto gather = [&](unsigned ticks) {
     if (tid < 64) {
       double v[3];
-      const bool all = gather_sums(a, rg.first, rg.rows, ticks, v);
+      const bool all = gather_sums<4>(a.sums + 4 * (int64_t)rg.first, a.flags + rg.first, rg.rows, a.call, wall_clock64() + ticks, v);
       if (tid == 0) {
         s_flag = all ? 1 : 0;
 #pragma unroll
         for (int k = 0; k < 3; ++k) s_sum[k] = v[k];
       }
       if (all) {
-        const bool note = tid < rg.rows && __hip_atomic_load(a.left + rg.first + tid, __ATOMIC_RELAXED,
-                                                             __HIP_MEMORY_SCOPE_AGENT) == a.call;
-        todo = __builtin_amdgcn_ballot_w64(note);
+        todo = __builtin_amdgcn_ballot_w64(tid < rg.rows && note_left(a.left + rg.first + tid, a.call));
       }
     }
     __syncthreads();
@@ -1988,7 +2155,7 @@ DEVI void adv_normalise_row(const AdvGaeArgs& a, int64_t b, const RowGroup& rg, 
     of_tiles([&](const f32x4& w, uint32_t) { return w; });
     __threadfence();
     __syncthreads();
-    if (tid == 0) atomicExch((unsigned long long*)a.left + b, (unsigned long long)a.call);
+    if (tid == 0) leave_note(a.left + b, a.call);
     if (!gather(0)) return;
     // (its own note among the others' now)
   } else {
@@ -2009,8 +2176,7 @@ DEVI void adv_normalise_row(const AdvGaeArgs& a, int64_t b, const RowGroup& rg, 
   for (uint64_t rest = s_todo; rest != 0; rest &= rest - 1) {
     const int64_t r = rg.first + __builtin_ctzll(rest);
     __syncthreads();
-    if (tid == 0)
-      s_flag = atomicCAS((unsigned long long*)a.left + r, (unsigned long long)a.call, (unsigned long long)~a.call) == a.call;
+    if (tid == 0) s_flag = take_note(a.left + r, a.call) ? 1 : 0;
     __syncthreads();
     if (s_flag == 0) continue;  // somebody else's
     __threadfence();
@@ -2547,6 +2713,9 @@ uint64_t next_call_number() {
   return z ^ (z >> 31);
 }
 
+// Ticks of the 100 MHz clock that a block waits for its group.
+unsigned group_wait_ticks(int us) { return 100u * (unsigned)(us < 0 ? 200 : std::min(us, 1000)); }
+
 // Whether the row sums ride in the scan of padded rows.
 bool row_sums_fit(int64_t n_seqs, int64_t uniform_len) {
   if (uniform_len > 64 * (int64_t)GAE_TILE || n_seqs > (1 << 30)) return false;
@@ -2799,6 +2968,68 @@ int areal_gae_packed_normalized(const float* rewards, const float* values, const
   const GroupOffsets go{nullptr, group_first, cu_seqlens, 0};
   hipLaunchKernelGGL(norm_apply_seg_kernel, dim3((unsigned)ceil_div_i64(n_tokens, SEG_APPLY_ELEMS)), dim3(NORM_THREADS),
                      0, stream, a, go);
+  AREAL_CHECK_LAUNCH();
+  return AREAL_OK;
+}
+
+// areal_gae_packed_normalized in one launch where it can be (gae_tile_norm_kernel), else in its two. max_group_seqs: the
+// sequences of the largest group; wait_us as areal_group_norm_spec.
+size_t areal_gae_packed_normalized_workspace_bytes(int64_t n_tokens, int64_t n_groups) {
+  if (n_tokens <= 0 || n_groups <= 0) return 0;
+  return std::max((size_t)(ceil_div_i64(n_tokens, GAE_TILE) + n_groups) * (SUMS_PITCH + 2) * sizeof(uint64_t),
+                  areal_gae_segment_stats_bytes(n_tokens, n_groups)) + 256;
+}
+int areal_gae_packed_normalized_ex(const float* rewards, const float* values, const float* loss_mask,
+                                   const int32_t* cu_seqlens, const uint8_t* no_eos, const float* lambda_seq,
+                                   int64_t n_tokens, int64_t n_seqs, float discount, float gae_lambda,
+                                   const int64_t* group_first, const int64_t* group_rows, int64_t n_groups,
+                                   int64_t max_group_seqs, int tail_group, int mean_level, int std_level, int unbiased,
+                                   double eps, int wait_us, float* advantages, float* returns, float* normalized,
+                                   void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  if (n_tokens < 0 || n_seqs < 0 || n_groups < 0) return AREAL_ERR_BAD_ARG;
+  if (n_tokens == 0) return AREAL_OK;
+  if (!rewards || !loss_mask || !advantages || !returns || !normalized || !cu_seqlens || !group_first ||
+      !group_rows || n_seqs == 0 || n_groups == 0)
+    return AREAL_ERR_BAD_ARG;
+  if (workspace == nullptr || workspace_bytes < areal_gae_packed_normalized_workspace_bytes(n_tokens, n_groups))
+    return AREAL_ERR_WORKSPACE;
+  uint64_t* const ws = (uint64_t*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
+  const int64_t nb = ceil_div_i64(n_tokens, GAE_TILE);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const bool known = hipStreamIsCapturing(stream, &capture) == hipSuccess;
+  if (!known) (void)hipGetLastError();
+  // While all tiles are on the chip at once (4 blocks a CU) one launch is the better one for groups of any size measured,
+  // up to 64 tiles; with more tiles the blocks that wait keep those that they wait for from starting. Two launches / one,
+  // us (tiles, tiles a group): 875, 14: 32.0 / 27.8; 875, 55: 32.5 / 31.0; 1024, 16: 49.7 / 46.6; 1024, 64: 50.3 / 49.7;
+  // 2000, 4: 54.4 / 51.0; 2000, 8: 60.3 / 59.3; 1953, 16: 53.7 / 61.9; 2000, 31: 57.6 / 72.8; 2048, 64: 73.5 / 155.7.
+  const int64_t most_tiles = nb <= 1024 ? 64 : 4;
+  const bool one = known && capture == hipStreamCaptureStatusNone && tail_group < 0 && mean_level != LEVEL_BATCH &&
+                   std_level != LEVEL_BATCH && nb <= (1 << 29) &&
+                   max_group_seqs * ceil_div_i64(n_tokens, n_seqs) <= most_tiles * GAE_TILE &&
+                   n_tokens / n_seqs <= 8 * GAE_TILE && n_tokens / n_groups >= 256 &&
+                   (((uintptr_t)rewards | (uintptr_t)values | (uintptr_t)advantages | (uintptr_t)loss_mask |
+                     (uintptr_t)normalized) & 15) == 0;
+  if (!one)
+    return areal_gae_packed_normalized(rewards, values, loss_mask, cu_seqlens, no_eos, lambda_seq, n_tokens, n_seqs, discount,
+                                       gae_lambda, group_first, group_rows, n_groups, tail_group, mean_level, std_level,
+                                       unbiased, eps, advantages, returns, normalized, (double*)ws,
+                                       areal_gae_segment_stats_bytes(n_tokens, n_groups), stream);
+  if (mean_level < 0 || mean_level > 2 || std_level < 0 || std_level > 2) return AREAL_ERR_BAD_ARG;
+  GaeNormArgs a{};
+  a.g = GaeArgs{rewards, values, loss_mask, cu_seqlens, no_eos, lambda_seq, n_tokens, (int)n_seqs,
+                0, discount, gae_lambda, advantages, returns, 0, nullptr};
+  a.g.gseq = group_first; a.g.n_groups = (int)n_groups; a.g.seg_slots = nb + n_groups;
+  a.norm.grows = group_rows; a.norm.G = (int)n_groups; a.norm.tail_group = -1;
+  a.norm.mean_level = mean_level; a.norm.std_level = std_level; a.norm.unbiased = unbiased; a.norm.eps = eps;
+  a.norm.out = normalized;
+  a.sums = ws;
+  a.flags = ws + SUMS_PITCH * a.g.seg_slots;
+  a.left = a.flags + a.g.seg_slots;
+  a.call = next_call_number();
+  a.wait_ticks = group_wait_ticks(wait_us);
+  const dim3 grid((unsigned)(ceil_div_i64(nb, 8) * 8));
+  if (lambda_seq != nullptr) hipLaunchKernelGGL((gae_tile_norm_kernel<true>), grid, dim3(GAE_THREADS), 0, stream, a);
+  else hipLaunchKernelGGL((gae_tile_norm_kernel<false>), grid, dim3(GAE_THREADS), 0, stream, a);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }
@@ -3119,7 +3350,7 @@ int areal_advantages_row_stats(const float* rewards, int score_mode, float bias,
 // what areal_advantages_row_stats does not take: a level of the batch, leave one out, ungrouped rows, groups of more than
 // 64 rows, rows of more than 8192 slots, and a stream that is being captured (a graph's replays would all carry one
 // call's number, and find the sums of the replay before them).
-size_t areal_advantages_normalized_workspace_bytes(int64_t bs) { return bs > 0 ? (size_t)bs * 5 * sizeof(uint64_t) + 256 : 0; }
+size_t areal_advantages_normalized_workspace_bytes(int64_t bs) { return bs > 0 ? (size_t)bs * 6 * sizeof(uint64_t) + 256 : 0; }
 
 int areal_advantages_normalized(const float* rewards, int score_mode, float bias, float scaling, float clip,
                                 const int64_t* group_offsets, const int64_t* group_rows, int64_t n_groups, int tail_group,
@@ -3147,9 +3378,10 @@ int areal_advantages_normalized(const float* rewards, int score_mode, float bias
   }
   if (capture != hipStreamCaptureStatusNone) return AREAL_ERR_UNSUPPORTED;
   a.sums = (uint64_t*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
-  a.left = a.sums + 4 * bs;
+  a.flags = a.sums + 4 * bs;
+  a.left = a.flags + bs;
   a.call = next_call_number();
-  a.wait_ticks = norm->wait_us < 0 ? ADV_WAIT_TICKS : 100u * (unsigned)std::min(norm->wait_us, 1000);
+  a.wait_ticks = group_wait_ticks(norm->wait_us);
   return launch_adv_gae<true>(a, stream);
 }
 

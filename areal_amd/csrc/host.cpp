@@ -1070,12 +1070,12 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> gae_packed_normalized(
   const auto& [first, rows, longest, tail, mean_level, std_level, loo, unbiased, eps] = norm;
   const int64_t n = r.numel(), n_seqs = cu.numel() - 1;
   const Tensor adv = at::empty_like(r), ret = at::empty_like(r), out = at::empty_like(r);
-  const size_t bytes = areal_gae_segment_stats_bytes(n, rows.numel());
-  const Tensor seg = workspace(r, bytes);
-  const int rc = areal_gae_packed_normalized(
+  const size_t bytes = areal_gae_packed_normalized_workspace_bytes(n, rows.numel());
+  const Tensor ws = workspace(r, bytes);
+  const int rc = areal_gae_packed_normalized_ex(
       ptr<float>(r), ptr<float>(v), ptr<float>(m), ptr<int32_t>(cu), ptr<uint8_t>(ne), ptr<float>(lam), n, n_seqs,
-      (float)discount, (float)lambda, ptr<int64_t>(first), ptr<int64_t>(rows), rows.numel(), tail, mean_level, std_level,
-      unbiased, eps, ptr<float>(adv), ptr<float>(ret), ptr<float>(out), ptr<double>(seg), bytes, stream_of(r));
+      (float)discount, (float)lambda, ptr<int64_t>(first), ptr<int64_t>(rows), rows.numel(), longest, tail, mean_level,
+      std_level, unbiased, eps, -1, ptr<float>(adv), ptr<float>(ret), ptr<float>(out), ptr<void>(ws), bytes, stream_of(r));
   if (rc == AREAL_ERR_UNSUPPORTED || rc == AREAL_ERR_ALIGNMENT) return std::nullopt;
   check(rc, "areal_gae_packed_normalized");
   return std::make_tuple(out, ret, adv);

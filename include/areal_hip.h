@@ -514,6 +514,19 @@ int areal_advantage_prep(const uint8_t* loss_mask, const uint8_t* attn_mask, con
                          float* kl_out, float* gkl_out, float* outcome_out, float* tot_out,
                          int64_t* seqlens_out, uint8_t* no_eos_out, areal_stream_t stream);
 
+/* areal_gae_packed_normalized in one launch where groups are short enough (no level the batch,
+ * no ungrouped sequences, the stream not being captured), else in its two. max_group_seqs: the sequences of
+ * the largest group; wait_us as areal_group_norm_spec. */
+size_t areal_gae_packed_normalized_workspace_bytes(int64_t n_tokens, int64_t n_groups);
+int areal_gae_packed_normalized_ex(const float* rewards, const float* values, const float* loss_mask,
+                                   const int32_t* cu_seqlens, const uint8_t* no_eos,
+                                   const float* lambda_seq, int64_t n_tokens, int64_t n_seqs,
+                                   float discount, float gae_lambda, const int64_t* group_first,
+                                   const int64_t* group_rows, int64_t n_groups, int64_t max_group_seqs,
+                                   int tail_group, int mean_level, int std_level, int unbiased, double eps,
+                                   int wait_us, float* advantages, float* returns, float* normalized,
+                                   void* workspace, size_t workspace_bytes, areal_stream_t stream);
+
 /* Reward scores (areal_reward_scores), areal_advantage_prep and areal_gae_padded_row_stats of a padded
  * [bs, L] batch in one launch, with their results. score_mode 0: rewards are the scores; 1: they are
  * shaped first; 2: shaped and normalised within groups of rows (no level may be the batch).

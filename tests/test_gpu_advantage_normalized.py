@@ -30,7 +30,7 @@ def _inputs(dev, bs, L, critic, ref):
                 rewards=torch.randn(bs, generator=g).to(dev))
 
 
-def _both(dev, x, offsets, levels, unbiased, wait_us, eps=1e-5):
+def _both(dev, x, offsets, levels, unbiased, wait_us, eps=1e-5, fill=0):
     """(two launches, one launch): normalised advantages and the other outputs."""
     lib = _lib.load()
     bs, L = x["logp"].shape
@@ -50,7 +50,7 @@ def _both(dev, x, offsets, levels, unbiased, wait_us, eps=1e-5):
         if fused:
             spec = _lib.GroupNormSpec(off.data_ptr(), len(rows), most, -1, *levels, 0, unbiased, wait_us, eps)
             nbytes = lib.areal_advantages_normalized_workspace_bytes(bs)
-            ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+            ws = torch.full((nbytes,), fill, dtype=torch.uint8, device=dev)
             _lib.check(lib.areal_advantages_normalized(*args, ctypes.byref(spec), p(ws), nbytes, s), "normalized")
         else:
             sums = torch.empty(5, bs, dtype=torch.float64, device=dev)
@@ -97,6 +97,17 @@ def test_many_groups_with_rows_that_leave(dev):
     """More rows than are on the chip at once, none of which waits."""
     x = _inputs(dev, 4096, 1800, True, False)
     _same(*_both(dev, x, list(range(0, 4097, 16)), (2, 2), 1, 0))
+
+
+@pytest.mark.parametrize("fill", [0, 0, 64, 255])
+def test_sums_of_few_bits(dev, fill):
+    """Counts and sums that are small integers, told from what the workspace held before."""
+    x = _inputs(dev, 1024, 1024, False, False)
+    x["loss"].fill_(True)
+    x["attn"].fill_(True)
+    x["logp"].fill_(-1.0)
+    x["rewards"].copy_((x["rewards"] > 0).float())
+    _same(*_both(dev, x, list(range(0, 1025, 16)), (2, 2), 1, -1, fill=fill))
 
 
 @pytest.mark.parametrize("change", ["batch", "tail", "long group", "long row", "leave one out"])

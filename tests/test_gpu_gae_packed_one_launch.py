@@ -1,0 +1,129 @@
+"""Packed GAE and the normalisation of its advantages in one launch (areal_gae_packed_normalized_ex) against the two launches
+it replaces (areal_gae_packed_normalized): the same scan, so the same bits of advantages and returns. A group's sums are
+added up in fp64 in another order (2^-52 a term, a few thousand of them at most), after which mean and deviation may round to the fp32
+neighbour: 2^-23 of each, so |difference| <= 2^-22 (|x| + |mean|) / deviation, with the mean below the largest |x|.
+
+Groups inside a tile, over many tiles, empty ones, more groups in a tile than a block has waves; sequences without
+tokens and longer than many tiles; tokens before the first and behind the last sequence; masks that are not 0 or 1, a
+group without a masked token, advantages that are not finite. With no time to wait every segment of a group that is not
+complete yet is left to the group's last wave, which has to give the same."""
+
+import pytest
+import torch
+
+from areal_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(dev, lens, sizes, levels, wait_us, *, unbiased=1, critic=True, lam=None, mask="binary", around=(0, 0), bad=None, fill=0):
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(len(lens) + sum(lens))
+    cu = torch.tensor([around[0]] + lens).cumsum(0).to(torch.int32)
+    n, n_seqs = int(cu[-1]) + around[1], len(lens)
+    m = (torch.rand(n, generator=g) > 0.4).float()
+    if mask == "ones":
+        m.fill_(1.0)
+    if mask == "weights":
+        m *= 0.25 + torch.rand(n, generator=g)
+    first = torch.tensor([0] + sizes).cumsum(0)
+    if mask == "silent group":
+        m[cu[first[1]]:cu[first[2]]] = 0
+    r, v = torch.randn(n, generator=g), torch.randn(n, generator=g)
+    if bad is not None:
+        r[bad], m[bad] = float("inf"), 1.0
+    no_eos = (torch.rand(n_seqs, generator=g) > 0.5).to(dev)
+    lam_seq = torch.rand(n_seqs, generator=g).to(dev) if lam else None
+    x = [t.to(dev) for t in (r, v, m, cu, first, torch.tensor(sizes))]
+    p, s = _lib.ptr, _lib.stream_ptr(dev)
+    res = []
+    for fused in (False, True):
+        adv, ret, out = (torch.full((n,), 7.5, device=dev) for _ in range(3))
+        head = [p(x[0]), p(x[1]) if critic else None, p(x[2]), p(x[3]), p(no_eos), p(lam_seq), n, n_seqs, 0.99, 0.95, p(x[4]), p(x[5]),
+                len(sizes)]
+        if fused:
+            nbytes = lib.areal_gae_packed_normalized_workspace_bytes(n, len(sizes))
+            ws = torch.full((nbytes,), fill, dtype=torch.uint8, device=dev)
+            _lib.check(lib.areal_gae_packed_normalized_ex(*head, max(sizes), -1, *levels, unbiased, 1e-5, wait_us, p(adv), p(ret),
+                                                          p(out), p(ws), nbytes, s), "ex")
+        else:
+            nbytes = lib.areal_gae_segment_stats_bytes(n, len(sizes))
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            _lib.check(lib.areal_gae_packed_normalized(*head, -1, *levels, unbiased, 1e-5, p(adv), p(ret), p(out), p(ws), nbytes, s),
+                       "two launches")
+        torch.cuda.synchronize()
+        res.append((out, adv, ret))
+    for k, (a, b) in enumerate(zip(*res)):
+        assert torch.equal(a.isnan(), b.isnan())
+        a, b = a.nan_to_num(3.25), b.nan_to_num(3.25)
+        if k == 0:
+            assert (a - b).abs().max().item() <= 2.0 ** -21 * a.abs().max().item()
+        else:
+            assert torch.equal(a, b)
+
+
+def _lens(n, mean, seed):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.exp(torch.randn(n, generator=g) * 0.8) * mean * 0.73).long().clamp(min=1).tolist()
+
+
+@pytest.mark.parametrize("wait_us", [-1, 0])
+@pytest.mark.parametrize("case", range(8))
+def test_same_bits_as_two_launches(dev, case, wait_us):
+    lens, sizes, options = [
+        (_lens(64, 700, 1), [4] * 16, dict()),
+        (_lens(96, 60, 2), [8] * 12, dict(unbiased=0)),                       # several groups in a tile
+        (_lens(240, 90, 3), [3, 1, 5, 7] * 15, dict(critic=False)),           # more of them than waves
+        (_lens(48, 5000, 4), [16] * 3, dict(lam=True)),                       # groups and sequences of many tiles
+        ([2048] * 8 + [0, 1, 4096, 0, 2047, 2049, 0, 0], [4, 4, 2, 2, 2, 2], dict(mask="silent group")),
+        (_lens(32, 1500, 6), [8, 8, 0, 8, 0, 8], dict(mask="weights")),
+        (_lens(20, 900, 7), [10, 10], dict(around=(37, 5000))),
+        (_lens(30, 1200, 8), [6] * 5, dict(bad=5000)),
+    ][case]
+    levels = [(2, 2), (0, 2), (2, 0), (0, 0)][case % 4]
+    _run(dev, lens, sizes, (2, 2), wait_us, **options)
+    _run(dev, lens, sizes, levels, wait_us, **options)
+
+
+@pytest.mark.parametrize("wait_us", [-1, 0])
+def test_more_tiles_than_the_chip_holds(dev, wait_us):
+    _run(dev, _lens(1600, 2200, 9), [16] * 100, (2, 2), wait_us)
+
+
+@pytest.mark.parametrize("fill", [0, 0, 0, 64, 255])
+def test_counts_of_few_bits(dev, fill):
+    """Whole tiles of masked tokens and small integers make sums with hardly a bit set, which have to be told from
+    what the workspace held before, however many of an entry's words have arrived."""
+    _run(dev, [2048] * 256 + [1500] * 512, [16] * 48, (2, 2), -1, critic=False, mask="ones", fill=fill)
+
+
+def test_short_groups(dev):
+    for n in (1, 2, 7, 8, 9, 255):
+        _run(dev, [n, 600], [1, 1], (2, 2), -1)
+
+
+def test_captured_call_takes_two_launches(dev):
+    """A graph's replays would all carry the captured call's number: they run the two launches and see new inputs."""
+    from areal_amd.config import NormConfig
+    from areal_amd.data import Normalization
+    from areal_amd.ppo.gae import compute_gae_packed_normalized
+
+    g = torch.Generator().manual_seed(0)
+    cu = torch.arange(0, 33 * 500, 500, dtype=torch.int32, device=dev)
+    r, v, m = (torch.randn(16000, generator=g).to(dev) for _ in range(3))
+    m = (m > 0).float()
+    norm = Normalization(NormConfig(mean_level="group", std_level="group", group_size=8))
+    call = lambda: compute_gae_packed_normalized(r, v, m, cu, None, 1.0, 0.95, norm)  # noqa: E731
+    side = torch.cuda.Stream(dev)
+    with torch.cuda.stream(side):
+        call()
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = call()
+    for k in range(3):
+        r.add_(v, alpha=0.3)
+        want = [t.clone() for t in call()]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), k
