@@ -196,15 +196,15 @@ DEVI T block_sum(T v, T* smem) {
 // ---------------------------------------------------------------------------------------
 // Segmented pass 1: per-sequence aggregate of the rejection metric.
 // Writes seq_rs[s] = {in_bounds, uniform weight exp(mean log ratio)}.
-// WPS waves per sequence: a block of 4 waves takes 4 / WPS sequences. Bound by HBM (9 bytes per
+// WPS waves per sequence: a block of 4 waves takes 4 / WPS sequences, one of more waves a single one. Bound by HBM (9 bytes per
 // token): a lane takes four tokens with 16-byte loads, aligned whatever the sequence's start is
 // (VEC = 4), the loads of a group do not wait for its mask, and many short sequences take a wave each
 // so that the lanes of a block are not idle. 4 Mi tokens in 2048 sequences: 38 us with one token per
 // lane and loads behind the mask.
 // ---------------------------------------------------------------------------------------
 template <int WPS, int VEC>
-__global__ __launch_bounds__(LOSS_THREADS) void seq_rs_kernel(LossIO io, LossCfg c, float* seq_rs) {
-  constexpr int NW = LOSS_THREADS / 64, SPB = NW / WPS;
+__global__ __launch_bounds__(WPS > 4 ? 64 * WPS : LOSS_THREADS) void seq_rs_kernel(LossIO io, LossCfg c, float* seq_rs) {
+  constexpr int NW = WPS > 4 ? WPS : LOSS_THREADS / 64, SPB = NW / WPS;
   __shared__ double sm_d[2][NW];
   __shared__ float sm_f[NW];
   __shared__ int sm_i[2][NW];
@@ -1077,9 +1077,18 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
     // 11.9 / 4.6 against 5.6 / 4.6).
     const bool short_seqs = n_seqs > 4096 && n_tokens <= n_seqs * 384;
     const bool vec = aligned_to(proximal, 16) && aligned_to(old_logprobs, 16) && aligned_to(loss_mask, 4);
-    const dim3 grid_s((unsigned)(short_seqs ? ceil_div_i64(n_seqs, LOSS_THREADS / 64) : n_seqs)), block(LOSS_THREADS);
+    // Otherwise the longest sequence sets the time, a memory latency per step of its block (a second step's loads in flight
+    // cost more than they gave: 21.7 -> 24.4 us in the first of these): as many waves a sequence as the chip holds of all
+    // sequences at once. 4, 8, 16 waves, us, lognormal lengths: 4 Mi tokens in 2048 21.9 / 16.6 / 23.8, in 1100 31.5 / 19.7 /
+    // 20.2, in 8192 18.4 / 25.2 / 62.1; 1 Mi in 512 13.9 / 9.4 / 9.0, in 2600 9.3 / 10.6 / 22.5; 256 Ki in 128 10.6 / 7.4 /
+    // 6.3, in 1024 5.2 / 5.4 / 9.2; 32 Ki in 32 5.6 / 4.8 / 4.8.
+    const int waves = short_seqs ? 1 : n_seqs > 2048 || n_tokens < n_seqs * 512 || !vec ? 4 : n_seqs > 512 ? 8 : 16;
+    const dim3 grid_s((unsigned)(short_seqs ? ceil_div_i64(n_seqs, LOSS_THREADS / 64) : n_seqs));
+    const dim3 block(waves > 4 ? 64 * waves : LOSS_THREADS);
     if (short_seqs && vec) hipLaunchKernelGGL((seq_rs_kernel<1, 4>), grid_s, block, 0, stream, io, c, seq_rs);
     else if (short_seqs) hipLaunchKernelGGL((seq_rs_kernel<1, 1>), grid_s, block, 0, stream, io, c, seq_rs);
+    else if (waves == 16) hipLaunchKernelGGL((seq_rs_kernel<16, 4>), grid_s, block, 0, stream, io, c, seq_rs);
+    else if (waves == 8) hipLaunchKernelGGL((seq_rs_kernel<8, 4>), grid_s, block, 0, stream, io, c, seq_rs);
     else if (vec) hipLaunchKernelGGL((seq_rs_kernel<4, 4>), grid_s, block, 0, stream, io, c, seq_rs);
     else hipLaunchKernelGGL((seq_rs_kernel<4, 1>), grid_s, block, 0, stream, io, c, seq_rs);
     AREAL_CHECK_LAUNCH();

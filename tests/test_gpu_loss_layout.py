@@ -50,6 +50,14 @@ def test_sequence_rejection(lens, offset, metric, agg):
     torch.testing.assert_close(got.behave_imp_weight.cpu(), want.behave_imp_weight, rtol=1e-5, atol=1e-6)
 
 
+# 16 waves a sequence up to 512 of at least 512 tokens on average, 8 up to 2048, 4 beyond; a step of a block is 4096, 2048, 1024 tokens
+@pytest.mark.parametrize("lens", [[4095, 4096, 4097, 0, 1], [511, 512] * 100 + [20000], [512] * 512, [513] * 513, [2047, 0, 2049] * 300,
+                                  [512] * 2048, [515] * 2049])
+@pytest.mark.parametrize("metric,agg", [("kl_k2", "mean"), ("kl_k3", "max"), ("ratio", "mean")])
+def test_sequence_rejection_of_long_sequences(lens, metric, agg):
+    test_sequence_rejection(lens, 0, metric, agg)
+
+
 # more than 4096 sequences take a wave each up to a mean of 384 tokens
 @pytest.mark.parametrize("offset", [0, 1])
 @pytest.mark.parametrize("lens", [[7] * 4096, [7, 1, 0, 300] * 1025, [2, 5000] + [65] * 4095, [384] * 4097, [385] * 4097])
