@@ -165,6 +165,11 @@ struct Mark {
   }
 };
 
+// Which statistics a result holds: (row, key, denominator). Made once per kind of call, so that a call converts no strings.
+struct StatRows {
+  std::vector<std::tuple<int, py::str, py::str>> rows;
+};
+
 struct HostResult {
   Tensor host;    // fp64, pinned
   Tensor device;  // the results of a captured call
@@ -216,9 +221,17 @@ struct HostResult {
     if (!device.defined() && !arrived()) behind.set(stream);
   }
   Tensor value() { wait(); return host; }
+  // The counters as Python floats. (As a tensor, each of the few numbers that a call looks at cost an indexing and an
+  // item(), one to two microseconds apiece while the GPU stands idle.)
+  py::list counters() {
+    wait();
+    py::list out;
+    for (int64_t i = 0; i < std::min<int64_t>(host.numel(), 9); ++i) out.append(py::float_(data()[i]));
+    return out;
+  }
   // {key: {sum, count, avg, min, max, denominator}} of rows `offset + 4 * row` of the result; avg, min and max
   // are None under an empty denominator.
-  void fill(py::dict out, const std::vector<std::tuple<int, py::str, py::str>>& rows, int64_t offset) {
+  void fill(py::dict out, const StatRows& stats, int64_t offset) {
     wait();
     static PyObject *k_sum = PyUnicode_InternFromString("sum"), *k_count = PyUnicode_InternFromString("count"),
                     *k_avg = PyUnicode_InternFromString("avg"), *k_min = PyUnicode_InternFromString("min"),
@@ -226,7 +239,7 @@ struct HostResult {
                     *k_den = PyUnicode_InternFromString("denominator");
     const double* h = data() + offset;
     auto set = [](py::dict& d, PyObject* k, const py::object& v) { PyDict_SetItem(d.ptr(), k, v.ptr()); };
-    for (const auto& [row, key, den] : rows) {
+    for (const auto& [row, key, den] : stats.rows) {
       const double* r = h + 4 * row;
       const bool empty = r[1] == 0.0;
       py::dict d;
@@ -1241,8 +1254,12 @@ OptTensor unpack_rows(const Tensor& packed, const py::list& seqlens, const std::
 
 PYBIND11_MODULE(_host, m) {
   m.def("set_error_class", [](py::object cls) { error_class = cls.release().ptr(); });
+  py::class_<StatRows>(m, "StatRows").def(py::init([](std::vector<std::tuple<int, py::str, py::str>> rows) {
+    return StatRows{std::move(rows)};
+  }));
   py::class_<HostResult, HostResultPtr>(m, "HostResult")
-      .def("value", &HostResult::value)
+      .def("wait", &HostResult::wait)
+      .def("counters", &HostResult::counters)
       .def("mark", &HostResult::mark)
       .def("fill", &HostResult::fill);
   m.def("actor_loss", &actor_loss);

@@ -73,7 +73,7 @@ class DeferredFloat:
 
     def __float__(self) -> float:
         if self._value is None:
-            self._value = float(self._fn(self._source.value()))
+            self._value = float(self._fn(self._source.counters()))
         return self._value
 
     def __repr__(self) -> str:
@@ -163,7 +163,7 @@ class StatReduction:
     def _fill_sapo(self, host, n_tokens: int) -> None:
         """Results of ``areal_sapo_loss``'s reduction. SAPO clips nothing: the clip ratios are
         zero on every token of the mask and the clipped-token statistics are empty."""
-        self._fill(host, n_tokens, False, True, keys=SAPO_REDUCED_STAT_KEYS, offset=8)
+        self._fill(host, n_tokens, False, True, sapo=True, offset=8)
         nv = self._denominators["n_valid_tokens"]
         zero = dict(sum=0.0, count=nv, avg=None if nv == 0 else 0.0, min=None if nv == 0 else 0.0,
                     max=None if nv == 0 else 0.0, denominator="n_valid_tokens")
@@ -180,10 +180,10 @@ class StatReduction:
         self._resolve()
         return self._denominators
 
-    def _fill(self, host, n_tokens: int, has_rs: bool, has_old: bool, keys=REDUCED_STAT_KEYS, offset: int = 9) -> None:
-        rows = _stat_rows(keys, self.entropy is not None, has_rs, has_old, tuple(self.extras))
+    def _fill(self, host, n_tokens: int, has_rs: bool, has_old: bool, sapo: bool = False, offset: int = 9) -> None:
+        rows = _stat_rows(sapo, self.entropy is not None, has_rs, has_old, tuple(self.extras))
         host.fill(self._results, rows, offset)
-        c = host.value()[:7].tolist()
+        c = host.counters()
         self._denominators = dict(n_tokens=float(n_tokens), n_valid_tokens=c[1], clipped_tokens=c[4],
                                   dual_clipped_tokens=c[5])
         if has_rs:
@@ -191,10 +191,10 @@ class StatReduction:
 
 
 @functools.lru_cache(maxsize=64)
-def _stat_rows(keys, has_entropy: bool, has_rs: bool, has_old: bool, extras: tuple):
-    """``(row, key, denominator)`` of the statistics a call with these inputs reduces."""
+def _stat_rows(sapo: bool, has_entropy: bool, has_rs: bool, has_old: bool, extras: tuple):
+    """``(row, key, denominator)`` of the statistics a call with these inputs reduces, as the native side takes them."""
     rows = []
-    for i, (key, denom) in enumerate(keys):
+    for i, (key, denom) in enumerate(SAPO_REDUCED_STAT_KEYS if sapo else REDUCED_STAT_KEYS):
         if key == "entropy" and not has_entropy:
             continue
         if key.startswith("behave_") and not has_rs:
@@ -207,7 +207,7 @@ def _stat_rows(keys, has_entropy: bool, has_rs: bool, has_old: bool, extras: tup
                 continue
             key = extras[j]
         rows.append((i, key, denom))
-    return rows
+    return _lib.host().StatRows(rows)
 
 
 def _fill_rs(cfg: _lib.LossConfig, rs: RejectionSamplingConfig | None) -> None:
@@ -390,27 +390,27 @@ def _loss_common(cfg, logprobs, proximal_logprobs, old_logprobs, advantages, los
         else:
             reduction._fill(*args)
     elif not defer:
-        host.value()
+        host.wait()
     return loss, out, host
 
 
 def _scalar_stats(loss_mask, host, defer):
     n_total = float(loss_mask.numel())
     if not defer:
-        n_valid = host.value()[1].item()
+        n_valid = host.counters()[1]
         return dict(n_total_tokens=n_total, n_valid_tokens=n_valid, n_masked_tokens=n_total - n_valid,
                     masked_token_ratio=1.0 - n_valid / max(n_total, 1.0))
     return dict(
         n_total_tokens=n_total,
         n_valid_tokens=DeferredFloat(host, lambda h: h[1]),
-        n_masked_tokens=DeferredFloat(host, lambda h: n_total - float(h[1])),
-        masked_token_ratio=DeferredFloat(host, lambda h: 1.0 - float(h[1]) / max(n_total, 1.0)),
+        n_masked_tokens=DeferredFloat(host, lambda h: n_total - h[1]),
+        masked_token_ratio=DeferredFloat(host, lambda h: 1.0 - h[1] / max(n_total, 1.0)),
     )
 
 
 def _filtered_fraction(host, defer):
-    fn = lambda h: float(h[3]) / max(float(h[1]), 1.0)  # noqa: E731
-    return DeferredFloat(host, fn) if defer else fn(host.value())
+    fn = lambda h: h[3] / max(h[1], 1.0)  # noqa: E731
+    return DeferredFloat(host, fn) if defer else fn(host.counters())
 
 
 _RS_STATS = ("behave_approx_kl", "behave_imp_weight", "behave_mask")

@@ -10,6 +10,7 @@ dict instead of the reference's process-wide ``stats_tracker``.
 
 from __future__ import annotations
 
+import functools
 import math
 from typing import Any
 
@@ -122,7 +123,6 @@ def grpo_loss_fn(
     advantages = input_data["advantages"]
     loss_mask = input_data["loss_mask"].bool()
     prox_logp_gt = input_data.get("prox_logp")
-    entropy = entropy.detach()
 
     if prox_logp_method == PROX_LOGP_METHOD_REUSE_TRAIN_LOGP:
         prox_logp_gt = logprobs.detach()
@@ -130,7 +130,7 @@ def grpo_loss_fn(
         prox_logp_gt=prox_logp_gt,
         prox_logp_method=prox_logp_method,
         old_logp=old_logp,
-        logprobs=logprobs.detach(),
+        logprobs=logprobs,
         versions=versions,
         current_version=current_version,
     )
@@ -188,7 +188,7 @@ def grpo_loss_fn(
         )
 
     if not defer:
-        _raise_if_nonfinite(host.value()[8] > 0, prox_logp_method)
+        _raise_if_nonfinite(host.counters()[8] > 0, prox_logp_method)
 
     # joint distillation (actor.py:629-658)
     teacher_logp = input_data.get("teacher_logp")
@@ -222,7 +222,7 @@ def grpo_loss_fn(
             if defer:
                 stats["compute_logp_reduction"] = _ProximalStats(host)
             else:
-                host.fill(stats, _PROX_STAT_ROWS, 9)
+                host.fill(stats, _prox_stat_rows(), 9)
                 stats["denominator/compute_logp/n_valid_tokens"] = stats["compute_logp/prox_logp_gt"]["count"]
         if vocab_mean_logits is not None or vocab_norm_logits is not None:
             more = {k: v for k, v in (("vocab_mean_logits", vocab_mean_logits), ("vocab_norm_logits", vocab_norm_logits))
@@ -256,7 +256,7 @@ def grpo_loss_fn(
             approx_kl=stat["approx_kl"],
             new_logp=lp,
             old_logp=old_logp,
-            entropy=entropy.float(),
+            entropy=entropy.detach().float(),
             actor_loss=stat["loss"],
             clip_ratio=out["clip_ratio"],
             dual_clip_ratio=out["dual_clip_ratio"],
@@ -298,8 +298,10 @@ def grpo_loss_fn(
     return loss
 
 
-# row of the proximal log-probs among the reduced statistics of areal_actor_loss_call
-_PROX_STAT_ROWS = [(17, "compute_logp/prox_logp_gt", "compute_logp/n_valid_tokens")]
+@functools.lru_cache(maxsize=1)
+def _prox_stat_rows():
+    """The row of the proximal log-probs among the reduced statistics of areal_actor_loss_call."""
+    return _lib.host().StatRows([(17, "compute_logp/prox_logp_gt", "compute_logp/n_valid_tokens")])
 
 
 class _ProximalStats:
@@ -313,7 +315,7 @@ class _ProximalStats:
     def results(self) -> dict[str, dict[str, float | None]]:
         if self._results is None:
             out: dict = {}
-            self._host.fill(out, _PROX_STAT_ROWS, 9)
+            self._host.fill(out, _prox_stat_rows(), 9)
             for v in out.values():
                 del v["denominator"]
             self._results = out
@@ -372,7 +374,7 @@ def compute_prox_logp_approximations(
     return out
 
 
-def _raise_if_nonfinite(flag: torch.Tensor, prox_logp_method: str) -> None:
+def _raise_if_nonfinite(flag, prox_logp_method: str) -> None:
     if bool(flag):
         raise RuntimeError(
             f"prox_logp contains NaN or Inf with prox_logp_method='{prox_logp_method}'. "
