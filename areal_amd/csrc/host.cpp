@@ -1100,6 +1100,10 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> gae_packed_normalized(
 // and one result unpacked (35 us of kernels): 164 us with a tensor call, a ctypes array or a copy for each, now 75.
 // ---------------------------------------------------------------------------------------
 constexpr size_t PACK_MAX_TENSORS = 8;  // of one launch
+// Up to this size of its result an unpacking's table is read from pinned host memory by the kernel itself (8 bytes per block
+// of 8 to 16 KiB) instead of being copied to the GPU first: 256 x 4096 fp32, kernels 8.0 -> 4.2 us and the host's part 12.1
+// -> 9.4; at 1024 x 8192 (32 MiB) the reads cost what the copy did, 11.5 against 9.1 + 2.6.
+constexpr int64_t UNPACK_DIRECT_BYTES = 32 << 20;
 
 int64_t token_bytes(const Tensor& t, int64_t lead) {
   int64_t n = t.element_size();
@@ -1220,33 +1224,37 @@ OptTensor unpack_rows(const Tensor& packed, const py::list& seqlens, const std::
     const int64_t v = PyLong_AsLongLongAndOverflow(x, &overflow);
     return overflow != 0 || v >= below ? -1 : v;
   };
-  const Tensor host = at::empty({n + 1 + (order.has_value() ? n : 0)},
-                                at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  const Tensor host = at::empty({n, 2}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
   int32_t* const t = (int32_t*)host.data_ptr();
+  std::vector<int32_t> first(n + 1);
   int64_t total = 0, longest = 0;
-  t[0] = 0;
   for (int64_t i = 0; i < n; ++i) {
     const int64_t len = entry(seqlens, i, (int64_t)INT32_MAX + 1);
     if (len < 0 || (total += len) > INT32_MAX) return std::nullopt;
-    t[i + 1] = (int32_t)total;
+    first[i + 1] = (int32_t)total;
     longest = std::max(longest, len);
   }
   if (total != packed.size(0)) return std::nullopt;
-  if (order.has_value()) {
-    std::vector<bool> seen(n);
-    for (int64_t i = 0; i < n; ++i) {
-      const int64_t r = entry(*order, i, n);
+  std::vector<bool> seen(order.has_value() ? n : 0);
+  for (int64_t i = 0; i < n; ++i) {
+    int64_t r = i;
+    if (order.has_value()) {
+      r = entry(*order, i, n);
       if (r < 0 || seen[r]) return std::nullopt;
       seen[r] = true;
-      t[n + 1 + i] = (int32_t)r;
     }
+    t[2 * i] = first[r];
+    t[2 * i + 1] = first[r + 1] - first[r];
   }
-  const Tensor table = host.to(packed.device(), /*non_blocking=*/true);
   const Tensor src = packed.contiguous(), out = tokens_like(src, {n, longest}, 1);
-  const int32_t* const cu = ptr<int32_t>(table);
-  check(areal_unpack_to_padded(ptr<void>(src), ptr<void>(out), cu, order.has_value() ? cu + n + 1 : nullptr, n, longest,
-                               token_bytes(src, 1), nullptr, 0, stream_of(src)),
-        "areal_unpack_to_padded");
+  // The kernel reads the table where it is, a pair per block; only a long one is worth a copy, see UNPACK_DIRECT_BYTES.
+  const bool direct = out.numel() * out.element_size() <= UNPACK_DIRECT_BYTES;
+  const Tensor table = direct ? host : host.to(packed.device(), /*non_blocking=*/true);
+  const auto stream = c10::hip::getCurrentHIPStream(src.device().index());
+  check(areal_unpack_rows(ptr<void>(src), ptr<void>(out), ptr<uint32_t>(table), n, longest, token_bytes(src, 1),
+                          (areal_stream_t)stream.stream()),
+        "areal_unpack_rows");
+  if (direct) keep_until_passed(host, stream);
   return out;
 }
 

@@ -215,6 +215,21 @@ __global__ __launch_bounds__(PK_THREADS) void unpack_kernel(const char* packed, 
   if (ncopy < nj) block_fill_bytes(d + ncopy * eb, (nj - ncopy) * eb, fill);
 }
 
+// unpack_kernel where a row's sequence is given as rows[row] = {first packed token, length}: one read, which may go to
+// host memory. (The pattern is an argument: of a constant the compiler makes a byte loop, 15 us in place of 4.)
+__global__ __launch_bounds__(PK_THREADS) void unpack_rows_kernel(const char* packed, char* padded, const u32x2* rows,
+                                                                 int64_t S, int64_t eb, Fill fill, int chunks, int chunk) {
+  const int64_t row = blockIdx.x / chunks;
+  const int64_t j0 = (int64_t)(blockIdx.x % chunks) * chunk;
+  const int64_t nj = S - j0 < chunk ? S - j0 : chunk;
+  const u32x2 seq = rows[row];
+  int64_t ncopy = (int64_t)seq[1] - j0;
+  ncopy = ncopy < 0 ? 0 : (ncopy > nj ? nj : ncopy);
+  char* d = padded + (row * S + j0) * eb;
+  if (ncopy > 0) block_copy_bytes(d, packed + ((int64_t)seq[0] + j0) * eb, ncopy * eb);
+  if (ncopy < nj) block_fill_bytes(d + ncopy * eb, (nj - ncopy) * eb, fill);
+}
+
 // dst[cu_new[s] + j] = j < old length of s ? src[cu_old[s] + j] : fill; sequences of cu_new
 // beyond n_old (a trailing pad segment) are all fill. arange != 0: dst is int64 position ids,
 // and the fill is j (position inside the new sequence, src == NULL) or j - old length instead.
@@ -477,6 +492,21 @@ int areal_unpack_to_padded(const void* packed, void* padded, const int32_t* cu_s
   hipLaunchKernelGGL(unpack_kernel, dim3((unsigned)(chunks * B)), dim3(PK_THREADS), 0, stream,
                      (const char*)packed, (char*)padded, cu_seqlens, row_seq, S, elem_bytes, f, (int)chunks,
                      (int)chunk);
+  AREAL_CHECK_LAUNCH();
+  return AREAL_OK;
+}
+
+// areal_unpack_to_padded whose rows are given as {first packed token, length} pairs and end in zeros. The pairs may lie in
+// pinned host memory (which has to stay until the launch has finished); a block reads one of them.
+int areal_unpack_rows(const void* packed, void* padded, const uint32_t* rows, int64_t B, int64_t S, int64_t elem_bytes,
+                      hipStream_t stream) {
+  if (B < 0 || S < 0 || elem_bytes <= 0) return AREAL_ERR_BAD_ARG;
+  if (B == 0 || S == 0) return AREAL_OK;
+  if (!padded || !rows) return AREAL_ERR_BAD_ARG;
+  const int64_t chunk = pk_chunk_tokens(elem_bytes), chunks = ceil_div_i64(S, chunk);
+  if (chunks * B >= ((int64_t)1 << 31)) return AREAL_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL(unpack_rows_kernel, dim3((unsigned)(chunks * B)), dim3(PK_THREADS), 0, stream, (const char*)packed,
+                     (char*)padded, (const u32x2*)rows, S, elem_bytes, Fill{{0u, 0u, 0u, 0u}, 16}, (int)chunks, (int)chunk);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }

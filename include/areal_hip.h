@@ -605,6 +605,10 @@ int areal_pack_padded_multi(const void* const* padded, void* const* packed,
 int areal_unpack_to_padded(const void* packed, void* padded, const int32_t* cu_seqlens,
                            const int32_t* row_seq, int64_t B, int64_t S, int64_t elem_bytes,
                            const void* fill, int fill_bytes, areal_stream_t stream);
+/* areal_unpack_to_padded whose rows are given as rows [B][2] = {first packed token, length}, zeros behind them; rows may be
+ * pinned host memory that stays until the launch has finished. */
+int areal_unpack_rows(const void* packed, void* padded, const uint32_t* rows, int64_t B, int64_t S,
+                      int64_t elem_bytes, areal_stream_t stream);
 /* Sequence s moves from cu_old to cu_new (new length >= old, tail filled); sequences of cu_new
  * beyond n_old are all fill. position_ids != 0 (int64 elements): src NULL writes 0..len-1 per
  * new sequence, otherwise the filled parts count 0, 1, 2, ... */

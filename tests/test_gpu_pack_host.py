@@ -42,6 +42,19 @@ def test_unpack_tables_of_several_calls_in_flight(dev):
             assert torch.equal(out[r, : lens[s]].cpu(), rows[s]) and not out[r, lens[s] :].any()
 
 
+@pytest.mark.parametrize("longest", [4095, 1 << 20, (1 << 20) + 1])
+def test_unpack_either_side_of_the_tables_copy(dev, longest):
+    """Results of up to 32 MiB (8 rows of 2^20 floats) read their table where the host made it."""
+    lens = [longest, 1, 0, longest // 2, 7, longest, 3, longest - 1]
+    order = [5, 2, 0, 7, 1, 6, 3, 4]
+    x = torch.randn(sum(lens), device=dev)
+    out = unpack_reorder_pad(x, lens, order)
+    rows = x.split(lens)
+    assert out.shape == (8, longest)
+    for r, s in enumerate(order):
+        assert torch.equal(out[r, : lens[s]], rows[s]) and not out[r, lens[s] :].any()
+
+
 @pytest.mark.parametrize("pad_value", [0.0, -0.0, 0, 1.0, True])
 def test_pad_fills_every_type(dev, pad_value):
     total, to = 100, 356
