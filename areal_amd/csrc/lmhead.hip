@@ -1386,17 +1386,19 @@ DEVI void stage16_read(const u16* stage, int lane, u32x4 (&v)[4]) {
   for (int p = 0; p < 4; ++p)
     v[p] = *(const u32x4*)((const char*)stage + (p * 4 + (lane >> 4)) * STAGE16_PITCH + (lane & 15) * 16);
 }
-template <bool EDGE, bool STREAM = false>
+// NCOLS < 128 (not EDGE): the sub-tile's width, whose last pieces are left out.
+template <bool EDGE, bool STREAM = false, int NCOLS = 128>
 DEVI void stage16_store(u32x4 (&v)[4], u16* out_row0, int64_t ld, int rows_valid, int cols_valid,
                         int cols_from, int lane) {
   const int piece = lane & 15;
   u16* out = out_row0 + (int64_t)(lane >> 4) * ld + piece * 8;
   // (used here, ahead of the predicates: the compiler would move the reads behind them)
   asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
-  const bool cols = !EDGE || (piece * 8 < cols_valid && piece * 8 >= cols_from);
+  const bool cols = EDGE ? piece * 8 < cols_valid && piece * 8 >= cols_from : NCOLS == 128 || piece * 8 < NCOLS;
+  if (!cols) return;
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
-    if (!EDGE || (cols && p * 4 + (lane >> 4) < rows_valid)) {
+    if (!EDGE || p * 4 + (lane >> 4) < rows_valid) {
       u32x4* dst = (u32x4*)(out + (int64_t)(p * 4) * ld);
       if (STREAM) __builtin_nontemporal_store(v[p], dst);
       else *dst = v[p];
@@ -1414,7 +1416,7 @@ template <bool EDGE, int MODE, int NA_>
 struct Store16Impl {
   static_assert(NA_ == 8 || EDGE, "narrow tiles use the bounds-checked instance");
   static constexpr int NA = NA_, TOKEN_BYTES = 0;
-  // Of a chain (VAR_TN): a whole sub-tile's stores, 8 columns of 4 (bf16) or of NA (fp32, of which the last 48 may be in
+  // Of a chain (VAR_TN): a whole sub-tile's stores, 8 columns of 4 (bf16) or of 8 (fp32, of which the last 48 may be in
   // flight). The other contractions have one tile per workgroup, whose first k-tile then need not wait for its second:
   // dHidden of 509 x 896 147.8 -> 144.3 us, 1024 x 1536 350.8 -> 343.0, from 2048 tokens on alike.
   static constexpr int PENDING_STORES = 0, CHAIN_STORES = MODE == 0 || MODE == 3 ? 32 : 48;
@@ -1424,54 +1426,119 @@ struct Store16Impl {
   static DEVI void close(State&, const Params&, int, int, int, int) {}
   static DEVI void end(State&, const Params&, int, int, int, int) {}
   static DEVI void split_output(Params& p, int64_t bytes) { p.out = (char*)p.out + bytes; }
+  // Most tiles of an EDGE launch are whole and take the body without predicates: one around each store made the
+  // epilogue 7400 clocks instead of 5600.
   static DEVI bool tile(State&, const Params& p, int i0, int j0, int lane, u16* stage, int, const void*) {
-    // bf16: column b leaves the staging area while column b + 1 is fetched and converted
+    const bool complete = !EDGE || (p.N - j0 >= 128 && p.M - i0 >= NA * 16);
+    if (complete) columns<false>(p, i0, j0, lane, stage);
+    else columns<true>(p, i0, j0, lane, stage);
+    return complete;
+  }
+
+  template <bool PART>
+  static DEVI void columns(const Params& p, int i0, int j0, int lane, u16* stage) {
+    if constexpr (MODE == 0 || MODE == 3) columns_bf16<PART>(p, i0, j0, lane, stage);
+    else columns_f32<PART>(p, i0, j0, lane, stage);
+  }
+
+  // Through the staging area, whole lines out (needs 16-byte aligned rows: the host only takes this path when
+  // ldo % 8 == 0 and the output is 16-byte aligned); column b leaves it while column b + 1 is fetched and converted.
+  template <bool PART>
+  static DEVI void columns_bf16(const Params& p, int i0, int j0, int lane, u16* stage) {
     u32x4 left[4];
     int cols_valid = p.M - i0;
     if (NA < 8) cols_valid = cols_valid < NA * 16 ? cols_valid : NA * 16;
     auto store_column = [&](int b) {
-      stage16_store<EDGE>(left, (u16*)p.out + (int64_t)(j0 + b * 16) * p.ldo + i0, p.ldo, p.N - (j0 + b * 16),
-                          cols_valid, 0, lane);
+      stage16_store<PART, false, NA * 16>(left, (u16*)p.out + (int64_t)(j0 + b * 16) * p.ldo + i0, p.ldo,
+                                          p.N - (j0 + b * 16), cols_valid, 0, lane);
     };
+    ML16_AGPR_FENCE();
     for_each_col([&](auto bc) {
       constexpr int b = decltype(bc)::value;
       float x[32];
       acc_col<b>(x);
       const int j = j0 + b * 16 + (lane & 15);
-      if (MODE == 0 || MODE == 3) {
-        // bf16: through the staging area, whole lines out (needs 16-byte aligned rows: the host
-        // only takes this path when ldo % 8 == 0 and the output is 16-byte aligned)
-        float js = 1.f;
-        if (MODE == 3) js = (!EDGE || j < p.N) ? p.jscale[j] : 0.f;
-        u32x2 pk[NA];
+      float js = 1.f;
+      if (MODE == 3) js = (!PART || j < p.N) ? p.jscale[j] : 0.f;
+      u32x2 pk[NA];
 #pragma unroll
-        for (int a = 0; a < NA; ++a) {
-          float x0 = x[a * 4], x1 = x[a * 4 + 1], x2 = x[a * 4 + 2], x3 = x[a * 4 + 3];
-          if (MODE == 3) { x0 *= js; x1 *= js; x2 *= js; x3 *= js; }
-          pk[a][0] = pack_bf16x2(x0, x1);
-          pk[a][1] = pack_bf16x2(x2, x3);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (b > 0) store_column(b - 1);
-#pragma unroll
-        for (int a = 0; a < NA; ++a) stage16_put(stage, lane, a, pk[a]);
-        stage16_read(stage, lane, left);
-        __builtin_amdgcn_sched_barrier(0);
-        if (b == 7) store_column(b);
-      } else {
-#pragma unroll
-        for (int a = 0; a < NA; ++a) {
-          const int i = i0 + a * 16 + 4 * (lane >> 4);
-          if (!EDGE || (j < p.N && i < p.M)) {
-            f32x4* dst = (f32x4*)((float*)p.out + (int64_t)j * p.ldo + i);
-            f32x4 v = {x[a * 4], x[a * 4 + 1], x[a * 4 + 2], x[a * 4 + 3]};
-            if (MODE == 2) v += *dst;
-            *dst = v;
-          }
-        }
+      for (int a = 0; a < NA; ++a) {
+        float x0 = x[a * 4], x1 = x[a * 4 + 1], x2 = x[a * 4 + 2], x3 = x[a * 4 + 3];
+        if (MODE == 3) { x0 *= js; x1 *= js; x2 *= js; x3 *= js; }
+        pk[a][0] = pack_bf16x2(x0, x1);
+        pk[a][1] = pack_bf16x2(x2, x3);
       }
+      __builtin_amdgcn_sched_barrier(0);
+      if (b > 0) store_column(b - 1);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) stage16_put(stage, lane, a, pk[a]);
+      stage16_read(stage, lane, left);
+      __builtin_amdgcn_sched_barrier(0);
+      if (b == 7) store_column(b);
     });
-    return !EDGE || (p.N - j0 >= 128 && p.M - i0 >= NA * 16);
+  }
+
+  // fp32: a column in two halves of 64 values i, each transposed through the staging area as 16 rows of 256 bytes.
+  // Straight from the accumulators a store is 64 bytes of each of 16 rows, which a CU takes at 16 B per clock
+  // (16.5 k clocks for a tile's 256 KB, 8 to 11 k this way) where whole lines go at 62. A half leaves the staging area
+  // while the next one is put there; values to add to are requested AHEAD halves before they are needed (a load is
+  // waited for together with the stores before it). Steps of 16384 x 1536 with fp32 gradients 16.66 -> 16.26 ms.
+  template <bool PART>
+  static DEVI void columns_f32(const Params& p, int i0, int j0, int lane, u16* stage) {
+    constexpr int AHEAD = MODE == 2 ? 4 : 1;
+    u32x4 left[2][4];
+    f32x4 old[AHEAD][4];
+    const int row = lane >> 4, piece = lane & 15;
+    float* const out = (float*)p.out + (int64_t)(j0 + row) * p.ldo + i0 + piece * 4;
+    // half n: rows j0 + 16 (n / 2), values i0 + 64 (n % 2)
+    auto each_row = [&](auto nc, auto&& f) {
+      constexpr int n = decltype(nc)::value;
+      constexpr int width = (NA * 16 - (n & 1) * 64) < 64 ? NA * 16 - (n & 1) * 64 : 64;
+      const bool cols = (width == 64 || piece * 4 < width) && (!PART || i0 + (n & 1) * 64 + piece * 4 < p.M);
+      if (!cols) return;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (!PART || j0 + (n >> 1) * 16 + q * 4 + row < p.N)
+          f(q, (f32x4*)(out + (int64_t)((n >> 1) * 16 + q * 4) * p.ldo + (n & 1) * 64));
+    };
+    auto fetch = [&](auto nc) {
+      constexpr int n = decltype(nc)::value;
+      if constexpr (MODE == 2 && n < 16) each_row(nc, [&](int q, const f32x4* src) { old[n % AHEAD][q] = *src; });
+    };
+    auto store_half = [&](auto nc) {
+      constexpr int n = decltype(nc)::value;
+      auto& v = left[n & 1];
+      asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+      each_row(nc, [&](int q, f32x4* dst) {
+        f32x4 y = __builtin_bit_cast(f32x4, v[q]);
+        if (MODE == 2) y += old[n % AHEAD][q];
+        *dst = y;
+      });
+      fetch(IntC<n + AHEAD>{});
+    };
+    fetch(IntC<0>{});
+    if constexpr (AHEAD > 1) { fetch(IntC<1>{}); fetch(IntC<2>{}); fetch(IntC<3>{}); }
+    ML16_AGPR_FENCE();
+    for_each_col([&](auto bc) {
+      constexpr int b = decltype(bc)::value;
+      float x[32];
+      acc_col<b>(x);
+      auto half = [&](auto hc) {
+        constexpr int h = decltype(hc)::value, n = 2 * b + h;
+#pragma unroll
+        for (int a = 4 * h; a < 4 * h + 4 && a < NA; ++a) {
+          const f32x4 v = {x[a * 4], x[a * 4 + 1], x[a * 4 + 2], x[a * 4 + 3]};
+          *(f32x4*)((char*)stage + piece * STAGE16_PITCH + (a - 4 * h) * 64 + row * 16) = v;
+        }
+        stage16_read(stage, lane, left[n & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (n > 0) store_half(IntC<n - 1>{});
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      half(IntC<0>{});
+      half(IntC<1>{});
+    });
+    store_half(IntC<15>{});
   }
 };
 template <bool EDGE, int MODE> struct Store16 : Store16Impl<EDGE, MODE, 8> {};
