@@ -262,6 +262,12 @@ def emit():
         lines = [f"v_accvgpr_read_b32 %{ia * 4 + r}, a{(ia * 2 + jb // 4) * 16 + (jb % 4) * 4 + r}"
                  for ia in range(8) for r in range(4)]
         out.append(f"#define ML16_READ_COL{jb} \\\n" + cstring(lines))
+    # Half a block column (blocks ia = 4 h .. 4 h + 3) straight to LDS in fp32: 16 bytes of a lane per block, 64 apart.
+    for jb in range(8):
+        for h in range(2):
+            base = [((4 * h + a) * 2 + jb // 4) * 16 + (jb % 4) * 4 for a in range(4)]
+            lines = [f"ds_write_b128 %0, a[{k}:{k + 3}] offset:{a * 64}" for a, k in enumerate(base)]
+            out.append(f"#define ML16_PUT_F32_COL{jb}_{h} \\\n" + cstring(lines))
     out.append("")
     for v in variants:
         n = v.name

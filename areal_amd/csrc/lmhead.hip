@@ -97,30 +97,40 @@ struct Sched {
   int chain;     // flat list: tiles per workgroup
 };
 
-// Tile `step` of workgroup `id` in the flat list.
-DEVI bool flat_decode(const Sched& sc, int id, int step, int& bj, int& ai) {
-  const int xcd = id & 7, n = sc.nbj * sc.nai;
-  const int t0 = (int)((int64_t)xcd * n / 8), t1 = (int)((int64_t)(xcd + 1) * n / 8);
-  const int t = t0 + ((id >> 8) * sc.chain + step) * 32 + ((id >> 3) & 31);
-  if (step >= sc.chain || t >= t1) return false;
-  const int blk = t / (sc.RB * sc.nai), r = t - blk * sc.RB * sc.nai;
-  const int left = sc.nbj - blk * sc.RB, rb = left < sc.RB ? left : sc.RB;
-  ai = r / rb;
-  bj = sc.bj0 + blk * sc.RB + (r - ai * rb);
-  ai += sc.ai0;
-  return true;
-}
+// A workgroup's walk through its XCD's part of the flat list: block `blk` of RB B tiles x all A tiles, place r in it.
+struct FlatWalk {
+  int blk, r, left;  // left: tiles still to come, this one included
+  DEVI bool first(const Sched& sc, int id) {
+    const int xcd = id & 7, n = sc.nbj * sc.nai;
+    const int t0 = (int)((int64_t)xcd * n / 8), t1 = (int)((int64_t)(xcd + 1) * n / 8);
+    const int t = t0 + (id >> 8) * sc.chain * 32 + ((id >> 3) & 31);
+    left = (t1 - t + 31) >> 5;
+    left = left < sc.chain ? left : sc.chain;
+    blk = t / (sc.RB * sc.nai);
+    r = t - blk * sc.RB * sc.nai;
+    return t < t1;
+  }
+  // (RB * nai >= 32, see xcd_block; only the last block is narrower. Divided afresh for every tile the
+  // walk took 850 clocks of a tile's 20000 to 30000 at 256 to 512 tokens.)
+  DEVI void next(const Sched& sc) {
+    r += 32;
+    if (r >= sc.RB * sc.nai) { r -= sc.RB * sc.nai; ++blk; }
+    --left;
+  }
+  DEVI void tile(const Sched& sc, int& bj, int& ai) const {
+    const int rb = sc.nbj - blk * sc.RB;
+    int q, m;
+    if (rb >= sc.RB) { q = r >> __builtin_ctz(sc.RB); m = r & (sc.RB - 1); }
+    else { q = r / rb; m = r - q * rb; }
+    ai = sc.ai0 + q;
+    bj = sc.bj0 + blk * sc.RB + m;
+  }
+};
 
 // z: the workgroup's copy of a split-K launch (XCD layout only; unchanged otherwise).
 DEVI bool sched_decode(const Sched& sc, int id, int& bj, int& split, int& ai_begin, int& ai_end, int& z) {
   const int xcd = id & 7;
   int q = id >> 3;
-  if (sc.xg < 0) {
-    split = 0;
-    if (!flat_decode(sc, id, 0, bj, ai_begin)) return false;
-    ai_end = ai_begin + 1;
-    return true;
-  }
   if (sc.xg > 0) {
     const int ag = xcd % sc.xg, xb = xcd / sc.xg, bgi = xb % sc.bg, kgi = xb / sc.bg;
     const int b0 = bgi * sc.nbj / sc.bg, nb = (bgi + 1) * sc.nbj / sc.bg - b0;
@@ -1108,6 +1118,18 @@ DEVI void acc_col(float (&x)[32]) {
   else if constexpr (JB == 6) asm volatile(ML16_READ_COL6 : ML16_COL_OUTPUTS(x) : : ML16_ACC_CLOBBERS);
   else asm volatile(ML16_READ_COL7 : ML16_COL_OUTPUTS(x) : : ML16_ACC_CLOBBERS);
 }
+// Half n of the 16 half columns in fp32 from the accumulators to LDS (a lane's first byte at addr).
+template <int N>
+DEVI void put_f32(uint32_t addr) {
+#define ML16_PUT(N_, TEXT) if constexpr (N == N_) asm volatile(TEXT : : "v"(addr) : "memory", ML16_ACC_CLOBBERS)
+  ML16_PUT(0, ML16_PUT_F32_COL0_0); ML16_PUT(1, ML16_PUT_F32_COL0_1); ML16_PUT(2, ML16_PUT_F32_COL1_0);
+  ML16_PUT(3, ML16_PUT_F32_COL1_1); ML16_PUT(4, ML16_PUT_F32_COL2_0); ML16_PUT(5, ML16_PUT_F32_COL2_1);
+  ML16_PUT(6, ML16_PUT_F32_COL3_0); ML16_PUT(7, ML16_PUT_F32_COL3_1); ML16_PUT(8, ML16_PUT_F32_COL4_0);
+  ML16_PUT(9, ML16_PUT_F32_COL4_1); ML16_PUT(10, ML16_PUT_F32_COL5_0); ML16_PUT(11, ML16_PUT_F32_COL5_1);
+  ML16_PUT(12, ML16_PUT_F32_COL6_0); ML16_PUT(13, ML16_PUT_F32_COL6_1); ML16_PUT(14, ML16_PUT_F32_COL7_0);
+  ML16_PUT(15, ML16_PUT_F32_COL7_1);
+#undef ML16_PUT
+}
 // Nothing the compiler allocates may sit in an accumulator register across this point. Its
 // register allocator treats free accumulator registers as good homes for long-lived values, and
 // it believes them free after the main loop; with these fences (and the same clobber list on
@@ -1142,6 +1164,8 @@ DEVI int km_window(int first, int nvalid) {
   const int w = (nvalid - TILE + 15) & ~15;
   return w > 0 ? w : 0;
 }
+// Blocks of 16 columns between the window's first column and the tile's.
+DEVI int km_shift(int first, int nvalid) { return (first - km_window(first, nvalid)) >> 4; }
 // LDS read addresses (stage 0) of a k-major operand's fragments: wave row / column W reads the nblk
 // blocks of 16 columns from block W * nblk + shift of the window on (blocks behind the window hold
 // columns past the end, whose results are discarded: they wrap to any block).
@@ -1227,7 +1251,15 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
     wg -= z * per_copy;
     wg = (wg & ~7) | ((wg - z * sc.n_sb) & 7);  // copies start on different XCDs
   }
-  if (!sched_decode(sc, wg, bj, split, ai_begin, ai_end, z)) return;
+  FlatWalk walk{0, 0, 1};
+  if (VAR == VAR_TN && sc.xg < 0) {
+    if (!walk.first(sc, wg)) return;
+    walk.tile(sc, bj, ai_begin);
+    ai_end = ai_begin + 1;
+    split = 0;
+  } else if (!sched_decode(sc, wg, bj, split, ai_begin, ai_end, z)) {
+    return;
+  }
   if (g.ksplit > 1) {
     const int kt0 = z * g.kt_per_split;
     nk -= kt0;
@@ -1303,7 +1335,11 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
     // the chain, or (after the last one) this tile again, whose first k-tiles are loaded and never used
     int ai_next = ai + 1, bj_next = bj;
     bool more = ai_next < ai_end;
-    if (VAR == VAR_TN) more = sc.xg < 0 && flat_decode(sc, wg, step, bj_next, ai_next);
+    if (VAR == VAR_TN) {
+      more = walk.left > 1;
+      walk.next(sc);
+      if (more) walk.tile(sc, bj_next, ai_next);
+    }
     if (!more) { ai_next = ai; bj_next = bj; }
     const char* pa_next = a_tile_ptr(ai_next);
     const char* pb_next = b_tile_ptr(bj_next);
@@ -1361,8 +1397,9 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
     Epi::close(st, ep, bj * TILE + wb * 128, split, wa, lane_e);
     if (!more) break;
     if (VAR == VAR_TN) {
-      if (ai_next != ai) km_fragments(wa, NA, (ai_next * TM - km_window(ai_next * TM, g.acols)) >> 4, 0, lane_e, lds_base, ra);
-      if (bj_next != bj) km_fragments(wb, 8, (bj_next * TILE - km_window(bj_next * TILE, g.bcols)) >> 4, 1, lane_e, lds_base, rb);
+      const int sa = km_shift(ai_next * TM, g.acols), sb = km_shift(bj_next * TILE, g.bcols);
+      if (sa != km_shift(ai * TM, g.acols)) km_fragments(wa, NA, sa, 0, lane_e, lds_base, ra);
+      if (sb != km_shift(bj * TILE, g.bcols)) km_fragments(wb, 8, sb, 1, lane_e, lds_base, rb);
     }
     ai = ai_next;
     bj = bj_next;
@@ -1387,11 +1424,21 @@ DEVI void stage16_read(const u16* stage, int lane, u32x4 (&v)[4]) {
     v[p] = *(const u32x4*)((const char*)stage + (p * 4 + (lane >> 4)) * STAGE16_PITCH + (lane & 15) * 16);
 }
 // NCOLS < 128 (not EDGE): the sub-tile's width, whose last pieces are left out.
+// Byte offsets of a lane's four pieces from the column's first element, the same for every column: the store's address is
+// that element's, in scalar registers, plus 32 bits (15 row pitches: STAGE16_MAX_LD). 64-bit addresses per
+// lane and column took 5 to 10 vector instructions of the column's 80 (plain store) to 300 (softmax).
+struct Pieces16 {
+  uint32_t off[4];
+  DEVI Pieces16(int64_t pitch, int lane) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) off[p] = (uint32_t)(p * 4 + (lane >> 4)) * (uint32_t)pitch + (uint32_t)(lane & 15) * 16;
+  }
+};
+constexpr int64_t STAGE16_MAX_LD = 1 << 26;  // elements, of 2 or 4 bytes
 template <bool EDGE, bool STREAM = false, int NCOLS = 128>
-DEVI void stage16_store(u32x4 (&v)[4], u16* out_row0, int64_t ld, int rows_valid, int cols_valid,
+DEVI void stage16_store(u32x4 (&v)[4], Pieces16& at, u16* out_row0, int rows_valid, int cols_valid,
                         int cols_from, int lane) {
   const int piece = lane & 15;
-  u16* out = out_row0 + (int64_t)(lane >> 4) * ld + piece * 8;
   // (used here, ahead of the predicates: the compiler would move the reads behind them)
   asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
   const bool cols = EDGE ? piece * 8 < cols_valid && piece * 8 >= cols_from : NCOLS == 128 || piece * 8 < NCOLS;
@@ -1399,7 +1446,9 @@ DEVI void stage16_store(u32x4 (&v)[4], u16* out_row0, int64_t ld, int rows_valid
 #pragma unroll
   for (int p = 0; p < 4; ++p) {
     if (!EDGE || p * 4 + (lane >> 4) < rows_valid) {
-      u32x4* dst = (u32x4*)(out + (int64_t)(p * 4) * ld);
+      // (its widening to 64 bits stays beside the store: kept from an earlier block, the two are added in vector registers)
+      asm volatile("" : "+v"(at.off[p]));
+      u32x4* dst = (u32x4*)((char*)out_row0 + at.off[p]);
       if (STREAM) __builtin_nontemporal_store(v[p], dst);
       else *dst = v[p];
     }
@@ -1448,9 +1497,11 @@ struct Store16Impl {
     u32x4 left[4];
     int cols_valid = p.M - i0;
     if (NA < 8) cols_valid = cols_valid < NA * 16 ? cols_valid : NA * 16;
+    Pieces16 at(p.ldo * 2, lane);
+    u16* out = (u16*)p.out + (int64_t)j0 * p.ldo + i0;
     auto store_column = [&](int b) {
-      stage16_store<PART, false, NA * 16>(left, (u16*)p.out + (int64_t)(j0 + b * 16) * p.ldo + i0, p.ldo,
-                                          p.N - (j0 + b * 16), cols_valid, 0, lane);
+      stage16_store<PART, false, NA * 16>(left, at, out, p.N - (j0 + b * 16), cols_valid, 0, lane);
+      out += 16 * p.ldo;
     };
     ML16_AGPR_FENCE();
     for_each_col([&](auto bc) {
@@ -1478,28 +1529,30 @@ struct Store16Impl {
     });
   }
 
-  // fp32: a column in two halves of 64 values i, each transposed through the staging area as 16 rows of 256 bytes.
+  // fp32: a column in two halves of 64 values i, each put into LDS straight from the accumulators and transposed through the staging area as 16 rows of 256 bytes.
   // Straight from the accumulators a store is 64 bytes of each of 16 rows, which a CU takes at 16 B per clock
   // (16.5 k clocks for a tile's 256 KB, 8 to 11 k this way) where whole lines go at 62. A half leaves the staging area
-  // while the next one is put there; values to add to are requested AHEAD halves before they are needed (a load is
+  // while the next two are put there (an LDS operation counted by the compiler is waited for together with the
+  // uncounted ones in front of it); values to add to are requested AHEAD halves before they are needed (a load is
   // waited for together with the stores before it). Steps of 16384 x 1536 with fp32 gradients 16.66 -> 16.26 ms.
   template <bool PART>
   static DEVI void columns_f32(const Params& p, int i0, int j0, int lane, u16* stage) {
     constexpr int AHEAD = MODE == 2 ? 4 : 1;
-    u32x4 left[2][4];
+    u32x4 left[3][4];
     f32x4 old[AHEAD][4];
     const int row = lane >> 4, piece = lane & 15;
-    float* const out = (float*)p.out + (int64_t)(j0 + row) * p.ldo + i0 + piece * 4;
+    const Pieces16 at(p.ldo * 4, lane);
+    char* const out0 = (char*)((float*)p.out + (int64_t)j0 * p.ldo + i0);
     // half n: rows j0 + 16 (n / 2), values i0 + 64 (n % 2)
     auto each_row = [&](auto nc, auto&& f) {
       constexpr int n = decltype(nc)::value;
       constexpr int width = (NA * 16 - (n & 1) * 64) < 64 ? NA * 16 - (n & 1) * 64 : 64;
       const bool cols = (width == 64 || piece * 4 < width) && (!PART || i0 + (n & 1) * 64 + piece * 4 < p.M);
       if (!cols) return;
+      char* const base = out0 + (int64_t)(n >> 1) * 64 * p.ldo + (n & 1) * 256;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if (!PART || j0 + (n >> 1) * 16 + q * 4 + row < p.N)
-          f(q, (f32x4*)(out + (int64_t)((n >> 1) * 16 + q * 4) * p.ldo + (n & 1) * 64));
+        if (!PART || j0 + (n >> 1) * 16 + q * 4 + row < p.N) f(q, (f32x4*)(base + at.off[q]));
     };
     auto fetch = [&](auto nc) {
       constexpr int n = decltype(nc)::value;
@@ -1507,7 +1560,7 @@ struct Store16Impl {
     };
     auto store_half = [&](auto nc) {
       constexpr int n = decltype(nc)::value;
-      auto& v = left[n & 1];
+      auto& v = left[n % 3];
       asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
       each_row(nc, [&](int q, f32x4* dst) {
         f32x4 y = __builtin_bit_cast(f32x4, v[q]);
@@ -1518,26 +1571,22 @@ struct Store16Impl {
     };
     fetch(IntC<0>{});
     if constexpr (AHEAD > 1) { fetch(IntC<1>{}); fetch(IntC<2>{}); fetch(IntC<3>{}); }
+    const uint32_t put = (uint32_t)(uintptr_t)LDS_AS(stage) + piece * STAGE16_PITCH + row * 16;
     ML16_AGPR_FENCE();
     for_each_col([&](auto bc) {
       constexpr int b = decltype(bc)::value;
-      float x[32];
-      acc_col<b>(x);
       auto half = [&](auto hc) {
-        constexpr int h = decltype(hc)::value, n = 2 * b + h;
-#pragma unroll
-        for (int a = 4 * h; a < 4 * h + 4 && a < NA; ++a) {
-          const f32x4 v = {x[a * 4], x[a * 4 + 1], x[a * 4 + 2], x[a * 4 + 3]};
-          *(f32x4*)((char*)stage + piece * STAGE16_PITCH + (a - 4 * h) * 64 + row * 16) = v;
-        }
-        stage16_read(stage, lane, left[n & 1]);
+        constexpr int n = 2 * b + decltype(hc)::value;
+        put_f32<n>(put);
+        stage16_read(stage, lane, left[n % 3]);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (n > 0) store_half(IntC<n - 1>{});
+        if constexpr (n > 1) store_half(IntC<n - 2>{});
         __builtin_amdgcn_sched_barrier(0);
       };
       half(IntC<0>{});
       half(IntC<1>{});
     });
+    store_half(IntC<14>{});
     store_half(IntC<15>{});
   }
 };
@@ -1674,7 +1723,8 @@ struct Fwd16 {
       if (SAVE) rr[b] = ((const float*)tokens)[128 + b * 16 + (lane & 15)];
     }
     const int v_from = overlap ? v_new : v0;
-    float* const label_logit = p.ws + 3 * (int64_t)p.P * p.T;
+    Pieces16 at(SAVE ? p.ldv * 2 : 0, lane);
+    u16* out = SAVE ? p.probs + (int64_t)t0 * p.ldv + v0 : nullptr;
     auto add = [](float a, float b) { return a + b; };
     auto lower = [](float a, float b) { return fminf(a, b); };
     auto upper = [](float a, float b) { return fmaxf(a, b); };
@@ -1769,11 +1819,11 @@ struct Fwd16 {
         }
         asm volatile("" : "+v"(s), "+v"(q) : : ML16_ACC_CLOBBERS);
         __builtin_amdgcn_sched_barrier(0);
-        u16* out = p.probs + (int64_t)(t0 + b * 16) * p.ldv + v0;
         if (!MASKED)
-          stage16_store<false, true>(left, out, p.ldv, 16, 128, 0, lane);
+          stage16_store<false, true>(left, at, out, 16, 128, 0, lane);
         else
-          stage16_store<true, true>(left, out, p.ldv, 16, (int)p.ldv - v0, overlap ? v_new - v0 : 0, lane);
+          stage16_store<true, true>(left, at, out, 16, (int)p.ldv - v0, overlap ? v_new - v0 : 0, lane);
+        out += 16 * p.ldv;
       }
       // the label's logit, if it is one of this lane's 32 entries (about one wave in 70 has one)
       const bool hit = (lab[b] >= v_from) && (lab[b] < v0 + 128);
@@ -1785,7 +1835,7 @@ struct Fwd16 {
           for (int r = 0; r < 4; ++r)
             if (vidx(a, r) == lab[b]) xl = x[a * 4 + r];
         const int t = t0 + b * 16 + (lane & 15);
-        if (hit && t < p.T && (((lab[b] - v0) >> 2) & 3) == group) label_logit[t] = xl;
+        if (hit && t < p.T && (((lab[b] - v0) >> 2) & 3) == group) p.ws[3 * (int64_t)p.P * p.T + t] = xl;
       }
       // The partial results pass through an empty block here: their readers come later (the last
       // one after the last column), and the compiler otherwise moves the summation chains of
@@ -2034,9 +2084,11 @@ struct Bwd16 {
   static DEVI bool tile(State& st, const Params& p, int v0, int t0, int lane, u16* stage, int, const void*) {
     const int vl = v0 + 4 * (lane >> 4);
     u32x4 left[4];  // column b leaves the staging area while column b + 1 is computed
+    Pieces16 at(p.ldv * 2, lane);
+    u16* out = p.dl + (int64_t)t0 * p.ldv + v0;
     auto store_column = [&](int b) {
-      stage16_store<EDGE, true>(left, p.dl + (int64_t)(t0 + b * 16) * p.ldv + v0, p.ldv, p.T - (t0 + b * 16),
-                                (int)p.ldv - v0, 0, lane);
+      stage16_store<EDGE, true>(left, at, out, p.T - (t0 + b * 16), (int)p.ldv - v0, 0, lane);
+      out += 16 * p.ldv;
     };
     for_each_col([&](auto bc) {
       constexpr int b = decltype(bc)::value;
@@ -2120,7 +2172,7 @@ int launch_sched(const GemmArgs& g, const Sched& sc, const typename Epi::Params&
     hipLaunchKernelGGL((gemm16_sweep<VAR, Epi>), dim3(sched_grid(sc) * (g.ksplit > 1 && sc.xg == 0 ? g.ksplit : 1)),
                        dim3(NTHREADS), 0, stream, g, sc, ep);
   } else {
-    if (g.ksplit > 1) return AREAL_ERR_UNSUPPORTED;
+    if (g.ksplit > 1 || sc.xg < 0) return AREAL_ERR_UNSUPPORTED;
     hipLaunchKernelGGL((gemm_nt_generic<Epi>), dim3(sched_grid(sc)), dim3(NTHREADS), 0, stream, g,
                        sc, ep);
   }
@@ -2160,7 +2212,7 @@ void fold_ragged_a(Regions& r, int64_t M) {
 }
 Regions plan_regions(int64_t M, int64_t N, int64_t K, int target_wgs, int S_fixed, bool allow16 = true) {
   Regions r;
-  r.k16 = allow16 && k16_ok(K);
+  r.k16 = allow16 && k16_ok(K) && M <= STAGE16_MAX_LD;
   r.fold_a = false;
   r.layout = nullptr;
   if (r.k16) {
@@ -2248,8 +2300,8 @@ bool narrow_a_tiles(int64_t M) {
 template <int KERNEL16>
 int launch_store(const GemmArgs& g, const StoreParams& ep, int mode, hipStream_t stream,
                  const Sched* layout = nullptr) {
-  bool allow16 = true;
-  if (mode == 0 || mode == 3) allow16 = ep.ldo % 8 == 0 && aligned16(ep.out) && ep.M % 8 == 0;
+  bool allow16 = ep.ldo <= STAGE16_MAX_LD;
+  if (mode == 0 || mode == 3) allow16 = allow16 && ep.ldo % 8 == 0 && aligned16(ep.out) && ep.M % 8 == 0;
   Regions r = plan_regions(ep.M, ep.N, g.K, 0, 1 << 20, allow16);
   Sched flat;
   if (KERNEL16 == KERNEL16_TN && layout == nullptr && g.ksplit <= 1 && dw_flat(g.acols, g.K)) {
