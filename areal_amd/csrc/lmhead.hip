@@ -465,11 +465,14 @@ template <bool E> using StoreBf16Scaled = StoreEpi<E, 3>;
 // the loss gradient) to stay a normal bf16 number. lmhead_merge_kernel checks that with the exact
 // row maximum and raises *status otherwise; the forward then runs again without saving.
 // One wave per REF_TOK tokens (the sampled weight rows are fetched once for all of them), bf16
-// pairs multiplied by v_dot2c_f32_bf16; also clears *status.
+// pairs multiplied by v_dot2c_f32_bf16; also clears *status. For few tokens a block per REF_TOK_SHARED: a wave
+// that walks H alone waits for memory H / 512 times, with most of the chip idle (256 x 896 8.2 -> 5.3 us, 1024 x 4096 17.8 -> 11.2,
+// 509 x 8192 27.0 -> 12.8, 2048 x 896 10.3 -> 7.5; alike at 4096 tokens, 13.6 -> 15.3 at 8192 x 896).
 constexpr int NREF = 8;
-constexpr int REF_TOK = 4;
+constexpr int REF_TOK = 4, REF_TOK_SHARED = 2;
 constexpr float REF_MARGIN = 16.f;
 constexpr float REF_WINDOW = 100.f;
+static bool rowref_shared(int64_t T) { return T <= 2048; }
 
 DEVI float dot8_bf16(u32x4 a, u32x4 b, float acc) {
 #pragma unroll
@@ -482,37 +485,40 @@ DEVI float dot8_bf16(u32x4 a, u32x4 b, float acc) {
   return acc;
 }
 
+// WAVES = 4: the four waves of a block share TOK tokens, each taking a quarter of the hidden size, see rowref_shared.
+template <int TOK, int WAVES>
 __global__ __launch_bounds__(256) void lmhead_rowref_kernel(
     const u16* __restrict__ hidden, const u16* __restrict__ weight, const float* __restrict__ bias,
     const int64_t* __restrict__ labels, int T, int H, int V, float scale, float c2,
     float* __restrict__ row_ref, int* __restrict__ status) {
+  static_assert(WAVES == 1 || WAVES == 4, "a wave, or the block's four, per group of tokens");
   if (blockIdx.x == 0 && threadIdx.x == 0) *status = 0;
-  const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * REF_TOK;
-  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t0 = (WAVES == 1 ? blockIdx.x * 4 + wave : blockIdx.x) * TOK;
   if (t0 >= T) return;
   int ids[NREF];  // ids[0]: replaced per token by its label
 #pragma unroll
   for (int k = 0; k < NREF; ++k) ids[k] = (int)(((int64_t)k * V) / NREF);
-  int lab[REF_TOK];
-  const u16* hrow[REF_TOK];
+  int lab[TOK];
+  const u16* hrow[TOK];
 #pragma unroll
-  for (int j = 0; j < REF_TOK; ++j) {
+  for (int j = 0; j < TOK; ++j) {
     const int t = t0 + j < T ? t0 + j : T - 1;  // a short last group repeats the last token
     const int64_t l = labels[t];
     lab[j] = (l >= 0 && l < V) ? (int)l : ids[0];
     hrow[j] = hidden + (int64_t)t * H;
   }
-  float acc[REF_TOK][NREF];
+  float acc[TOK][NREF];
 #pragma unroll
-  for (int j = 0; j < REF_TOK; ++j)
+  for (int j = 0; j < TOK; ++j)
 #pragma unroll
     for (int k = 0; k < NREF; ++k) acc[j][k] = 0.f;
-  for (int h = lane * 8; h < H; h += 512) {  // H % 8 == 0
+  for (int h = ((WAVES == 1 ? 0 : wave * 64) + lane) * 8; h < H; h += WAVES * 512) {  // H % 8 == 0
     u32x4 wf[NREF];
 #pragma unroll
     for (int k = 1; k < NREF; ++k) wf[k] = *(const u32x4*)(weight + (int64_t)ids[k] * H + h);
 #pragma unroll
-    for (int j = 0; j < REF_TOK; ++j) {
+    for (int j = 0; j < TOK; ++j) {
       const u32x4 hv = *(const u32x4*)(hrow[j] + h);
       const u32x4 lv = *(const u32x4*)(weight + (int64_t)lab[j] * H + h);
       acc[j][0] = dot8_bf16(hv, lv, acc[j][0]);
@@ -520,16 +526,42 @@ __global__ __launch_bounds__(256) void lmhead_rowref_kernel(
       for (int k = 1; k < NREF; ++k) acc[j][k] = dot8_bf16(hv, wf[k], acc[j][k]);
     }
   }
+  if constexpr (WAVES == 1) {
 #pragma unroll
-  for (int j = 0; j < REF_TOK; ++j) {
+    for (int j = 0; j < TOK; ++j) {
+      float mx = neg_inf();
+#pragma unroll
+      for (int k = 0; k < NREF; ++k) {
+        const int id = k == 0 ? lab[j] : ids[k];
+        const float x = (wave_sum(acc[j][k]) + (bias != nullptr ? bias[id] : 0.f)) * scale;
+        mx = fmaxf(mx, x);
+      }
+      if (lane == 0 && t0 + j < T) row_ref[t0 + j] = fmaf(mx, c2, REF_MARGIN);
+    }
+  } else {
+    __shared__ float part[WAVES][TOK * NREF];
+#pragma unroll
+    for (int j = 0; j < TOK; ++j)
+#pragma unroll
+      for (int k = 0; k < NREF; ++k) {
+        const float x = wave_sum(acc[j][k]);
+        if (lane == 0) part[wave][j * NREF + k] = x;
+      }
+    __syncthreads();
+    if (threadIdx.x >= TOK) return;
+    const int t = t0 + (int)threadIdx.x;
+    if (t >= T) return;
+    const int64_t l = labels[t];
     float mx = neg_inf();
 #pragma unroll
     for (int k = 0; k < NREF; ++k) {
-      const int id = k == 0 ? lab[j] : ids[k];
-      const float x = (wave_sum(acc[j][k]) + (bias != nullptr ? bias[id] : 0.f)) * scale;
-      mx = fmaxf(mx, x);
+      float x = 0.f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) x += part[w][threadIdx.x * NREF + k];
+      const int id = k == 0 && l >= 0 && l < V ? (int)l : ids[k];
+      mx = fmaxf(mx, (x + (bias != nullptr ? bias[id] : 0.f)) * scale);
     }
-    if (lane == 0 && t0 + j < T) row_ref[t0 + j] = fmaf(mx, c2, REF_MARGIN);
+    row_ref[t] = fmaf(mx, c2, REF_MARGIN);
   }
 }
 
@@ -724,7 +756,8 @@ template <bool E> using FwdAffineMomSave = FwdEpi<E, true, true, true>;
 // a wave 64 / TOK slots at a time (loads stay coalesced along the tokens), the partial results meet in
 // LDS and wave 0 adds them in a fixed order. Latency-bound: with TOK = 64 the 509 tokens of a short batch
 // are 8 blocks whose waves walk 74 slots one after the other (33 us); TOK = 16 and one pass
-// for the saving sweep's sums take 9.8 (10007 tokens: 18.9 -> 9.9).
+// for the saving sweep's sums take 9.8 (10007 tokens: 18.9 -> 9.9). The slots of a row are read 4 at a time, all
+// requested before the first is used: 256 x 896 (400 slots) 13.6 -> 7.4, 509 x 896 10.4 -> 6.8, 509 x 8192 13.0 -> 7.9.
 // labels (nullable): the slots hold no label logits, a valid label's is entry t of that statistic's plane.
 // ref_sums = 2: the slots hold a reference of their own (in binades) and the sum relative to it, nothing
 // else (Logp16); the final expression is evaluated in fp64 as for 1.
@@ -754,10 +787,18 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
   const int tt = t < T ? t : T - 1;  // lanes past the end repeat the last token and write nothing
   const int64_t PT = (int64_t)P * T;
   const bool moments = vmean != nullptr || vnorm != nullptr;
+  // AHEAD slots' values in flight (past the end the last one's again)
+  constexpr int AHEAD = 4;
+  auto slot = [&](int p0, int k) { return p0 + k * ROWS < P ? p0 + k * ROWS : P - 1; };
   float M = neg_inf();
   if (ref_sums != 1) {  // the sums need the maximum first
-#pragma unroll 4
-    for (int p = row; p < P; p += ROWS) M = fmaxf(M, ws[(int64_t)p * T + tt]);
+    for (int p0 = row; p0 < P; p0 += AHEAD * ROWS) {
+      float m[AHEAD];
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) m[k] = ws[(int64_t)slot(p0, k) * T + tt];
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) M = fmaxf(M, m[k]);
+    }
     sh_f[0][row][tok] = M;
     __syncthreads();
 #pragma unroll
@@ -767,27 +808,42 @@ __global__ __launch_bounds__(64 * MERGE_WAVES) void lmhead_merge_kernel(
   }
   float S = 0.f, Q = 0.f, xl = 0.f, mn = pos_inf();
   double sx = 0.0, sx2 = 0.0;
-#pragma unroll 4
-  for (int p = row; p < P; p += ROWS) {
-    const float* w = ws + (int64_t)p * T + tt;
-    const float m = w[0];
-    if (ref_sums == 2) {
-      S += exp2f(m - M) * w[1 * PT];
-      continue;
+  for (int p0 = row; p0 < P; p0 += AHEAD * ROWS) {
+    float wm[AHEAD], wS[AHEAD], wQ[AHEAD], wl[AHEAD], wn[AHEAD];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) {
+      const float* w = ws + (int64_t)slot(p0, k) * T + tt;
+      wm[k] = w[0];
+      wS[k] = w[1 * PT];
+      wQ[k] = wl[k] = wn[k] = 0.f;
+      if (ref_sums != 2) { wQ[k] = w[2 * PT]; wn[k] = w[4 * PT]; }
+      if (ref_sums != 2 && labels == nullptr) wl[k] = w[3 * PT];
     }
-    if (ref_sums) {
-      M = fmaxf(M, m);
-      S += w[1 * PT];
-      Q += w[2 * PT];
-    } else if (m > neg_inf()) {
-      const float dl = ref_diff(m, M, c2);  // as in the epilogue
-      const float alpha = exp2f(dl);
-      S += alpha * w[1 * PT];
-      Q += alpha * fmaf(dl, w[1 * PT], w[2 * PT]);
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) {
+      if (p0 + k * ROWS >= P) break;
+      if (ref_sums == 2) {
+        S += exp2f(wm[k] - M) * wS[k];
+        continue;
+      }
+      if (ref_sums) {
+        M = fmaxf(M, wm[k]);
+        S += wS[k];
+        Q += wQ[k];
+      } else if (wm[k] > neg_inf()) {
+        const float dl = ref_diff(wm[k], M, c2);  // as in the epilogue
+        const float alpha = exp2f(dl);
+        S += alpha * wS[k];
+        Q += alpha * fmaf(dl, wS[k], wQ[k]);
+      }
+      xl += wl[k];
+      mn = fminf(mn, wn[k]);
+      if (moments) {
+        const float* w = ws + (int64_t)(p0 + k * ROWS) * T + tt;
+        sx += (double)w[5 * PT];
+        sx2 += (double)w[6 * PT];
+      }
     }
-    if (labels == nullptr) xl += w[3 * PT];
-    mn = fminf(mn, w[4 * PT]);
-    if (moments) { sx += (double)w[5 * PT]; sx2 += (double)w[6 * PT]; }
   }
   if (ref_sums == 1) sh_f[0][row][tok] = M;
   sh_f[1][row][tok] = S; sh_f[2][row][tok] = Q; sh_f[3][row][tok] = xl; sh_f[4][row][tok] = mn;
@@ -1060,9 +1116,25 @@ __global__ void splitk_reduce_bf16_kernel(const float* __restrict__ part, int Z,
   const int64_t stride = (int64_t)gridDim.x * blockDim.x * 4;
   for (; i < n; i += stride) {  // n % 4 == 0
     f32x4 a = *(const f32x4*)(part + i);
-    for (int z = 1; z < Z; ++z) {
-      const f32x4 b = *(const f32x4*)(part + (int64_t)z * zstride + i);
-      a[0] += b[0]; a[1] += b[1]; a[2] += b[2]; a[3] += b[3];
+    // AHEAD partial results in flight, added in their order (one at a time the latency of 32 loads was all of it:
+    // 256 x 896 12.9 -> 8.0 us, 509 x 896 13.6 -> 11.2 at 5.2 TB/s, which larger ones had)
+    auto add = [&](const f32x4& b) { a[0] += b[0]; a[1] += b[1]; a[2] += b[2]; a[3] += b[3]; };
+    constexpr int AHEAD = 8, REST = 4;
+    int z = 1;
+    for (; z + AHEAD <= Z; z += AHEAD) {
+      f32x4 b[AHEAD];
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) b[k] = *(const f32x4*)(part + (int64_t)(z + k) * zstride + i);
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) add(b[k]);
+    }
+    for (; z < Z; z += REST) {
+      f32x4 b[REST];
+#pragma unroll
+      for (int k = 0; k < REST; ++k) b[k] = *(const f32x4*)(part + (int64_t)(z + k < Z ? z + k : Z - 1) * zstride + i);
+#pragma unroll
+      for (int k = 0; k < REST; ++k)
+        if (z + k < Z) add(b[k]);
     }
     if (scale != nullptr) {
       const float f = scale[i / row_len];
@@ -2658,9 +2730,14 @@ int areal_lmhead_fwd_ex(const void* hidden, const void* weight, const float* bia
   const bool moments = (vocab_mean != nullptr) || (vocab_norm != nullptr);
   const float c2 = inv_temperature * LOG2E;
   if (probs != nullptr) {
-    hipLaunchKernelGGL(lmhead_rowref_kernel, dim3((unsigned)ceil_div_i64(T, 4 * REF_TOK)), dim3(256), 0, stream,
-                       (const u16*)hidden, (const u16*)weight, bias, labels, (int)T, (int)H, (int)V,
-                       logit_scale, c2, probs_ref, probs_status);
+    if (rowref_shared(T))
+      hipLaunchKernelGGL((lmhead_rowref_kernel<REF_TOK_SHARED, 4>), dim3((unsigned)ceil_div_i64(T, REF_TOK_SHARED)),
+                         dim3(256), 0, stream, (const u16*)hidden, (const u16*)weight, bias, labels, (int)T, (int)H,
+                         (int)V, logit_scale, c2, probs_ref, probs_status);
+    else
+      hipLaunchKernelGGL((lmhead_rowref_kernel<REF_TOK, 1>), dim3((unsigned)ceil_div_i64(T, 4 * REF_TOK)), dim3(256), 0,
+                         stream, (const u16*)hidden, (const u16*)weight, bias, labels, (int)T, (int)H, (int)V,
+                         logit_scale, c2, probs_ref, probs_status);
     AREAL_CHECK_LAUNCH();
   }
   // (each launch_gemm names the epilogue for the hand-scheduled kernel and the one for the generic kernel)
@@ -2677,7 +2754,8 @@ int areal_lmhead_fwd_ex(const void* hidden, const void* weight, const float* bia
     return launch_gemm<Fwd16AffineMomSave, FwdAffineMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
   };
   auto merge = [&](int ref_sums, const float* ref, const int* gate, int gate_run_if_set, int* host) {
-    // blocks of 64 tokens only when they are at least one per CU
+    // blocks of 64 tokens only when they are at least one per CU (blocks of 4 for few tokens: 7.6 us for 7.4 at
+    // 256 x 896, 8.0 for 6.2 at 1024 x 4096)
     const int tok = T >= 64 * 256 ? 64 : 16;
     hipLaunchKernelGGL((tok == 64 ? lmhead_merge_kernel<64> : lmhead_merge_kernel<16>),
                        dim3((unsigned)ceil_div_i64(T, tok)), dim3(64 * MERGE_WAVES), 0, stream,
