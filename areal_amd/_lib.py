@@ -106,6 +106,7 @@ SIGNATURES: dict[str, tuple] = {
     "areal_group_norm_from_segment_stats": (I, [P, P, I64, P, P, I64, I64, I, I, I, I, D, P, P, P]),
     "areal_seqlens_from_mask": (I, [P, I64, I64, P, P, P, P]),
     "areal_seqlens_from_mask_ex": (I, [P, I64, I64, P, P, P, P, P]),
+    "areal_seqlens_from_mask_rows": (I, [P, I64, I64, P, P, P, P, P]),
     "areal_int_to_host": (I, [P, P, P]),
     "areal_pack_padded": (I, [P, P, P, I64, I64, I64, I64, P]),
     "areal_pack_padded_multi": (I, [P, P, P, I, P, I64, I64, I64, P]),

@@ -25,9 +25,10 @@ DEVI int nonzero_bytes(uint32_t x) {
   return __popc(x);
 }
 
-// lens[b] = number of nonzero entries of mask row b (one block per row), 16 mask bytes per load.
+// lens[b] = number of nonzero entries of mask row b (one block per row), 16 mask bytes per load. host (nullable, host
+// memory): the same numbers.
 __global__ __launch_bounds__(PK_THREADS) void rowlens_kernel(const uint8_t* mask, int64_t S,
-                                                             int32_t* lens) {
+                                                             int32_t* lens, double* host) {
   __shared__ int sm[4];
   const uint8_t* row = mask + (int64_t)blockIdx.x * S;
   int len = 0;
@@ -41,7 +42,11 @@ __global__ __launch_bounds__(PK_THREADS) void rowlens_kernel(const uint8_t* mask
   len = wave_sum(len);
   if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = len;
   __syncthreads();
-  if (threadIdx.x == 0) lens[blockIdx.x] = sm[0] + sm[1] + sm[2] + sm[3];
+  if (threadIdx.x == 0) {
+    len = sm[0] + sm[1] + sm[2] + sm[3];
+    lens[blockIdx.x] = len;
+    if (host != nullptr) host[blockIdx.x] = (double)len;
+  }
 }
 
 // Inclusive prefix sum over the wave's 64 lanes: inside each row of 16 through DPP, then the
@@ -414,20 +419,30 @@ extern "C" {
 
 // attention_mask [B, S] bytes (nonzero = token) -> lens [B], cu_seqlens [B+1], *max_len, all
 // int32 on the device (data.py:513-517).
-int areal_seqlens_from_mask_ex(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
-                               int32_t* cu_seqlens, int32_t* max_len, double* host, hipStream_t stream) {
+static int seqlens_from_mask(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens, int32_t* cu_seqlens,
+                             int32_t* max_len, double* host, double* host_lens, hipStream_t stream) {
   if (B < 0 || S < 0) return AREAL_ERR_BAD_ARG;
   if (!cu_seqlens || !max_len || (B > 0 && (!attention_mask || !lens))) return AREAL_ERR_BAD_ARG;
   if (B > (1 << 30) || B * S >= ((int64_t)1 << 31)) return AREAL_ERR_UNSUPPORTED;
   if (B > 0) {
     hipLaunchKernelGGL(rowlens_kernel, dim3((unsigned)B), dim3(PK_THREADS), 0, stream,
-                       attention_mask, S, lens);
+                       attention_mask, S, lens, host_lens);
     AREAL_CHECK_LAUNCH();
   }
   hipLaunchKernelGGL(cu_scan_kernel, dim3(1), dim3(PK_THREADS), 0, stream, lens, B, cu_seqlens,
                      max_len, host);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
+}
+
+int areal_seqlens_from_mask_ex(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
+                               int32_t* cu_seqlens, int32_t* max_len, double* host, hipStream_t stream) {
+  return seqlens_from_mask(attention_mask, B, S, lens, cu_seqlens, max_len, host, nullptr, stream);
+}
+
+int areal_seqlens_from_mask_rows(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
+                                 int32_t* cu_seqlens, int32_t* max_len, double* host_lens, hipStream_t stream) {
+  return seqlens_from_mask(attention_mask, B, S, lens, cu_seqlens, max_len, nullptr, host_lens, stream);
 }
 
 int areal_seqlens_from_mask(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,

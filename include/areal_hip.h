@@ -592,6 +592,9 @@ int areal_seqlens_from_mask(const uint8_t* attention_mask, int64_t B, int64_t S,
 /* The same; host (nullable) is memory of the host that the device can write: {total, longest}. */
 int areal_seqlens_from_mask_ex(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
                                int32_t* cu_seqlens, int32_t* max_len, double* host, areal_stream_t stream);
+/* The same; host_lens (nullable) is such memory of B entries: the rows' lengths, there before the offsets are made. */
+int areal_seqlens_from_mask_rows(const uint8_t* attention_mask, int64_t B, int64_t S, int32_t* lens,
+                               int32_t* cu_seqlens, int32_t* max_len, double* host_lens, areal_stream_t stream);
 /* *host (memory of the host that the device can write) = *value, in stream order. */
 int areal_int_to_host(const int32_t* value, double* host, areal_stream_t stream);
 int areal_pack_padded(const void* padded, void* packed, const int32_t* cu_seqlens, int64_t B,

@@ -84,3 +84,16 @@ def test_nothing_to_move(dev):
     padded, pad, old, _ = pad_packed_tensor_dict(packed, 8)
     assert pad == 5 and old.tolist() == [0, 2, 3] and padded["cu_seqlens"].tolist() == [0, 2, 3, 8]
     assert padded["max_seqlen"] == 5
+
+
+@pytest.mark.parametrize("rows,length", [(1, 1), (7, 33), (512, 17), (513, 17)])
+def test_sizes_either_side_of_the_rows_the_host_adds(dev, rows, length):
+    """Up to 512 rows the host has their lengths, beyond the total and the longest; empty rows, and none but empty ones."""
+    g = torch.Generator().manual_seed(rows)
+    for lens in (torch.randint(0, length + 1, (rows,), generator=g), torch.zeros(rows, dtype=torch.long)):
+        mask = torch.arange(length)[None] < lens[:, None]
+        x = torch.randn(rows, length, generator=g)
+        packed = pack_tensor_dict(dict(attention_mask=mask.to(dev), x=x.to(dev)))
+        assert packed["max_seqlen"] == int(lens.max()) and packed["x"].shape == (int(lens.sum()),)
+        assert torch.equal(packed["cu_seqlens"].cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), lens.cumsum(0)]))
+        assert torch.equal(packed["x"].cpu(), x[mask])
