@@ -8,6 +8,8 @@
 // _min_of, _max_of (:455-560), which reduce every logged tensor under its denominator mask.
 #include "common.hpp"
 
+#include <algorithm>
+
 namespace {
 
 constexpr int PK_THREADS = 256;
@@ -115,33 +117,34 @@ __global__ void int_to_host_kernel(const int32_t* x, double* host) { host[0] = (
 // at clamped indices. With a predicate each, every load was waited for before the next was issued:
 // unpacking 557 Ki tokens of 4 bytes into 256 rows took 18.0 us and takes 4.4, packing six tensors of them
 // 21.9 and 9.4.
-DEVI void block_copy_bytes(char* dst, const char* src, int64_t n) {
+template <int THREADS>
+DEVI void copy_bytes(char* dst, const char* src, int64_t n, int thread) {
   if (n < 16) {
-    if ((int64_t)threadIdx.x < n) dst[threadIdx.x] = src[threadIdx.x];
+    if ((int64_t)thread < n) dst[thread] = src[thread];
     return;
   }
   const int64_t pieces = (n + 15) >> 4;
-  for (int64_t i0 = threadIdx.x; i0 < pieces; i0 += 4 * (int64_t)blockDim.x) {
+  for (int64_t i0 = thread; i0 < pieces; i0 += 4 * THREADS) {
     Bytes16 v[4];
     int64_t at[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int64_t o = 16 * (i0 + u * (int64_t)blockDim.x);
+      const int64_t o = 16 * (i0 + u * THREADS);
       at[u] = o < n - 16 ? o : n - 16;
       v[u] = *(const Bytes16*)(src + at[u]);
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      if (i0 + u * (int64_t)blockDim.x < pieces) *(Bytes16*)(dst + at[u]) = v[u];
+      if (i0 + u * THREADS < pieces) *(Bytes16*)(dst + at[u]) = v[u];
   }
 }
+DEVI void block_copy_bytes(char* dst, const char* src, int64_t n) { copy_bytes<PK_THREADS>(dst, src, n, threadIdx.x); }
 
 // Several tensors packed in one launch. Block (c, k) writes packed tokens [c * chunk, (c + 1) *
 // chunk) of tensor k: it finds the sequence of its first token (every wave searches cu_seqlens
 // with 64 probes per round) and then walks the sequences its chunk touches, each one contiguous
-// run of a padded row to one contiguous run of the packed array. No block is empty. The chunk is
-// 16 KiB of the widest tensor (at most 2048 tokens), so a thread has four loads of 16 bytes in
-// flight at once.
+// run of a padded row to one contiguous run of the packed array. No block is empty. The chunk is at
+// most 16 KiB of the widest tensor and 2048 tokens, a thread has four loads of 16 bytes in flight at once.
 constexpr int PK_MAX_TENSORS = 8;
 constexpr int PK_CHUNK_BYTES = 16384, PK_CHUNK_MAX = 2048;
 struct PackArgs {
@@ -153,6 +156,9 @@ struct PackArgs {
   int64_t S, total;
   int chunk;  // tokens per block
 };
+// BY_WAVE: a chunk's sequences go to the block's four waves in turn, 63 of them known from one load of cu_seqlens (see
+// pack_plan). Bound by the latency of cu_seqlens and the copies for short rows, by HBM from 2 Mi tokens on.
+template <bool BY_WAVE>
 __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
   const int k = blockIdx.y;
   int64_t t = (int64_t)blockIdx.x * a.chunk;
@@ -164,6 +170,22 @@ __global__ __launch_bounds__(PK_THREADS) void pack_rows_kernel(PackArgs a) {
     if (k == i) { src = a.src[i]; dst = a.dst[i]; eb = a.eb[i]; }
   // sequence of token t: the number of sequence ends at or before it (same value in every wave)
   int b = wave_count_le(a.cu + 1, a.n_seqs, t, threadIdx.x & 63);
+  if constexpr (BY_WAVE) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (; b < a.n_seqs; b += 63) {
+      const int entry = a.cu[b + lane < a.n_seqs ? b + lane : a.n_seqs];
+      const int n = a.n_seqs - b < 63 ? a.n_seqs - b : 63;
+      for (int i = wave; i < n; i += PK_THREADS / 64) {
+        const int64_t start = lane_value(entry, i), end = lane_value(entry, i + 1);
+        if (start >= t1) return;
+        const int64_t from = start > t ? start : t, stop = end < t1 ? end : t1;
+        if (stop > from)
+          copy_bytes<64>(dst + from * eb, src + ((int64_t)(b + i) * a.S + (from - start)) * eb, (stop - from) * eb, lane);
+      }
+      if (lane_value(entry, n) >= t1) return;
+    }
+    return;
+  }
   while (t < t1 && b < a.n_seqs) {
     const int64_t start = a.cu[b], end = a.cu[b + 1];
     const int64_t stop = end < t1 ? end : t1;
@@ -200,6 +222,22 @@ DEVI void block_fill_bytes(char* dst, int64_t n, const Fill& f) {
 static int64_t pk_chunk_tokens(int64_t eb) {
   const int64_t c = PK_CHUNK_BYTES / eb;
   return c < 1 ? 1 : (c > PK_CHUNK_MAX ? PK_CHUNK_MAX : c);
+}
+
+// How pack_rows_kernel cuts `total` tokens of `rows` rows. By waves unless a token is wider than 512 bytes: the whole block
+// copies one run after the other, each with its latency, and has most threads idle on runs of under 4 KiB. Six tensors
+// (25 B a token), whole block / waves, us: 1024 rows of mean 105 17.1 / 5.6, 64 of 105 13.7 / 3.7, 1024 of 271 12.5 / 7.5,
+// 512 of 1062 10.5 / 7.9, 256 of 2175 9.8 / 7.8, 512 of 4351 21.1 / 19.2 (5.8 TB/s); wide tokens: 64 rows of 530 x 512 B
+// 8.5 / 8.6, of 530 x 4 KiB 42.8 / 44.3, 8 of 158 x 4 KiB 3.9 / 4.4.
+// Chunks of four runs (two, four, eight, sixteen: 64 rows of mean 66 3.0, 3.6, 4.0, 5.0; 1024 of 271 9.1, 7.9, 7.4, 7.4; 512 of
+// 756 7.9, 6.4, 7.7, 7.7; only 1024 of 74 prefers eight, 5.4 for 7.8), and few rather than full ones while
+// there are less than 128 (8 rows of 4351: 3.3 for 4.1); smaller ones otherwise cost their start (512 of 4351 in 512s 34.2).
+struct PackPlan { bool by_wave; int64_t chunk; };
+static PackPlan pack_plan(int64_t rows, int64_t total, int64_t max_eb) {
+  const int64_t whole = pk_chunk_tokens(max_eb);
+  if (max_eb > 512) return {false, whole};
+  const int64_t runs = round_up_i64(4 * (total / rows + 1), 64), spread = round_up_i64(total / 128 + 1, 256);
+  return {true, std::min(whole, std::min(runs, spread))};
 }
 
 // padded[row][j] = j < len_b ? packed[cu[b] + j] : fill, b = row_seq[row] (or row). Block
@@ -474,12 +512,12 @@ int areal_pack_padded_multi(const void* const* padded, void* const* packed, cons
   }
   int64_t max_eb = 1;
   for (int k = 0; k < n_tensors; ++k) max_eb = elem_bytes[k] > max_eb ? elem_bytes[k] : max_eb;
-  const int64_t chunk = pk_chunk_tokens(max_eb);
+  const auto [by_wave, chunk] = pack_plan(B, total, max_eb);
   const int64_t chunks = ceil_div_i64(total, chunk);
   if (chunks >= ((int64_t)1 << 31) || B > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
   a.cu = cu_seqlens; a.n_seqs = (int)B; a.S = S; a.total = total; a.chunk = (int)chunk;
   const dim3 grid((unsigned)chunks, (unsigned)n_tensors);
-  hipLaunchKernelGGL(pack_rows_kernel, grid, dim3(PK_THREADS), 0, stream, a);
+  hipLaunchKernelGGL((by_wave ? pack_rows_kernel<true> : pack_rows_kernel<false>), grid, dim3(PK_THREADS), 0, stream, a);
   AREAL_CHECK_LAUNCH();
   return AREAL_OK;
 }

@@ -97,3 +97,23 @@ def test_sizes_either_side_of_the_rows_the_host_adds(dev, rows, length):
         assert packed["max_seqlen"] == int(lens.max()) and packed["x"].shape == (int(lens.sum()),)
         assert torch.equal(packed["cu_seqlens"].cpu().long(), torch.cat([torch.zeros(1, dtype=torch.long), lens.cumsum(0)]))
         assert torch.equal(packed["x"].cpu(), x[mask])
+
+
+@pytest.mark.parametrize("rows,length", [(1, 5000), (130, 3), (200, 9), (70, 300), (3, 9000), (64, 2100)])
+@pytest.mark.parametrize("trailing", [(), (128,), (129,)])
+def test_packing_by_waves_and_by_blocks(dev, rows, length, trailing):
+    """Rows from one token to several chunks, runs of empty ones longer than a load of cu_seqlens (63), and tokens
+    either side of the line between the two forms (512 bytes)."""
+    if trailing and rows * length > 30000:
+        pytest.skip("the same chunks as fewer rows")
+    g = torch.Generator().manual_seed(rows + length)
+    lens = torch.randint(0, length + 1, (rows,), generator=g)
+    lens[rows // 4 : rows // 4 + 70] = 0
+    lens[-1] = length
+    mask = torch.arange(length)[None] < lens[:, None]
+    data = dict(attention_mask=mask, x=torch.randn(rows, length, *trailing, generator=g), flag=mask.clone(),
+                ids=torch.randint(0, 1 << 40, (rows, length), generator=g),
+                odd=torch.randint(0, 255, (rows, length, 3), generator=g, dtype=torch.uint8))
+    packed = pack_tensor_dict({k: v.to(dev) for k, v in data.items()})
+    for key in ("x", "flag", "ids", "odd"):
+        assert torch.equal(packed[key].cpu(), data[key][mask]), key
