@@ -66,6 +66,14 @@ def test_sequence_rejection_of_many_sequences(lens, offset, metric, agg):
     test_sequence_rejection(lens, offset, metric, agg)
 
 
+# such a wave reads four steps of 256 tokens (64 unaligned) at once while its lanes have them
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("metric,agg", [("kl_k2", "mean"), ("kl_k3", "max")])
+def test_sequence_rejection_of_waves_with_several_steps(offset, metric, agg):
+    lens = [255, 257, 1023, 1024, 1025, 1027, 1028, 769, 2047, 2049, 5, 4100] + [3, 2] * 2050
+    test_sequence_rejection(lens, offset, metric, agg)
+
+
 @pytest.mark.parametrize("offset", [0, 1])
 @pytest.mark.parametrize("n", [1, 63, 65, 4097, 262144, 262147])
 @pytest.mark.parametrize("cispo", [False, True])
