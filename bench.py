@@ -286,10 +286,10 @@ def hbm_rooflines(dev):
                     ref_logp=torch.randn(1024, 8192, device=dev) * 0.1 - 1, values=vp,
                     rewards=(torch.rand(1024, device=dev) > 0.5).float())
     gnorm = Normalization(NormConfig(mean_level="group", std_level="group", group_size=16))
-    add("adv_gae_kernel + norm_apply_cf_kernel (compute_advantages, API level)",
+    add("adv_gae_kernel (compute_advantages, API level)",
         "config 3 padded form: [1024, 8192], one launch for the reward normalisation, the KL-shaped rewards, GAE and each row's "
-        "masked sums, then the group normalisation as its apply pass alone; 42 + 12 B/slot",
-        54 * rp.numel(),
+        "masked sums, with the group normalisation in it; 42 B/slot",
+        42 * rp.numel(),
         timed(lambda: compute_advantages(dict(adv_data), kl_ctl=0.01, kl_estimator=KLEstimator("k1"),
                                          reward_norm=gnorm, adv_norm=gnorm, discount=1.0, gae_lambda=0.95)))
     del rp, vp, mp, adv_data
