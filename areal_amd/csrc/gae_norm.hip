@@ -193,7 +193,19 @@ DEVI bool gather_sums(const uint64_t* from, const uint64_t* flags, int n, uint64
 DEVI bool note_left(const uint64_t* left, uint64_t call) {
   return __hip_atomic_load(left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == call;
 }
-DEVI void leave_note(uint64_t* left, uint64_t call) { atomicExch((unsigned long long*)left, (unsigned long long)call); }
+// A block that leaves a note and looks at the sums again, and one that publishes its sums and looks for notes, each store
+// to one address and load from another: both loads could be served ahead of both stores, each would miss the other, and
+// the row or segment would stay without its normalisation. So a store and a fence come before the load on either side:
+//   leaver      note    | fence                | flags of the sums
+//   publisher   flag    | wait for its store   | notes
+// Whichever store is performed later, the load behind it sees the earlier one. The publisher's loads go past every cache
+// that is not shared, so that waiting for the store is all of the fence it needs; store and load are of one wave on both
+// sides. It costs nothing that shows: advantages of 64 x 1000 15.0 us, packed GAE of 1024 x 1750 30.4, both as without.
+DEVI void leave_note(uint64_t* left, uint64_t call) {  // by one thread, whose wave looks again
+  atomicExch((unsigned long long*)left, (unsigned long long)call);
+  __threadfence();
+}
+DEVI void published_before_notes() { asm volatile("s_waitcnt vmcnt(0) ; flag out before notes are read" ::: "memory"); }
 DEVI bool take_note(uint64_t* left, uint64_t call) {
   return atomicCAS((unsigned long long*)left, (unsigned long long)call, (unsigned long long)~call) == call;
 }
@@ -1389,7 +1401,7 @@ DEVI float norm_one(const NormParams& p, float x, float m, bool has_mask) {
 // the sizes of groups stands at areal_gae_packed_normalized_ex.
 // No wait is unbounded, as with adv_normalise_row: when the time is up, the block leaves a note for the (tile, group)
 // segment, whose advantages are in memory anyway, and a wave that finds all sums of a group looks for notes of its tiles and
-// takes them. Leaving a note is followed by another look at the sums, publishing comes before the look for notes.
+// takes them. Leaving a note is followed by another look at the sums, publishing comes before the look for notes (leave_note).
 constexpr int SUMS_PITCH = 8;  // words an entry: five sums, their seal, a line of 64 bytes to itself
 struct GaeNormArgs {
   GaeArgs g;
@@ -1449,6 +1461,7 @@ DEVI void gae_tile_normalise(const GaeNormArgs& a, int64_t tile, int64_t lo, int
       return true;
     };
     auto take_notes = [&] {  // of the wave's group
+      published_before_notes();
       for (int64_t kb = k0; kb <= k1; kb += 64) {
         uint64_t notes = __builtin_amdgcn_ballot_w64(kb + lane <= k1 && note_left(a.left + kb + lane + gi, a.call));
         for (; notes != 0; notes &= notes - 1) {
@@ -2108,7 +2121,7 @@ struct AdvGaeArgs {
 // are on the chip together. A block whose time is up stores its row as it is and leaves a note (`left`); it, or any
 // block of the group that finds all sums, then takes the note (one of them, by compare and swap) and normalises that row
 // from memory. Leaving a note is followed by another look at the sums, publishing one's sums precedes the look for notes:
-// of the block that leaves one and the last of the group to publish, one sees the other.
+// of the block that leaves one and the last of the group to publish, one sees the other (the order stands at leave_note).
 constexpr int ADV_GROUP_ROWS = 64;                   // one lane per row
 constexpr int ADV_NORM_TILES = 4;                    // of a row, 8 mask bits each
 struct RowGroup { int g, first, rows; };  // group of a row: its first row and their number
@@ -2145,6 +2158,7 @@ DEVI void adv_normalise_row(const AdvGaeArgs& a, int64_t b, const RowGroup& rg, 
         for (int k = 0; k < 3; ++k) s_sum[k] = v[k];
       }
       if (all) {
+        published_before_notes();
         todo = __builtin_amdgcn_ballot_w64(tid < rg.rows && note_left(a.left + rg.first + tid, a.call));
       }
     }
