@@ -16,6 +16,17 @@ from areal_amd import _lib
 pytestmark = pytest.mark.gpu
 
 
+def _took_one_launch(ws, n, cu, first):
+    """Every tile's flag of each of its groups holds the call's number."""
+    tiles, groups = -(-n // 2048), first.numel() - 1
+    flags = ws.view(torch.int64)[8 * (tiles + groups) : 9 * (tiles + groups)].cpu()
+    slots = []
+    for g, (a, b) in enumerate(zip(cu[first[:-1]].tolist(), cu[first[1:]].tolist())):
+        if a < b:
+            slots += [k + g for k in range(a // 2048, (b - 1) // 2048 + 1)]
+    assert len(set(flags[slots].tolist())) == 1
+
+
 def _run(dev, lens, sizes, levels, wait_us, *, unbiased=1, critic=True, lam=None, mask="binary", around=(0, 0), bad=None, fill=0):
     lib = _lib.load()
     g = torch.Generator().manual_seed(len(lens) + sum(lens))
@@ -53,6 +64,7 @@ def _run(dev, lens, sizes, levels, wait_us, *, unbiased=1, critic=True, lam=None
                        "two launches")
         torch.cuda.synchronize()
         res.append((out, adv, ret))
+    _took_one_launch(ws, n, cu, first)
     for k, (a, b) in enumerate(zip(*res)):
         assert torch.equal(a.isnan(), b.isnan())
         a, b = a.nan_to_num(3.25), b.nan_to_num(3.25)
@@ -87,7 +99,7 @@ def test_same_bits_as_two_launches(dev, case, wait_us):
 
 @pytest.mark.parametrize("wait_us", [-1, 0])
 def test_more_tiles_than_the_chip_holds(dev, wait_us):
-    _run(dev, _lens(1600, 2200, 9), [16] * 100, (2, 2), wait_us)
+    _run(dev, _lens(4800, 700, 9), [4] * 1200, (2, 2), wait_us)
 
 
 @pytest.mark.parametrize("fill", [0, 0, 0, 64, 255])
