@@ -1402,6 +1402,12 @@ DEVI float norm_one(const NormParams& p, float x, float m, bool has_mask) {
 // No wait is unbounded, as with adv_normalise_row: when the time is up, the block leaves a note for the (tile, group)
 // segment, whose advantages are in memory anyway, and a wave that finds all sums of a group looks for notes of its tiles and
 // takes them. Leaving a note is followed by another look at the sums, publishing comes before the look for notes (leave_note).
+// Where not all tiles are on the chip at once, only the last GAE_WAIT_TILES tiles of a group on an XCD wait (it holds 128), the
+// ones before them leave a note at once: all of them waiting would keep the last ones from starting until the time is up, and
+// those would find every note alone. The rule at areal_gae_packed_normalized_ex goes by average lengths, and one group may be far
+// longer. 3200 sequences of 700 tokens and a group of 195 tiles, us: behind them 441 -> 172, in front 491 -> 195, in the middle
+// 112 (two launches 118, 133, 119); a group of 78 tiles 52 (64), eight of 117 126 (109).
+constexpr int GAE_TILES_AT_ONCE = 1024, GAE_WAIT_TILES = 112;
 constexpr int SUMS_PITCH = 8;  // words an entry: five sums, their seal, a line of 64 bytes to itself
 struct GaeNormArgs {
   GaeArgs g;
@@ -1438,6 +1444,7 @@ DEVI void gae_tile_normalise(const GaeNormArgs& a, int64_t tile, int64_t lo, int
     if (gb + GAE_SEG_WAVES <= tg.g_last) __syncthreads();
   }
   const uint64_t deadline = wall_clock64() + a.wait_ticks;
+  const int64_t per_xcd = (gridDim.x + 7) >> 3, xcd_last = ((blockIdx.x & 7) + 1) * per_xcd - 1;
   float r[GAE_ITEMS];
   unsigned keep = 0;  // tokens of groups that were left
 #pragma unroll
@@ -1463,9 +1470,12 @@ DEVI void gae_tile_normalise(const GaeNormArgs& a, int64_t tile, int64_t lo, int
     auto take_notes = [&] {  // of the wave's group
       published_before_notes();
       for (int64_t kb = k0; kb <= k1; kb += 64) {
-        uint64_t notes = __builtin_amdgcn_ballot_w64(kb + lane <= k1 && note_left(a.left + kb + lane + gi, a.call));
-        for (; notes != 0; notes &= notes - 1) {
-          const int64_t k = kb + __builtin_ctzll(notes);
+        for (;;) {
+          const uint64_t notes = __builtin_amdgcn_ballot_w64(kb + lane <= k1 && note_left(a.left + kb + lane + gi, a.call));
+          if (notes == 0) break;
+          // (from the wave's own place on: of those that look together not all try for the same one)
+          const uint64_t behind = notes & (~0ull << (tile & 63));
+          const int64_t k = kb + __builtin_ctzll(behind != 0 ? behind : notes);
           int got = 0;
           if (lane == 0) got = take_note(a.left + k + gi, a.call) ? 1 : 0;
           if (__builtin_amdgcn_readfirstlane(got) == 0) continue;  // somebody else's
@@ -1479,7 +1489,9 @@ DEVI void gae_tile_normalise(const GaeNormArgs& a, int64_t tile, int64_t lo, int
         }
       }
     };
-    const bool ready = mine && gather(deadline);
+    const int64_t to_come = (k1 < xcd_last ? k1 : xcd_last) - tile;  // on this XCD
+    const bool patient = gridDim.x <= GAE_TILES_AT_ONCE || to_come < GAE_WAIT_TILES;
+    const bool ready = mine && gather(patient ? deadline : 0);
     if (lane == 0) {
       s_mean[wave] = mean;
       s_den[wave] = den;
@@ -3016,7 +3028,7 @@ int areal_gae_packed_normalized_ex(const float* rewards, const float* values, co
   // up to 64 tiles; with more tiles the blocks that wait keep those that they wait for from starting. Two launches / one,
   // us (tiles, tiles a group): 875, 14: 32.0 / 27.8; 875, 55: 32.5 / 31.0; 1024, 16: 49.7 / 46.6; 1024, 64: 50.3 / 49.7;
   // 2000, 4: 54.4 / 51.0; 2000, 8: 60.3 / 59.3; 1953, 16: 53.7 / 61.9; 2000, 31: 57.6 / 72.8; 2048, 64: 73.5 / 155.7.
-  const int64_t most_tiles = nb <= 1024 ? 64 : 4;
+  const int64_t most_tiles = nb <= GAE_TILES_AT_ONCE ? 64 : 4;
   const bool one = known && capture == hipStreamCaptureStatusNone && tail_group < 0 && mean_level != LEVEL_BATCH &&
                    std_level != LEVEL_BATCH && nb <= (1 << 29) &&
                    max_group_seqs * ceil_div_i64(n_tokens, n_seqs) <= most_tiles * GAE_TILE &&

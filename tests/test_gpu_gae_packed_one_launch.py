@@ -55,8 +55,11 @@ def _run(dev, lens, sizes, levels, wait_us, *, unbiased=1, critic=True, lam=None
         if fused:
             nbytes = lib.areal_gae_packed_normalized_workspace_bytes(n, len(sizes))
             ws = torch.full((nbytes,), fill, dtype=torch.uint8, device=dev)
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
             _lib.check(lib.areal_gae_packed_normalized_ex(*head, max(sizes), -1, *levels, unbiased, 1e-5, wait_us, p(adv), p(ret),
                                                           p(out), p(ws), nbytes, s), "ex")
+            end.record()
         else:
             nbytes = lib.areal_gae_segment_stats_bytes(n, len(sizes))
             ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
@@ -72,6 +75,7 @@ def _run(dev, lens, sizes, levels, wait_us, *, unbiased=1, critic=True, lam=None
             assert (a - b).abs().max().item() <= 2.0 ** -21 * a.abs().max().item()
         else:
             assert torch.equal(a, b)
+    return begin.elapsed_time(end) * 1e3
 
 
 def _lens(n, mean, seed):
@@ -100,6 +104,17 @@ def test_same_bits_as_two_launches(dev, case, wait_us):
 @pytest.mark.parametrize("wait_us", [-1, 0])
 def test_more_tiles_than_the_chip_holds(dev, wait_us):
     _run(dev, _lens(4800, 700, 9), [4] * 1200, (2, 2), wait_us)
+
+
+@pytest.mark.parametrize("place", [0, 1600, 3200])
+def test_a_group_longer_than_an_xcd_holds(dev, place):
+    """More tiles than the chip holds, 195 of them of one group, 128 of which are on an XCD at once: the others have to start
+    before the time is up that a tile waits at most, here a millisecond (all of the call takes about 0.2)."""
+    lens = _lens(3200, 700, 10)
+    lens[place:place] = [100000] * 4
+    for _ in range(2):  # (the first one loads the kernels)
+        us = _run(dev, lens, [4] * 801, (2, 2), 1000)
+    assert us < 900
 
 
 @pytest.mark.parametrize("fill", [0, 0, 0, 64, 255])
