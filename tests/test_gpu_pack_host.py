@@ -3,6 +3,7 @@
 import pytest
 import torch
 
+from areal_amd import _lib
 from areal_amd.packing import pack_tensor_dict, pad_packed_tensor_dict, unpack_reorder_pad
 from oracle import packing as P
 
@@ -53,6 +54,13 @@ def test_unpack_either_side_of_the_tables_copy(dev, longest):
     assert out.shape == (8, longest)
     for r, s in enumerate(order):
         assert torch.equal(out[r, : lens[s]], rows[s]) and not out[r, lens[s] :].any()
+
+
+def test_a_table_that_cannot_be_held_is_refused(dev):
+    """A kernel reads its table where the host made it only if the pinned allocator keeps that memory for it."""
+    _lib.host().hold_for_reads(torch.zeros(8, 2, dtype=torch.int32, pin_memory=True), 0)
+    with pytest.raises(_lib.ArealHipError, match="pinned"):
+        _lib.host().hold_for_reads(torch.zeros(8, 2, dtype=torch.int32), 0)
 
 
 @pytest.mark.parametrize("pad_value", [0.0, -0.0, 0, 1.0, True])
