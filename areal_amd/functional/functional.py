@@ -144,8 +144,9 @@ class StatReduction:
         extras = dict(extras or {})
         if len(extras) > 2:
             raise ValueError(f"at most two extra statistics ride along, got {len(extras)}")
-        self.entropy = entropy
-        self.extras = extras
+        # a reduction outlives its call and must not hold the graph, and the logits saved in it, with it
+        self.entropy = entropy.detach() if entropy is not None and entropy.requires_grad else entropy
+        self.extras = {k: x.detach() if x.requires_grad else x for k, x in extras.items()}
         # the one per-token output a caller may still need (1 byte per token): the tokens that pass
         # rejection sampling with a positive weight, the denominator of the diagnostics that
         # grpo_loss_fn reduces in a launch of their own

@@ -3,13 +3,14 @@ queued behind that call: the lm_head's backward returns once its forward has fin
 loss call can be read while later work runs. All at sizes where the GPU is busy for milliseconds."""
 
 import functools
+import math
 
 import pytest
 import torch
 
 from areal_amd.config import NormConfig, RejectionSamplingConfig
 from areal_amd.data import KLEstimator, Normalization
-from areal_amd.functional import fused_lm_head_logprobs_entropy
+from areal_amd.functional import fused_lm_head_logprobs_entropy, gather_logprobs_entropy
 from areal_amd.ppo.actor import compute_advantages, grpo_loss_fn
 
 pytestmark = pytest.mark.gpu
@@ -112,3 +113,28 @@ def test_turn_ids_are_checked_without_waiting_for_the_normalisation(dev):
     call(dict(data), adv_norm=adv_norm)
     assert not done[0].query()
     done[0].synchronize()
+
+
+def test_deferred_statistics_do_not_hold_the_logits(dev):
+    """Statistics that nobody has read yet keep the entropies, not the graph with the logits behind them."""
+    n, vocab = 512, 32768
+    data = _loss_data(dev, n, 5)
+    labels = torch.zeros(n, dtype=torch.long, device=dev)
+
+    def step():
+        logits = torch.zeros(n, vocab, device=dev, requires_grad=True)
+        logp, entropy = gather_logprobs_entropy(logits, labels)
+        stats = {}
+        LOSS(logp, entropy, data, stats=stats)
+        return stats
+
+    before = torch.cuda.memory_allocated(dev)
+    stats = step()
+    assert torch.cuda.memory_allocated(dev) - before < 4 * n * vocab
+    assert stats["reduction"].results["entropy"]["avg"] == pytest.approx(math.log(vocab), rel=1e-5)
+
+
+def test_an_entropy_is_asked_for(dev):
+    data = _loss_data(dev, 64, 6)
+    with pytest.raises(AttributeError):
+        LOSS(data["prox_logp"].clone().requires_grad_(True), None, data, stats={})
