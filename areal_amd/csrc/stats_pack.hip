@@ -237,7 +237,8 @@ static PackPlan pack_plan(int64_t rows, int64_t total, int64_t max_eb) {
   const int64_t whole = pk_chunk_tokens(max_eb);
   if (max_eb > 512) return {false, whole};
   const int64_t runs = round_up_i64(4 * (total / rows + 1), 64), spread = round_up_i64(total / 128 + 1, 256);
-  return {true, std::min(whole, std::min(runs, spread))};
+  // (a launch takes less than 2^24 blocks of 256 threads: more than 67 million rows of a few tokens each)
+  return {true, std::max(std::min(whole, std::min(runs, spread)), total / (1 << 23) + 1)};
 }
 
 // padded[row][j] = j < len_b ? packed[cu[b] + j] : fill, b = row_seq[row] (or row). Block

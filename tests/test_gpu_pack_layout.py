@@ -5,6 +5,7 @@ element size; byte for byte against the oracle."""
 import pytest
 import torch
 
+from areal_amd import _lib
 from areal_amd.packing import pack_tensor_dict, pad_packed_tensor_dict, unpack_reorder_pad
 from oracle import packing as P
 
@@ -62,3 +63,15 @@ def test_batch_pad(total, extra, channels):
         got = pad_packed_tensor_dict(_to(data), total + extra, value)
         _same(got[0], want[0])
         assert got[1] == want[1] and torch.equal(got[2].cpu(), want[2])
+
+
+def test_more_short_rows_than_a_launch_has_blocks(dev):
+    """1.2e9 tokens in rows of 12: chunks of five rows are 18.7 million blocks, and a launch takes 2^24 of 256 threads."""
+    rows, length = 100_000_000, 12
+    padded = torch.randint(0, 255, (rows * length,), dtype=torch.uint8, device=dev)
+    packed = torch.zeros_like(padded)
+    cu = torch.arange(0, rows * length + 1, length, dtype=torch.int32, device=dev)
+    rc = _lib.load().areal_pack_padded(_lib.ptr(padded), _lib.ptr(packed), _lib.ptr(cu), rows, length, 1, rows * length,
+                                       _lib.stream_ptr(dev))
+    _lib.check(rc, "areal_pack_padded")
+    assert torch.equal(packed, padded)
