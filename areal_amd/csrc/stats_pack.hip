@@ -13,6 +13,8 @@
 namespace {
 
 constexpr int PK_THREADS = 256;
+// Blocks of a launch: HIP runs one of 2^32 threads or more without its last blocks, and without an error.
+constexpr int64_t PK_MAX_BLOCKS = ((int64_t)1 << 32) / PK_THREADS - 1;
 
 // 16 bytes at any address. The compiler picks the access the target allows for the alignment
 // (gfx950 runs with unaligned access enabled, where this is still one 16-byte instruction).
@@ -462,7 +464,7 @@ static int seqlens_from_mask(const uint8_t* attention_mask, int64_t B, int64_t S
                              int32_t* max_len, double* host, double* host_lens, hipStream_t stream) {
   if (B < 0 || S < 0) return AREAL_ERR_BAD_ARG;
   if (!cu_seqlens || !max_len || (B > 0 && (!attention_mask || !lens))) return AREAL_ERR_BAD_ARG;
-  if (B > (1 << 30) || B * S >= ((int64_t)1 << 31)) return AREAL_ERR_UNSUPPORTED;
+  if (B > PK_MAX_BLOCKS || B * S >= ((int64_t)1 << 31)) return AREAL_ERR_UNSUPPORTED;
   if (B > 0) {
     hipLaunchKernelGGL(rowlens_kernel, dim3((unsigned)B), dim3(PK_THREADS), 0, stream,
                        attention_mask, S, lens, host_lens);
@@ -515,7 +517,7 @@ int areal_pack_padded_multi(const void* const* padded, void* const* packed, cons
   for (int k = 0; k < n_tensors; ++k) max_eb = elem_bytes[k] > max_eb ? elem_bytes[k] : max_eb;
   const auto [by_wave, chunk] = pack_plan(B, total, max_eb);
   const int64_t chunks = ceil_div_i64(total, chunk);
-  if (chunks >= ((int64_t)1 << 31) || B > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
+  if (chunks > PK_MAX_BLOCKS || B > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
   a.cu = cu_seqlens; a.n_seqs = (int)B; a.S = S; a.total = total; a.chunk = (int)chunk;
   const dim3 grid((unsigned)chunks, (unsigned)n_tensors);
   hipLaunchKernelGGL((by_wave ? pack_rows_kernel<true> : pack_rows_kernel<false>), grid, dim3(PK_THREADS), 0, stream, a);
@@ -542,7 +544,7 @@ int areal_unpack_to_padded(const void* packed, void* padded, const int32_t* cu_s
   Fill f;
   if (!make_fill(fill, fill_bytes, f)) return AREAL_ERR_BAD_ARG;
   const int64_t chunk = pk_chunk_tokens(elem_bytes), chunks = ceil_div_i64(S, chunk);
-  if (chunks * B >= ((int64_t)1 << 31)) return AREAL_ERR_UNSUPPORTED;
+  if (chunks * B > PK_MAX_BLOCKS) return AREAL_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(unpack_kernel, dim3((unsigned)(chunks * B)), dim3(PK_THREADS), 0, stream,
                      (const char*)packed, (char*)padded, cu_seqlens, row_seq, S, elem_bytes, f, (int)chunks,
                      (int)chunk);
@@ -558,7 +560,7 @@ int areal_unpack_rows(const void* packed, void* padded, const uint32_t* rows, in
   if (B == 0 || S == 0) return AREAL_OK;
   if (!padded || !rows) return AREAL_ERR_BAD_ARG;
   const int64_t chunk = pk_chunk_tokens(elem_bytes), chunks = ceil_div_i64(S, chunk);
-  if (chunks * B >= ((int64_t)1 << 31)) return AREAL_ERR_UNSUPPORTED;
+  if (chunks * B > PK_MAX_BLOCKS) return AREAL_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(unpack_rows_kernel, dim3((unsigned)(chunks * B)), dim3(PK_THREADS), 0, stream, (const char*)packed,
                      (char*)padded, (const u32x2*)rows, S, elem_bytes, Fill{{0u, 0u, 0u, 0u}, 16}, (int)chunks, (int)chunk);
   AREAL_CHECK_LAUNCH();
@@ -582,7 +584,7 @@ int areal_realign_packed(const void* src, void* dst, const int32_t* cu_old, int6
   Fill f;
   if (!make_fill(fill, fill_bytes, f)) return AREAL_ERR_BAD_ARG;
   const int64_t chunk = pk_chunk_tokens(elem_bytes), chunks = ceil_div_i64(total_new, chunk);
-  if (chunks >= ((int64_t)1 << 31) || n_new > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
+  if (chunks > PK_MAX_BLOCKS || n_new > (1 << 30)) return AREAL_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(realign_kernel, dim3((unsigned)chunks), dim3(PK_THREADS), 0, stream,
                      (const char*)src, (char*)dst, cu_old, (int)n_old, cu_new, (int)n_new,
                      elem_bytes, f, position_ids, total_new, (int)chunk);
@@ -618,6 +620,7 @@ int areal_pad_packed_multi(const void* const* src, void* const* dst, const int64
   a.cu = cu_seqlens; a.cu_copy = cu_copy; a.cu_new = cu_new; a.n_seqs = (int)n_seqs; a.n_tensors = n_tensors;
   a.total = total; a.total_new = total_new; a.chunk = (int)pk_chunk_tokens(max_eb);
   const int64_t chunks = ceil_div_i64(total_new, a.chunk);
+  if (chunks > PK_MAX_BLOCKS) return AREAL_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(pad_packed_kernel, dim3((unsigned)chunks, (unsigned)(n_tensors > 0 ? n_tensors : 1)),
                      dim3(PK_THREADS), 0, stream, a);
   AREAL_CHECK_LAUNCH();

@@ -341,3 +341,15 @@ def test_chunked_lm_head_wrapper_refuses_what_the_reference_refuses():
     with pytest.raises(_lib.ArealHipError):  # valid arguments reach the kernels, which need the GPU
         head(ok, h, w, y, temperature=1.0, chunk_size=4)
 
+
+def test_packing_refuses_more_blocks_than_a_launch_runs():
+    """HIP runs a launch of 2^32 threads or more without its last blocks and without an error: blocks of 256 threads, one to
+    a row or a piece of one, stay below 2^24."""
+    lib = _lib.load()
+    fake, rows = 0x10000, 1 << 24  # never dereferenced: the limit comes first
+    for entry in (lib.areal_seqlens_from_mask_ex, lib.areal_seqlens_from_mask_rows):
+        assert entry(fake, rows, 2, fake, fake, fake, fake, None) == _lib.ERR_UNSUPPORTED
+    assert lib.areal_unpack_to_padded(fake, fake, fake, None, rows, 2, 4, None, 0, None) == _lib.ERR_UNSUPPORTED
+    assert lib.areal_unpack_rows(fake, fake, fake, rows, 2, 4, None) == _lib.ERR_UNSUPPORTED
+    wide = 1 << 14  # bytes of a token, a block each
+    assert lib.areal_realign_packed(fake, fake, fake, 1, fake, 2, wide, None, 0, 0, rows, None) == _lib.ERR_UNSUPPORTED
