@@ -139,9 +139,14 @@ bool hold_until_passed(const Tensor& pinned, const c10::hip::HIPStream& stream) 
   return at::getHostAllocator(at::kCUDA)->record_event(pinned.data_ptr(), pinned.storage().data_ptr().get_context(),
                                                        c10::hip::HIPStreamMasqueradingAsCUDA(stream).unwrap());
 }
-// For memory that a kernel takes addresses or offsets from: in front of its launch, so that nothing reads what may be overwritten.
-void hold_for_reads(const Tensor& pinned, const c10::hip::HIPStream& stream) {
-  if (!hold_until_passed(pinned, stream)) fail("a table in host memory that is not the pinned allocator's");
+// For memory that a queued kernel takes addresses or offsets from: behind the launch, which need not wait for it.
+void hold_or_wait(const Tensor& pinned, const c10::hip::HIPStream& stream) {
+  bool held = false;
+  try {
+    held = hold_until_passed(pinned, stream);
+  } catch (...) {
+  }
+  if (!held) stream.synchronize();  // or the next pinned allocation could overwrite what the kernel reads
 }
 // For results that nobody waited for, in destructors: nothing may be thrown.
 void keep_until_passed(const Tensor& pinned, const c10::hip::HIPStream& stream) noexcept {
@@ -1277,10 +1282,10 @@ OptTensor unpack_rows(const Tensor& packed, const py::list& seqlens, const std::
   const bool direct = out.numel() * out.element_size() <= UNPACK_DIRECT_BYTES;
   const Tensor table = direct ? host : host.to(packed.device(), /*non_blocking=*/true);
   const auto stream = c10::hip::getCurrentHIPStream(src.device().index());
-  if (direct) hold_for_reads(host, stream);
   check(areal_unpack_rows(ptr<void>(src), ptr<void>(out), ptr<uint32_t>(table), n, longest, token_bytes(src, 1),
                           (areal_stream_t)stream.stream()),
         "areal_unpack_rows");
+  if (direct) hold_or_wait(host, stream);
   return out;
 }
 
@@ -1296,8 +1301,8 @@ PYBIND11_MODULE(_host, m) {
       .def("counters", &HostResult::counters)
       .def("mark", &HostResult::mark)
       .def("fill", &HostResult::fill);
-  m.def("hold_for_reads", [](const Tensor& pinned, int64_t device) {
-    hold_for_reads(pinned, c10::hip::getCurrentHIPStream((c10::DeviceIndex)device));
+  m.def("hold_or_wait", [](const Tensor& pinned, int64_t device) {
+    hold_or_wait(pinned, c10::hip::getCurrentHIPStream((c10::DeviceIndex)device));
   });
   m.def("actor_loss", &actor_loss);
   m.def("proximal_stats", &proximal_stats);

@@ -56,11 +56,17 @@ def test_unpack_either_side_of_the_tables_copy(dev, longest):
         assert torch.equal(out[r, : lens[s]], rows[s]) and not out[r, lens[s] :].any()
 
 
-def test_a_table_that_cannot_be_held_is_refused(dev):
-    """A kernel reads its table where the host made it only if the pinned allocator keeps that memory for it."""
-    _lib.host().hold_for_reads(torch.zeros(8, 2, dtype=torch.int32, pin_memory=True), 0)
-    with pytest.raises(_lib.ArealHipError, match="pinned"):
-        _lib.host().hold_for_reads(torch.zeros(8, 2, dtype=torch.int32), 0)
+def test_a_table_that_cannot_be_held_is_waited_for(dev):
+    """A kernel reads its table where the host made it: the pinned allocator keeps that memory for it, or the call waits."""
+    a = torch.ones(8192, 8192, dtype=torch.bfloat16, device=dev)
+    pinned, other = torch.zeros(8, 2, dtype=torch.int32, pin_memory=True), torch.zeros(8, 2, dtype=torch.int32)
+    out = torch.mm(a, a)
+    torch.cuda.synchronize()
+    for table, waits in ((pinned, False), (other, True)):
+        for _ in range(20):  # a millisecond each
+            torch.mm(a, a, out=out)
+        _lib.host().hold_or_wait(table, 0)
+        assert torch.cuda.current_stream().query() == waits
 
 
 @pytest.mark.parametrize("pad_value", [0.0, -0.0, 0, 1.0, True])
