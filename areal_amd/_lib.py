@@ -174,7 +174,6 @@ class LossConfig(ctypes.Structure):
     ]
 
 
-
 class GroupNormSpec(ctypes.Structure):
     """``areal_group_norm_spec``: normalisation within groups of rows."""
 

@@ -134,7 +134,7 @@ DEVI void block_sum_n(double (&v)[N], double* smem /* [4][N] */) {
 // down the ones they waited for: packed GAE
 // of 1.79 Mi tokens 31.4 -> 29.0 us). Whoever reads words that fit has
 // all of them, whatever the memory held before (a chance of 2^-64 an entry otherwise), and nothing has to be cleared.
-// Every word goes through a mix of its own: sums are doubles with few bits set (a count of 512 has one above its
+// Every word goes through a mix of its own (the multipliers of splitmix64): sums are doubles with few bits set (a count of 512 has one above its
 // exponent's), and a sum of their products with odd numbers took entries for whole of which two counts were missing.
 template <int N>
 DEVI uint64_t sums_seal(uint64_t call, const uint64_t (&w)[N]) {
@@ -840,7 +840,9 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
 // once): faster on 64 x 16384 tokens and on 4 x 32768, where a walking block has 16 tiles in a row.
 // The kernel is bound by vector instruction issue (about 1150 vector and 250 scalar instructions
 // per wave and tile on 1024 sequences of mean length 1760) with four blocks resident per CU, so
-// that all blocks of a 1.8 M-token batch run at once; that leaves 128 registers.
+// that all blocks of a 1.8 M-token batch run at once; that leaves 128 registers, of which the instances with group sums
+// spill 6 (28 bytes of scratch a lane). Against a step of a whole tile at a time, which spills none, the two launches that
+// normalise take, us: 1024 x 1750 33.6 -> 33.0, 64 x 8192 38.2 -> 33.5, 4096 x 1000 62.8 -> 62.6, 4096 x 100 57.8 -> 58.8.
 constexpr int GAE_CHUNK = 64 * GAE_ITEMS;  // tokens of a wave's step through the crossing sequence
 constexpr int GAE_CU_LDS = 16 * GAE_THREADS;  // entries of cu_seqlens the block can hold (>= TILE + 2)
 
@@ -2127,7 +2129,7 @@ struct AdvGaeArgs {
 
 // ---- Normalisation in the launch that made the advantages: a row's block keeps them in LDS, hands the row's sums to
 // the blocks of its group and waits for theirs, up to ADV_GROUP_ROWS rows. The batch's advantages then go to memory once
-// instead of being written, read back with the mask and written again by a launch of its own (46 against 54 B a
+// instead of being written, read back with the mask and written again by a launch of its own (42 against 54 B a
 // slot, and 5 us less for a small batch).
 // No wait is unbounded: the blocks of a group lie next to each other in the grid, but nobody promises that they
 // are on the chip together. A block whose time is up stores its row as it is and leaves a note (`left`); it, or any

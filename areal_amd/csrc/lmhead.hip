@@ -1548,7 +1548,7 @@ struct Store16Impl {
   static DEVI void end(State&, const Params&, int, int, int, int) {}
   static DEVI void split_output(Params& p, int64_t bytes) { p.out = (char*)p.out + bytes; }
   // Most tiles of an EDGE launch are whole and take the body without predicates: one around each store made the
-  // epilogue 7400 clocks instead of 5600.
+  // epilogue 7400 clocks instead of 5800 (5100 with the pieces' 32-bit offsets).
   static DEVI bool tile(State&, const Params& p, int i0, int j0, int lane, u16* stage, int, const void*) {
     const bool complete = !EDGE || (p.N - j0 >= 128 && p.M - i0 >= NA * 16);
     if (complete) columns<false>(p, i0, j0, lane, stage);

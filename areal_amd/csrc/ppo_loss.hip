@@ -1100,10 +1100,16 @@ int actor_loss_impl(const float* logprobs, const float* proximal, const float* o
     const bool short_seqs = n_seqs > 4096 && n_tokens <= n_seqs * 384;
     const bool vec = aligned_to(proximal, 16) && aligned_to(old_logprobs, 16) && aligned_to(loss_mask, 4);
     // Otherwise the longest sequence sets the time, a memory latency per step of its block (a second step's loads in flight
-    // cost more than they gave: 21.7 -> 24.4 us in the first of these): as many waves a sequence as the chip holds of all
-    // sequences at once. 4, 8, 16 waves, us, lognormal lengths: 4 Mi tokens in 2048 21.9 / 16.6 / 23.8, in 1100 31.5 / 19.7 /
-    // 20.2, in 8192 18.4 / 25.2 / 62.1; 1 Mi in 512 13.9 / 9.4 / 9.0, in 2600 9.3 / 10.6 / 22.5; 256 Ki in 128 10.6 / 7.4 /
-    // 6.3, in 1024 5.2 / 5.4 / 9.2; 32 Ki in 32 5.6 / 4.8 / 4.8.
+    // cost more than they gave: 21.7 -> 24.4 us in the first of these). More waves a sequence shorten it, and make the other
+    // blocks dearer: a block's start and its sums take as long whatever it has to do, and fewer blocks are on the chip (512 of
+    // 16 waves, 1024 of 8, 2048 of 4). 4, 8, 16 waves, us, lognormal lengths: 4 Mi tokens in 400 80.0 / 43.8 / 26.0, in 600
+    // 50.4 / 29.0 / 20.1, in 1100 29.4 / 18.6 / 19.6, in 1600 24.3 / 17.9 / 23.1, in 2048 20.1 / 15.4 / 22.4, in 2600
+    // 18.0 / 15.7 / 26.0, in 3200 15.9 / 15.9 / 30.5, in 4096 16.6 / 17.4 / 35.6, in 8192 18.4 / 25.2 / 62.1; 2 Mi in 1024 17.6 / 11.6 /
+    // 13.7, in 2048 12.9 / 11.2 / 18.9, in 2600 11.9 / 11.7 / 22.2, in 4000 11.9 / 14.3 / 31.1; 1 Mi in 400 22.0 / 13.2 / 9.2, in 512
+    // 16.1 / 10.6 / 9.8, in 600 14.6 / 9.7 / 10.0, in 1024 9.7 / 7.1 / 11.6, in 2000 8.2 / 8.7 / 16.7, in 2600 9.3 / 10.6 / 22.5; 256 Ki
+    // in 128 10.6 / 7.4 / 6.3, in 1024 5.2 / 5.4 / 9.2; 32 Ki in 32 5.6 / 4.8 / 4.8. 16 and 8 meet between 512 and 1100, 8 and 4 at 2000
+    // for 1 Mi tokens and at 3200 for 4 Mi. The lines are 512 and 2048; behind 2048 of 4 Mi tokens 8 waves would take 15 % less, behind 512
+    // of them, 7000 tokens a sequence, 16 waves 30 % less.
     const int waves = short_seqs ? 1 : n_seqs > 2048 || n_tokens < n_seqs * 512 || !vec ? 4 : n_seqs > 512 ? 8 : 16;
     const dim3 grid_s((unsigned)(short_seqs ? ceil_div_i64(n_seqs, LOSS_THREADS / 64) : n_seqs));
     const dim3 block(waves > 4 ? 64 * waves : LOSS_THREADS);

@@ -694,9 +694,10 @@ def compute_advantages(
             rewards, values, loss_mask, turn_ids, True, seq_no_eos_mask, discount, gae_lambda, gae_kl_rewards
         )
     else:
-        # With padded rows and a normalisation that needs one statistics pass, the GAE kernel
-        # sums each row's advantages under the mask while it writes them, and the normalisation
-        # is its apply pass alone: two launches for the two stages (same results).
+        # With padded rows and a normalisation that needs one statistics pass, the advantages come out
+        # normalised from the launch that makes them (no row sums then). Where that launch does not take the
+        # batch, the GAE kernel sums each row's advantages under the mask while it writes them and the
+        # normalisation is its apply pass alone: two launches (same results).
         fused = None
         if one_pass and rewards.ndim == 2:
             fused = _token_level_gae_with_row_stats(

@@ -247,7 +247,7 @@ def hbm_rooflines(dev):
     add("gae_tile_kernel + norm_stats5_kernel + norm_apply_cf_kernel (C ABI)",
         f"config 3: 1024 packed sequences, {T} tokens, GAE then group normalisation of the advantages, "
         "launches back to back, 20 + 20 B/token", 40 * T, timed(gae_then_norm))
-    # the same in two launches (what compute_gae_packed_normalized queues): the GAE kernel leaves the
+    # the same in two launches (captured calls, and what one launch does not take): the GAE kernel leaves the
     # per-(tile, group) sums of its advantages, the apply pass of the normalisation starts from them
     gseq = torch.arange(0, 1025, 16, device=dev, dtype=torch.int64)
     seg_n = lib_.areal_gae_segment_stats_bytes(T, 64)
@@ -261,8 +261,21 @@ def hbm_rooflines(dev):
 
     add("gae_tile_kernel<stats> + norm_apply_seg_kernel (C ABI)",
         f"config 3: 1024 packed sequences, {T} tokens, GAE that leaves the normalisation's sums, then the apply "
-        "pass: two launches, 20 + 20 B/token", 40 * T, timed(gae_stats_then_apply))
-    del adv_o, ret_o, nrm_o, seg
+        "pass: two launches, 20 + 12 B/token", 32 * T, timed(gae_stats_then_apply))
+    # and in one (what compute_gae_packed_normalized queues at this size)
+    one_n = lib_.areal_gae_packed_normalized_workspace_bytes(T, 64)
+    one = L_.workspace(one_n, dev)
+
+    def gae_normalised():
+        rc = lib_.areal_gae_packed_normalized_ex(L_.ptr(r), L_.ptr(v), L_.ptr(m), L_.ptr(cu), None, None, T, 1024, 1.0,
+                                                 0.95, L_.ptr(gseq), L_.ptr(grow), 64, 16, -1, 2, 2, 1, 1e-5, -1,
+                                                 L_.ptr(adv_o), L_.ptr(ret_o), L_.ptr(nrm_o), L_.ptr(one), one_n, strm)
+        assert rc == 0
+
+    add("gae_tile_norm_kernel (C ABI)",
+        f"config 3: 1024 packed sequences, {T} tokens, GAE and the normalisation of its advantages in one launch, "
+        "24 B/token", 24 * T, timed(gae_normalised))
+    del adv_o, ret_o, nrm_o, seg, one
     # the padded drop-in signature on the same batch: [1024, 8192] (8.39 M slots)
     from areal_amd.ppo.gae import _compute_token_level_gae
 
