@@ -96,6 +96,7 @@ def sapo_loss_fn(
         extras[1] if len(extras) > 1 else None,
     )
     if red is not None:
+        red._detach_inputs()
         n = loss_mask.numel()
         red._fill_sapo(host, n)  # the one wait for the GPU of the call
         n_valid = red.denominators["n_valid_tokens"]

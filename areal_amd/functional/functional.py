@@ -144,9 +144,8 @@ class StatReduction:
         extras = dict(extras or {})
         if len(extras) > 2:
             raise ValueError(f"at most two extra statistics ride along, got {len(extras)}")
-        # a reduction outlives its call and must not hold the graph, and the logits saved in it, with it
-        self.entropy = entropy.detach() if entropy is not None and entropy.requires_grad else entropy
-        self.extras = {k: x.detach() if x.requires_grad else x for k, x in extras.items()}
+        self.entropy = entropy
+        self.extras = extras
         # the one per-token output a caller may still need (1 byte per token): the tokens that pass
         # rejection sampling with a positive weight, the denominator of the diagnostics that
         # grpo_loss_fn reduces in a launch of their own
@@ -155,6 +154,15 @@ class StatReduction:
         self._results: dict[str, dict[str, float | None]] = {}
         self._denominators: dict[str, float] = {}
         self._pending = None  # (host result, arguments of _fill) of a call with deferred host reads
+
+    def _detach_inputs(self) -> None:
+        """A reduction outlives its call and must not hold the inputs' graph, and the logits saved in it, with it. Behind
+        the call's launches, where the GPU does not wait for it."""
+        if self.entropy is not None and self.entropy.requires_grad:
+            self.entropy = self.entropy.detach()
+        for k, x in self.extras.items():
+            if x.requires_grad:
+                self.extras[k] = x.detach()
 
     def _resolve(self) -> None:
         if self._pending is not None:
@@ -383,6 +391,7 @@ def _loss_common(cfg, logprobs, proximal_logprobs, old_logprobs, advantages, los
     if defer:
         host.mark()  # whoever reads the results waits for this call, not for what is queued behind it
     if reduction is not None:
+        reduction._detach_inputs()
         if reduction.keep_behave_mask:
             reduction.behave_mask = out.get("behave_mask")
         args = (host, loss_mask.numel(), rejection_sampling is not None, want_old)

@@ -108,8 +108,8 @@ def grpo_loss_fn(
     if stats_mode not in ("tensors", "reduced"):
         raise ValueError(f"stats_mode must be 'tensors' or 'reduced', got {stats_mode!r}")
     reduction = None
-    if entropy.requires_grad:  # (only then: a detach is two microseconds)
-        entropy = entropy.detach()
+    if entropy is None:
+        raise AttributeError("grpo_loss_fn takes the entropies, also where no statistics are asked for")
     versions = input_data.get("versions")
     # with token versions the reduced mode evaluates further per-token tensors under the behave mask
     versioned = versions is not None and current_version is not None
@@ -258,7 +258,7 @@ def grpo_loss_fn(
             approx_kl=stat["approx_kl"],
             new_logp=lp,
             old_logp=old_logp,
-            entropy=entropy.float(),
+            entropy=entropy.detach().float(),
             actor_loss=stat["loss"],
             clip_ratio=out["clip_ratio"],
             dual_clip_ratio=out["dual_clip_ratio"],

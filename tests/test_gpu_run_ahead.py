@@ -10,7 +10,8 @@ import torch
 
 from areal_amd.config import NormConfig, RejectionSamplingConfig
 from areal_amd.data import KLEstimator, Normalization
-from areal_amd.functional import fused_lm_head_logprobs_entropy, gather_logprobs_entropy
+from areal_amd.functional import StatReduction, fused_lm_head_logprobs_entropy, gather_logprobs_entropy
+from areal_amd.ppo import actor
 from areal_amd.ppo.actor import compute_advantages, grpo_loss_fn
 
 pytestmark = pytest.mark.gpu
@@ -115,23 +116,31 @@ def test_turn_ids_are_checked_without_waiting_for_the_normalisation(dev):
     done[0].synchronize()
 
 
-def test_deferred_statistics_do_not_hold_the_logits(dev):
-    """Statistics that nobody has read yet keep the entropies, not the graph with the logits behind them."""
+@pytest.mark.parametrize("options", [dict(), dict(defer_host_reads=False), dict(use_sapo_loss=True, rejection_sampling=None)])
+def test_statistics_do_not_hold_the_logits(dev, options, monkeypatch):
+    """A reduction keeps the entropies, read or not, but not the graph with the logits behind them."""
     n, vocab = 512, 32768
     data = _loss_data(dev, n, 5)
     labels = torch.zeros(n, dtype=torch.long, device=dev)
 
+    kept = []
+
+    class Kept(StatReduction):
+        def __init__(self, *args, **kwargs):
+            super().__init__(*args, **kwargs)
+            kept.append(self)
+
+    monkeypatch.setattr(actor, "StatReduction", Kept)
+
     def step():
         logits = torch.zeros(n, vocab, device=dev, requires_grad=True)
         logp, entropy = gather_logprobs_entropy(logits, labels)
-        stats = {}
-        LOSS(logp, entropy, data, stats=stats)
-        return stats
+        LOSS(logp, entropy, data, stats={}, **options)
 
     before = torch.cuda.memory_allocated(dev)
-    stats = step()
+    step()
     assert torch.cuda.memory_allocated(dev) - before < 4 * n * vocab
-    assert stats["reduction"].results["entropy"]["avg"] == pytest.approx(math.log(vocab), rel=1e-5)
+    assert kept[0].results["entropy"]["avg"] == pytest.approx(math.log(vocab), rel=1e-5)
 
 
 def test_an_entropy_is_asked_for(dev):
