@@ -15,6 +15,7 @@
 // recurrence. Maps are held in fp64 (five coefficients); outputs are rounded to fp32.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <random>
 
 #include "common.hpp"
@@ -2731,9 +2732,16 @@ void launch_gae_owned(const GaeArgs& g, int64_t grid, hipStream_t stream) {
   }
 }
 
+uint64_t call_seed() noexcept {  // (random_device may throw, and no exception may leave a C entry)
+  try {
+    return ((uint64_t)std::random_device{}() << 32) ^ std::random_device{}();
+  } catch (...) {
+    return (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() * 0x9e3779b97f4a7c15ull;
+  }
+}
 // A number no other call has, and no memory by chance.
 uint64_t next_call_number() {
-  static const uint64_t seed = ((uint64_t)std::random_device{}() << 32) ^ std::random_device{}();
+  static const uint64_t seed = call_seed();
   static std::atomic<uint64_t> calls{0};
   uint64_t z = seed + (calls.fetch_add(1, std::memory_order_relaxed) + 1) * 0x9e3779b97f4a7c15ull;  // splitmix64
   z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
