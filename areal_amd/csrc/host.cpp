@@ -816,7 +816,7 @@ py::tuple lm_head(const Tensor& hidden, const Tensor& weight, const OptTensor& b
 // ---------------------------------------------------------------------------------------
 struct Logits : public torch::autograd::Function<Logits> {
   static variable_list forward(AutogradContext* ctx, const Tensor& logits, const Tensor& labels, double temperature,
-                               bool with_entropy) {
+                               bool with_entropy, bool needs_grad) {
     const int64_t V = logits.size(-1);
     Tensor rows = logits.scalar_type() == at::kFloat || logits.scalar_type() == at::kBFloat16 ? logits
                                                                                             : logits.to(at::kFloat);
@@ -826,7 +826,7 @@ struct Logits : public torch::autograd::Function<Logits> {
     const Tensor lab = flat(labels, at::kLong);
     const Tensor lp = empty(rows, labels.sizes(), at::kFloat);
     const Tensor ent = with_entropy ? empty(rows, labels.sizes(), at::kFloat) : Tensor();
-    const Tensor lse2 = empty_f32(rows, T);
+    const Tensor lse2 = needs_grad ? empty_f32(rows, T) : Tensor();
     check(areal_logits_logprobs_entropy_fwd(ptr<void>(rows), rows.scalar_type() == at::kBFloat16 ? 1 : 0,
                                             T > 1 ? rows.stride(0) : V, ptr<int64_t>(lab), T, V,
                                             (float)(1.0 / temperature), ptr<float>(lp), ptr<float>(ent),
@@ -841,7 +841,7 @@ struct Logits : public torch::autograd::Function<Logits> {
     return {lp};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    variable_list r(4);
+    variable_list r(5);
     const Tensor glp_arg = grads[0], gen_arg = grads.size() > 1 ? grads[1] : Tensor();
     if (!glp_arg.defined() && !gen_arg.defined()) return r;
     const auto saved = ctx->get_saved_variables();
@@ -866,7 +866,7 @@ struct Logits : public torch::autograd::Function<Logits> {
 variable_list logits_logprobs(const Tensor& logits, const Tensor& labels, double temperature, bool with_entropy) {
   require_gpu(logits, labels);
   const c10::hip::HIPGuard guard(logits.device().index());
-  return Logits::apply(logits, labels, temperature, with_entropy);
+  return Logits::apply(logits, labels, temperature, with_entropy, wants_grad(logits));
 }
 
 // ---------------------------------------------------------------------------------------

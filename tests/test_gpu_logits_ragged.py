@@ -70,3 +70,31 @@ def test_logits_that_are_not_finite(dev, value, vocab, rows):
         want_lp, want_ent = L.gather_logprobs_entropy(x, y)
         torch.testing.assert_close(lp.cpu(), want_lp, rtol=1e-5, atol=2e-5, equal_nan=True)
         torch.testing.assert_close(ent.cpu(), want_ent, rtol=1e-5, atol=2e-5, equal_nan=True)
+
+
+# bytes either side of the rule on how many rows the forward keeps in the memory-side cache for the backward: none of a
+# batch left out, a few, and more than half of one above 512 MB
+@pytest.mark.parametrize("rows", [1046, 1047, 1100, 2200])
+def test_rows_kept_for_the_backward(dev, rows):
+    """Same bits whether a row is kept or not (a forward without a gradient keeps none); against 64 bits either side of the line."""
+    vocab = 128256
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = (torch.randn(rows, vocab, generator=g, device=dev) * 2).bfloat16()
+    y = torch.randint(0, vocab, (rows,), generator=g, device=dev)
+    w = torch.randn(rows, generator=g, device=dev)
+    xg = x.detach().requires_grad_(True)
+    lp, ent = gather_logprobs_entropy(xg, y)
+    with torch.no_grad():
+        plain_lp, plain_ent = gather_logprobs_entropy(x, y)
+    assert torch.equal(lp, plain_lp) and torch.equal(ent, plain_ent)
+    (lp * w).sum().backward()
+    size = 2 * vocab
+    line = ((256 if rows * size <= 512 << 20 else 320) << 20) // size
+    at = sorted({i for i in (0, 1, line - 1, line, rows - 2, rows - 1) if 0 <= i < rows})
+    logp = torch.log_softmax(x[at].double(), -1)
+    pick = (torch.arange(len(at), device=dev), y[at])
+    torch.testing.assert_close(lp[at].double(), logp[pick], rtol=1e-5, atol=2e-5)
+    torch.testing.assert_close(ent[at].double(), -(logp.exp() * logp).sum(-1), rtol=1e-5, atol=2e-5)
+    want = -logp.exp() * w[at, None].double()
+    want[pick] += w[at].double()
+    torch.testing.assert_close(xg.grad[at].double(), want, rtol=1e-2, atol=1e-6)
