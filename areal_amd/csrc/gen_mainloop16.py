@@ -25,7 +25,8 @@ order is the one written here, whatever the compiler would have scheduled:
 
 Operand layouts: ``kc`` = k contiguous (row = i or j, 128 B of k per stage row, 16-byte chunks
 XOR-swizzled), ``km`` = k major (row = k, 512 B of i or j per stage row, fetched with
-``ds_read_b64_tr_b16``).  Variants: nt = (kc, kc), tn = (km, km), mix = (km, kc).
+``ds_read_b64_tr_b16``).  Variants: nt = (kc, kc), tn = (km, km), mix = (km, kc); nts and mixs are nt and
+mix with the A operand's loads under the non-temporal hint.
 
 An odd number of k-tiles runs as one more pair whose second k-tile is "dead": it keeps the
 pipeline's loads, fragment reads and barriers (the next output tile's first two k-tiles arrive in
@@ -54,8 +55,8 @@ OPER_BYTES = 2 * HALF_BYTES   # both stages of one operand
 
 
 class Variant:
-    def __init__(self, name: str, a_km: bool, b_km: bool):
-        self.name, self.km = name, (a_km, b_km)
+    def __init__(self, name: str, a_km: bool, b_km: bool, stream_a: bool = False):
+        self.name, self.km, self.stream_a = name, (a_km, b_km), stream_a
         top = 256
 
         def alloc(n):
@@ -96,7 +97,8 @@ class Variant:
         imm = oper * OPER_BYTES + stage * HALF_BYTES + i * 1024
         ptr = S_PA if oper == 0 else S_PB
         return (f"s_add_u32 m0, s{S_LDSW}, {imm}",
-                f"global_load_lds_dwordx4 v{self.off[oper] + i}, s[{ptr}:{ptr + 1}]")
+                f"global_load_lds_dwordx4 v{self.off[oper] + i}, s[{ptr}:{ptr + 1}]"
+                + (" nt" if self.stream_a and oper == 0 else ""))
 
     @staticmethod
     def advance(oper, eff=False):
@@ -241,7 +243,8 @@ def cstring(lines):
 
 
 def emit():
-    variants = [Variant("NT", False, False), Variant("TN", True, True), Variant("MIX", True, False)]
+    variants = [Variant("NT", False, False), Variant("TN", True, True), Variant("MIX", True, False),
+                Variant("NTS", False, False, True), Variant("MIXS", True, False, True)]
     out = ["// Generated by gen_mainloop16.py: do not edit.", "#pragma once", ""]
     out += [f"#define ML16_S_PA \"{{s[{S_PA}:{S_PA + 1}]}}\"", f"#define ML16_S_PB \"{{s[{S_PB}:{S_PB + 1}]}}\"",
             f"#define ML16_S_PA_NEXT \"{{s[{S_PA_NEXT}:{S_PA_NEXT + 1}]}}\"",
@@ -271,15 +274,16 @@ def emit():
     out.append("")
     for v in variants:
         n = v.name
-        out.append(f"// ---- {n}: A {'k-major' if v.km[0] else 'k-contiguous'}, "
+        out.append(f"// ---- {n}: A {'k-major' if v.km[0] else 'k-contiguous'}{', streamed' if v.stream_a else ''}, "
                    f"B {'k-major' if v.km[1] else 'k-contiguous'}; asm block uses v[{v.first_vgpr}:255]")
-        out.append(f"#define ML16_{n}_FIRST_VGPR {v.first_vgpr}")
-        ins = [f'"{{v{v.off[0] + i}}}"(oa[{i}])' for i in range(8)]
-        ins += [f'"{{v{v.off[1] + i}}}"(ob[{i}])' for i in range(8)]
-        ins += [f'"{{v{v.rd[0] + i}}}"(ra[{i}])' for i in range(8 if v.km[0] else 2)]
-        ins += [f'"{{v{v.rd[1] + i}}}"(rb[{i}])' for i in range(8 if v.km[1] else 2)]
-        out.append(f"#define ML16_{n}_VGPR_INPUTS(oa, ob, ra, rb) " + ", ".join(ins))
-        out.append(f"#define ML16_{n}_CLOBBERS " + ", ".join(f'"{c}"' for c in v.clobbers()))
+        if not v.stream_a:  # (the registers are those of the variant without the hint)
+            out.append(f"#define ML16_{n}_FIRST_VGPR {v.first_vgpr}")
+            ins = [f'"{{v{v.off[0] + i}}}"(oa[{i}])' for i in range(8)]
+            ins += [f'"{{v{v.off[1] + i}}}"(ob[{i}])' for i in range(8)]
+            ins += [f'"{{v{v.rd[0] + i}}}"(ra[{i}])' for i in range(8 if v.km[0] else 2)]
+            ins += [f'"{{v{v.rd[1] + i}}}"(rb[{i}])' for i in range(8 if v.km[1] else 2)]
+            out.append(f"#define ML16_{n}_VGPR_INPUTS(oa, ob, ra, rb) " + ", ".join(ins))
+            out.append(f"#define ML16_{n}_CLOBBERS " + ", ".join(f'"{c}"' for c in v.clobbers()))
         out.append(f"#define ML16_{n}_PROLOGUE \\\n" + cstring(v.prologue()))
         out.append(f"#define ML16_{n}_TILE \\\n" + cstring(v.tile_loop()))
         if v.km[0]:  # narrower A tiles exist for a k-major A (its tile column is a lane offset)

@@ -227,6 +227,18 @@ static double xcd_distinct(int nb, int S) {
   return d;
 }
 
+// Whether the exponentials stay in the memory-side cache (256 MB) for the two contractions of the backward: they are then
+// written without the non-temporal hint, and what passes through once, the weight (forward, dHidden) and its bf16 gradient,
+// goes under it. Short batches spend most of a k-tile waiting for memory (2600 to 3000 clocks for 2050). Kernels, us,
+// before / so, forward, dWeight, dHidden: 509 x 896 153, 154, 119 / 137, 137, 124; 256 x 896 108, 114, 93 / 94, 94, 104; 300 x
+// 2048 290, 277, 231 / 272, 235, 232; 400 x 5120 620, 699, 550 / 588, 645, 552; 700 x 896 237, 210, 176 / 223, 198, 181 (222 MB of
+// exponentials; dHidden in front of dWeight 225, 211, 183). With more of them than the cache holds the hints only cost: steps
+// of 1000 x 1024 (304 MB) 822 / 829, of 4096 x 896 2600 / 2760. A weight that fits it itself is not streamed.
+constexpr int64_t PAST_PROBS_MOST = (int64_t)224 << 20, PAST_WEIGHT_LEAST = (int64_t)240 << 20;
+static bool past_cache(int64_t T, int64_t H, int64_t V) {
+  return round_up_i64(T, 2 * BK) * round_up_i64(V, BK) * 2 <= PAST_PROBS_MOST && V * H * 2 >= PAST_WEIGHT_LEAST;
+}
+
 // The layout of a sweep of nai A tiles against each of nbj B tiles of nk k-tiles: the numbers of A
 // groups and of splits that the busiest XCD's 32 CUs finish first. A tile takes about 1.2 us per
 // k-tile (H = 896 to 5120) and 11 us for its softmax epilogue, a workgroup's start and end 5 us more
@@ -1310,6 +1322,7 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
   __shared__ __attribute__((aligned(1024))) unsigned char lds[RING16_BYTES + 4 * (STAGE16_BYTES + Epi::TOKEN_BYTES)];
   constexpr bool A_KM = VAR != VAR_NT, B_KM = VAR == VAR_TN;
   constexpr int NA = Epi::NA;
+  constexpr bool STREAM_A = Epi::PAST && VAR != VAR_TN;
   static_assert(NA == 8 || (NA == 7 && A_KM), "narrow A tiles need a k-major A");
   constexpr int TM = NA * 32;  // A rows (output index i) per tile
   // Stores that every complete epilogue leaves in flight: the next tile starts without waiting for them.
@@ -1374,24 +1387,17 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
   const uint32_t pen_a = odd ? 0u : stride_a, pen_b = odd ? 0u : stride_b;
   u16* stage = (u16*)(lds + RING16_BYTES + wave * STAGE16_BYTES);
 
-  if (VAR == VAR_NT)
-    asm volatile(ML16_NT_PROLOGUE
-                 : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb)
-                 : ML16_S_LDSW(ldsw), ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b),
-                   ML16_NT_VGPR_INPUTS(oa, ob, ra, rb)
-                 : "memory", "scc");
-  else if (VAR == VAR_TN)
-    asm volatile(ML16_TN_PROLOGUE
-                 : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb)
-                 : ML16_S_LDSW(ldsw), ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b),
-                   ML16_TN_VGPR_INPUTS(oa, ob, ra, rb)
-                 : "memory", "scc");
-  else
-    asm volatile(ML16_MIX_PROLOGUE
-                 : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb)
-                 : ML16_S_LDSW(ldsw), ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b),
-                   ML16_MIX_VGPR_INPUTS(oa, ob, ra, rb)
-                 : "memory", "scc");
+#define ML16_PROLOGUE_ASM(TEXT, V)                                                                    \
+  asm volatile(TEXT : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb)                                            \
+               : ML16_S_LDSW(ldsw), ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b),             \
+                 ML16_##V##_VGPR_INPUTS(oa, ob, ra, rb)                                               \
+               : "memory", "scc")
+  if constexpr (VAR == VAR_NT && STREAM_A) ML16_PROLOGUE_ASM(ML16_NTS_PROLOGUE, NT);
+  else if constexpr (VAR == VAR_NT) ML16_PROLOGUE_ASM(ML16_NT_PROLOGUE, NT);
+  else if constexpr (VAR == VAR_TN) ML16_PROLOGUE_ASM(ML16_TN_PROLOGUE, TN);
+  else if constexpr (STREAM_A) ML16_PROLOGUE_ASM(ML16_MIXS_PROLOGUE, MIX);
+  else ML16_PROLOGUE_ASM(ML16_MIX_PROLOGUE, MIX);
+#undef ML16_PROLOGUE_ASM
 
   // what the epilogue needs to know of the wave's 128 output rows j, from LDS at every tile of the sweep
   unsigned char* const tokens = lds + RING16_BYTES + 4 * STAGE16_BYTES + wave * Epi::TOKEN_BYTES;
@@ -1417,46 +1423,22 @@ __global__ __launch_bounds__(NTHREADS) void gemm16_sweep(GemmArgs g, Sched sc, t
     const char* pb_next = b_tile_ptr(bj_next);
     int cnt = npairs;
     if (npairs == 1) { pa = pa_next; pb = pb_next; }
-    if (VAR == VAR_NT)
-      asm volatile(ML16_NT_TILE
-                   : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
-                   : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
-                     ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_NT_VGPR_INPUTS(oa, ob, ra, rb),
-                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
-                   : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_NT_CLOBBERS, ML16_ACC_CLOBBERS);
-    else if (VAR == VAR_TN && NA == 7)
-      asm volatile(ML16_TN_TILE7
-                   : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
-                   : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
-                     ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_TN_VGPR_INPUTS(oa, ob, ra, rb),
-                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
-                   : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_TN_CLOBBERS, ML16_ACC_CLOBBERS);
-    else if (VAR == VAR_TN)
-      asm volatile(ML16_TN_TILE
-                   : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
-                   : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
-                     ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_TN_VGPR_INPUTS(oa, ob, ra, rb),
-                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
-                   : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_TN_CLOBBERS, ML16_ACC_CLOBBERS);
-    else if (NA == 7)
-      asm volatile(ML16_MIX_TILE7
-                   : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
-                   : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
-                     ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_MIX_VGPR_INPUTS(oa, ob, ra, rb),
-                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
-                   : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_MIX_CLOBBERS, ML16_ACC_CLOBBERS);
-    else
-      asm volatile(ML16_MIX_TILE
-                   : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)
-                   : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),
-                     ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),
-                     ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_MIX_VGPR_INPUTS(oa, ob, ra, rb),
-                     [pending] "n"(PENDING), [landed] "n"(8 + PENDING)
-                   : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_MIX_CLOBBERS, ML16_ACC_CLOBBERS);
+#define ML16_TILE_ASM(TEXT, V)                                                                                 \
+  asm volatile(TEXT : "+" ML16_S_PA(pa), "+" ML16_S_PB(pb), "+" ML16_S_CNT(cnt)                                \
+               : ML16_S_PA_NEXT(pa_next), ML16_S_PB_NEXT(pb_next), ML16_S_LDSW(ldsw),                          \
+                 ML16_S_STRIDE_A(stride_a), ML16_S_STRIDE_B(stride_b), ML16_S_ODD(odd),                        \
+                 ML16_S_PEN_A(pen_a), ML16_S_PEN_B(pen_b), ML16_##V##_VGPR_INPUTS(oa, ob, ra, rb),             \
+                 [pending] "n"(PENDING), [landed] "n"(8 + PENDING)                                             \
+               : "memory", "scc", ML16_S_SCRATCH_CLOBBERS, ML16_##V##_CLOBBERS, ML16_ACC_CLOBBERS)
+    if constexpr (VAR == VAR_NT && STREAM_A) ML16_TILE_ASM(ML16_NTS_TILE, NT);
+    else if constexpr (VAR == VAR_NT) ML16_TILE_ASM(ML16_NT_TILE, NT);
+    else if constexpr (VAR == VAR_TN && NA == 7) ML16_TILE_ASM(ML16_TN_TILE7, TN);
+    else if constexpr (VAR == VAR_TN) ML16_TILE_ASM(ML16_TN_TILE, TN);
+    else if constexpr (NA == 7 && STREAM_A) ML16_TILE_ASM(ML16_MIXS_TILE7, MIX);
+    else if constexpr (NA == 7) ML16_TILE_ASM(ML16_MIX_TILE7, MIX);
+    else if constexpr (STREAM_A) ML16_TILE_ASM(ML16_MIXS_TILE, MIX);
+    else ML16_TILE_ASM(ML16_MIX_TILE, MIX);
+#undef ML16_TILE_ASM
     // The lane number goes through an empty block so that nothing of the epilogue's per-lane
     // address arithmetic is computed ahead of the main loop, which leaves the compiler only
     // v[0:ML16_*_FIRST_VGPR) for values that live across it.
@@ -1533,10 +1515,12 @@ DEVI void stage16_put(u16* stage, int lane, int ia, u32x2 v) {
 // ---- plain store (dHidden, dWeight, stand-alone GEMM): out[j * ldo + i]
 // NA < 8: the wave's sub-tile has only NA blocks of 16 values i (gemm16_sweep's narrow A tiles); the
 // bounds of the EDGE instance then also stop at the sub-tile's width.
-template <bool EDGE, int MODE, int NA_>
+// PAST (see past_cache): dHidden's weight (its A operand) and dWeight's bf16 output under the non-temporal hint.
+template <bool EDGE, int MODE, int NA_, bool PAST_>
 struct Store16Impl {
   static_assert(NA_ == 8 || EDGE, "narrow tiles use the bounds-checked instance");
   static constexpr int NA = NA_, TOKEN_BYTES = 0;
+  static constexpr bool PAST = PAST_;
   // Of a chain (VAR_TN): a whole sub-tile's stores, 8 columns of 4 (bf16) or of 8 (fp32, of which the last 48 may be in
   // flight). The other contractions have one tile per workgroup, whose first k-tile then need not wait for its second:
   // dHidden of 509 x 896 147.8 -> 144.3 us, 1024 x 1536 350.8 -> 343.0, from 2048 tokens on alike.
@@ -1572,7 +1556,7 @@ struct Store16Impl {
     Pieces16 at(p.ldo * 2, lane);
     u16* out = (u16*)p.out + (int64_t)j0 * p.ldo + i0;
     auto store_column = [&](int b) {
-      stage16_store<PART, false, NA * 16>(left, at, out, p.N - (j0 + b * 16), cols_valid, 0, lane);
+      stage16_store<PART, PAST, NA * 16>(left, at, out, p.N - (j0 + b * 16), cols_valid, 0, lane);
       out += 16 * p.ldo;
     };
     ML16_AGPR_FENCE();
@@ -1662,12 +1646,14 @@ struct Store16Impl {
     store_half(IntC<15>{});
   }
 };
-template <bool EDGE, int MODE> struct Store16 : Store16Impl<EDGE, MODE, 8> {};
-template <int MODE> struct Store16Narrow : Store16Impl<true, MODE, 7> {};
+template <bool EDGE, int MODE, bool PAST = false> struct Store16 : Store16Impl<EDGE, MODE, 8, PAST> {};
+template <int MODE, bool PAST = false> struct Store16Narrow : Store16Impl<true, MODE, 7, PAST> {};
 template <bool E> using Store16Bf16 = Store16<E, 0>;
 template <bool E> using Store16F32 = Store16<E, 1>;
 template <bool E> using Accum16F32 = Store16<E, 2>;
 template <bool E> using Store16Bf16Scaled = Store16<E, 3>;
+template <bool E> using Store16Bf16Past = Store16<E, 0, true>;
+template <bool E> using Store16F32Past = Store16<E, 1, true>;
 
 
 // ---- forward: online softmax statistics (see FwdEpi). In a block column the 16 lanes l % 16 own
@@ -1719,9 +1705,11 @@ constexpr float MASKED_LOGIT = -1e30f;
 // all 128 rows, those past the end being rows [T, round_up(T, 128)) of the saved buffer (cleared
 // before anything reads them). Row predicates on the stores instead cost 4 to 7 % of the sweep, and
 // a launch of its own for the ragged tile kept 1 / S of the chip busy for the length of a sweep.
-template <bool EDGE, bool AFFINE, bool MOMENTS, bool SAVE>
+// PAST (see past_cache): the weight is read under the non-temporal hint and the exponentials written without it.
+template <bool EDGE, bool AFFINE, bool MOMENTS, bool SAVE, bool PAST_ = false>
 struct Fwd16 {
   static constexpr int NA = 8;
+  static constexpr bool PAST = PAST_;
   static constexpr bool RAGGED_B = true;
   static constexpr int TOKEN_BYTES = 1024;
   // An interior tile's: 8 columns of 4. Waiting for them before the next tile starts cost 1.5 to 3 % of the
@@ -1892,9 +1880,9 @@ struct Fwd16 {
         asm volatile("" : "+v"(s), "+v"(q) : : ML16_ACC_CLOBBERS);
         __builtin_amdgcn_sched_barrier(0);
         if (!MASKED)
-          stage16_store<false, true>(left, at, out, 16, 128, 0, lane);
+          stage16_store<false, !PAST>(left, at, out, 16, 128, 0, lane);
         else
-          stage16_store<true, true>(left, at, out, 16, (int)p.ldv - v0, overlap ? v_new - v0 : 0, lane);
+          stage16_store<true, !PAST>(left, at, out, 16, (int)p.ldv - v0, overlap ? v_new - v0 : 0, lane);
         out += 16 * p.ldv;
       }
       // the label's logit, if it is one of this lane's 32 entries (about one wave in 70 has one)
@@ -1978,6 +1966,7 @@ template <bool E> using Fwd16PlainMom = Fwd16<E, false, true, false>;
 template <bool E> using Fwd16Affine = Fwd16<E, true, false, false>;
 template <bool E> using Fwd16AffineMom = Fwd16<E, true, true, false>;
 template <bool E> using Fwd16PlainSave = Fwd16<E, false, false, true>;
+template <bool E> using Fwd16PlainSavePast = Fwd16<E, false, false, true, !E>;
 template <bool E> using Fwd16PlainMomSave = Fwd16<E, false, true, true>;
 template <bool E> using Fwd16AffineSave = Fwd16<E, true, false, true>;
 template <bool E> using Fwd16AffineMomSave = Fwd16<E, true, true, true>;
@@ -2002,6 +1991,7 @@ constexpr float LOGP_NO_REF = -3e38f;   // so far below every logit that the fir
 template <bool EDGE, bool AFFINE>
 struct Logp16 {
   static constexpr int NA = 8;
+  static constexpr bool PAST = false;
   static constexpr bool RAGGED_B = true;
   static constexpr int TOKEN_BYTES = 1024, PENDING_STORES = 0;
   typedef FwdParams Params;
@@ -2127,6 +2117,7 @@ template <bool E> using Logp16Affine = Logp16<E, true>;
 template <bool EDGE, bool AFFINE>
 struct Bwd16 {
   static constexpr int NA = 8;
+  static constexpr bool PAST = false;
   static constexpr bool RAGGED_B = EDGE;
   static constexpr int TOKEN_BYTES = 0, PENDING_STORES = 0;
   typedef BwdParams Params;
@@ -2371,7 +2362,9 @@ bool narrow_a_tiles(int64_t M) {
 // layout: of the hand-scheduled kernel's tiles (null: super-blocks).
 template <int KERNEL16>
 int launch_store(const GemmArgs& g, const StoreParams& ep, int mode, hipStream_t stream,
-                 const Sched* layout = nullptr) {
+                 const Sched* layout = nullptr, bool past = false) {
+  // (past_cache has these two)
+  constexpr int PAST_MODE = KERNEL16 == KERNEL16_TN ? 0 : KERNEL16 == KERNEL16_MIX ? 1 : -1;
   bool allow16 = ep.ldo <= STAGE16_MAX_LD;
   if (mode == 0 || mode == 3) allow16 = allow16 && ep.ldo % 8 == 0 && aligned16(ep.out) && ep.M % 8 == 0;
   Regions r = plan_regions(ep.M, ep.N, g.K, 0, 1 << 20, allow16);
@@ -2388,11 +2381,18 @@ int launch_store(const GemmArgs& g, const StoreParams& ep, int mode, hipStream_t
     if (r.k16 && mode != UNUSED_MODE && narrow_a_tiles(ep.M)) {
       const int nai = (int)ceil_div_i64(ep.M, TILE), nbj = (int)ceil_div_i64(ep.N, TILE);
       const Sched sc = layout != nullptr ? *layout : make_sched(0, nbj, 0, nai, nai, g.sb_wgs == 8 ? 8 : 32);
+      if constexpr (PAST_MODE >= 0) {
+        if (past && mode == PAST_MODE) return launch_sched<Store16Narrow<PAST_MODE, true>, KERNEL16>(g, sc, ep, stream);
+      }
       if (mode == 0) return launch_sched<Store16Narrow<0>, KERNEL16>(g, sc, ep, stream);
       if (mode == 1) return launch_sched<Store16Narrow<1>, KERNEL16>(g, sc, ep, stream);
       constexpr int LAST_MODE = KERNEL16 == KERNEL16_TN ? 2 : 3;
       return launch_sched<Store16Narrow<LAST_MODE>, KERNEL16>(g, sc, ep, stream);
     }
+  }
+  if (past && mode == PAST_MODE) {
+    if constexpr (PAST_MODE == 0) return launch_gemm<Store16Bf16Past, StoreBf16, StoreParams, KERNEL16, false>(g, r, ep, ep, stream);
+    if constexpr (PAST_MODE == 1) return launch_gemm<Store16F32Past, StoreF32, StoreParams, KERNEL16, false>(g, r, ep, ep, stream);
   }
   switch (mode) {
     case 0: return launch_gemm<Store16Bf16, StoreBf16, StoreParams, KERNEL16, false>(g, r, ep, ep, stream);
@@ -2497,7 +2497,7 @@ bool dh_weight_in_place(int64_t V) { return V % BK == 0 && V >= 2 * BK; }
 // dh_weight_in_place(V), else its transposed copy W^T [H, ldv].
 template <int KERNEL16>
 int launch_dhidden_k(const GemmArgs& g0, int64_t H, int64_t T, int64_t ldv, void* dhidden,
-                     float* partial, const float* tscale, int z_fixed, hipStream_t stream) {
+                     float* partial, const float* tscale, int z_fixed, hipStream_t stream, bool past = false) {
   GemmArgs g = g0;
   const DhPlan plan = plan_dh(H, T, ldv, z_fixed);
   int z = plan.z;
@@ -2511,7 +2511,7 @@ int launch_dhidden_k(const GemmArgs& g0, int64_t H, int64_t T, int64_t ldv, void
   g.kt_per_split = kps;
   g.zstride = T * H * (int64_t)sizeof(float);
   const StoreParams ep{partial, H, (int)H, (int)T, nullptr};
-  int rc = launch_store<KERNEL16>(g, ep, 1, stream, &plan.sc);
+  int rc = launch_store<KERNEL16>(g, ep, 1, stream, &plan.sc, past);
   if (rc != AREAL_OK) return rc;
   int64_t blocks = ceil_div_i64(T * H, 256 * 4);
   if (blocks > 65535) blocks = 65535;
@@ -2526,7 +2526,7 @@ int launch_dhidden(const u16* w, int64_t V, const u16* dl, int64_t ldv, int64_t 
   if (dh_weight_in_place(V)) {
     GemmArgs g{w, H, (int)H, dl, ldv, (int)T, (int)ldv, (int)H, 0};
     g.skip_if_set = skip_if_set;
-    return launch_dhidden_k<KERNEL16_MIX>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream);
+    return launch_dhidden_k<KERNEL16_MIX>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream, past_cache(T, H, V));
   }
   GemmArgs g{w, ldv, (int)H, dl, ldv, (int)T, (int)ldv, 0, 0};
   g.skip_if_set = skip_if_set;
@@ -2597,17 +2597,18 @@ size_t dw_tail_bytes(int64_t H, int64_t V, int64_t Tpad) {
 int launch_dweight_bf16(GemmArgs g, int64_t H, int64_t V, int64_t ldv, void* dweight, float* dw_part,
                         hipStream_t stream) {
   const int64_t K = g.K;
+  const bool past = past_cache(K, H, V);
   const DwTail tail = dw_part != nullptr ? plan_dw_tail(H, V, K) : DwTail{0, 1, 0, 0, 32};
   int rc;
   if (tail.z <= 1) {
     const StoreParams ep{dweight, H, (int)H, (int)V, nullptr};
-    return launch_store<KERNEL16_TN>(g, ep, 0, stream);
+    return launch_store<KERNEL16_TN>(g, ep, 0, stream, nullptr, past);
   }
   const int64_t v0 = (int64_t)tail.nbj_main * TILE;
   GemmArgs gm = g;
   gm.N = (int)v0;
   const StoreParams ep{dweight, H, (int)H, (int)v0, nullptr};
-  rc = launch_store<KERNEL16_TN>(gm, ep, 0, stream);
+  rc = launch_store<KERNEL16_TN>(gm, ep, 0, stream, nullptr, past);
   if (rc != AREAL_OK) return rc;
   GemmArgs gt = g;
   gt.B = g.B + v0;
@@ -2748,6 +2749,8 @@ int areal_lmhead_fwd_ex(const void* hidden, const void* weight, const float* bia
     return launch_gemm<Fwd16AffineMom, FwdAffineMom, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
   };
   auto fwd_save = [&](const GemmArgs& gg) {
+    if (!affine && !moments && past_cache(T, H, V))
+      return launch_gemm<Fwd16PlainSavePast, FwdPlainSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
     if (!affine && !moments) return launch_gemm<Fwd16PlainSave, FwdPlainSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
     if (!affine) return launch_gemm<Fwd16PlainMomSave, FwdPlainMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
     if (!moments) return launch_gemm<Fwd16AffineSave, FwdAffineSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
@@ -2989,32 +2992,38 @@ int areal_lmhead_bwd_saved(const void* hidden, const void* weight, const int64_t
                      (int)H, (int)V, inv_temperature * LOG2E, inv_temperature * logit_scale, rowfac,
                      dweight != nullptr ? hs : nullptr, probs_status);
   AREAL_CHECK_LAUNCH();
-  if (dhidden != nullptr) {
+  auto dhidden_launches = [&]() -> int {
+    if (dhidden == nullptr) return AREAL_OK;
     if (!w_in_place) {
       hipLaunchKernelGGL(transpose_pad_bf16_kernel,
                          dim3((unsigned)ceil_div_i64(H, 64), (unsigned)ceil_div_i64(ldv, 64)),
                          dim3(256), 0, stream, (const u16*)weight, H, (int)V, (int)H, wT, ldv);
       AREAL_CHECK_LAUNCH();
     }
-    if ((rc = launch_dhidden(w_in_place ? (const u16*)weight : wT, V, e, ldv, H, T, dhidden, dh_part,
-                             rowfac, probs_status, 0, stream)) != AREAL_OK)
-      return rc;
-  }
-  if (dbias != nullptr) {
-    hipLaunchKernelGGL(colsum_bf16_kernel, dim3((unsigned)ceil_div_i64(V, 64)), dim3(256), 0, stream,
-                       e, ldv, T, (int)V, dweight_mode == 1 ? 1 : 0, (const float*)rowfac, dbias, probs_status);
-    AREAL_CHECK_LAUNCH();
-  }
-  if (dweight != nullptr) {
+    return launch_dhidden(w_in_place ? (const u16*)weight : wT, V, e, ldv, H, T, dhidden, dh_part, rowfac, probs_status, 0,
+                          stream);
+  };
+  auto dweight_launches = [&]() -> int {
+    if (dweight == nullptr) return AREAL_OK;
     // dWeight[v, h] += sum_t e'[t, v] * hs[t, h], k-major over the Tpad rows of both (rows past
     // T are cleared)
     GemmArgs g{hs, H, (int)H, e, ldv, (int)V, (int)Tpad, (int)H, (int)ldv};
     g.skip_if_set = probs_status;
     if (dweight_mode == 2) return launch_dweight_bf16(g, H, V, ldv, dweight, dw_part, stream);
     const StoreParams ep{dweight, H, (int)H, (int)V, nullptr};
-    rc = launch_store<KERNEL16_TN>(g, ep, dweight_mode == 1 ? 2 : 1, stream);
-    if (rc != AREAL_OK) return rc;
+    return launch_store<KERNEL16_TN>(g, ep, dweight_mode == 1 ? 2 : 1, stream);
+  };
+  // dWeight in front where e' lies in the memory-side cache: the weight that dHidden reads would push some of it out. The
+  // other way round elsewhere: steps of 4096 x 896 2610 us for 2635, of 16384 x 1536 with fp32 masters 16350 for 16490.
+  const bool dw_first = past_cache(T, H, V);
+  if (dw_first && (rc = dweight_launches()) != AREAL_OK) return rc;
+  if ((rc = dhidden_launches()) != AREAL_OK) return rc;
+  if (dbias != nullptr) {
+    hipLaunchKernelGGL(colsum_bf16_kernel, dim3((unsigned)ceil_div_i64(V, 64)), dim3(256), 0, stream,
+                       e, ldv, T, (int)V, dweight_mode == 1 ? 1 : 0, (const float*)rowfac, dbias, probs_status);
+    AREAL_CHECK_LAUNCH();
   }
+  if (!dw_first && (rc = dweight_launches()) != AREAL_OK) return rc;
   return AREAL_OK;
 }
 

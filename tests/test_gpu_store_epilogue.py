@@ -40,3 +40,31 @@ def test_three_outputs_of_dweight_agree(dev, T, H, V):
     d *= grad[:, None]
     for got, want in ((plain, d.t() @ h32), (dh.float(), d @ w32)):
         assert (got - want).abs().max().item() <= 2e-2 * want.abs().max().item()
+
+
+# either side of the rule on keeping the exponentials in the memory-side cache (768 tokens of this vocabulary), 224-wide and
+# whole tiles, a bias (another forward epilogue), a vocabulary that is no multiple of 64 (the transposed weight)
+@pytest.mark.parametrize("T,H,V,bias", [(130, 896, 151936, False), (768, 896, 151936, False), (769, 896, 151936, False),
+                                        (509, 1024, 128256, False), (200, 1024, 128256, True), (200, 1024, 128250, False)])
+def test_exponentials_kept_for_the_backward(dev, T, H, V, bias):
+    g = torch.Generator(device=dev).manual_seed(T + H + V)
+    hidden = torch.randn(T, H, generator=g, device=dev).bfloat16().requires_grad_(True)
+    weight = (torch.randn(V, H, generator=g, device=dev) * (2.0 / H ** 0.5)).bfloat16().requires_grad_(True)
+    b = torch.randn(V, generator=g, device=dev) if bias else None
+    labels = torch.randint(0, V, (T,), generator=g, device=dev)
+    grad = torch.randn(T, generator=g, device=dev)
+    out = fused_lm_head_logprobs_entropy(hidden, weight, labels, bias=b, save_probs=True)
+    out.logprobs.backward(grad)
+    h32, w32 = hidden.detach().float(), weight.detach().float()
+    logits = h32 @ w32.t()
+    if bias:
+        logits += b
+    logp = torch.log_softmax(logits, -1)
+    own = torch.arange(T, device=dev)
+    torch.testing.assert_close(out.logprobs.detach(), logp[own, labels], rtol=1e-5, atol=1e-4)
+    d = -logp.exp()
+    del logits, logp
+    d[own, labels] += 1
+    d *= grad[:, None]
+    for got, want in ((weight.grad, d.t() @ h32), (hidden.grad, d @ w32)):
+        assert (got.float() - want).abs().max().item() <= 2e-2 * want.abs().max().item()
