@@ -113,6 +113,7 @@ SIGNATURES: dict[str, tuple] = {
     "areal_unpack_to_padded": (I, [P, P, P, P, I64, I64, I64, P, I, P]),
     "areal_unpack_rows": (I, [P, P, P, I64, I64, I64, P]),
     "areal_pad_packed_multi": (I, [P, P, P, P, P, P, I, P, I64, P, P, I64, I64, P]),
+    "areal_pad_packed_multi_ex": (I, [P, P, P, P, P, P, I, P, I64, P, P, I64, I64, P, P]),
     "areal_realign_packed": (I, [P, P, P, I64, P, I64, I64, P, I, I, I64, P]),
     "areal_masked_stats_workspace_bytes": (SZ, [I]),
     "areal_masked_stats": (I, [P, P, I, I64, P, P, SZ, P]),

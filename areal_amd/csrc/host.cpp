@@ -1110,8 +1110,9 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> gae_packed_normalized(
 
 // ---------------------------------------------------------------------------------------
 // Packing: the sizes that the API returns as numbers travel as the losses' results do (HostResult), and the
-// allocations and launches of a dict's tensors are one call. A batch of 256 x 4096 with six tensors packed, padded
-// and one result unpacked (35 us of kernels): 164 us with a tensor call, a ctypes array or a copy for each, now 75.
+// allocations and launches of a dict's tensors are one call, and so are the walks over the dict. A batch of 256 x 4096 with six
+// tensors packed, padded and one result unpacked (25 us of kernels): 164 us with a tensor call, a ctypes array or a copy for
+// each, 65.6 with the dicts walked in Python and the padding prepared when its total had been waited for, now 50.5.
 // ---------------------------------------------------------------------------------------
 constexpr size_t PACK_MAX_TENSORS = 8;  // of one launch
 // Up to this size of its result an unpacking's table is read from pinned host memory by the kernel itself (8 bytes per block
@@ -1165,17 +1166,27 @@ std::tuple<Tensor, int64_t, int64_t> seqlens_of_mask(const Tensor& mask) {
   return {cu, (int64_t)h[0], (int64_t)h[1]};
 }
 
-// Last entry of an int32 array.
-int64_t last_value(const Tensor& x) {
-  require_gpu(x);
-  if (x.numel() == 0) throw py::index_error("index -1 is out of bounds for dimension 0 with size 0");
-  const c10::hip::HIPGuard guard(x.device().index());
-  const Tensor last = x.narrow(0, x.numel() - 1, 1);
-  HostResult host(last);
-  if (host.target() != nullptr)
-    check(areal_int_to_host(ptr<int32_t>(last), host.target(), stream_of(x)), "areal_int_to_host");
-  return (int64_t)*(const double*)host.value().to(at::kDouble).data_ptr();
-}
+// Last entry of an int32 array for the host: read by a kernel that is launched anyway (pad_rows), or by one of its own when
+// it is waited for without.
+struct LastValue {
+  Tensor last;
+  HostResult host;
+  bool queued = false;
+  static Tensor last_of(const Tensor& x) {
+    require_gpu(x);
+    if (x.numel() == 0) throw py::index_error("index -1 is out of bounds for dimension 0 with size 0");
+    return x.narrow(0, x.numel() - 1, 1);
+  }
+  explicit LastValue(const Tensor& x) : last(last_of(x)), host(last) {}
+  int64_t wait() {
+    if (!queued && host.target() != nullptr) {
+      const c10::hip::HIPGuard guard(last.device().index());
+      check(areal_int_to_host(ptr<int32_t>(last), host.target(), stream_of(last)), "areal_int_to_host");
+      queued = true;
+    }
+    return (int64_t)*(const double*)host.value().to(at::kDouble).data_ptr();
+  }
+};
 
 // The padded [bs, S, ...] tensors packed to [total, ...].
 std::vector<Tensor> pack_rows(const std::vector<Tensor>& padded, const Tensor& cu, int64_t bs, int64_t S, int64_t total) {
@@ -1204,9 +1215,10 @@ std::vector<Tensor> pack_rows(const std::vector<Tensor>& padded, const Tensor& c
 }
 
 // The packed [total, ...] tensors with one more sequence behind the others, up to total_new tokens of their fill
-// pattern (at most 16 bytes; none: position ids, which count up). Also writes cu_copy and cu_new.
+// pattern (at most 16 bytes; none: position ids, which count up). Also writes cu_copy and cu_new. last (nullable): of cu.
 std::vector<Tensor> pad_rows(const std::vector<Tensor>& packed, const std::vector<std::string>& fills, const Tensor& cu,
-                             const Tensor& cu_copy, const Tensor& cu_new, int64_t total, int64_t total_new) {
+                             const Tensor& cu_copy, const Tensor& cu_new, int64_t total, int64_t total_new,
+                             LastValue* last) {
   require_gpu(cu);
   const c10::hip::HIPGuard guard(cu.device().index());
   std::vector<Tensor> src, out;
@@ -1231,11 +1243,103 @@ std::vector<Tensor> pad_rows(const std::vector<Tensor>& packed, const std::vecto
       pattern_bytes[k] = fill.empty() ? 1 : (int)fill.size();
       fill.copy(patterns + 16 * k, 16);
     }
-    check(areal_pad_packed_multi(from, to, sizes, patterns, pattern_bytes, ids, (int)n, ptr<int32_t>(cu), cu.numel() - 1,
-                                 ptr<int32_t>(cu_copy), ptr<int32_t>(cu_new), total, total_new, stream_of(cu)),
+    double* const host_total = last != nullptr && !last->queued ? last->host.target() : nullptr;
+    check(areal_pad_packed_multi_ex(from, to, sizes, patterns, pattern_bytes, ids, (int)n, ptr<int32_t>(cu), cu.numel() - 1,
+                                    ptr<int32_t>(cu_copy), ptr<int32_t>(cu_new), total, total_new, host_total, stream_of(cu)),
           "areal_pad_packed_multi");
+    if (host_total != nullptr) last->queued = true;
   }
   return out;
+}
+
+// The tensors and keys of a batch dict, without a Python call per entry. (A tensor subclass is a tensor here as it is there.)
+const Tensor* tensor_of(PyObject* x) { return THPVariable_Check(x) ? &THPVariable_Unpack(x) : nullptr; }
+bool is_key(PyObject* k, const char* name) { return PyUnicode_Check(k) && PyUnicode_CompareWithASCIIString(k, name) == 0; }
+
+// A batch dict packed: pack_tensor_dict of areal_amd/packing.py behind its checks.
+py::dict pack_dict(const py::dict& data, const Tensor& attention_mask) {
+  const int64_t bs = attention_mask.size(0), S = attention_mask.size(1);
+  const auto [cu, total, longest] = seqlens_of_mask(attention_mask);
+  py::dict out;
+  std::vector<PyObject*> keys;
+  std::vector<Tensor> moved;
+  PyObject *key, *value;
+  Py_ssize_t at = 0;
+  auto set = [&](PyObject* k, PyObject* v) {
+    if (PyDict_SetItem(out.ptr(), k, v) != 0) throw py::error_already_set();
+  };
+  while (PyDict_Next(data.ptr(), &at, &key, &value)) {
+    if (is_key(key, "attention_mask")) {
+      out["cu_seqlens"] = cu;
+      out["max_seqlen"] = longest;
+      continue;
+    }
+    set(key, value);
+    const Tensor* const t = tensor_of(value);
+    if (t == nullptr || t->dim() < 2 || t->size(0) != bs || t->size(1) != S) continue;
+    keys.push_back(key);
+    moved.push_back(*t);
+  }
+  const std::vector<Tensor> packed = pack_rows(moved, cu, bs, S, total);
+  for (size_t i = 0; i < keys.size(); ++i) set(keys[i], py::cast(packed[i]).ptr());
+  return out;
+}
+
+// A packed batch padded with zeros to `to` tokens, for the total that its tensors' shapes suggest (the longest one-dimensional
+// one's elements): (padded dict, pad length, copy of the offsets). The launch reports the total it met. Where that is another one,
+// it (the caller pads anew); nothing where this is not the way (no such tensor, position ids, a length that is no
+// plain int, tensors that the kernel does not take: the caller's own way says what is wrong with them, if it meets them).
+py::object pad_likely(const py::dict& data, const Tensor& cu, int64_t to) {
+  int64_t total = 0, longest = 0;
+  PyObject *key, *value;
+  Py_ssize_t at = 0;
+  while (PyDict_Next(data.ptr(), &at, &key, &value)) {
+    if (is_key(key, "position_ids")) return py::none();
+    if (is_key(key, "max_seqlen")) {
+      int overflow = 0;
+      if (!PyLong_CheckExact(value) || (longest = PyLong_AsLongLongAndOverflow(value, &overflow), overflow != 0)) return py::none();
+    }
+    const Tensor* const t = is_key(key, "cu_seqlens") ? nullptr : tensor_of(value);
+    if (t != nullptr && t->dim() == 1) total = std::max(total, t->numel());
+  }
+  if (total <= 0 || total >= to) return py::none();
+  LastValue last(cu);
+  const c10::hip::HIPGuard guard(cu.device().index());
+  const Tensor cu_new = empty(cu, {cu.numel() + 1}, at::kInt), cu_copy = at::empty_like(cu);
+  py::dict out;
+  std::vector<PyObject*> keys;
+  std::vector<Tensor> moved;
+  auto set = [&](PyObject* k, PyObject* v) {
+    if (PyDict_SetItem(out.ptr(), k, v) != 0) throw py::error_already_set();
+  };
+  for (at = 0; PyDict_Next(data.ptr(), &at, &key, &value);) {
+    if (is_key(key, "cu_seqlens")) {
+      set(key, py::cast(cu_new).ptr());
+    } else if (is_key(key, "max_seqlen")) {
+      set(key, py::cast(std::max(longest, to - total)).ptr());
+    } else {
+      set(key, value);
+      const Tensor* const t = tensor_of(value);
+      if (t == nullptr || t->numel() != total) continue;
+      keys.push_back(key);
+      moved.push_back(*t);
+    }
+  }
+  try {
+    std::vector<std::string> fills;
+    for (Tensor& t : moved) {
+      if (t.dim() != 1) t = t.reshape({total});
+      fills.emplace_back(t.element_size(), '\0');
+    }
+    const std::vector<Tensor> padded = pad_rows(moved, fills, cu, cu_copy, cu_new, total, to, &last);
+    for (size_t i = 0; i < keys.size(); ++i) set(keys[i], py::cast(padded[i]).ptr());
+  } catch (...) {
+    PyErr_Clear();
+    return py::none();
+  }
+  const int64_t met = last.wait();
+  if (met != total) return py::int_(met);
+  return py::make_tuple(out, to - total, cu_copy);
 }
 
 // Rows of a packed tensor, zero padded, in the given order; nothing where the arguments are not plain lists of
@@ -1324,11 +1428,13 @@ PYBIND11_MODULE(_host, m) {
   m.def("turn_gae", &turn_gae);
   m.def("gae_packed_normalized", &gae_packed_normalized);
   m.def("seqlens_of_mask", &seqlens_of_mask);
-  m.def("last_value", &last_value);
+  py::class_<LastValue>(m, "LastValue").def(py::init<const Tensor&>()).def("wait", &LastValue::wait);
   m.def("pack_rows", &pack_rows);
+  m.def("pack_dict", &pack_dict);
+  m.def("pad_likely", &pad_likely);
   m.def("pad_rows", [](const std::vector<Tensor>& packed, const std::vector<py::bytes>& fills, const Tensor& cu,
                        const Tensor& cu_copy, const Tensor& cu_new, int64_t total, int64_t total_new) {
-    return pad_rows(packed, std::vector<std::string>(fills.begin(), fills.end()), cu, cu_copy, cu_new, total, total_new);
+    return pad_rows(packed, std::vector<std::string>(fills.begin(), fills.end()), cu, cu_copy, cu_new, total, total_new, nullptr);
   });
   m.def("unpack_rows", &unpack_rows);
 }

@@ -330,10 +330,12 @@ struct PadArgs {
   int n_seqs, n_tensors;
   int64_t total, total_new;
   int chunk;
+  double* host_total;  // nullable, pinned host memory: receives cu[n_seqs]
 };
 __global__ __launch_bounds__(PK_THREADS) void pad_packed_kernel(PadArgs a) {
   const int k = blockIdx.y;
   if (k == 0 && blockIdx.x == 0) {
+    if (threadIdx.x == 0 && a.host_total != nullptr) *a.host_total = (double)a.cu[a.n_seqs];
     for (int i = threadIdx.x; i <= a.n_seqs; i += PK_THREADS) {
       const int32_t c = a.cu[i];
       a.cu_copy[i] = c;
@@ -600,6 +602,14 @@ int areal_pad_packed_multi(const void* const* src, void* const* dst, const int64
                            const int* fill_bytes, const int* position_ids, int n_tensors,
                            const int32_t* cu_seqlens, int64_t n_seqs, int32_t* cu_copy, int32_t* cu_new,
                            int64_t total, int64_t total_new, hipStream_t stream) {
+  return areal_pad_packed_multi_ex(src, dst, elem_bytes, fills, fill_bytes, position_ids, n_tensors, cu_seqlens, n_seqs,
+                                   cu_copy, cu_new, total, total_new, nullptr, stream);
+}
+// ... and cu_seqlens[n_seqs] to pinned host memory (nullable), for a caller that took `total` from the tensors' shapes.
+int areal_pad_packed_multi_ex(const void* const* src, void* const* dst, const int64_t* elem_bytes, const void* fills,
+                              const int* fill_bytes, const int* position_ids, int n_tensors,
+                              const int32_t* cu_seqlens, int64_t n_seqs, int32_t* cu_copy, int32_t* cu_new,
+                              int64_t total, int64_t total_new, double* host_total, hipStream_t stream) {
   if (n_tensors < 0 || n_tensors > PK_MAX_TENSORS || n_seqs < 0 || total < 0 || total_new <= total)
     return AREAL_ERR_BAD_ARG;
   if (!cu_seqlens || !cu_copy || !cu_new) return AREAL_ERR_BAD_ARG;
@@ -618,7 +628,7 @@ int areal_pad_packed_multi(const void* const* src, void* const* dst, const int64
     max_eb = elem_bytes[k] > max_eb ? elem_bytes[k] : max_eb;
   }
   a.cu = cu_seqlens; a.cu_copy = cu_copy; a.cu_new = cu_new; a.n_seqs = (int)n_seqs; a.n_tensors = n_tensors;
-  a.total = total; a.total_new = total_new; a.chunk = (int)pk_chunk_tokens(max_eb);
+  a.total = total; a.total_new = total_new; a.chunk = (int)pk_chunk_tokens(max_eb); a.host_total = host_total;
   const int64_t chunks = ceil_div_i64(total_new, a.chunk);
   if (chunks > PK_MAX_BLOCKS) return AREAL_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(pad_packed_kernel, dim3((unsigned)chunks, (unsigned)(n_tensors > 0 ? n_tensors : 1)),

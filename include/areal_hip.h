@@ -627,6 +627,13 @@ int areal_pad_packed_multi(const void* const* src, void* const* dst, const int64
                            const void* fills, const int* fill_bytes, const int* position_ids,
                            int n_tensors, const int32_t* cu_seqlens, int64_t n_seqs, int32_t* cu_copy,
                            int32_t* cu_new, int64_t total, int64_t total_new, areal_stream_t stream);
+/* The same, and cu_seqlens[n_seqs] to pinned host memory (NULL allowed), for a caller that took total from the
+ * tensors' shapes: the outputs are right if the two agree. */
+int areal_pad_packed_multi_ex(const void* const* src, void* const* dst, const int64_t* elem_bytes,
+                              const void* fills, const int* fill_bytes, const int* position_ids,
+                              int n_tensors, const int32_t* cu_seqlens, int64_t n_seqs, int32_t* cu_copy,
+                              int32_t* cu_new, int64_t total, int64_t total_new, double* host_total,
+                              areal_stream_t stream);
 size_t areal_masked_stats_workspace_bytes(int K);
 /* out [K][4] double = {sum, count, min, max} of values[k] where masks[k] != 0 (NULL mask: all).
  * values / masks are HOST arrays of K <= 32 device pointers. */

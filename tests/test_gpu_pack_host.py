@@ -131,3 +131,48 @@ def test_packing_by_waves_and_by_blocks(dev, rows, length, trailing):
     packed = pack_tensor_dict({k: v.to(dev) for k, v in data.items()})
     for key in ("x", "flag", "ids", "odd"):
         assert torch.equal(packed[key].cpu(), data[key][mask]), key
+
+
+class _Other(dict):
+    """A batch that the native walk over plain dicts does not take."""
+
+
+def _packed_batch(dev, total, extra):
+    g = torch.Generator(device=dev).manual_seed(total)
+    cu = torch.tensor([0, total // 3, total // 3, total], dtype=torch.int32, device=dev)
+    data = dict(cu_seqlens=cu, max_seqlen=total - total // 3, input_ids=torch.randint(0, 99, (total,), generator=g, device=dev),
+                logprobs=torch.randn(total, generator=g, device=dev), loss_mask=torch.rand(total, generator=g, device=dev) > 0.5,
+                folded=torch.randn(total // 2, 2, generator=g, device=dev) if total % 2 == 0 else torch.randn(total, 3, device=dev),
+                name="batch", rewards=torch.randn(3, generator=g, device=dev))
+    data.update(extra)
+    return data
+
+
+# the total that the shapes suggest is the right one, or a longer tensor that is no token tensor leads astray (shorter and longer
+# than the padded batch), nothing suggests one, or the call is not one for the native walk
+@pytest.mark.parametrize("case", ["plain", "long", "longer", "none", "ids", "tensor length", "huge length", "value"])
+@pytest.mark.parametrize("total, to", [(1, 2), (640, 641), (4001, 4096)])
+def test_padding_for_the_likely_total(dev, case, total, to):
+    extra = {"long": dict(other=torch.zeros(to - 1, device=dev)), "longer": dict(other=torch.zeros(to + 5, device=dev)),
+             "ids": dict(position_ids=torch.arange(total, device=dev)),
+             "tensor length": dict(max_seqlen=torch.tensor(total - total // 3)), "huge length": dict(max_seqlen=1 << 70)}
+    data = _packed_batch(dev, total, extra.get(case, {}))
+    if case == "none":
+        for k in ("input_ids", "logprobs", "loss_mask", "rewards"):
+            data[k] = data[k][None]
+    value = 2.5 if case == "value" else 0.0
+    got, got_length, got_cu, got_align = pad_packed_tensor_dict(data, to, pad_value=value)
+    want, want_length, want_cu, want_align = pad_packed_tensor_dict(_Other(data), to, pad_value=value)
+    assert (got_length, got_align) == (want_length, want_align) == (to - total, None)
+    assert torch.equal(got_cu, want_cu) and torch.equal(got_cu, data["cu_seqlens"])
+    assert list(got) == list(want)
+    for k, v in want.items():
+        assert type(got[k]) is type(v)
+        if torch.is_tensor(v):
+            assert got[k].dtype == v.dtype and torch.equal(got[k], v), k
+        else:
+            assert got[k] == v, k
+    tail = got["input_ids"].reshape(-1)[total:]
+    assert tail.numel() == to - total and bool((tail == int(value)).all())
+    with pytest.raises(ValueError, match="smaller than total length"):
+        pad_packed_tensor_dict(data, total - 1)
