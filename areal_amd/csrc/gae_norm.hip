@@ -129,8 +129,9 @@ DEVI void block_sum_n(double (&v)[N], double* smem /* [4][N] */) {
 }
 
 // ---- Sums handed from block to block inside a launch (adv_normalise_row, gae_tile_normalise): sealed words, N numbers
-// and a check word made of them and the call's number, and a flag per entry, the call's number again, stored when they have
-// left. All go out and come in as agent-scope atomics (past the XCD's own L2); flags lie next to each other, so that
+// and a check word made of them and the call's number, and a flag per entry, the call's number again, stored right behind
+// them (a reader that sees the flag first finds the check word wrong and looks again; waiting for the words before storing
+// it: packed GAE of 1.79 Mi tokens 27.1 -> 28.1 us). All go out and come in as agent-scope atomics (past the XCD's own L2); flags lie next to each other, so that
 // looking again costs a line or two (with the words themselves looked at, 900 waiting blocks of 14 entries each slowed
 // down the ones they waited for: packed GAE
 // of 1.79 Mi tokens 31.4 -> 29.0 us). Whoever reads words that fit has
@@ -157,7 +158,6 @@ DEVI void publish_sums(uint64_t* to, uint64_t* flag, uint64_t call, const double
     __hip_atomic_store(to + k, w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __hip_atomic_store(to + N, sums_seal(call, w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the seal is what the reader relies on)
   __hip_atomic_store(flag, call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // The sums of n entries PITCH words apart, added up by a whole wave: lane i takes every 64th from the i-th on, then the
@@ -197,11 +197,11 @@ DEVI bool note_left(const uint64_t* left, uint64_t call) {
 // A block that leaves a note and looks at the sums again, and one that publishes its sums and looks for notes, each store
 // to one address and load from another: both loads could be served ahead of both stores, each would miss the other, and
 // the row or segment would stay without its normalisation. So a store and a fence come before the load on either side:
-//   leaver      note    | fence                | flags of the sums
-//   publisher   flag    | wait for its store   | notes
+//   leaver      note       | fence               | flags of the sums, sums
+//   publisher   sums, flag | wait for the stores | notes
 // Whichever store is performed later, the load behind it sees the earlier one. The publisher's loads go past every cache
 // that is not shared, so that waiting for the store is all of the fence it needs; store and load are of one wave on both
-// sides. It costs nothing that shows: advantages of 64 x 1000 15.0 us, packed GAE of 1024 x 1750 30.4, both as without.
+// sides. It costs nothing that shows: advantages of 64 x 1000 15.0 us, packed GAE of 1024 x 1750 27.1, both as without.
 DEVI void leave_note(uint64_t* left, uint64_t call) {  // by one thread, whose wave looks again
   atomicExch((unsigned long long*)left, (unsigned long long)call);
   __threadfence();
@@ -421,13 +421,13 @@ __global__ __launch_bounds__(GAE_THREADS) void gae_apply_kernel(GaeArgs g, const
 
 // ---------------------------------------------------------------------------------------
 // Single-pass GAE: one launch, every token read once and written once (20 B/token), no block
-// waits for another. Sequences are independent, so nothing enters a sequence's last token from
+// has to wait for another. Sequences are independent, so nothing enters a sequence's last token from
 // its right. Two kernels:
 //  * padded rows (gae_owned_kernel): block b owns the rows whose END lies in the token range
 //    (b*TILE, (b+1)*TILE] (one block per row when rows are at least a tile long) and walks them
 //    right to left tile by tile, carrying (A, nv) across its tiles;
-//  * packed sequences (gae_tile_kernel): block = tile; the state entering the tile is recomputed
-//    from the crossing sequence's remaining tokens.
+//  * packed sequences (gae_tile_kernel): block = tile; the state entering the tile is made from the maps of the
+//    crossing sequence's remaining tokens, recomputed or, where the launch hands them over, those of their blocks.
 // Tiles are absolute multiples of TILE, so the 16-byte loads stay aligned. The host picks the
 // three-launch scan above when sequences are long on average.
 // ---------------------------------------------------------------------------------------
@@ -832,20 +832,28 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
 
 // Single-pass GAE for packed sequences of ordinary length, one block per tile. What enters the
 // tile from its right is the state of the sequence that crosses the tile's right edge, and it
-// depends only on that sequence's tokens beyond the edge: the block reads them too (rewards,
-// values, mask; nothing written), a run of chunks of 512 per wave, the next chunk on its way while one is
-// composed, and applies the waves' maps to the zero state (512 x 8192 tokens 59.9 -> 54.3 us, 64 x 8192 30.7 -> 25.8
-// against steps of a whole tile with two barriers each). No block waits for another, and the remainder is read once per tile of the sequence, from L2 mostly:
-// the blocks of an XCD are neighbours in the array. Against blocks that walk the sequences they
-// own tile by tile, carrying the state (the padded-row kernel above, which also took cu_seqlens
-// once): faster on 64 x 16384 tokens and on 4 x 32768, where a walking block has 16 tiles in a row.
+// depends only on that sequence's tokens beyond the edge: maps of chunks of 512 tokens, a wave each, applied to the zero
+// state in fp64 from the right. Those of the tile with its last token the block makes itself (rewards, values, mask are read,
+// nothing written, the next chunk on its way while one is composed; a wave whose chunk holds none of it reads nothing). Those
+// of whole tiles between are the totals that these tiles' blocks need anyway: the launch that normalises hands them
+// over (TileMaps), 16 tiles at a time, for otherwise a sequence of k tiles is read k / 2 times, one chunk after the other;
+// where they do not come in time, and in gae_tile_kernel, which has no words for them, the block makes them too: the same
+// numbers, so the same bits. One launch, us, made by each block / handed over: 1024 x 1750 28.9 / 27.1, 512 x 4000 36.6 / 30,
+// 64 x 8192 48 / 22, 128 x 8192 40.7 / 25, 512 x 3000 of deviation 1.5 41.7 / 27.5, 256 x 1750 21.7 / 18.0. For a sequence over one or two whole tiles
+// too (1024 x 1600 25.2; from 2 tiles on 26.4, from 3 27.4).
+// Against blocks that walk the sequences they own tile by tile, carrying the state (the padded-row kernel above, which
+// also took cu_seqlens once): faster on 64 x 16384 tokens and on 4 x 32768, where a walking block has 16 tiles in a row.
+// The layout comes first. Up to 2048 sequences (and 1024 groups) cu_seqlens and the groups' first sequences go to LDS
+// whole, and what the tile has to find in them is counted from the registers on the way: one barrier, no load that waits
+// for another. With 4096 (16 loads a thread) the search in memory is as fast: 3000 x 300 22.3 against 21.5 us, 4096 x 300 24.5
+// against 23.3. There the wave that has no group to find finds the sequences, meanwhile.
 // The kernel is bound by vector instruction issue (about 1150 vector and 250 scalar instructions
-// per wave and tile on 1024 sequences of mean length 1760) with four blocks resident per CU, so
-// that all blocks of a 1.8 M-token batch run at once; that leaves 128 registers, of which the instances with group sums
-// spill 6 (28 bytes of scratch a lane). Against a step of a whole tile at a time, which spills none, the two launches that
-// normalise take, us: 1024 x 1750 33.6 -> 33.0, 64 x 8192 38.2 -> 33.5, 4096 x 1000 62.8 -> 62.6, 4096 x 100 57.8 -> 58.8.
+// per wave and tile on 1024 sequences of mean length 1760, half as many again with the group sums) for half of its time and by
+// the chain of loads, maps and sums for the other half, with four blocks resident per CU, so
+// that all blocks of a 1.8 M-token batch run at once; that leaves 128 registers.
 constexpr int GAE_CHUNK = 64 * GAE_ITEMS;  // tokens of a wave's step through the crossing sequence
-constexpr int GAE_CU_LDS = 16 * GAE_THREADS;  // entries of cu_seqlens the block can hold (>= TILE + 2)
+constexpr int GAE_CU_LDS = 8 * GAE_THREADS;  // sequences whose starts the block can hold (>= TILE + 1)
+constexpr int GAE_GROUPS_LDS = 4 * GAE_THREADS;  // groups whose first sequences it can hold
 
 // Groups of a tile for GaeArgs::seg_stats: those of the tile's first and last token and of the next
 // tile's first token, each the number of group ends at or before the token. Waves 0..2 search
@@ -864,9 +872,11 @@ DEVI void gae_tile_group_search(const GaeArgs& g, int64_t lo, int64_t hi, int* s
 struct GaeTileGroups {
   int g_first, g_last, g_next;
   int64_t b[3];
+  const int32_t *cu, *gseq;  // cu_seqlens and the groups' first sequences in LDS, or null
 };
 DEVI GaeTileGroups gae_tile_groups(const GaeArgs& g, int64_t lo, const int* s_grp) {
   GaeTileGroups r;
+  r.cu = r.gseq = nullptr;
   r.g_first = s_grp[0];
   r.g_last = s_grp[1] < g.n_groups ? s_grp[1] : g.n_groups - 1;
   r.g_next = s_grp[2];
@@ -877,12 +887,35 @@ DEVI GaeTileGroups gae_tile_groups(const GaeArgs& g, int64_t lo, const int* s_gr
   }
   return r;
 }
+// The same from LDS, by every wave for itself. n_lo, n_hi, n_behind: how many sequences end at or before each of the three
+// tokens; a group has ended there exactly when the next one's first sequence is not among those still to come.
+DEVI GaeTileGroups gae_tile_groups_lds(const GaeArgs& g, int64_t lo, const int32_t* cu, const int32_t* gseq, int n_lo, int n_hi,
+                                       int n_behind) {
+  const int lane = threadIdx.x & 63;
+  GaeTileGroups r;
+  r.cu = cu; r.gseq = gseq;
+  int c0 = 0, c1 = 0, c2 = 0;
+  for (int j0 = 1; j0 <= g.n_groups; j0 += 64) {
+    const int j = j0 + lane;
+    const int s = gseq[j <= g.n_groups ? j : g.n_groups];
+    c0 += __popcll(__builtin_amdgcn_ballot_w64(j <= g.n_groups && s <= n_lo));
+    c1 += __popcll(__builtin_amdgcn_ballot_w64(j <= g.n_groups && s <= n_hi));
+    c2 += __popcll(__builtin_amdgcn_ballot_w64(j <= g.n_groups && s <= n_behind));
+  }
+  r.g_first = c0;
+  r.g_last = c1 < g.n_groups ? c1 : g.n_groups - 1;
+  r.g_next = c2;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) r.b[i] = (int64_t)cu[gseq[r.g_first + i <= g.n_groups ? r.g_first + i : g.n_groups]] - lo;
+  return r;
+}
 
 // Where the k-th group of the tile lies, relative to the tile's first token.
 // (selects, not an index: an indexed register array would live in scratch memory)
 DEVI void tile_group_bounds(const GaeArgs& g, const GaeTileGroups& tg, int64_t lo, int k, int64_t& b0, int64_t& b1) {
-  b0 = k == 0 ? tg.b[0] : k == 1 ? tg.b[1] : k == 2 ? tg.b[2] : group_offsets(g)[tg.g_first + k] - lo;
-  b1 = k == 0 ? tg.b[1] : k == 1 ? tg.b[2] : group_offsets(g)[tg.g_first + k + 1] - lo;
+  auto bound = [&](int j) { return (tg.cu != nullptr ? (int64_t)tg.cu[tg.gseq[j]] : group_offsets(g)[j]) - lo; };
+  b0 = k == 0 ? tg.b[0] : k == 1 ? tg.b[1] : k == 2 ? tg.b[2] : bound(tg.g_first + k);
+  b1 = k == 0 ? tg.b[1] : k == 1 ? tg.b[2] : bound(tg.g_first + k + 1);
 }
 // The five masked sums of the tile's advantages per group and wave (GaeArgs::seg_stats): x = oa
 // (zero for tokens outside every sequence), m = the thread's 8 mask values (zero beyond the
@@ -959,15 +992,75 @@ DEVI void gae_tile_group_stats(const GaeArgs& g, int64_t tile, int64_t lo, int64
   }
 }
 
+// The maps of whole tiles, handed from block to block inside a launch: each wave's total, five floats and a check word made
+// of them, each in a word of its own next to a tag made of the call's number and its place, so that a word says by itself
+// whether it is this call's. The check tells one word that is not from any other (every step of it is one to one), so that a
+// wrong map takes two tags that fit by chance, 2^-64. (Sealed as a whole like the sums, a map cost its writer and its readers
+// a microsecond of 64-bit multiplications each.)
+constexpr int GAE_LOOK_TILES = 16, MAP_WORDS = 6, MAP_PITCH = 8;  // a line of 64 bytes a wave
+struct TileMaps {
+  uint64_t* at;      // [tiles][GAE_SEG_WAVES][MAP_PITCH]
+  uint64_t call;
+  unsigned ticks;    // how long a block waits for them before it makes them itself
+};
+DEVI uint32_t map_tag(uint64_t call, int k) { return (uint32_t)(call >> (k & 1 ? 32 : 0)) + 0x9e3779b9u * (uint32_t)(k + 1); }
+DEVI uint32_t map_check(const MapF& m) {
+  const float x[5] = {m.a11, m.a12, m.a22, m.b1, m.b2};
+  uint32_t h = 0;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    h = (h ^ __builtin_bit_cast(uint32_t, x[k])) * 0x9e3779b1u;
+    h ^= h >> 15;
+  }
+  return h;
+}
+DEVI void publish_wave_map(const TileMaps& t, int64_t tile, int wave, const MapF& m) {  // m in every lane
+  const int k = threadIdx.x & 63;
+  const float x = k == 0 ? m.a11 : k == 1 ? m.a12 : k == 2 ? m.a22 : k == 3 ? m.b1 : m.b2;
+  const uint32_t w = k == 5 ? map_check(m) : __builtin_bit_cast(uint32_t, x);
+  if (k < MAP_WORDS)
+    __hip_atomic_store(t.at + (GAE_SEG_WAVES * tile + wave) * MAP_PITCH + k, (uint64_t)map_tag(t.call, k) << 32 | w,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Those of n <= GAE_LOOK_TILES tiles from `first` on, by a whole wave, a lane each. False when they were not all there in time.
+DEVI bool gather_tile_maps(const TileMaps& t, int64_t first, int n, MapF* chunks) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t* const from = t.at + (GAE_SEG_WAVES * first + lane) * MAP_PITCH;
+  const uint64_t deadline = wall_clock64() + t.ticks;
+  bool have = lane >= GAE_SEG_WAVES * n;
+  for (;;) {
+    if (!have) {
+      uint64_t w[MAP_WORDS];
+      bool all = true;
+#pragma unroll
+      for (int k = 0; k < MAP_WORDS; ++k) w[k] = __hip_atomic_load(from + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int k = 0; k < MAP_WORDS; ++k) all &= (uint32_t)(w[k] >> 32) == map_tag(t.call, k);
+      auto of = [&](int k) { return __builtin_bit_cast(float, (uint32_t)w[k]); };
+      const MapF m{of(0), of(1), of(2), of(3), of(4)};
+      if (all && (uint32_t)w[5] == map_check(m)) {
+        chunks[lane] = m;
+        have = true;
+      }
+    }
+    if (__builtin_amdgcn_ballot_w64(!have) == 0) return true;
+    if (wall_clock64() >= deadline) return false;
+    __builtin_amdgcn_s_sleep(2);
+  }
+}
+
 // STATS: tail(tile, lo, hi, groups of the tile, advantages, masks) gets what the group sums are made of.
-template <bool LAMBDAS, bool STATS, class Tail>
-DEVI void gae_tile(const GaeArgs& g, const Tail& tail) {
+// LOOK: the maps of tiles inside a crossing sequence come from their blocks.
+template <bool LAMBDAS, bool STATS, bool LOOK, class Tail>
+DEVI void gae_tile(const GaeArgs& g, const TileMaps& look, const Tail& tail) {
   __shared__ MapF smem[GAE_THREADS / 64];
   __shared__ int s_grp[3];
   __shared__ MapF all[GAE_THREADS];
-  __shared__ Map s_part[GAE_SEG_WAVES];
-  __shared__ int32_t s_cu[GAE_CU_LDS];
-  __shared__ int s_own[2];
+  __shared__ MapF s_chunk[GAE_LOOK_TILES * GAE_SEG_WAVES], s_end[GAE_SEG_WAVES];
+  __shared__ int s_have;
+  __shared__ int32_t s_cu[GAE_CU_LDS + 1];
+  __shared__ int32_t s_gseq[STATS ? GAE_GROUPS_LDS + 1 : 1];
+  __shared__ int s_own[GAE_SEG_WAVES][3];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // XCD x (workgroup ids congruent to x modulo 8) takes the x-th eighth of the tiles
   const int64_t per_xcd = (gridDim.x + 7) >> 3;
@@ -975,76 +1068,110 @@ DEVI void gae_tile(const GaeArgs& g, const Tail& tail) {
   const int64_t lo = tile * GAE_TILE;
   if (tile >= per_xcd * 8 || lo >= g.n) return;
   const int64_t hi = lo + GAE_TILE < g.n ? lo + GAE_TILE : g.n;
-  // The tile's inputs do not depend on the sequence layout: their loads go out first, together
-  // with those of the layout.
+  // All that the block reads at its start goes out together, the layout first (loads come back in their order): the whole
+  // of cu_seqlens and the groups' first sequences for LDS, and the tile's inputs.
+  const bool cu_in_lds = g.n_seqs <= GAE_CU_LDS;
+  const bool groups_in_lds = STATS && cu_in_lds && g.goff == nullptr && g.n_groups <= GAE_GROUPS_LDS;
+  constexpr int CU_LOADS = GAE_CU_LDS / GAE_THREADS, CU_FIRST = 5, GROUP_LOADS = STATS ? GAE_GROUPS_LDS / GAE_THREADS : 1;
+  int32_t c[CU_LOADS], gq[GROUP_LOADS];
+  const bool many = g.n_seqs >= CU_FIRST * GAE_THREADS;  // (uniform)
+  auto cu_of = [&](int k) { const int i = tid + k * GAE_THREADS; return g.cu[i < g.n_seqs ? i : g.n_seqs]; };  // (behind them: cov_hi)
+  if (cu_in_lds) {
+#pragma unroll
+    for (int k = 0; k < CU_FIRST; ++k) c[k] = cu_of(k);
+    if (many) {
+#pragma unroll
+      for (int k = CU_FIRST; k < CU_LOADS; ++k) c[k] = cu_of(k);
+    }
+    if (groups_in_lds) {
+#pragma unroll
+      for (int k = 0; k < GROUP_LOADS; ++k) {
+        const int i = tid + k * GAE_THREADS;
+        if (k == 0 || k * GAE_THREADS < g.n_groups) gq[k] = (int32_t)g.gseq[i < g.n_groups ? i : g.n_groups];
+      }
+    }
+  }
   float rw[GAE_ITEMS], v[GAE_ITEMS], ms[GAE_ITEMS];
   gae_load_items(g, lo + (int64_t)tid * GAE_ITEMS, true, rw, v, ms);
-  const bool cu_in_lds = g.n_seqs + 1 <= GAE_CU_LDS;
-  int64_t cov_lo, cov_hi;
+  if constexpr (STATS) {
+    if (!groups_in_lds) gae_tile_group_search(g, lo, hi, s_grp);  // (a barrier follows either way)
+  }
+  const int64_t cov_lo = (int64_t)g.cu[0], cov_hi = (int64_t)g.cu[g.n_seqs];
+  const int64_t gseq_end = groups_in_lds ? g.gseq[g.n_groups] : 0;
+  const int64_t t_begin = lo > cov_lo ? lo : cov_lo;
+  const int64_t t_end = hi < cov_hi ? hi : cov_hi;
+  const bool groups_from_lds = groups_in_lds && lo >= cov_lo && hi <= cov_hi;
+  if constexpr (STATS) {
+    if (groups_in_lds && !groups_from_lds) gae_tile_group_search(g, lo, hi, s_grp);
+  }
+  // Sequences that end at or before the first token, the last token, and the token behind the tile.
+  int n_lo = 0, n_hi = 0, n_behind = 0;
   if (cu_in_lds) {
-    // the whole of cu_seqlens into LDS, every load in flight at once
-    int32_t c[GAE_CU_LDS / GAE_THREADS];
-#pragma unroll
-    for (int k = 0; k < GAE_CU_LDS / GAE_THREADS; ++k) {
+    const int64_t top = (int64_t)INT32_MAX;
+    const int32_t x0 = (int32_t)(t_begin < top ? t_begin : top), x1 = (int32_t)(t_end - 1 < top ? t_end - 1 : top),
+                  x2 = (int32_t)(hi < top ? hi : top);
+    auto count = [&](int k) {
       const int i = tid + k * GAE_THREADS;
-      c[k] = i <= g.n_seqs ? g.cu[i] : 0;
-    }
-    // (after the loads above are on their way: the search waits for its own)
-    if constexpr (STATS) gae_tile_group_search(g, lo, hi, s_grp);
+      s_cu[i] = c[k];
+      const bool end = i >= 1 && i < g.n_seqs;
+      n_lo += __popcll(__builtin_amdgcn_ballot_w64(end && c[k] <= x0));
+      n_hi += __popcll(__builtin_amdgcn_ballot_w64(end && c[k] <= x1));
+      if constexpr (STATS) n_behind += __popcll(__builtin_amdgcn_ballot_w64(end && c[k] <= x2));
+    };
 #pragma unroll
-    for (int k = 0; k < GAE_CU_LDS / GAE_THREADS; ++k) s_cu[tid + k * GAE_THREADS] = c[k];
-    if (tid < 2) s_own[tid] = 0;
+    for (int k = 0; k < CU_FIRST; ++k) count(k);
+    if (many) {
+#pragma unroll
+      for (int k = CU_FIRST; k < CU_LOADS; ++k) count(k);
+    }
+    if constexpr (STATS) {
+      if (groups_in_lds) {
+#pragma unroll
+        for (int k = 0; k < GROUP_LOADS; ++k)
+          if (k == 0 || k * GAE_THREADS < g.n_groups) s_gseq[tid + k * GAE_THREADS] = gq[k];
+      }
+    }
+    if (tid == 0) {  // the last entry of each
+      s_cu[g.n_seqs] = (int32_t)cov_hi;
+      if (STATS && groups_in_lds) s_gseq[g.n_groups] = (int32_t)gseq_end;
+      n_lo += (int32_t)cov_hi <= x0;
+      n_hi += (int32_t)cov_hi <= x1;
+      if constexpr (STATS) n_behind += (int32_t)cov_hi <= x2;
+    }
+    if (lane == 0) { s_own[wave][0] = n_lo; s_own[wave][1] = n_hi; s_own[wave][2] = n_behind; }
     __syncthreads();
-    cov_lo = (int64_t)s_cu[0];
-    cov_hi = (int64_t)s_cu[g.n_seqs];
-  } else {
-    if constexpr (STATS) gae_tile_group_search(g, lo, hi, s_grp);
-    cov_lo = (int64_t)g.cu[0];
-    cov_hi = (int64_t)g.cu[g.n_seqs];
+    n_lo = n_hi = n_behind = 0;
+#pragma unroll
+    for (int w = 0; w < GAE_SEG_WAVES; ++w) { n_lo += s_own[w][0]; n_hi += s_own[w][1]; n_behind += s_own[w][2]; }
   }
   // tokens outside every sequence (none in a well-formed batch) are written as zero
   if (lo < cov_lo || hi > cov_hi) {
     for (int64_t t = lo + tid; t < hi; t += GAE_THREADS)
       if (t < cov_lo || t >= cov_hi) { g.adv[t] = 0.f; g.ret[t] = 0.f; }
   }
-  const int64_t t_begin = lo > cov_lo ? lo : cov_lo;
-  const int64_t t_end = hi < cov_hi ? hi : cov_hi;
-  if (t_end <= t_begin) {  // uniform for the block
-    if constexpr (STATS) {
-      const float zero[GAE_ITEMS] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      __syncthreads();
-      tail(tile, lo, hi, gae_tile_groups(g, lo, s_grp), zero, ms);
-    }
-    return;
-  }
+  const bool none = t_end <= t_begin;  // no token of a sequence (uniform for the block)
+  if (!STATS && none) return;
 
-  // sequences holding the first and the last token of [t_begin, t_end): the number of sequence
-  // ends at or before each
+  // sequences holding the first and the last token of [t_begin, t_end)
   const int32_t* cu_own;
   int s_first, s_last;
   if (cu_in_lds) {
-    int n_lo = 0, n_hi = 0;
-    for (int i = tid + 1; i <= g.n_seqs; i += GAE_THREADS) {
-      const int64_t end = (int64_t)s_cu[i];
-      n_lo += end <= t_begin;
-      n_hi += end <= t_end - 1;
-    }
-    n_lo = wave_sum(n_lo);
-    n_hi = wave_sum(n_hi);
-    if (lane == 0) { atomicAdd(&s_own[0], n_lo); atomicAdd(&s_own[1], n_hi); }
-    __syncthreads();
-    s_first = s_own[0];
-    s_last = s_own[1];
+    s_first = __builtin_amdgcn_readfirstlane(n_lo);
+    s_last = __builtin_amdgcn_readfirstlane(n_hi);
     cu_own = s_cu + s_first;
   } else {
-    if (tid < 128) {  // one wave each
-      const int r = wave_count_le(g.cu + 1, g.n_seqs, wave ? t_end - 1 : t_begin, lane);
-      if (lane == 0) s_own[wave] = r;
+    if (wave == GAE_SEG_WAVES - 1) {  // (the one that searches for no group, at the same time)
+      const int r = wave_count_le(g.cu + 1, g.n_seqs, t_begin, lane);
+      // the next 64 ends hold the last token's as a rule
+      const int i = r + lane;
+      int l = __popcll(__builtin_amdgcn_ballot_w64(i < g.n_seqs && (int64_t)g.cu[i + 1] <= t_end - 1));
+      if (l == 64) l += wave_count_le(g.cu + 1 + r + 64, g.n_seqs - r - 64, t_end - 1, lane);
+      if (lane == 0) { s_own[0][0] = r; s_own[0][1] = r + l; }
     }
     __syncthreads();
-    s_first = s_own[0];
-    s_last = s_own[1];
-    if (s_last - s_first + 2 <= GAE_CU_LDS) {
+    s_first = s_own[0][0];
+    s_last = s_own[0][1];
+    if (s_last - s_first + 1 <= GAE_CU_LDS) {
       for (int i = tid; i <= s_last - s_first + 1; i += GAE_THREADS) s_cu[i] = g.cu[s_first + i];
       __syncthreads();
       cu_own = s_cu;
@@ -1054,24 +1181,26 @@ DEVI void gae_tile(const GaeArgs& g, const Tail& tail) {
   }
   const int n_own = s_last - s_first + 1;
   GaeTileGroups tg;
-  if constexpr (STATS) tg = gae_tile_groups(g, lo, s_grp);  // a barrier has passed since the search
+  if constexpr (STATS) {
+    tg = groups_from_lds ? gae_tile_groups_lds(g, lo, s_cu, s_gseq, s_first, s_last, n_behind) : gae_tile_groups(g, lo, s_grp);
+  }
 
-  // the crossing sequence's tokens [t_end, e), from t_end (a multiple of the tile when e > t_end)
+  // The crossing sequence's tokens [t_end, e) lie in `full` whole tiles and the tile with its last token. Their maps, a wave's
+  // chunk of 512 tokens at a time, are applied in fp64 one after the other from the right: those of the last tile made here,
+  // those of whole tiles taken from the blocks of these tiles (LOOK), or made here as well; the same numbers either way.
   double A0 = 0.0, nv0 = 0.0;
-  const int64_t e = (int64_t)cu_own[n_own];
+  const int64_t e = none ? 0 : (int64_t)cu_own[n_own];
   if (e > t_end) {
+    const int64_t last_tile = (e - 1) / GAE_TILE;
+    const int full = (int)(last_tile - tile) - 1;
     const float gam = g.discount;
     const float c = gam * (LAMBDAS ? g.lam_seq[s_last] : g.lam);
     const bool boot = g.no_eos != nullptr && g.no_eos[s_last] != 0;
     // (without values the mask is read in their place and dropped: no branch between the loads)
     const float* const values = g.values != nullptr ? g.values : g.mask;
-    // Runs of whole chunks of 512 tokens, one run per wave: each wave composes its own from the right, the next chunk
-    // on its way, and the block meets once at the end.
-    const int64_t chunks = (e - t_end + GAE_CHUNK - 1) / GAE_CHUNK, per_wave = (chunks + GAE_SEG_WAVES - 1) / GAE_SEG_WAVES;
-    const int64_t c_lo = wave * per_wave, c_hi = c_lo + per_wave < chunks ? c_lo + per_wave : chunks;
+    auto token_of = [&](int64_t from, int k) { return from * GAE_TILE + k * GAE_CHUNK + (int64_t)lane * GAE_ITEMS; };
     float crw[GAE_ITEMS], cv[GAE_ITEMS], cms[GAE_ITEMS];
-    auto fetch = [&](int64_t chunk) {
-      const int64_t t0 = t_end + chunk * GAE_CHUNK + (int64_t)lane * GAE_ITEMS;
+    auto fetch = [&](int64_t t0) {
       if (t0 + GAE_ITEMS <= g.n) {
 #pragma unroll
         for (int q = 0; q < GAE_ITEMS / 4; ++q) {
@@ -1095,50 +1224,107 @@ DEVI void gae_tile(const GaeArgs& g, const Tail& tail) {
         for (int i = 0; i < GAE_ITEMS; ++i) cv[i] = 0.f;
       }
     };
-    Map run = map_identity();
-    if (c_lo < c_hi) fetch(c_hi - 1);
-    for (int64_t chunk = c_hi - 1; chunk >= c_lo; --chunk) {
-      const int64_t t0 = t_end + chunk * GAE_CHUNK + (int64_t)lane * GAE_ITEMS;
-      const int64_t left = e - t0;  // the thread's tokens of the sequence
-      float xr[GAE_ITEMS], xv[GAE_ITEMS], xm[GAE_ITEMS];
-#pragma unroll
-      for (int i = 0; i < GAE_ITEMS; ++i) { xr[i] = crw[i]; xv[i] = cv[i]; xm[i] = cms[i]; }
-      if (chunk > c_lo) fetch(chunk - 1);
+    // whole: of a tile inside the sequence (its last token lies in a later one)
+    auto chunk_map = [&](auto whole, int64_t t0, const float (&r)[GAE_ITEMS], const float (&val)[GAE_ITEMS],
+                         const float (&mask)[GAE_ITEMS]) {
+      constexpr bool WHOLE = decltype(whole)::value;
+      const int left = e - t0 < 2 * GAE_ITEMS ? (int)(e - t0) : 2 * GAE_ITEMS;  // the thread's tokens of the sequence
       MapF acc = map_identity_t<float>();
 #pragma unroll
       for (int i = GAE_ITEMS - 1; i >= 0; --i) {
         // beyond the sequence (or the batch): identity; its last token: the constant map
-        const float m = i < left ? xm[i] : 0.f;
+        const float m = WHOLE || i < left ? mask[i] : 0.f;
         MapF f;
         f.a11 = fmaf(c, m, 1.f - m);
         f.a12 = gam * m;
         f.a22 = 1.f - m;
-        f.b1 = (xr[i] - xv[i]) * m;
-        f.b2 = xv[i] * m;
-        if (i == left - 1) f = MapF{0.f, 0.f, 0.f, 0.f, boot ? xv[i] : 0.f};
+        f.b1 = (r[i] - val[i]) * m;
+        f.b2 = val[i] * m;
+        if (!WHOLE && i == left - 1) f = MapF{0.f, 0.f, 0.f, 0.f, boot ? val[i] : 0.f};
         acc = compose(f, acc);
       }
-      const MapF part = wave_total_map(acc);
-      run = compose(Map{(double)part.a11, (double)part.a12, (double)part.a22, (double)part.b1, (double)part.b2}, run);
-    }
-    if (lane == 0) s_part[wave] = run;
-    __syncthreads();
-#pragma unroll
-    for (int w = GAE_SEG_WAVES - 1; w >= 0; --w) {
-      const Map m = s_part[w];
-      const double A1 = fma(m.a11, A0, fma(m.a12, nv0, m.b1));
-      nv0 = fma(m.a22, nv0, m.b2);
+      return wave_total_map(acc);
+    };
+    auto apply = [&](const MapF& m) {
+      const double A1 = fma((double)m.a11, A0, fma((double)m.a12, nv0, (double)m.b1));
+      nv0 = fma((double)m.a22, nv0, (double)m.b2);
       A0 = A1;
+    };
+    float xr[GAE_ITEMS], xv[GAE_ITEMS], xm[GAE_ITEMS];
+    auto take = [&] {
+#pragma unroll
+      for (int i = 0; i < GAE_ITEMS; ++i) { xr[i] = crw[i]; xv[i] = cv[i]; xm[i] = cms[i]; }
+    };
+    // whole tiles from the right, GAE_LOOK_TILES at a time
+    bool ask = LOOK;  // until one wait was in vain
+    int right = full, n = right < GAE_LOOK_TILES ? right : GAE_LOOK_TILES;
+    int64_t first = tile + 1 + right - n;
+    const bool in_end = last_tile * GAE_TILE + wave * GAE_CHUNK < e;  // the wave's chunk of the last tile holds tokens of it
+    if (in_end) fetch(token_of(last_tile, wave));
+    if constexpr (LOOK) {
+      // a tile inside one sequence that goes on behind it: tiles on its left may want its maps
+      if (n_own == 1 && (int64_t)cu_own[0] < lo)
+        publish_wave_map(look, tile, wave, chunk_map(std::true_type{}, lo + (int64_t)tid * GAE_ITEMS, rw, v, ms));
+    }
+    take();
+    if (!ask && n > 0) fetch(token_of(first, wave));  // on its way meanwhile
+    {
+      MapF m = map_identity_t<float>();
+      if (in_end) m = chunk_map(std::false_type{}, token_of(last_tile, wave), xr, xv, xm);
+      if (lane == 0) s_end[wave] = m;
+    }
+    for (bool at_end = true;; at_end = false) {  // uniform for the block
+      bool have = n == 0;
+      if (ask) {
+        if (!have && wave == 0) {
+          const bool all_there = gather_tile_maps(look, first, n, s_chunk);
+          if (lane == 0) s_have = all_there ? 1 : 0;
+        }
+        __syncthreads();
+        have = have || s_have != 0;
+        if (!have) { ask = false; fetch(token_of(first, wave)); }
+      }
+      if (!have) {
+        for (int k = wave; k < n * GAE_SEG_WAVES; k += GAE_SEG_WAVES) {
+          take();
+          if (k + GAE_SEG_WAVES < n * GAE_SEG_WAVES) fetch(token_of(first, k + GAE_SEG_WAVES));
+          const MapF m = chunk_map(std::true_type{}, token_of(first, k), xr, xv, xm);
+          if (lane == 0) s_chunk[k] = m;
+        }
+      }
+      if (!ask) __syncthreads();
+      if (at_end) {
+#pragma unroll
+        for (int w = GAE_SEG_WAVES - 1; w >= 0; --w) apply(s_end[w]);
+      }
+      for (int t = n - 1; t >= 0; --t) {
+        MapF m[GAE_SEG_WAVES];  // (read together: the chain is that of the products alone)
+#pragma unroll
+        for (int w = 0; w < GAE_SEG_WAVES; ++w) m[w] = s_chunk[t * GAE_SEG_WAVES + w];
+#pragma unroll
+        for (int w = GAE_SEG_WAVES - 1; w >= 0; --w) apply(m[w]);
+      }
+      right -= n;
+      if (right <= 0) break;
+      n = right < GAE_LOOK_TILES ? right : GAE_LOOK_TILES;
+      first = tile + 1 + right - n;
+      if (!ask) fetch(token_of(first, wave));
+      __syncthreads();  // s_chunk has been read
     }
   }
   float oa[GAE_ITEMS];
-  gae_one_tile<GAE_LAYOUT_CU, LAMBDAS>(g, tile, t_begin, t_end, s_first, n_own, cu_own, A0, nv0, smem, all, rw, v, ms, oa);
+  if (none) {
+#pragma unroll
+    for (int i = 0; i < GAE_ITEMS; ++i) oa[i] = 0.f;
+  } else {
+    gae_one_tile<GAE_LAYOUT_CU, LAMBDAS>(g, tile, t_begin, t_end, s_first, n_own, cu_own, A0, nv0, smem, all, rw, v, ms, oa);
+  }
   if constexpr (STATS) tail(tile, lo, hi, tg, oa, ms);
 }
 // STATS: also leaves the per-(tile, group) sums of GaeArgs::seg_stats.
 template <bool LAMBDAS, bool STATS>
 __global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_kernel(GaeArgs g) {
-  gae_tile<LAMBDAS, STATS>(g, [&](int64_t tile, int64_t lo, int64_t hi, const GaeTileGroups& tg, const float (&oa)[GAE_ITEMS],
+  gae_tile<LAMBDAS, STATS, false>(g, TileMaps{}, [&](int64_t tile, int64_t lo, int64_t hi, const GaeTileGroups& tg, const float (&oa)[GAE_ITEMS],
                                   const float (&ms)[GAE_ITEMS]) { gae_tile_group_stats(g, tile, lo, hi, tg, oa, ms); });
 }
 
@@ -1399,8 +1585,8 @@ DEVI float norm_one(const NormParams& p, float x, float m, bool has_mask) {
 // ---- Packed GAE and the normalisation of its advantages within groups of sequences in one launch: a tile's block keeps its
 // advantages in registers, publishes its sums per group and waits for those of the other tiles of its groups, each
 // wave for another group. A launch of its own read advantages and masks back and searched the groups again, several loads
-// that wait for each other. Both forms, GAE included, us: 1024 sequences of 1750 tokens in groups of 16 32.0 -> 27.8, 4096 of
-// 100 in fours (five groups to a tile) 55.9 -> 34.2, 64 of 300 22.2 -> 16.1, 64 of 8192 in eights 35.5 -> 32.2. The rule for
+// that wait for each other. Both forms, GAE included, us: 1024 sequences of 1750 tokens in groups of 16 30.4 / 27.1, 4096 of
+// 100 in fours (five groups to a tile) 56.3 / 35.2, 64 of 300 21.6 / 16.9, 64 of 8192 in eights 48 / 22. The rule for
 // the sizes of groups stands at areal_gae_packed_normalized_ex.
 // No wait is unbounded, as with adv_normalise_row: when the time is up, the block leaves a note for the (tile, group)
 // segment, whose advantages are in memory anyway, and a wave that finds all sums of a group looks for notes of its tiles and
@@ -1418,6 +1604,7 @@ struct GaeNormArgs {
   uint64_t *sums, *flags, *left;  // [seg_slots][SUMS_PITCH] and twice [seg_slots] in the workspace
   uint64_t call;
   unsigned wait_ticks;
+  TileMaps maps;
 };
 DEVI void gae_tile_normalise(const GaeNormArgs& a, int64_t tile, int64_t lo, int64_t hi, const GaeTileGroups& tg,
                              const float (&oa)[GAE_ITEMS], const float (&ms)[GAE_ITEMS]) {
@@ -1540,7 +1727,7 @@ DEVI void gae_tile_normalise(const GaeNormArgs& a, int64_t tile, int64_t lo, int
 }
 template <bool LAMBDAS>
 __global__ __launch_bounds__(GAE_THREADS, 4) void gae_tile_norm_kernel(GaeNormArgs a) {
-  gae_tile<LAMBDAS, true>(a.g, [&](int64_t tile, int64_t lo, int64_t hi, const GaeTileGroups& tg, const float (&oa)[GAE_ITEMS],
+  gae_tile<LAMBDAS, true, true>(a.g, a.maps, [&](int64_t tile, int64_t lo, int64_t hi, const GaeTileGroups& tg, const float (&oa)[GAE_ITEMS],
                                    const float (&ms)[GAE_ITEMS]) { gae_tile_normalise(a, tile, lo, hi, tg, oa, ms); });
 }
 
@@ -3012,7 +3199,8 @@ int areal_gae_packed_normalized(const float* rewards, const float* values, const
 // sequences of the largest group; wait_us as areal_group_norm_spec.
 size_t areal_gae_packed_normalized_workspace_bytes(int64_t n_tokens, int64_t n_groups) {
   if (n_tokens <= 0 || n_groups <= 0) return 0;
-  return std::max((size_t)(ceil_div_i64(n_tokens, GAE_TILE) + n_groups) * (SUMS_PITCH + 2) * sizeof(uint64_t),
+  const size_t tiles = (size_t)ceil_div_i64(n_tokens, GAE_TILE);
+  return std::max(((tiles + (size_t)n_groups) * (SUMS_PITCH + 2) + tiles * GAE_SEG_WAVES * MAP_PITCH) * sizeof(uint64_t),
                   areal_gae_segment_stats_bytes(n_tokens, n_groups)) + 256;
 }
 int areal_gae_packed_normalized_ex(const float* rewards, const float* values, const float* loss_mask,
@@ -3036,8 +3224,9 @@ int areal_gae_packed_normalized_ex(const float* rewards, const float* values, co
   if (!known) (void)hipGetLastError();
   // While all tiles are on the chip at once (4 blocks a CU) one launch is the better one for groups of any size measured,
   // up to 64 tiles; with more tiles the blocks that wait keep those that they wait for from starting. Two launches / one,
-  // us (tiles, tiles a group): 875, 14: 32.0 / 27.8; 875, 55: 32.5 / 31.0; 1024, 16: 49.7 / 46.6; 1024, 64: 50.3 / 49.7;
-  // 2000, 4: 54.4 / 51.0; 2000, 8: 60.3 / 59.3; 1953, 16: 53.7 / 61.9; 2000, 31: 57.6 / 72.8; 2048, 64: 73.5 / 155.7.
+  // us (tiles, tiles a group): 875, 14: 30.5 / 27.1; 875, 55: 31.1 / 29.5; 1024, 16: 35.0 / 28.8; 2000, 4: 57.2 / 53.3; and,
+  // with every block making the maps of whole tiles, 2000, 8: 60.3 / 59.3; 1953, 16: 53.7 / 61.9; 2000, 31: 57.6 / 72.8;
+  // 2048, 64: 73.5 / 155.7.
   const int64_t most_tiles = nb <= GAE_TILES_AT_ONCE ? 64 : 4;
   const bool one = known && capture == hipStreamCaptureStatusNone && tail_group < 0 && mean_level != LEVEL_BATCH &&
                    std_level != LEVEL_BATCH && nb <= (1 << 29) &&
@@ -3061,8 +3250,11 @@ int areal_gae_packed_normalized_ex(const float* rewards, const float* values, co
   a.sums = ws;
   a.flags = ws + SUMS_PITCH * a.g.seg_slots;
   a.left = a.flags + a.g.seg_slots;
+  a.maps.at = a.left + a.g.seg_slots;
   a.call = next_call_number();
   a.wait_ticks = group_wait_ticks(wait_us);
+  a.maps.call = a.call;
+  a.maps.ticks = nb <= GAE_TILES_AT_ONCE ? a.wait_ticks : 0;  // (a tile that is not on the chip yet is not waited for)
   const dim3 grid((unsigned)(ceil_div_i64(nb, 8) * 8));
   if (lambda_seq != nullptr) hipLaunchKernelGGL((gae_tile_norm_kernel<true>), grid, dim3(GAE_THREADS), 0, stream, a);
   else hipLaunchKernelGGL((gae_tile_norm_kernel<false>), grid, dim3(GAE_THREADS), 0, stream, a);

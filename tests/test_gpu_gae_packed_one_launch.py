@@ -38,6 +38,8 @@ def _run(dev, lens, sizes, levels, wait_us, *, unbiased=1, critic=True, lam=None
     if mask == "weights":
         m *= 0.25 + torch.rand(n, generator=g)
     first = torch.tensor([0] + sizes).cumsum(0)
+    if mask == "sparse":
+        m = (torch.rand(n, generator=g) > 0.999).float()
     if mask == "silent group":
         m[cu[first[1]]:cu[first[2]]] = 0
     r, v = torch.randn(n, generator=g), torch.randn(n, generator=g)
@@ -75,7 +77,27 @@ def _run(dev, lens, sizes, levels, wait_us, *, unbiased=1, critic=True, lam=None
             assert (a - b).abs().max().item() <= 2.0 ** -21 * a.abs().max().item()
         else:
             assert torch.equal(a, b)
+    if mask == "sparse":
+        want = _recurrence(r, v if critic else torch.zeros(n), m, cu, no_eos.cpu(), lam_seq.cpu() if lam else torch.full((n_seqs,), 0.95))
+        # masked tokens alone change the state, and each takes the error before it by 0.99 lambda < 0.95: 20 tokens' worth
+        # stays, of at most 24 roundings each (8 tokens, 6 steps of the wave's tree, two operations a step)
+        assert (res[1][1].cpu().double() - want).abs().max().item() <= 20 * 24 * 2.0 ** -24 * want.abs().max().item()
     return begin.elapsed_time(end) * 1e3
+
+
+def _recurrence(r, v, m, cu, no_eos, lam):
+    """Advantages in fp64, token by token."""
+    r, v, m, ends = r.double().tolist(), v.double().tolist(), m.double().tolist(), cu.tolist()
+    want = torch.zeros(len(r), dtype=torch.float64)
+    for s, (a, b) in enumerate(zip(ends, ends[1:])):
+        c, adv, nv = 0.99 * float(lam[s]), 0.0, 0.0
+        for t in range(b - 1, a - 1, -1):
+            if t == b - 1:
+                nv = v[t] if no_eos[s] else 0.0
+            else:
+                adv, nv = (c * m[t] + 1 - m[t]) * adv + m[t] * (0.99 * nv + r[t] - v[t]), (1 - m[t]) * nv + m[t] * v[t]
+            want[t] = adv
+    return want
 
 
 def _lens(n, mean, seed):
@@ -99,6 +121,22 @@ def test_same_bits_as_two_launches(dev, case, wait_us):
     levels = [(2, 2), (0, 2), (2, 0), (0, 0)][case % 4]
     _run(dev, lens, sizes, (2, 2), wait_us, **options)
     _run(dev, lens, sizes, levels, wait_us, **options)
+
+
+@pytest.mark.parametrize("wait_us", [-1, 0])
+@pytest.mark.parametrize("case", range(5))
+def test_state_carried_over_whole_tiles(dev, case, wait_us):
+    """Sequences over 0, 1, 16, 17 and 40 whole tiles, whose maps come from their blocks 16 tiles at a time; as many sequences
+    and groups as fit a block's memory and one more of each. One token in 1000 is masked in, so the state goes far."""
+    long = [40 * 2048 + 5, 3, 17 * 2048, 18 * 2048 + 1, 0, 1, 2047, 2048, 2049, 3 * 2048, 4095, 5, 0, 1, 17 * 2048 + 2047, 9]
+    lens, sizes, options = [
+        (long, [8, 8], dict()),
+        (long, [8, 8], dict(lam=True, around=(37, 5000))),
+        (long[::-1], [8, 8], dict(critic=False)),
+        ([120] * 2047 + [30000], [2] * 1023 + [1, 1], dict()),
+        ([30000] + [120] * 2048, [2] * 1023 + [3], dict()),
+    ][case]
+    _run(dev, lens, sizes, (2, 2), wait_us, mask="sparse", **options)
 
 
 @pytest.mark.parametrize("wait_us", [-1, 0])
