@@ -1171,7 +1171,9 @@ DEVI void gae_tile(const GaeArgs& g, const TileMaps& look, const Tail& tail) {
     __syncthreads();
     s_first = s_own[0][0];
     s_last = s_own[0][1];
-    if (s_last - s_first + 1 <= GAE_CU_LDS) {
+    if (none) {
+      cu_own = g.cu;  // (not read: behind the last sequence there is no next entry)
+    } else if (s_last - s_first + 1 <= GAE_CU_LDS) {
       for (int i = tid; i <= s_last - s_first + 1; i += GAE_THREADS) s_cu[i] = g.cu[s_first + i];
       __syncthreads();
       cu_own = s_cu;

@@ -140,6 +140,23 @@ def test_state_carried_over_whole_tiles(dev, case, wait_us):
 
 
 @pytest.mark.parametrize("wait_us", [-1, 0])
+@pytest.mark.parametrize("case", range(6))
+def test_more_sequences_than_a_block_holds(dev, case, wait_us):
+    """Above 2048 sequences a wave searches for them, and what it finds tells the groups while these fit (up to 1024): ends of
+    more than 64 sequences in a tile, more sequences in a tile than the block's memory holds, empty groups, tiles before the
+    first and behind the last sequence."""
+    lens, sizes, options = [
+        ([120] * 2049, [3] * 683, dict(around=(37, 5000))),
+        ([200] * 2100, [2, 1] * 700, dict(around=(4100, 5000), lam=True)),            # more groups than the block holds
+        (_lens(3000, 40, 11), [16, 0, 8] * 125, dict()),
+        ([0] * 2500 + [700] * 30 + [0] * 2500 + [1500], [1, 2499, 30, 2500, 1], dict()),
+        ([1] * 4200 + [9000] + [1] * 63 + [2048] * 2, [100] * 42 + [66], dict(critic=False)),
+        (_lens(4097, 60, 12), [17] * 241, dict()),
+    ][case]
+    _run(dev, lens, sizes, (2, 2), wait_us, mask="sparse", **options)
+
+
+@pytest.mark.parametrize("wait_us", [-1, 0])
 def test_more_tiles_than_the_chip_holds(dev, wait_us):
     _run(dev, _lens(4800, 700, 9), [4] * 1200, (2, 2), wait_us)
 
