@@ -845,8 +845,11 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
 // also took cu_seqlens once): faster on 64 x 16384 tokens and on 4 x 32768, where a walking block has 16 tiles in a row.
 // The layout comes first. Up to 2048 sequences (and 1024 groups) cu_seqlens and the groups' first sequences go to LDS
 // whole, and what the tile has to find in them is counted from the registers on the way: one barrier, no load that waits
-// for another. With 4096 (16 loads a thread) the search in memory is as fast: 3000 x 300 22.3 against 21.5 us, 4096 x 300 24.5
-// against 23.3. There the wave that has no group to find finds the sequences, meanwhile.
+// for another. Above 2048 a wave searches for the sequences: its first 64 probes go out with the block's first loads, one more
+// load of 128 entries holds all that the tile needs of up to 4096 sequences, and the groups are counted in LDS from what it
+// finds. With 4096 in LDS (16 loads a thread) 4000 sequences of 300 took 23.0 us, with this search 22.4; with searches that wait
+// for each other (of groups, first and last sequence, then their starts) 4096 x 300 took 22.8, with this one 22.3, 4096 x 1000
+// 51.8 and 50.4.
 // The kernel is bound by vector instruction issue (about 1150 vector and 250 scalar instructions
 // per wave and tile on 1024 sequences of mean length 1760, half as many again with the group sums) for half of its time and by
 // the chain of loads, maps and sums for the other half, with four blocks resident per CU, so
@@ -872,10 +875,17 @@ DEVI void gae_tile_group_search(const GaeArgs& g, int64_t lo, int64_t hi, int* s
 struct GaeTileGroups {
   int g_first, g_last, g_next;
   int64_t b[3];
-  const int32_t *cu, *gseq;  // cu_seqlens and the groups' first sequences in LDS, or null
+  bool cu_in_lds, gseq_in_lds;
+  const int32_t *cu, *gseq;  // cu_seqlens and the groups' first sequences there
+  DEVI int64_t bound(const GaeArgs& g, int j) const {
+    if (!gseq_in_lds) return group_offsets(g)[j];
+    const int s = gseq[j];
+    return cu_in_lds ? (int64_t)cu[s] : (int64_t)g.cu[s];
+  }
 };
 DEVI GaeTileGroups gae_tile_groups(const GaeArgs& g, int64_t lo, const int* s_grp) {
   GaeTileGroups r;
+  r.cu_in_lds = r.gseq_in_lds = false;
   r.cu = r.gseq = nullptr;
   r.g_first = s_grp[0];
   r.g_last = s_grp[1] < g.n_groups ? s_grp[1] : g.n_groups - 1;
@@ -889,10 +899,11 @@ DEVI GaeTileGroups gae_tile_groups(const GaeArgs& g, int64_t lo, const int* s_gr
 }
 // The same from LDS, by every wave for itself. n_lo, n_hi, n_behind: how many sequences end at or before each of the three
 // tokens; a group has ended there exactly when the next one's first sequence is not among those still to come.
-DEVI GaeTileGroups gae_tile_groups_lds(const GaeArgs& g, int64_t lo, const int32_t* cu, const int32_t* gseq, int n_lo, int n_hi,
-                                       int n_behind) {
+DEVI GaeTileGroups gae_tile_groups_lds(const GaeArgs& g, int64_t lo, bool cu_in_lds, const int32_t* cu, const int32_t* gseq,
+                                       int n_lo, int n_hi, int n_behind) {
   const int lane = threadIdx.x & 63;
   GaeTileGroups r;
+  r.cu_in_lds = cu_in_lds; r.gseq_in_lds = true;
   r.cu = cu; r.gseq = gseq;
   int c0 = 0, c1 = 0, c2 = 0;
   for (int j0 = 1; j0 <= g.n_groups; j0 += 64) {
@@ -906,14 +917,14 @@ DEVI GaeTileGroups gae_tile_groups_lds(const GaeArgs& g, int64_t lo, const int32
   r.g_last = c1 < g.n_groups ? c1 : g.n_groups - 1;
   r.g_next = c2;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) r.b[i] = (int64_t)cu[gseq[r.g_first + i <= g.n_groups ? r.g_first + i : g.n_groups]] - lo;
+  for (int i = 0; i < 3; ++i) r.b[i] = r.bound(g, r.g_first + i <= g.n_groups ? r.g_first + i : g.n_groups) - lo;
   return r;
 }
 
 // Where the k-th group of the tile lies, relative to the tile's first token.
 // (selects, not an index: an indexed register array would live in scratch memory)
 DEVI void tile_group_bounds(const GaeArgs& g, const GaeTileGroups& tg, int64_t lo, int k, int64_t& b0, int64_t& b1) {
-  auto bound = [&](int j) { return (tg.cu != nullptr ? (int64_t)tg.cu[tg.gseq[j]] : group_offsets(g)[j]) - lo; };
+  auto bound = [&](int j) { return tg.bound(g, j) - lo; };
   b0 = k == 0 ? tg.b[0] : k == 1 ? tg.b[1] : k == 2 ? tg.b[2] : bound(tg.g_first + k);
   b1 = k == 0 ? tg.b[1] : k == 1 ? tg.b[2] : bound(tg.g_first + k + 1);
 }
@@ -1071,10 +1082,11 @@ DEVI void gae_tile(const GaeArgs& g, const TileMaps& look, const Tail& tail) {
   // All that the block reads at its start goes out together, the layout first (loads come back in their order): the whole
   // of cu_seqlens and the groups' first sequences for LDS, and the tile's inputs.
   const bool cu_in_lds = g.n_seqs <= GAE_CU_LDS;
-  const bool groups_in_lds = STATS && cu_in_lds && g.goff == nullptr && g.n_groups <= GAE_GROUPS_LDS;
+  const bool groups_in_lds = STATS && g.goff == nullptr && g.n_groups <= GAE_GROUPS_LDS;
   constexpr int CU_LOADS = GAE_CU_LDS / GAE_THREADS, CU_FIRST = 5, GROUP_LOADS = STATS ? GAE_GROUPS_LDS / GAE_THREADS : 1;
   int32_t c[CU_LOADS], gq[GROUP_LOADS];
   const bool many = g.n_seqs >= CU_FIRST * GAE_THREADS;  // (uniform)
+  const int probe_step = (g.n_seqs + 63) >> 6;
   auto cu_of = [&](int k) { const int i = tid + k * GAE_THREADS; return g.cu[i < g.n_seqs ? i : g.n_seqs]; };  // (behind them: cov_hi)
   if (cu_in_lds) {
 #pragma unroll
@@ -1083,12 +1095,14 @@ DEVI void gae_tile(const GaeArgs& g, const TileMaps& look, const Tail& tail) {
 #pragma unroll
       for (int k = CU_FIRST; k < CU_LOADS; ++k) c[k] = cu_of(k);
     }
-    if (groups_in_lds) {
+  } else {  // the first probes of the search, which need no other load either
+    c[0] = g.cu[1 + (lane * probe_step < g.n_seqs ? lane * probe_step : g.n_seqs - 1)];
+  }
+  if (groups_in_lds) {
 #pragma unroll
-      for (int k = 0; k < GROUP_LOADS; ++k) {
-        const int i = tid + k * GAE_THREADS;
-        if (k == 0 || k * GAE_THREADS < g.n_groups) gq[k] = (int32_t)g.gseq[i < g.n_groups ? i : g.n_groups];
-      }
+    for (int k = 0; k < GROUP_LOADS; ++k) {
+      const int i = tid + k * GAE_THREADS;
+      if (k == 0 || k * GAE_THREADS < g.n_groups) gq[k] = (int32_t)g.gseq[i < g.n_groups ? i : g.n_groups];
     }
   }
   float rw[GAE_ITEMS], v[GAE_ITEMS], ms[GAE_ITEMS];
@@ -1104,6 +1118,15 @@ DEVI void gae_tile(const GaeArgs& g, const TileMaps& look, const Tail& tail) {
   if constexpr (STATS) {
     if (groups_in_lds && !groups_from_lds) gae_tile_group_search(g, lo, hi, s_grp);
   }
+  auto store_groups = [&] {
+    if constexpr (STATS) {
+      if (!groups_in_lds) return;
+#pragma unroll
+      for (int k = 0; k < GROUP_LOADS; ++k)
+        if (k == 0 || k * GAE_THREADS < g.n_groups) s_gseq[tid + k * GAE_THREADS] = gq[k];
+      if (tid == 0) s_gseq[g.n_groups] = (int32_t)gseq_end;
+    }
+  };
   // Sequences that end at or before the first token, the last token, and the token behind the tile.
   int n_lo = 0, n_hi = 0, n_behind = 0;
   if (cu_in_lds) {
@@ -1124,16 +1147,9 @@ DEVI void gae_tile(const GaeArgs& g, const TileMaps& look, const Tail& tail) {
 #pragma unroll
       for (int k = CU_FIRST; k < CU_LOADS; ++k) count(k);
     }
-    if constexpr (STATS) {
-      if (groups_in_lds) {
-#pragma unroll
-        for (int k = 0; k < GROUP_LOADS; ++k)
-          if (k == 0 || k * GAE_THREADS < g.n_groups) s_gseq[tid + k * GAE_THREADS] = gq[k];
-      }
-    }
-    if (tid == 0) {  // the last entry of each
+    store_groups();
+    if (tid == 0) {  // the last entry
       s_cu[g.n_seqs] = (int32_t)cov_hi;
-      if (STATS && groups_in_lds) s_gseq[g.n_groups] = (int32_t)gseq_end;
       n_lo += (int32_t)cov_hi <= x0;
       n_hi += (int32_t)cov_hi <= x1;
       if constexpr (STATS) n_behind += (int32_t)cov_hi <= x2;
@@ -1160,19 +1176,39 @@ DEVI void gae_tile(const GaeArgs& g, const TileMaps& look, const Tail& tail) {
     s_last = __builtin_amdgcn_readfirstlane(n_hi);
     cu_own = s_cu + s_first;
   } else {
-    if (wave == GAE_SEG_WAVES - 1) {  // (the one that searches for no group, at the same time)
-      const int r = wave_count_le(g.cu + 1, g.n_seqs, t_begin, lane);
-      // the next 64 ends hold the last token's as a rule
-      const int i = r + lane;
-      int l = __popcll(__builtin_amdgcn_ballot_w64(i < g.n_seqs && (int64_t)g.cu[i + 1] <= t_end - 1));
-      if (l == 64) l += wave_count_le(g.cu + 1 + r + 64, g.n_seqs - r - 64, t_end - 1, lane);
-      if (lane == 0) { s_own[0][0] = r; s_own[0][1] = r + l; }
+    if (wave == GAE_SEG_WAVES - 1) {  // (the one that searches for no group, where groups are searched for)
+      const int hits = __popcll(__builtin_amdgcn_ballot_w64(lane * probe_step < g.n_seqs && (int64_t)c[0] <= t_begin));
+      const int most = hits > 0 ? probe_step - 1 : 0;
+      int from = hits > 0 ? (hits - 1) * probe_step + 1 : 0;
+      if (probe_step > 64) from += wave_count_le(g.cu + 1 + from, most < g.n_seqs - from ? most : g.n_seqs - from, t_begin, lane);
+      // cu_seqlens from `from` on: the first token's sequence is one of the next 64, and as a rule all that the tile has to
+      // know follows within 64 more
+      const int i0 = from + lane, i1 = i0 + 64;
+      const int32_t e0 = g.cu[i0 < g.n_seqs ? i0 : g.n_seqs], e1 = g.cu[i1 < g.n_seqs ? i1 : g.n_seqs];
+      auto ended = [&](int64_t x) {
+        return from + __popcll(__builtin_amdgcn_ballot_w64(lane > 0 && i0 <= g.n_seqs && (int64_t)e0 <= x)) +
+               __popcll(__builtin_amdgcn_ballot_w64(i1 <= g.n_seqs && (int64_t)e1 <= x));
+      };
+      const int r = ended(t_begin);
+      int l = ended(t_end - 1), b = STATS ? ended(hi) : 0;
+      const bool held = l < from + 127;
+      if (!held) l += wave_count_le(g.cu + 1 + l, g.n_seqs - l, t_end - 1, lane);
+      if (STATS && b == from + 127) b += wave_count_le(g.cu + 1 + b, g.n_seqs - b, hi, lane);
+      if (held) {
+        if (i0 >= r && i0 <= l + 1) s_cu[i0 - r] = e0;
+        if (i1 >= r && i1 <= l + 1) s_cu[i1 - r] = e1;
+      }
+      if (lane == 0) { s_own[0][0] = r; s_own[0][1] = l; s_own[0][2] = b; s_own[1][0] = held; }
     }
+    store_groups();
     __syncthreads();
-    s_first = s_own[0][0];
-    s_last = s_own[0][1];
+    s_first = __builtin_amdgcn_readfirstlane(s_own[0][0]);
+    s_last = __builtin_amdgcn_readfirstlane(s_own[0][1]);
+    n_behind = s_own[0][2];
     if (none) {
       cu_own = g.cu;  // (not read: behind the last sequence there is no next entry)
+    } else if (s_own[1][0] != 0) {
+      cu_own = s_cu;
     } else if (s_last - s_first + 1 <= GAE_CU_LDS) {
       for (int i = tid; i <= s_last - s_first + 1; i += GAE_THREADS) s_cu[i] = g.cu[s_first + i];
       __syncthreads();
@@ -1184,7 +1220,8 @@ DEVI void gae_tile(const GaeArgs& g, const TileMaps& look, const Tail& tail) {
   const int n_own = s_last - s_first + 1;
   GaeTileGroups tg;
   if constexpr (STATS) {
-    tg = groups_from_lds ? gae_tile_groups_lds(g, lo, s_cu, s_gseq, s_first, s_last, n_behind) : gae_tile_groups(g, lo, s_grp);
+    tg = groups_from_lds ? gae_tile_groups_lds(g, lo, cu_in_lds, s_cu, s_gseq, s_first, s_last, n_behind)
+                         : gae_tile_groups(g, lo, s_grp);
   }
 
   // The crossing sequence's tokens [t_end, e) lie in `full` whole tiles and the tile with its last token. Their maps, a wave's
