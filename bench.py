@@ -26,13 +26,13 @@ PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA peak used for the roofline f
 
 # The contraction kernels of the default workload as rocprofv3 names them (checked against the
 # loaded library before they are printed). gemm16_sweep<variant, epilogue>: variant 0 = both
-# operands k-contiguous, 1 = both k-major, 2 = A k-major; Fwd16<edge, affine, moments, save>,
-# Store16<edge, mode> with mode 0 = bf16, 3 = bf16 scaled per output row.
-KERNEL_FWD_SAVE = "gemm16_sweep<0, Fwd16<false, false, false, true> >"
-KERNEL_FWD = "gemm16_sweep<0, Fwd16<false, false, false, false> >"
+# operands k-contiguous, 1 = both k-major, 2 = A k-major; Fwd16<edge, affine, moments, save, past>,
+# Store16<edge, mode, past> with mode 0 = bf16, 3 = bf16 scaled per output row.
+KERNEL_FWD_SAVE = "gemm16_sweep<0, Fwd16<false, false, false, true, false> >"
+KERNEL_FWD = "gemm16_sweep<0, Fwd16<false, false, false, false, false> >"
 KERNEL_RECOMPUTE = "gemm16_sweep<0, Bwd16<false, false> >"
-KERNEL_DHIDDEN = "gemm16_sweep<2, Store16<false, 3> >"
-KERNEL_DWEIGHT = "gemm16_sweep<1, Store16<false, 0> >"
+KERNEL_DHIDDEN = "gemm16_sweep<2, Store16<false, 3, false> >"
+KERNEL_DWEIGHT = "gemm16_sweep<1, Store16<false, 0, false> >"
 
 WORKLOADS = {
     # name: (T, H, n_seqs, min_len, max_len, seed, description)
