@@ -234,6 +234,19 @@ static double xcd_distinct(int nb, int S) {
 // 2048 290, 277, 231 / 272, 235, 232; 400 x 5120 620, 699, 550 / 588, 645, 552; 700 x 896 237, 210, 176 / 223, 198, 181 (222 MB of
 // exponentials; dHidden in front of dWeight 225, 211, 183). With more of them than the cache holds the hints only cost: steps
 // of 1000 x 1024 (304 MB) 822 / 829, of 4096 x 896 2600 / 2760. A weight that fits it itself is not streamed.
+// With a bias, a scale or moments too, bf16 steps: 509 x 896 486 / 458, 480 / 446, 471 / 434; 400 x 5120 1926 / 1833, 1911 / 1822,
+// 1898 / 1815.
+// Which contraction comes first is the gradient's matter. In bf16 dWeight goes past the cache, and dHidden behind it still finds
+// the exponentials. An fp32 dWeight is stored or added to through the cache (4 or 8 bytes a weight, 0.5 GB at the least) and
+// leaves nothing of them: dHidden comes first. Steps with fp32 gradients, us, no hints / dWeight first / dHidden first: 500 x 896
+// 620 / 615 / 603, 300 x 2048 984 / 1029 / 950, 300 x 8192 2691 / 2748 / 2621, 700 x 1024 795 / 829 / 791, 600 x 4096 2340 / 2386 /
+// 2360; stored, then added to by a second such batch: 896 1253 / 1277 / 1241, 1536 1742 / 1743 / 1706, 4096 4201 / 4262 / 4179.
+// Added to alone: 509 x 896 588 / 592 / 586, 256 x 896 474 / 482 / 481, 700 x 896 744 / 777 / 753, 700 x 1024 779 / 811 / 780, 600 x
+// 2048 1357 / 1405 / 1350, 400 x 5120 2543 / 2635 / 2545, 300 x 8192 3344 / 3389 / 3273.
+// A backward that makes dlogits anew writes them past the cache, and its contractions gain from the hints even so where both read
+// them as they are written: 256 x 2048 750 -> 650, 512 x 1536 837 -> 799 (fp32 1002 -> 985, 1029 -> 1030). Where dWeight reads a
+// transposed copy (a chunk that is no multiple of 64 tokens) the hints cost: 700 x 1024 1022 / 1035, 400 x 5120 4388 / 4412 (fp32
+// 1155 / 1173, 5224 / 5244).
 constexpr int64_t PAST_PROBS_MOST = (int64_t)224 << 20, PAST_WEIGHT_LEAST = (int64_t)240 << 20;
 static bool past_cache(int64_t T, int64_t H, int64_t V) {
   return round_up_i64(T, 2 * BK) * round_up_i64(V, BK) * 2 <= PAST_PROBS_MOST && V * H * 2 >= PAST_WEIGHT_LEAST;
@@ -1966,10 +1979,13 @@ template <bool E> using Fwd16PlainMom = Fwd16<E, false, true, false>;
 template <bool E> using Fwd16Affine = Fwd16<E, true, false, false>;
 template <bool E> using Fwd16AffineMom = Fwd16<E, true, true, false>;
 template <bool E> using Fwd16PlainSave = Fwd16<E, false, false, true>;
-template <bool E> using Fwd16PlainSavePast = Fwd16<E, false, false, true, !E>;
 template <bool E> using Fwd16PlainMomSave = Fwd16<E, false, true, true>;
 template <bool E> using Fwd16AffineSave = Fwd16<E, true, false, true>;
 template <bool E> using Fwd16AffineMomSave = Fwd16<E, true, true, true>;
+template <bool E> using Fwd16PlainSavePast = Fwd16<E, false, false, true, !E>;
+template <bool E> using Fwd16PlainMomSavePast = Fwd16<E, false, true, true, !E>;
+template <bool E> using Fwd16AffineSavePast = Fwd16<E, true, false, true, !E>;
+template <bool E> using Fwd16AffineMomSavePast = Fwd16<E, true, true, true, !E>;
 
 // ---- forward for the label log-probabilities alone (see Fwd16): the sum of a token's exponentials relative to
 // a reference of its own, at first the largest logit of the first column. Per logit one accumulator read, one
@@ -2497,7 +2513,7 @@ bool dh_weight_in_place(int64_t V) { return V % BK == 0 && V >= 2 * BK; }
 // dh_weight_in_place(V), else its transposed copy W^T [H, ldv].
 template <int KERNEL16>
 int launch_dhidden_k(const GemmArgs& g0, int64_t H, int64_t T, int64_t ldv, void* dhidden,
-                     float* partial, const float* tscale, int z_fixed, hipStream_t stream, bool past = false) {
+                     float* partial, const float* tscale, int z_fixed, hipStream_t stream, bool past) {
   GemmArgs g = g0;
   const DhPlan plan = plan_dh(H, T, ldv, z_fixed);
   int z = plan.z;
@@ -2522,15 +2538,15 @@ int launch_dhidden_k(const GemmArgs& g0, int64_t H, int64_t T, int64_t ldv, void
 }
 int launch_dhidden(const u16* w, int64_t V, const u16* dl, int64_t ldv, int64_t H, int64_t T,
                    void* dhidden, float* partial, const float* tscale, const int* skip_if_set,
-                   int z_fixed, hipStream_t stream) {
+                   int z_fixed, hipStream_t stream, bool past) {
   if (dh_weight_in_place(V)) {
     GemmArgs g{w, H, (int)H, dl, ldv, (int)T, (int)ldv, (int)H, 0};
     g.skip_if_set = skip_if_set;
-    return launch_dhidden_k<KERNEL16_MIX>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream, past_cache(T, H, V));
+    return launch_dhidden_k<KERNEL16_MIX>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream, past);
   }
   GemmArgs g{w, ldv, (int)H, dl, ldv, (int)T, (int)ldv, 0, 0};
   g.skip_if_set = skip_if_set;
-  return launch_dhidden_k<KERNEL16_NT>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream);
+  return launch_dhidden_k<KERNEL16_NT>(g, H, T, ldv, dhidden, partial, tscale, z_fixed, stream, false);
 }
 
 // dWeight [V, H] in bf16 has ceil(V / 256) x ceil(H / 256) output tiles. When their number is not a
@@ -2595,9 +2611,8 @@ size_t dw_tail_bytes(int64_t H, int64_t V, int64_t Tpad) {
 // g.B [K, ldv]: whole rounds in one launch, then (plan_dw_tail) the remaining
 // vocabulary rows with the token range split, through dw_part (dw_tail_bytes(H, V, K) bytes).
 int launch_dweight_bf16(GemmArgs g, int64_t H, int64_t V, int64_t ldv, void* dweight, float* dw_part,
-                        hipStream_t stream) {
+                        hipStream_t stream, bool past) {
   const int64_t K = g.K;
-  const bool past = past_cache(K, H, V);
   const DwTail tail = dw_part != nullptr ? plan_dw_tail(H, V, K) : DwTail{0, 1, 0, 0, 32};
   int rc;
   if (tail.z <= 1) {
@@ -2749,8 +2764,12 @@ int areal_lmhead_fwd_ex(const void* hidden, const void* weight, const float* bia
     return launch_gemm<Fwd16AffineMom, FwdAffineMom, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
   };
   auto fwd_save = [&](const GemmArgs& gg) {
-    if (!affine && !moments && past_cache(T, H, V))
-      return launch_gemm<Fwd16PlainSavePast, FwdPlainSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+    if (past_cache(T, H, V)) {
+      if (!affine && !moments) return launch_gemm<Fwd16PlainSavePast, FwdPlainSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+      if (!affine) return launch_gemm<Fwd16PlainMomSavePast, FwdPlainMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+      if (!moments) return launch_gemm<Fwd16AffineSavePast, FwdAffineSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+      return launch_gemm<Fwd16AffineMomSavePast, FwdAffineMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
+    }
     if (!affine && !moments) return launch_gemm<Fwd16PlainSave, FwdPlainSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
     if (!affine) return launch_gemm<Fwd16PlainMomSave, FwdPlainMomSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
     if (!moments) return launch_gemm<Fwd16AffineSave, FwdAffineSave, FwdParams, KERNEL16_NT, true>(gg, r, ep, ep_a, stream);
@@ -2883,6 +2902,7 @@ int areal_lmhead_bwd(const void* hidden, const void* weight, const float* bias,
     // dWeight reads dl and hidden k-major (no transposed copies) when the chunk is a multiple
     // of 64 tokens (at least 128); otherwise it goes through dlT and hidden^T.
     const bool tn = k16_ok(Tc) && dweight_f32 != nullptr;
+    const bool past = k16_ok(Tc) && past_cache(Tc, H, V);
     const bool need_dlT = dweight_f32 != nullptr && !tn;
     // 1. recompute logits of the chunk, emit dlogits
     {
@@ -2902,7 +2922,7 @@ int areal_lmhead_bwd(const void* hidden, const void* weight, const float* bias,
     // 2. dHidden[t, h] = sum_v dl[t, v] * W^T[h, v]
     if (dhidden != nullptr) {
       if ((rc = launch_dhidden(w_in_place ? (const u16*)weight : wT, V, dl, ldv, H, Tc,
-                               (u16*)dhidden + t0 * H, dh_part, nullptr, nullptr, dh_z, stream)) != AREAL_OK)
+                               (u16*)dhidden + t0 * H, dh_part, nullptr, nullptr, dh_z, stream, past)) != AREAL_OK)
         return rc;
     }
     // dBias[v] += sum_t dl[t, v]
@@ -2915,7 +2935,7 @@ int areal_lmhead_bwd(const void* hidden, const void* weight, const float* bias,
     if (tn) {
       GemmArgs g{hid_c, H, (int)H, dl, ldv, (int)V, (int)Tc, (int)H, (int)ldv};
       const StoreParams ep{dweight_f32, H, (int)H, (int)V};
-      rc = dw_bf16 ? launch_dweight_bf16(g, H, V, ldv, dweight, dw_part, stream)
+      rc = dw_bf16 ? launch_dweight_bf16(g, H, V, ldv, dweight, dw_part, stream, past)
                    : launch_store<KERNEL16_TN>(g, ep, (accumulate == 1 || t0 > 0) ? 2 : 1, stream);
       if (rc != AREAL_OK) return rc;
     } else if (dweight_f32 != nullptr) {
@@ -2992,6 +3012,7 @@ int areal_lmhead_bwd_saved(const void* hidden, const void* weight, const int64_t
                      (int)H, (int)V, inv_temperature * LOG2E, inv_temperature * logit_scale, rowfac,
                      dweight != nullptr ? hs : nullptr, probs_status);
   AREAL_CHECK_LAUNCH();
+  const bool past = past_cache(T, H, V);  // as the forward that wrote e'
   auto dhidden_launches = [&]() -> int {
     if (dhidden == nullptr) return AREAL_OK;
     if (!w_in_place) {
@@ -3001,7 +3022,7 @@ int areal_lmhead_bwd_saved(const void* hidden, const void* weight, const int64_t
       AREAL_CHECK_LAUNCH();
     }
     return launch_dhidden(w_in_place ? (const u16*)weight : wT, V, e, ldv, H, T, dhidden, dh_part, rowfac, probs_status, 0,
-                          stream);
+                          stream, past);
   };
   auto dweight_launches = [&]() -> int {
     if (dweight == nullptr) return AREAL_OK;
@@ -3009,13 +3030,13 @@ int areal_lmhead_bwd_saved(const void* hidden, const void* weight, const int64_t
     // T are cleared)
     GemmArgs g{hs, H, (int)H, e, ldv, (int)V, (int)Tpad, (int)H, (int)ldv};
     g.skip_if_set = probs_status;
-    if (dweight_mode == 2) return launch_dweight_bf16(g, H, V, ldv, dweight, dw_part, stream);
+    if (dweight_mode == 2) return launch_dweight_bf16(g, H, V, ldv, dweight, dw_part, stream, past);
     const StoreParams ep{dweight, H, (int)H, (int)V, nullptr};
     return launch_store<KERNEL16_TN>(g, ep, dweight_mode == 1 ? 2 : 1, stream);
   };
-  // dWeight in front where e' lies in the memory-side cache: the weight that dHidden reads would push some of it out. The
-  // other way round elsewhere: steps of 4096 x 896 2610 us for 2635, of 16384 x 1536 with fp32 masters 16350 for 16490.
-  const bool dw_first = past_cache(T, H, V);
+  // dWeight in front where e' lies in the memory-side cache and dWeight goes past it: the weight that dHidden reads would push some
+  // of e' out. The other way round elsewhere: steps of 4096 x 896 2610 us for 2635, of 16384 x 1536 with fp32 masters 16350 for 16490.
+  const bool dw_first = past && dweight_mode == 2;
   if (dw_first && (rc = dweight_launches()) != AREAL_OK) return rc;
   if ((rc = dhidden_launches()) != AREAL_OK) return rc;
   if (dbias != nullptr) {
