@@ -1285,12 +1285,13 @@ py::dict pack_dict(const py::dict& data, const Tensor& attention_mask) {
   return out;
 }
 
-// A packed batch padded with zeros to `to` tokens, for the total that its tensors' shapes suggest (the longest one-dimensional
-// one's elements): (padded dict, pad length, copy of the offsets). The launch reports the total it met. Where that is another one,
-// it (the caller pads anew); nothing where this is not the way (no such tensor, position ids, a length that is no
-// plain int, tensors that the kernel does not take: the caller's own way says what is wrong with them, if it meets them).
+// A packed batch padded with zeros to `to` tokens, for the total that its tensors' shapes suggest (the elements of the
+// one-dimensional ones): (padded dict, pad length, copy of the offsets). The launch reports the total it met. Where that is another
+// one, it (the caller pads anew); nothing where this is not the way (no such tensor, or of several lengths, position
+// ids, a length that is no plain int, tensors that the kernel does not take: the caller's own way says what is wrong with them).
 py::object pad_likely(const py::dict& data, const Tensor& cu, int64_t to) {
-  int64_t total = 0, longest = 0;
+  // (a tensor of one entry a sequence is no token tensor; of one that is longer than the batch the padding would be for nothing)
+  int64_t total = 0, second = 0, longest = 0;
   PyObject *key, *value;
   Py_ssize_t at = 0;
   while (PyDict_Next(data.ptr(), &at, &key, &value)) {
@@ -1300,9 +1301,11 @@ py::object pad_likely(const py::dict& data, const Tensor& cu, int64_t to) {
       if (!PyLong_CheckExact(value) || (longest = PyLong_AsLongLongAndOverflow(value, &overflow), overflow != 0)) return py::none();
     }
     const Tensor* const t = is_key(key, "cu_seqlens") ? nullptr : tensor_of(value);
-    if (t != nullptr && t->dim() == 1) total = std::max(total, t->numel());
+    if (t == nullptr || t->dim() != 1 || t->numel() == total) continue;
+    second = std::max(second, std::min(total, t->numel()));
+    total = std::max(total, t->numel());
   }
-  if (total <= 0 || total >= to) return py::none();
+  if (total <= 0 || total >= to || second > cu.numel()) return py::none();
   LastValue last(cu);
   const c10::hip::HIPGuard guard(cu.device().index());
   const Tensor cu_new = empty(cu, {cu.numel() + 1}, at::kInt), cu_copy = at::empty_like(cu);
