@@ -1306,8 +1306,9 @@ py::object pad_likely(const py::dict& data, const Tensor& cu, int64_t to) {
     total = std::max(total, t->numel());
   }
   if (total <= 0 || total >= to || second > cu.numel()) return py::none();
-  LastValue last(cu);
+  require_gpu(cu);
   const c10::hip::HIPGuard guard(cu.device().index());
+  LastValue last(cu);
   const Tensor cu_new = empty(cu, {cu.numel() + 1}, at::kInt), cu_copy = at::empty_like(cu);
   py::dict out;
   std::vector<PyObject*> keys;
@@ -1324,6 +1325,7 @@ py::object pad_likely(const py::dict& data, const Tensor& cu, int64_t to) {
       set(key, value);
       const Tensor* const t = tensor_of(value);
       if (t == nullptr || t->numel() != total) continue;
+      if (t->device() != cu.device() || t->layout() != at::kStrided || t->is_nested() || t->element_size() > 16) return py::none();
       keys.push_back(key);
       moved.push_back(*t);
     }
@@ -1336,9 +1338,10 @@ py::object pad_likely(const py::dict& data, const Tensor& cu, int64_t to) {
     }
     const std::vector<Tensor> padded = pad_rows(moved, fills, cu, cu_copy, cu_new, total, to, &last);
     for (size_t i = 0; i < keys.size(); ++i) set(keys[i], py::cast(padded[i]).ptr());
-  } catch (...) {
-    PyErr_Clear();
-    return py::none();
+  } catch (const c10::OutOfMemoryError&) {  // (nothing is launched yet) of a padding that nobody has asked for it is not the caller's
+    const int64_t met = last.wait();
+    if (met == total) throw;
+    return py::int_(met);
   }
   const int64_t met = last.wait();
   if (met != total) return py::int_(met);
@@ -1431,7 +1434,13 @@ PYBIND11_MODULE(_host, m) {
   m.def("turn_gae", &turn_gae);
   m.def("gae_packed_normalized", &gae_packed_normalized);
   m.def("seqlens_of_mask", &seqlens_of_mask);
-  py::class_<LastValue>(m, "LastValue").def(py::init<const Tensor&>()).def("wait", &LastValue::wait);
+  py::class_<LastValue>(m, "LastValue")
+      .def(py::init([](const Tensor& x) {
+        require_gpu(x);
+        const c10::hip::HIPGuard guard(x.device().index());
+        return std::make_unique<LastValue>(x);
+      }))
+      .def("wait", &LastValue::wait);
   m.def("pack_rows", &pack_rows);
   m.def("pack_dict", &pack_dict);
   m.def("pad_likely", &pad_likely);

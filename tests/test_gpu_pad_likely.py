@@ -26,3 +26,39 @@ def test_not_tried_where_the_shapes_disagree(dev, sizes, tried):
         assert pad == 384 and torch.equal(cu, data["cu_seqlens"])
         assert torch.equal(got["ids"], torch.cat([data["ids"], torch.zeros(384, dtype=torch.int64, device=dev)]))
         assert all(got[k] is data[k] for k in data if k.startswith("x"))
+
+
+@pytest.fixture
+def little_memory(dev):
+    """A quarter GiB for what is allocated from here on."""
+
+    def limit():
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        room = torch.cuda.memory_reserved(dev) + (256 << 20)
+        torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(dev).total_memory, dev)
+
+    yield limit
+    torch.cuda.set_per_process_memory_fraction(1.0, dev)
+
+
+def test_out_of_memory_is_reported_once(dev, little_memory):
+    """A padding that does not fit is not tried a second time on the way for other batches."""
+    data = _batch(dev, 1000)
+    little_memory()
+    before = torch.cuda.memory_stats(dev)["num_ooms"]
+    with pytest.raises(torch.OutOfMemoryError):
+        pad_packed_tensor_dict(data, 1 << 27)
+    assert torch.cuda.memory_stats(dev)["num_ooms"] == before + 1
+    assert pad_packed_tensor_dict(data, 2000)[1] == 1000
+
+
+def test_a_wrong_padding_that_does_not_fit(dev, little_memory):
+    """The one-dimensional tensors are no token tensors: only the padding that nobody asked for is too large."""
+    data = _batch(dev, 1000, **{f"table{i}": torch.ones(10 << 20, device=dev) for i in range(3)})
+    data["ids"] = data["ids"].view(1, -1)
+    little_memory()
+    got, pad, _, _ = pad_packed_tensor_dict(data, 30 << 20)
+    assert pad == (30 << 20) - 1000 and all(got[k] is data[k] for k in data if k.startswith("table"))
+    torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert torch.equal(got["ids"], torch.nn.functional.pad(data["ids"][0], (0, pad)))
