@@ -58,3 +58,16 @@ def test_a_flag_is_out_before_notes_are_looked_at(kernels):
             behind = lines[i + 1 :]
             first = next(k for k, line in enumerate(behind) if re.match(r"(global|flat|buffer)_(load|store|atomic)", line))
             assert re.match(r"global_load_dwordx2\b.*\bsc1\b", behind[first]), (name, behind[first])
+
+
+def test_a_tile_waits_once(kernels):
+    """gae_tile_norm_kernel waits for maps and then for sums: both until one time. The clock is read to set it, in front of all
+    else, and where the loops look at it: the two that wait, and the one that looks at sums once."""
+    for name, lines in kernels.items():
+        if "gae_tile_norm_kernel" not in name:
+            continue
+        reads = [i for i, line in enumerate(lines) if line.startswith("s_memrealtime")]
+        waits = [i for i, line in enumerate(lines) if line.startswith("s_sleep")]
+        assert len(reads) == 1 + 3 and len(waits) == 2, (name, reads, waits)
+        for i in reads[1:]:
+            assert not any(line.startswith("s_add_u32") for line in lines[i + 1 : i + 9]), (name, lines[i : i + 9])
