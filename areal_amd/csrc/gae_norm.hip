@@ -3239,7 +3239,8 @@ int areal_gae_packed_normalized(const float* rewards, const float* values, const
 size_t areal_gae_packed_normalized_workspace_bytes(int64_t n_tokens, int64_t n_groups) {
   if (n_tokens <= 0 || n_groups <= 0) return 0;
   const size_t tiles = (size_t)ceil_div_i64(n_tokens, GAE_TILE);
-  return std::max(((tiles + (size_t)n_groups) * (SUMS_PITCH + 2) + tiles * GAE_SEG_WAVES * MAP_PITCH) * sizeof(uint64_t),
+  const size_t sums = round_up_i64((int64_t)(tiles + (size_t)n_groups) * (SUMS_PITCH + 2), MAP_PITCH);
+  return std::max((sums + tiles * GAE_SEG_WAVES * MAP_PITCH) * sizeof(uint64_t),
                   areal_gae_segment_stats_bytes(n_tokens, n_groups)) + 256;
 }
 int areal_gae_packed_normalized_ex(const float* rewards, const float* values, const float* loss_mask,
@@ -3289,7 +3290,7 @@ int areal_gae_packed_normalized_ex(const float* rewards, const float* values, co
   a.sums = ws;
   a.flags = ws + SUMS_PITCH * a.g.seg_slots;
   a.left = a.flags + a.g.seg_slots;
-  a.maps.at = a.left + a.g.seg_slots;
+  a.maps.at = ws + round_up_i64(a.g.seg_slots * (SUMS_PITCH + 2), MAP_PITCH);
   a.call = next_call_number();
   a.maps.call = a.call;
   a.maps.ticks = group_wait_ticks(wait_us);

@@ -209,3 +209,28 @@ def test_captured_call_takes_two_launches(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, want)), k
+
+
+@pytest.mark.parametrize("groups", [1, 2, 3, 4])
+def test_a_wave_s_map_lies_in_one_line(dev, groups):
+    """Whatever the numbers of tiles and groups: six words at the start of a line of 64 bytes, so that a map leaves and comes in
+    one piece."""
+    lib = _lib.load()
+    lens = [5 * 2048 + 7] * groups
+    n = sum(lens)
+    cu = torch.tensor([0] + lens, device=dev).cumsum(0).to(torch.int32)
+    first, rows = torch.arange(groups + 1, device=dev), torch.ones(groups, dtype=torch.int64, device=dev)
+    x = [torch.randn(n, device=dev) for _ in range(2)] + [torch.ones(n, device=dev)]
+    out = [torch.empty(n, device=dev) for _ in range(3)]
+    nbytes = lib.areal_gae_packed_normalized_workspace_bytes(n, groups)
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+    assert ws.data_ptr() % 256 == 0
+    p = _lib.ptr
+    _lib.check(lib.areal_gae_packed_normalized_ex(*map(p, x), p(cu), None, None, n, groups, 0.99, 0.95, p(first), p(rows), groups, 1, -1,
+                                                  2, 2, 1, 1e-5, -1, *map(p, out), p(ws), nbytes, _lib.stream_ptr(dev)), "ex")
+    tiles = -(-n // 2048)
+    words = ws.view(torch.int64).cpu()
+    at = words.nonzero().flatten()
+    at = at[at >= 10 * (tiles + groups)]
+    assert len(at) >= 4 * 6 * 3 * groups  # three whole tiles inside each sequence at the least
+    assert set((at % 8).tolist()) == {0, 1, 2, 3, 4, 5}
