@@ -1004,10 +1004,12 @@ DEVI void gae_tile_group_stats(const GaeArgs& g, int64_t tile, int64_t lo, int64
 }
 
 // The maps of whole tiles, handed from block to block inside a launch: each wave's total, five floats and a check word made
-// of them, each in a word of its own next to a tag made of the call's number and its place, so that a word says by itself
-// whether it is this call's. The check tells one word that is not from any other (every step of it is one to one), so that a
-// wrong map takes two tags that fit by chance, 2^-64. (Sealed as a whole like the sums, a map cost its writer and its readers
-// a microsecond of 64-bit multiplications each.)
+// of them and of the call's number, each in a word of its own next to a tag made of the call's number and its place, so that a
+// word says by itself whether it is this call's. A tag is half of the number, so that those of words 0, 2, 4 (1, 3, 5) of an
+// earlier call fit together, by chance 2^-32: the maps of two calls often differ in b1 (word 3) alone. The check tells them all the same,
+// for it starts from the half that is not in its own word's tag: of a call whose upper half fits, the lower half does not (no two
+// calls have one number), and each step of the check is one to one. A wrong map takes one more chance of 2^-32, in all
+// 2^-64. (Sealed as a whole like the sums, a map cost its writer and its readers a microsecond of 64-bit multiplications each.)
 constexpr int GAE_LOOK_TILES = 16, MAP_WORDS = 6, MAP_PITCH = 8;  // a line of 64 bytes a wave
 struct TileMaps {
   uint64_t* at;      // [tiles][GAE_SEG_WAVES][MAP_PITCH]
@@ -1016,9 +1018,9 @@ struct TileMaps {
   int wait;          // 0: it looks for maps once, and makes those that are not there itself
 };
 DEVI uint32_t map_tag(uint64_t call, int k) { return (uint32_t)(call >> (k & 1 ? 32 : 0)) + 0x9e3779b9u * (uint32_t)(k + 1); }
-DEVI uint32_t map_check(const MapF& m) {
+DEVI uint32_t map_check(uint64_t call, const MapF& m) {
   const float x[5] = {m.a11, m.a12, m.a22, m.b1, m.b2};
-  uint32_t h = 0;
+  uint32_t h = (uint32_t)call;
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
     h = (h ^ __builtin_bit_cast(uint32_t, x[k])) * 0x9e3779b1u;
@@ -1029,7 +1031,7 @@ DEVI uint32_t map_check(const MapF& m) {
 DEVI void publish_wave_map(const TileMaps& t, int64_t tile, int wave, const MapF& m) {  // m in every lane
   const int k = threadIdx.x & 63;
   const float x = k == 0 ? m.a11 : k == 1 ? m.a12 : k == 2 ? m.a22 : k == 3 ? m.b1 : m.b2;
-  const uint32_t w = k == 5 ? map_check(m) : __builtin_bit_cast(uint32_t, x);
+  const uint32_t w = k == 5 ? map_check(t.call, m) : __builtin_bit_cast(uint32_t, x);
   if (k < MAP_WORDS)
     __hip_atomic_store(t.at + (GAE_SEG_WAVES * tile + wave) * MAP_PITCH + k, (uint64_t)map_tag(t.call, k) << 32 | w,
                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1049,7 +1051,7 @@ DEVI bool gather_tile_maps(const TileMaps& t, uint64_t deadline, int64_t first, 
       for (int k = 0; k < MAP_WORDS; ++k) all &= (uint32_t)(w[k] >> 32) == map_tag(t.call, k);
       auto of = [&](int k) { return __builtin_bit_cast(float, (uint32_t)w[k]); };
       const MapF m{of(0), of(1), of(2), of(3), of(4)};
-      if (all && (uint32_t)w[5] == map_check(m)) {
+      if (all && (uint32_t)w[5] == map_check(t.call, m)) {
         chunks[lane] = m;
         have = true;
       }
