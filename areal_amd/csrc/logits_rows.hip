@@ -156,23 +156,22 @@ DEVI Online block_merge(Online st, Online* smem) {
   return r;
 }
 
-// The rows go from the last to the first, and the last ones read (rows [0, T - keep_from)) without the non-temporal hint:
-// the backward starts with them, from the first row on, while the memory-side cache of 256 MB still holds them. (The other
-// way round, the backward from the last row on, costs it 1.5 % of its own; all rows kept, the first ones push the last
-// out.) Forward and backward, bf16, us before / with it: 4096 x 151936 590 / 565, 2048 x 151936 295 / 282, 1500 x 128256
-// 184 / 180, 1000 x 151936 150 / 148; fp32 700 x 151936 204 / 196, 2000 x 128256 487 / 476. 320 MB kept where there are more
-// than 512 (2048 x 151936 286 with 256), 256 below (1500 x 128256 195 with 300). A forward that no backward follows
-// (no lse2) keeps the hint for all: 190, 193 to 203 with 260 to 700 MB kept.
-constexpr int64_t KEEP_SMALL = (int64_t)256 << 20, KEEP_LARGE = (int64_t)320 << 20, KEEP_LARGE_FROM = (int64_t)512 << 20;
+// Where a backward follows (lse2 is asked for) the logits are read without the non-temporal hint: part of the backward's reads then come
+// from the memory-side cache of 256 MB. Forward and backward, inputs new to the caches, us, under the hint / so: bf16 4096 x
+// 151936 588 / 570, 2000 x 151936 289 / 275, 1200 x 151936 174 / 168, 2000 x 128256 245 / 238, 4000 x 50257 198 / 190, 8000 x 32000 249 /
+// 242, 4000 x 64000 246 / 245, 2000 x 32000 68 / 67; fp32 500 x 128256 128 / 121, 2000 x 50257 201 / 190, 4000 x 32000 247 / 244.
+// Only the rows read last under no hint, and these the ones that the backward starts with (the forward from the last row on), is as
+// fast with long rows (568, 275, 171, 241) and slower than the hint for all with short ones (8000 x 32000 254, fp32 505 for
+// 497, 4000 x 64000 252). A forward that no backward follows keeps the hint: 2000 x 151936 190 alone, 193 to 203 without.
 // lse2[t] = max + log2(sum) in base-2 units of z2 = x * inv_temp * log2(e).
 template <typename T, int THREADS>
 __global__ __launch_bounds__(THREADS) void rows_fwd_kernel(const T* __restrict__ logits, int64_t ld,
                                                            const int64_t* __restrict__ labels, int V,
                                                            float inv_temp, float* __restrict__ logprobs,
                                                            float* __restrict__ entropy,
-                                                           float* __restrict__ lse2_out, unsigned keep_from) {
+                                                           float* __restrict__ lse2_out) {
   __shared__ Online smem[THREADS / 64];
-  const int64_t row = gridDim.x - 1 - blockIdx.x;
+  const int64_t row = blockIdx.x;
   const T* x = logits + row * ld;
   const float c2 = inv_temp * LOG2E_F;
   Online st{neg_inf(), 0.f, 0.f};
@@ -193,7 +192,7 @@ __global__ __launch_bounds__(THREADS) void rows_fwd_kernel(const T* __restrict__
       online_add(st, z, c2);
     }
   };
-  if (blockIdx.x >= keep_from) sweep(std::true_type{});
+  if (lse2_out != nullptr) sweep(std::true_type{});
   else sweep(std::false_type{});
   if ((int)threadIdx.x < rs.edge) {
     float z[1] = {Elem<T>::load(x + rs.edge_index(threadIdx.x))};
@@ -274,13 +273,10 @@ __global__ __launch_bounds__(BWD_THREADS) void rows_bwd_kernel(
 template <typename T>
 int launch_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int64_t T_, int64_t V,
                     float inv_temp, float* lp, float* ent, float* lse2, hipStream_t stream) {
-  const int64_t row_bytes = V * (int64_t)sizeof(T);
-  const int64_t keep_bytes = T_ * row_bytes <= KEEP_LARGE_FROM ? KEEP_SMALL : KEEP_LARGE;
-  const unsigned keep_from = (unsigned)(lse2 == nullptr ? T_ : std::max<int64_t>(T_ - keep_bytes / row_bytes, 0));
   auto launch = [&](auto threads) {
     constexpr int THREADS = decltype(threads)::value;
     hipLaunchKernelGGL((rows_fwd_kernel<T, THREADS>), dim3((unsigned)T_), dim3(THREADS), 0, stream,
-                       (const T*)logits, ld, labels, (int)V, inv_temp, lp, ent, lse2, keep_from);
+                       (const T*)logits, ld, labels, (int)V, inv_temp, lp, ent, lse2);
   };
   if (T_ < FWD_FEW_ROWS)
     launch(std::integral_constant<int, 1024>{});
