@@ -156,20 +156,23 @@ DEVI Online block_merge(Online st, Online* smem) {
   return r;
 }
 
-// Where a backward follows (lse2 is asked for) the logits are read without the non-temporal hint: part of the backward's reads then come
-// from the memory-side cache of 256 MB. Forward and backward, inputs new to the caches, us, under the hint / so: bf16 4096 x
-// 151936 588 / 570, 2000 x 151936 289 / 275, 1200 x 151936 174 / 168, 2000 x 128256 245 / 238, 4000 x 50257 198 / 190, 8000 x 32000 249 /
-// 242, 4000 x 64000 246 / 245, 2000 x 32000 68 / 67; fp32 500 x 128256 128 / 121, 2000 x 50257 201 / 190, 4000 x 32000 247 / 244.
-// Only the rows read last under no hint, and these the ones that the backward starts with (the forward from the last row on), is as
-// fast with long rows (568, 275, 171, 241) and slower than the hint for all with short ones (8000 x 32000 254, fp32 505 for
-// 497, 4000 x 64000 252). A forward that no backward follows keeps the hint: 2000 x 151936 190 alone, 193 to 203 without.
+// Where a backward follows (lse2 is asked for) the last rows are read without the non-temporal hint, as much as the memory-side cache
+// of 256 MB holds, or twice that of more than 900 MB, so that part of the backward's reads come from there. Forward and
+// backward, inputs new to the caches, us, all under the hint / last 256 MB without / 512 MB / all: bf16 4096 x 151936 588 / 568 /
+// 557 / 574, 3300 x 151936 477 / 457 / 454, 3500 x 128256 427 / 415 / 424 / 435, 2000 x 151936 289 / 274 / 273 / 277, 1500 x 128256 183 /
+// 176 / 187 / 187, 1200 x 151936 174 / 165 / 167 / 168, 9500 x 50257 463 / 445 / 443, 9000 x 32000 278 / 269 / 271 / 272; fp32 2000 x
+// 151936 576 / 560 / 546 / 566, 1800 x 128256 441 / 425 / 414, 4000 x 50257 390 / 377 / 375 / 379, 4000 x 32000 245 / 236 / 244 / 244. The rows
+// read from the last to the first, so that the ones kept are those that the backward starts with, give less: 562 with 320 MB at
+// 4096 x 151936, and they lose with rows of up to 128 KB (9000 x 32000 289, fp32 570 for 545) and at 128256 (3500 rows 444 with 320 MB). A
+// forward that no backward follows keeps the hint: 2000 x 151936 190, 193 to 203 without.
+constexpr int64_t KEEP_LAST = (int64_t)256 << 20, KEEP_MORE = (int64_t)512 << 20, KEEP_MORE_FROM = (int64_t)900 << 20;
 // lse2[t] = max + log2(sum) in base-2 units of z2 = x * inv_temp * log2(e).
 template <typename T, int THREADS>
 __global__ __launch_bounds__(THREADS) void rows_fwd_kernel(const T* __restrict__ logits, int64_t ld,
                                                            const int64_t* __restrict__ labels, int V,
                                                            float inv_temp, float* __restrict__ logprobs,
                                                            float* __restrict__ entropy,
-                                                           float* __restrict__ lse2_out) {
+                                                           float* __restrict__ lse2_out, unsigned keep_from) {
   __shared__ Online smem[THREADS / 64];
   const int64_t row = blockIdx.x;
   const T* x = logits + row * ld;
@@ -192,7 +195,7 @@ __global__ __launch_bounds__(THREADS) void rows_fwd_kernel(const T* __restrict__
       online_add(st, z, c2);
     }
   };
-  if (lse2_out != nullptr) sweep(std::true_type{});
+  if (blockIdx.x >= keep_from) sweep(std::true_type{});
   else sweep(std::false_type{});
   if ((int)threadIdx.x < rs.edge) {
     float z[1] = {Elem<T>::load(x + rs.edge_index(threadIdx.x))};
@@ -273,10 +276,13 @@ __global__ __launch_bounds__(BWD_THREADS) void rows_bwd_kernel(
 template <typename T>
 int launch_rows_fwd(const void* logits, int64_t ld, const int64_t* labels, int64_t T_, int64_t V,
                     float inv_temp, float* lp, float* ent, float* lse2, hipStream_t stream) {
+  const int64_t row_bytes = V * (int64_t)sizeof(T);
+  const int64_t keep_bytes = T_ * row_bytes <= KEEP_MORE_FROM ? KEEP_LAST : KEEP_MORE;
+  const unsigned keep_from = (unsigned)(lse2 == nullptr ? T_ : std::max<int64_t>(T_ - keep_bytes / row_bytes, 0));
   auto launch = [&](auto threads) {
     constexpr int THREADS = decltype(threads)::value;
     hipLaunchKernelGGL((rows_fwd_kernel<T, THREADS>), dim3((unsigned)T_), dim3(THREADS), 0, stream,
-                       (const T*)logits, ld, labels, (int)V, inv_temp, lp, ent, lse2);
+                       (const T*)logits, ld, labels, (int)V, inv_temp, lp, ent, lse2, keep_from);
   };
   if (T_ < FWD_FEW_ROWS)
     launch(std::integral_constant<int, 1024>{});

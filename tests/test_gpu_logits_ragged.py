@@ -98,3 +98,28 @@ def test_rows_kept_for_the_backward(dev, rows):
     want = -logp.exp() * w[at, None].double()
     want[pick] += w[at].double()
     torch.testing.assert_close(xg.grad[at].double(), want, rtol=1e-2, atol=1e-6)
+
+
+@pytest.mark.parametrize("rows", [1046, 1047, 3678, 3680])
+def test_the_rows_either_side_of_those_kept(dev, rows):
+    """The last 256 MB of the rows, or 512 of more than 900, are read without the non-temporal hint when a gradient is wanted: the
+    same bits as without one, on rows either side of the line; their gradient against 64 bits."""
+    vocab = 128256
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = (torch.randn(rows, vocab, generator=g, device=dev) * 2).bfloat16().requires_grad_(True)
+    y = torch.randint(0, vocab, (rows,), generator=g, device=dev)
+    w = torch.randn(rows, generator=g, device=dev)
+    lp, ent = gather_logprobs_entropy(x, y)
+    with torch.no_grad():
+        plain_lp, plain_ent = gather_logprobs_entropy(x.detach(), y)
+    assert torch.equal(lp, plain_lp) and torch.equal(ent, plain_ent)
+    (lp * w).sum().backward()
+    size = 2 * vocab
+    line = rows - ((256 if rows * size <= 900 << 20 else 512) << 20) // size
+    at = sorted({i for i in (0, line - 1, line, line + 1, rows - 1) if 0 <= i < rows})
+    logp = torch.log_softmax(x.detach()[at].double(), -1)
+    pick = (torch.arange(len(at), device=dev), y[at])
+    torch.testing.assert_close(lp[at].double(), logp[pick], rtol=1e-5, atol=2e-5)
+    want = -logp.exp() * w[at, None].double()
+    want[pick] += w[at].double()
+    torch.testing.assert_close(x.grad[at].double(), want, rtol=1e-2, atol=1e-6)
