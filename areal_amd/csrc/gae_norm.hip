@@ -838,18 +838,21 @@ __global__ __launch_bounds__(GAE_THREADS, 4) void gae_owned_kernel(GaeArgs g) {
 // of whole tiles between are the totals that these tiles' blocks need anyway: the launch that normalises hands them
 // over (TileMaps), 16 tiles at a time, for otherwise a sequence of k tiles is read k / 2 times, one chunk after the other;
 // where they do not come in time, and in gae_tile_kernel, which has no words for them, the block makes them too: the same
-// numbers, so the same bits. One launch, us, made by each block / handed over: 1024 x 1750 28.9 / 27.1, 512 x 4000 36.6 / 30,
-// 64 x 8192 48 / 22, 128 x 8192 40.7 / 25, 512 x 3000 of deviation 1.5 41.7 / 27.5, 256 x 1750 21.7 / 18.0. For a sequence over one or two whole tiles
-// too (1024 x 1600 25.2; from 2 tiles on 26.4, from 3 27.4).
+// numbers, so the same bits. One launch, us, with the code that made them all in each block / so, lognormal lengths of deviation 0.8:
+// 1024 x 1750 26.4 / 25.1 (29.4 / 28.7 with inputs new to the caches), 512 x 4000 35.7 / 27.1, 64 x 8192 41.0 / 18.8, 256 x 1750 19.1 /
+// 15.9; of deviation 1.5, 512 x 3000 57.2 / 29.1; 0.5, 32 x 16000 31.6 / 19.1; equal lengths, which cross two whole tiles at most,
+// 64 x 8192 15.1 / 15.3, 128 x 8192 19.3 / 19.1 (new inputs 21.5 / 21.9). Two launches, where each block still makes them, chunk by
+// chunk: 64 x 8192 42.6 / 40.1, 512 x 3000 58.7 / 55.1, 512 x 8192 of equal lengths 52.8 / 48.3. Handing over maps of a sequence over one
+// or two whole tiles too pays (1024 x 1600 25.2; from 2 tiles on 26.4, from 3 27.4).
 // Against blocks that walk the sequences they own tile by tile, carrying the state (the padded-row kernel above, which
 // also took cu_seqlens once): faster on 64 x 16384 tokens and on 4 x 32768, where a walking block has 16 tiles in a row.
 // The layout comes first. Up to 2048 sequences (and 1024 groups) cu_seqlens and the groups' first sequences go to LDS
 // whole, and what the tile has to find in them is counted from the registers on the way: one barrier, no load that waits
 // for another. Above 2048 a wave searches for the sequences: its first 64 probes go out with the block's first loads, one more
 // load of 128 entries holds all that the tile needs of up to 4096 sequences, and the groups are counted in LDS from what it
-// finds. With 4096 in LDS (16 loads a thread) 4000 sequences of 300 took 23.0 us, with this search 22.4; with searches that wait
-// for each other (of groups, first and last sequence, then their starts) 4096 x 300 took 22.8, with this one 22.3, 4096 x 1000
-// 51.8 and 50.4.
+// finds. With 4096 in LDS (16 loads a thread) 4000 sequences of 300 took 21.3 us, with this search 20.7; with searches by all
+// waves that wait for each other (of groups, first and last sequence, then their starts) 4096 x 300 took 20.2, with this one 20.6, 4096 x
+// 1000 in eights 54.0 and 51.8.
 // The kernel is bound by vector instruction issue (about 1150 vector and 250 scalar instructions
 // per wave and tile on 1024 sequences of mean length 1760, half as many again with the group sums) for half of its time and by
 // the chain of loads, maps and sums for the other half, with four blocks resident per CU, so
@@ -1628,10 +1631,10 @@ DEVI float norm_one(const NormParams& p, float x, float m, bool has_mask) {
 // ---- Packed GAE and the normalisation of its advantages within groups of sequences in one launch: a tile's block keeps its
 // advantages in registers, publishes its sums per group and waits for those of the other tiles of its groups, each
 // wave for another group. A launch of its own read advantages and masks back and searched the groups again, several loads
-// that wait for each other. Both forms, GAE included, us: 1024 sequences of 1750 tokens in groups of 16 30.4 / 27.1, 4096 of
-// 100 in fours (five groups to a tile) 56.3 / 35.2, 64 of 300 21.6 / 16.9, 64 of 8192 in eights 48 / 22. The rule for
-// the sizes of groups stands at areal_gae_packed_normalized_ex.
-// No wait is unbounded, as with adv_normalise_row: when the time is up, the block leaves a note for the (tile, group)
+// that wait for each other. Two launches / one, GAE included, us: 1024 sequences of 1750 tokens in groups of 16 28.1 / 25.1, 4096 of
+// 100 in fours (five groups to a tile) 56.0 / 34.0, 64 of 300 17.1 / 14.5, 64 of 8192 in eights 40.1 / 18.8 (equal lengths 16.8 /
+// 15.3). The rule for the sizes of groups stands at areal_gae_packed_normalized_ex.
+// No wait is unbounded, as with adv_normalise_row, and maps and sums have one time together: when it is up, the block leaves a note for the (tile, group)
 // segment, whose advantages are in memory anyway, and a wave that finds all sums of a group looks for notes of its tiles and
 // takes them. Leaving a note is followed by another look at the sums, publishing comes before the look for notes (leave_note).
 // Where not all tiles are on the chip at once, only the last GAE_WAIT_TILES tiles of a group on an XCD wait (it holds 128), the
@@ -3266,9 +3269,10 @@ int areal_gae_packed_normalized_ex(const float* rewards, const float* values, co
   if (!known) (void)hipGetLastError();
   // While all tiles are on the chip at once (4 blocks a CU) one launch is the better one for groups of any size measured,
   // up to 64 tiles; with more tiles the blocks that wait keep those that they wait for from starting. Two launches / one,
-  // us (tiles, tiles a group): 875, 14: 30.5 / 27.1; 875, 55: 31.1 / 29.5; 1024, 16: 35.0 / 28.8; 2000, 4: 57.2 / 53.3; and,
-  // with every block making the maps of whole tiles, 2000, 8: 60.3 / 59.3; 1953, 16: 53.7 / 61.9; 2000, 31: 57.6 / 72.8;
-  // 2048, 64: 73.5 / 155.7.
+  // us (tiles, tiles a group): 875, 14: 28.2 / 25.1; 875, 55: 28.8 / 27.5; 1024, 16: 31.7 / 26.9; 1024, 64: 32.7 / 28.6; 1040, 4:
+  // 38.0 / 33.3; 2000, 4: 56.5 / 52.0; 2000, 8: 55.0 / 53.0, of shorter sequences 49.7 / 50.6; 1200, 16: 40.1 / 39.2; 2000, 16: 54.2 /
+  // 58.6; 2000, 32: 53.1 / 64.0; 2048, 64: 54.0 / 115.3. The mean length is bounded as areal_gae_packed's, by what making all maps in each block
+  // bears: where they are handed over, longer ones would gain too (whole call of 32 x 32768 in fours 75, in one launch 25).
   const int64_t most_tiles = nb <= GAE_TILES_AT_ONCE ? 64 : 4;
   const bool one = known && capture == hipStreamCaptureStatusNone && tail_group < 0 && mean_level != LEVEL_BATCH &&
                    std_level != LEVEL_BATCH && nb <= (1 << 29) &&
