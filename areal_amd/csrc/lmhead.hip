@@ -233,7 +233,8 @@ static double xcd_distinct(int nb, int S) {
 // before / so, forward, dWeight, dHidden: 509 x 896 153, 154, 119 / 137, 137, 124; 256 x 896 108, 114, 93 / 94, 94, 104; 300 x
 // 2048 290, 277, 231 / 272, 235, 232; 400 x 5120 620, 699, 550 / 588, 645, 552; 700 x 896 237, 210, 176 / 223, 198, 181 (222 MB of
 // exponentials; dHidden in front of dWeight 225, 211, 183). With more of them than the cache holds the hints only cost: steps
-// of 1000 x 1024 (304 MB) 822 / 829, of 4096 x 896 2600 / 2760. A weight that fits it itself is not streamed.
+// of 1000 x 1024 (304 MB) 822 / 829, of 4096 x 896 2600 / 2760. A weight that fits it itself is not streamed. Of a small vocabulary
+// the cache holds more tokens, but those wait for memory no longer: 1500 x 4096 x 32000 948 / 957, 3400 1940 / 1974, dHidden alone 1332 / 1352.
 // With a bias, a scale or moments too, bf16 steps: 509 x 896 486 / 458, 480 / 446, 471 / 434; 400 x 5120 1926 / 1833, 1911 / 1822,
 // 1898 / 1815.
 // Which contraction comes first is the gradient's matter. In bf16 dWeight goes past the cache, and dHidden behind it still finds
@@ -243,13 +244,20 @@ static double xcd_distinct(int nb, int S) {
 // 2360; stored, then added to by a second such batch: 896 1253 / 1277 / 1241, 1536 1742 / 1743 / 1706, 4096 4201 / 4262 / 4179.
 // Added to alone: 509 x 896 588 / 592 / 586, 256 x 896 474 / 482 / 481, 700 x 896 744 / 777 / 753, 700 x 1024 779 / 811 / 780, 600 x
 // 2048 1357 / 1405 / 1350, 400 x 5120 2543 / 2635 / 2545, 300 x 8192 3344 / 3389 / 3273.
-// A backward that makes dlogits anew writes them past the cache, and its contractions gain from the hints even so where both read
-// them as they are written: 256 x 2048 750 -> 650, 512 x 1536 837 -> 799 (fp32 1002 -> 985, 1029 -> 1030). Where dWeight reads a
-// transposed copy (a chunk that is no multiple of 64 tokens) the hints cost: 700 x 1024 1022 / 1035, 400 x 5120 4388 / 4412 (fp32
-// 1155 / 1173, 5224 / 5244).
-constexpr int64_t PAST_PROBS_MOST = (int64_t)224 << 20, PAST_WEIGHT_LEAST = (int64_t)240 << 20;
+// dHidden alone (a weight that takes no gradient) of one tile of tokens reads the weight without the hint: 256 x 896 212 / 224, 130 x 2048 352 /
+// 369, 256 x 2048 357 / 377, 256 x 5120 758 / 766, with the exponentials kept and no hint 210, 348, 354, 749; two tiles gain, 400 x 896
+// 297 / 291, without the hint 299.
+constexpr int64_t PAST_TOKENS_MOST = 896, PAST_PROBS_MOST = (int64_t)224 << 20, PAST_WEIGHT_LEAST = (int64_t)240 << 20;
 static bool past_cache(int64_t T, int64_t H, int64_t V) {
-  return round_up_i64(T, 2 * BK) * round_up_i64(V, BK) * 2 <= PAST_PROBS_MOST && V * H * 2 >= PAST_WEIGHT_LEAST;
+  return T <= PAST_TOKENS_MOST && round_up_i64(T, 2 * BK) * round_up_i64(V, BK) * 2 <= PAST_PROBS_MOST && V * H * 2 >= PAST_WEIGHT_LEAST;
+}
+// A backward that makes dlogits anew writes them past the cache. Its contractions gain from the hints even so where dWeight is
+// bf16 and reads them as they are written: 256 x 896 392 -> 372, 256 x 2048 747 -> 663, 320 x 2048 1043 -> 1002, 512 x 8192 3326 -> 3247; not
+// of many tokens of a short row (640 x 896 847 / 866, 704 x 1024 797 / 801). Elsewhere they cost: dWeight in fp32 320 x 896 693 / 711, 384 x
+// 4096 2043 / 2081 (256 x 2048 1004 / 988); from a transposed copy (a chunk that is no multiple of 64 tokens) 700 x 1024 1022 / 1035, 400 x
+// 5120 4388 / 4412; dHidden alone 192 x 896 286 / 298, 320 x 896 436 / 457 (256 x 2048 493 / 486).
+static bool past_cache_recomputed(int64_t T, int64_t H, int64_t V, bool dw_bf16_as_written) {
+  return dw_bf16_as_written && (T <= 512 || H >= 2048) && past_cache(T, H, V);
 }
 
 // The layout of a sweep of nai A tiles against each of nbj B tiles of nk k-tiles: the numbers of A
@@ -2902,7 +2910,7 @@ int areal_lmhead_bwd(const void* hidden, const void* weight, const float* bias,
     // dWeight reads dl and hidden k-major (no transposed copies) when the chunk is a multiple
     // of 64 tokens (at least 128); otherwise it goes through dlT and hidden^T.
     const bool tn = k16_ok(Tc) && dweight_f32 != nullptr;
-    const bool past = k16_ok(Tc) && past_cache(Tc, H, V);
+    const bool past = past_cache_recomputed(Tc, H, V, dw_bf16 && tn);
     const bool need_dlT = dweight_f32 != nullptr && !tn;
     // 1. recompute logits of the chunk, emit dlogits
     {
@@ -3022,7 +3030,7 @@ int areal_lmhead_bwd_saved(const void* hidden, const void* weight, const int64_t
       AREAL_CHECK_LAUNCH();
     }
     return launch_dhidden(w_in_place ? (const u16*)weight : wT, V, e, ldv, H, T, dhidden, dh_part, rowfac, probs_status, 0,
-                          stream, past);
+                          stream, past && (T > TILE || dweight != nullptr));
   };
   auto dweight_launches = [&]() -> int {
     if (dweight == nullptr) return AREAL_OK;

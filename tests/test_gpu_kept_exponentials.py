@@ -24,9 +24,9 @@ def _inputs(dev, T):
     return hidden, weight, torch.randint(0, V, (T,), generator=g, device=dev), torch.randn(T, generator=g, device=dev), g
 
 
-def _backward(inputs, accum, **options):
+def _backward(inputs, accum, *, frozen=False, **options):
     hidden, weight, labels, grad = inputs[:4]
-    h, w = hidden.clone().requires_grad_(True), weight.clone().requires_grad_(True)
+    h, w = hidden.clone().requires_grad_(True), weight.clone().requires_grad_(not frozen)
     out = fused_lm_head_logprobs_entropy(h, w, labels, weight_grad_accum=accum, **options)
     out.logprobs.backward(grad)
     return (w.grad if accum is None else accum), h.grad, out
@@ -91,3 +91,26 @@ def test_order_and_hints(dev, gradient, kind):
     assert first[2][1] is True, first            # dHidden streams the weight
     assert first[1][1] is (gradient == "bf16"), first
     assert (first[1][0] < first[2][0]) is (gradient == "bf16"), first
+
+
+@pytest.mark.parametrize("T, gradient, saved, hint", [
+    (256, None, True, False), (300, None, True, True), (256, None, False, False), (320, None, False, False),
+    (256, "bf16", True, True), (256, "bf16", False, True), (300, "bf16", False, False), (640, "bf16", False, False),
+    (256, "fp32", True, True), (256, "fp32", False, False), (640, "fp32", False, False)])
+def test_weight_under_the_hint(dev, T, gradient, saved, hint):
+    """Whether dHidden reads the weight past the cache: not of one tile of tokens alone (a weight without a gradient), and of dlogits made
+    anew only next to a bf16 dWeight that reads them as they are written, of few tokens. Its values do not depend on it."""
+    inputs = _inputs(dev, T)
+    accum = torch.zeros(V, H, device=dev) if gradient == "fp32" else None
+    _backward(inputs, accum, save_probs=saved, frozen=gradient is None)
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        _, dh, _ = _backward(inputs, accum, save_probs=saved, frozen=gradient is None)
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if "gemm16_sweep<2" in e.name]
+    assert names and all(re.search(r"(true|false)\s*>", n).group(1) == str(hint).lower() for n in names), names
+    hidden, weight, labels, grad, _ = inputs
+    d = -torch.softmax(hidden.float() @ weight.float().t(), -1)
+    d[torch.arange(T, device=dev), labels] += 1
+    want = (d * grad[:, None]) @ weight.float()
+    assert (dh.float() - want).abs().max().item() <= 2e-2 * want.abs().max().item()
