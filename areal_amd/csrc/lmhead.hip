@@ -233,8 +233,11 @@ static double xcd_distinct(int nb, int S) {
 // before / so, forward, dWeight, dHidden: 509 x 896 153, 154, 119 / 137, 137, 124; 256 x 896 108, 114, 93 / 94, 94, 104; 300 x
 // 2048 290, 277, 231 / 272, 235, 232; 400 x 5120 620, 699, 550 / 588, 645, 552; 700 x 896 237, 210, 176 / 223, 198, 181 (222 MB of
 // exponentials; dHidden in front of dWeight 225, 211, 183). With more of them than the cache holds the hints only cost: steps
-// of 1000 x 1024 (304 MB) 822 / 829, of 4096 x 896 2600 / 2760. A weight that fits it itself is not streamed. Of a small vocabulary
-// the cache holds more tokens, but those wait for memory no longer: 1500 x 4096 x 32000 948 / 957, 3400 1940 / 1974, dHidden alone 1332 / 1352.
+// of 1000 x 1024 (304 MB) 822 / 829, of 4096 x 896 2600 / 2760. Of a small vocabulary
+// the cache holds more tokens, but those wait for memory no longer: 2000 x 4096 x 50304 1779 / 1794, dHidden alone 1179 / 1195.
+// A weight that fits the cache itself is not streamed: 500 x 4096 x 32000 (250 MB) 428 / 437, with fp32 gradients 540 / 568, dHidden alone 278 /
+// 311 (but 700 tokens 528 / 517; 700 x 1024 x 128256, 251 MB, 558 / 534); one that nearly does, not for the few exponentials of 128 tokens:
+// 128 x 896 (260 MB) 290 / 300, 64 x 896 289 / 295, 130 x 896 335 / 313; 128 x 1024 (297 MB) 304 / 266.
 // With a bias, a scale or moments too, bf16 steps: 509 x 896 486 / 458, 480 / 446, 471 / 434; 400 x 5120 1926 / 1833, 1911 / 1822,
 // 1898 / 1815.
 // Which contraction comes first is the gradient's matter. In bf16 dWeight goes past the cache, and dHidden behind it still finds
@@ -247,9 +250,11 @@ static double xcd_distinct(int nb, int S) {
 // dHidden alone (a weight that takes no gradient) of one tile of tokens reads the weight without the hint: 256 x 896 212 / 224, 130 x 2048 352 /
 // 369, 256 x 2048 357 / 377, 256 x 5120 758 / 766, with the exponentials kept and no hint 210, 348, 354, 749; two tiles gain, 400 x 896
 // 297 / 291, without the hint 299.
-constexpr int64_t PAST_TOKENS_MOST = 896, PAST_PROBS_MOST = (int64_t)224 << 20, PAST_WEIGHT_LEAST = (int64_t)240 << 20;
+constexpr int64_t PAST_TOKENS_MOST = 896, PAST_PROBS_MOST = (int64_t)224 << 20, PAST_WEIGHT_LEAST = (int64_t)256 << 20,
+                  PAST_WEIGHT_LARGE = (int64_t)288 << 20;
 static bool past_cache(int64_t T, int64_t H, int64_t V) {
-  return T <= PAST_TOKENS_MOST && round_up_i64(T, 2 * BK) * round_up_i64(V, BK) * 2 <= PAST_PROBS_MOST && V * H * 2 >= PAST_WEIGHT_LEAST;
+  return T <= PAST_TOKENS_MOST && round_up_i64(T, 2 * BK) * round_up_i64(V, BK) * 2 <= PAST_PROBS_MOST &&
+         V * H * 2 >= (T > 2 * BK ? PAST_WEIGHT_LEAST : PAST_WEIGHT_LARGE);
 }
 // A backward that makes dlogits anew writes them past the cache. Its contractions gain from the hints even so where dWeight is
 // bf16 and reads them as they are written: 256 x 896 392 -> 372, 256 x 2048 747 -> 663, 320 x 2048 1043 -> 1002, 512 x 8192 3326 -> 3247; not

@@ -13,11 +13,11 @@ from areal_amd.functional import fused_lm_head_logprobs_entropy
 
 pytestmark = pytest.mark.gpu
 
-V = 128256  # x 1024 hidden: 250 MiB of weight; 256 or 300 tokens: 63 or 94 MiB of exponentials
+V = 137984  # x 1024 hidden: 270 MiB of weight, more than the cache holds; 256 or 300 tokens: 67 or 101 MiB of exponentials
 H = 1024
 
 
-def _inputs(dev, T):
+def _inputs(dev, T, V=V):
     g = torch.Generator(device=dev).manual_seed(T)
     hidden = torch.randn(T, H, generator=g, device=dev).bfloat16()
     weight = (torch.randn(V, H, generator=g, device=dev) * (2.0 / H ** 0.5)).bfloat16()
@@ -91,6 +91,22 @@ def test_order_and_hints(dev, gradient, kind):
     assert first[2][1] is True, first            # dHidden streams the weight
     assert first[1][1] is (gradient == "bf16"), first
     assert (first[1][0] < first[2][0]) is (gradient == "bf16"), first
+
+
+@pytest.mark.parametrize("T, vocab, kept", [(256, V, True), (256, 131008, False), (129, V, True), (128, V, False), (128, 151936, True), (768, V, True),
+                                            (896, 131136, False), (897, 131136, False)])
+def test_sizes_that_keep(dev, T, vocab, kept):
+    """A weight that fits the cache itself is not streamed (131008 x 1024), one that nearly does not for 128 tokens, and of many
+    tokens or exponentials (224 MiB) nothing is kept."""
+    inputs = _inputs(dev, T, vocab)
+    _backward(inputs, None, save_probs=True)
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        _backward(inputs, None, save_probs=True)
+        torch.cuda.synchronize()
+    events = sorted((e.time_range.start, e.name) for e in prof.events() if "gemm16_sweep<" in e.name)
+    past = {v: [re.search(r"(true|false)\s*>", n).group(1) == "true" for _, n in events if f"gemm16_sweep<{v}" in n][0] for v in (0, 1, 2)}
+    assert past == {0: kept, 1: kept, 2: kept}
 
 
 @pytest.mark.parametrize("T, gradient, saved, hint", [
